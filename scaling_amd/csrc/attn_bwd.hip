@@ -717,25 +717,14 @@ extern "C" size_t mi_attn_bwd_workspace_bytes(int64_t total_q, int32_t n_q_heads
 extern "C" size_t mi_attn_bwd_workspace_bytes(int64_t total_q, int32_t n_q_heads, int32_t head_dim);
 #endif
 
-namespace {
-// query-head split of the dK/dV launch: enough workgroup groups for the 8 XCDs when there are fewer than 8 KV heads
-int dkdv_head_split(int nq, int nkv) {
-    const int n_rep = nq / nkv;
-    int h = 1;
-    while (nkv * h < 8 && n_rep % (2 * h) == 0) h *= 2;
-    return h;
-}
-size_t delta_bytes_aligned(int64_t total_q, int nq) { return ((size_t)total_q * (size_t)nq * sizeof(float) + 255) & ~(size_t)255; }
-}  // namespace
-
 #ifndef MI_ELEM_F16
 extern "C" size_t mi_attn_bwd_workspace_bytes_kv(int64_t total_q, int64_t total_k, int32_t n_q_heads, int32_t n_kv_heads,
                                                  int32_t head_dim) {
     if (total_q <= 0 || total_k <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads != 0 || head_dim <= 0)
         return mi_attn_bwd_workspace_bytes(total_q, n_q_heads, head_dim);
-    const int h = dkdv_head_split(n_q_heads, n_kv_heads);
+    const int h = mi_dkdv_head_split(n_q_heads, n_kv_heads);
     if (h == 1) return mi_attn_bwd_workspace_bytes(total_q, n_q_heads, head_dim);
-    return delta_bytes_aligned(total_q, n_q_heads) + (size_t)2 * h * (size_t)total_k * n_kv_heads * head_dim * sizeof(float);
+    return mi_delta_bytes_aligned(total_q, n_q_heads) + (size_t)2 * h * (size_t)total_k * n_kv_heads * head_dim * sizeof(float);
 }
 #endif
 
@@ -764,17 +753,7 @@ int MI_ENTRY(mi_attn_bwd_impl)(const mi_attn_bwd_args* b) {
     p.dv_st = b->dv_stride_token; p.dv_sh = b->dv_stride_head;
     p.delta = (float*)b->workspace;
     p.unrotate = a->rotary_cos == nullptr ? 0 : (a->rotary_interleaved ? 2 : 1);
-    p.hsplit = 1;
-    {   // fewer than 8 KV heads: split the query heads of a group over workgroups if the workspace has room for the partials
-        const int h = dkdv_head_split(a->n_q_heads, a->n_kv_heads);
-        const size_t part = (size_t)h * (size_t)a->total_k * a->n_kv_heads * a->head_dim * sizeof(float);
-        const size_t base = delta_bytes_aligned(a->total_q, a->n_q_heads);
-        if (h > 1 && b->workspace_bytes >= base + 2 * part) {
-            p.hsplit = h;
-            p.dk_part = (float*)((char*)b->workspace + base);
-            p.dv_part = (float*)((char*)b->workspace + base + part);
-        }
-    }
+    mi_set_head_split(a, b, &p);
     {                                                                                               // dQ: 256-query blocks
         const int per_doc = mi_blocks_per_doc(a->total_q, a->n_docs, 256);
         if (p.n_rep == 1) p.across_q = per_doc;

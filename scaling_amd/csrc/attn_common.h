@@ -583,3 +583,24 @@ static inline void mi_attn_fill_params(const mi_attn_args* a, AttnParams* p) {
     }
 }
 
+// query-head split of the dK/dV launch: enough workgroup groups for the 8 XCDs when there are fewer than 8 KV heads
+static inline int mi_dkdv_head_split(int nq, int nkv) {
+    const int n_rep = nq / nkv;
+    int h = 1;
+    while (nkv * h < 8 && n_rep % (2 * h) == 0) h *= 2;
+    return h;
+}
+static inline size_t mi_delta_bytes_aligned(int64_t total_q, int nq) { return ((size_t)total_q * (size_t)nq * sizeof(float) + 255) & ~(size_t)255; }
+
+// splits the query heads of a group over workgroups if the workspace has room for the fp32 partial sums behind delta
+static inline void mi_set_head_split(const mi_attn_args* a, const mi_attn_bwd_args* b, AttnParams* p) {
+    p->hsplit = 1;
+    const int h = mi_dkdv_head_split(a->n_q_heads, a->n_kv_heads);
+    const size_t part = (size_t)h * (size_t)a->total_k * a->n_kv_heads * a->head_dim * sizeof(float);
+    const size_t base = mi_delta_bytes_aligned(a->total_q, a->n_q_heads);
+    if (h > 1 && b->workspace_bytes >= base + 2 * part) {
+        p->hsplit = h;
+        p->dk_part = (float*)((char*)b->workspace + base);
+        p->dv_part = (float*)((char*)b->workspace + base + part);
+    }
+}

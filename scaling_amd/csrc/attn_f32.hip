@@ -2,21 +2,33 @@
 //
 // Exact fp32 semantics of core/nn/attention/attention.py:108-213 with an fp32 tensor dtype: scores, softmax,
 // probabilities and both products in fp32 (probs.to(value.dtype) is the identity), on the fp32 matrix pipe
-// (v_mfma_f32_32x32x2_f32, 157 TFLOP/s class, a sixteenth of the bf16 rate).  This is the completeness path for
-// `precision: float32` models, not a tuned one: one wavefront per workgroup, 32 x 32 score tiles, every operand
-// tile staged once in LDS with rows padded by one float (conflict-free for both the row-operand and the
-// column-gather access), no software pipelining.  Same masks, GQA index math, layouts, lse and workspace contract
-// as the 16-bit kernels; no dropout and no fused rotary (rotate with mi_rotary / mi_rotary_complex first).
+// (v_mfma_f32_32x32x2_f32, 157 TFLOP/s class, a sixteenth of the bf16 rate).  Same masks, GQA index math, layouts,
+// lse and workspace contract as the 16-bit kernels; no dropout and no fused rotary (rotate with mi_rotary /
+// mi_rotary_complex first).
 //
 // v_mfma_f32_32x32x2_f32 operands, lane = 32 g + l32:  A: row l32, k = g;  B: column l32, k = g;
-// C / D: column l32, rows 8 (r / 4) + 4 g + r % 4 for r = 0..15.  A C tile is reused as the B operand of the next
-// product one register at a time: register r contributes the two contraction indices 8 (r / 4) + r % 4 (lanes of
-// g = 0) and 4 more (g = 1), and the A operand gathers exactly those two rows.
+// C / D: column l32, rows 8 (r / 4) + 4 g + r % 4 for r = 0..15.  One such product takes 64 cycles of a SIMD, so the
+// kernels are bound by the matrix pipe as long as its operands arrive, and what matters is that every SIMD always has
+// products to issue:
+//   * a workgroup is four wavefronts that stream tiles of 32 rows through LDS, loaded global -> LDS directly, one
+//     step ahead of their use (one barrier per step);
+//   * a contraction over features may visit them in any order, so lane half g takes features 8 j + 4 g .. + 3 of step j:
+//     one 128-bit LDS read feeds four products;
+//   * a C tile is reused as the B operand of the next product one register at a time (register r stands for the
+//     contraction indices 8 (r / 4) + r % 4 and 4 more); the A operand is a row of the tile read along the features, and
+//     output row l32 of tile dt stands for feature DT l32 + dt, so that one 128-bit read feeds all DT = 4 products of
+//     head_dim 128 (64-bit for 64; head_dim 96 keeps 32 dt + l32);
+//   * LDS rows are unpadded (a direct load writes 64 x 16 consecutive bytes); the 16-byte unit index of a row is XORed
+//     with F32Tile::f(row), which spreads the 16 rows that one pass of a 128-bit read touches over all banks.
+// One wavefront per workgroup with synchronous staging, the earlier form of these kernels, kept three of the four SIMDs
+// of a compute unit busy at most and each of them waiting for its own loads: 19.1 ms for a forward + backward at 32 / 8
+// heads of 128 and 4096 causal tokens (25 TFLOP/s), now 5.3 ms (91 TFLOP/s; forward 1.18, dK/dV 2.49, dQ 1.71 ms).
 #include "attn_common.h"
 
 namespace {
 
 constexpr float kLog2eF = 1.4426950408889634f;
+constexpr int kF32Waves = 4;
 
 __device__ __forceinline__ f32x16_t mfma_f32(float a, float b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -31,89 +43,238 @@ struct F32Params {
     AttnParams m;     // masks, sizes, strides (the pointer members of m are not used)
 };
 
-// 32 rows x D floats, rows first_row .. first_row + 31 of `base` (row stride `st`, rows past last_row repeat it),
-// into an LDS tile with LD = D + 1 floats per row; one wavefront, 128-bit global reads.
-template <int D>
-__device__ __forceinline__ void stage_tile(float* tile, const float* base, int64_t st, int first_row, int last_row, int lane) {
-    constexpr int LD = D + 1, VPR = D / 4;
-#pragma unroll
-    for (int j = 0; j < 32 * VPR / 64; ++j) {
-        const int idx = j * 64 + lane;
-        const int row = idx / VPR, c4 = idx % VPR;
-        int src_row = first_row + row;
-        src_row = src_row < last_row ? src_row : last_row;
-        src_row = src_row < 0 ? 0 : src_row;
-        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(base + (int64_t)src_row * st + 4 * c4);
-        float* d = tile + row * LD + 4 * c4;
-        d[0] = x[0]; d[1] = x[1]; d[2] = x[2]; d[3] = x[3];
+// ---- LDS tile of D floats per row ------------------------------------------------------------------------------------
+template <int D> struct F32Tile {
+    static constexpr int UPR = D / 4;         // 16-byte units per row
+    static constexpr int RB = 4 * D;          // bytes per row
+    static constexpr int DT = D / 32;
+    // rows of 16 k units start on the same bank, rows of 8 and 24 units on two alternating ones
+    static __device__ __forceinline__ int f(int r) { return UPR % 16 == 0 ? (r & 15) : ((r >> 1) & 7); }
+    // feature of row `row` of output tile dt (see the header)
+    static __device__ __forceinline__ int feature(int row, int dt) { return DT == 3 ? 32 * dt + row : DT * row + dt; }
+
+    // features 8 j + 4 g .. + 3 of row `row`
+    static __device__ __forceinline__ f32x4_t row4(const char* tile, int row, int j, int g) {
+        return *reinterpret_cast<const f32x4_t*>(tile + row * RB + (((2 * j + g) ^ f(row)) << 4));
     }
+    // the features of output row l32 in all DT tiles, taken from tile row `row`
+    static __device__ __forceinline__ void cols(const char* tile, int row, int l32, float (&x)[DT]) {
+        const char* base = tile + row * RB;
+        if constexpr (DT == 4) {
+            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(base + ((l32 ^ f(row)) << 4));
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) x[dt] = v[dt];
+        } else if constexpr (DT == 2) {
+            const float2 v = *reinterpret_cast<const float2*>(base + (((l32 >> 1) ^ f(row)) << 4) + 8 * (l32 & 1));
+            x[0] = v.x; x[1] = v.y;
+        } else {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+                x[dt] = *reinterpret_cast<const float*>(base + (((8 * dt + (l32 >> 2)) ^ f(row)) << 4) + 4 * (l32 & 3));
+        }
+    }
+};
+
+// Direct global -> LDS loads of tiles of ROWS rows by the four wavefronts of a workgroup (see DmaPlan in attn_common.h
+// for the reasons behind the inline assembly; completion is tracked with wait_vmcnt).
+template <int D, int ROWS> struct F32Dma {
+    using T = F32Tile<D>;
+    static constexpr int kCount = ROWS * T::UPR / (64 * kF32Waves);   // instructions per wavefront
+    static_assert(kCount >= 1 && ROWS * T::UPR % (64 * kF32Waves) == 0, "whole instructions");
+    uint32_t off[kCount];
+    int n0, lane;
+
+    __device__ __forceinline__ static void src_of(int n, int lane_, int& row, int& byte) {
+        const int u = 64 * n + lane_;
+        row = u / T::UPR;
+        byte = 16 * ((u % T::UPR) ^ T::f(row));
+    }
+    __device__ __forceinline__ void init(int wave, int lane_, int64_t row_stride) {
+        n0 = wave * kCount;
+        lane = lane_;
+#pragma unroll
+        for (int j = 0; j < kCount; ++j) {
+            int row, byte;
+            src_of(n0 + j, lane, row, byte);
+            off[j] = (uint32_t)(row * (int)row_stride * 4 + byte);
+        }
+    }
+    // rows row0 .. row0 + ROWS - 1 of `base` (rows past last_row repeat it) into `tile`
+    __device__ __forceinline__ void issue(const float* base, int64_t row_stride, int row0, int last_row, char* tile) const {
+        char* dst = tile + 1024 * n0;
+        const int first = min(row0, last_row);
+        const float* tile_base = base + (int64_t)first * row_stride;
+        if (row0 + ROWS - 1 <= last_row) {
+#pragma unroll
+            for (int j = 0; j < kCount; ++j) DmaPlan<D, 1>::issue_one(off[j], tile_base, dst + 1024 * j);
+        } else {
+            int l = lane;
+            asm volatile("" : "+v"(l));   // opaque: keeps this rarely used arithmetic from being hoisted out of the caller's loop
+#pragma unroll
+            for (int j = 0; j < kCount; ++j) {
+                int row, byte;
+                src_of(n0 + j, l, row, byte);
+                row = min(row, last_row - first);
+                DmaPlan<D, 1>::issue_one((uint32_t)(row * (int)row_stride * 4 + byte), tile_base, dst + 1024 * j);
+            }
+        }
+    }
+};
+
+// this lane's share of a row as the B operand of a contraction over features: features 8 j + 4 g .. + 3, j = 0 .. D/8 - 1
+template <int D> __device__ __forceinline__ void load_operand(const float* row, int g, f32x4_t (&x)[D / 8]) {
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) x[j] = *reinterpret_cast<const f32x4_t*>(row + 8 * j + 4 * g);
+    // consumed here: otherwise the loads count as possibly outstanding inside the tile loop
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) asm volatile("" : "+v"(x[j]));
 }
 
-// C (+)= A B^T over the head dimension: A rows from tile_a (row l32), B rows from tile_b (row l32)
+// C = A B^T over the features: A rows row0 .. row0 + 31 of an LDS tile, B from registers
 template <int D>
-__device__ __forceinline__ f32x16_t rows_product(const float* tile_a, const float* tile_b, int l32, int g) {
-    constexpr int LD = D + 1;
+__device__ __forceinline__ f32x16_t rows_product(const char* tile, int row, int g, const f32x4_t (&b)[D / 8]) {
     f32x16_t c;
 #pragma unroll
     for (int r = 0; r < 16; ++r) c[r] = 0.f;
-    const float* ar = tile_a + l32 * LD + g;
-    const float* br = tile_b + l32 * LD + g;
-#pragma unroll 8
-    for (int ks = 0; ks < D / 2; ++ks) c = mfma_f32(ar[2 * ks], br[2 * ks], c);
+    f32x4_t a[2];
+    a[0] = F32Tile<D>::row4(tile, row, 0, g);
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+        if (j + 1 < D / 8) a[(j + 1) & 1] = F32Tile<D>::row4(tile, row, j + 1, g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c = mfma_f32(a[j & 1][i], b[j][i], c);
+    }
     return c;
 }
 
-// acc[dt] += gather(tile)^T x : contraction over the 32 rows of `tile`, x = a C tile used register by register
+// acc[dt] += columns(tile)^T x: contraction over the 32 rows of the tile from row0 on, x = a C tile register by register
 template <int D>
-__device__ __forceinline__ void cols_product(f32x16_t (&acc)[D / 32], const float* tile, const f32x16_t& x, int l32, int g) {
-    constexpr int LD = D + 1;
+__device__ __forceinline__ void cols_product(f32x16_t (&acc)[D / 32], const char* tile, int row0, const f32x16_t& x, int l32, int g) {
+    constexpr int DT = D / 32;
+    float a[2][DT];
+    F32Tile<D>::cols(tile, row0 + acc_row(0, g), l32, a[0]);
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int r = 0; r < 16; ++r) {
+        if (r + 1 < 16) F32Tile<D>::cols(tile, row0 + acc_row(r + 1, g), l32, a[(r + 1) & 1]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[dt] = mfma_f32(tile[acc_row(r, g) * LD + 32 * dt + l32], x[r], acc[dt]);
-}
-
-// lane (token, g): acc[dt][r] is feature 32 dt + 8 (r / 4) + 4 g + r % 4 of the token's row
-template <int D>
-__device__ __forceinline__ void store_rows(float* row, const f32x16_t (&acc)[D / 32], float scale, int g) {
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            f32x4_t x;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) x[c] = acc[dt][4 * a + c] * scale;
-            *reinterpret_cast<f32x4_t*>(row + 32 * dt + 8 * a + 4 * g) = x;
-        }
-}
-
-__device__ __forceinline__ void wave_min_max(int& lo, int& hi) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        lo = min(lo, __shfl_xor(lo, off, 64));
-        hi = max(hi, __shfl_xor(hi, off, 64));
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = mfma_f32(a[r & 1][dt], x[r], acc[dt]);
     }
 }
 
-// ---- forward: a wavefront owns 32 queries of one head; S^T = K Q^T (lane = query), O^T += V^T P^T -----------------
-template <int D>
-__global__ __launch_bounds__(64) void attn_f32_fwd_kernel(const F32Params fp) {
-    constexpr int LD = D + 1, DT = D / 32;
-    __shared__ float q_s[32 * LD], k_s[32 * LD], v_s[32 * LD];
+// stores the features that accumulator registers r0 .. r0 + N - 1 hold of one token's row
+template <int D, int N>
+__device__ __forceinline__ void store_row(float* row, const f32x16_t (&acc)[D / 32], int r0, float scale, int g) {
+    constexpr int DT = D / 32;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int r = r0 + i, fr = acc_row(r, g);
+        if constexpr (DT == 4) {
+            f32x4_t x;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) x[dt] = acc[dt][r] * scale;
+            *reinterpret_cast<f32x4_t*>(row + 4 * fr) = x;
+        } else if constexpr (DT == 2) {
+            *reinterpret_cast<float2*>(row + 2 * fr) = make_float2(acc[0][r] * scale, acc[1][r] * scale);
+        } else {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) row[F32Tile<D>::feature(fr, dt)] = acc[dt][r] * scale;
+        }
+    }
+}
+
+// Sum of the accumulators that the N wavefronts of a group hold for the same 32 tokens, in a fixed order; wavefront `part`
+// stores registers part * 16 / N .. of the token's row.  `slot` is the group's LDS area (N x DT x 16 x 64 floats, free for
+// use); all wavefronts of the workgroup call (two barriers).
+template <int D, int N>
+__device__ __forceinline__ void sum_and_store(f32x16_t (&acc)[D / 32], float* slot, int part, int lane, int g, float* row, bool live, float scale) {
+    constexpr int DT = D / 32, R = 16 / N;
+    if constexpr (N == 1) {
+        if (live) store_row<D, 16>(row, acc, 0, scale, g);
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) slot[((part * DT + dt) * 16 + r) * 64 + lane] = acc[dt][r];
+        __syncthreads();
+        // the register index must be a constant, the part is not: one copy of the code per part
+        static_for<N>([&](auto part_c) {
+            constexpr int P = decltype(part_c)::value;
+            if (part == P) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < R; ++i) {
+                        float s = slot[((0 * DT + dt) * 16 + P * R + i) * 64 + lane];
+#pragma unroll
+                        for (int n = 1; n < N; ++n) s += slot[((n * DT + dt) * 16 + P * R + i) * 64 + lane];
+                        acc[dt][P * R + i] = s;
+                    }
+                if (live) store_row<D, R>(row, acc, P * R, scale, g);
+            }
+        });
+    }
+}
+
+// first and one-past-last token of the union of the wavefronts' ranges (empty: 0, 0); one barrier
+__device__ __forceinline__ void block_range(int wmin, int wmax, int wave, int lane, int* lds, int& bmin, int& bmax) {
+    if (lane == 0) { lds[wave] = wmin; lds[kF32Waves + wave] = wmax; }
+    __syncthreads();
+    bmin = 0x7fffffff;
+    bmax = 0;
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w) { bmin = min(bmin, lds[w]); bmax = max(bmax, lds[kF32Waves + w]); }
+    if (bmax <= bmin) { bmin = 0; bmax = 0; }
+    bmin = __builtin_amdgcn_readfirstlane(bmin);
+    bmax = __builtin_amdgcn_readfirstlane(bmax);
+}
+
+// LDS bytes and stages of a kernel that streams two tensors in steps of ROWS rows: two stages where they fit twice into a
+// compute unit's 160 KB together with a second workgroup (FOR_TWO) or alone, else one
+template <int D, int ROWS> constexpr int stage_bytes() { return 2 * ROWS * 4 * D; }
+template <int D, int ROWS> constexpr int n_stages() { return 2 * stage_bytes<D, ROWS>() <= 128 * 1024 ? 2 : 1; }
+
+// ---- forward: QG groups of 32 queries of one head, 4 / QG wavefronts per group that take different 32-key tiles of a
+// step; S^T = K Q^T (lane = query), O^T += V^T P^T -----------------------------------------------------------------------
+template <int D, int QG>
+__global__ __launch_bounds__(64 * kF32Waves, 2) void attn_f32_fwd_kernel(const F32Params fp) {
+    constexpr int DT = D / 32, KG = kF32Waves / QG, BN = 32 * KG, BM = 32 * QG;
+    constexpr int NS = n_stages<D, BN>(), TILE = BN * 4 * D;
+    __shared__ __attribute__((aligned(1024))) char smem[NS * 2 * TILE];
+    __shared__ int range_lds[2 * kF32Waves];
+    __shared__ float ml_lds[2][kF32Waves][32];
     const AttnParams& p = fp.m;
-    const int lane = threadIdx.x, l32 = lane & 31, g = lane >> 5;
-    const int head = blockIdx.x % p.nq, qb = blockIdx.x / p.nq;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qg = wave % QG, kg = wave / QG;
+    const int nqb = (p.total_q + BM - 1) / BM;
+    int head, rank;
+    head_and_rank(blockIdx.x, p.nq, head, rank);
+    const int qb = block_for_rank(rank, nqb, p.n_docs, 0, true);
     const int kvh = head / p.n_rep;
-    const int tq = qb * 32 + l32;
+    const int tq = qb * BM + qg * 32 + l32;
     int klo, khi;
     key_range(p, tq, klo, khi);
-    int wmin = khi > klo ? klo : 0x7fffffff, wmax = khi > klo ? khi : 0;
-    wave_min_max(wmin, wmax);
-    if (wmax <= wmin) { wmin = 0; wmax = 0; }
-    const int kt0 = wmin & ~31;
-    const int n_tiles = (wmax - kt0 + 31) / 32;
+    const int wmin = __builtin_amdgcn_readfirstlane(group_min<64>(khi > klo ? klo : 0x7fffffff));
+    const int wmax = __builtin_amdgcn_readfirstlane(group_max<64>(khi > klo ? khi : 0));
+    int bmin, bmax;
+    block_range(wmin, wmax, wave, lane, range_lds, bmin, bmax);
+    const int kt0 = bmin & ~31, n_steps = (bmax - kt0 + BN - 1) / BN;
 
-    stage_tile<D>(q_s, fp.q + (int64_t)head * p.q_sh, p.q_st, qb * 32, p.total_q - 1, lane);
+    const float* kbase = fp.k + (int64_t)kvh * p.k_sh;
+    const float* vbase = fp.v + (int64_t)kvh * p.v_sh;
+    F32Dma<D, BN> k_dma, v_dma;
+    k_dma.init(wave, lane, p.k_st);
+    v_dma.init(wave, lane, p.v_st);
+    auto issue = [&](int t) {
+        if (t >= n_steps) return;
+        char* st = smem + (t % NS) * 2 * TILE;
+        k_dma.issue(kbase, p.k_st, kt0 + t * BN, p.total_k - 1, st);
+        v_dma.issue(vbase, p.v_st, kt0 + t * BN, p.total_k - 1, st + TILE);
+    };
+    f32x4_t qf[D / 8];
+    load_operand<D>(fp.q + (int64_t)min(tq, p.total_q - 1) * p.q_st + (int64_t)head * p.q_sh, g, qf);
+    issue(0);
     f32x16_t o_acc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -121,44 +282,78 @@ __global__ __launch_bounds__(64) void attn_f32_fwd_kernel(const F32Params fp) {
         for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
     float m_i = -INFINITY, l_i = 0.f;
     const float c2 = p.scale_log2;
-    for (int t = 0; t < n_tiles; ++t) {
-        const int kt = kt0 + 32 * t;
-        __syncthreads();                  // the previous tile's readers are done
-        stage_tile<D>(k_s, fp.k + (int64_t)kvh * p.k_sh, p.k_st, kt, p.total_k - 1, lane);
-        stage_tile<D>(v_s, fp.v + (int64_t)kvh * p.v_sh, p.v_st, kt, p.total_k - 1, lane);
+    for (int t = 0; t < n_steps; ++t) {
+        wait_vmcnt<0>();
+        __syncthreads();                  // step t has landed, and the readers of step t - 1 are done
+        if constexpr (NS == 2) issue(t + 1);
+        const int kt = kt0 + t * BN + 32 * kg;
+        if (kt < wmax && kt + 32 > wmin) {
+            const char* k_s = smem + (t % NS) * 2 * TILE;
+            const char* v_s = k_s + TILE;
+            f32x16_t s = rows_product<D>(k_s, 32 * kg + l32, g, qf);        // rows = keys, column = this lane's query
+            if (__any(kt < klo || kt + 32 > khi)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = kt + acc_row(r, g);
+                    if (key < klo || key >= khi) s[r] = -INFINITY;
+                }
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            const float m_cand = pair_max(mx) * c2;
+            if (__any(m_cand > m_i)) {    // rare after the first tiles: the accumulators are rescaled only then
+                const float m_new = fmaxf(m_i, m_cand);
+                float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_i - m_new);
+                asm volatile("" : "+v"(alpha));
+                m_i = m_new;
+                l_i *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
+            }
+            const float m_use = m_i == -INFINITY ? 0.f : m_i;
+            float rs = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = fast_exp2(s[r] * c2 - m_use);
+                rs += s[r];
+            }
+            l_i += rs;
+            cols_product<D>(o_acc, v_s, 32 * kg, s, l32, g);
+        }
+        if constexpr (NS == 1) {
+            __syncthreads();
+            issue(t + 1);
+        }
+    }
+    float l_tot = pair_sum(l_i), scale = 1.0f;
+    if constexpr (KG > 1) {               // bring the partial results of the group's wavefronts to one maximum
+        if (g == 0) { ml_lds[0][wave][l32] = m_i; ml_lds[1][wave][l32] = l_tot; }
         __syncthreads();
-        f32x16_t s = rows_product<D>(k_s, q_s, l32, g);        // rows = keys, column = this lane's query
-        float mx = -INFINITY;
+        float m_all = -INFINITY, l_all = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int key = kt + acc_row(r, g);
-            if (key < klo || key >= khi) s[r] = -INFINITY;
-            mx = fmaxf(mx, s[r]);
-        }
-        mx = pair_max(mx);
-        const float m_new = fmaxf(m_i, mx * c2);
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float alpha = (m_new == -INFINITY) ? 1.0f : fast_exp2(m_i - m_new);
-        m_i = m_new;
-        float rs = 0.f;
+        for (int n = 0; n < KG; ++n) m_all = fmaxf(m_all, ml_lds[0][n * QG + qg][l32]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            s[r] = fast_exp2(s[r] * c2 - m_use);
-            rs += s[r];
+        for (int n = 0; n < KG; ++n) {
+            const float m_n = ml_lds[0][n * QG + qg][l32];
+            l_all += m_n == -INFINITY ? 0.f : ml_lds[1][n * QG + qg][l32] * fast_exp2(m_n - m_all);
         }
-        l_i = l_i * alpha + rs;
+        scale = m_i == -INFINITY ? 0.f : fast_exp2(m_i - m_all);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
-        cols_product<D>(o_acc, v_s, s, l32, g);
+            for (int r = 0; r < 16; ++r) o_acc[dt][r] *= scale;
+        m_i = m_all;
+        l_tot = l_all;
     }
-    const float l_tot = pair_sum(l_i);
-    if (tq < p.total_q) {
-        store_rows<D>(fp.o + (int64_t)tq * p.o_st + (int64_t)head * p.o_sh, o_acc, l_tot > 0.f ? 1.0f / l_tot : 0.f, g);
-        if (g == 0 && fp.lse != nullptr)
-            fp.lse[(int64_t)head * p.total_q + tq] = l_tot > 0.f ? (m_i + __log2f(l_tot)) * 0.6931471805599453f : INFINITY;
-    }
+    const bool live = tq < p.total_q;
+    float* slot = reinterpret_cast<float*>(smem) + (size_t)qg * KG * DT * 16 * 64;
+    static_assert(QG * KG * DT * 16 * 64 * 4 <= NS * 2 * TILE || KG == 1, "the exchange reuses the tile stages");
+    sum_and_store<D, KG>(o_acc, slot, kg, lane, g, fp.o + (int64_t)tq * p.o_st + (int64_t)head * p.o_sh, live, l_tot > 0.f ? 1.0f / l_tot : 0.f);
+    if (live && kg == 0 && g == 0 && fp.lse != nullptr)
+        fp.lse[(int64_t)head * p.total_q + tq] = l_tot > 0.f ? (m_i + __log2f(l_tot)) * 0.6931471805599453f : INFINITY;
 }
 
 // ---- delta[h][t] = sum_d dO[t][h][d] O[t][h][d] -----------------------------------------------------------------------
@@ -183,109 +378,220 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(const F32Params fp)
     if (row < n_rows && c == 0) fp.delta[(int64_t)h * p.total_q + t] = acc;
 }
 
-// ---- dK / dV: a wavefront owns 32 keys of one KV head (K, V rows resident in LDS), loops over the group's query
-// heads and over 32-query tiles: S = Q K^T, dP = dO V^T (lane = key), dV^T += dO^T P, dK^T += Q^T dS ----------------
-template <int D>
-__global__ __launch_bounds__(64) void attn_f32_dkdv_kernel(const F32Params fp) {
-    constexpr int LD = D + 1, DT = D / 32;
-    __shared__ float k_s[32 * LD], v_s[32 * LD], q_s[32 * LD], do_s[32 * LD];
-    __shared__ float lse_s[32], delta_s[32];
+// ---- dK / dV: KGRP groups of 32 keys of one KV head (K, V rows in registers), 4 / KGRP wavefronts per group that take
+// different 32-query tiles of a step; loops over the group's query heads and over the query steps: S = Q K^T, dP = dO V^T
+// (lane = key), dV^T += dO^T P, dK^T += Q^T dS.  One wavefront per SIMD: K, V and both accumulators take 256 registers. ----
+template <int D, int KGRP>
+__global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const F32Params fp) {
+    constexpr int DT = D / 32, QS = kF32Waves / KGRP, BQ = 32 * QS, BK = 32 * KGRP;
+    constexpr int NS = n_stages<D, BQ>(), TILE = BQ * 4 * D;
+    __shared__ __attribute__((aligned(1024))) char smem[NS * 2 * TILE];
+    __shared__ __attribute__((aligned(16))) float lse_lds[2][BQ], delta_lds[2][BQ];
+    __shared__ int range_lds[2 * kF32Waves];
     const AttnParams& p = fp.m;
-    const int lane = threadIdx.x, l32 = lane & 31, g = lane >> 5;
-    const int kvh = blockIdx.x % p.nkv, kb = blockIdx.x / p.nkv;
-    const int key = kb * 32 + l32;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kgrp = wave % KGRP, qs = wave / KGRP;
+    const int nkb = (p.total_k + BK - 1) / BK;
+    // (KV head, split of its query heads) groups; the workgroup takes query heads kvh * n_rep + hs * hpw .. + hpw
+    int group, rank;
+    head_and_rank(blockIdx.x, p.nkv * p.hsplit, group, rank);
+    const int kvh = group / p.hsplit, hs = group - kvh * p.hsplit, hpw = p.n_rep / p.hsplit;
+    const int kb = block_for_rank(rank, nkb, p.n_docs, 0, false);
+    const int key = kb * BK + kgrp * 32 + l32;
     int qlo, qhi;
     query_range(p, key, qlo, qhi);
-    int wmin = qhi > qlo ? qlo : 0x7fffffff, wmax = qhi > qlo ? qhi : 0;
-    wave_min_max(wmin, wmax);
-    if (wmax <= wmin) { wmin = 0; wmax = 0; }
-    const int qt0 = wmin & ~31;
-    const int n_tiles = (wmax - qt0 + 31) / 32;
-    stage_tile<D>(k_s, fp.k + (int64_t)kvh * p.k_sh, p.k_st, kb * 32, p.total_k - 1, lane);
-    stage_tile<D>(v_s, fp.v + (int64_t)kvh * p.v_sh, p.v_st, kb * 32, p.total_k - 1, lane);
+    const int wmin = __builtin_amdgcn_readfirstlane(group_min<64>(qhi > qlo ? qlo : 0x7fffffff));
+    const int wmax = __builtin_amdgcn_readfirstlane(group_max<64>(qhi > qlo ? qhi : 0));
+    int bmin, bmax;
+    block_range(wmin, wmax, wave, lane, range_lds, bmin, bmax);
+    const int qt0 = bmin & ~31, n_tiles = (bmax - qt0 + BQ - 1) / BQ, n_steps = n_tiles * hpw;
+
+    F32Dma<D, BQ> q_dma, do_dma;
+    q_dma.init(wave, lane, p.q_st);
+    do_dma.init(wave, lane, p.o_st);
+    // (query head of the group, query tile) of the next step; heads outermost, in a fixed order: bit-reproducible sums
+    int nxt_rep = 0, nxt_tile = 0, nxt = 0;
+    float stat = 0.f;
+    const float* stat_base = tid < BQ ? fp.lse : fp.delta;
+    auto issue = [&]() {
+        if (nxt >= n_steps) return;
+        const int head = kvh * p.n_rep + hs * hpw + nxt_rep, qt = qt0 + nxt_tile * BQ;
+        char* st = smem + (nxt % NS) * 2 * TILE;
+        q_dma.issue(fp.q + (int64_t)head * p.q_sh, p.q_st, qt, p.total_q - 1, st);
+        do_dma.issue(fp.d_o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, st + TILE);
+        if (tid < 2 * BQ) stat = stat_base[(int64_t)head * p.total_q + min(qt + (tid & (BQ - 1)), p.total_q - 1)];
+        if (++nxt_tile == n_tiles) { nxt_tile = 0; ++nxt_rep; }
+        ++nxt;
+    };
+    auto put_stat = [&](int step) {
+        if (tid < BQ) lse_lds[step & 1][tid] = stat * kLog2eF;
+        else if (tid < 2 * BQ) delta_lds[step & 1][tid - BQ] = stat;
+    };
+    f32x4_t kf[D / 8], vf[D / 8];
+    {
+        const int kk = min(key, p.total_k - 1);
+        load_operand<D>(fp.k + (int64_t)kk * p.k_st + (int64_t)kvh * p.k_sh, g, kf);
+        load_operand<D>(fp.v + (int64_t)kk * p.v_st + (int64_t)kvh * p.v_sh, g, vf);
+    }
+    issue();
     f32x16_t dk_acc[DT], dv_acc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) { dk_acc[dt][r] = 0.f; dv_acc[dt][r] = 0.f; }
     const float c2 = p.scale_log2;
-    for (int rep = 0; rep < p.n_rep; ++rep) {       // fixed order: bit-reproducible sums over the group's query heads
-        const int head = kvh * p.n_rep + rep;
-        for (int t = 0; t < n_tiles; ++t) {
-            const int qt = qt0 + 32 * t;
-            __syncthreads();
-            stage_tile<D>(q_s, fp.q + (int64_t)head * p.q_sh, p.q_st, qt, p.total_q - 1, lane);
-            stage_tile<D>(do_s, fp.d_o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, lane);
-            if (lane < 32) {
-                const int tok = min(qt + lane, p.total_q - 1);
-                lse_s[lane] = fp.lse[(int64_t)head * p.total_q + tok] * kLog2eF;
-                delta_s[lane] = fp.delta[(int64_t)head * p.total_q + tok];
-            }
-            __syncthreads();
-            f32x16_t s = rows_product<D>(q_s, k_s, l32, g);        // rows = queries, column = this lane's key
-            f32x16_t dp = rows_product<D>(do_s, v_s, l32, g);
+    int tile = 0;
+    for (int step = 0; step < n_steps; ++step) {
+        put_stat(step);
+        wait_vmcnt<0>();
+        __syncthreads();                  // the step has landed, and the readers of the one before are done
+        if constexpr (NS == 2) issue();
+        const int qt = qt0 + tile * BQ + 32 * qs;
+        if (++tile == n_tiles) tile = 0;
+        if (qt < wmax && qt + 32 > wmin) {
+            const char* q_s = smem + (step % NS) * 2 * TILE;
+            const char* do_s = q_s + TILE;
+            f32x16_t s = rows_product<D>(q_s, 32 * qs + l32, g, kf);         // rows = queries, column = this lane's key
+            f32x16_t dp = rows_product<D>(do_s, 32 * qs + l32, g, vf);
+            const bool edge = __any(qt < qlo || qt + 32 > qhi);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = acc_row(r, g), q = qt + row;
-                const float pv = (q >= qlo && q < qhi) ? fast_exp2(s[r] * c2 - lse_s[row]) : 0.f;
-                s[r] = pv;
-                dp[r] = pv * (dp[r] - delta_s[row]);
+            for (int a = 0; a < 4; ++a) {
+                const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&lse_lds[step & 1][32 * qs + 8 * a + 4 * g]);
+                const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&delta_lds[step & 1][32 * qs + 8 * a + 4 * g]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int r = 4 * a + c;
+                    float pv = fast_exp2(s[r] * c2 - l4[c]);
+                    if (edge) {
+                        const int q = qt + 8 * a + 4 * g + c;
+                        if (q < qlo || q >= qhi) pv = 0.f;
+                    }
+                    s[r] = pv;
+                    dp[r] = pv * (dp[r] - d4[c]);
+                }
             }
-            cols_product<D>(dv_acc, do_s, s, l32, g);
-            cols_product<D>(dk_acc, q_s, dp, l32, g);
+            cols_product<D>(dv_acc, do_s, 32 * qs, s, l32, g);
+            cols_product<D>(dk_acc, q_s, 32 * qs, dp, l32, g);
+        }
+        if constexpr (NS == 1) {
+            __syncthreads();
+            issue();
         }
     }
-    if (key < p.total_k) {
-        store_rows<D>(fp.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh, dk_acc, p.scale, g);
-        store_rows<D>(fp.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh, dv_acc, 1.0f, g);
+    const bool live = key < p.total_k;
+    float* slot = reinterpret_cast<float*>(smem) + (size_t)kgrp * QS * DT * 16 * 64;
+    static_assert(KGRP * QS * DT * 16 * 64 * 4 <= NS * 2 * TILE || QS == 1, "the exchange reuses the tile stages");
+    float* dk_row = fp.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh;
+    float* dv_row = fp.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh;
+    if (p.hsplit > 1) {
+        const int64_t off = (((int64_t)hs * p.total_k + key) * p.nkv + kvh) * D;
+        dk_row = p.dk_part + off;
+        dv_row = p.dv_part + off;
     }
+    sum_and_store<D, QS>(dk_acc, slot, qs, lane, g, dk_row, live, p.scale);
+    sum_and_store<D, QS>(dv_acc, slot, qs, lane, g, dv_row, live, 1.0f);
 }
 
-// ---- dQ: a wavefront owns 32 queries of one head: S^T = K Q^T, dP^T = V dO^T (lane = query), dQ^T += K^T dS^T -------
+// sum of the hsplit partial dK / dV rows of a split launch, in a fixed order; one thread per four features
 template <int D>
-__global__ __launch_bounds__(64) void attn_f32_dq_kernel(const F32Params fp) {
-    constexpr int LD = D + 1, DT = D / 32;
-    __shared__ float q_s[32 * LD], do_s[32 * LD], k_s[32 * LD], v_s[32 * LD];
+__global__ __launch_bounds__(256) void attn_f32_dkdv_reduce_kernel(const F32Params fp) {
     const AttnParams& p = fp.m;
-    const int lane = threadIdx.x, l32 = lane & 31, g = lane >> 5;
-    const int head = blockIdx.x % p.nq, qb = blockIdx.x / p.nq;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x, n = (int64_t)p.total_k * p.nkv * (D / 4);
+    if (idx >= n) return;
+    const int c = (int)(idx % (D / 4)), kvh = (int)((idx / (D / 4)) % p.nkv);
+    const int64_t key = idx / ((int64_t)(D / 4) * p.nkv), stride = (int64_t)p.total_k * p.nkv * D;
+    f32x4_t k4 = *reinterpret_cast<const f32x4_t*>(p.dk_part + 4 * idx), v4 = *reinterpret_cast<const f32x4_t*>(p.dv_part + 4 * idx);
+    for (int s = 1; s < p.hsplit; ++s) {
+        k4 += *reinterpret_cast<const f32x4_t*>(p.dk_part + s * stride + 4 * idx);
+        v4 += *reinterpret_cast<const f32x4_t*>(p.dv_part + s * stride + 4 * idx);
+    }
+    *reinterpret_cast<f32x4_t*>(fp.dk + key * p.dk_st + (int64_t)kvh * p.dk_sh + 4 * c) = k4;
+    *reinterpret_cast<f32x4_t*>(fp.dv + key * p.dv_st + (int64_t)kvh * p.dv_sh + 4 * c) = v4;
+}
+
+// ---- dQ: QG groups of 32 queries of one head, 4 / QG wavefronts per group that take different 32-key tiles of a step:
+// S^T = K Q^T, dP^T = V dO^T (lane = query), dQ^T += K^T dS^T.  head_dim 128: Q, dO and dQ take 192 registers, so one
+// wavefront per SIMD (two, with 58 registers spilled: 2.1 against 1.8 ms at 4096 tokens of 32 / 8 heads) ----
+template <int D, int QG>
+__global__ __launch_bounds__(64 * kF32Waves, D == 128 ? 1 : 2) void attn_f32_dq_kernel(const F32Params fp) {
+    constexpr int DT = D / 32, KG = kF32Waves / QG, BN = 32 * KG, BM = 32 * QG;
+    constexpr int NS = n_stages<D, BN>(), TILE = BN * 4 * D;
+    __shared__ __attribute__((aligned(1024))) char smem[NS * 2 * TILE];
+    __shared__ int range_lds[2 * kF32Waves];
+    const AttnParams& p = fp.m;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qg = wave % QG, kg = wave / QG;
+    const int nqb = (p.total_q + BM - 1) / BM;
+    int head, rank;
+    head_and_rank(blockIdx.x, p.nq, head, rank);
+    const int qb = block_for_rank(rank, nqb, p.n_docs, 0, true);
     const int kvh = head / p.n_rep;
-    const int tq = qb * 32 + l32;
+    const int tq = qb * BM + qg * 32 + l32;
     int klo, khi;
     key_range(p, tq, klo, khi);
-    int wmin = khi > klo ? klo : 0x7fffffff, wmax = khi > klo ? khi : 0;
-    wave_min_max(wmin, wmax);
-    if (wmax <= wmin) { wmin = 0; wmax = 0; }
-    const int kt0 = wmin & ~31;
-    const int n_tiles = (wmax - kt0 + 31) / 32;
-    stage_tile<D>(q_s, fp.q + (int64_t)head * p.q_sh, p.q_st, qb * 32, p.total_q - 1, lane);
-    stage_tile<D>(do_s, fp.d_o + (int64_t)head * p.o_sh, p.o_st, qb * 32, p.total_q - 1, lane);
-    const int tl = tq < p.total_q ? tq : p.total_q - 1;
-    const float lse2 = fp.lse[(int64_t)head * p.total_q + tl] * kLog2eF;
-    const float delta = fp.delta[(int64_t)head * p.total_q + tl];
+    const int wmin = __builtin_amdgcn_readfirstlane(group_min<64>(khi > klo ? klo : 0x7fffffff));
+    const int wmax = __builtin_amdgcn_readfirstlane(group_max<64>(khi > klo ? khi : 0));
+    int bmin, bmax;
+    block_range(wmin, wmax, wave, lane, range_lds, bmin, bmax);
+    const int kt0 = bmin & ~31, n_steps = (bmax - kt0 + BN - 1) / BN;
+
+    const float* kbase = fp.k + (int64_t)kvh * p.k_sh;
+    const float* vbase = fp.v + (int64_t)kvh * p.v_sh;
+    F32Dma<D, BN> k_dma, v_dma;
+    k_dma.init(wave, lane, p.k_st);
+    v_dma.init(wave, lane, p.v_st);
+    auto issue = [&](int t) {
+        if (t >= n_steps) return;
+        char* st = smem + (t % NS) * 2 * TILE;
+        k_dma.issue(kbase, p.k_st, kt0 + t * BN, p.total_k - 1, st);
+        v_dma.issue(vbase, p.v_st, kt0 + t * BN, p.total_k - 1, st + TILE);
+    };
+    const int tl = min(tq, p.total_q - 1);
+    f32x4_t qf[D / 8], dof[D / 8];
+    load_operand<D>(fp.q + (int64_t)tl * p.q_st + (int64_t)head * p.q_sh, g, qf);
+    load_operand<D>(fp.d_o + (int64_t)tl * p.o_st + (int64_t)head * p.o_sh, g, dof);
+    float lse2 = fp.lse[(int64_t)head * p.total_q + tl] * kLog2eF;
+    float delta = fp.delta[(int64_t)head * p.total_q + tl];
+    asm volatile("" : "+v"(lse2), "+v"(delta));
+    issue(0);
     f32x16_t dq_acc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq_acc[dt][r] = 0.f;
     const float c2 = p.scale_log2;
-    for (int t = 0; t < n_tiles; ++t) {
-        const int kt = kt0 + 32 * t;
+    for (int t = 0; t < n_steps; ++t) {
+        wait_vmcnt<0>();
         __syncthreads();
-        stage_tile<D>(k_s, fp.k + (int64_t)kvh * p.k_sh, p.k_st, kt, p.total_k - 1, lane);
-        stage_tile<D>(v_s, fp.v + (int64_t)kvh * p.v_sh, p.v_st, kt, p.total_k - 1, lane);
-        __syncthreads();
-        f32x16_t s = rows_product<D>(k_s, q_s, l32, g);            // rows = keys, column = this lane's query
-        f32x16_t dp = rows_product<D>(v_s, do_s, l32, g);
+        if constexpr (NS == 2) issue(t + 1);
+        const int kt = kt0 + t * BN + 32 * kg;
+        if (kt < wmax && kt + 32 > wmin) {
+            const char* k_s = smem + (t % NS) * 2 * TILE;
+            const char* v_s = k_s + TILE;
+            f32x16_t s = rows_product<D>(k_s, 32 * kg + l32, g, qf);            // rows = keys, column = this lane's query
+            f32x16_t dp = rows_product<D>(v_s, 32 * kg + l32, g, dof);
+            const bool edge = __any(kt < klo || kt + 32 > khi);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int k_idx = kt + acc_row(r, g);
-            const float pv = (k_idx >= klo && k_idx < khi) ? fast_exp2(s[r] * c2 - lse2) : 0.f;
-            dp[r] = pv * (dp[r] - delta);
+            for (int r = 0; r < 16; ++r) {
+                float pv = fast_exp2(s[r] * c2 - lse2);
+                if (edge) {
+                    const int key = kt + acc_row(r, g);
+                    if (key < klo || key >= khi) pv = 0.f;
+                }
+                dp[r] = pv * (dp[r] - delta);
+            }
+            cols_product<D>(dq_acc, k_s, 32 * kg, dp, l32, g);
         }
-        cols_product<D>(dq_acc, k_s, dp, l32, g);
+        if constexpr (NS == 1) {
+            __syncthreads();
+            issue(t + 1);
+        }
     }
-    if (tq < p.total_q) store_rows<D>(fp.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh, dq_acc, p.scale, g);
+    float* slot = reinterpret_cast<float*>(smem) + (size_t)qg * KG * DT * 16 * 64;
+    static_assert(QG * KG * DT * 16 * 64 * 4 <= NS * 2 * TILE || KG == 1, "the exchange reuses the tile stages");
+    sum_and_store<D, KG>(dq_acc, slot, kg, lane, g, fp.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh, tq < p.total_q, p.scale);
 }
 
 int validate_f32(const mi_attn_args* a, const char* who) {
@@ -303,6 +609,18 @@ void fill(const mi_attn_args* a, F32Params* fp) {
     fp->o = (float*)a->o; fp->lse = a->lse;
 }
 
+// Four query groups per workgroup (every staged K / V tile feeds four wavefronts) once that gives two workgroups per compute
+// unit; below that, one query group whose four wavefronts split the keys.  Measured (head_dim 128, four groups / one):
+// 512 blocks of 128 queries 385 / 407 us, 256 blocks 277 / 208 us, 16 blocks 39 / 17 us.
+template <int D> int launch_fwd_f32(const F32Params& fp, hipStream_t st) {
+    const AttnParams& p = fp.m;
+    const dim3 block(64 * kF32Waves);
+    const int64_t wide = (((int64_t)p.total_q + 127) / 128) * p.nq, narrow = (((int64_t)p.total_q + 31) / 32) * p.nq;
+    if (wide >= 2 * mi_compute_units()) attn_f32_fwd_kernel<D, 4><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+    else attn_f32_fwd_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
+    return mi_check_launch("attn_fwd (f32)");
+}
+
 }  // namespace
 
 int mi_attn_fwd_impl_f32(const mi_attn_args* a) {
@@ -314,23 +632,22 @@ int mi_attn_fwd_impl_f32(const mi_attn_args* a) {
     if (a->total_q == 0) return MI_OK;
     F32Params fp;
     fill(a, &fp);
-    const int64_t grid = ((a->total_q + 31) / 32) * a->n_q_heads;
-    if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_fwd: too many work items");
+    if (((a->total_q + 31) / 32) * a->n_q_heads > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_fwd: too many work items");
     hipStream_t st = (hipStream_t)a->stream;
     switch (a->head_dim) {
-        case 32: attn_f32_fwd_kernel<32><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp); break;
-        case 64: attn_f32_fwd_kernel<64><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp); break;
-        case 96: attn_f32_fwd_kernel<96><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp); break;
-        case 128: attn_f32_fwd_kernel<128><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp); break;
+        case 32: return launch_fwd_f32<32>(fp, st);
+        case 64: return launch_fwd_f32<64>(fp, st);
+        case 96: return launch_fwd_f32<96>(fp, st);
+        case 128: return launch_fwd_f32<128>(fp, st);
         default: return mi_fail(MI_E_SHAPE, "attn_fwd: head_dim %d unsupported (32, 64, 96, 128)", a->head_dim);
     }
-    return mi_check_launch("attn_fwd (f32)");
 }
 
 template <int D> static int launch_bwd_f32(const F32Params& fp, int flags, hipStream_t st) {
     const AttnParams& p = fp.m;
     const int stages = flags & (MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ);
     const bool all = stages == 0;
+    const dim3 block(64 * kF32Waves);
     if (all || (stages & MI_ATTN_BWD_DELTA)) {
         const int64_t rows = (int64_t)p.total_q * p.nq;
         attn_f32_delta_kernel<D><<<dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, st>>>(fp);
@@ -338,14 +655,28 @@ template <int D> static int launch_bwd_f32(const F32Params& fp, int flags, hipSt
         if (rc != MI_OK) return rc;
     }
     if (all || (stages & MI_ATTN_BWD_DKDV)) {
-        const int64_t grid = (((int64_t)p.total_k + 31) / 32) * p.nkv;
-        attn_f32_dkdv_kernel<D><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp);
+        // two key groups per workgroup (each staged Q / dO tile feeds two wavefronts) from two workgroups per compute unit
+        // on, which a causal mask needs to pair long key blocks with short ones; below that, one key group whose four
+        // wavefronts split the queries.  Measured (head_dim 128, two groups / one): 512 blocks of 64 keys 331 / 377 us,
+        // 384 blocks 1751 / 1656 us, 256 blocks 1168 / 700 us
+        const int64_t groups = (int64_t)p.nkv * p.hsplit;
+        const int64_t wide = (((int64_t)p.total_k + 63) / 64) * groups, narrow = (((int64_t)p.total_k + 31) / 32) * groups;
+        if (wide >= 2 * mi_compute_units()) attn_f32_dkdv_kernel<D, 2><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+        else attn_f32_dkdv_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
         int rc = mi_check_launch("attn_bwd_dkdv (f32)");
         if (rc != MI_OK) return rc;
+        if (p.hsplit > 1) {
+            const int64_t n = (int64_t)p.total_k * p.nkv * (D / 4);
+            attn_f32_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(fp);
+            rc = mi_check_launch("attn_bwd_dkdv_reduce (f32)");
+            if (rc != MI_OK) return rc;
+        }
     }
     if (all || (stages & MI_ATTN_BWD_DQ)) {
-        const int64_t grid = (((int64_t)p.total_q + 31) / 32) * p.nq;
-        attn_f32_dq_kernel<D><<<dim3((unsigned)grid), dim3(64), 0, st>>>(fp);
+        const int64_t wide = (((int64_t)p.total_q + 127) / 128) * p.nq, narrow = (((int64_t)p.total_q + 31) / 32) * p.nq;
+        // as for the forward (512 blocks of 128 queries 450 / 553 us, 256 blocks 414 / 278 us at head_dim 128)
+        if (wide >= 2 * mi_compute_units()) attn_f32_dq_kernel<D, 4><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+        else attn_f32_dq_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
         return mi_check_launch("attn_bwd_dq (f32)");
     }
     return MI_OK;
@@ -374,6 +705,7 @@ int mi_attn_bwd_impl_f32(const mi_attn_bwd_args* b) {
     fp.m.dk_st = b->dk_stride_token; fp.m.dk_sh = b->dk_stride_head;
     fp.m.dv_st = b->dv_stride_token; fp.m.dv_sh = b->dv_stride_head;
     fp.delta = (float*)b->workspace;
+    mi_set_head_split(a, b, &fp.m);
     hipStream_t st = (hipStream_t)a->stream;
     switch (a->head_dim) {
         case 32: return launch_bwd_f32<32>(fp, a->flags, st);

@@ -613,6 +613,28 @@ def test_attention_float32_fwd_bwd_parity(b, s, nq, nkv, d, causal, cuts):
         assert torch.equal(o3, o2)
 
 
+@pytest.mark.parametrize("b,s,nq,nkv,d,causal,cuts", [
+    (1, 1025, 64, 64, 32, True, ()),              # one token past a 128-query, a 64-key and a 32-token boundary
+    (1, 1025, 64, 16, 128, True, (31, 32, 700)),
+    (2, 513, 64, 32, 96, False, (130,)),
+    (1, 1023, 64, 16, 64, True, (1022,)),
+])
+def test_attention_float32_wide_tilings(b, s, nq, nkv, d, causal, cuts):
+    """Enough (head, block) items for the tilings with four query groups / two key groups per workgroup (512 workgroups of
+    128 queries, 256 of 64 keys); the sums run over the same numbers of terms as in the parity test above, hence its gates."""
+    print(f"case attn f32 wide b={b} s={s} nq={nq} nkv={nkv} d={d} causal={causal} cuts={cuts}", flush=True)
+    q, k, v, do = U.make_qkv(b, s, nq, nkv, d, seed=3 + s + d, dtype=torch.float32)
+    cu = U.make_cu(b, s, cuts)
+    scale = 1.0 / math.sqrt(d)
+    ref = U.oracle_attention(q, k, v, cu, b, s, causal, scale, torch.float32, do)
+    qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    o = ops.attention(qg, kg, vg, cu.to(DEV), None, causal, scale)
+    o.backward(do.to(DEV))
+    torch.cuda.synchronize()
+    for name, got, r in (("o", o, ref[0]), ("dq", qg.grad, ref[1]), ("dk", kg.grad, ref[2]), ("dv", vg.grad, ref[3])):
+        check(f"attn.f32.wide.{name}", got, r, literal=True, max_abs_tol=1e-4, mean_rel_tol=1e-5)
+
+
 def test_attention_float32_cross_length_and_rotary():
     """fp32: keys longer than queries (causal diagonal aligned to the end of the keys), and the rotary embedding applied
     by the stand-alone kernel in front of the fp32 core when ops.attention is handed fp32 tables."""
