@@ -52,6 +52,37 @@ const char* mi_status_string(int status);
 int mi_check_device(void);
 
 /* ------------------------------------------------------------------------------------------
+ * Matrix products of small problems (the projections of core/nn/linear/column_parallel_linear.py:109-116 and
+ * row_parallel_linear.py:117-124 at tensor-parallel size 1, and what autograd derives from them):
+ *     c[m][n] = sum_s sum_k P_s[m][k] Q_s[n][k]  (+ bias[n])  (+ add[m][n], the product rounded to `dtype` first)
+ * fp32 accumulation.  P / Q are stored with the contraction index contiguous (element (m, k) at p[m * ldp + k]) or, with
+ * p_kmajor / q_kmajor, outermost (p[k * ldp + m]); p_kmajor implies q_kmajor.
+ *   y = x W^T:    P = x, Q = W          dx = dy W:   P = dy, Q = W with q_kmajor
+ *   dW = dy^T x:  P = dy, Q = x, both kmajor; p_sum (may be NULL) then receives sum_k P[m][k], the bias gradient
+ * Up to MI_GEMM_MAX_SEGMENTS products are summed into one c; up to MI_GEMM_MAX_PROBLEMS independent problems are
+ * computed by one launch.  Pointers 16-byte aligned, leading dimensions and the contiguous extent of every operand
+ * multiples of 8 elements (4 for fp32), n a multiple of 4.  m == 0 is not an error.
+ * ------------------------------------------------------------------------------------------ */
+#define MI_GEMM_MAX_SEGMENTS 3
+#define MI_GEMM_MAX_PROBLEMS 6
+typedef struct mi_gemm_segment {
+    const void* p;
+    const void* q;
+    int64_t ldp, ldq;
+    int32_t k;
+} mi_gemm_segment;
+typedef struct mi_gemm_problem {
+    mi_gemm_segment segments[MI_GEMM_MAX_SEGMENTS];
+    void* c;
+    const void* bias;              /* [n] or NULL */
+    const void* add;               /* [m, n] with row stride ldadd, or NULL; may be c */
+    void* p_sum;                   /* [m] or NULL (p_kmajor only) */
+    int64_t ldc, ldadd;
+    int32_t n_segments, p_kmajor, q_kmajor, m, n;
+} mi_gemm_problem;
+int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream);
+
+/* ------------------------------------------------------------------------------------------
  * RMSNorm.  Replaces core/nn/norm/rms_norm.py:47-50:  y = x * rsqrt(mean(x^2, -1) + eps) * weight.
  * Arithmetic in fp32, one rounding to `dtype` on store.  x, y: [n_rows, hidden]; weight: [hidden].
  * rstd (optional, may be NULL): fp32 [n_rows], receives rsqrt(mean(x^2)+eps).

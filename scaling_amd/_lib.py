@@ -1,10 +1,12 @@
-"""ctypes binding of libmi355_layer.so (C ABI declared in include/mi355_layer.h).
+"""Bindings of libmi355_layer.so (C ABI declared in include/mi355_layer.h): ctypes, and the native host path `mi355_host`
+(csrc/host.cpp), a Python extension module that calls the same C ABI.
 
-The library is loaded lazily.  There is no CPU or PyTorch fallback: if the shared object has not
+Both are loaded lazily.  There is no CPU or PyTorch fallback: if a shared object has not
 been built, or a kernel returns an error status, a RuntimeError is raised.
 """
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_uint64, POINTER, Structure, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 
@@ -12,6 +14,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libmi355_layer.so")
+HOST_PATH = os.path.join(_HERE, "csrc", "mi355_host.so")
 
 MI_BF16, MI_F16, MI_F32 = 0, 1, 2
 _DTYPE_CODE = {torch.bfloat16: MI_BF16, torch.float16: MI_F16, torch.float32: MI_F32}
@@ -22,7 +25,7 @@ EXPORTS = (
     "mi_layernorm_fwd", "mi_layernorm_bwd_workspace_bytes", "mi_layernorm_bwd", "mi_gelu_fwd", "mi_gelu_bwd", "mi_cross_entropy",
     "mi_swiglu_fwd", "mi_swiglu_bwd", "mi_rotary", "mi_rotary_complex",
     "mi_attn_fwd", "mi_attn_bwd_workspace_bytes", "mi_attn_bwd_workspace_bytes_kv", "mi_attn_bwd",
-    "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
+    "mi_gemm", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
 )
 
 
@@ -74,7 +77,21 @@ class MiDecodeArgs(Structure):
     ]
 
 
+class MiGemmSegment(Structure):
+    _fields_ = [("p", c_void_p), ("q", c_void_p), ("ldp", c_int64), ("ldq", c_int64), ("k", c_int32)]
+
+
+class MiGemmProblem(Structure):
+    _fields_ = [
+        ("segments", MiGemmSegment * 3),
+        ("c", c_void_p), ("bias", c_void_p), ("add", c_void_p), ("p_sum", c_void_p),
+        ("ldc", c_int64), ("ldadd", c_int64),
+        ("n_segments", c_int32), ("p_kmajor", c_int32), ("q_kmajor", c_int32), ("m", c_int32), ("n", c_int32),
+    ]
+
+
 _lib = None
+_host = None
 _device_checked = False
 
 
@@ -118,6 +135,8 @@ def _declare(lib):
     lib.mi_rotary_complex.restype = c_int
     lib.mi_rotary_complex.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32,
                                       c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_void_p]
+    lib.mi_gemm.restype = c_int
+    lib.mi_gemm.argtypes = [POINTER(MiGemmProblem), c_int, c_int, c_void_p]
     lib.mi_attn_fwd.restype = c_int
     lib.mi_attn_fwd.argtypes = [POINTER(MiAttnArgs)]
     lib.mi_attn_bwd_workspace_bytes.restype = c_size_t
@@ -149,6 +168,21 @@ def load(path: str = LIB_PATH):
         _declare(lib)
         _lib = lib
     return _lib
+
+
+def host():
+    """Returns the native host module; raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()                           # the module links against it
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: the host extension has not been built "
+                               "(run `python -m scaling_amd.csrc.build`); there is no fallback path")
+        spec = importlib.util.spec_from_file_location("mi355_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(status: int, what: str) -> None:

@@ -1,0 +1,322 @@
+// Matrix products of small problems for gfx950: the projections of layers whose products do not fill the chip (and whose
+// library calls cost the host more than the device), in every dtype of the package, with the epilogues the layer needs.
+//
+//     C[m][n] = sum_s sum_k P_s[m][k] Q_s[n][k]  (+ bias[n])  (+ add[m][n])
+//
+// Each operand is stored either with the contraction index contiguous ("rows": the activations and weights of a forward
+// product) or with the contraction index outermost ("kmajor": P[k][m]; the weights of an input gradient, both operands of a
+// weight gradient).  Up to three segments s are summed in one pass (the input gradient of projections that share their
+// input), and several problems go out in one launch (those projections themselves, or input and weight gradient of one).
+//
+// What bounds these calls is latency: a 256 x 256 x 256 product is 0.03 GFLOP, and with tiles of 64 x 64 it would keep 16
+// compute units busy for four dependent steps.  A workgroup of four wavefronts (2 x 2) therefore owns a TILE x TILE block with
+// TILE = 32 until there are enough 64 x 64 blocks to fill the chip; tiles pass global -> registers -> LDS with the loads of the next
+// step in flight during the products of the current one, double-buffered, one barrier per step.
+//   16-bit: v_mfma_f32_16x16x32 / 32x32x16, kmajor operands through LDS transpose reads
+//   fp32:   v_mfma_f32_16x16x4 / 32x32x2, one 128-bit read of a "rows" operand feeds four products (the contraction index is
+//           visited in an order in which a lane's four values are consecutive)
+#include "common.h"
+
+int mi_compute_units();
+
+namespace {
+
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef short v4i16_t __attribute__((ext_vector_type(4)));
+typedef short v8i16_t __attribute__((ext_vector_type(8)));
+
+constexpr int kThreads = 256;
+constexpr int kMaxProblems = MI_GEMM_MAX_PROBLEMS, kMaxSegments = MI_GEMM_MAX_SEGMENTS;
+
+struct Segment { const void* p; const void* q; int64_t ldp, ldq; int k; };
+struct Problem {
+    Segment seg[kMaxSegments];
+    void* c; const void* bias; const void* add; void* p_sum;
+    int64_t ldc, ldadd;
+    int n_seg, p_kmajor, q_kmajor, m, n, tiles_n, first_tile;
+};
+struct Problems { Problem p[kMaxProblems]; int count; };
+
+template <typename T> struct Mfma;
+#define MI_GEMM_MFMA16(T, V8, B16, B32)                                                                                          \
+    template <> struct Mfma<T> {                                                                                                 \
+        typedef V8 frag_t;                                                                                                       \
+        static constexpr int kStep16 = 32, kStep32 = 16;   /* contraction indices per product of the 16- / 32-row shape */       \
+        static __device__ __forceinline__ f32x4v mma(frag_t a, frag_t b, f32x4v c) { return B16(a, b, c, 0, 0, 0); }             \
+        static __device__ __forceinline__ f32x16_t mma(frag_t a, frag_t b, f32x16_t c) { return B32(a, b, c, 0, 0, 0); }         \
+    };
+MI_GEMM_MFMA16(__bf16, bf16x8_t, __builtin_amdgcn_mfma_f32_16x16x32_bf16, __builtin_amdgcn_mfma_f32_32x32x16_bf16)
+MI_GEMM_MFMA16(_Float16, f16x8_t, __builtin_amdgcn_mfma_f32_16x16x32_f16, __builtin_amdgcn_mfma_f32_32x32x16_f16)
+#undef MI_GEMM_MFMA16
+template <> struct Mfma<float> {
+    typedef f32x4_t frag_t;                                // four products' worth of one lane
+    static constexpr int kStep16 = 16, kStep32 = 8;
+    static __device__ __forceinline__ f32x4v mma(frag_t a, frag_t b, f32x4v c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+        return c;
+    }
+    static __device__ __forceinline__ f32x16_t mma(frag_t a, frag_t b, f32x16_t c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], c, 0, 0, 0);
+        return c;
+    }
+};
+
+// One operand's TILE x BK block in LDS.  BK = 128 (TILE 64) or 256 (TILE 32) bytes of contraction indices.
+//   rows:   TILE rows of BK, 16 bytes of padding (16 consecutive rows of a 128-bit read hit all banks once)
+//   kmajor: BK rows of TILE elements; the padding puts the rows that one transpose read (16-bit) or the lane groups of one
+//           32-bit read (fp32) touch on different banks
+template <typename T, int TILE> struct Block {
+    static constexpr int kSpan = TILE == 64 ? 128 : 256;
+    static constexpr int V = 16 / (int)sizeof(T), BK = kSpan / (int)sizeof(T);
+    static constexpr int kRowBytes = kSpan + 16;
+    static constexpr int kPad = sizeof(T) == 2 ? (TILE == 64 ? 64 : 0) : (TILE == 64 ? 32 : 16);
+    static constexpr int kKBytes = TILE * (int)sizeof(T) + kPad;
+    static constexpr int kBytes = TILE * kRowBytes > BK * kKBytes ? TILE * kRowBytes : BK * kKBytes;
+    static constexpr int kVecs = TILE * BK / V / kThreads;          // 128-bit vectors per thread
+    static_assert(kVecs * kThreads * V == TILE * BK, "whole vectors");
+
+    // vector j of this thread: (row, 16-byte unit) of the block as it is stored in memory
+    template <bool KMAJOR> static __device__ __forceinline__ void vec_pos(int j, int& row, int& unit) {
+        constexpr int UPR = KMAJOR ? TILE / V : BK / V;
+        const int v = (int)threadIdx.x + j * kThreads;
+        row = v / UPR;
+        unit = v % UPR;
+    }
+    template <bool KMAJOR> static __device__ __forceinline__ char* vec_addr(char* lds, int j) {
+        int row, unit;
+        vec_pos<KMAJOR>(j, row, unit);
+        return lds + row * (KMAJOR ? kKBytes : kRowBytes) + 16 * unit;
+    }
+    // Requests the block of rows row0.. and contraction indices k0.. .  Elements outside the matrix are marked in `ok` and
+    // zeroed where they are used: their load goes to the first vector of the matrix, so that every load is unconditional and
+    // the compiler can count the ones in flight.
+    template <bool KMAJOR> static __device__ __forceinline__ void fetch(u32x4_t (&v)[kVecs], bool (&ok)[kVecs], const T* base, int64_t ld, int row0,
+                                                                        int rows, int k0, int k) {
+#pragma unroll
+        for (int j = 0; j < kVecs; ++j) {
+            int r, u;
+            vec_pos<KMAJOR>(j, r, u);
+            const int outer = (KMAJOR ? k0 : row0) + r, inner = (KMAJOR ? row0 : k0) + u * V;
+            ok[j] = outer < (KMAJOR ? k : rows) && inner < (KMAJOR ? rows : k);
+            const int64_t off = ok[j] ? (int64_t)outer * ld + inner : 0;
+            v[j] = *reinterpret_cast<const u32x4_t*>(base + off);
+        }
+    }
+    // fragment of the SHAPE rows from `row` on for the product that covers contraction indices [k, k + step)
+    template <bool KMAJOR, int SHAPE> static __device__ __forceinline__ typename Mfma<T>::frag_t frag(const char* lds, int row, int k, int lane) {
+        using F = typename Mfma<T>::frag_t;
+        const int l = lane % SHAPE, g = lane / SHAPE;      // row of the fragment, group of contraction indices
+        if constexpr (!KMAJOR) {
+            return *reinterpret_cast<const F*>(lds + (row + l) * kRowBytes + (k + V * g) * (int)sizeof(T));
+        } else if constexpr (sizeof(T) == 2) {
+            // each block of 16 lanes reads four contraction rows of 16 elements and gets them transposed
+            const int i = lane & 15, blk = (lane >> 4) & 1;
+            const int col = row + (SHAPE == 32 ? 16 * blk : 0) + 4 * (i & 3);
+            const char* a = lds + (k + 8 * g + (i >> 2)) * kKBytes + 2 * col;
+            typedef __attribute__((address_space(3))) v4i16_t lds_v4;
+            const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(__attribute__((address_space(3))) void*)(void*)a);
+            const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(__attribute__((address_space(3))) void*)(void*)(a + 4 * kKBytes));
+            return __builtin_bit_cast(F, (v8i16_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        } else {
+            F x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const float*>(lds + (k + 4 * g + i) * kKBytes + 4 * (row + l));
+            return x;
+        }
+    }
+};
+
+template <typename T, int TILE, bool PK, bool QK>
+__device__ __forceinline__ void gemm_tile(const Problem& pr, int tm, int tn, char* smem) {
+    using B = Block<T, TILE>;
+    constexpr int SHAPE = TILE / 2, STEP = SHAPE == 32 ? Mfma<T>::kStep32 : Mfma<T>::kStep16;
+    constexpr int NR = SHAPE * SHAPE / 64;               // accumulator registers
+    typedef float acc_t __attribute__((ext_vector_type(NR)));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave & 1) * SHAPE, wn = (wave >> 1) * SHAPE;
+    const int m0 = tm * TILE, n0 = tn * TILE;
+    acc_t acc;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] = 0.f;
+    float psum[B::V];
+#pragma unroll
+    for (int i = 0; i < B::V; ++i) psum[i] = 0.f;
+    const bool want_sum = PK && pr.p_sum != nullptr && tn == 0;
+
+    // DEPTH steps are in flight: their vectors wait in registers, so a step costs its LDS traffic and a barrier, not a trip
+    // to memory (one step ahead, a 3 x 1024 x 1024 product took 8.1 us, 0.5 us per step of 64; now 6.5)
+    constexpr int DEPTH = TILE == 64 ? 2 : 4;
+    u32x4_t pv[DEPTH][B::kVecs], qv[DEPTH][B::kVecs];
+    bool pok[DEPTH][B::kVecs], qok[DEPTH][B::kVecs];
+    int seg = 0, k0 = 0, steps = 0;
+    for (int i = 0; i < pr.n_seg; ++i) steps += (pr.seg[i].k + B::BK - 1) / B::BK;
+    auto fetch = [&](int d) {                              // the next step; past the last one everything is outside the matrix
+        const Segment& s = pr.seg[seg];
+        B::template fetch<PK>(pv[d], pok[d], (const T*)s.p, s.ldp, m0, pr.m, k0, s.k);
+        B::template fetch<QK>(qv[d], qok[d], (const T*)s.q, s.ldq, n0, pr.n, k0, s.k);
+        k0 += B::BK;
+        if (k0 >= s.k && seg + 1 < pr.n_seg) { k0 = 0; ++seg; }
+    };
+    auto step = [&](auto d_c) {
+        constexpr int d = decltype(d_c)::value;
+        char* p_lds = smem + (d & 1) * 2 * B::kBytes;
+        char* q_lds = p_lds + B::kBytes;
+        const u32x4_t zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < B::kVecs; ++j) {
+            const u32x4_t a = pok[d][j] ? pv[d][j] : zero, b = qok[d][j] ? qv[d][j] : zero;
+            if constexpr (PK) {
+                if (want_sum) {
+                    float f[B::V];
+                    Elem<T>::unpack(make_uint4(a[0], a[1], a[2], a[3]), f);
+#pragma unroll
+                    for (int i = 0; i < B::V; ++i) psum[i] += f[i];
+                }
+            }
+            *reinterpret_cast<u32x4_t*>(B::template vec_addr<PK>(p_lds, j)) = a;
+            *reinterpret_cast<u32x4_t*>(B::template vec_addr<QK>(q_lds, j)) = b;
+        }
+        fetch(d);
+        __syncthreads();                                   // this step's blocks are in LDS; the other buffer's readers are done
+#pragma unroll
+        for (int k = 0; k < B::BK; k += STEP) {
+            // A = Q rows (output features), B = P rows: a lane's registers are consecutive features of one output row
+            const auto a = B::template frag<QK, SHAPE>(q_lds, wn, k, lane);
+            const auto b = B::template frag<PK, SHAPE>(p_lds, wm, k, lane);
+            acc = Mfma<T>::mma(a, b, acc);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(d);
+    for (int i = 0; i < steps; i += DEPTH) {
+        step(std::integral_constant<int, 0>{});
+        if (i + 1 < steps) step(std::integral_constant<int, 1>{});
+        if constexpr (DEPTH == 4) {
+            if (i + 2 < steps) step(std::integral_constant<int, 2>{});
+            if (i + 3 < steps) step(std::integral_constant<int, 3>{});
+        }
+    }
+    // ---- epilogue: lane = output row, registers in groups of four consecutive features
+    const int m = m0 + wm + lane % SHAPE, g = lane / SHAPE;
+    if (m < pr.m) {
+#pragma unroll
+        for (int q = 0; q < NR / 4; ++q) {
+            const int n = n0 + wn + (SHAPE == 32 ? 8 * q + 4 * g : 4 * g);
+            if (n >= pr.n) continue;                       // n is a multiple of four, as is pr.n
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = acc[4 * q + i];
+            if (pr.bias != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] += Elem<T>::load1((const T*)pr.bias + n + i);
+            }
+            if constexpr (sizeof(T) == 2) {
+                typedef T t4 __attribute__((ext_vector_type(4)));
+                if (pr.add != nullptr) {
+                    // the product is rounded before it is added, as a separate product and sum would round it
+                    const t4 a4 = *reinterpret_cast<const t4*>((const T*)pr.add + (int64_t)m * pr.ldadd + n);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = (float)(T)x[i] + (float)a4[i];
+                }
+                t4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (T)x[i];
+                *reinterpret_cast<t4*>((T*)pr.c + (int64_t)m * pr.ldc + n) = o;
+            } else {
+                if (pr.add != nullptr) {
+                    const f32x4_t a4 = *reinterpret_cast<const f32x4_t*>((const float*)pr.add + (int64_t)m * pr.ldadd + n);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] += a4[i];
+                }
+                const f32x4_t o = {x[0], x[1], x[2], x[3]};
+                *reinterpret_cast<f32x4_t*>((float*)pr.c + (int64_t)m * pr.ldc + n) = o;
+            }
+        }
+    }
+    if constexpr (PK) {
+        if (want_sum) {                                    // the same for the whole workgroup
+            // the threads of one 16-byte unit hold the sums of its elements over different contraction rows
+            constexpr int UPR = TILE / B::V, ROWS = kThreads / UPR;
+            float* lds = reinterpret_cast<float*>(smem);
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < B::V; ++i) lds[(tid / UPR) * (TILE + 1) + (tid % UPR) * B::V + i] = psum[i];
+            __syncthreads();
+            if (tid < TILE && m0 + tid < pr.m) {
+                float s = 0.f;
+                for (int r = 0; r < ROWS; ++r) s += lds[r * (TILE + 1) + tid];
+                Elem<T>::store1((T*)pr.p_sum + m0 + tid, s);
+            }
+        }
+    }
+}
+
+template <typename T, int TILE>
+__global__ __launch_bounds__(kThreads) void gemm_kernel(const Problems ps) {
+    using B = Block<T, TILE>;
+    constexpr int kSum = kThreads / (TILE / B::V) * (TILE + 1) * 4;
+    constexpr int kLds = 4 * B::kBytes > kSum ? 4 * B::kBytes : kSum;
+    __shared__ __attribute__((aligned(16))) char smem[kLds];
+    int i = 0;
+    while (i + 1 < ps.count && (int)blockIdx.x >= ps.p[i + 1].first_tile) ++i;
+    const Problem& pr = ps.p[i];
+    const int t = blockIdx.x - pr.first_tile;
+    const int tm = t / pr.tiles_n, tn = t - tm * pr.tiles_n;
+    if (pr.p_kmajor) gemm_tile<T, TILE, true, true>(pr, tm, tn, smem);
+    else if (pr.q_kmajor) gemm_tile<T, TILE, false, true>(pr, tm, tn, smem);
+    else gemm_tile<T, TILE, false, false>(pr, tm, tn, smem);
+}
+
+template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {
+    constexpr int V = Elem<T>::kVec;
+    Problems ps;
+    ps.count = count;
+    int64_t tiles64 = 0;
+    for (int i = 0; i < count; ++i) {
+        const mi_gemm_problem& a = in[i];
+        if (a.m < 0 || a.n <= 0 || a.n % 4 || a.n_segments < 1 || a.n_segments > kMaxSegments)
+            return mi_fail(MI_E_SHAPE, "gemm: bad shape m=%d n=%d segments=%d", a.m, a.n, a.n_segments);
+        if (!a.c || !mi_aligned16(a.c) || a.ldc % 4 || (a.add && (!mi_aligned16(a.add) || a.ldadd % 4)))
+            return mi_fail(MI_E_ALIGN, "gemm: c and add must be 16-byte aligned with leading dimensions that are multiples of 4");
+        if (a.p_kmajor && !a.q_kmajor) return mi_fail(MI_E_SHAPE, "gemm: a contraction-major P needs a contraction-major Q");
+        if (a.p_sum && !a.p_kmajor) return mi_fail(MI_E_SHAPE, "gemm: p_sum needs a contraction-major P");
+        Problem& p = ps.p[i];
+        for (int s = 0; s < a.n_segments; ++s) {
+            const auto& g = a.segments[s];
+            if (!g.p || !g.q || g.k <= 0) return mi_fail(MI_E_NULL, "gemm: empty segment");
+            if (!mi_aligned16(g.p) || !mi_aligned16(g.q) || g.ldp % V || g.ldq % V)
+                return mi_fail(MI_E_ALIGN, "gemm: operands must be 16-byte aligned with leading dimensions that are multiples of %d", V);
+            // the contiguous extent of each operand is read in whole vectors
+            if ((a.p_kmajor ? a.m : g.k) % V || (a.q_kmajor ? a.n : g.k) % V)
+                return mi_fail(MI_E_SHAPE, "gemm: contiguous extents must be multiples of %d elements", V);
+            p.seg[s] = Segment{g.p, g.q, g.ldp, g.ldq, g.k};
+        }
+        p.c = a.c; p.bias = a.bias; p.add = a.add; p.p_sum = a.p_sum;
+        p.ldc = a.ldc; p.ldadd = a.ldadd; p.n_seg = a.n_segments; p.p_kmajor = a.p_kmajor; p.q_kmajor = a.q_kmajor; p.m = a.m; p.n = a.n;
+        tiles64 += (int64_t)((a.m + 63) / 64) * ((a.n + 63) / 64);
+    }
+    // 64 x 64 blocks need half the traffic per product; below one of them per compute unit the finer blocks win on latency
+    const int tile = tiles64 >= mi_compute_units() ? 64 : 32;
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        Problem& p = ps.p[i];
+        p.tiles_n = (p.n + tile - 1) / tile;
+        p.first_tile = (int)total;
+        total += (int64_t)((p.m + tile - 1) / tile) * p.tiles_n;
+        if (total > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "gemm: too many tiles");
+    }
+    if (total == 0) return MI_OK;
+    if (tile == 64) gemm_kernel<T, 64><<<dim3((unsigned)total), dim3(kThreads), 0, st>>>(ps);
+    else gemm_kernel<T, 32><<<dim3((unsigned)total), dim3(kThreads), 0, st>>>(ps);
+    return mi_check_launch("gemm");
+}
+
+}  // namespace
+
+extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
+    if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
+    MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
+    return MI_OK;
+}

@@ -1,0 +1,646 @@
+// Native host path of the package: argument blocks, output allocation, launches and autograd nodes of the layer operations
+// in C++, as the Python extension module `mi355_host`.  The kernels stay behind the C ABI of libmi355_layer.so.
+//
+// Why it exists: a layer step on a few hundred tokens is 40 launches of a few microseconds each, and the Python form of
+// these functions took 10 - 40 us of host time per operation (argument blocks built field by field through ctypes, a
+// torch.cuda.current_stream() per launch, a Python autograd node per operation whose backward waits for the interpreter).
+// Here an operation costs its allocations and launches, and a backward pass runs without the interpreter.
+//
+// Linear projections run on the library product (at::mm) or, where they are too small to fill the chip, on mi_gemm; see
+// small_product for the line between the two.
+#include <torch/extension.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <ATen/autocast_mode.h>
+#include <c10/hip/HIPStream.h>
+#include <c10/hip/HIPGuard.h>
+#include <optional>
+#include <tuple>
+#include <vector>
+#include "../../include/mi355_layer.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+// ---- plumbing ----------------------------------------------------------------------------------------------------------
+void check(int status, const char* what) {
+    if (status != MI_OK)
+        throw std::runtime_error(std::string(what) + " failed: " + mi_status_string(status) + " (" + std::to_string(status) + "): " + mi_last_error());
+}
+
+void need_gpu(const Tensor& t) {
+    if (!t.is_cuda()) throw std::runtime_error("scaling_amd ops take GPU tensors only (got a CPU tensor); there is no CPU path");
+    static const int arch = mi_check_device();            // once per process; a failure is reported by every call
+    if (arch != MI_OK) check(mi_check_device(), "mi_check_device");
+}
+
+int code_of(const Tensor& t) {
+    switch (t.scalar_type()) {
+        case at::kBFloat16: return MI_BF16;
+        case at::kHalf: return MI_F16;
+        case at::kFloat: return MI_F32;
+        default: throw py::type_error(std::string("dtype ") + c10::toString(t.scalar_type()) + " is not supported by the HIP kernels");
+    }
+}
+
+// device of the tensors, and that device's current stream
+struct Launch {
+    c10::hip::HIPGuard guard;
+    void* stream;
+    explicit Launch(const Tensor& t) : guard(t.device().index()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+};
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+Tensor float_buffer(size_t bytes, const Tensor& like) {
+    return at::empty({(int64_t)((bytes + 3) / 4)}, like.options().dtype(at::kFloat));
+}
+// x as rows of its last dimension
+int64_t row_count(const Tensor& x) { return x.size(-1) == 0 ? 0 : x.numel() / x.size(-1); }
+
+// ---- norms -------------------------------------------------------------------------------------------------------------
+Tensor op_rms_norm_forward(const Tensor& x_, const Tensor& w_, double eps) {
+    need_gpu(x_);
+    TORCH_CHECK(x_.scalar_type() == w_.scalar_type() && x_.size(-1) == w_.size(0), "rms_norm: x and weight do not match");
+    Launch l(x_);
+    const Tensor x = x_.contiguous(), w = w_.contiguous();
+    Tensor y = at::empty_like(x);
+    check(mi_rmsnorm_fwd(ptr(x), ptr(w), ptr(y), nullptr, row_count(x), x.size(-1), (float)eps, code_of(x), l.stream), "mi_rmsnorm_fwd");
+    return y;
+}
+
+std::tuple<Tensor, Tensor> op_rms_norm_backward(const Tensor& x_, const Tensor& w_, const Tensor& dy_, double eps) {
+    need_gpu(x_);
+    if (x_.numel() == 0) return {at::empty_like(x_), at::zeros_like(w_)};   // no rows: the weight gradient is a sum over nothing
+    Launch l(x_);
+    const Tensor x = x_.contiguous(), w = w_.contiguous(), dy = dy_.contiguous();
+    Tensor dx = at::empty_like(x), dw = at::empty_like(w);
+    const size_t bytes = mi_rmsnorm_bwd_workspace_bytes(row_count(x), x.size(-1));
+    Tensor ws = float_buffer(bytes, x);
+    check(mi_rmsnorm_bwd(ptr(x), ptr(w), ptr(dy), ptr(dx), ptr(dw), ptr(ws), bytes, row_count(x), x.size(-1), (float)eps, code_of(x), l.stream),
+          "mi_rmsnorm_bwd");
+    return {dx, dw};
+}
+
+struct RmsNorm : Function<RmsNorm> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["eps"] = eps;
+        return op_rms_norm_forward(x, w, eps);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [dx, dw] = op_rms_norm_backward(saved[0], saved[1], g[0], ctx->saved_data["eps"].toDouble());
+        return {dx, dw, Tensor()};
+    }
+};
+
+std::tuple<Tensor, Tensor> op_layer_norm_forward(const Tensor& x_, const Tensor& w_, const OptTensor& b_, double eps, bool save_stats) {
+    need_gpu(x_);
+    TORCH_CHECK(x_.scalar_type() == w_.scalar_type() && x_.size(-1) == w_.size(0), "layer_norm: x and weight do not match");
+    Launch l(x_);
+    const Tensor x = x_.contiguous(), w = w_.contiguous(), b = b_.has_value() ? b_->contiguous() : Tensor();
+    Tensor y = at::empty_like(x), stats;
+    const int64_t rows = row_count(x);
+    if (save_stats) stats = at::empty({2, rows}, x.options().dtype(at::kFloat));
+    float* mean = save_stats ? stats.data_ptr<float>() : nullptr;
+    check(mi_layernorm_fwd(ptr(x), ptr(w), ptr(b), ptr(y), mean, mean ? mean + rows : nullptr, rows, x.size(-1), (float)eps, code_of(x), l.stream),
+          "mi_layernorm_fwd");
+    return {y, stats};
+}
+
+std::tuple<Tensor, Tensor, Tensor> op_layer_norm_backward(const Tensor& x_, const Tensor& w_, const Tensor& dy_, double eps, bool need_bias_grad,
+                                                       const OptTensor& stats) {
+    need_gpu(x_);
+    if (x_.numel() == 0) return {at::empty_like(x_), at::zeros_like(w_), need_bias_grad ? at::zeros_like(w_) : Tensor()};
+    Launch l(x_);
+    const Tensor x = x_.contiguous(), w = w_.contiguous(), dy = dy_.contiguous();
+    Tensor dx = at::empty_like(x), dw = at::empty_like(w), db = need_bias_grad ? at::empty_like(w) : Tensor();
+    const int64_t rows = row_count(x);
+    const float* mean = stats.has_value() && stats->defined() ? stats->data_ptr<float>() : nullptr;
+    const size_t bytes = mi_layernorm_bwd_workspace_bytes(rows, x.size(-1));
+    Tensor ws = float_buffer(bytes, x);
+    check(mi_layernorm_bwd(ptr(x), ptr(w), ptr(dy), mean, mean ? mean + rows : nullptr, ptr(dx), ptr(dw), ptr(db), ptr(ws), bytes, rows, x.size(-1),
+                           (float)eps, code_of(x), l.stream),
+          "mi_layernorm_bwd");
+    return {dx, dw, db};
+}
+
+struct LayerNorm : Function<LayerNorm> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& b, double eps) {
+        auto [y, stats] = op_layer_norm_forward(x, w, b, eps, true);
+        ctx->save_for_backward({x, w, stats});
+        ctx->saved_data["eps"] = eps;
+        ctx->saved_data["bias"] = b.has_value();
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [dx, dw, db] = op_layer_norm_backward(saved[0], saved[1], g[0], ctx->saved_data["eps"].toDouble(), ctx->saved_data["bias"].toBool(), saved[2]);
+        return {dx, dw, db, Tensor()};
+    }
+};
+
+// ---- activations -------------------------------------------------------------------------------------------------------
+Tensor op_gelu_forward(const Tensor& x_) {
+    need_gpu(x_);
+    Launch l(x_);
+    const Tensor x = x_.contiguous();
+    Tensor y = at::empty_like(x);
+    check(mi_gelu_fwd(ptr(x), ptr(y), x.numel(), code_of(x), l.stream), "mi_gelu_fwd");
+    return y;
+}
+
+Tensor op_gelu_backward(const Tensor& x_, const Tensor& dy_) {
+    need_gpu(x_);
+    Launch l(x_);
+    const Tensor x = x_.contiguous(), dy = dy_.contiguous();
+    Tensor dx = at::empty_like(x);
+    check(mi_gelu_bwd(ptr(x), ptr(dy), ptr(dx), x.numel(), code_of(x), l.stream), "mi_gelu_bwd");
+    return dx;
+}
+
+struct Gelu : Function<Gelu> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x) {
+        ctx->save_for_backward({x});
+        return op_gelu_forward(x);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) { return {op_gelu_backward(ctx->get_saved_variables()[0], g[0])}; }
+};
+
+Tensor op_swiglu_forward(const Tensor& a_, const Tensor& gate_) {
+    need_gpu(a_);
+    need_gpu(gate_);
+    TORCH_CHECK(a_.sizes() == gate_.sizes() && a_.scalar_type() == gate_.scalar_type(), "swiglu: a and gate do not match");
+    Launch l(a_);
+    const Tensor a = a_.contiguous(), gate = gate_.contiguous();
+    Tensor out = at::empty_like(a);
+    check(mi_swiglu_fwd(ptr(a), ptr(gate), ptr(out), a.numel(), code_of(a), l.stream), "mi_swiglu_fwd");
+    return out;
+}
+
+std::tuple<Tensor, Tensor> op_swiglu_backward(const Tensor& a_, const Tensor& gate_, const Tensor& dout_) {
+    need_gpu(a_);
+    Launch l(a_);
+    const Tensor a = a_.contiguous(), gate = gate_.contiguous(), dout = dout_.contiguous();
+    Tensor da = at::empty_like(a), dg = at::empty_like(a);
+    check(mi_swiglu_bwd(ptr(a), ptr(gate), ptr(dout), ptr(da), ptr(dg), a.numel(), code_of(a), l.stream), "mi_swiglu_bwd");
+    return {da, dg};
+}
+
+struct SwiGlu : Function<SwiGlu> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& a, const Tensor& gate) {
+        ctx->save_for_backward({a, gate});
+        return op_swiglu_forward(a, gate);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [da, dg] = op_swiglu_backward(saved[0], saved[1], g[0]);
+        return {da, dg};
+    }
+};
+
+// ---- rotary ------------------------------------------------------------------------------------------------------------
+// x [tokens, heads, head_dim] with contiguous features; the tables decide the pairing: fp32 [rows, head_dim / 2] with
+// `interleaved`, else [rows, rot_dim]
+Tensor rotary_launch(const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len_for_null_ids, bool inverse,
+                     bool interleaved) {
+    need_gpu(x);
+    TORCH_CHECK(x.dim() == 3 && x.stride(2) == 1 && cos.is_contiguous() && sin.is_contiguous(), "rotary: bad layout");
+    Launch l(x);
+    Tensor out = at::empty(x.sizes(), x.options());
+    const Tensor pos = ids.has_value() && ids->defined() ? ids->contiguous() : Tensor();
+    TORCH_CHECK(!pos.defined() || (pos.scalar_type() == at::kLong && pos.numel() == x.size(0)), "rotary: one int64 position id per token");
+    if (interleaved)
+        check(mi_rotary_complex(ptr(x), ptr(out), (const float*)ptr(cos), (const float*)ptr(sin), (const int64_t*)ptr(pos), x.size(0), (int)x.size(1),
+                                (int)x.size(2), x.stride(0), x.stride(1), out.stride(0), out.stride(1), cos.size(0), seq_len_for_null_ids, inverse,
+                                code_of(x), l.stream),
+              "mi_rotary_complex");
+    else
+        check(mi_rotary(ptr(x), ptr(out), ptr(cos), ptr(sin), (const int64_t*)ptr(pos), x.size(0), (int)x.size(1), (int)x.size(2), (int)cos.size(1),
+                        x.stride(0), x.stride(1), out.stride(0), out.stride(1), cos.size(0), seq_len_for_null_ids, inverse, code_of(x), code_of(cos),
+                        l.stream),
+              "mi_rotary");
+    return out;
+}
+
+struct Rotary : Function<Rotary> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len, bool interleaved) {
+        ctx->save_for_backward({cos, sin, opt(ids)});
+        ctx->saved_data["seq_len"] = seq_len;
+        ctx->saved_data["interleaved"] = interleaved;
+        return rotary_launch(x, cos, sin, ids, seq_len, false, interleaved);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor dout = g[0].stride(-1) == 1 ? g[0] : g[0].contiguous();
+        return {rotary_launch(dout, saved[0], saved[1], saved[2], ctx->saved_data["seq_len"].toInt(), true, ctx->saved_data["interleaved"].toBool()),
+                Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// ---- linear projections ------------------------------------------------------------------------------------------------
+// Whether a product of m x n x k multiply-adds goes to mi_gemm.  A library call costs the host 18 us whatever its size (the
+// heuristic lookup), mi_gemm 3; on the device the two meet near 3 GFLOP (16-bit: 1024 x 1024 x 1024, forward + both
+// gradients 26.7 us here and 28.6 on the library, 2048 x 512 x 2048 53 and 39 us) and 0.75 GFLOP (fp32: 333 x 1000 x 520
+// 30.5 and 29.0 us, 1024 x 1024 x 1024 80 and 57; below it the library also picks 256 x 256 blocks for
+// 256 x 256 x 256 and takes 63 us per product where mi_gemm takes 6).
+bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
+    const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
+    const double work = 2.0 * (double)m * (double)n * (double)k;
+    return n % v == 0 && k % v == 0 && work <= (v == 4 ? 0.75e9 : 3e9);
+}
+bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows that start on 16-byte boundaries
+    const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
+    return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+}
+
+void segment(mi_gemm_problem& pr, const Tensor& p, const Tensor& q, int64_t k) {
+    mi_gemm_segment& s = pr.segments[pr.n_segments++];
+    s.p = ptr(p); s.q = ptr(q); s.ldp = p.stride(0); s.ldq = q.stride(0); s.k = (int32_t)k;
+}
+mi_gemm_problem problem(const Tensor& c, bool p_kmajor, bool q_kmajor) {
+    mi_gemm_problem pr{};
+    pr.c = ptr(c); pr.ldc = c.stride(0); pr.m = (int32_t)c.size(0); pr.n = (int32_t)c.size(1);
+    pr.p_kmajor = p_kmajor; pr.q_kmajor = q_kmajor;
+    return pr;
+}
+
+// Several projections of one input: y_i = x W_i^T + b_i.  Their input gradient is one sum, their forward products and (for small
+// problems) all their gradients are one launch each.
+struct Projections : Function<Projections> {
+    // params: the n weights, then the biases of those projections whose has_bias is set (an autograd node takes no undefined
+    // tensors); bias_at gives the position of projection i's bias in params, -1 without one
+    static std::vector<int64_t> bias_at(const std::vector<int64_t>& has_bias) {
+        std::vector<int64_t> at(has_bias.size(), -1);
+        int64_t next = (int64_t)has_bias.size();
+        for (size_t i = 0; i < has_bias.size(); ++i)
+            if (has_bias[i]) at[i] = next++;
+        return at;
+    }
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, const std::vector<int64_t>& has_bias) {
+        const int64_t n = (int64_t)has_bias.size(), in = x.size(-1);
+        const auto at = bias_at(has_bias);
+        const Tensor x2 = x.reshape({-1, in});
+        const int64_t rows = x2.size(0);
+        variable_list saved{x2}, out;
+        bool small = aligned(x2);
+        for (int64_t i = 0; i < n; ++i) {
+            const Tensor& w = params[i];
+            TORCH_CHECK(w.dim() == 2 && w.size(1) == in && w.scalar_type() == x.scalar_type(), "linear: input and weight do not match");
+            small = small && aligned(w) && small_product(x, rows, w.size(0), in);
+            saved.push_back(w);
+        }
+        std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+        if (small) {
+            Launch l(x);
+            mi_gemm_problem pr[MI_GEMM_MAX_PROBLEMS];
+            for (int64_t i = 0; i < n; ++i) {
+                shape.back() = params[i].size(0);
+                out.push_back(at::empty(shape, x.options()));
+                pr[i] = problem(out.back().view({rows, shape.back()}), false, false);
+                segment(pr[i], x2, params[i], in);
+                if (at[i] >= 0) pr[i].bias = ptr(params[at[i]]);
+            }
+            check(mi_gemm(pr, (int)n, code_of(x), l.stream), "mi_gemm");
+        } else {
+            for (int64_t i = 0; i < n; ++i) {
+                shape.back() = params[i].size(0);
+                const Tensor wt = params[i].t();
+                out.push_back((at[i] >= 0 ? at::addmm(params[at[i]], x2, wt) : at::mm(x2, wt)).view(shape));
+            }
+        }
+        ctx->save_for_backward(saved);
+        ctx->saved_data["x_shape"] = x.sizes().vec();
+        ctx->saved_data["has_bias"] = has_bias;
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor& x = saved[0];
+        const int64_t n = (int64_t)g.size(), in = x.size(1), rows = x.size(0);
+        const auto has_bias = ctx->saved_data["has_bias"].toIntVector();
+        const auto at = bias_at(has_bias);                 // tensor input 1 + at[i] of the node
+        const bool need_dx = ctx->needs_input_grad(0);
+        const auto need_weight = [&](int64_t i) { return ctx->needs_input_grad(1 + i); };
+        const auto need_bias = [&](int64_t i) { return at[i] >= 0 && ctx->needs_input_grad(1 + at[i]); };
+        std::vector<Tensor> dy(n), dw(n), db(n);
+        bool small = rows > 0 && aligned(x);
+        for (int64_t i = 0; i < n; ++i) {
+            if (!g[i].defined()) continue;                 // this projection does not reach the loss
+            dy[i] = g[i].reshape({rows, saved[1 + i].size(0)});
+            if (!aligned(dy[i])) dy[i] = dy[i].contiguous();
+            small = small && aligned(dy[i]) && small_product(x, rows, dy[i].size(1), in);
+        }
+        Tensor dx;
+        if (small) {
+            Launch l(x);
+            mi_gemm_problem pr[MI_GEMM_MAX_PROBLEMS];
+            int count = 0;
+            if (need_dx) {
+                dx = at::empty({rows, in}, x.options());
+                mi_gemm_problem p = problem(dx, false, true);
+                for (int64_t i = 0; i < n; ++i)
+                    if (dy[i].defined()) segment(p, dy[i], saved[1 + i], dy[i].size(1));
+                if (p.n_segments > 0) pr[count++] = p; else dx = Tensor();
+            }
+            for (int64_t i = 0; i < n; ++i) {
+                if (!dy[i].defined()) continue;
+                if (!need_weight(i) && !need_bias(i)) continue;
+                dw[i] = at::empty({dy[i].size(1), in}, x.options());
+                mi_gemm_problem p = problem(dw[i], true, true);
+                segment(p, dy[i], x, rows);
+                if (need_bias(i)) {
+                    db[i] = at::empty({dy[i].size(1)}, x.options());
+                    p.p_sum = ptr(db[i]);
+                }
+                pr[count++] = p;
+            }
+            if (count > 0) check(mi_gemm(pr, count, code_of(x), l.stream), "mi_gemm");
+        } else {
+            for (int64_t i = 0; i < n; ++i) {
+                if (!dy[i].defined()) continue;
+                const Tensor& w = saved[1 + i];
+                if (need_dx) {
+                    if (dx.defined()) dx.addmm_(dy[i], w);  // summed inside the product
+                    else dx = at::mm(dy[i], w);
+                }
+                if (need_weight(i)) dw[i] = at::mm(dy[i].t(), x);
+                if (need_bias(i)) db[i] = dy[i].sum(0);
+            }
+        }
+        variable_list grads{dx.defined() ? dx.view(ctx->saved_data["x_shape"].toIntVector()) : Tensor()};
+        for (int64_t i = 0; i < n; ++i) grads.push_back(need_weight(i) ? dw[i] : Tensor());
+        for (int64_t i = 0; i < n; ++i)
+            if (at[i] >= 0) grads.push_back(db[i]);
+        grads.emplace_back();                              // has_bias
+        return grads;
+    }
+};
+
+// the plain library call where the native nodes do not apply: autocast chooses the dtype, CPU tensors have no kernel
+bool plain_linear(const Tensor& x, const Tensor& w) {
+    return !x.is_cuda() || x.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA) || x.scalar_type() != w.scalar_type() || x.dim() < 1 ||
+           (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat);
+}
+
+std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases) {
+    TORCH_CHECK(weights.size() == biases.size() && weights.size() >= 1 && weights.size() <= 3, "projections: one to three weights");
+    bool plain = false;
+    for (const Tensor& w : weights) plain = plain || plain_linear(x, w);
+    if (plain) {
+        std::vector<Tensor> out;
+        for (size_t i = 0; i < weights.size(); ++i) out.push_back(at::linear(x, weights[i], biases[i]));
+        return out;
+    }
+    variable_list params(weights.begin(), weights.end());
+    std::vector<int64_t> has_bias;
+    for (const OptTensor& b : biases) {
+        has_bias.push_back(b.has_value());
+        if (b.has_value()) params.push_back(*b);
+    }
+    return Projections::apply(x, at::TensorList(params), has_bias);
+}
+
+Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b) { return op_projections(x, {w}, {b})[0]; }
+
+// ---- attention core ----------------------------------------------------------------------------------------------------
+struct AttnOptions {
+    bool causal = true;
+    double scale = 1.0, dropout_p = 0.0;
+    uint64_t seed = 0;
+    int flags = 0;
+    bool interleaved = false;
+    Tensor cos, sin, pos_q, pos_k;      // undefined: no rotary; pos_k undefined (forward): k arrives rotated
+};
+
+void fill_args(mi_attn_args& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& cu_q,
+               const Tensor& cu_k, const AttnOptions& opts, void* stream) {
+    a = mi_attn_args{};
+    a.flags = opts.flags;
+    a.q = ptr(q); a.k = ptr(k); a.v = ptr(v); a.o = ptr(o); a.lse = (float*)ptr(lse);
+    a.cu_seqlens_q = (const int32_t*)ptr(cu_q); a.cu_seqlens_k = (const int32_t*)ptr(cu_k);
+    a.n_docs = (int32_t)cu_q.numel() - 1;
+    a.causal = opts.causal;
+    a.total_q = q.size(0); a.total_k = k.size(0);
+    a.n_q_heads = (int32_t)q.size(1); a.n_kv_heads = (int32_t)k.size(1); a.head_dim = (int32_t)q.size(2);
+    a.dtype = code_of(q);
+    a.q_stride_token = q.stride(0); a.q_stride_head = q.stride(1);
+    a.k_stride_token = k.stride(0); a.k_stride_head = k.stride(1);
+    a.v_stride_token = v.stride(0); a.v_stride_head = v.stride(1);
+    a.o_stride_token = o.stride(0); a.o_stride_head = o.stride(1);
+    a.softmax_scale = (float)opts.scale;
+    if (opts.cos.defined()) {
+        a.rotary_cos = ptr(opts.cos); a.rotary_sin = ptr(opts.sin);
+        a.position_ids_q = (const int64_t*)ptr(opts.pos_q); a.position_ids_k = (const int64_t*)ptr(opts.pos_k);
+        a.rotary_table_rows = opts.cos.size(0);
+        a.rotary_interleaved = opts.interleaved;
+    }
+    if (opts.dropout_p > 0.0) { a.dropout_p = (float)opts.dropout_p; a.dropout_seed = opts.seed; }
+    a.stream = stream;
+}
+
+void check_qkv(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k) {
+    need_gpu(q); need_gpu(k); need_gpu(v); need_gpu(cu_q);
+    for (const Tensor* t : {&q, &k, &v})
+        TORCH_CHECK(t->dim() == 3 && t->stride(2) == 1, "q/k/v must be [tokens, heads, head_dim] with contiguous features");
+    TORCH_CHECK(k.sizes() == v.sizes() && q.size(2) == k.size(2) && q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(),
+                "attention: q, k and v do not match");
+    TORCH_CHECK(cu_q.scalar_type() == at::kInt && cu_q.is_contiguous() && cu_q.numel() >= 1, "attention: int32 cumulative sequence lengths");
+    TORCH_CHECK(!cu_k.defined() || (cu_k.scalar_type() == at::kInt && cu_k.is_contiguous() && cu_k.numel() == cu_q.numel()),
+                "attention: int32 cumulative key lengths, as many as for the queries");
+}
+
+std::tuple<Tensor, Tensor> attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k,
+                                        const AttnOptions& opts, const Tensor& q_rot) {
+    Launch l(q);
+    Tensor o = at::empty({q.size(0), q.size(1), q.size(2)}, q.options());
+    Tensor lse = at::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat));
+    mi_attn_args a;
+    fill_args(a, q, k, v, o, lse, cu_q, cu_k, opts, l.stream);
+    a.q_rot_out = ptr(q_rot);
+    check(mi_attn_fwd(&a), "mi_attn_fwd");
+    return {o, lse};
+}
+
+// dq must have the strides of q; `ws` may be undefined
+void attn_backward(const Tensor& d_o_, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& cu_q,
+                   const Tensor& cu_k, const AttnOptions& opts, const Tensor& dq, const Tensor& dk, const Tensor& dv, Tensor ws) {
+    Launch l(q);
+    TORCH_CHECK(dq.strides() == q.strides(), "attention backward: dq needs the layout of q");
+    Tensor d_o = d_o_;
+    if (d_o.strides() != o.strides()) d_o = at::empty_strided(o.sizes(), o.strides(), o.options()).copy_(d_o_);
+    if (!ws.defined()) ws = float_buffer(std::max<size_t>(16, mi_attn_bwd_workspace_bytes_kv(q.size(0), k.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2))), q);
+    mi_attn_bwd_args b{};
+    fill_args(b.fwd, q, k, v, o, lse, cu_q, cu_k, opts, l.stream);
+    b.d_o = ptr(d_o); b.dq = ptr(dq); b.dk = ptr(dk); b.dv = ptr(dv);
+    b.dk_stride_token = dk.stride(0); b.dk_stride_head = dk.stride(1);
+    b.dv_stride_token = dv.stride(0); b.dv_stride_head = dv.stride(1);
+    b.workspace = ptr(ws);
+    b.workspace_bytes = (size_t)ws.numel() * 4;
+    check(mi_attn_bwd(&b), "mi_attn_bwd");
+}
+
+AttnOptions options(bool causal, double scale, int flags, double dropout_p, uint64_t seed, const OptTensor& cos, const OptTensor& sin,
+                    const OptTensor& pos_q, const OptTensor& pos_k, bool interleaved) {
+    AttnOptions o;
+    o.causal = causal; o.scale = scale; o.flags = flags; o.dropout_p = dropout_p; o.seed = seed; o.interleaved = interleaved;
+    o.cos = opt(cos); o.sin = opt(sin); o.pos_q = opt(pos_q); o.pos_k = opt(pos_k);
+    return o;
+}
+
+std::tuple<Tensor, Tensor, Tensor> op_attention_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const OptTensor& cu_k,
+                                                     bool causal, double scale, int flags, double dropout_p, uint64_t seed, const OptTensor& cos,
+                                                     const OptTensor& sin, const OptTensor& pos_q, const OptTensor& pos_k, bool interleaved,
+                                                     bool return_rotated_q) {
+    check_qkv(q, k, v, cu_q, opt(cu_k));
+    Tensor q_rot;
+    if (return_rotated_q) q_rot = at::empty_strided(q.sizes(), q.strides(), q.options());
+    auto [o, lse] = attn_forward(q, k, v, cu_q, opt(cu_k), options(causal, scale, flags, dropout_p, seed, cos, sin, pos_q, pos_k, interleaved), q_rot);
+    return {o, lse, q_rot};
+}
+
+std::tuple<Tensor, Tensor, Tensor> op_attention_backward(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                                      const Tensor& lse, const Tensor& cu_q, const OptTensor& cu_k, bool causal, double scale, int flags,
+                                                      double dropout_p, uint64_t seed, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos_q,
+                                                      const OptTensor& pos_k, bool interleaved, const OptTensor& dq_, const OptTensor& dk_,
+                                                      const OptTensor& dv_, const OptTensor& ws) {
+    check_qkv(q, k, v, cu_q, opt(cu_k));
+    const Tensor dq = dq_.has_value() ? *dq_ : at::empty_strided(q.sizes(), q.strides(), q.options());
+    const Tensor dk = dk_.has_value() ? *dk_ : at::empty(k.sizes(), k.options());
+    const Tensor dv = dv_.has_value() ? *dv_ : at::empty(v.sizes(), v.options());
+    attn_backward(d_o, q, k, v, o, lse, cu_q, opt(cu_k), options(causal, scale, flags, dropout_p, seed, cos, sin, pos_q, pos_k, interleaved), dq, dk, dv, opt(ws));
+    return {dq, dk, dv};
+}
+
+// What the autograd node of the attention core keeps beside its tensors
+void keep_options(AutogradContext* ctx, const AttnOptions& o) {
+    ctx->saved_data["causal"] = o.causal;
+    ctx->saved_data["scale"] = o.scale;
+    ctx->saved_data["dropout_p"] = o.dropout_p;
+    ctx->saved_data["seed"] = (int64_t)o.seed;
+    ctx->saved_data["flags"] = (int64_t)o.flags;
+    ctx->saved_data["interleaved"] = o.interleaved;
+}
+AttnOptions kept_options(AutogradContext* ctx) {
+    AttnOptions o;
+    o.causal = ctx->saved_data["causal"].toBool();
+    o.scale = ctx->saved_data["scale"].toDouble();
+    o.dropout_p = ctx->saved_data["dropout_p"].toDouble();
+    o.seed = (uint64_t)ctx->saved_data["seed"].toInt();
+    o.flags = (int)ctx->saved_data["flags"].toInt();
+    o.interleaved = ctx->saved_data["interleaved"].toBool();
+    return o;
+}
+
+// Forward of either node; with rotary, k is rotated once by the stand-alone kernel and q while the attention kernel loads it, and
+// the rotated tensors are what the backward kernels stream, so they are kept instead of q and k.
+Tensor attention_node_forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k,
+                              const AttnOptions& opts, bool need_grad) {
+    check_qkv(q, k, v, cu_q, cu_k);
+    keep_options(ctx, opts);
+    if (!opts.cos.defined()) {
+        auto [o, lse] = attn_forward(q, k, v, cu_q, cu_k, opts, Tensor());
+        ctx->save_for_backward({q, k, v, o, lse, cu_q, cu_k, Tensor(), Tensor(), Tensor(), Tensor()});
+        return o;
+    }
+    const Tensor k_rot = rotary_launch(k, opts.cos, opts.sin, opts.pos_k, 0, false, opts.interleaved);
+    AttnOptions f = opts;
+    f.pos_k = Tensor();
+    // nothing to differentiate: the rotated q is not written out
+    const Tensor q_rot = need_grad ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
+    auto [o, lse] = attn_forward(q, k_rot, v, cu_q, cu_k, f, q_rot);
+    if (need_grad) ctx->save_for_backward({q_rot, k_rot, v, o, lse, cu_q, cu_k, opts.cos, opts.sin, opts.pos_q, opts.pos_k});
+    return o;
+}
+
+struct Attention : Function<Attention> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const OptTensor& cu_k,
+                          const AttnOptions* opts, bool need_grad) {
+        return attention_node_forward(ctx, q, k, v, cu_q, opt(cu_k), *opts, need_grad);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto s = ctx->get_saved_variables();         // read once: saved-tensor hooks unpack on access
+        AttnOptions opts = kept_options(ctx);
+        opts.cos = s[7]; opts.sin = s[8]; opts.pos_q = s[9]; opts.pos_k = s[10];
+        const Tensor &q = s[0], &k = s[1], &v = s[2];
+        const Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
+        attn_backward(g[0], q, k, v, s[3], s[4], s[5], s[6], opts, dq, dk, dv, Tensor());
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor op_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const OptTensor& cu_k, bool causal, double scale,
+                 double dropout_p, uint64_t seed, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos_q, const OptTensor& pos_k,
+                 bool interleaved, bool precise) {
+    const AttnOptions o = options(causal, scale, precise ? MI_ATTN_SPLIT_P : 0, dropout_p, seed, cos, sin, pos_q, pos_k, interleaved);
+    const bool need_grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+    return Attention::apply(q, k, v, cu_q, cu_k, &o, need_grad);
+}
+
+// ---- decode ------------------------------------------------------------------------------------------------------------
+void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, const OptTensor& k_new,
+                      const OptTensor& v_new, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos, bool interleaved, double scale,
+                      const OptTensor& workspace, int n_splits, const Tensor& out, bool static_scratch) {
+    need_gpu(q); need_gpu(k_cache); need_gpu(v_cache); need_gpu(ctx_len);
+    Launch l(q);
+    mi_decode_args a{};
+    a.q = ptr(q); a.k_cache = ptr(k_cache); a.v_cache = ptr(v_cache); a.o = ptr(out); a.ctx_len = (const int32_t*)ptr(ctx_len);
+    a.q_stride_batch = q.stride(0);
+    if (k_new.has_value()) {
+        a.k_new = ptr(*k_new); a.v_new = ptr(*v_new);
+        a.k_new_stride_batch = k_new->stride(0); a.v_new_stride_batch = v_new->stride(0);
+    }
+    if (cos.has_value()) {
+        a.rotary_cos = ptr(*cos); a.rotary_sin = ptr(*sin); a.position_ids = (const int64_t*)ptr(*pos);
+        a.rotary_table_rows = cos->size(0);
+        a.rotary_interleaved = interleaved;
+    }
+    a.batch = (int32_t)q.size(0); a.max_ctx = (int32_t)k_cache.size(1); a.n_q_heads = (int32_t)q.size(1); a.n_kv_heads = (int32_t)k_cache.size(2);
+    a.head_dim = (int32_t)q.size(2);
+    a.dtype = code_of(q);
+    a.cache_stride_batch = k_cache.stride(0); a.cache_stride_token = k_cache.stride(1); a.cache_stride_head = k_cache.stride(2);
+    a.softmax_scale = (float)scale;
+    a.n_splits = n_splits;
+    a.stream = l.stream;
+    if (static_scratch) {
+        check(mi_attn_decode_static(&a), "mi_attn_decode_static");
+        return;
+    }
+    a.workspace = ptr(*workspace);
+    a.workspace_bytes = (size_t)workspace->numel() * 4;
+    check(mi_attn_decode(&a), "mi_attn_decode");
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    // none of these touches Python objects: other interpreter threads run meanwhile
+    const auto def = [&](const char* name, auto f) { m.def(name, f, py::call_guard<py::gil_scoped_release>()); };
+    def("rms_norm_forward", &op_rms_norm_forward);
+    def("rms_norm_backward", &op_rms_norm_backward);
+    def("rms_norm", [](const Tensor& x, const Tensor& w, double eps) { return RmsNorm::apply(x, w, eps); });
+    def("layer_norm_forward", &op_layer_norm_forward);
+    def("layer_norm_backward", &op_layer_norm_backward);
+    def("layer_norm", [](const Tensor& x, const Tensor& w, const OptTensor& b, double eps) { return LayerNorm::apply(x, w, b, eps); });
+    def("gelu_forward", &op_gelu_forward);
+    def("gelu_backward", &op_gelu_backward);
+    def("gelu", [](const Tensor& x) { return Gelu::apply(x); });
+    def("swiglu_forward", &op_swiglu_forward);
+    def("swiglu_backward", &op_swiglu_backward);
+    def("swiglu", [](const Tensor& a, const Tensor& g) { return SwiGlu::apply(a, g); });
+    def("rotary_launch", &rotary_launch);
+    def("rotary", [](const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len, bool interleaved) {
+        return Rotary::apply(x, cos, sin, ids, seq_len, interleaved);
+    });
+    def("linear", &op_linear);
+    def("projections", &op_projections);
+    def("attention_forward", &op_attention_forward);
+    def("attention_backward", &op_attention_backward);
+    def("attention", &op_attention);
+    def("decode_attention", &op_decode_attention);
+}

@@ -2,8 +2,8 @@
 
 Constructor arguments, forward signatures, sub-module names and parameter names follow the
 reference's modules (see each class), so state dicts and the per-layer checkpoint files of the
-reference load unchanged.  Linear projections stay on PyTorch-ROCm matmul.  Everything else on the
-path (norm, rotary, attention core, SwiGLU) runs the HIP kernels of this package; options the kernels
+reference load unchanged.  Linear projections run on PyTorch-ROCm matmul or, where they are too small for
+it, on the matrix kernel of this package.  Everything else on the path (norm, rotary, attention core, SwiGLU) runs the HIP kernels of this package; options the kernels
 do not cover raise `NotImplementedError` instead of silently taking another path.
 """
 
@@ -11,7 +11,6 @@ import math
 from typing import Callable, Dict, Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 
 from . import ops
 from .config import (LayerNormConfig, MaskedSoftmaxConfig, MaskedSoftmaxKernel, NormType,
@@ -70,7 +69,20 @@ class _Linear(torch.nn.Module):
             self.register_parameter("bias", None)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
+
+
+def _direct(*modules: torch.nn.Module) -> bool:
+    """Whether calling the modules comes to using their weights: plain projections that nobody replaced or hooked."""
+    return all(type(m) is _Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+               for m in modules)
+
+
+def _project_together(x: torch.Tensor, *modules: torch.nn.Module):
+    """The outputs of several projections of one input."""
+    if _direct(*modules):
+        return ops.projections(x, [m.weight for m in modules], [m.bias for m in modules])
+    return [m(x) for m in modules]
 
 
 class RMSNorm(torch.nn.Module):
@@ -214,7 +226,7 @@ class ParallelSwiGLUMLP(torch.nn.Module):
         self.dense_out = _Linear(inter, io_features, bias, device, dtype, init_method)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.dense_out(ops.swiglu(self.dense_in(x), self.siglu_weight(x)))
+        return self.dense_out(ops.swiglu(*_project_together(x, self.dense_in, self.siglu_weight)))
 
 
 class ParallelMLP(torch.nn.Module):
@@ -443,13 +455,11 @@ class ParallelSelfAttention(torch.nn.Module):
             # inference (eval mode, so that a no-grad forward that activation checkpointing recomputes with grad takes
             # the same GEMMs both times): one projection GEMM over the row-stacked weights; q, k, v are column slices
             w, bias = self._fused_qkv()
-            out = F.linear(x, w, bias).view(b * s, (nq + 2 * nkv) * d)
+            out = ops.linear(x, w, bias).view(b * s, (nq + 2 * nkv) * d)
             return (out[:, :nq * d].view(b * s, nq, d), out[:, nq * d:(nq + nkv) * d].view(b * s, nkv, d),
                     out[:, (nq + nkv) * d:].view(b * s, nkv, d))
-        q = self.query(x).view(b * s, nq, d)
-        k = self.key(x).view(b * s, nkv, d)
-        v = self.value(x).view(b * s, nkv, d)
-        return q, k, v
+        q, k, v = _project_together(x, self.query, self.key, self.value)
+        return q.view(b * s, nq, d), k.view(b * s, nkv, d), v.view(b * s, nkv, d)
 
     def _fused_qkv(self):
         """The weights (and biases) of `query`, `key`, `value` as row blocks of one tensor.  Built on first use: the

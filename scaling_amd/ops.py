@@ -2,18 +2,19 @@
 
 Every function here launches a hand-written gfx950 kernel on the current stream.  None of them falls
 back to PyTorch arithmetic: tensors must live on the GPU, and shapes or dtypes a kernel does not
-support raise.  Autograd functions keep tensors with ``ctx.save_for_backward`` only, so they work
+support raise.  The checks are here; argument blocks, allocations, launches and autograd nodes are native
+(csrc/host.cpp).  The nodes keep tensors with ``save_for_backward`` only, so they work
 under saved-tensor hooks (activation checkpointing) and are deterministic under recomputation.
 """
 
-import ctypes
+import ctypes  # noqa: F401 - for callers that fill an argument block with _fill_attn_args and hand it to the C ABI
 import math
 from typing import Optional, Tuple
 
 import torch
 
 from . import _lib
-from ._lib import MiAttnArgs, MiAttnBwdArgs, MiDecodeArgs, check, dtype_code, ptr, stream_ptr
+from ._lib import MiAttnArgs, check, dtype_code, ptr, stream_ptr
 
 __all__ = [
     "rms_norm", "swiglu", "rotary_embedding", "rotary_embedding_complex", "attention", "attention_forward", "attention_backward",
@@ -47,48 +48,19 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
 def rms_norm_forward(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     _need_cuda(x, weight)
     assert x.shape[-1] == weight.shape[0] and weight.dtype == x.dtype
-    x2 = x.contiguous().view(-1, x.shape[-1])
-    w = weight.contiguous()
-    y = torch.empty_like(x2)
-    check(_lib.load().mi_rmsnorm_fwd(ptr(x2), ptr(w), ptr(y), None, x2.shape[0], x2.shape[1], float(eps),
-                                     dtype_code(x.dtype), stream_ptr()), "mi_rmsnorm_fwd")
-    return y.view(x.shape)
+    return _lib.host().rms_norm_forward(x, weight, eps)
 
 
 def rms_norm_backward(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor, eps: float):
     _need_cuda(x, weight, dy)
-    lib = _lib.load()
-    if x.numel() == 0:                   # no rows: no launch, the weight gradient is a sum over nothing
-        return torch.empty_like(x), torch.zeros_like(weight)
-    x2 = x.contiguous().view(-1, x.shape[-1])
-    dy2 = dy.contiguous().view(-1, x.shape[-1])
-    w = weight.contiguous()
-    dx = torch.empty_like(x2)
-    dw = torch.empty_like(w)
-    nbytes = lib.mi_rmsnorm_bwd_workspace_bytes(x2.shape[0], x2.shape[1])
-    ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-    check(lib.mi_rmsnorm_bwd(ptr(x2), ptr(w), ptr(dy2), ptr(dx), ptr(dw), ptr(ws), nbytes, x2.shape[0], x2.shape[1],
-                             float(eps), dtype_code(x.dtype), stream_ptr()), "mi_rmsnorm_bwd")
-    return dx.view(x.shape), dw
-
-
-class _RMSNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, eps):
-        ctx.save_for_backward(x, weight)
-        ctx.eps = eps
-        return rms_norm_forward(x, weight, eps)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, weight = ctx.saved_tensors
-        dx, dw = rms_norm_backward(x, weight, dy, ctx.eps)
-        return dx, dw, None
+    return _lib.host().rms_norm_backward(x, weight, dy, eps)
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
     """y = x * rsqrt(mean(x^2, -1) + eps) * weight (fp32 math, one rounding)."""
-    return _RMSNorm.apply(x, weight, eps)
+    _need_cuda(x, weight)
+    assert x.shape[-1] == weight.shape[0] and weight.dtype == x.dtype
+    return _lib.host().rms_norm(x, weight, eps)
 
 
 # ------------------------------------------------------------------------------------------------
@@ -100,15 +72,8 @@ def layer_norm_forward(x: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
     for layer_norm_backward when save_stats is set."""
     _need_cuda(x, weight, bias)
     assert x.shape[-1] == weight.shape[0] and weight.dtype == x.dtype
-    x2 = x.contiguous().view(-1, x.shape[-1])
-    w = weight.contiguous()
-    b = bias.contiguous() if bias is not None else None
-    y = torch.empty_like(x2)
-    stats = torch.empty(2, x2.shape[0], dtype=torch.float32, device=x.device) if save_stats else None
-    check(_lib.load().mi_layernorm_fwd(ptr(x2), ptr(w), ptr(b), ptr(y), ptr(stats[0]) if save_stats else None,
-                                       ptr(stats[1]) if save_stats else None, x2.shape[0], x2.shape[1], float(eps),
-                                       dtype_code(x.dtype), stream_ptr()), "mi_layernorm_fwd")
-    return (y.view(x.shape), stats) if save_stats else y.view(x.shape)
+    y, stats = _lib.host().layer_norm_forward(x, weight, bias, eps, save_stats)
+    return (y, stats) if save_stats else y
 
 
 def layer_norm_backward(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor, eps: float, need_bias_grad: bool = True,
@@ -116,77 +81,32 @@ def layer_norm_backward(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor,
     """(dx, dweight, dbias).  `stats` is what layer_norm_forward(save_stats=True) returned for the same x, or
     None to have the statistics recomputed."""
     _need_cuda(x, weight, dy)
-    lib = _lib.load()
-    if x.numel() == 0:                   # no rows: no launch, the parameter gradients are sums over nothing
-        return torch.empty_like(x), torch.zeros_like(weight), (torch.zeros_like(weight) if need_bias_grad else None)
-    if stats is not None:
+    if stats is not None and x.numel() != 0:
         assert stats.dtype == torch.float32 and stats.is_contiguous() and stats.shape == (2, x.numel() // x.shape[-1])
-    x2 = x.contiguous().view(-1, x.shape[-1])
-    dy2 = dy.contiguous().view(-1, x.shape[-1])
-    w = weight.contiguous()
-    dx = torch.empty_like(x2)
-    dw = torch.empty_like(w)
-    db = torch.empty_like(w) if need_bias_grad else None
-    nbytes = lib.mi_layernorm_bwd_workspace_bytes(x2.shape[0], x2.shape[1])
-    ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-    check(lib.mi_layernorm_bwd(ptr(x2), ptr(w), ptr(dy2), ptr(stats[0]) if stats is not None else None,
-                               ptr(stats[1]) if stats is not None else None, ptr(dx), ptr(dw), ptr(db), ptr(ws), nbytes,
-                               x2.shape[0], x2.shape[1], float(eps), dtype_code(x.dtype), stream_ptr()), "mi_layernorm_bwd")
-    return dx.view(x.shape), dw, db
-
-
-class _LayerNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, bias, eps):
-        y, stats = layer_norm_forward(x, weight, bias, eps, save_stats=True)
-        ctx.save_for_backward(x, weight, stats)
-        ctx.eps = eps
-        ctx.has_bias = bias is not None
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, weight, stats = ctx.saved_tensors
-        dx, dw, db = layer_norm_backward(x, weight, dy, ctx.eps, ctx.has_bias, stats)
-        return dx, dw, db, None
+    return _lib.host().layer_norm_backward(x, weight, dy, eps, need_bias_grad, stats)
 
 
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, eps: float = 1e-5) -> torch.Tensor:
     """(x - mean) * rsqrt(var + eps) * weight + bias over the last dimension (fp32 math, one rounding)."""
-    return _LayerNorm.apply(x, weight, bias, eps)
+    _need_cuda(x, weight, bias)
+    assert x.shape[-1] == weight.shape[0] and weight.dtype == x.dtype
+    return _lib.host().layer_norm(x, weight, bias, eps)
 
 
 def gelu_forward(x: torch.Tensor) -> torch.Tensor:
     _need_cuda(x)
-    x = x.contiguous()
-    y = torch.empty_like(x)
-    check(_lib.load().mi_gelu_fwd(ptr(x), ptr(y), x.numel(), dtype_code(x.dtype), stream_ptr()), "mi_gelu_fwd")
-    return y
+    return _lib.host().gelu_forward(x)
 
 
 def gelu_backward(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
     _need_cuda(x, dy)
-    x, dy = x.contiguous(), dy.contiguous()
-    dx = torch.empty_like(x)
-    check(_lib.load().mi_gelu_bwd(ptr(x), ptr(dy), ptr(dx), x.numel(), dtype_code(x.dtype), stream_ptr()), "mi_gelu_bwd")
-    return dx
-
-
-class _GELU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x):
-        ctx.save_for_backward(x)
-        return gelu_forward(x)
-
-    @staticmethod
-    def backward(ctx, dy):
-        (x,) = ctx.saved_tensors
-        return gelu_backward(x, dy)
+    return _lib.host().gelu_backward(x, dy)
 
 
 def gelu(x: torch.Tensor) -> torch.Tensor:
     """Exact (erf) GELU."""
-    return _GELU.apply(x)
+    _need_cuda(x)
+    return _lib.host().gelu(x)
 
 
 # ------------------------------------------------------------------------------------------------
@@ -195,118 +115,64 @@ def gelu(x: torch.Tensor) -> torch.Tensor:
 def swiglu_forward(a: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     _need_cuda(a, gate)
     assert a.shape == gate.shape and a.dtype == gate.dtype
-    a, gate = a.contiguous(), gate.contiguous()
-    out = torch.empty_like(a)
-    check(_lib.load().mi_swiglu_fwd(ptr(a), ptr(gate), ptr(out), a.numel(), dtype_code(a.dtype), stream_ptr()),
-          "mi_swiglu_fwd")
-    return out
+    return _lib.host().swiglu_forward(a, gate)
 
 
 def swiglu_backward(a: torch.Tensor, gate: torch.Tensor, dout: torch.Tensor):
     _need_cuda(a, gate, dout)
-    a, gate, dout = a.contiguous(), gate.contiguous(), dout.contiguous()
-    da, dg = torch.empty_like(a), torch.empty_like(gate)
-    check(_lib.load().mi_swiglu_bwd(ptr(a), ptr(gate), ptr(dout), ptr(da), ptr(dg), a.numel(), dtype_code(a.dtype),
-                                    stream_ptr()), "mi_swiglu_bwd")
-    return da, dg
-
-
-class _SwiGLU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, a, gate):
-        ctx.save_for_backward(a, gate)
-        return swiglu_forward(a, gate)
-
-    @staticmethod
-    def backward(ctx, dout):
-        a, gate = ctx.saved_tensors
-        return swiglu_backward(a, gate, dout)
+    return _lib.host().swiglu_backward(a, gate, dout)
 
 
 def swiglu(a: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """silu(a) * gate."""
-    return _SwiGLU.apply(a, gate)
+    _need_cuda(a, gate)
+    assert a.shape == gate.shape and a.dtype == gate.dtype
+    return _lib.host().swiglu(a, gate)
+
+
+# ------------------------------------------------------------------------------------------------
+# linear projections
+# ------------------------------------------------------------------------------------------------
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T + b (torch.nn.functional.linear), on the matrix kernel of this package where the product is too small to fill
+    the chip and on the library product elsewhere."""
+    return _lib.host().linear(x, weight, bias)
+
+
+def projections(x: torch.Tensor, weights, biases):
+    """[linear(x, w, b) for up to three (w, b)] of one input, whose gradient is then one sum inside the products."""
+    return _lib.host().projections(x, weights, biases)
 
 
 # ------------------------------------------------------------------------------------------------
 # rotary (stand-alone kernel)
 # ------------------------------------------------------------------------------------------------
-def _rotary_launch(x, cos, sin, position_ids, seq_len_for_null_ids, inverse, out=None):
-    """x: [tokens, heads, head_dim] view whose last dim is contiguous; cos/sin: [rows, rot_dim]."""
+def _check_rotary(x, cos, sin, position_ids):
     _need_cuda(x, cos, sin, position_ids)
     assert x.dim() == 3 and x.stride(2) == 1
     assert cos.is_contiguous() and sin.is_contiguous() and cos.shape == sin.shape and cos.dim() == 2
-    if out is None:
-        out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    if position_ids is not None:
-        position_ids = position_ids.contiguous()
-        assert position_ids.dtype == torch.int64 and position_ids.numel() == x.shape[0]
-    check(_lib.load().mi_rotary(ptr(x), ptr(out), ptr(cos), ptr(sin), ptr(position_ids), x.shape[0], x.shape[1],
-                                x.shape[2], cos.shape[1], x.stride(0), x.stride(1), out.stride(0), out.stride(1),
-                                cos.shape[0], int(seq_len_for_null_ids), int(bool(inverse)), dtype_code(x.dtype),
-                                dtype_code(cos.dtype), stream_ptr()), "mi_rotary")
-    return out
+    assert position_ids is None or (position_ids.dtype == torch.int64 and position_ids.numel() == x.shape[0])
 
 
-class _Rotary(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, cos, sin, position_ids, seq_len_for_null_ids):
-        ctx.save_for_backward(cos, sin, position_ids if position_ids is not None else torch.empty(0, device=x.device))
-        ctx.has_ids = position_ids is not None
-        ctx.seq_len = seq_len_for_null_ids
-        return _rotary_launch(x, cos, sin, position_ids, seq_len_for_null_ids, False)
-
-    @staticmethod
-    def backward(ctx, dout):
-        cos, sin, ids = ctx.saved_tensors
-        if dout.stride(-1) != 1:
-            dout = dout.contiguous()
-        dx = _rotary_launch(dout, cos, sin, ids if ctx.has_ids else None, ctx.seq_len, True)
-        return dx, None, None, None, None
+def _rotary_launch(x, cos, sin, position_ids, seq_len_for_null_ids, inverse):
+    """x: [tokens, heads, head_dim] view whose last dim is contiguous; cos/sin: [rows, rot_dim]."""
+    _check_rotary(x, cos, sin, position_ids)
+    return _lib.host().rotary_launch(x, cos, sin, position_ids, int(seq_len_for_null_ids), bool(inverse), False)
 
 
 def rotary_embedding(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                      position_ids: Optional[torch.Tensor] = None, seq_len_for_null_ids: int = 0) -> torch.Tensor:
     """Rotate-half rotary on x [tokens, heads, head_dim]; position_ids int64 [tokens] (flattened (b s))."""
-    return _Rotary.apply(x, cos, sin, position_ids, seq_len_for_null_ids)
-
-
-def _rotary_complex_launch(x, cos, sin, position_ids, seq_len_for_null_ids, inverse):
-    _need_cuda(x, cos, sin, position_ids)
-    assert x.dim() == 3 and x.stride(2) == 1
-    assert cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous()
-    assert cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] * 2 == x.shape[2]
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    if position_ids is not None:
-        position_ids = position_ids.contiguous()
-        assert position_ids.dtype == torch.int64 and position_ids.numel() == x.shape[0]
-    check(_lib.load().mi_rotary_complex(ptr(x), ptr(out), ptr(cos), ptr(sin), ptr(position_ids), x.shape[0], x.shape[1],
-                                        x.shape[2], x.stride(0), x.stride(1), out.stride(0), out.stride(1), cos.shape[0],
-                                        int(seq_len_for_null_ids), int(bool(inverse)), dtype_code(x.dtype), stream_ptr()),
-          "mi_rotary_complex")
-    return out
-
-
-class _RotaryComplex(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, cos, sin, position_ids, seq_len_for_null_ids):
-        ctx.save_for_backward(cos, sin, position_ids if position_ids is not None else torch.empty(0, device=x.device))
-        ctx.has_ids = position_ids is not None
-        ctx.seq_len = seq_len_for_null_ids
-        return _rotary_complex_launch(x, cos, sin, position_ids, seq_len_for_null_ids, False)
-
-    @staticmethod
-    def backward(ctx, dout):
-        cos, sin, ids = ctx.saved_tensors
-        if dout.stride(-1) != 1:
-            dout = dout.contiguous()
-        return _rotary_complex_launch(dout, cos, sin, ids if ctx.has_ids else None, ctx.seq_len, True), None, None, None, None
+    _check_rotary(x, cos, sin, position_ids)
+    return _lib.host().rotary(x, cos, sin, position_ids, int(seq_len_for_null_ids), False)
 
 
 def rotary_embedding_complex(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                              position_ids: Optional[torch.Tensor] = None, seq_len_for_null_ids: int = 0) -> torch.Tensor:
     """Interleaved-pair rotary on x [tokens, heads, head_dim]; cos / sin fp32 [rows, head_dim/2]."""
-    return _RotaryComplex.apply(x, cos, sin, position_ids, seq_len_for_null_ids)
+    _check_rotary(x, cos, sin, position_ids)
+    assert cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.shape[1] * 2 == x.shape[2]
+    return _lib.host().rotary(x, cos, sin, position_ids, int(seq_len_for_null_ids), True)
 
 
 # ------------------------------------------------------------------------------------------------
@@ -473,6 +339,11 @@ def _check_qkv(q, k, v, cu_q, cu_k):
         assert cu_k.dtype == torch.int32 and cu_k.is_contiguous() and cu_k.numel() == cu_q.numel()
 
 
+def _dropout_args(dropout):
+    """(p, seed as an unsigned 64-bit integer) of an optional (p, seed) pair."""
+    return (float(dropout[0]), int(dropout[1]) & 0xFFFFFFFFFFFFFFFF) if dropout is not None and dropout[0] > 0.0 else (0.0, 0)
+
+
 SPLIT_P = 4   # MI_ATTN_SPLIT_P
 
 
@@ -494,20 +365,18 @@ def attention_forward(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=True, sof
         softmax_scale = 1.0 / math.sqrt(q.shape[2])
     if precise:
         flags |= SPLIT_P
-    q_rot = None
+    cos = sin = pos_q = pos_k = None
+    interleaved = False
     if rotary is not None:
         cos, sin, pos_q, pos_k = rotary
-        _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
+        interleaved = _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
         assert pos_q.dtype == torch.int64 and pos_q.is_contiguous() and pos_q.numel() == q.shape[0]
         assert pos_k is None or (pos_k.dtype == torch.int64 and pos_k.is_contiguous() and pos_k.numel() == k.shape[0])
-        if return_rotated_q:
-            q_rot = torch.empty_strided(q.shape, q.stride(), dtype=q.dtype, device=q.device)
     else:
         assert not return_rotated_q
-    o = torch.empty((q.shape[0], q.shape[1], q.shape[2]), dtype=q.dtype, device=q.device)
-    lse = torch.empty((q.shape[1], q.shape[0]), dtype=torch.float32, device=q.device)
-    a = _fill_attn_args(q, k, v, o, lse, cu_seqlens_q, cu_seqlens_k, causal, softmax_scale, rotary, flags, dropout, q_rot)
-    check(_lib.load().mi_attn_fwd(ctypes.byref(a)), "mi_attn_fwd")
+    p, seed = _dropout_args(dropout)
+    o, lse, q_rot = _lib.host().attention_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, bool(causal), float(softmax_scale), int(flags), p, seed,
+                                                  cos, sin, pos_q, pos_k, interleaved, bool(return_rotated_q))
     return (o, lse, q_rot) if return_rotated_q else (o, lse)
 
 
@@ -523,66 +392,20 @@ def attention_backward(do, q, k, v, o, lse, cu_seqlens_q, cu_seqlens_k=None, cau
     buffers: optional (dq, dk, dv, workspace) to reuse across calls.
     precise: accuracy mode (P and dS enter their MFMAs as two bf16 terms each; no dropout)."""
     _check_qkv(q, k, v, cu_seqlens_q, cu_seqlens_k)
-    lib = _lib.load()
     if precise:
         flags |= SPLIT_P
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(q.shape[2])
-    if do.stride() != o.stride():
-        do = do.contiguous()
-        assert do.stride() == o.stride()
-    if buffers is not None:
-        dq, dk, dv, ws = buffers
-        assert dq.stride() == q.stride()
-    else:
-        dq = torch.empty_like(q)
-        if dq.stride() != q.stride():
-            dq = torch.empty_strided(q.shape, q.stride(), dtype=q.dtype, device=q.device)
-        dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
-        dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
-        nbytes = lib.mi_attn_bwd_workspace_bytes_kv(q.shape[0], k.shape[0], q.shape[1], k.shape[1], q.shape[2])
-        ws = torch.empty(max(nbytes // 4, 4), dtype=torch.float32, device=q.device)
-    b = MiAttnBwdArgs()
-    b.fwd = _fill_attn_args(q, k, v, o, lse, cu_seqlens_q, cu_seqlens_k, causal, softmax_scale, rotary, flags, dropout)
-    b.d_o, b.dq, b.dk, b.dv = ptr(do), ptr(dq), ptr(dk), ptr(dv)
-    b.dk_stride_token, b.dk_stride_head = dk.stride(0), dk.stride(1)
-    b.dv_stride_token, b.dv_stride_head = dv.stride(0), dv.stride(1)
-    b.workspace, b.workspace_bytes = ptr(ws), ws.numel() * 4
-    check(lib.mi_attn_bwd(ctypes.byref(b)), "mi_attn_bwd")
-    return dq, dk, dv
-
-
-class _Attention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, cu_q, cu_k, causal, scale, dropout_p, dropout_seed, cos, sin, pos_q, pos_k, precise):
-        dropout = (dropout_p, dropout_seed) if dropout_p > 0.0 else None
-        ctx.precise = precise
-        if cos is None:
-            o, lse = attention_forward(q, k, v, cu_q, cu_k, causal, scale, dropout=dropout, precise=precise)
-            ctx.save_for_backward(q, k, v, o, lse, cu_q, cu_k if cu_k is not None else cu_q)
-        else:
-            # rotary: k is rotated once by the stand-alone kernel, q while the attention kernel loads it; the rotated
-            # tensors are what the backward kernels stream, so they are kept instead of q and k
-            interleaved = _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
-            k_rot = (_rotary_complex_launch if interleaved else _rotary_launch)(k, cos, sin, pos_k, 0, False)
-            if any(ctx.needs_input_grad[:3]):
-                o, lse, q_rot = attention_forward(q, k_rot, v, cu_q, cu_k, causal, scale, rotary=(cos, sin, pos_q, None),
-                                                  dropout=dropout, return_rotated_q=True, precise=precise)
-                ctx.save_for_backward(q_rot, k_rot, v, o, lse, cu_q, cu_k if cu_k is not None else cu_q, cos, sin, pos_q, pos_k)
-            else:   # nothing to differentiate: the rotated q is not written out
-                o, lse = attention_forward(q, k_rot, v, cu_q, cu_k, causal, scale, rotary=(cos, sin, pos_q, None), dropout=dropout,
-                                           precise=precise)
-        ctx.causal, ctx.scale, ctx.dropout, ctx.rotary = causal, scale, dropout, cos is not None
-        return o
-
-    @staticmethod
-    def backward(ctx, do):
-        saved = ctx.saved_tensors           # read once: saved-tensor hooks (activation checkpointing) unpack on access
-        q, k, v, o, lse, cu_q, cu_k = saved[:7]
-        rotary = tuple(saved[7:11]) if ctx.rotary else None
-        dq, dk, dv = attention_backward(do, q, k, v, o, lse, cu_q, cu_k, ctx.causal, ctx.scale, dropout=ctx.dropout, rotary=rotary,
-                                        precise=ctx.precise)
-        return (dq, dk, dv) + (None,) * 11
+    dq, dk, dv, ws = buffers if buffers is not None else (None, None, None, None)
+    assert dq is None or dq.stride() == q.stride()
+    cos = sin = pos_q = pos_k = None
+    interleaved = False
+    if rotary is not None:
+        cos, sin, pos_q, pos_k = rotary
+        interleaved = _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
+    p, seed = _dropout_args(dropout)
+    return _lib.host().attention_backward(do, q, k, v, o, lse, cu_seqlens_q, cu_seqlens_k, bool(causal), float(softmax_scale), int(flags), p, seed,
+                                          cos, sin, pos_q, pos_k, interleaved, dq, dk, dv, ws)
 
 
 def next_dropout_seed(device: torch.device) -> int:
@@ -631,13 +454,16 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q: t
         rot = rotary_embedding_complex if cos.shape[1] * 2 == q.shape[2] else rotary_embedding
         q, k = rot(q, cos, sin, pos_q), rot(k, cos, sin, pos_k)
         rotary = cos = sin = pos_q = pos_k = None
+    _check_qkv(q, k, v, cu_seqlens_q, cu_seqlens_k)
+    interleaved = False
     if rotary is not None:
         cos, sin, pos_q, pos_k = rotary
-        _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
+        interleaved = _fused_rotary_kind(cos, sin, q.shape[2], q.dtype)
         assert pos_q.dtype == torch.int64 and pos_q.is_contiguous() and pos_q.numel() == q.shape[0]
         assert pos_k.dtype == torch.int64 and pos_k.is_contiguous() and pos_k.numel() == k.shape[0]
-    return _Attention.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, causal, float(softmax_scale), float(dropout_p),
-                            int(dropout_seed) if dropout_seed is not None else 0, cos, sin, pos_q, pos_k, bool(precise))
+    p, seed = _dropout_args((dropout_p, dropout_seed if dropout_seed is not None else 0))
+    return _lib.host().attention(q, k, v, cu_seqlens_q, cu_seqlens_k, bool(causal), float(softmax_scale), p, seed, cos, sin, pos_q, pos_k,
+                                 interleaved, bool(precise))
 
 
 # ------------------------------------------------------------------------------------------------
@@ -663,9 +489,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     _need_cuda(q, k_cache, v_cache, ctx_len)
     B, nq, d = q.shape
 
-    def _rows(t):
+    def _check_rows(t):
         assert t.stride(2) == 1 and t.stride(1) == d and t.stride(0) % 8 == 0, "each sequence's [heads, d] block must be contiguous"
-        return t.stride(0)
 
     assert k_cache.dim() == 4 and k_cache.shape == v_cache.shape
     assert k_cache.stride() == v_cache.stride() and k_cache.stride(3) == 1
@@ -676,28 +501,17 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         workspace = decode_workspace(B, nq, d, k_cache.shape[1], q.device)
     if out is None:
         out = torch.empty((B, nq, d), dtype=q.dtype, device=q.device)
-    a = MiDecodeArgs()
-    a.q, a.k_cache, a.v_cache, a.o, a.ctx_len = ptr(q), ptr(k_cache), ptr(v_cache), ptr(out), ptr(ctx_len)
-    a.q_stride_batch = _rows(q)
+    _check_rows(q)
     if k_new is not None:
         assert k_new.shape == (B, k_cache.shape[2], d) and v_new.shape == k_new.shape
-        a.k_new, a.v_new = ptr(k_new), ptr(v_new)
-        a.k_new_stride_batch, a.v_new_stride_batch = _rows(k_new), _rows(v_new)
+        _check_rows(k_new)
+        _check_rows(v_new)
+    cos = sin = pos = None
+    interleaved = False
     if rotary is not None:
         cos, sin, pos = rotary
-        a.rotary_interleaved = int(_fused_rotary_kind(cos, sin, d, q.dtype))
+        interleaved = _fused_rotary_kind(cos, sin, d, q.dtype)
         assert pos.dtype == torch.int64 and pos.numel() == B and pos.is_contiguous()
-        a.rotary_cos, a.rotary_sin, a.position_ids = ptr(cos), ptr(sin), ptr(pos)
-        a.rotary_table_rows = cos.shape[0]
-    a.batch, a.max_ctx, a.n_q_heads, a.n_kv_heads, a.head_dim = B, k_cache.shape[1], nq, k_cache.shape[2], d
-    a.dtype = dtype_code(q.dtype)
-    a.cache_stride_batch, a.cache_stride_token, a.cache_stride_head = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.softmax_scale = float(softmax_scale)
-    a.n_splits = int(n_splits)
-    a.stream = stream_ptr()
-    if static_scratch:
-        check(_lib.load().mi_attn_decode_static(ctypes.byref(a)), "mi_attn_decode_static")
-        return out
-    a.workspace, a.workspace_bytes = ptr(workspace), workspace.numel() * 4
-    check(_lib.load().mi_attn_decode(ctypes.byref(a)), "mi_attn_decode")
+    _lib.host().decode_attention(q, k_cache, v_cache, ctx_len, k_new, v_new, cos, sin, pos, interleaved, float(softmax_scale),
+                                 None if static_scratch else workspace, int(n_splits), out, bool(static_scratch))
     return out

@@ -1,0 +1,71 @@
+"""The matrix kernel of small projections (mi_gemm through ops.linear / ops.projections): forward products, input, weight and
+bias gradients against float64 products of the same rounded operands."""
+
+import pytest
+import torch
+
+from scaling_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# unit roundoff: half an ulp over the smallest value of a binade, 2^-p for a significand of p bits (8, 11 and 24)
+HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _close(name, got, ref, magnitude, k, dtype):
+    """One rounding of the result (half an ulp of its value, or of the smallest normal number) and k fp32 additions, each off
+    by at most 2^-24 of the running sum of magnitudes."""
+    tiny = 2.0 ** -25 if dtype == torch.float16 else 2.0 ** -133
+    bound = HALF_ULP[dtype] * ref.abs() + (k + 1) * 2.0 ** -24 * magnitude + tiny
+    err = (got.double().cpu() - ref).abs()
+    assert bool((err <= bound * 1.001).all()), f"{name}: {float((err / bound).max()):.2f} x the bound"
+
+
+def _case(rows, ins, outs, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, ins, generator=g).to(dtype)
+    ws = [(torch.randn(o, ins, generator=g) * 0.1).to(dtype) for o in outs]
+    bs = [torch.randn(o, generator=g).to(dtype) if i != 1 else None for i, o in enumerate(outs)]
+    dys = [torch.randn(rows, o, generator=g).to(dtype) for o in outs]
+    return x, ws, bs, dys
+
+
+# rows around the 32- and 64-row blocks, contractions of less than a step, of several prefetch rounds and with a remainder; the
+# wide ones have a 64 x 64 block per compute unit (256) and take that tiling
+@pytest.mark.parametrize("rows,ins,outs", [
+    (1, 8, (8,)), (3, 264, (40, 8, 16)), (33, 72, (64, 24)), (65, 520, (136,)), (127, 256, (264, 64, 64)),
+    (1030, 136, (1048,)), (520, 1032, (1096, 1032)),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_projections_and_their_gradients(rows, ins, outs, dtype):
+    print(f"case gemm rows={rows} in={ins} out={outs} dtype={dtype}", flush=True)
+    x, ws, bs, dys = _case(rows, ins, outs, dtype, rows + ins)
+    xg = x.to(DEV).requires_grad_()
+    wg = [w.to(DEV).requires_grad_() for w in ws]
+    bg = [b.to(DEV).requires_grad_() if b is not None else None for b in bs]
+    ys = ops.projections(xg, wg, bg)
+    torch.autograd.backward(ys, [d.to(DEV) for d in dys])
+    torch.cuda.synchronize()
+    xd, wd, dyd = x.double(), [w.double() for w in ws], [d.double() for d in dys]
+    for i in range(len(outs)):
+        b = bs[i].double() if bs[i] is not None else torch.zeros(outs[i], dtype=torch.float64)
+        _close(f"y{i}", ys[i].detach(), xd @ wd[i].t() + b, xd.abs() @ wd[i].abs().t() + b.abs(), ins, dtype)
+        _close(f"dw{i}", wg[i].grad, dyd[i].t() @ xd, dyd[i].abs().t() @ xd.abs(), rows, dtype)
+        if bs[i] is not None:
+            _close(f"db{i}", bg[i].grad, dyd[i].sum(0), dyd[i].abs().sum(0), rows, dtype)
+    _close("dx", xg.grad, sum(d @ w for d, w in zip(dyd, wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd, wd)), sum(outs), dtype)
+
+
+def test_projection_that_does_not_reach_the_loss():
+    """Only the used outputs contribute; frozen weights get no gradient; an odd width runs on the library product."""
+    x, ws, bs, dys = _case(40, 64, (32, 48, 16), torch.float32, 5)
+    xg, wg = x.to(DEV).requires_grad_(), [w.to(DEV) for w in ws]
+    wg[2].requires_grad_()
+    ys = ops.projections(xg, wg, [None, None, None])
+    ys[2].backward(dys[2].to(DEV))
+    assert wg[0].grad is None and wg[1].grad is None
+    _close("dx", xg.grad, dys[2].double() @ ws[2].double(), dys[2].double().abs() @ ws[2].double().abs(), 16, torch.float32)
+    _close("dw", wg[2].grad, dys[2].double().t() @ x.double(), dys[2].double().abs().t() @ x.double().abs(), 40, torch.float32)
+    odd = torch.randn(7, 64)
+    _close("odd", ops.linear(xg.detach(), odd.to(DEV)), x.double() @ odd.double().t(), x.double().abs() @ odd.double().abs().t(), 64, torch.float32)
+    assert ops.linear(torch.empty(0, 64, device=DEV), wg[0]).shape == (0, 32)
