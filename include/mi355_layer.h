@@ -82,6 +82,10 @@ typedef struct mi_gemm_problem {
 } mi_gemm_problem;
 int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream);
 
+/* out[c] = sum_r x[r * row_stride + c], fp32 accumulation, fixed order: the bias gradient of a projection.  n_cols and
+ * row_stride multiples of 8 elements (4 for fp32), x 16-byte aligned. */
+int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * RMSNorm.  Replaces core/nn/norm/rms_norm.py:47-50:  y = x * rsqrt(mean(x^2, -1) + eps) * weight.
  * Arithmetic in fp32, one rounding to `dtype` on store.  x, y: [n_rows, hidden]; weight: [hidden].
@@ -94,11 +98,11 @@ int mi_rmsnorm_fwd(const void* x, const void* weight, void* y, float* rstd,
 /* Residual add fused into the norm that follows it (transformer/model/layers/layer.py:252-293 with
  * core/nn/residual.py:49-65 at inference): sum_out = x + residual rounded to `dtype`, y = rmsnorm(sum_out) * weight
  * exactly as mi_rmsnorm_fwd computes it from the stored sum.  sum_out may alias x or residual; y may not alias.
- * Forward only.  Algorithmic HBM bytes: 4 * n_rows * hidden * e. */
+ * Algorithmic HBM bytes: 4 * n_rows * hidden * e. */
 int mi_add_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* sum_out, void* y,
                        int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
 
-/* Backward of the above (what autograd derives from rms_norm.py:47-50):
+/* Backward of mi_rmsnorm_fwd (what autograd derives from rms_norm.py:47-50):
  *   dx = rstd * (dy*w) - x * rstd^3 * mean(dy*w*x),   dweight = sum_rows dy * x * rstd.
  * rstd is recomputed from x.  `workspace` holds per-block fp32 partial sums of dweight and must be
  * at least mi_rmsnorm_bwd_workspace_bytes(n_rows, hidden) bytes; the partials are reduced in a
@@ -107,6 +111,12 @@ size_t mi_rmsnorm_bwd_workspace_bytes(int64_t n_rows, int64_t hidden);
 int mi_rmsnorm_bwd(const void* x, const void* weight, const void* dy, void* dx, void* dweight,
                    void* workspace, size_t workspace_bytes,
                    int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
+/* Backward of mi_add_rmsnorm_fwd with respect to the sum (x here is sum_out): as mi_rmsnorm_bwd, plus `dsum` (may be NULL),
+ * the gradient that reaches sum_out directly (the residual stream), added to the rounded result.  The gradients of both
+ * addends are dx. */
+int mi_add_rmsnorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, void* dx, void* dweight,
+                       void* workspace, size_t workspace_bytes,
+                       int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * LayerNorm.  Replaces core/nn/norm/layernorm.py:75-86 (torch.nn.functional.layer_norm over the last
@@ -125,6 +135,14 @@ size_t mi_layernorm_bwd_workspace_bytes(int64_t n_rows, int64_t hidden);
 int mi_layernorm_bwd(const void* x, const void* weight, const void* dy, const float* mean, const float* rstd,
                      void* dx, void* dweight, void* dbias, void* workspace, size_t workspace_bytes,
                      int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
+
+/* The same with the residual add in front, as mi_add_rmsnorm_fwd / mi_add_rmsnorm_bwd (mean and rstd are required with
+ * dsum). */
+int mi_add_layernorm_fwd(const void* x, const void* residual, const void* weight, const void* bias, void* sum_out, void* y,
+                         float* mean, float* rstd, int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
+int mi_add_layernorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, const float* mean, const float* rstd,
+                         void* dx, void* dweight, void* dbias, void* workspace, size_t workspace_bytes,
+                         int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * GELU activation of the default MLP.  Replaces core/nn/mlp.py:135-139 with

@@ -25,7 +25,7 @@ EXPORTS = (
     "mi_layernorm_fwd", "mi_layernorm_bwd_workspace_bytes", "mi_layernorm_bwd", "mi_gelu_fwd", "mi_gelu_bwd", "mi_cross_entropy",
     "mi_swiglu_fwd", "mi_swiglu_bwd", "mi_rotary", "mi_rotary_complex",
     "mi_attn_fwd", "mi_attn_bwd_workspace_bytes", "mi_attn_bwd_workspace_bytes_kv", "mi_attn_bwd",
-    "mi_gemm", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
+    "mi_gemm", "mi_column_sum", "mi_add_rmsnorm_bwd", "mi_add_layernorm_fwd", "mi_add_layernorm_bwd", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
 )
 
 
@@ -137,6 +137,15 @@ def _declare(lib):
                                       c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_void_p]
     lib.mi_gemm.restype = c_int
     lib.mi_gemm.argtypes = [POINTER(MiGemmProblem), c_int, c_int, c_void_p]
+    lib.mi_column_sum.restype = c_int
+    lib.mi_column_sum.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p]
+    lib.mi_add_rmsnorm_bwd.restype = c_int
+    lib.mi_add_rmsnorm_bwd.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_int64,
+                                       c_int64, c_float, c_int, c_void_p]
+    lib.mi_add_layernorm_fwd.restype = c_int
+    lib.mi_add_layernorm_fwd.argtypes = [c_void_p] * 8 + [c_int64, c_int64, c_float, c_int, c_void_p]
+    lib.mi_add_layernorm_bwd.restype = c_int
+    lib.mi_add_layernorm_bwd.argtypes = [c_void_p] * 10 + [c_size_t, c_int64, c_int64, c_float, c_int, c_void_p]
     lib.mi_attn_fwd.restype = c_int
     lib.mi_attn_fwd.argtypes = [POINTER(MiAttnArgs)]
     lib.mi_attn_bwd_workspace_bytes.restype = c_size_t

@@ -145,6 +145,83 @@ struct LayerNorm : Function<LayerNorm> {
     }
 };
 
+// A norm together with the residual stream it branches off: sum = x + residual (x itself without a residual), y = norm(sum).  Both
+// outputs are differentiable; the gradient that reaches `sum` directly is added inside the norm's backward kernel.
+struct AddNorm : Function<AddNorm> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x_, const OptTensor& residual_, const Tensor& w_, const OptTensor& b_, double eps,
+                                 bool layer_norm) {
+        need_gpu(x_);
+        TORCH_CHECK(x_.scalar_type() == w_.scalar_type() && x_.dim() >= 1 && x_.size(-1) == w_.size(0), "norm: x and weight do not match");
+        TORCH_CHECK(!residual_.has_value() || (residual_->sizes() == x_.sizes() && residual_->scalar_type() == x_.scalar_type()),
+                    "norm: x and residual do not match");
+        Launch l(x_);
+        const Tensor x = x_.contiguous(), w = w_.contiguous(), b = b_.has_value() ? b_->contiguous() : Tensor();
+        const Tensor residual = residual_.has_value() ? residual_->contiguous() : Tensor();
+        const int64_t rows = row_count(x), hidden = x.size(-1);
+        const Tensor sum = residual.defined() ? at::empty_like(x) : x_;
+        Tensor y = at::empty_like(x), stats;
+        if (layer_norm) {
+            stats = at::empty({2, rows}, x.options().dtype(at::kFloat));
+            float *mean = stats.data_ptr<float>(), *rstd = mean + rows;
+            if (residual.defined())
+                check(mi_add_layernorm_fwd(ptr(x), ptr(residual), ptr(w), ptr(b), ptr(sum), ptr(y), mean, rstd, rows, hidden, (float)eps, code_of(x), l.stream),
+                      "mi_add_layernorm_fwd");
+            else
+                check(mi_layernorm_fwd(ptr(x), ptr(w), ptr(b), ptr(y), mean, rstd, rows, hidden, (float)eps, code_of(x), l.stream), "mi_layernorm_fwd");
+        } else if (residual.defined()) {
+            check(mi_add_rmsnorm_fwd(ptr(x), ptr(residual), ptr(w), ptr(sum), ptr(y), rows, hidden, (float)eps, code_of(x), l.stream), "mi_add_rmsnorm_fwd");
+        } else {
+            check(mi_rmsnorm_fwd(ptr(x), ptr(w), ptr(y), nullptr, rows, hidden, (float)eps, code_of(x), l.stream), "mi_rmsnorm_fwd");
+        }
+        ctx->save_for_backward({sum, w_, stats});
+        ctx->saved_data["eps"] = eps;
+        ctx->saved_data["layer_norm"] = layer_norm;
+        ctx->saved_data["residual"] = residual.defined();
+        ctx->saved_data["bias"] = b.defined();
+        return {sum, y};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const bool layer_norm = ctx->saved_data["layer_norm"].toBool(), bias = ctx->saved_data["bias"].toBool();
+        const Tensor& dsum_ = g[0];
+        Tensor dx, dw, db;
+        if (!g[1].defined()) {                             // the norm does not reach the loss
+            dx = dsum_;
+        } else if (saved[0].numel() == 0) {
+            dx = at::empty_like(saved[0]);
+            dw = at::zeros_like(saved[1]);
+            if (bias) db = at::zeros_like(saved[1]);
+        } else {
+            Launch l(saved[0]);
+            const Tensor x = saved[0].contiguous(), w = saved[1].contiguous(), dy = g[1].contiguous(), dsum = dsum_.defined() ? dsum_.contiguous() : Tensor();
+            const int64_t rows = row_count(x), hidden = x.size(-1);
+            const float eps = (float)ctx->saved_data["eps"].toDouble();
+            dx = at::empty_like(x);
+            dw = at::empty_like(w);
+            if (layer_norm) {
+                const float* mean = saved[2].data_ptr<float>();
+                if (bias) db = at::empty_like(w);
+                const size_t bytes = mi_layernorm_bwd_workspace_bytes(rows, hidden);
+                Tensor ws = float_buffer(bytes, x);
+                check(mi_add_layernorm_bwd(ptr(x), ptr(w), ptr(dy), ptr(dsum), mean, mean + rows, ptr(dx), ptr(dw), ptr(db), ptr(ws), bytes, rows, hidden, eps,
+                                           code_of(x), l.stream),
+                      "mi_add_layernorm_bwd");
+            } else {
+                const size_t bytes = mi_rmsnorm_bwd_workspace_bytes(rows, hidden);
+                Tensor ws = float_buffer(bytes, x);
+                check(mi_add_rmsnorm_bwd(ptr(x), ptr(w), ptr(dy), ptr(dsum), ptr(dx), ptr(dw), ptr(ws), bytes, rows, hidden, eps, code_of(x), l.stream),
+                      "mi_add_rmsnorm_bwd");
+            }
+        }
+        return {dx, ctx->saved_data["residual"].toBool() ? dx : Tensor(), dw, db, Tensor(), Tensor()};
+    }
+};
+
+std::tuple<Tensor, Tensor> op_add_norm(const Tensor& x, const OptTensor& residual, const Tensor& w, const OptTensor& b, double eps, bool layer_norm) {
+    const auto out = AddNorm::apply(x, residual, w, b, eps, layer_norm);
+    return {out[0], out[1]};
+}
+
 // ---- activations -------------------------------------------------------------------------------------------------------
 Tensor op_gelu_forward(const Tensor& x_) {
     need_gpu(x_);
@@ -270,6 +347,16 @@ mi_gemm_problem problem(const Tensor& c, bool p_kmajor, bool q_kmajor) {
     return pr;
 }
 
+Tensor bias_gradient(const Tensor& dy) {
+    if (!aligned(dy) || dy.size(0) == 0) return dy.sum(0);
+    const int64_t v = dy.scalar_type() == at::kFloat ? 4 : 8;
+    if (dy.size(1) % v != 0) return dy.sum(0);
+    Launch l(dy);
+    Tensor db = at::empty({dy.size(1)}, dy.options());
+    check(mi_column_sum(ptr(dy), dy.stride(0), dy.size(0), dy.size(1), ptr(db), code_of(dy), l.stream), "mi_column_sum");
+    return db;
+}
+
 // Several projections of one input: y_i = x W_i^T + b_i.  Their input gradient is one sum, their forward products and (for small
 // problems) all their gradients are one launch each.
 struct Projections : Function<Projections> {
@@ -282,7 +369,8 @@ struct Projections : Function<Projections> {
             if (has_bias[i]) at[i] = next++;
         return at;
     }
-    static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, const std::vector<int64_t>& has_bias) {
+    // residual (one projection only): added to the output
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, const OptTensor& residual, const std::vector<int64_t>& has_bias) {
         const int64_t n = (int64_t)has_bias.size(), in = x.size(-1);
         const auto at = bias_at(has_bias);
         const Tensor x2 = x.reshape({-1, in});
@@ -306,6 +394,12 @@ struct Projections : Function<Projections> {
                 segment(pr[i], x2, params[i], in);
                 if (at[i] >= 0) pr[i].bias = ptr(params[at[i]]);
             }
+            Tensor add;
+            if (residual.has_value()) {
+                add = residual->contiguous();
+                pr[0].add = ptr(add);
+                pr[0].ldadd = pr[0].n;
+            }
             check(mi_gemm(pr, (int)n, code_of(x), l.stream), "mi_gemm");
         } else {
             for (int64_t i = 0; i < n; ++i) {
@@ -313,9 +407,11 @@ struct Projections : Function<Projections> {
                 const Tensor wt = params[i].t();
                 out.push_back((at[i] >= 0 ? at::addmm(params[at[i]], x2, wt) : at::mm(x2, wt)).view(shape));
             }
+            if (residual.has_value()) out[0].add_(*residual);
         }
         ctx->save_for_backward(saved);
         ctx->saved_data["x_shape"] = x.sizes().vec();
+        ctx->saved_data["residual"] = residual.has_value();
         ctx->saved_data["has_bias"] = has_bias;
         return out;
     }
@@ -370,13 +466,15 @@ struct Projections : Function<Projections> {
                     else dx = at::mm(dy[i], w);
                 }
                 if (need_weight(i)) dw[i] = at::mm(dy[i].t(), x);
-                if (need_bias(i)) db[i] = dy[i].sum(0);
+                if (need_bias(i)) db[i] = bias_gradient(dy[i]);
             }
         }
         variable_list grads{dx.defined() ? dx.view(ctx->saved_data["x_shape"].toIntVector()) : Tensor()};
         for (int64_t i = 0; i < n; ++i) grads.push_back(need_weight(i) ? dw[i] : Tensor());
         for (int64_t i = 0; i < n; ++i)
             if (at[i] >= 0) grads.push_back(db[i]);
+        grads.push_back(g[0]);                             // residual (ignored without one)
+        if (!ctx->saved_data["residual"].toBool()) grads.back() = Tensor();
         grads.emplace_back();                              // has_bias
         return grads;
     }
@@ -403,10 +501,21 @@ std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& w
         has_bias.push_back(b.has_value());
         if (b.has_value()) params.push_back(*b);
     }
-    return Projections::apply(x, at::TensorList(params), has_bias);
+    return Projections::apply(x, at::TensorList(params), OptTensor(), has_bias);
 }
 
-Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b) { return op_projections(x, {w}, {b})[0]; }
+Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b, const OptTensor& residual) {
+    if (plain_linear(x, w)) {
+        const Tensor y = at::linear(x, w, b);
+        return residual.has_value() ? y + *residual : y;
+    }
+    variable_list params{w};
+    if (b.has_value()) params.push_back(*b);
+    OptTensor add = residual;
+    if (add.has_value() && (add->scalar_type() != x.scalar_type() || add->dim() != x.dim() || add->size(-1) != w.size(0) || add->numel() / w.size(0) != x.numel() / w.size(1)))
+        return Projections::apply(x, at::TensorList(params), OptTensor(), std::vector<int64_t>{b.has_value()})[0] + *residual;
+    return Projections::apply(x, at::TensorList(params), add, std::vector<int64_t>{b.has_value()})[0];
+}
 
 // ---- attention core ----------------------------------------------------------------------------------------------------
 struct AttnOptions {
@@ -582,6 +691,33 @@ Tensor op_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Ten
     return Attention::apply(q, k, v, cu_q, cu_k, &o, need_grad);
 }
 
+// The same on one projection output qkv [tokens, heads, 3 d] (per head q, then k, then v): the gradient is written into one tensor of
+// that layout by the kernels themselves.  (As three slices of qkv, each gradient would be padded with zeros to the
+// size of qkv and the three summed: eight passes over a tensor of that size.)
+struct AttentionQkv : Function<AttentionQkv> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cu_q, const OptTensor& cu_k, const AttnOptions* opts, bool need_grad) {
+        const int64_t d = qkv.size(2) / 3;
+        return attention_node_forward(ctx, qkv.narrow(2, 0, d), qkv.narrow(2, d, d), qkv.narrow(2, 2 * d, d), cu_q, opt(cu_k), *opts, need_grad);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto s = ctx->get_saved_variables();
+        AttnOptions opts = kept_options(ctx);
+        opts.cos = s[7]; opts.sin = s[8]; opts.pos_q = s[9]; opts.pos_k = s[10];
+        const Tensor& q = s[0];
+        const int64_t d = q.size(2);
+        const Tensor dqkv = at::empty({q.size(0), q.size(1), 3 * d}, q.options());
+        attn_backward(g[0], q, s[1], s[2], s[3], s[4], s[5], s[6], opts, dqkv.narrow(2, 0, d), dqkv.narrow(2, d, d), dqkv.narrow(2, 2 * d, d), Tensor());
+        return {dqkv, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor op_attention_qkv(const Tensor& qkv, const Tensor& cu_q, const OptTensor& cu_k, bool causal, double scale, double dropout_p, uint64_t seed,
+                        const OptTensor& cos, const OptTensor& sin, const OptTensor& pos_q, const OptTensor& pos_k, bool interleaved) {
+    TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && qkv.size(2) % 3 == 0, "qkv must be contiguous [tokens, heads, 3 head_dim]");
+    const AttnOptions o = options(causal, scale, 0, dropout_p, seed, cos, sin, pos_q, pos_k, interleaved);
+    return AttentionQkv::apply(qkv, cu_q, cu_k, &o, at::GradMode::is_enabled() && qkv.requires_grad());
+}
+
 // ---- decode ------------------------------------------------------------------------------------------------------------
 void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, const OptTensor& k_new,
                       const OptTensor& v_new, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos, bool interleaved, double scale,
@@ -642,5 +778,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("attention_forward", &op_attention_forward);
     def("attention_backward", &op_attention_backward);
     def("attention", &op_attention);
+    def("attention_qkv", &op_attention_qkv);
+    def("add_norm", &op_add_norm);
     def("decode_attention", &op_decode_attention);
 }

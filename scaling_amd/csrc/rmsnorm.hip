@@ -12,6 +12,8 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kMaxBwdBlocks = 512;
 
+template <typename T> __device__ __forceinline__ float round_to(float v) { return (float)(T)v; }
+
 template <int TPR> __device__ __forceinline__ float row_sum(float v, float* lds) {
     if constexpr (TPR <= 64) {
         return group_sum<TPR>(v);
@@ -86,9 +88,12 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_fwd_kernel(const T* __restrict
     }
 }
 
+// dres (nullable, here and in the other backward kernels): gradient that reaches the normalised row past the norm (the
+// residual stream).  It is added to the rounded dx, as a separate sum of the two gradients would, without that sum's three passes
+// over memory.
 template <typename T, int TPR, int CH>
 __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                              const T* __restrict__ dy, T* __restrict__ dx,
+                                                              const T* __restrict__ dy, const T* __restrict__ dres, T* __restrict__ dx,
                                                               float* __restrict__ dw_partial, int64_t n_rows,
                                                               int hidden, float eps) {
     constexpr int V = Elem<T>::kVec;
@@ -120,13 +125,14 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
         const bool row_ok = row < n_rows;
         const uint4* xr = reinterpret_cast<const uint4*>(x + (row_ok ? row : 0) * hidden);
         const uint4* gr = reinterpret_cast<const uint4*>(dy + (row_ok ? row : 0) * hidden);
-        uint4 xraw[CH], graw[CH];
+        uint4 xraw[CH], graw[CH], rraw[CH];
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const int v = c * TPR + tr;
             const bool ok = row_ok && v < vecs;
             xraw[c] = ok ? xr[v] : make_uint4(0, 0, 0, 0);
             graw[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
+            rraw[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
         }
         float ss = 0.f, dot = 0.f;
 #pragma unroll
@@ -150,12 +156,13 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
             for (int c = 0; c < CH; ++c) {
                 const int v = c * TPR + tr;
                 if (v < vecs) {
-                    float xf[V], gf[V], o[V];
+                    float xf[V], gf[V], o[V], rf[V];
                     Elem<T>::unpack(xraw[c], xf);
                     Elem<T>::unpack(graw[c], gf);
+                    Elem<T>::unpack(rraw[c], rf);
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
-                        o[i] = rstd * (gf[i] * wf[c][i]) - xf[i] * coef;
+                        o[i] = round_to<T>(rstd * (gf[i] * wf[c][i]) - xf[i] * coef) + rf[i];
                         acc[c][i] += gf[i] * (xf[i] * rstd);
                     }
                     dxr[v] = Elem<T>::pack(o);
@@ -193,9 +200,10 @@ constexpr int kRmsWideBlock = 1024; // RMSNorm backward: one block per compute u
 constexpr int kWideMaxBlocks = 256;
 constexpr int kLnMaxBlocks = 512;     // partial dweight / dbias rows of the LayerNorm backward
 
-template <typename T, int TPR, int CH>
+template <typename T, int TPR, int CH, bool RES>
 __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                                          const T* __restrict__ dy, T* __restrict__ dx,
+                                                                          const T* __restrict__ dy, const T* __restrict__ dres,
+                                                                          T* __restrict__ dx,
                                                                           float* __restrict__ dw_partial, int64_t n_rows,
                                                                           int hidden, float eps) {
     constexpr int V = Elem<T>::kVec;
@@ -223,8 +231,10 @@ __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T
     const int64_t iters = (n_rows + row_step - 1) / row_step;
     // the rows of iteration it + 1 are fetched while iteration it is reduced, so loads stay in flight
     // across the block-wide reductions
-    uint4 xraw[CH], graw[CH], xnext[CH], gnext[CH];
-    auto fetch = [&](int64_t it, uint4 (&xv)[CH], uint4 (&gv)[CH]) {
+    // dres is prefetched with the rows where one vector per thread leaves room for it, else requested before the reductions
+    constexpr bool kResAhead = RES && CH == 1;
+    struct Rows { uint4 x[CH], g[CH], r[kResAhead ? CH : 1]; };
+    auto fetch = [&](int64_t it, Rows& rows) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
         const bool row_ok = row < n_rows;
         const uint4* xr = reinterpret_cast<const uint4*>(x + (row_ok ? row : 0) * hidden);
@@ -233,20 +243,29 @@ __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T
         for (int c = 0; c < CH; ++c) {
             const int v = c * TPR + tr;
             const bool ok = row_ok && v < vecs;
-            xv[c] = ok ? xr[v] : make_uint4(0, 0, 0, 0);
-            gv[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
+            rows.x[c] = ok ? xr[v] : make_uint4(0, 0, 0, 0);
+            rows.g[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
+            if constexpr (kResAhead) rows.r[c] = ok ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
         }
     };
     // one row step: reduce the two row sums over the row's wavefronts (one barrier), write dx, add to dweight
-    auto process = [&](int64_t it, const uint4 (&xv)[CH], const uint4 (&gv)[CH]) {
+    auto process = [&](int64_t it, const Rows& rows) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
         const bool row_ok = row < n_rows;
+        uint4 res[RES && !kResAhead ? CH : 1];
+        if constexpr (RES && !kResAhead) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const int v = c * TPR + tr;
+                res[c] = row_ok && v < vecs ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
+            }
+        }
         float ss = 0.f, dot = 0.f;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             float xf[V], gf[V], wf[V];
-            Elem<T>::unpack(xv[c], xf);
-            Elem<T>::unpack(gv[c], gf);
+            Elem<T>::unpack(rows.x[c], xf);
+            Elem<T>::unpack(rows.g[c], gf);
             const int v0 = (c * TPR + tr < vecs ? c * TPR + tr : 0) * V;
 #pragma unroll
             for (int i = 0; i < V; i += 4) *reinterpret_cast<f32x4_t*>(wf + i) = *reinterpret_cast<const f32x4_t*>(w_lds + v0 + i);
@@ -278,14 +297,21 @@ __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T
                 const int v = c * TPR + tr;
                 if (v < vecs) {
                     float xf[V], gf[V], wf[V], o[V];
-                    Elem<T>::unpack(xv[c], xf);
-                    Elem<T>::unpack(gv[c], gf);
+                    Elem<T>::unpack(rows.x[c], xf);
+                    Elem<T>::unpack(rows.g[c], gf);
 #pragma unroll
                     for (int i = 0; i < V; i += 4) *reinterpret_cast<f32x4_t*>(wf + i) = *reinterpret_cast<const f32x4_t*>(w_lds + v * V + i);
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
                         o[i] = rstd * (gf[i] * wf[i]) - xf[i] * coef;
                         acc[c][i] += gf[i] * (xf[i] * rstd);
+                    }
+                    if constexpr (RES) {
+                        float rf[V];
+                        if constexpr (kResAhead) Elem<T>::unpack(rows.r[c], rf);
+                        else Elem<T>::unpack(res[c], rf);
+#pragma unroll
+                        for (int i = 0; i < V; ++i) o[i] = round_to<T>(o[i]) + rf[i];
                     }
                     dxr[v] = Elem<T>::pack(o);
                 }
@@ -297,36 +323,37 @@ __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T
     // made every wavefront issue its loads at the same moment and the memory pipe ran dry in between).  The loop
     // is unrolled by three so that every set is addressed statically; `iters` is the same for the whole block.
     constexpr bool kDeep = CH == 1;       // three register sets fit without spilling only for one vector per thread
+    Rows r0, r1;
     if constexpr (kDeep) {
-        uint4 x2[CH], g2[CH];
-        if (iters > 0) fetch(0, xraw, graw);
-        if (iters > 1) fetch(1, xnext, gnext);
+        Rows r2;
+        if (iters > 0) fetch(0, r0);
+        if (iters > 1) fetch(1, r1);
         for (int64_t it = 0; it < iters; it += 3) {
-            if (it + 2 < iters) fetch(it + 2, x2, g2);
-            process(it, xraw, graw);
+            if (it + 2 < iters) fetch(it + 2, r2);
+            process(it, r0);
             if (it + 1 < iters) {
-                if (it + 3 < iters) fetch(it + 3, xraw, graw);
-                process(it + 1, xnext, gnext);
+                if (it + 3 < iters) fetch(it + 3, r0);
+                process(it + 1, r1);
             }
             if (it + 2 < iters) {
-                if (it + 4 < iters) fetch(it + 4, xnext, gnext);
-                process(it + 2, x2, g2);
+                if (it + 4 < iters) fetch(it + 4, r1);
+                process(it + 2, r2);
             }
         }
     } else if constexpr (CH <= 2) {       // two sets: the rows of step it + 1 are in flight while step it is reduced
-        if (iters > 0) fetch(0, xraw, graw);
+        if (iters > 0) fetch(0, r0);
         for (int64_t it = 0; it < iters; it += 2) {
-            if (it + 1 < iters) fetch(it + 1, xnext, gnext);
-            process(it, xraw, graw);
+            if (it + 1 < iters) fetch(it + 1, r1);
+            process(it, r0);
             if (it + 1 < iters) {
-                if (it + 2 < iters) fetch(it + 2, xraw, graw);
-                process(it + 1, xnext, gnext);
+                if (it + 2 < iters) fetch(it + 2, r0);
+                process(it + 1, r1);
             }
         }
     } else {
         for (int64_t it = 0; it < iters; ++it) {
-            fetch(it, xraw, graw);
-            process(it, xraw, graw);
+            fetch(it, r0);
+            process(it, r0);
         }
     }
     for (int i = threadIdx.x; i < hidden; i += kRmsWideBlock) dw_lds[i] = 0.f;
@@ -462,7 +489,7 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t n_row
 }
 
 template <typename T>
-int launch_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw, void* ws, size_t ws_bytes,
+int launch_bwd(const void* x, const void* w, const void* dy, const void* dres, void* dx, void* dw, void* ws, size_t ws_bytes,
                int64_t n_rows, int64_t hidden, float eps, hipStream_t st) {
     Plan plan;
     if (!make_plan<T>(hidden, &plan))
@@ -484,12 +511,14 @@ int launch_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw,
     if (wide) {
         const int ch = (int)((vecs + wide_tpr - 1) / wide_tpr);
         const size_t lds = 2 * hidden * sizeof(float);
-#define RMS_WIDE(TPRV, CHV) rmsnorm_bwd_wide_kernel<T, TPRV, CHV><<<dim3(blocks), dim3(kRmsWideBlock), lds, st>>>( \
-            (const T*)x, (const T*)w, (const T*)dy, (T*)dx, (float*)ws, n_rows, (int)hidden, eps)
+#define RMS_WIDE_R(TPRV, CHV, RESV) rmsnorm_bwd_wide_kernel<T, TPRV, CHV, RESV><<<dim3(blocks), dim3(kRmsWideBlock), lds, st>>>( \
+            (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, (T*)dx, (float*)ws, n_rows, (int)hidden, eps)
+#define RMS_WIDE(TPRV, CHV) do { if (dres != nullptr) RMS_WIDE_R(TPRV, CHV, true); else RMS_WIDE_R(TPRV, CHV, false); } while (0)
         if (wide_tpr == 256) { if (ch <= 1) RMS_WIDE(256, 1); else RMS_WIDE(256, 2); }
         else if (wide_tpr == 512) { if (ch <= 1) RMS_WIDE(512, 1); else RMS_WIDE(512, 2); }
         else RMS_WIDE(1024, 2);
 #undef RMS_WIDE
+#undef RMS_WIDE_R
         int rcw = mi_check_launch("rmsnorm_bwd_wide");
         if (rcw != MI_OK) return rcw;
         rmsnorm_dw_reduce_kernel<T><<<dim3((unsigned)((hidden + kDwCols - 1) / kDwCols)), dim3(kBlock), 0, st>>>((const float*)ws, (T*)dw,
@@ -500,7 +529,7 @@ int launch_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw,
         constexpr int TPR = decltype(tag)::TPR;
         constexpr int CH = decltype(tag)::CH;
         rmsnorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), hidden * sizeof(float), st>>>(
-            (const T*)x, (const T*)w, (const T*)dy, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
+            (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
     });
     if (!launched) return mi_fail(MI_E_SHAPE, "rmsnorm: no kernel for hidden=%lld", (long long)hidden);
     int rc = mi_check_launch("rmsnorm_bwd");
@@ -513,11 +542,13 @@ int launch_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw,
 // ---- LayerNorm (weight and optional bias) -----------------------------------------------------------------
 // Same row ownership as the RMSNorm kernels.  Mean and variance are taken in fp32 from the register copy of
 // the row (two passes over registers, one over HBM).
-template <typename T, int TPR, int CH>
+// ADD as in rmsnorm_fwd_kernel.
+template <typename T, int TPR, int CH, bool ADD = false>
 __global__ __launch_bounds__(kBlock) void layernorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                                 const T* __restrict__ b, T* __restrict__ y,
                                                                 float* __restrict__ mean_out, float* __restrict__ rstd_out,
-                                                                int64_t n_rows, int hidden, float eps) {
+                                                                int64_t n_rows, int hidden, float eps,
+                                                                const T* residual = nullptr, T* sum_out = nullptr) {
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kBlock / TPR;
     __shared__ float lds[4];
@@ -532,7 +563,18 @@ __global__ __launch_bounds__(kBlock) void layernorm_fwd_kernel(const T* __restri
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         const int v = c * TPR + tr;
-        const uint4 raw = (row_ok && v < vecs) ? ldg_nt(xr + v) : make_uint4(0, 0, 0, 0);
+        uint4 raw = (row_ok && v < vecs) ? (ADD ? xr[v] : ldg_nt(xr + v)) : make_uint4(0, 0, 0, 0);
+        if constexpr (ADD) {
+            if (row_ok && v < vecs) {
+                float a[V], r[V];
+                Elem<T>::unpack(raw, a);
+                Elem<T>::unpack(reinterpret_cast<const uint4*>(residual + row * hidden)[v], r);
+#pragma unroll
+                for (int i = 0; i < V; ++i) a[i] += r[i];
+                raw = Elem<T>::pack(a);                // the norm sees the sum as it is stored
+                reinterpret_cast<uint4*>(sum_out + row * hidden)[v] = raw;
+            }
+        }
         Elem<T>::unpack(raw, f[c]);
 #pragma unroll
         for (int i = 0; i < V; ++i) sum += f[c][i];
@@ -572,7 +614,8 @@ __global__ __launch_bounds__(kBlock) void layernorm_fwd_kernel(const T* __restri
 // partial rows: [gridDim.x][hidden] of dw followed by [gridDim.x][hidden] of db
 template <typename T, int TPR, int CH>
 __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                                const T* __restrict__ dy, T* __restrict__ dx,
+                                                                const T* __restrict__ dy, const T* __restrict__ dres,
+                                                                T* __restrict__ dx,
                                                                 float* __restrict__ partial, int64_t n_rows, int hidden,
                                                                 float eps) {
     constexpr int V = Elem<T>::kVec;
@@ -599,7 +642,7 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
         const uint4* xr = reinterpret_cast<const uint4*>(x + (row_ok ? row : 0) * hidden);
         const uint4* gr = reinterpret_cast<const uint4*>(dy + (row_ok ? row : 0) * hidden);
         float xf[CH][V], gw[CH][V];
-        uint4 graw[CH];
+        uint4 graw[CH], rraw[CH];
         float sum = 0.f;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
@@ -607,6 +650,7 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
             const bool ok = row_ok && v < vecs;
             const uint4 xraw = ok ? xr[v] : make_uint4(0, 0, 0, 0);
             graw[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
+            rraw[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
             Elem<T>::unpack(xraw, xf[c]);
 #pragma unroll
             for (int i = 0; i < V; ++i) sum += xf[c][i];
@@ -648,9 +692,10 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
             for (int c = 0; c < CH; ++c) {
                 const int v = c * TPR + tr;
                 if (v < vecs) {
-                    float o[V];
+                    float o[V], rf[V];
+                    Elem<T>::unpack(rraw[c], rf);
 #pragma unroll
-                    for (int i = 0; i < V; ++i) o[i] = rstd * (gw[c][i] - s1 - xf[c][i] * s2);
+                    for (int i = 0; i < V; ++i) o[i] = round_to<T>(rstd * (gw[c][i] - s1 - xf[c][i] * s2)) + rf[i];
                     dxr[v] = Elem<T>::pack(o);
                 }
             }
@@ -832,9 +877,9 @@ __global__ __launch_bounds__(kWideBlock, 4) void layernorm_bwd_wide_kernel(const
 // Backward for wide rows when the forward pass saved mean and rstd: the two row sums (g*w and g*w*xhat) no
 // longer wait for the statistics, so a row step takes one block-wide reduction, as in rmsnorm_bwd_wide_kernel
 // (same block shape: kRmsWideBlock threads, one block per compute unit, one barrier per row step).
-template <typename T, int TPR, int CH>
+template <typename T, int TPR, int CH, bool RES>
 __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                                             const T* __restrict__ dy,
+                                                                             const T* __restrict__ dy, const T* __restrict__ dres,
                                                                              const float* __restrict__ mean_in,
                                                                              const float* __restrict__ rstd_in, T* __restrict__ dx,
                                                                              float* __restrict__ partial, int64_t n_rows,
@@ -860,7 +905,7 @@ __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(cons
     __syncthreads();
     const int64_t row_step = (int64_t)gridDim.x * RPB;
     const int64_t iters = (n_rows + row_step - 1) / row_step;
-    uint4 xraw[CH], graw[CH], xnext[CH], gnext[CH];
+    uint4 xraw[CH], graw[CH], xnext[CH], gnext[CH], rraw[RES ? CH : 1];
     float mean = 0.f, rstd = 0.f, mean_next = 0.f, rstd_next = 0.f;
     auto fetch = [&](int64_t it, uint4 (&xv)[CH], uint4 (&gv)[CH], float& mu, float& rs) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
@@ -881,6 +926,13 @@ __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(cons
     for (int64_t it = 0; it < iters; ++it) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
         const bool row_ok = row < n_rows;
+        if constexpr (RES) {                           // used after the reductions: its latency hides behind them
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const int v = c * TPR + tr;
+                rraw[c] = row_ok && v < vecs ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
+            }
+        }
         if (it + 1 < iters) fetch(it + 1, xnext, gnext, mean_next, rstd_next);
         float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -931,6 +983,12 @@ __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(cons
                         acc_w[c][i] += gf[i] * xhat;
                         acc_b[c][i] += gf[i];
                     }
+                    if constexpr (RES) {
+                        float rf[V];
+                        Elem<T>::unpack(rraw[c], rf);
+#pragma unroll
+                        for (int i = 0; i < V; ++i) o[i] = round_to<T>(o[i]) + rf[i];
+                    }
                     dxr[v] = Elem<T>::pack(o);
                 }
             }
@@ -965,7 +1023,7 @@ __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(cons
 
 template <typename T>
 int launch_ln_fwd(const void* x, const void* w, const void* b, void* y, float* mean, float* rstd, int64_t n_rows,
-                  int64_t hidden, float eps, hipStream_t st) {
+                  int64_t hidden, float eps, hipStream_t st, const void* residual = nullptr, void* sum_out = nullptr) {
     Plan plan;
     if (!make_plan<T>(hidden, &plan))
         return mi_fail(MI_E_SHAPE, "layernorm: hidden=%lld unsupported (must be a multiple of %d and <= %d)",
@@ -975,15 +1033,19 @@ int launch_ln_fwd(const void* x, const void* w, const void* b, void* y, float* m
         constexpr int CH = decltype(tag)::CH;
         const int rpb = kBlock / TPR;
         const unsigned grid = (unsigned)((n_rows + rpb - 1) / rpb);
-        layernorm_fwd_kernel<T, TPR, CH><<<dim3(grid), dim3(kBlock), 0, st>>>((const T*)x, (const T*)w, (const T*)b, (T*)y,
-                                                                              mean, rstd, n_rows, (int)hidden, eps);
+        if (residual != nullptr)
+            layernorm_fwd_kernel<T, TPR, CH, true><<<dim3(grid), dim3(kBlock), 0, st>>>((const T*)x, (const T*)w, (const T*)b, (T*)y, mean, rstd,
+                                                                                        n_rows, (int)hidden, eps, (const T*)residual, (T*)sum_out);
+        else
+            layernorm_fwd_kernel<T, TPR, CH><<<dim3(grid), dim3(kBlock), 0, st>>>((const T*)x, (const T*)w, (const T*)b, (T*)y,
+                                                                                  mean, rstd, n_rows, (int)hidden, eps);
     });
     if (!launched) return mi_fail(MI_E_SHAPE, "layernorm: no kernel for hidden=%lld", (long long)hidden);
     return mi_check_launch("layernorm_fwd");
 }
 
 template <typename T>
-int launch_ln_bwd(const void* x, const void* w, const void* dy, const float* mean, const float* rstd, void* dx, void* dw,
+int launch_ln_bwd(const void* x, const void* w, const void* dy, const void* dres, const float* mean, const float* rstd, void* dx, void* dw,
                   void* db, void* ws, size_t ws_bytes, int64_t n_rows, int64_t hidden, float eps, hipStream_t st) {
     Plan plan;
     if (!make_plan<T>(hidden, &plan)) return mi_fail(MI_E_SHAPE, "layernorm: hidden=%lld unsupported", (long long)hidden);
@@ -1007,12 +1069,14 @@ int launch_ln_bwd(const void* x, const void* w, const void* dy, const float* mea
     if (stats) {
         const int ch = (int)((vecs + wide_tpr - 1) / wide_tpr);
         const size_t lds = 3 * hidden * sizeof(float);
-#define LN_STATS(TPRV, CHV) layernorm_bwd_stats_kernel<T, TPRV, CHV><<<dim3(blocks), dim3(kRmsWideBlock), lds, st>>>( \
-            (const T*)x, (const T*)w, (const T*)dy, mean, rstd, (T*)dx, (float*)ws, n_rows, (int)hidden)
+#define LN_STATS_R(TPRV, CHV, RESV) layernorm_bwd_stats_kernel<T, TPRV, CHV, RESV><<<dim3(blocks), dim3(kRmsWideBlock), lds, st>>>( \
+            (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, mean, rstd, (T*)dx, (float*)ws, n_rows, (int)hidden)
+#define LN_STATS(TPRV, CHV) do { if (dres != nullptr) LN_STATS_R(TPRV, CHV, true); else LN_STATS_R(TPRV, CHV, false); } while (0)
         if (wide_tpr == 256) { if (ch <= 1) LN_STATS(256, 1); else LN_STATS(256, 2); }
         else if (wide_tpr == 512) LN_STATS(512, 2);
         else LN_STATS(1024, 2);
 #undef LN_STATS
+#undef LN_STATS_R
     } else if (wide) {
         const int ch = (int)((vecs + wide_tpr - 1) / wide_tpr);
         const size_t lds = 3 * hidden * sizeof(float);
@@ -1026,7 +1090,7 @@ int launch_ln_bwd(const void* x, const void* w, const void* dy, const float* mea
             constexpr int TPR = decltype(tag)::TPR;
             constexpr int CH = decltype(tag)::CH;
             layernorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), 2 * hidden * sizeof(float), st>>>(
-                (const T*)x, (const T*)w, (const T*)dy, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
+                (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
         });
     }
     if (!launched) return mi_fail(MI_E_SHAPE, "layernorm: no kernel for hidden=%lld", (long long)hidden);
@@ -1069,16 +1133,22 @@ size_t mi_rmsnorm_bwd_workspace_bytes(int64_t n_rows, int64_t hidden) {
     return (size_t)kMaxBwdBlocks * (size_t)(hidden > 0 ? hidden : 0) * sizeof(float);
 }
 
-int mi_rmsnorm_bwd(const void* x, const void* weight, const void* dy, void* dx, void* dweight, void* workspace,
-                   size_t workspace_bytes, int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream) {
+int mi_add_rmsnorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, void* dx, void* dweight, void* workspace,
+                       size_t workspace_bytes, int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream) {
     if (!x || !weight || !dy || !dx || !dweight) return mi_fail(MI_E_NULL, "rmsnorm_bwd: null pointer");
     if (n_rows <= 0 || hidden <= 0) return mi_fail(MI_E_SHAPE, "rmsnorm_bwd: bad shape [%lld, %lld]", (long long)n_rows, (long long)hidden);
     if (!mi_aligned16(x) || !mi_aligned16(weight) || !mi_aligned16(dy) || !mi_aligned16(dx) || !mi_aligned16(workspace))
         return mi_fail(MI_E_ALIGN, "rmsnorm_bwd: pointers must be 16-byte aligned");
+    if (dsum && !mi_aligned16(dsum)) return mi_fail(MI_E_ALIGN, "rmsnorm_bwd: pointers must be 16-byte aligned");
     if (2 * hidden * sizeof(float) > 160 * 1024 - 256) return mi_fail(MI_E_SHAPE, "rmsnorm_bwd: hidden too large for LDS");
-    MI_DISPATCH_DTYPE(dtype, return launch_bwd<T>(x, weight, dy, dx, dweight, workspace, workspace_bytes, n_rows, hidden,
+    MI_DISPATCH_DTYPE(dtype, return launch_bwd<T>(x, weight, dy, dsum, dx, dweight, workspace, workspace_bytes, n_rows, hidden,
                                                   eps, (hipStream_t)stream));
     return MI_OK;
+}
+
+int mi_rmsnorm_bwd(const void* x, const void* weight, const void* dy, void* dx, void* dweight, void* workspace,
+                   size_t workspace_bytes, int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream) {
+    return mi_add_rmsnorm_bwd(x, weight, dy, nullptr, dx, dweight, workspace, workspace_bytes, n_rows, hidden, eps, dtype, stream);
 }
 
 int mi_layernorm_fwd(const void* x, const void* weight, const void* bias, void* y, float* mean, float* rstd,
@@ -1093,23 +1163,45 @@ int mi_layernorm_fwd(const void* x, const void* weight, const void* bias, void* 
     return MI_OK;
 }
 
+int mi_add_layernorm_fwd(const void* x, const void* residual, const void* weight, const void* bias, void* sum_out, void* y, float* mean,
+                         float* rstd, int64_t n_rows, int64_t hidden, float eps, int dtype, void* stream) {
+    if (n_rows == 0) return MI_OK;       // nothing to do (an empty tensor may come with a null pointer)
+    if (!x || !residual || !weight || !sum_out || !y) return mi_fail(MI_E_NULL, "add_layernorm_fwd: null pointer");
+    if ((mean == nullptr) != (rstd == nullptr)) return mi_fail(MI_E_NULL, "add_layernorm_fwd: mean and rstd go together");
+    if (n_rows < 0 || hidden <= 0) return mi_fail(MI_E_SHAPE, "add_layernorm_fwd: bad shape [%lld, %lld]", (long long)n_rows, (long long)hidden);
+    if (!mi_aligned16(x) || !mi_aligned16(residual) || !mi_aligned16(weight) || !mi_aligned16(sum_out) || !mi_aligned16(y) ||
+        (bias && !mi_aligned16(bias)))
+        return mi_fail(MI_E_ALIGN, "add_layernorm_fwd: pointers must be 16-byte aligned");
+    if (y == sum_out || y == x || y == residual) return mi_fail(MI_E_SHAPE, "add_layernorm_fwd: y must not alias the other tensors");
+    MI_DISPATCH_DTYPE(dtype, return launch_ln_fwd<T>(x, weight, bias, y, mean, rstd, n_rows, hidden, eps, (hipStream_t)stream, residual, sum_out));
+    return MI_OK;
+}
+
 size_t mi_layernorm_bwd_workspace_bytes(int64_t n_rows, int64_t hidden) {
     (void)n_rows;
     return (size_t)2 * kLnMaxBlocks * (size_t)(hidden > 0 ? hidden : 0) * sizeof(float);
 }
 
-int mi_layernorm_bwd(const void* x, const void* weight, const void* dy, const float* mean, const float* rstd, void* dx,
-                     void* dweight, void* dbias, void* workspace, size_t workspace_bytes, int64_t n_rows, int64_t hidden,
-                     float eps, int dtype, void* stream) {
+int mi_add_layernorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, const float* mean, const float* rstd,
+                         void* dx, void* dweight, void* dbias, void* workspace, size_t workspace_bytes, int64_t n_rows, int64_t hidden,
+                         float eps, int dtype, void* stream) {
     if (!x || !weight || !dy || !dx || !dweight) return mi_fail(MI_E_NULL, "layernorm_bwd: null pointer");
     if ((mean == nullptr) != (rstd == nullptr)) return mi_fail(MI_E_NULL, "layernorm_bwd: mean and rstd go together");
     if (n_rows <= 0 || hidden <= 0) return mi_fail(MI_E_SHAPE, "layernorm_bwd: bad shape [%lld, %lld]", (long long)n_rows, (long long)hidden);
     if (!mi_aligned16(x) || !mi_aligned16(weight) || !mi_aligned16(dy) || !mi_aligned16(dx) || !mi_aligned16(workspace))
         return mi_fail(MI_E_ALIGN, "layernorm_bwd: pointers must be 16-byte aligned");
+    if (dsum && !mean) return mi_fail(MI_E_NULL, "layernorm_bwd: with dsum the saved mean and rstd are required");
+    if (dsum && !mi_aligned16(dsum)) return mi_fail(MI_E_ALIGN, "layernorm_bwd: pointers must be 16-byte aligned");
     if (2 * hidden * sizeof(float) > 160 * 1024 - 256) return mi_fail(MI_E_SHAPE, "layernorm_bwd: hidden too large for LDS");
-    MI_DISPATCH_DTYPE(dtype, return launch_ln_bwd<T>(x, weight, dy, mean, rstd, dx, dweight, dbias, workspace, workspace_bytes,
+    MI_DISPATCH_DTYPE(dtype, return launch_ln_bwd<T>(x, weight, dy, dsum, mean, rstd, dx, dweight, dbias, workspace, workspace_bytes,
                                                      n_rows, hidden, eps, (hipStream_t)stream));
     return MI_OK;
+}
+
+int mi_layernorm_bwd(const void* x, const void* weight, const void* dy, const float* mean, const float* rstd, void* dx,
+                     void* dweight, void* dbias, void* workspace, size_t workspace_bytes, int64_t n_rows, int64_t hidden,
+                     float eps, int dtype, void* stream) {
+    return mi_add_layernorm_bwd(x, weight, dy, nullptr, mean, rstd, dx, dweight, dbias, workspace, workspace_bytes, n_rows, hidden, eps, dtype, stream);
 }
 
 }  // extern "C"

@@ -10,7 +10,7 @@ from typing import Callable, List, Optional
 import torch
 
 from .config import MLPType, TransformerArchitectureConfig
-from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, get_norm
+from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, fuses_residual, get_norm
 
 
 class InferenceSettings:
@@ -114,10 +114,25 @@ class TransformerLayer(torch.nn.Module):
         s = x.inference_settings
         use_cache, reset_cache, cache_index = (False, False, 0) if s is None else (s.use_cache, s.reset_cache, s.cache_index)
         assert x.cumulative_seq_lengths is not None
-        h = self.attention_block(x.activations, x.cumulative_seq_lengths, x.position_ids, use_cache=use_cache,
-                                 reset_cache=reset_cache, cache_index=cache_index,
-                                 attention_scores_manipulation=x.attention_scores_manipulation)
-        h = self.mlp_block(h)
+        cls = type(self)
+        blocks_as_here = cls.attention_block is TransformerLayer.attention_block and cls.mlp_block is TransformerLayer.mlp_block
+        if blocks_as_here and fuses_residual(self.input_layernorm) and fuses_residual(self.post_attention_layernorm):
+            # the same arithmetic as attention_block and mlp_block, with the residual stream taken through the norms (and, where
+            # nothing comes between, the last projection): its sums and the sums of its gradients need no passes of their own
+            h, n = self.input_layernorm.with_residual(x.activations)
+            a = self.self_attention(n, cumulative_seq_lengths=x.cumulative_seq_lengths,
+                                    attention_scores_manipulation=x.attention_scores_manipulation, position_ids=x.position_ids,
+                                    use_cache=use_cache, reset_cache=reset_cache, cache_index=cache_index)
+            h, n = self.post_attention_layernorm.with_residual(self.dropout_attention(a), h)
+            if fuses_residual(self.mlp) and (self.dropout_mlp.p == 0.0 or not self.dropout_mlp.training):
+                h = self.mlp(n, h)
+            else:
+                h = self.dropout_mlp(self.mlp(n)) + h
+        else:
+            h = self.attention_block(x.activations, x.cumulative_seq_lengths, x.position_ids, use_cache=use_cache,
+                                     reset_cache=reset_cache, cache_index=cache_index,
+                                     attention_scores_manipulation=x.attention_scores_manipulation)
+            h = self.mlp_block(h)
         return TransformerLayerIO(activations=h, cumulative_seq_lengths=x.cumulative_seq_lengths,
                                   cumulative_seq_lengths_padded=x.cumulative_seq_lengths_padded,
                                   attention_scores_manipulation=x.attention_scores_manipulation,

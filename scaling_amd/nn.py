@@ -68,14 +68,25 @@ class _Linear(torch.nn.Module):
         else:
             self.register_parameter("bias", None)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(x, self.weight, self.bias)
+    def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        return ops.linear(x, self.weight, self.bias, residual)
+
+
+def _unhooked(m: torch.nn.Module) -> bool:
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
 
 
 def _direct(*modules: torch.nn.Module) -> bool:
     """Whether calling the modules comes to using their weights: plain projections that nobody replaced or hooked."""
-    return all(type(m) is _Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-               for m in modules)
+    return all(type(m) is _Linear and _unhooked(m) for m in modules)
+
+
+def fuses_residual(m: torch.nn.Module) -> bool:
+    """Whether the residual stream may pass through the module (norm.with_residual, mlp(x, residual)): one of this package's
+    norms or MLPs that nobody replaced or hooked, so that no observer sees other tensors than before."""
+    if type(m) in (RMSNorm, LayerNorm):
+        return _unhooked(m)
+    return type(m) in (ParallelSwiGLUMLP, ParallelMLP) and _unhooked(m) and _direct(m.dense_out)
 
 
 def _project_together(x: torch.Tensor, *modules: torch.nn.Module):
@@ -100,6 +111,10 @@ class RMSNorm(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return ops.rms_norm(x, self.weight, self.eps)
 
+    def with_residual(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+        """(s, norm(s)) with s = x + residual (x itself without a residual) in one launch."""
+        return ops.add_norm(x, residual, self.weight, None, self.eps, False)
+
 
 class LayerNorm(torch.nn.Module):
     """Mirror of core/nn/norm/layernorm.py:16-86 (`optimization_type: torch`; u-muP and bitfit bias names
@@ -121,6 +136,10 @@ class LayerNorm(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return ops.layer_norm(x, self.weight, self.bias, self.eps)
+
+    def with_residual(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+        """(s, norm(s)) with s = x + residual (x itself without a residual) in one launch."""
+        return ops.add_norm(x, residual, self.weight, self.bias, self.eps, True)
 
 
 def get_norm(norm_type: NormType, layernorm_config: Optional[LayerNormConfig], dimensions: int,
@@ -225,8 +244,10 @@ class ParallelSwiGLUMLP(torch.nn.Module):
         self.siglu_weight = _Linear(io_features, inter, bias, device, dtype, init_method)
         self.dense_out = _Linear(inter, io_features, bias, device, dtype, init_method)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.dense_out(ops.swiglu(*_project_together(x, self.dense_in, self.siglu_weight)))
+    def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """`residual` (optional, see fuses_residual) is added to the output."""
+        act = ops.swiglu(*_project_together(x, self.dense_in, self.siglu_weight))
+        return self.dense_out(act) if residual is None else self.dense_out(act, residual)
 
 
 class ParallelMLP(torch.nn.Module):
@@ -252,8 +273,10 @@ class ParallelMLP(torch.nn.Module):
         self.dense_in = _Linear(io_features, inter, bias, device, dtype, init_method)
         self.dense_out = _Linear(inter, io_features, bias, device, dtype, init_method)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.dense_out(ops.gelu(self.dense_in(x)))
+    def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """`residual` (optional, see fuses_residual) is added to the output."""
+        act = ops.gelu(self.dense_in(x))
+        return self.dense_out(act) if residual is None else self.dense_out(act, residual)
 
 
 class MaskedSoftmax(torch.nn.Module):
@@ -310,6 +333,12 @@ class ScaledDotProductAttention(torch.nn.Module):
         return ops.attention(q, k, v, cumulative_seq_lengths, cumulative_seq_lengths_key, self.causal, self.softmax_scale,
                              dropout_p=self.dropout_p if self.training else 0.0, rotary=rotary,
                              deterministic=self.masked_softmax_config.deterministic_flash_attn_bwd)
+
+    def forward_qkv(self, qkv: torch.Tensor, cumulative_seq_lengths: torch.Tensor,
+                    cumulative_seq_lengths_key: Optional[torch.Tensor] = None, rotary=None) -> torch.Tensor:
+        """qkv [tokens, n, 3 d] (per head q, then k, then v: the output of one projection) -> [tokens, n, d]."""
+        return ops.attention_qkv(qkv, cumulative_seq_lengths, cumulative_seq_lengths_key, self.causal, self.softmax_scale,
+                                 dropout_p=self.dropout_p if self.training else 0.0, rotary=rotary)
 
     def forward(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cumulative_seq_lengths: torch.Tensor,
                 attention_scores_manipulation: Optional[torch.Tensor] = None,
@@ -522,13 +551,23 @@ class ParallelSelfAttention(torch.nn.Module):
             raise NotImplementedError("attention_scores_manipulation is not available with the hip kernel")
         b, s, hidden = x.shape
         nq, nkv, d = self.num_attention_heads, self.num_kv_heads_per_partition, self.hidden_size_per_attention_head
+        pos = None if position_ids is None else position_ids.reshape(-1).contiguous()
+        cu = cumulative_seq_lengths.to(torch.int32)
+        sdpa = self.scaled_dot_product_attention
+        if self.qkv_in_one and not use_cache and not self.key_query_norm and \
+                (self.rotary_embedding is None or (self._fusable_rotary and pos is not None)):
+            # nothing touches q, k or v between the projection and the attention core: it takes the projection output as it is
+            if reset_cache:
+                self.cache[cache_index] = None
+            self._check_positions(pos)
+            cu_k = None if cumulative_seq_lengths_key is None else cumulative_seq_lengths_key.to(torch.int32)
+            rotary = (*self.rotary_embedding.tables(), pos, pos) if self.rotary_embedding is not None else None
+            ctx = sdpa.forward_qkv(self.query_key_value(x).view(b * s, nq, 3 * d), cu, cu_k, rotary)
+            return self.dense(ctx.view(b, s, nq * d))
         q, k, v = self._project(x)
         if self.key_query_norm:
             q = self.norm_query(q)
             k = self.norm_key(k)
-        pos = None if position_ids is None else position_ids.reshape(-1).contiguous()
-        cu = cumulative_seq_lengths.to(torch.int32)
-        sdpa = self.scaled_dot_product_attention
 
         if use_cache:
             if not self.causal:

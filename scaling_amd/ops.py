@@ -38,11 +38,17 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
     to the tensor dtype before it is normalised, as the separate add and norm would do."""
     _need_cuda(x, residual, weight)
     assert x.shape == residual.shape and x.dtype == residual.dtype == weight.dtype and x.shape[-1] == weight.shape[0]
-    x2, r2 = x.contiguous().view(-1, x.shape[-1]), residual.contiguous().view(-1, x.shape[-1])
-    total, y = torch.empty_like(x2), torch.empty_like(x2)
-    check(_lib.load().mi_add_rmsnorm_fwd(ptr(x2), ptr(r2), ptr(weight.contiguous()), ptr(total), ptr(y), x2.shape[0], x2.shape[1],
-                                         float(eps), dtype_code(x.dtype), stream_ptr()), "mi_add_rmsnorm_fwd")
-    return total.view(x.shape), y.view(x.shape)
+    with torch.no_grad():
+        return _lib.host().add_norm(x, residual, weight, None, eps, False)
+
+
+def add_norm(x: torch.Tensor, residual: Optional[torch.Tensor], weight: torch.Tensor, bias: Optional[torch.Tensor], eps: float,
+             layer_norm: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(s, norm(s)) with s = x + residual, or s = x without a residual, in one launch; differentiable, with the gradient that
+    reaches s directly added inside the norm's backward kernel.  LayerNorm or RMSNorm (no bias)."""
+    _need_cuda(x, residual, weight, bias)
+    assert x.shape[-1] == weight.shape[0] and weight.dtype == x.dtype and (residual is None or residual.shape == x.shape)
+    return _lib.host().add_norm(x, residual, weight, bias, eps, layer_norm)
 
 
 def rms_norm_forward(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -133,10 +139,11 @@ def swiglu(a: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
 # ------------------------------------------------------------------------------------------------
 # linear projections
 # ------------------------------------------------------------------------------------------------
-def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x W^T + b (torch.nn.functional.linear), on the matrix kernel of this package where the product is too small to fill
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+           residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T + b (torch.nn.functional.linear) (+ residual), on the matrix kernel of this package where the product is too small to fill
     the chip and on the library product elsewhere."""
-    return _lib.host().linear(x, weight, bias)
+    return _lib.host().linear(x, weight, bias, residual)
 
 
 def projections(x: torch.Tensor, weights, biases):
@@ -464,6 +471,26 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q: t
     p, seed = _dropout_args((dropout_p, dropout_seed if dropout_seed is not None else 0))
     return _lib.host().attention(q, k, v, cu_seqlens_q, cu_seqlens_k, bool(causal), float(softmax_scale), p, seed, cos, sin, pos_q, pos_k,
                                  interleaved, bool(precise))
+
+
+def attention_qkv(qkv: torch.Tensor, cu_seqlens_q: torch.Tensor, cu_seqlens_k: Optional[torch.Tensor] = None, causal: bool = True,
+                  softmax_scale: Optional[float] = None, dropout_p: float = 0.0, dropout_seed: Optional[int] = None, rotary=None) -> torch.Tensor:
+    """`attention` on one projection output qkv [tokens, heads, 3 d] (per head q, then k, then v), whose gradient comes back in
+    the same layout."""
+    d = qkv.shape[2] // 3
+    if softmax_scale is None:
+        softmax_scale = 1.0 / math.sqrt(d)
+    if dropout_p > 0.0 and dropout_seed is None:
+        dropout_seed = next_dropout_seed(qkv.device)
+    cos = sin = pos_q = pos_k = None
+    interleaved = False
+    if rotary is not None:
+        cos, sin, pos_q, pos_k = rotary
+        interleaved = _fused_rotary_kind(cos, sin, d, qkv.dtype)
+        assert pos_q.dtype == torch.int64 and pos_q.is_contiguous() and pos_q.numel() == qkv.shape[0]
+        assert pos_k.dtype == torch.int64 and pos_k.is_contiguous() and pos_k.numel() == qkv.shape[0]
+    p, seed = _dropout_args((dropout_p, dropout_seed if dropout_seed is not None else 0))
+    return _lib.host().attention_qkv(qkv, cu_seqlens_q, cu_seqlens_k, bool(causal), float(softmax_scale), p, seed, cos, sin, pos_q, pos_k, interleaved)
 
 
 # ------------------------------------------------------------------------------------------------

@@ -1,0 +1,95 @@
+"""Fused launches of the layer step against the separate launches they replace: residual add + norm (forward and
+backward), the packed-QKV attention node, column sums."""
+
+import pytest
+import torch
+
+from scaling_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# one per tiling of the norm kernels: 16 and 64 lanes a row, wide rows of one and two vectors per thread at each width
+@pytest.mark.parametrize("rows,hidden", [(1, 64), (7, 264), (257, 1024), (1025, 2048), (300, 4096), (33, 8192), (5, 12288)])
+@pytest.mark.parametrize("layer_norm", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_residual_through_the_norm_matches_separate_launches(rows, hidden, layer_norm, dtype):
+    if dtype == torch.float32:
+        hidden = min(hidden, 8192)           # the widest float32 row the norms take
+    print(f"case add_norm rows={rows} hidden={hidden} layer_norm={layer_norm} dtype={dtype}", flush=True)
+    g = torch.Generator().manual_seed(rows + hidden)
+    x, r, dy, ds = (torch.randn(rows, hidden, generator=g).to(dtype).to(DEV) for _ in range(4))
+    w, b = ((k + 0.1 * torch.randn(hidden, generator=g)).to(dtype).to(DEV) for k in (1.0, 0.0))
+    b = b if layer_norm else None
+
+    def separate(with_residual):
+        a, c, wt = x.clone().requires_grad_(), r.clone().requires_grad_(), w.clone().requires_grad_()
+        bt = b.clone().requires_grad_() if b is not None else None
+        s = a + c if with_residual else a
+        y = ops.layer_norm(s, wt, bt, 1e-5) if layer_norm else ops.rms_norm(s, wt, 1e-5)
+        torch.autograd.backward([s * 1.0, y], [ds, dy])
+        return [s.detach(), y.detach(), a.grad, c.grad, wt.grad, bt.grad if bt is not None else None]
+
+    def fused(with_residual):
+        a, c, wt = x.clone().requires_grad_(), r.clone().requires_grad_(), w.clone().requires_grad_()
+        bt = b.clone().requires_grad_() if b is not None else None
+        s, y = ops.add_norm(a, c if with_residual else None, wt, bt, 1e-5, layer_norm)
+        torch.autograd.backward([s, y], [ds, dy])
+        return [s.detach(), y.detach(), a.grad, c.grad, wt.grad, bt.grad if bt is not None else None]
+
+    for with_residual in (True, False):
+        for name, want, got in zip(("sum", "y", "dx", "dresidual", "dw", "db"), separate(with_residual), fused(with_residual)):
+            # the same arithmetic in the same order: the same bits
+            assert (want is None and got is None) or torch.equal(want, got), (name, with_residual)
+
+
+def test_norm_outputs_that_do_not_reach_the_loss():
+    x = torch.randn(9, 128, device=DEV, requires_grad=True)
+    w = torch.ones(128, device=DEV, requires_grad=True)
+    s, y = ops.add_norm(x, None, w, None, 1e-5, False)
+    s.sum().backward()
+    assert torch.equal(x.grad, torch.ones_like(x)) and w.grad is None
+    x.grad = None
+    s, y = ops.add_norm(x, x, w, None, 1e-5, False)          # both addends are the same tensor
+    y.sum().backward()
+    a = x.detach().clone().requires_grad_()
+    ops.rms_norm(a + a, w.detach(), 1e-5).sum().backward()
+    assert torch.equal(x.grad, a.grad)
+
+
+@pytest.mark.parametrize("heads,d,rotary,causal,docs", [(3, 64, True, True, (40,)), (2, 128, True, False, ()), (2, 96, False, True, (7, 100)), (4, 32, False, True, ())])
+def test_packed_qkv_attention_matches_three_slices(heads, d, rotary, causal, docs):
+    print(f"case attention_qkv heads={heads} d={d} rotary={rotary}", flush=True)
+    tokens = 150
+    g = torch.Generator().manual_seed(d)
+    qkv = torch.randn(tokens, heads, 3 * d, generator=g).bfloat16().to(DEV)
+    do = torch.randn(tokens, heads, d, generator=g).bfloat16().to(DEV)
+    cu = torch.tensor([0, *docs, tokens], dtype=torch.int32, device=DEV)
+    rot = None
+    if rotary:
+        ang = torch.outer(torch.arange(tokens).float(), 1.0 / 10000 ** (torch.arange(0, d, 2).float() / d))
+        ang = torch.cat((ang, ang), -1)
+        pos = torch.arange(tokens, device=DEV)
+        rot = (ang.cos().bfloat16().to(DEV), ang.sin().bfloat16().to(DEV), pos, pos)
+    a = qkv.clone().requires_grad_()
+    o = ops.attention(a[..., :d], a[..., d:2 * d], a[..., 2 * d:], cu, None, causal, rotary=rot)
+    o.backward(do)
+    b = qkv.clone().requires_grad_()
+    o2 = ops.attention_qkv(b, cu, None, causal, rotary=rot)
+    o2.backward(do)
+    assert torch.equal(o, o2) and torch.equal(a.grad, b.grad)
+
+
+@pytest.mark.parametrize("rows,cols,stride", [(1, 8, 8), (63, 72, 80), (512, 64, 64), (513, 136, 136), (4084, 1024, 3072)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_column_sum(rows, cols, stride, dtype):
+    """Rows fewer than the row groups of a workgroup, one whole prefetch round, and remainders of both axes; the bound is one
+    rounding of the result plus rows fp32 additions."""
+    x = torch.randn(rows, stride, generator=torch.Generator().manual_seed(rows)).to(dtype).to(DEV)
+    out = torch.empty(cols, dtype=dtype, device=DEV)
+    _lib.check(_lib.load().mi_column_sum(x.data_ptr(), stride, rows, cols, out.data_ptr(), _lib.dtype_code(dtype), _lib.stream_ptr()), "mi_column_sum")
+    xd = x[:, :cols].double()
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    bound = u * xd.sum(0).abs() + (rows + 1) * 2.0 ** -24 * xd.abs().sum(0) + 2.0 ** -25
+    assert bool(((out.double() - xd.sum(0)).abs() <= bound).all())
