@@ -40,8 +40,16 @@ def test_residual_through_the_norm_matches_separate_launches(rows, hidden, layer
 
     for with_residual in (True, False):
         for name, want, got in zip(("sum", "y", "dx", "dresidual", "dw", "db"), separate(with_residual), fused(with_residual)):
-            # the same arithmetic in the same order: the same bits
-            assert (want is None and got is None) or torch.equal(want, got), (name, with_residual)
+            assert (want is None) == (got is None), name
+            if want is None:
+                continue
+            if dtype == torch.float32 and name in ("dx", "dresidual"):
+                # the compiler contracts the norm's last multiplication with the added gradient: the fused result lacks the
+                # rounding of the norm's dx (half an ulp of it), and each side rounds its own sum (half an ulp each)
+                bound = 2.0 ** -24 * (1.01 * (want - ds).abs() + 2.01 * want.abs()) + 2.0 ** -126
+                assert bool(((want - got).abs() <= bound).all()), (name, with_residual)
+            else:                            # the same arithmetic in the same order: the same bits
+                assert torch.equal(want, got), (name, with_residual)
 
 
 def test_norm_outputs_that_do_not_reach_the_loss():
