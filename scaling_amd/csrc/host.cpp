@@ -173,6 +173,7 @@ struct AddNorm : Function<AddNorm> {
         } else {
             check(mi_rmsnorm_fwd(ptr(x), ptr(w), ptr(y), nullptr, rows, hidden, (float)eps, code_of(x), l.stream), "mi_rmsnorm_fwd");
         }
+        ctx->set_materialize_grads(false);                 // an output that does not reach the loss costs nothing
         ctx->save_for_backward({sum, w_, stats});
         ctx->saved_data["eps"] = eps;
         ctx->saved_data["layer_norm"] = layer_norm;
@@ -409,6 +410,7 @@ struct Projections : Function<Projections> {
             }
             if (residual.has_value()) out[0].add_(*residual);
         }
+        ctx->set_materialize_grads(false);
         ctx->save_for_backward(saved);
         ctx->saved_data["x_shape"] = x.sizes().vec();
         ctx->saved_data["residual"] = residual.has_value();
