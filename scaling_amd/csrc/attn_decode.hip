@@ -7,9 +7,10 @@
 //                                   memory in operand layout, B = Q^T (heads of the group, zero padded)
 //     online softmax over keys      the lane's column is a head; 8 in-lane keys + 2 lane exchanges
 //     O^T[d][head]   += V^T * P^T   A = V^T read from a transposed per-wavefront LDS copy of the chunk
-// Partial (max, sum, O) per split go to a workspace and are merged by a second kernel.
-// A small first kernel appends the new K/V row in place (instead of the reference's torch.cat) and
-// applies rotary to it; the query is rotated while its fragments are loaded.
+// Partial (max, sum, O) per split go to a workspace and are merged by a second kernel (none with a single split).
+// The wavefront whose keys include the new token first appends the new K/V row in place (instead of the
+// reference's torch.cat), rotated, and then reads it back with the rest of its chunk; the query is rotated while its
+// fragments are loaded.  (A launch of its own for the append took 3 - 5 us: a third of a step at batch 1.)
 #include "attn_common.h"
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
@@ -42,27 +43,21 @@ __device__ __forceinline__ f32x4v mfma_16x16x32(elem8_t a, elem8_t b, f32x4v c) 
 #endif
 }
 
-// ---- in-place append of the new K/V row (optionally rotated) -------------------------------------
+// ---- in-place append of the new K/V row (optionally rotated) by one wavefront -------------------------
 template <int D>
-__global__ void decode_append_kernel(const DecodeParams p) {
-    // one thread per (batch, kv head, 8-feature vector of the first half)
-    constexpr int HV = D / 16;
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= p.batch * p.nkv * HV) return;
-    const int c = idx % HV, kvh = (idx / HV) % p.nkv, b = idx / (HV * p.nkv);
-    const int ctx = p.ctx_len[b];
-    if (ctx < 1 || ctx > p.max_ctx) return;
+__device__ __forceinline__ void append_row(const DecodeParams& p, int b, int kvh, int ctx, int lane) {
+    // one lane per 8-feature vector of the first half
+    if (lane >= D / 16) return;
+    const int c = lane;
     const int64_t src = (int64_t)b * p.kn_sb + (int64_t)kvh * D + 8 * c;
     const int64_t src_v = (int64_t)b * p.vn_sb + (int64_t)kvh * D + 8 * c;
     const int64_t dst = (int64_t)b * p.c_sb + (int64_t)(ctx - 1) * p.c_st + (int64_t)kvh * p.c_sh + 8 * c;
-    uint4 lo = *reinterpret_cast<const uint4*>(p.k_new + src);
-    uint4 hi = *reinterpret_cast<const uint4*>(p.k_new + src + D / 2);
+    uint4 lo = ld128(p.k_new + src), hi = ld128(p.k_new + src + D / 2);
+    const uint4 vlo = ld128(p.v_new + src_v), vhi = ld128(p.v_new + src_v + D / 2);
     if (p.cos != nullptr) {
         int64_t pos = p.pos[b];
         pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
-        const uint4 cv = *reinterpret_cast<const uint4*>(p.cos + pos * D + 8 * c);
-        const uint4 sv = *reinterpret_cast<const uint4*>(p.sin + pos * D + 8 * c);
-        rotate_pair(lo, hi, cv, sv, 1.0f);
+        rotate_pair(lo, hi, ld128(p.cos + pos * D + 8 * c), ld128(p.sin + pos * D + 8 * c), 1.0f);
     } else if (p.cos32 != nullptr) {
         int64_t pos = p.pos[b];
         pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
@@ -71,10 +66,10 @@ __global__ void decode_append_kernel(const DecodeParams p) {
         rotate_interleaved(lo, ld128(cr), ld128(sr), 1.0f);
         rotate_interleaved(hi, ld128(cr + D / 4), ld128(sr + D / 4), 1.0f);
     }
-    *reinterpret_cast<uint4*>(p.kc + dst) = lo;
-    *reinterpret_cast<uint4*>(p.kc + dst + D / 2) = hi;
-    *reinterpret_cast<uint4*>(p.vc + dst) = *reinterpret_cast<const uint4*>(p.v_new + src_v);
-    *reinterpret_cast<uint4*>(p.vc + dst + D / 2) = *reinterpret_cast<const uint4*>(p.v_new + src_v + D / 2);
+    st128(p.kc + dst, lo);
+    st128(p.kc + dst + D / 2, hi);
+    st128(p.vc + dst, vlo);
+    st128(p.vc + dst + D / 2, vhi);
 }
 
 // ---- split kernel ----------------------------------------------------------------------------------
@@ -96,7 +91,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     __shared__ float wo_lds[NWV][16][D + 1];
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, l16 = lane & 15, G = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, G = lane >> 4;
 
     const int split = blockIdx.x % p.n_splits;
     const int kv_hc = (blockIdx.x / p.n_splits) % (p.nkv * p.n_hc);
@@ -108,6 +103,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     const int n_heads = min(16, p.n_rep - 16 * hc);
 
     int ctx = p.ctx_len[b];
+    const bool append = p.k_new != nullptr && ctx >= 1 && ctx <= p.max_ctx;
     ctx = ctx < 0 ? 0 : (ctx > p.max_ctx ? p.max_ctx : ctx);
     // keys of this split: [s0, s1), split length rounded up to whole workgroup iterations
     int per = (ctx + p.n_splits - 1) / p.n_splits;
@@ -115,6 +111,13 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     const int s0 = split * per;
     const int s1 = min(ctx, s0 + per);
     const int n_iter = s1 > s0 ? (s1 - s0 + NWV * kChunk - 1) / (NWV * kChunk) : 0;
+
+    // The last key of this split is the new token: the wavefront whose chunk (iteration it_new) holds it writes it now and waits
+    // for its own stores before that chunk is requested.  (Groups of more than 16 heads: each of their workgroups does,
+    // with the same bytes, since each reads the row.)
+    const int c_new = (ctx - 1 - s0) / kChunk;
+    const int it_new = append && ctx - 1 >= s0 && ctx - 1 < s1 && c_new % NWV == wave ? c_new / NWV : -1;   // wave-uniform
+    if (it_new >= 0) append_row<D>(p, b, kvh, ctx, lane);
 
     // Q^T fragments: column = head slot l16 (valid when < n_rep), contraction = features 32*ks + 8*G + i
     elem8_t qf[KS];
@@ -170,6 +173,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     auto load_chunk = [&](ChunkRegs& c, int it) {
         const int key0 = s0 + (NWV * it + wave) * kChunk;
         if (key0 >= s1) return;
+        if (it == it_new) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the appended row is in the cache
         const int last = s1 - 1;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -299,33 +303,53 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 }
 
 // ---- merge of the splits ------------------------------------------------------------------------------
+// One thread per (batch, head, two features), its partial results requested eight splits at a time before the first is
+// used: a launch of 16 splits is two latencies, not sixteen.  (With the append's launch gone as well, batch 1 over a cache of
+// 1,024: 21.5 -> 11.2 us for a call; batch 32: 83.8 -> 81.6.)
 template <int D>
-__global__ void decode_merge_kernel(const DecodeParams p) {
-    // one thread per (batch, head, feature)
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)p.batch * p.nq * D) return;
-    const int d = (int)(idx % D);
-    const int64_t bh = idx / D;
-    float M = -INFINITY;
-    for (int s = 0; s < p.n_splits; ++s) M = fmaxf(M, p.ws_ml[(bh * p.n_splits + s) * 2]);
-    float L = 0.f, O = 0.f;
-    for (int s = 0; s < p.n_splits; ++s) {
-        const float m = p.ws_ml[(bh * p.n_splits + s) * 2];
-        const float f = m == -INFINITY ? 0.f : fast_exp2(m - M);
-        L += f * p.ws_ml[(bh * p.n_splits + s) * 2 + 1];
-        O += f * p.ws_o[(bh * p.n_splits + s) * D + d];
+__global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeParams p) {
+    constexpr int kDepth = 8;
+    const int64_t bh = (int64_t)blockIdx.x * (128 / D > 0 ? 128 / D : 1) + (2 * threadIdx.x) / D;
+    const int d = (2 * threadIdx.x) % D;
+    if (2 * threadIdx.x >= (128 / D > 0 ? 128 / D : 1) * D || bh >= (int64_t)p.batch * p.nq) return;
+    const float* ml = p.ws_ml + bh * p.n_splits * 2;
+    const float* wo = p.ws_o + bh * p.n_splits * D + d;
+    float M = -INFINITY, L = 0.f, O0 = 0.f, O1 = 0.f;
+    for (int s0 = 0; s0 < p.n_splits; s0 += kDepth) {
+        float2 mls[kDepth], os[kDepth];
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) {                 // past the last split: its values again, with no weight below
+            const int s = min(s0 + i, p.n_splits - 1);
+            mls[i] = *reinterpret_cast<const float2*>(ml + 2 * s);
+            os[i] = *reinterpret_cast<const float2*>(wo + (int64_t)s * D);
+        }
+        float m = M;
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) m = fmaxf(m, mls[i].x);
+        const float a = M == -INFINITY ? 0.f : fast_exp2(M - m);
+        L *= a; O0 *= a; O1 *= a;
+        M = m;
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) {
+            const float f = s0 + i >= p.n_splits || mls[i].x == -INFINITY ? 0.f : fast_exp2(mls[i].x - M);
+            L += f * mls[i].y;
+            O0 += f * os[i].x;
+            O1 += f * os[i].y;
+        }
     }
-    p.o[bh * D + d] = (elem_t)(L > 0.f ? O / L : 0.f);
+    *reinterpret_cast<uint32_t*>(p.o + bh * D + d) = pack_elem2(L > 0.f ? O0 / L : 0.f, L > 0.f ? O1 / L : 0.f);
 }
 
 // 8-wavefront workgroups (one per compute unit) once there is a (batch, KV head) pair for most of the 256
-// compute units: then one split does and the merge kernel is not launched; otherwise 4-wavefront workgroups
-// and enough splits for about two workgroups per compute unit.
-bool wide_blocks(int batch, int nkv) { return (int64_t)batch * nkv >= 192; }
+// compute units, or when the whole cache is one 32-key chunk per wavefront or less: then one split does and the merge
+// kernel is not launched; otherwise 4-wavefront workgroups and enough splits for about one workgroup per compute unit.
+// One split / split and merge, microseconds, batch 1 with 32 query heads on 8, d 128: 6.1 / 6.8 with a cache of 256 tokens and
+// 8.7 / 6.8 with 512; batch 8: 6.2 / 7.0 and 10.3 / 7.3; batch 3, 16 heads on 4, d 64: 4.4 / 5.5 and 5.6 / 5.5.
+bool wide_blocks(int batch, int nkv, int max_ctx) { return (int64_t)batch * nkv >= 192 || max_ctx <= 8 * kChunk; }
 
 int choose_splits(int batch, int nkv, int max_ctx) {
     const int64_t pairs = (int64_t)batch * nkv;
-    if (wide_blocks(batch, nkv)) return 1;
+    if (wide_blocks(batch, nkv, max_ctx)) return 1;
     // one workgroup per compute unit: measured best or within a few percent of it for batch 1 - 16 at contexts
     // of 1k - 16k (two per compute unit, the earlier choice, cost 5 - 10 % in merge work at batch 4 - 16)
     int64_t s = (256 + pairs - 1) / pairs;
@@ -348,17 +372,12 @@ template <int D, int NWV> int launch_split(const DecodeParams& p, int rot, hipSt
     return mi_check_launch("decode_split");
 }
 
-template <int D> int launch_decode(const DecodeParams& p, bool append, int rot, hipStream_t st) {
-    if (append) {
-        const int n = p.batch * p.nkv * (D / 16);
-        decode_append_kernel<D><<<dim3((n + 127) / 128), dim3(128), 0, st>>>(p);
-        int rc = mi_check_launch("decode_append");
-        if (rc != MI_OK) return rc;
-    }
-    const int rc = wide_blocks(p.batch, p.nkv * p.n_hc) ? launch_split<D, 8>(p, rot, st) : launch_split<D, 4>(p, rot, st);
+template <int D> int launch_decode(const DecodeParams& p, int rot, hipStream_t st) {
+    const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8>(p, rot, st) : launch_split<D, 4>(p, rot, st);
     if (rc != MI_OK || p.n_splits == 1) return rc;
-    const int64_t n = (int64_t)p.batch * p.nq * D;
-    decode_merge_kernel<D><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(p);
+    constexpr int kRows = 128 / D > 0 ? 128 / D : 1;
+    const int64_t n = (int64_t)p.batch * p.nq;
+    decode_merge_kernel<D><<<dim3((unsigned)((n + kRows - 1) / kRows)), dim3(64), 0, st>>>(p);
     return mi_check_launch("decode_merge");
 }
 
@@ -433,10 +452,10 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
     hipStream_t st = (hipStream_t)a->stream;
     const int rot_mode = rot ? (a->rotary_interleaved ? 2 : 1) : 0;
     switch (a->head_dim) {
-        case 32: return launch_decode<32>(p, a->k_new != nullptr, rot_mode, st);
-        case 64: return launch_decode<64>(p, a->k_new != nullptr, rot_mode, st);
-        case 96: return launch_decode<96>(p, a->k_new != nullptr, rot_mode, st);
-        default: return launch_decode<128>(p, a->k_new != nullptr, rot_mode, st);
+        case 32: return launch_decode<32>(p, rot_mode, st);
+        case 64: return launch_decode<64>(p, rot_mode, st);
+        case 96: return launch_decode<96>(p, rot_mode, st);
+        default: return launch_decode<128>(p, rot_mode, st);
     }
 }
 }  // namespace

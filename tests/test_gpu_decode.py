@@ -212,3 +212,30 @@ def test_decode_float16_parity(B, nq, nkv, d, max_ctx, lens):
     assert out.dtype == torch.float16
     check("decode.f16.o", out, ref, ref_o, kind="decode")
     assert torch.equal(kcd.cpu(), kc_ref) and torch.equal(vcd.cpu(), vc_ref)
+
+
+@pytest.mark.parametrize("B,nq,nkv,d,max_ctx,n_splits", [
+    # one split up to a cache of 256 tokens, then several; the new token first or last of a 32-key chunk, or alone in its split
+    (5, 4, 2, 128, 256, 0), (5, 4, 2, 128, 257, 0), (5, 4, 2, 32, 700, 0), (5, 8, 2, 64, 700, 3), (5, 4, 2, 96, 1300, 11),
+    (5, 32, 1, 64, 300, 2),         # two workgroups share a KV head and its new row
+])
+def test_decode_append_at_chunk_and_split_edges(B, nq, nkv, d, max_ctx, n_splits):
+    """The wavefront that owns the new key writes it and reads it back: the same as with the row already in the cache."""
+    print(f"case decode append edges B={B} nq={nq} nkv={nkv} d={d} max_ctx={max_ctx} splits={n_splits}", flush=True)
+    g = torch.Generator().manual_seed(max_ctx + d)
+    lens = [1, 32, 129, max_ctx - 1, max_ctx]
+    q = torch.randn(B, nq, d, generator=g).bfloat16()
+    kc, vc = (torch.randn(B, max_ctx, nkv, d, generator=g).bfloat16() for _ in range(2))
+    k_new, v_new = (torch.randn(B, nkv, d, generator=g).bfloat16() for _ in range(2))
+    ctx = torch.tensor(lens, dtype=torch.int32)
+    kc_ref, vc_ref = kc.clone(), vc.clone()
+    for b in range(B):
+        kc_ref[b, lens[b] - 1], vc_ref[b, lens[b] - 1] = k_new[b], v_new[b]
+    scale = 1 / math.sqrt(d)
+    kcd, vcd = kc.to(DEV), vc.to(DEV)
+    out = ops.decode_attention(q.to(DEV), kcd, vcd, ctx.to(DEV), k_new.to(DEV), v_new.to(DEV), softmax_scale=scale, n_splits=n_splits)
+    present = ops.decode_attention(q.to(DEV), kc_ref.to(DEV), vc_ref.to(DEV), ctx.to(DEV), softmax_scale=scale, n_splits=n_splits)
+    torch.cuda.synchronize()
+    check("decode.o(append edges)", out, _oracle_decode(q, kc_ref, vc_ref, ctx, scale, torch.float32),
+          _oracle_decode(q, kc_ref, vc_ref, ctx, scale, torch.bfloat16), kind="decode")
+    assert torch.equal(out, present) and torch.equal(kcd.cpu(), kc_ref) and torch.equal(vcd.cpu(), vc_ref)
