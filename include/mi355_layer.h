@@ -173,6 +173,25 @@ int mi_gelu_bwd(const void* x, const void* dy, void* dx, int64_t n_elem, int dty
 int mi_cross_entropy(const void* logits, const int64_t* targets, const float* row_scale, float* losses, float* lse,
                      int32_t* argmax, void* dlogits, int64_t n_rows, int64_t vocab, int64_t logits_row_stride,
                      int64_t dlogits_row_stride, int dtype, void* stream);
+/* The same with the gradient in place, for logits whose rows own the memory up to row_stride: the elements between vocab
+ * and the next whole 16-byte vector may be overwritten (with zeros), which lets a ragged vocabulary take the single-launch
+ * kernel.  `lse` as above. */
+int mi_cross_entropy_padded(void* logits, const int64_t* targets, const float* row_scale, float* losses, float* lse, int32_t* argmax,
+                            int64_t n_rows, int64_t vocab, int64_t row_stride, int dtype, void* stream);
+/* The weighted mean of cross_entropy.py:30 and the accuracy of :81-86 in one launch:
+ *   loss = sum(losses * weights) / sum(weights),  total = sum(weights),
+ *   accuracy = share of the rows with weights > 0 whose argmax is the target
+ * and its gradient with respect to the logits, from the lse that the forward pass wrote:
+ *   dlogits[r][i] = weights[r] * (*grad / *total) * (exp(x_i - lse) - [i == t])
+ * mi_loss_row_scale: row_scale[r] = weights[r] / sum(weights).  mi_scale_inplace: x *= *scale, without touching memory when
+ * *scale is 1.  One workgroup does each of the two sums: for up to some ten thousand rows. */
+int mi_loss_reduce(const float* losses, const int32_t* argmax, const int64_t* targets, const float* weights, int64_t n_rows,
+                   float* loss, float* total, float* accuracy, void* stream);
+int mi_cross_entropy_mean_grad(const void* logits, const int64_t* targets, const float* lse, const float* weights, const float* grad,
+                               const float* total, void* dlogits, int64_t n_rows, int64_t vocab, int64_t logits_row_stride,
+                               int64_t dlogits_row_stride, int dtype, void* stream);
+int mi_loss_row_scale(const float* weights, int64_t n_rows, float* row_scale, void* stream);
+int mi_scale_inplace(void* x, int64_t n_elem, const float* scale, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * SwiGLU activation.  Replaces core/nn/mlp.py:248-249:  out = silu(a) * gate, elementwise over

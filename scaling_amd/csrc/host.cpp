@@ -10,6 +10,7 @@
 // small_product for the line between the two.
 #include <torch/extension.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <ATen/autocast_mode.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
@@ -720,6 +721,143 @@ Tensor op_attention_qkv(const Tensor& qkv, const Tensor& cu_q, const OptTensor& 
     return AttentionQkv::apply(qkv, cu_q, cu_k, &o, at::GradMode::is_enabled() && qkv.requires_grad());
 }
 
+// ---- loss --------------------------------------------------------------------------------------------------------------
+// Weighted mean of the cross entropy of logits [rows, vocab], and the accuracy.  The gradient takes the log-sum-exp of the forward
+// pass, so it reads the logits once.
+struct WeightedCrossEntropy : Function<WeightedCrossEntropy> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, const Tensor& weights) {
+        Launch l(logits);
+        const int64_t n = logits.size(0), vocab = logits.size(1);
+        const auto f32 = logits.options().dtype(at::kFloat);
+        const Tensor rows = at::empty({2, n}, f32), argmax = at::empty({n}, f32.dtype(at::kInt));
+        const Tensor loss = at::empty({}, f32), total = at::empty({}, f32), accuracy = at::empty({}, f32);
+        float *losses = rows.data_ptr<float>(), *lse = losses + n;
+        check(mi_cross_entropy(ptr(logits), targets.data_ptr<int64_t>(), nullptr, losses, lse, argmax.data_ptr<int32_t>(), nullptr, n, vocab,
+                               logits.stride(0), 0, code_of(logits), l.stream),
+              "mi_cross_entropy");
+        check(mi_loss_reduce(losses, argmax.data_ptr<int32_t>(), targets.data_ptr<int64_t>(), weights.data_ptr<float>(), n, loss.data_ptr<float>(),
+                             total.data_ptr<float>(), accuracy.data_ptr<float>(), l.stream),
+              "mi_loss_reduce");
+        ctx->set_materialize_grads(false);
+        ctx->mark_non_differentiable({accuracy});
+        ctx->save_for_backward({logits, targets, weights, rows, total});
+        return {loss, accuracy};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+        const auto saved = ctx->get_saved_variables();
+        const Tensor& logits = saved[0];
+        Launch l(logits);
+        const Tensor dloss = g[0].contiguous(), dlogits = at::empty_like(logits);
+        const int64_t n = logits.size(0);
+        check(mi_cross_entropy_mean_grad(ptr(logits), saved[1].data_ptr<int64_t>(), saved[3].data_ptr<float>() + n, saved[2].data_ptr<float>(),
+                                         dloss.data_ptr<float>(), saved[4].data_ptr<float>(), ptr(dlogits), n, logits.size(1), logits.stride(0),
+                                         dlogits.stride(0), code_of(logits), l.stream),
+              "mi_cross_entropy_mean_grad");
+        return {dlogits, Tensor(), Tensor()};
+    }
+};
+
+std::tuple<Tensor, Tensor> op_weighted_cross_entropy(const Tensor& logits, const Tensor& targets, const Tensor& weights) {
+    need_gpu(logits); need_gpu(targets); need_gpu(weights);
+    TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1 && targets.scalar_type() == at::kLong && targets.is_contiguous() &&
+                    targets.numel() == logits.size(0) && weights.scalar_type() == at::kFloat && weights.is_contiguous() &&
+                    weights.numel() == logits.size(0),
+                "cross entropy: logits [rows, vocab], one int64 target and one float32 weight per row");
+    const auto out = WeightedCrossEntropy::apply(logits, targets, weights);
+    return {out[0], out[1]};
+}
+
+// LM head and weighted mean loss, chunk by chunk: a chunk's logits become their gradient in place and are folded into dh and dW at
+// once, so the gradients exist when the forward pass ends and the backward pass only scales them.
+struct LinearCrossEntropy : Function<LinearCrossEntropy> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& h, const Tensor& weight, const Tensor& targets, const Tensor& weights, int64_t chunk,
+                                 bool need_dh, bool need_dw) {
+        Launch l(h);
+        const int64_t n = h.size(0), vocab = weight.size(0);
+        const auto f32 = h.options().dtype(at::kFloat);
+        const Tensor rows = at::empty({3, n}, f32), argmax = at::empty({n}, f32.dtype(at::kInt));
+        const Tensor loss = at::empty({}, f32), total = at::empty({}, f32), accuracy = at::empty({}, f32);
+        float *losses = rows.data_ptr<float>(), *lse = losses + n, *row_scale = lse + n;
+        const bool grad = need_dh || need_dw;
+        if (grad) check(mi_loss_row_scale(weights.data_ptr<float>(), n, row_scale, l.stream), "mi_loss_row_scale");
+        Tensor dh = need_dh ? at::empty_like(h) : Tensor(), dw;       // dw: one chunk: the product itself; several: their sum in fp32
+        // Rows of the logits start on 128-byte boundaries (16-bit types) whatever the vocabulary: the library's three products of
+        // 2047 x 50257 x 1024 take 776 us with a stride of 50304 and 846 with 50257, and the loss kernel reads and writes
+        // whole vectors.
+        const int64_t ld = (vocab + 63) / 64 * 64;
+        const Tensor buffer = at::empty({std::min(n, chunk), ld}, h.options()), wt = weight.t();
+        for (int64_t r0 = 0; r0 < n; r0 += chunk) {
+            const int64_t r = std::min(n - r0, chunk);
+            const Tensor hc = h.narrow(0, r0, r);
+            Tensor logits = buffer.narrow(0, 0, r).narrow(1, 0, vocab);
+            at::mm_out(logits, hc, wt);
+            const int64_t* t = targets.data_ptr<int64_t>() + r0;
+            if (grad)
+                check(mi_cross_entropy_padded(ptr(logits), t, row_scale + r0, losses + r0, lse + r0, argmax.data_ptr<int32_t>() + r0, r, vocab, ld,
+                                              code_of(h), l.stream),
+                      "mi_cross_entropy_padded");
+            else
+                check(mi_cross_entropy(ptr(logits), t, nullptr, losses + r0, nullptr, argmax.data_ptr<int32_t>() + r0, nullptr, r, vocab, ld, 0, code_of(h),
+                                       l.stream),
+                      "mi_cross_entropy");
+            if (need_dh) {
+                Tensor out = dh.narrow(0, r0, r);
+                at::mm_out(out, logits, weight);
+            }
+            if (need_dw) {
+                const Tensor product = at::mm(logits.t(), hc);
+                if (n <= chunk) dw = product;
+                else if (!dw.defined()) dw = product.to(at::kFloat);
+                else dw.add_(product);
+            }
+        }
+        if (need_dw && !dw.defined()) dw = at::zeros_like(weight);    // no rows
+        check(mi_loss_reduce(losses, argmax.data_ptr<int32_t>(), targets.data_ptr<int64_t>(), weights.data_ptr<float>(), n, loss.data_ptr<float>(),
+                             total.data_ptr<float>(), accuracy.data_ptr<float>(), l.stream),
+              "mi_loss_reduce");
+        ctx->set_materialize_grads(false);
+        ctx->mark_non_differentiable({argmax, accuracy});
+        ctx->save_for_backward({dh, dw});
+        ctx->saved_data["dtype"] = (int64_t)weight.scalar_type();
+        return {loss, argmax, accuracy};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        variable_list grads(7);
+        if (!g[0].defined()) return grads;
+        const auto saved = ctx->get_saved_variables();
+        // A graph that is used up by this pass hands its gradients over, scaled in place; one that is kept (or differentiated
+        // further) keeps them.
+        const bool hand_over = !torch::autograd::get_current_graph_task_keep_graph() && !at::GradMode::is_enabled();
+        const Tensor dloss = g[0].contiguous();
+        for (int i = 0; i < 2; ++i) {
+            const Tensor& x = saved[i];
+            if (!x.defined()) continue;
+            if (hand_over && x.is_non_overlapping_and_dense()) {
+                Launch l(x);
+                check(mi_scale_inplace(ptr(x), x.numel(), dloss.data_ptr<float>(), code_of(x), l.stream), "mi_scale_inplace");
+                grads[i] = x;
+            } else {
+                grads[i] = x * dloss;
+            }
+        }
+        const auto dtype = (at::ScalarType)ctx->saved_data["dtype"].toInt();
+        if (grads[1].defined()) grads[1] = grads[1].to(dtype);
+        return grads;
+    }
+};
+
+std::tuple<Tensor, Tensor, Tensor> op_linear_cross_entropy(const Tensor& h, const Tensor& weight, const Tensor& targets, const Tensor& weights, int64_t chunk) {
+    need_gpu(h); need_gpu(weight); need_gpu(targets); need_gpu(weights);
+    TORCH_CHECK(h.dim() == 2 && h.is_contiguous() && weight.dim() == 2 && h.size(1) == weight.size(1) && h.scalar_type() == weight.scalar_type() &&
+                    targets.scalar_type() == at::kLong && targets.is_contiguous() && targets.numel() == h.size(0) &&
+                    weights.scalar_type() == at::kFloat && weights.is_contiguous() && weights.numel() == h.size(0) && chunk >= 1,
+                "linear cross entropy: h [rows, hidden], weight [vocab, hidden], one int64 target and one float32 weight per row");
+    const bool on = at::GradMode::is_enabled();
+    const auto out = LinearCrossEntropy::apply(h, weight, targets, weights, chunk, on && h.requires_grad(), on && weight.requires_grad());
+    return {out[0], out[1], out[2]};
+}
+
 // ---- decode ------------------------------------------------------------------------------------------------------------
 void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, const OptTensor& k_new,
                       const OptTensor& v_new, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos, bool interleaved, double scale,
@@ -782,5 +920,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("attention", &op_attention);
     def("attention_qkv", &op_attention_qkv);
     def("add_norm", &op_add_norm);
+    def("weighted_cross_entropy", &op_weighted_cross_entropy);
+    def("linear_cross_entropy", &op_linear_cross_entropy);
     def("decode_attention", &op_decode_attention);
 }

@@ -19,7 +19,7 @@ from ._lib import MiAttnArgs, check, dtype_code, ptr, stream_ptr
 __all__ = [
     "rms_norm", "swiglu", "rotary_embedding", "rotary_embedding_complex", "attention", "attention_forward", "attention_backward",
     "decode_attention", "rms_norm_forward", "rms_norm_backward", "swiglu_forward", "swiglu_backward",
-    "cross_entropy", "cross_entropy_forward", "linear_cross_entropy", "add_rms_norm",
+    "cross_entropy", "cross_entropy_forward", "linear_cross_entropy", "weighted_cross_entropy", "add_rms_norm",
 ]
 
 
@@ -234,49 +234,13 @@ def cross_entropy(logits: torch.Tensor, targets: torch.Tensor) -> Tuple[torch.Te
     return _CrossEntropy.apply(logits, targets.contiguous())
 
 
-class _LinearCrossEntropy(torch.autograd.Function):
-    """loss = sum_r w_r * CE(h_r W^T, t_r) / sum_r w_r without ever holding the [rows, vocab] logits: rows are
-    processed in chunks, each chunk's logits become its gradient in place and are folded into dh / dW at once."""
-
-    @staticmethod
-    def forward(ctx, h, weight, targets, loss_weights, chunk_rows):
-        n = h.shape[0]
-        w32 = loss_weights.float().contiguous()
-        total = w32.sum()
-        row_scale = (w32 / total).contiguous()
-        need_dh, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        dh = torch.empty_like(h) if need_dh else None
-        dw = None      # one chunk: the product itself; several chunks: their sum, accumulated in fp32
-        losses = torch.empty(n, dtype=torch.float32, device=h.device)
-        argmax = torch.empty(n, dtype=torch.int32, device=h.device)
-        for r0 in range(0, n, chunk_rows):
-            r1 = min(n, r0 + chunk_rows)
-            logits = torch.matmul(h[r0:r1], weight.t())                       # PyTorch GEMM, [chunk, vocab]
-            grad_buf = logits if (need_dh or need_dw) else None
-            lc, ac = cross_entropy_forward(logits, targets[r0:r1], row_scale=row_scale[r0:r1], dlogits=grad_buf)
-            losses[r0:r1] = lc
-            argmax[r0:r1] = ac
-            if need_dh:
-                torch.matmul(logits, weight, out=dh[r0:r1])
-            if need_dw:
-                prod = torch.matmul(logits.t(), h[r0:r1])
-                if n <= chunk_rows:
-                    dw = prod
-                elif dw is None:
-                    dw = prod.float()
-                else:
-                    dw.add_(prod)
-        loss = (losses * w32).sum() / total
-        ctx.save_for_backward(dh if need_dh else torch.empty(0), dw if need_dw else torch.empty(0))
-        ctx.flags = (need_dh, need_dw, weight.dtype)
-        ctx.mark_non_differentiable(argmax)
-        return loss, argmax
-
-    @staticmethod
-    def backward(ctx, dloss, _dargmax):
-        dh, dw = ctx.saved_tensors
-        need_dh, need_dw, wdtype = ctx.flags
-        return (dh * dloss.to(dh.dtype) if need_dh else None, (dw * dloss).to(wdtype) if need_dw else None, None, None, None)
+def weighted_cross_entropy(logits: torch.Tensor, targets: torch.Tensor, weights: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(loss, accuracy) of logits [rows, vocab]: loss = sum(w * CE) / sum(w), accuracy = hit rate of the row argmax among the
+    rows with w > 0; weights float32 [rows], not differentiable here.  Two launches forward, one backward."""
+    _need_cuda(logits, targets, weights)
+    if logits.stride(1) != 1:
+        logits = logits.contiguous()
+    return _lib.host().weighted_cross_entropy(logits, targets.contiguous(), weights.contiguous())
 
 
 def linear_cross_entropy(h: torch.Tensor, weight: torch.Tensor, targets: torch.Tensor, loss_weights: torch.Tensor,
@@ -287,10 +251,15 @@ def linear_cross_entropy(h: torch.Tensor, weight: torch.Tensor, targets: torch.T
     23.4 ms with one chunk, 28.4 ms with four, 39.9 ms with eight).
 
     Returns (loss, argmax int32 [rows]); the gradients of h and weight are computed in the forward pass."""
+    return _linear_cross_entropy(h, weight, targets, loss_weights, chunk_rows)[:2]
+
+
+def _linear_cross_entropy(h, weight, targets, loss_weights, chunk_rows):
+    """(loss, argmax, accuracy)"""
     _need_cuda(h, weight, targets, loss_weights)
     assert h.dim() == 2 and weight.dim() == 2 and h.shape[1] == weight.shape[1] and h.dtype == weight.dtype
-    return _LinearCrossEntropy.apply(h.contiguous(), weight, targets.contiguous().view(-1), loss_weights.contiguous().view(-1),
-                                     int(chunk_rows))
+    return _lib.host().linear_cross_entropy(h.contiguous(), weight, targets.contiguous().view(-1),
+                                            loss_weights.detach().float().contiguous().view(-1), int(chunk_rows))
 
 
 # ------------------------------------------------------------------------------------------------

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle
-from scaling_amd import ops
+from scaling_amd import _lib, ops
 from scaling_amd.config import TransformerArchitectureConfig
 from scaling_amd.layer import TransformerLayerIO
 from scaling_amd.loss import CrossEntropyLoss, TransformerLMHead
@@ -231,3 +231,85 @@ def test_cross_entropy_edge_shapes_and_errors():
         ops.cross_entropy_forward(x.to(DEV).t(), t.to(DEV))                 # vocabulary dimension not contiguous
     with pytest.raises(RuntimeError):
         ops.cross_entropy_forward(x, t)                                       # CPU tensors: there is no CPU path
+
+
+# One vocabulary per register count of the row kernel, ragged by one element either way; 73721 ends inside the last vector that is
+# staged through LDS, 73729 one vector behind it, 131071 in the last register.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1, 9, 8191, 8193, 16385, 32769, 65535, 73721, 73729, 131071])
+def test_cross_entropy_padded_rows(vocab, dtype):
+    print(f"case cross_entropy_padded vocab={vocab} dtype={dtype}", flush=True)
+    rows, ld = 259, (vocab + 63) // 64 * 64          # more rows than workgroups: some walk a second row
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    buf = torch.full((rows, ld), float("nan"), dtype=dtype, device=DEV)
+    buf[:, :vocab] = torch.randn(rows, vocab, generator=g, device=DEV) * 2
+    logits = buf[:, :vocab].double()
+    targets = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    targets[0], targets[-1] = vocab - 1, -100
+    scale = torch.rand(rows, generator=g, device=DEV)
+    losses, lse = torch.empty(2, rows, device=DEV)
+    argmax = torch.empty(rows, dtype=torch.int32, device=DEV)
+    p = _lib.ptr
+    _lib.check(_lib.load().mi_cross_entropy_padded(p(buf), p(targets), p(scale), p(losses), p(lse), p(argmax), rows, vocab, ld,
+                                                   _lib.dtype_code(dtype), _lib.stream_ptr()), "mi_cross_entropy_padded")
+    ref_lse = torch.logsumexp(logits, -1)
+    seen = targets >= 0
+    x_t = logits.gather(1, targets.clamp(min=0)[:, None])[:, 0]
+    assert torch.allclose(losses.double(), torch.where(seen, ref_lse - x_t, 0.0), rtol=1e-5, atol=2e-5)
+    assert torch.equal(logits.gather(1, argmax.long()[:, None])[:, 0], logits.max(-1).values)
+    grad = torch.softmax(logits, -1)
+    grad[torch.arange(rows, device=DEV), targets.clamp(min=0)] -= 1.0
+    grad *= (scale * seen)[:, None]
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2e-5       # one rounding to the type; fp32: exp2 of an argument rounded at |x| < 32
+    assert bool(((buf[:, :vocab].double() - grad).abs() <= eps * grad.abs() + 1e-6).all())
+    vec = 16 // buf.element_size()
+    last = (vocab + vec - 1) // vec * vec
+    if vocab % vec and vocab <= 16 * 1024 * vec:       # longer rows do not fit the registers: the general path leaves the padding alone
+        assert bool((buf[:, vocab:last] == 0).all())
+    assert bool(torch.isnan(buf[:, last:].float()).all())
+
+
+@pytest.mark.parametrize("rows,vocab,stride,offset", [(1, 1, 1, 0), (300, 1000, 1000, 0), (67, 50257, 50257, 0), (5, 1003, 1008, 3),
+                                                      (3, 140001, 140001, 0)])
+def test_weighted_cross_entropy_equals_composition(rows, vocab, stride, offset):
+    print(f"case weighted_cross_entropy rows={rows} vocab={vocab} stride={stride} offset={offset}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    store = torch.randn(rows * stride + offset, generator=g, device=DEV).bfloat16()
+    targets = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    weights = torch.rand(rows, generator=g, device=DEV) * (torch.rand(rows, generator=g, device=DEV) > 0.3)
+    weights[0] = 0.5
+    got = []
+    for fused in (True, False):
+        leaf = store.clone().requires_grad_()
+        x = leaf[offset:].view(rows, stride)[:, :vocab]
+        if fused:
+            loss, acc = ops.weighted_cross_entropy(x, targets, weights)
+        else:
+            losses, argmax = ops.cross_entropy(x, targets)
+            loss = (losses * weights).sum() / weights.sum()
+            acc = ((argmax == targets) & (weights > 0)).sum() / (weights > 0).sum()
+        (loss * 1.5).backward()
+        got.append((loss, acc, leaf.grad))
+    (l1, a1, g1), (l2, a2, g2) = got
+    assert torch.allclose(l1, l2, rtol=1e-5) and torch.allclose(a1, a2, rtol=1e-6)      # sums of `rows` terms in another order
+    # the same arithmetic up to the rounding of the scale and of exp2's argument, then one rounding to bfloat16
+    assert bool(((g1.float() - g2.float()).abs() <= 2.0 ** -7 * g2.float().abs() + 1e-9).all())
+    none = ops.weighted_cross_entropy(store[:vocab][None].expand(1, vocab), targets[:1], torch.zeros(1, device=DEV))[0]
+    assert bool(torch.isnan(none))                                                         # no weight: 0 / 0, as the composition
+
+
+@pytest.mark.parametrize("chunk", [64, 4096])
+def test_linear_cross_entropy_gradients_are_kept_with_the_graph(chunk):
+    print(f"case linear_cross_entropy kept graph chunk={chunk}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    h = torch.randn(150, 64, generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(333, 64, generator=g, device=DEV) * 0.2).bfloat16().requires_grad_()
+    t = torch.randint(0, 333, (150,), generator=g, device=DEV)
+    loss, _ = ops.linear_cross_entropy(h, w, t, torch.ones(150, device=DEV), chunk_rows=chunk)
+    one = torch.autograd.grad(loss, (h, w), retain_graph=True)
+    kept = [x.clone() for x in one]
+    for x in one:
+        x.mul_(0)                                     # the caller owns what it received
+    two = torch.autograd.grad(loss * 2.0, (h, w))     # the last pass hands the gradients over
+    for a, b in zip(kept, two):
+        assert torch.equal(a * 2, b)                  # a power of two: exact
