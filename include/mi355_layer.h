@@ -82,6 +82,32 @@ typedef struct mi_gemm_problem {
 } mi_gemm_problem;
 int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream);
 
+/* ------------------------------------------------------------------------------------------
+ * Products of up to 16 rows (a decode step) with up to three matrices [n, k] that share their input:
+ *   out_i[m][j] = sum_k X[m][k] W_i[j][k]  (+ bias_i[j])  (rounded)  (+ add_i[m][j]),   X = x, or with norm_weight
+ *   x * rsqrt(mean(x^2) + eps) * norm_weight rounded to `dtype` (core/nn/norm/rms_norm.py:47-50);
+ *   glu (two weights): out_0 = silu(X W_0^T) * (X W_1^T), each product rounded first (core/nn/mlp.py:248-249).
+ * 16-bit types, fp32 accumulation; k a multiple of 32; x, norm_weight and w 16-byte aligned with strides of whole vectors.
+ * count_up (optional): int32 [rows], each raised by one (the context lengths of a decode step).
+ * ------------------------------------------------------------------------------------------ */
+#define MI_ROWS_MAX 16
+#define MI_ROWS_MAX_WEIGHTS 3
+typedef struct mi_rows_args {
+    const void* x;
+    const void* norm_weight;       /* [k] or NULL */
+    const void* w[MI_ROWS_MAX_WEIGHTS];
+    const void* bias[MI_ROWS_MAX_WEIGHTS];
+    const void* add[MI_ROWS_MAX_WEIGHTS];
+    void* out[MI_ROWS_MAX_WEIGHTS];
+    int64_t ldx, ldw[MI_ROWS_MAX_WEIGHTS], ldadd[MI_ROWS_MAX_WEIGHTS], ldo[MI_ROWS_MAX_WEIGHTS];
+    int32_t* count_up;
+    int32_t n[MI_ROWS_MAX_WEIGHTS];
+    int32_t n_weights, rows, k, glu, dtype;
+    float eps;
+    void* stream;
+} mi_rows_args;
+int mi_rows_product(const mi_rows_args* args);
+
 /* out[c] = sum_r x[r * row_stride + c], fp32 accumulation, fixed order: the bias gradient of a projection.  n_cols and
  * row_stride multiples of 8 elements (4 for fp32), x 16-byte aligned. */
 int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int dtype, void* stream);

@@ -17,6 +17,8 @@
 //           visited in an order in which a lane's four values are consecutive)
 #include "common.h"
 
+#include <type_traits>
+
 int mi_compute_units();
 
 namespace {
@@ -269,6 +271,23 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(const Problems ps) {
     else gemm_tile<T, TILE, false, false>(pr, tm, tn, smem);
 }
 
+// Forward products of a few rows that share their input are weight reads and go to mi_rows_product (3 x 1024 x 1024 in a decode
+// step: 9.2 us here, 6.2 there).
+template <typename T> bool few_rows(const mi_gemm_problem* in, int count, mi_rows_args& r) {
+    if (sizeof(T) != 2 || count > MI_ROWS_MAX_WEIGHTS) return false;
+    r = mi_rows_args{};
+    for (int i = 0; i < count; ++i) {
+        const mi_gemm_problem& a = in[i];
+        const auto &s = a.segments[0], &s0 = in[0].segments[0];
+        if (a.n_segments != 1 || a.p_kmajor || a.q_kmajor || a.m < 1 || a.m > MI_ROWS_MAX || a.m != in[0].m || s.p != s0.p || s.ldp != s0.ldp || s.k != s0.k ||
+            s.k % 32 != 0)
+            return false;
+        r.w[i] = s.q; r.ldw[i] = s.ldq; r.bias[i] = a.bias; r.add[i] = a.add; r.ldadd[i] = a.ldadd; r.out[i] = a.c; r.ldo[i] = a.ldc; r.n[i] = a.n;
+    }
+    r.x = in[0].segments[0].p; r.ldx = in[0].segments[0].ldp; r.k = in[0].segments[0].k; r.rows = in[0].m; r.n_weights = count;
+    return true;
+}
+
 template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {
     constexpr int V = Elem<T>::kVec;
     Problems ps;
@@ -308,6 +327,12 @@ template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream
         if (total > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "gemm: too many tiles");
     }
     if (total == 0) return MI_OK;
+    mi_rows_args rows;
+    if (few_rows<T>(in, count, rows)) {                    // everything has been checked above
+        rows.dtype = std::is_same<T, __bf16>::value ? MI_BF16 : MI_F16;
+        rows.stream = st;
+        return mi_rows_product(&rows);
+    }
     if (tile == 64) gemm_kernel<T, 64><<<dim3((unsigned)total), dim3(kThreads), 0, st>>>(ps);
     else gemm_kernel<T, 32><<<dim3((unsigned)total), dim3(kThreads), 0, st>>>(ps);
     return mi_check_launch("gemm");

@@ -892,6 +892,119 @@ void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v
     check(mi_attn_decode(&a), "mi_attn_decode");
 }
 
+// ---- a decode step's layer ---------------------------------------------------------------------------------------------
+bool rows_weight(const Tensor& w, const Tensor& x, int64_t k) {
+    return w.dim() == 2 && w.size(0) > 0 && w.size(1) == k && w.scalar_type() == x.scalar_type() && w.device() == x.device() && aligned(w);
+}
+bool rows_norm(const Tensor& w, const Tensor& x, int64_t k) {
+    return w.dim() == 1 && w.size(0) == k && w.stride(0) == 1 && w.scalar_type() == x.scalar_type() && w.device() == x.device() &&
+           (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0;
+}
+bool rows_input(const Tensor& x) {                         // [rows, k]
+    return x.is_cuda() && x.dim() == 2 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(0) >= 1 &&
+           x.size(0) <= MI_ROWS_MAX && x.size(1) > 0 && x.size(1) % 32 == 0 && aligned(x);
+}
+
+mi_rows_args rows_args(const Tensor& x, const Tensor& norm, double eps, const Launch& l) {
+    mi_rows_args a{};
+    a.x = ptr(x); a.norm_weight = ptr(norm); a.ldx = x.stride(0); a.rows = (int32_t)x.size(0); a.k = (int32_t)x.size(1);
+    a.eps = (float)eps; a.dtype = code_of(x); a.stream = l.stream;
+    return a;
+}
+void rows_weight(mi_rows_args& a, const Tensor& w, void* out, int64_t ldo) {
+    const int i = a.n_weights++;
+    a.w[i] = ptr(w); a.ldw[i] = w.stride(0); a.n[i] = (int32_t)w.size(0); a.out[i] = out; a.ldo[i] = ldo;
+}
+
+// The norm in front of a product of few rows: inside the product while few workgroups repeat it (3 x 1024 -> 1536: 5.2 us where the two
+// launches take 4.1 + 2.6), a launch of its own in front of wide ones, where normalising the operand in every workgroup
+// outweighs the launch (16 x 4096 -> 28672: 84 us inside, 36 + 3 as two; 3 x 1024 -> 32000: 20 and 12.6 + 3).
+struct RowsNorm {
+    Tensor x, weight;
+    RowsNorm(const Tensor& x_, const Tensor& weight_, double eps, int64_t features, const Launch& l) : x(x_), weight(weight_) {
+        if (features <= 8192) return;
+        x = x_.is_contiguous() ? at::empty_like(x_) : at::empty(x_.sizes(), x_.options());
+        const Tensor in = x_.contiguous();
+        check(mi_rmsnorm_fwd(ptr(in), ptr(weight), ptr(x), nullptr, in.size(0), in.size(1), (float)eps, code_of(in), l.stream), "mi_rmsnorm_fwd");
+        weight = Tensor();
+    }
+};
+
+// rms_norm(x) W^T of a few rows [rows, k]; nothing where mi_rows_product does not apply.
+OptTensor op_norm_linear_rows(const Tensor& x, const Tensor& norm, double eps, const Tensor& w) {
+    if (!rows_input(x) || !rows_norm(norm, x, x.size(1)) || !rows_weight(w, x, x.size(1))) return std::nullopt;
+    need_gpu(x);
+    Launch l(x);
+    const Tensor out = at::empty({x.size(0), w.size(0)}, x.options());
+    const RowsNorm in(x, norm, eps, w.size(0), l);
+    mi_rows_args a = rows_args(in.x, in.weight, eps, l);
+    rows_weight(a, w, ptr(out), out.stride(0));
+    check(mi_rows_product(&a), "mi_rows_product");
+    return out;
+}
+
+// One token per sequence through a pre-norm layer (RMSNorm, separate q / k / v, SwiGLU, no biases): five launches, plus the merge of
+// the decode attention and the norms in front of wide products.  x [batch, 1, hidden]; raises ctx_len by one and appends to the caches.  Nothing happens, and nothing
+// is returned, where a shape, type or alignment does not suit the kernels.
+OptTensor op_decode_layer(const Tensor& x, const Tensor& pos, const Tensor& norm1, double eps1, const std::vector<Tensor>& qkv_w, const Tensor& dense,
+                          const Tensor& norm2, double eps2, const Tensor& w_in, const Tensor& w_gate, const Tensor& w_out, int64_t head_dim,
+                          const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, const Tensor& cos, const Tensor& sin, bool interleaved,
+                          double scale, const Tensor& workspace) {
+    if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous()) return std::nullopt;
+    const Tensor x2 = x.view({x.size(0), x.size(2)});
+    const int64_t b = x2.size(0), hidden = x2.size(1);
+    if (!rows_input(x2) || !rows_norm(norm1, x, hidden) || !rows_norm(norm2, x, hidden) || qkv_w.size() != 3) return std::nullopt;
+    for (const Tensor& w : qkv_w)
+        if (!rows_weight(w, x, hidden) || w.size(0) % head_dim != 0) return std::nullopt;
+    const int64_t q_rows = qkv_w[0].size(0), kv_rows = qkv_w[1].size(0), inter = w_in.size(0);
+    if (qkv_w[2].size(0) != kv_rows || q_rows % 32 != 0 || inter % 32 != 0 || !rows_weight(dense, x, q_rows) || dense.size(0) != hidden ||
+        !rows_weight(w_in, x, hidden) || !rows_weight(w_gate, x, hidden) || w_gate.size(0) != inter || !rows_weight(w_out, x, inter) ||
+        w_out.size(0) != hidden || pos.scalar_type() != at::kLong || pos.numel() != b || !pos.is_contiguous() || pos.device() != x.device() ||
+        k_cache.scalar_type() != x.scalar_type() || k_cache.size(0) != b || k_cache.size(2) * head_dim != kv_rows || k_cache.size(3) != head_dim)
+        return std::nullopt;
+    need_gpu(x);
+    Launch l(x);
+    const int64_t width = q_rows + 2 * kv_rows, e = x.element_size();
+    const Tensor qkv = at::empty({b, width}, x.options()), ctx = at::empty({b, q_rows}, x.options()), h = at::empty({b, hidden}, x.options()),
+                 act = at::empty({b, inter}, x.options()), y = at::empty(x.sizes(), x.options());
+    char* base = static_cast<char*>(ptr(qkv));
+    const RowsNorm in1(x2, norm1, eps1, width, l);
+    mi_rows_args a = rows_args(in1.x, in1.weight, eps1, l);
+    a.count_up = static_cast<int32_t*>(ptr(ctx_len));
+    rows_weight(a, qkv_w[0], base, width);
+    rows_weight(a, qkv_w[1], base + q_rows * e, width);
+    rows_weight(a, qkv_w[2], base + (q_rows + kv_rows) * e, width);
+    check(mi_rows_product(&a), "mi_rows_product");
+
+    mi_decode_args d{};
+    d.q = base; d.k_new = base + q_rows * e; d.v_new = base + (q_rows + kv_rows) * e;
+    d.q_stride_batch = d.k_new_stride_batch = d.v_new_stride_batch = width;
+    d.k_cache = ptr(k_cache); d.v_cache = ptr(v_cache); d.o = ptr(ctx); d.ctx_len = static_cast<const int32_t*>(ptr(ctx_len));
+    d.rotary_cos = ptr(cos); d.rotary_sin = ptr(sin); d.position_ids = static_cast<const int64_t*>(ptr(pos));
+    d.rotary_table_rows = cos.size(0); d.rotary_interleaved = interleaved;
+    d.batch = (int32_t)b; d.max_ctx = (int32_t)k_cache.size(1); d.n_q_heads = (int32_t)(q_rows / head_dim); d.n_kv_heads = (int32_t)(kv_rows / head_dim);
+    d.head_dim = (int32_t)head_dim; d.dtype = code_of(x);
+    d.cache_stride_batch = k_cache.stride(0); d.cache_stride_token = k_cache.stride(1); d.cache_stride_head = k_cache.stride(2);
+    d.softmax_scale = (float)scale; d.workspace = ptr(workspace); d.workspace_bytes = (size_t)workspace.numel() * 4; d.stream = l.stream;
+    check(mi_attn_decode(&d), "mi_attn_decode");
+
+    a = rows_args(ctx, Tensor(), 0.0, l);
+    rows_weight(a, dense, ptr(h), hidden);
+    a.add[0] = ptr(x2); a.ldadd[0] = hidden;
+    check(mi_rows_product(&a), "mi_rows_product");
+    const RowsNorm in2(h, norm2, eps2, 2 * inter, l);
+    a = rows_args(in2.x, in2.weight, eps2, l);
+    a.glu = 1;
+    rows_weight(a, w_in, ptr(act), inter);
+    rows_weight(a, w_gate, nullptr, 0);
+    check(mi_rows_product(&a), "mi_rows_product");
+    a = rows_args(act, Tensor(), 0.0, l);
+    rows_weight(a, w_out, ptr(y), hidden);
+    a.add[0] = ptr(h); a.ldadd[0] = hidden;
+    check(mi_rows_product(&a), "mi_rows_product");
+    return y;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -923,4 +1036,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("weighted_cross_entropy", &op_weighted_cross_entropy);
     def("linear_cross_entropy", &op_linear_cross_entropy);
     def("decode_attention", &op_decode_attention);
+    def("norm_linear_rows", &op_norm_linear_rows);
+    def("decode_layer", &op_decode_layer);
 }

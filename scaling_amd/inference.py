@@ -20,8 +20,10 @@ import torch
 
 from .config import TransformerArchitectureConfig, architecture_from_config_file
 from .data import get_cumulative_seq_lengths, get_position_ids
+from . import ops
 from .layer import InferenceSettings, LayerNormWrapper, TransformerLayer, TransformerLayerIO
 from .loss import TransformerLMHead
+from .nn import RMSNorm, _unhooked, decode_arguments
 
 # class names written by older versions of the reference (partitioned_module.py:25-32)
 LEGACY_CLASS_NAMES = {"LuminousEmbeddingInput": "EmbeddingInput", "LuminousLayer": "TransformerLayer",
@@ -130,9 +132,46 @@ class TransformerInferenceModule(torch.nn.Module):
         for layer in self._layers[1:-2]:
             x = layer(x)
         if last_token_only:
+            logits = self._last_logits(x.activations)
+            if logits is not None:
+                return logits
             x.activations = x.activations[:, -1:, :].contiguous()
         x = self._layers[-2](x)
         return self._layers[-1].linear(x.activations)
+
+    def _last_logits(self, h: torch.Tensor) -> Optional[torch.Tensor]:
+        """Logits [b, 1, vocab] of the last position through one product with the norm inside, where final norm and head are this package's, unhooked, and the
+        rows are few; else None."""
+        wrapper, linear = self._layers[-2], self._layers[-1].linear
+        if type(wrapper) is not LayerNormWrapper or type(wrapper.norm) is not RMSNorm or type(linear) is not torch.nn.Linear or linear.bias is not None \
+                or not (_unhooked(wrapper) and _unhooked(wrapper.norm) and _unhooked(linear)) or torch.is_autocast_enabled() or not h.is_cuda:
+            return None
+        logits = ops.norm_linear_rows(h[:, -1], wrapper.norm.weight, wrapper.norm.eps, linear.weight)
+        return None if logits is None else logits.unsqueeze(1)
+
+    def _native_layers(self, batch: int, tokens: int) -> Optional[list]:
+        """(cache, arguments of ops.decode_layer) per layer for the next `tokens` cached steps, or None where a layer or this module
+        is not the package's own as it is."""
+        layers = list(self._layers[1:-2])
+        if type(self).forward is not TransformerInferenceModule.forward or not layers or \
+                not all(type(layer) is TransformerLayer and _unhooked(layer) and layer._decodes_natively() for layer in layers):
+            return None
+        native = [(layer.self_attention.cache.get(0), decode_arguments(layer, batch, tokens, 0)) for layer in layers]
+        return native if all(arguments is not None for _, arguments in native) else None
+
+    def _native_step(self, native: list, token_ids: torch.Tensor, position_ids: torch.Tensor) -> Optional[torch.Tensor]:
+        """Logits [b, 1, vocab] of one token per sequence; None, with nothing done, where the kernels refuse the first layer (the layers
+        of a model have one shape)."""
+        h = self._layers[0](token_ids)
+        for i, (cache, arguments) in enumerate(native):
+            y = ops.decode_layer(h, position_ids, arguments)
+            if y is None:
+                assert i == 0, "the layers of a model have one shape"
+                return None
+            cache.length += 1
+            h = y
+        logits = self._last_logits(h)
+        return self._layers[-1].linear(self._layers[-2](TransformerLayerIO(activations=h, position_ids=None)).activations) if logits is None else logits
 
     def logits(self, input_tokens: Sequence[int]) -> torch.Tensor:
         return self.forward(torch.tensor([list(input_tokens)])).squeeze(0)
@@ -162,7 +201,6 @@ class TransformerInferenceModule(torch.nn.Module):
             att = layer.self_attention
             cache = att.cache[0]
             if cache.workspace is None:
-                from . import ops
                 cache.workspace = ops.decode_workspace(b, att.num_attention_heads, att.hidden_size_per_attention_head,
                                                        cache.max_ctx, self.device)
 
@@ -172,8 +210,6 @@ class TransformerInferenceModule(torch.nn.Module):
         for layer in layers[1:]:
             layer.self_attention.cache[0].ctx_len = shared_ctx
 
-        from .nn import RMSNorm
-        from . import ops
         final_norm = self._layers[-2].norm
         fuse_add_norm = all(isinstance(n, RMSNorm) for layer in layers for n in (layer.input_layernorm, layer.post_attention_layernorm)) \
             and isinstance(final_norm, RMSNorm)
@@ -241,19 +277,29 @@ class TransformerInferenceModule(torch.nn.Module):
         completions: List[List[int]] = [[] for _ in range(b)]
         step_logits = []
         if use_cache:
-            settings = InferenceSettings(use_cache=True, reset_cache=True)
-            cur, pos = ids, None
+            # every step's positions, and the lengths of one token per row, are known now; the tokens are read back once at the
+            # end unless a stop token may end the loop, so that the host issues the next step while this one runs
+            positions = torch.arange(n_prompt, n_prompt + max_tokens, device=self.device).view(-1, 1, 1).expand(-1, b, 1).contiguous()
+            one_each = torch.arange(b + 1, dtype=torch.int32, device=self.device)
+            logits = self.forward(ids, inference_settings=InferenceSettings(use_cache=True, reset_cache=True), last_token_only=True)
+            settings = InferenceSettings(use_cache=True, reset_cache=False)
+            native = self._native_layers(b, max_tokens - 1)
+            tokens = []
             for k in range(max_tokens):
-                logits = self.forward(cur, position_ids=pos, inference_settings=settings, last_token_only=True)
                 nxt = sample_argmax(logits)
                 step_logits.append(logits[:, -1, :])
-                for i, t in enumerate(nxt.tolist()):
-                    completions[i].append(t)
-                settings = InferenceSettings(use_cache=True, reset_cache=False)
-                cur = nxt.unsqueeze(1)
-                pos = torch.full((b, 1), n_prompt + k, dtype=torch.int64, device=self.device)
-                if b == 1 and completions[0][-1] in stop:
+                tokens.append(nxt)
+                if b == 1 and stop and int(nxt) in stop:
                     break
+                if k + 1 < max_tokens and native is not None:
+                    logits = self._native_step(native, nxt.unsqueeze(1), positions[k].view(-1))
+                    if logits is not None:
+                        continue
+                    native = None                        # a shape the kernels do not cover: nothing has been done yet
+                if k + 1 < max_tokens:
+                    logits = self.forward(nxt.unsqueeze(1), position_ids=positions[k], cumulative_seq_lengths=one_each,
+                                          inference_settings=settings, last_token_only=True)
+            completions = torch.stack(tokens, dim=1).tolist()
         else:
             cur = ids
             for _ in range(max_tokens):

@@ -671,3 +671,33 @@ class ParallelSelfAttention(torch.nn.Module):
             cache.workspace = ops.decode_workspace(b, nq, d, cache.max_ctx, q.device)
         return ops.decode_attention(self._decode_operand(q), cache.k, cache.v, cache.ctx_len, self._decode_operand(k),
                                     self._decode_operand(v), rotary=rotary, softmax_scale=self.softmax_scale, workspace=cache.workspace)
+
+
+def decode_arguments(layer, batch: int, tokens: int, cache_index: int) -> Optional[tuple]:
+    """The arguments of `ops.decode_layer` for the next `tokens` tokens of a layer of this package; None where such a step has
+    to be refused (the module path raises): no cache, another batch, no room in the cache or the rotary table."""
+    att, mlp = layer.self_attention, layer.mlp
+    cache = att.cache.get(cache_index)
+    if cache is None or cache.k.shape[0] != batch or cache.length + tokens > min(cache.max_ctx, att.rotary_embedding.max_seq_length):
+        return None
+    if cache.workspace is None:
+        cache.workspace = ops.decode_workspace(batch, att.num_attention_heads, att.hidden_size_per_attention_head, cache.max_ctx, cache.k.device)
+    return ops.decode_layer_arguments(
+        layer.input_layernorm.weight, layer.input_layernorm.eps, (att.query.weight, att.key.weight, att.value.weight), att.dense.weight,
+        layer.post_attention_layernorm.weight, layer.post_attention_layernorm.eps, mlp.dense_in.weight, mlp.siglu_weight.weight,
+        mlp.dense_out.weight, att.hidden_size_per_attention_head, cache.k, cache.v, cache.ctx_len, att.rotary_embedding.tables(),
+        att.softmax_scale, cache.workspace, cache.k.dtype)
+
+
+def decode_layer(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tensor, position_ids: Optional[torch.Tensor],
+                 cache_index: int) -> Optional[torch.Tensor]:
+    """One cached token per sequence through a whole layer (norms, projections, decode attention, MLP, residuals) in one native call.
+    None, with nothing changed, where the call has to be refused or the kernels do not apply: the module path then raises or
+    computes it."""
+    if position_ids is None or x.dim() != 3 or x.shape[1] != 1 or not x.is_cuda or cumulative_seq_lengths.numel() != x.shape[0] + 1:
+        return None
+    arguments = decode_arguments(layer, x.shape[0], 1, cache_index)
+    y = None if arguments is None else ops.decode_layer(x, position_ids.reshape(-1).contiguous(), arguments)
+    if y is not None:
+        layer.self_attention.cache[cache_index].length += 1
+    return y

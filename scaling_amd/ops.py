@@ -511,3 +511,23 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     _lib.host().decode_attention(q, k_cache, v_cache, ctx_len, k_new, v_new, cos, sin, pos, interleaved, float(softmax_scale),
                                  None if static_scratch else workspace, int(n_splits), out, bool(static_scratch))
     return out
+
+
+def norm_linear_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """rms_norm(x) @ weight.T of up to 16 rows [rows, k] (inference); None where the kernel does not apply."""
+    return _lib.host().norm_linear_rows(x, norm_weight, eps, weight)
+
+
+def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, tables,
+                           softmax_scale, workspace, dtype) -> tuple:
+    """What `decode_layer` takes beside the token: the layer's weights, its caches and rotary tables."""
+    cos, sin = tables
+    interleaved = _fused_rotary_kind(cos, sin, head_dim, dtype)
+    return (norm1, eps1, list(qkv_weights), dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, cos, sin, interleaved,
+            float(softmax_scale), workspace)
+
+
+def decode_layer(x: torch.Tensor, position_ids: torch.Tensor, arguments: tuple) -> Optional[torch.Tensor]:
+    """A cached decode step of a whole layer, x [batch, 1, hidden] of up to 16 sequences, position_ids int64 [batch]: raises the context
+    lengths by one, appends to the caches and returns the layer's output.  None, with nothing done, where the kernels do not apply."""
+    return _lib.host().decode_layer(x, position_ids, *arguments)
