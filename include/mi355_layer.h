@@ -297,6 +297,10 @@ int mi_rotary_complex(const void* x, void* out, const float* cos, const float* s
  * reference's fp32 evaluation attends with), which leaves mean-relative errors of about 2e-3 in either mode. */
 #define MI_ATTN_SPLIT_P 4
 /* backward: run only the named kernels (for per-kernel timing; all three when none of the bits is set) */
+/* 16-bit types: which tiling, for measurements and tests (without either bit the library chooses by size; a call that the short-context
+ * kernels do not cover - dropout, MI_ATTN_SPLIT_P, single backward stages - is tiled whatever the bits) */
+#define MI_ATTN_SHORT 128
+#define MI_ATTN_TILED 256
 #define MI_ATTN_BWD_DELTA 16
 #define MI_ATTN_BWD_DKDV 32
 #define MI_ATTN_BWD_DQ 64

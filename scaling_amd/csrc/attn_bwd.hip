@@ -1,6 +1,6 @@
 // Attention backward for gfx950 (bf16 MFMA, fp32 softmax recomputation from the saved log-sum-exp).
 //
-// Three kernels (four with fewer than 8 KV heads), no atomics, fixed summation order (bit-reproducible):
+// Long contexts: three kernels (four with fewer than 8 KV heads; short contexts: attn_short.h), no atomics, fixed summation order (bit-reproducible):
 //   1. delta[h][t] = sum_d dO[t][h][d] * O[t][h][d]
 //   2. dK/dV: a workgroup owns 128 keys of one KV head (K and V rows stay in LDS), loops over the query
 //      heads of the group and over 64-query tiles staged in LDS:
@@ -15,6 +15,7 @@
 // LDS transpose reads without bank conflicts (LdsTile in attn_common.h); score tiles are consumed in their
 // accumulator layout.
 #include "attn_common.h"
+#include "attn_short.h"
 
 #include <type_traits>
 
@@ -705,6 +706,22 @@ template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) 
     return MI_OK;
 }
 
+// dQ first: it leaves delta for dK / dV
+template <int D> int launch_short(const AttnParams& p, hipStream_t st) {
+    const int64_t grid_q = ((int64_t)p.total_q + kShortRows - 1) / kShortRows * p.nq;
+    const int64_t grid_k = ((int64_t)p.total_k + kShortRows - 1) / kShortRows * p.nkv * p.hsplit;
+    if (grid_q > 0x7fffffffLL || grid_k > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+    attn_short_dq_kernel<D><<<dim3((unsigned)grid_q), dim3(64 * kShortWaves), 0, st>>>(p);
+    int rc = mi_check_launch("attn_short_dq");
+    if (rc != MI_OK) return rc;
+    attn_short_dkdv_kernel<D><<<dim3((unsigned)grid_k), dim3(64 * kShortWaves), 0, st>>>(p);
+    rc = mi_check_launch("attn_short_dkdv");
+    if (rc != MI_OK || p.hsplit == 1) return rc;
+    const int64_t n = (int64_t)p.total_k * p.nkv * (D / 8);
+    attn_bwd_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>(p);
+    return mi_check_launch("attn_bwd_dkdv_reduce");
+}
+
 }  // namespace
 
 #ifndef MI_ELEM_F16
@@ -754,6 +771,14 @@ int MI_ENTRY(mi_attn_bwd_impl)(const mi_attn_bwd_args* b) {
     p.delta = (float*)b->workspace;
     p.unrotate = a->rotary_cos == nullptr ? 0 : (a->rotary_interleaved ? 2 : 1);
     mi_set_head_split(a, b, &p);
+    if (mi_attn_is_short(a, true) && !(a->flags & (MI_ATTN_SPLIT_P | MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ)) && p.drop_thr == 0) {
+        switch (a->head_dim) {
+            case 32: return launch_short<32>(p, (hipStream_t)a->stream);
+            case 64: return launch_short<64>(p, (hipStream_t)a->stream);
+            case 96: return launch_short<96>(p, (hipStream_t)a->stream);
+            default: return launch_short<128>(p, (hipStream_t)a->stream);
+        }
+    }
     {                                                                                               // dQ: 256-query blocks
         const int per_doc = mi_blocks_per_doc(a->total_q, a->n_docs, 256);
         if (p.n_rep == 1) p.across_q = per_doc;

@@ -16,6 +16,7 @@
 // The mask is a per-lane key interval [klo, khi) derived from the cumulative sequence lengths; tiles
 // outside the union of the intervals are never loaded, tiles inside every interval skip the compare.
 #include "attn_common.h"
+#include "attn_short.h"
 
 #include <type_traits>
 
@@ -485,6 +486,23 @@ template <int D> int launch_d(const AttnParams& p, int rot, bool q_only, int nw,
     return nw == 8 ? launch<D, 8, 0, false>(p, st) : launch<D, 4, 0, false>(p, st);
 }
 
+template <int D> int launch_short(const AttnParams& p, int rot, bool q_only, hipStream_t st) {
+    const int64_t grid = ((int64_t)p.total_q + kShortRows - 1) / kShortRows * p.nq;
+    if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_fwd: too many work items");
+    const dim3 g((unsigned)grid), b(64 * kShortWaves);
+    if constexpr (D == 64 || D == 128) {
+        if (rot == 2 && q_only) attn_short_fwd_kernel<D, 2, false><<<g, b, 0, st>>>(p);
+        else if (rot == 2) attn_short_fwd_kernel<D, 2, true><<<g, b, 0, st>>>(p);
+        else if (rot == 1 && q_only) attn_short_fwd_kernel<D, 1, false><<<g, b, 0, st>>>(p);
+        else if (rot == 1) attn_short_fwd_kernel<D, 1, true><<<g, b, 0, st>>>(p);
+        else attn_short_fwd_kernel<D, 0, false><<<g, b, 0, st>>>(p);
+    } else {
+        if (rot) return mi_fail(MI_E_SHAPE, "attn_fwd: fused rotary needs head_dim 64 or 128");
+        attn_short_fwd_kernel<D, 0, false><<<g, b, 0, st>>>(p);
+    }
+    return mi_check_launch("attn_short_fwd");
+}
+
 }  // namespace
 
 int MI_ENTRY(mi_attn_fwd_impl)(const mi_attn_args* a) {
@@ -502,6 +520,14 @@ int MI_ENTRY(mi_attn_fwd_impl)(const mi_attn_args* a) {
         if (!rot) return mi_fail(MI_E_NULL, "attn_fwd: q_rot_out needs the fused rotary");
         if (!mi_aligned16(a->q_rot_out)) return mi_fail(MI_E_ALIGN, "attn_fwd: q_rot_out must be 16-byte aligned");
         p.q_rot = (elem_t*)a->q_rot_out;
+    }
+    if (mi_attn_is_short(a, false) && !(a->flags & MI_ATTN_SPLIT_P) && p.drop_thr == 0) {
+        switch (a->head_dim) {
+            case 32: return launch_short<32>(p, rot, q_only, (hipStream_t)a->stream);
+            case 64: return launch_short<64>(p, rot, q_only, (hipStream_t)a->stream);
+            case 96: return launch_short<96>(p, rot, q_only, (hipStream_t)a->stream);
+            default: return launch_short<128>(p, rot, q_only, (hipStream_t)a->stream);
+        }
     }
     // 256-query workgroups (two groups of wavefronts a phase apart) beat 128-query ones at every size measured,
     // also when they leave most compute units without work (1 x 512 tokens x 32 heads: 22 against 25 us,

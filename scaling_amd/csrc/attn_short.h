@@ -1,0 +1,577 @@
+// Attention kernels for short contexts (documents of a few hundred tokens, small batches), forward and backward.
+//
+// The tiled kernels give a workgroup 128 - 256 rows and walk its keys (queries) in one chain of barriers; with short documents that
+// chain is most of the launch, its workgroups leave compute units idle, and 256 rows span several documents.  Here a workgroup of
+// four wavefronts owns 32 rows, and the wavefronts split the other axis: wavefront w takes tiles w, w + 4, ... of 32 tokens,
+// each through its own LDS stages with direct global -> LDS loads and no barrier, and the four partial results meet in
+// LDS at the end, in a fixed order.  A document of 512 tokens is a chain of at most four tiles.  The mask interval of a row comes from one
+// load of the cumulative lengths and a search in registers.
+// The price is operand traffic: a tile serves 32 rows instead of 128 or 256, so long contexts stay with the tiled kernels
+// (see mi_attn_is_short).
+#pragma once
+#include "attn_common.h"
+
+namespace {
+
+constexpr int kShortWaves = 4, kShortRows = 32;
+
+// Largest j < n_docs with cu[j] <= t and the bounds of that document on both axes, as find_doc gives them; for up to 63 documents the
+// lengths sit one per lane.
+struct DocBounds { int qs, qe, ks, ke; };
+template <bool KEY>
+__device__ __forceinline__ DocBounds short_doc(const AttnParams& p, int t, int lane) {
+    DocBounds d;
+    if (p.n_docs == 1) {
+        d.qs = p.cu_q[0]; d.qe = p.cu_q[1]; d.ks = p.cu_k[0]; d.ke = p.cu_k[1];
+    } else if (p.n_docs <= 63) {
+        const int at = lane < p.n_docs ? lane : p.n_docs;
+        const int cq = p.cu_q[at], ck = p.cu_k[at];
+        const int c = KEY ? ck : cq;
+        int j = 0;
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1) {
+            const int mid = j + step, v = __shfl(c, mid & 63, MI_WAVE);
+            if (mid < p.n_docs && v <= t) j = mid;
+        }
+        d.qs = __shfl(cq, j, MI_WAVE); d.qe = __shfl(cq, j + 1, MI_WAVE);
+        d.ks = __shfl(ck, j, MI_WAVE); d.ke = __shfl(ck, j + 1, MI_WAVE);
+    } else {
+        const int j = find_doc(KEY ? p.cu_k : p.cu_q, p.n_docs, t);
+        d.qs = p.cu_q[j]; d.qe = p.cu_q[j + 1]; d.ks = p.cu_k[j]; d.ke = p.cu_k[j + 1];
+    }
+    return d;
+}
+// key_range / query_range of attn_common.h
+__device__ __forceinline__ void short_key_range(const AttnParams& p, int t, int lane, int& klo, int& khi) {
+    const DocBounds d = short_doc<false>(p, t, lane);
+    klo = d.ks;
+    khi = p.causal ? min(d.ks + (t - d.qs) + (d.ke - d.ks) - (d.qe - d.qs) + 1, d.ke) : d.ke;
+    if (t >= p.total_q) klo = khi = 0;
+    if (khi < klo) khi = klo;
+}
+__device__ __forceinline__ void short_query_range(const AttnParams& p, int u, int lane, int& qlo, int& qhi) {
+    const DocBounds d = short_doc<true>(p, u, lane);
+    qhi = d.qe;
+    qlo = p.causal ? max(d.qs + (u - d.ks) - ((d.ke - d.ks) - (d.qe - d.qs)), d.qs) : d.qs;
+    if (u >= p.total_k) qlo = qhi = 0;
+    if (qlo > qhi) qlo = qhi;
+}
+// union of the wavefront's intervals, from a multiple of 32 on
+__device__ __forceinline__ void short_tiles(int lo, int hi, int& wmin, int& wmax, int& t0, int& n_tiles) {
+    wmin = group_min<64>(hi > lo ? lo : 0x7fffffff);
+    wmax = group_max<64>(hi > lo ? hi : 0);
+    // the same in every lane; made scalar, as loop control and the base address of a direct load have to be
+    const bool any = wmax > wmin;
+    t0 = __builtin_amdgcn_readfirstlane(any ? wmin & ~31 : 0);
+    n_tiles = __builtin_amdgcn_readfirstlane(any ? (wmax - t0 + 31) / 32 : 0);
+}
+
+// One wavefront's two tiles of 32 tokens, in STAGES stages.  The chains are short, so what hides the loads is the other workgroups of the
+// compute unit: one stage (8192 tokens x 32 heads of 128 in documents of 512: forward 240 us with two, 137 with one), except for dK / dV
+// of 96 and 128 features, whose registers leave room for one workgroup anyway.
+template <int D, int STAGES = 1> struct ShortStages {
+    using Tile = LdsTile<D>;
+    static constexpr int kTile = 32 * Tile::RB, kLoads = Tile::kInstrs / 2;
+    static constexpr int kBytes = 2 * STAGES * kTile;
+    static constexpr int kSmem = kShortWaves * kBytes;
+    char* base;
+    __device__ __forceinline__ char* first(int buf = 0) const { return base + buf * 2 * kTile; }
+    __device__ __forceinline__ char* second(int buf = 0) const { return base + buf * 2 * kTile + kTile; }
+    // Before a stage is loaded again its reads must have returned.
+    static __device__ __forceinline__ void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+};
+
+// Sum over the wavefronts of quad a = wave of every feature tile, from the per-wavefront copies in LDS ([wave][16 DT][64] floats).
+template <int D> __device__ __forceinline__ void short_store(float* red, int wave, int lane, const f32x16_t (&acc)[D / 32]) {
+    float* mine = red + wave * (16 * (D / 32) * 64) + lane;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[(dt * 16 + r) * 64] = acc[dt][r];
+}
+template <int D> __device__ __forceinline__ void short_sum(const float* red, int wave, int lane, float (&x)[D / 32][4]) {
+    constexpr int kSet = 16 * (D / 32) * 64;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float* at = red + (dt * 16 + 4 * wave + c) * 64 + lane;
+            x[dt][c] = (at[0] + at[kSet]) + (at[2 * kSet] + at[3 * kSet]);
+        }
+}
+// Rotation by minus the position's angles of features 32 dt + 8 a + 4 g + c (see unrotate_acc)
+template <int D> __device__ __forceinline__ void short_unrotate(float (&x)[D / 32][4], const AttnParams& p, int64_t pos, int a, int g) {
+    constexpr int DT = D / 32;
+    pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+    if (p.unrotate == 1) {
+        const elem_t* cr = p.cos + pos * D + 8 * a + 4 * g;
+        const elem_t* sr = p.sin + pos * D + 8 * a + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < DT / 2; ++dt) {
+            const uint2 cw = *reinterpret_cast<const uint2*>(cr + 32 * dt), sw = *reinterpret_cast<const uint2*>(sr + 32 * dt);
+            const float c4[4] = {elem_lo(cw.x), elem_hi(cw.x), elem_lo(cw.y), elem_hi(cw.y)};
+            const float s4[4] = {elem_lo(sw.x), elem_hi(sw.x), elem_lo(sw.y), elem_hi(sw.y)};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float x0 = x[dt][c], x1 = x[dt + DT / 2][c];
+                x[dt][c] = x0 * c4[c] + x1 * s4[c];
+                x[dt + DT / 2][c] = x1 * c4[c] - x0 * s4[c];
+            }
+        }
+    } else {
+        const float* cr = p.cos32 + pos * (D / 2) + 4 * a + 2 * g;
+        const float* sr = p.sin32 + pos * (D / 2) + 4 * a + 2 * g;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const float2 c2 = *reinterpret_cast<const float2*>(cr + 16 * dt), s2 = *reinterpret_cast<const float2*>(sr + 16 * dt);
+            rotate_complex_pair(x[dt][0], x[dt][1], c2.x, -s2.x);
+            rotate_complex_pair(x[dt][2], x[dt][3], c2.y, -s2.y);
+        }
+    }
+}
+template <int D> __device__ __forceinline__ void short_write(elem_t* row, const float (&x)[D / 32][4], float scale) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+        *reinterpret_cast<uint2*>(row + 32 * dt) = make_uint2(pack_elem2(x[dt][0] * scale, x[dt][1] * scale), pack_elem2(x[dt][2] * scale, x[dt][3] * scale));
+}
+
+// Host side: whether a call goes to these kernels: up to 2048 workgroups of 32 rows, which is about twice what the chip holds, and 1024
+// in the forward pass above 64 features, where a compute unit holds two.  Tiled / short, us, forward and backward:
+//   12 heads of 64, 3001 tokens in documents of 17 - 400 (1128 workgroups)     20.9 / 12.3   48.4 / 37.1
+//   8 heads of 64, 2048 tokens (512)                                           46.1 / 15.9   90.0 / 44.9
+//   16 heads of 64, 4084 tokens in documents of 16 - 600 (2048)                25.3 / 20.7   62.4 / 59.9
+//   16 heads of 64, 8192 tokens in documents of 1024 (4096)                    42.0 / 50.9    115 / 139
+//   32 / 8 heads of 128, 512 tokens (512)                                      21.8 / 10.7   81.9 / 48.1
+//   32 / 8 heads of 128, 1024 tokens (1024)                                    34.7 / 23.9    145 / 91.8
+//   32 / 8 heads of 128, 2048 tokens (2048)                                    63.6 / 71.5    271 / 206
+//   32 / 8 heads of 128, 4096 tokens in documents of 512 (4096)                45.0 / 73.6    130 / 199
+// Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
+// backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
+static inline bool mi_attn_is_short(const mi_attn_args* a, bool backward) {
+    if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return false;
+    if (a->flags & MI_ATTN_SHORT) return true;
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k;
+    const int per_unit = backward || a->head_dim <= 64 ? 8 : 4;
+    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads <= (int64_t)per_unit * mi_compute_units();
+}
+
+// ---- forward: 32 queries of one head --------------------------------------------------------------------------------
+// QROT: 0 = q as it is, 1 = rotate-half, 2 = interleaved rotary on the q load; KROT: k is rotated too, in its LDS tile (otherwise it
+// arrives rotated, as training passes it)
+template <int D, int QROT, bool KROT>
+__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_fwd_kernel(const AttnParams p) {
+    constexpr int KS = D / 16, DT = D / 32;
+    using Stages = ShortStages<D>;
+    using Tile = LdsTile<D>;
+    constexpr int RB = Tile::RB;
+    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
+    __shared__ float m_lds[kShortWaves][32], l_lds[kShortWaves][32];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nqb = (p.total_q + 31) / 32;
+    int head, rank;
+    head_and_rank(blockIdx.x, p.nq, head, rank);
+    const int qb = nqb - 1 - rank, kvh = head / p.n_rep;
+    const int tq = qb * 32 + l32, tl = min(tq, p.total_q - 1);
+
+    elem8_t qf[KS];
+    {
+        const elem_t* qrow = p.q + (int64_t)tl * p.q_st + (int64_t)head * p.q_sh + 8 * g;
+        uint4 raw[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) raw[ks] = ld128(qrow + 16 * ks);
+        if constexpr (QROT != 0) {
+            int64_t pos = p.pos_q[tl];
+            pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+            if constexpr (QROT == 1) {
+#pragma unroll
+                for (int ks = 0; ks < KS / 2; ++ks)
+                    rotate_pair(raw[ks], raw[ks + KS / 2], ld128(p.cos + pos * D + 16 * ks + 8 * g), ld128(p.sin + pos * D + 16 * ks + 8 * g), 1.0f);
+            } else {
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    rotate_interleaved(raw[ks], ld128(p.cos32 + pos * (D / 2) + 8 * ks + 4 * g), ld128(p.sin32 + pos * (D / 2) + 8 * ks + 4 * g), 1.0f);
+            }
+            if (p.q_rot != nullptr && wave == 0 && tq < p.total_q) {
+                elem_t* qo = p.q_rot + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh + 8 * g;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) st128(qo + 16 * ks, raw[ks]);
+            }
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = __builtin_bit_cast(elem8_t, raw[ks]);
+    }
+    int klo, khi, wmin, wmax, kt0, n_tiles;
+    short_key_range(p, tq, lane, klo, khi);
+    short_tiles(klo, khi, wmin, wmax, kt0, n_tiles);
+
+    f32x16_t o_acc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
+    float m_i = -INFINITY, l_i = 0.f;
+
+    const Stages st{smem + wave * Stages::kBytes};
+    const elem_t* kbase = p.k + (int64_t)kvh * p.k_sh;
+    const elem_t* vbase = p.v + (int64_t)kvh * p.v_sh;
+    DmaPlan<D, Stages::kLoads> k_plan, v_plan;
+    k_plan.init(0, lane, p.k_st);
+    v_plan.init(0, lane, p.v_st);
+    auto issue_k = [&](int tile) { k_plan.issue(kbase, p.k_st, kt0 + 32 * tile, p.total_k - 1, st.first()); };
+    auto issue_v = [&](int tile) { v_plan.issue(vbase, p.v_st, kt0 + 32 * tile, p.total_k - 1, st.second()); };
+    const char *ks_ = st.first(), *vs_ = st.second();
+    int h0, h1;
+    Tile::tr_bases(lane, h0, h1);
+    const int k_row = Tile::row_base(l32, g);
+    if (wave < n_tiles) { issue_k(wave); issue_v(wave); }
+    for (int tile = wave; tile < n_tiles; tile += kShortWaves) {
+        const bool next = tile + kShortWaves < n_tiles;
+        const int kt = kt0 + 32 * tile;
+        wait_vmcnt<Stages::kLoads>();     // K has landed, V may still be in flight
+        if constexpr (KROT) {
+#pragma unroll
+            for (int j = 0; j < D / 32; ++j) {
+                const int row = (lane + 64 * j) / (D / 16), c = (lane + 64 * j) % (D / 16);
+                char *at0 = st.first() + Tile::unit_offset(row, c), *at1 = st.first() + Tile::unit_offset(row, c + D / 16);
+                uint4 lo = ld128(at0), hi = ld128(at1);
+                int64_t pos = p.pos_k[min(kt + row, p.total_k - 1)];
+                pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+                if constexpr (QROT == 1) {
+                    rotate_pair(lo, hi, ld128(p.cos + pos * D + 8 * c), ld128(p.sin + pos * D + 8 * c), 1.0f);
+                } else {
+                    const float *cr = p.cos32 + pos * (D / 2) + 4 * c, *sr = p.sin32 + pos * (D / 2) + 4 * c;
+                    rotate_interleaved(lo, ld128(cr), ld128(sr), 1.0f);
+                    rotate_interleaved(hi, ld128(cr + D / 4), ld128(sr + D / 4), 1.0f);
+                }
+                st128(at0, lo);
+                st128(at1, hi);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+        f32x16_t s_acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) s_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(ks_ + (k_row ^ (ks << 5))), qf[ks], s_acc);
+        Stages::reads_done();
+        if (next) issue_k(tile + kShortWaves);
+        // rows of the accumulator are keys kt + 8 a + 4 g + c, the column is this lane's query
+        if (__any((kt < klo) || (kt + 32 > khi))) {
+            const int rel0 = kt + 4 * g - klo;
+            const unsigned len = (unsigned)(khi - klo);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if ((unsigned)(rel0 + 8 * (r >> 2) + (r & 3)) >= len) s_acc[r] = -INFINITY;
+        }
+        float mx = s_acc[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s_acc[r]);
+        const float m_new = fmaxf(m_i, pair_max(mx) * p.scale_log2);
+        if (__any(m_new > m_i)) {
+            const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_i - m_new);
+            m_i = m_new;
+            l_i *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
+        }
+        const float m_use = m_i == -INFINITY ? 0.f : m_i;
+        elem8_t pf[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float e = fast_exp2(s_acc[r] * p.scale_log2 - m_use);
+            l_i += e;
+            pf[r >> 3][r & 7] = (elem_t)e;
+        }
+        if (next) wait_vmcnt<Stages::kLoads>(); else wait_vmcnt<0>();     // V has landed, the next K may be in flight
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+                o_acc[dt] = mfma_32x32x16(tr_pair(vs_ + (h0 ^ (dt << 6)) + 16 * m * RB, vs_ + (h1 ^ (dt << 6)) + 16 * m * RB), pf[m], o_acc[dt]);
+        Stages::reads_done();
+        if (next) issue_v(tile + kShortWaves);
+    }
+    // ---- merge
+    l_i = pair_sum(l_i);
+    if (g == 0) { m_lds[wave][l32] = m_i; l_lds[wave][l32] = l_i; }
+    __syncthreads();
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) M = fmaxf(M, m_lds[w][l32]);
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) L += m_lds[w][l32] == -INFINITY ? 0.f : l_lds[w][l32] * fast_exp2(m_lds[w][l32] - M);
+    const float f = m_i == -INFINITY ? 0.f : fast_exp2(m_i - M);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[dt][r] *= f;
+    float* red = reinterpret_cast<float*>(smem);
+    short_store<D>(red, wave, lane, o_acc);
+    __syncthreads();
+    if (tq >= p.total_q) return;
+    float x[DT][4];
+    short_sum<D>(red, wave, lane, x);
+    short_write<D>(p.o + (int64_t)tq * p.o_st + (int64_t)head * p.o_sh + 8 * wave + 4 * g, x, L > 0.f ? 1.0f / L : 0.f);
+    if (wave == 0 && g == 0 && p.lse != nullptr)
+        p.lse[(int64_t)head * p.total_q + tq] = L > 0.f ? (M + __log2f(L)) * 0.6931471805599453f : INFINITY;
+}
+
+// ---- backward: dQ and delta of 32 queries of one head ------------------------------------------------------------------
+template <int D>
+__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 2) void attn_short_dq_kernel(const AttnParams p) {
+    constexpr int KS = D / 16, DT = D / 32;
+    using Stages = ShortStages<D>;
+    using Tile = LdsTile<D>;
+    constexpr int RB = Tile::RB;
+    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nqb = (p.total_q + 31) / 32;
+    int head, rank;
+    head_and_rank(blockIdx.x, p.nq, head, rank);
+    const int qb = nqb - 1 - rank, kvh = head / p.n_rep;
+    const int tq = qb * 32 + l32, tl = min(tq, p.total_q - 1);
+
+    elem8_t qf[KS], dof[KS];
+    float delta = 0.f;
+    {
+        const elem_t* qr = p.q + (int64_t)tl * p.q_st + (int64_t)head * p.q_sh + 8 * g;
+        const elem_t* dr = p.d_o + (int64_t)tl * p.o_st + (int64_t)head * p.o_sh + 8 * g;
+        const elem_t* orow = p.o + (int64_t)tl * p.o_st + (int64_t)head * p.o_sh + 8 * g;
+        uint4 o_raw[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            qf[ks] = __builtin_bit_cast(elem8_t, ld128(qr + 16 * ks));
+            dof[ks] = __builtin_bit_cast(elem8_t, ld128(dr + 16 * ks));
+            o_raw[ks] = ld128(orow + 16 * ks);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            float a[8], b[8];
+            Elem<elem_t>::unpack(o_raw[ks], a);
+            Elem<elem_t>::unpack(__builtin_bit_cast(uint4, dof[ks]), b);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) delta += a[i] * b[i];
+        }
+        delta = pair_sum(delta);
+        if (wave == 0 && g == 0 && tq < p.total_q) p.delta[(int64_t)head * p.total_q + tq] = delta;
+    }
+    const float lse2 = p.lse[(int64_t)head * p.total_q + tl] * 1.4426950408889634f;
+    int klo, khi, wmin, wmax, kt0, n_tiles;
+    short_key_range(p, tq, lane, klo, khi);
+    short_tiles(klo, khi, wmin, wmax, kt0, n_tiles);
+
+    f32x16_t dq_acc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dq_acc[dt][r] = 0.f;
+    const Stages st{smem + wave * Stages::kBytes};
+    const elem_t* kbase = p.k + (int64_t)kvh * p.k_sh;
+    const elem_t* vbase = p.v + (int64_t)kvh * p.v_sh;
+    DmaPlan<D, Stages::kLoads> k_plan, v_plan;
+    k_plan.init(0, lane, p.k_st);
+    v_plan.init(0, lane, p.v_st);
+    auto issue_k = [&](int tile) { k_plan.issue(kbase, p.k_st, kt0 + 32 * tile, p.total_k - 1, st.first()); };
+    auto issue_v = [&](int tile) { v_plan.issue(vbase, p.v_st, kt0 + 32 * tile, p.total_k - 1, st.second()); };
+    const char *ks_ = st.first(), *vs_ = st.second();
+    int h0, h1;
+    Tile::tr_bases(lane, h0, h1);
+    const int a_row = Tile::row_base(l32, g);
+    if (wave < n_tiles) { issue_v(wave); issue_k(wave); }
+    for (int tile = wave; tile < n_tiles; tile += kShortWaves) {
+        const bool next = tile + kShortWaves < n_tiles;
+        const int kt = kt0 + 32 * tile;
+        wait_vmcnt<0>();
+        f32x16_t s_acc, dp_acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { s_acc[r] = 0.f; dp_acc[r] = 0.f; }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            s_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(ks_ + (a_row ^ (ks << 5))), qf[ks], s_acc);
+            dp_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(vs_ + (a_row ^ (ks << 5))), dof[ks], dp_acc);
+        }
+        Stages::reads_done();
+        if (next) issue_v(tile + kShortWaves);
+        if (__any((kt < klo) || (kt + 32 > khi))) {
+            const int rel0 = kt + 4 * g - klo;
+            const unsigned len = (unsigned)(khi - klo);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if ((unsigned)(rel0 + 8 * (r >> 2) + (r & 3)) >= len) s_acc[r] = -INFINITY;
+        }
+        elem8_t dsf[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dsf[r >> 3][r & 7] = (elem_t)(fast_exp2(s_acc[r] * p.scale_log2 - lse2) * (dp_acc[r] - delta));
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+                dq_acc[dt] = mfma_32x32x16(tr_pair(ks_ + (h0 ^ (dt << 6)) + 16 * m * RB, ks_ + (h1 ^ (dt << 6)) + 16 * m * RB), dsf[m], dq_acc[dt]);
+        Stages::reads_done();
+        if (next) issue_k(tile + kShortWaves);
+    }
+    __syncthreads();                      // every wavefront is done with its stages
+    float* red = reinterpret_cast<float*>(smem);
+    short_store<D>(red, wave, lane, dq_acc);
+    __syncthreads();
+    if (tq >= p.total_q) return;
+    float x[DT][4];
+    short_sum<D>(red, wave, lane, x);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[dt][c] *= p.scale;
+    if constexpr (D == 64 || D == 128) {
+        if (p.unrotate != 0) short_unrotate<D>(x, p, p.pos_q[tq], wave, g);
+    }
+    short_write<D>(p.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh + 8 * wave + 4 * g, x, 1.0f);
+}
+
+// ---- backward: dK and dV of 32 keys of one KV head (of one share of its query heads: hsplit) ------------------------------
+// The wavefronts take (query tile, query head) pairs in turn; delta has been written by the dQ launch.
+template <int D>
+__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_dkdv_kernel(const AttnParams p) {
+    constexpr int KS = D / 16, DT = D / 32;
+    constexpr int STAGES = D <= 64 ? 1 : 2;
+    using Stages = ShortStages<D, STAGES>;
+    using Tile = LdsTile<D>;
+    constexpr int RB = Tile::RB;
+    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
+    __shared__ __attribute__((aligned(16))) float stat_lds[kShortWaves][64];      // 32 log-sum-exps, 32 deltas of the wavefront's tile
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int group, kb;
+    head_and_rank(blockIdx.x, p.nkv * p.hsplit, group, kb);       // key blocks with the most queries come first
+    const int kvh = group / p.hsplit, hs = group - kvh * p.hsplit, hpw = p.n_rep / p.hsplit;
+    const int key = kb * 32 + l32, kl = min(key, p.total_k - 1);
+
+    elem8_t kf[KS], vf[KS];
+    {
+        const elem_t* kr = p.k + (int64_t)kl * p.k_st + (int64_t)kvh * p.k_sh + 8 * g;
+        const elem_t* vr = p.v + (int64_t)kl * p.v_st + (int64_t)kvh * p.v_sh + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            kf[ks] = __builtin_bit_cast(elem8_t, ld128(kr + 16 * ks));
+            vf[ks] = __builtin_bit_cast(elem8_t, ld128(vr + 16 * ks));
+        }
+    }
+    int qlo, qhi, wmin, wmax, qt0, n_tiles;
+    short_query_range(p, key, lane, qlo, qhi);
+    short_tiles(qlo, qhi, wmin, wmax, qt0, n_tiles);
+
+    f32x16_t dk_acc[DT], dv_acc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { dk_acc[dt][r] = 0.f; dv_acc[dt][r] = 0.f; }
+    const Stages st{smem + wave * Stages::kBytes};
+    DmaPlan<D, Stages::kLoads> q_plan, do_plan;
+    q_plan.init(0, lane, p.q_st);
+    do_plan.init(0, lane, p.o_st);
+    const float* stat_base = g == 0 ? p.lse : p.delta;
+    const float stat_scale = g == 0 ? 1.4426950408889634f : 1.0f;
+    const int iters = n_tiles * hpw;
+    float stat = 0.f;
+    auto issue = [&](int iter, int buf) {
+        const int tile = iter / hpw, head = kvh * p.n_rep + hs * hpw + (iter - tile * hpw), qt = qt0 + 32 * tile;
+        stat = stat_base[(int64_t)head * p.total_q + min(qt + l32, p.total_q - 1)];
+        q_plan.issue(p.q + (int64_t)head * p.q_sh, p.q_st, qt, p.total_q - 1, st.first(buf));
+        do_plan.issue(p.d_o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, st.second(buf));
+    };
+    int h0, h1;
+    Tile::tr_bases(lane, h0, h1);
+    const int a_row = Tile::row_base(l32, g);
+    if (wave < iters) issue(wave, 0);
+    int buf = 0;
+    for (int iter = wave; iter < iters; iter += kShortWaves) {
+        const bool next = iter + kShortWaves < iters;
+        stat_lds[wave][lane] = stat * stat_scale;
+        const char *qs_ = st.first(buf), *ds_ = st.second(buf);
+        if (STAGES == 2 && next) {
+            issue(iter + kShortWaves, buf ^ 1);
+            wait_vmcnt<2 * Stages::kLoads>();             // this step's tiles have landed, the next one's may be in flight
+        } else {
+            wait_vmcnt<0>();
+        }
+        const int qs = qt0 + 32 * (iter / hpw);
+        f32x16_t s_acc, dp_acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { s_acc[r] = 0.f; dp_acc[r] = 0.f; }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            s_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(qs_ + (a_row ^ (ks << 5))), kf[ks], s_acc);
+            dp_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(ds_ + (a_row ^ (ks << 5))), vf[ks], dp_acc);
+        }
+        // rows of the accumulators are queries qs + 8 a + 4 g + c, the column is this lane's key
+        if (__any((qs < qlo) || (qs + 32 > qhi))) {
+            const int rel0 = qs + 4 * g - qlo;
+            const unsigned len = (unsigned)(qhi - qlo);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if ((unsigned)(rel0 + 8 * (r >> 2) + (r & 3)) >= len) s_acc[r] = -INFINITY;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // stat_lds: one wavefront's LDS accesses complete in program order
+        elem8_t pf[2], dsf[2];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&stat_lds[wave][8 * a + 4 * g]);
+            const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&stat_lds[wave][32 + 8 * a + 4 * g]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int r = 4 * a + c;
+                const float pv = fast_exp2(s_acc[r] * p.scale_log2 - l4[c]);
+                pf[r >> 3][r & 7] = (elem_t)pv;
+                dsf[r >> 3][r & 7] = (elem_t)(pv * (dp_acc[r] - d4[c]));
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const int o0 = (h0 ^ (dt << 6)) + 16 * m * RB, o1 = (h1 ^ (dt << 6)) + 16 * m * RB;
+                dv_acc[dt] = mfma_32x32x16(tr_pair(ds_ + o0, ds_ + o1), pf[m], dv_acc[dt]);
+                dk_acc[dt] = mfma_32x32x16(tr_pair(qs_ + o0, qs_ + o1), dsf[m], dk_acc[dt]);
+            }
+        Stages::reads_done();
+        if (STAGES == 2) buf ^= 1;
+        else if (next) issue(iter + kShortWaves, 0);
+    }
+    __syncthreads();                      // every wavefront is done with its stages
+    float* red = reinterpret_cast<float*>(smem);
+    short_store<D>(red, wave, lane, dk_acc);
+    __syncthreads();
+    float dk[DT][4], dv[DT][4];
+    short_sum<D>(red, wave, lane, dk);
+    __syncthreads();
+    short_store<D>(red, wave, lane, dv_acc);
+    __syncthreads();
+    if (key >= p.total_k) return;
+    short_sum<D>(red, wave, lane, dv);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) dk[dt][c] *= p.scale;
+    if (p.hsplit > 1) {
+        const int64_t row = (((int64_t)hs * p.total_k + key) * p.nkv + kvh) * D + 8 * wave + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            *reinterpret_cast<f32x4_t*>(p.dk_part + row + 32 * dt) = f32x4_t{dk[dt][0], dk[dt][1], dk[dt][2], dk[dt][3]};
+            *reinterpret_cast<f32x4_t*>(p.dv_part + row + 32 * dt) = f32x4_t{dv[dt][0], dv[dt][1], dv[dt][2], dv[dt][3]};
+        }
+        return;
+    }
+    if constexpr (D == 64 || D == 128) {
+        if (p.unrotate != 0) short_unrotate<D>(dk, p, p.pos_k[key], wave, g);
+    }
+    short_write<D>(p.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh + 8 * wave + 4 * g, dk, 1.0f);
+    short_write<D>(p.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh + 8 * wave + 4 * g, dv, 1.0f);
+}
+
+}  // namespace

@@ -1,0 +1,88 @@
+"""The two families of 16-bit attention kernels - tiled, and the ones for short contexts that small calls go to - over the same cases,
+each pinned by its flag: against the oracle, and with the rotary inside against each other."""
+
+import math
+
+import pytest
+import torch
+
+import oracle
+from scaling_amd import ops
+from tests import attn_utils as U
+from tests.parity import check
+from tests.test_gpu_attention import CASES
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SHORT, TILED = 128, 256
+
+
+@pytest.mark.parametrize("flags", [SHORT, TILED])
+@pytest.mark.parametrize("b,s,nq,nkv,d,causal,cuts", CASES)
+def test_attention_routes_parity(b, s, nq, nkv, d, causal, cuts, flags):
+    print(f"case route={flags} b={b} s={s} nq={nq} nkv={nkv} d={d} causal={causal} cuts={cuts}", flush=True)
+    q, k, v, do = U.make_qkv(b, s, nq, nkv, d, seed=b * 1000 + s + d)
+    cu = U.make_cu(b, s, cuts)
+    scale = 1.0 / math.sqrt(d)
+    ref = U.oracle_attention(q, k, v, cu, b, s, causal, scale, torch.float32, do)
+    ref_o = U.oracle_attention(q, k, v, cu, b, s, causal, scale, torch.bfloat16, do)
+    qd, kd, vd, dod, cud = (t.to(DEV) for t in (q, k, v, do, cu))
+    o, lse = ops.attention_forward(qd, kd, vd, cud, None, causal, scale, flags=flags)
+    dq, dk, dv = ops.attention_backward(dod, qd, kd, vd, o, lse, cud, None, causal, scale, flags=flags)
+    torch.cuda.synchronize()
+    check("route.o", o, ref[0], ref_o[0], kind="o")
+    check("route.dq", dq, ref[1], ref_o[1], kind="grad")
+    check("route.dk", dk, ref[2], ref_o[2], kind="grad")
+    check("route.dv", dv, ref[3], ref_o[3], kind="grad")
+
+
+# q of another length than k (one document per row), documents without a key for the first queries, and more documents than lanes
+@pytest.mark.parametrize("lens_q,lens_k", [((40, 7, 90), (100, 7, 33)), ((1,) * 70, (5,) * 70), ((129,), (32,))])
+@pytest.mark.parametrize("causal", [True, False])
+def test_attention_routes_agree_on_unequal_lengths(lens_q, lens_k, causal):
+    print(f"case unequal lengths q={lens_q} k={lens_k} causal={causal}", flush=True)
+    g = torch.Generator().manual_seed(len(lens_q))
+    nq, nkv, d = 4, 2, 64
+    cu_q, cu_k = (torch.tensor([0] + list(torch.tensor(x).cumsum(0)), dtype=torch.int32, device=DEV) for x in (lens_q, lens_k))
+    q, do = (torch.randn(sum(lens_q), nq, d, generator=g).half().to(DEV) for _ in range(2))
+    k, v = (torch.randn(sum(lens_k), nkv, d, generator=g).half().to(DEV) for _ in range(2))
+    out = []
+    for flags in (SHORT, TILED):
+        o, lse = ops.attention_forward(q, k, v, cu_q, cu_k, causal, None, flags=flags)
+        out.append([o, lse] + list(ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, None, flags=flags)))
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv"), *out):
+        if name == "lse":
+            assert torch.equal(torch.isinf(x), torch.isinf(y)) and torch.allclose(x, y, atol=1e-5)      # sums of exponentials in another order
+        else:
+            # probabilities and dS are rounded to float16 relative to other maxima: two roundings each way, 4 x 2^-11 in the 2-norm
+            assert float((x.float() - y.float()).norm()) <= 2.0 ** -9 * float(y.float().norm()) + 1e-6, name
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_attention_routes_agree_with_rotary(d, interleaved):
+    print(f"case routes rotary d={d} interleaved={interleaved}", flush=True)
+    total, nq, nkv = 333, 8, 2
+    g = torch.Generator().manual_seed(d)
+    q, do = (torch.randn(total, nq, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    k, v = (torch.randn(total, nkv, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    cu = torch.tensor([0, 100, 101, 300, total], dtype=torch.int32)
+    pos = U.position_ids_from_cu(cu, total).to(DEV)
+    cu = cu.to(DEV)
+    if interleaved:
+        ang = torch.outer(torch.arange(512).float(), 1.0 / (10000.0 ** (torch.arange(0, d, 2).float() / d))).to(DEV)
+        cos, sin = ang.cos().contiguous(), ang.sin().contiguous()
+        k_rot = ops.rotary_embedding_complex(k, cos, sin, pos, total)
+    else:
+        tabs = oracle.rotary_tables(d, 512, 10000, torch.bfloat16)
+        cos, sin = tabs.cos.to(DEV).view(512, d), tabs.sin.to(DEV).view(512, d)
+        k_rot = ops.rotary_embedding(k, cos, sin, pos, total)
+    out = []
+    for flags in (SHORT, TILED):
+        o, lse, q_rot = ops.attention_forward(q, k_rot, v, cu, None, True, None, rotary=(cos, sin, pos, None), flags=flags, return_rotated_q=True)
+        out.append([o, lse, q_rot] + list(ops.attention_backward(do, q_rot, k_rot, v, o, lse, cu, None, True, None, flags=flags, rotary=(cos, sin, pos, pos))))
+    fused, _ = ops.attention_forward(q, k, v, cu, None, True, None, rotary=(cos, sin, pos, pos), flags=SHORT)
+    assert torch.equal(fused, out[0][0])                   # k rotated in the kernel or before it
+    assert torch.equal(out[0][2], out[1][2])               # the same rotation, bit for bit
+    for name, x, y in zip(("o", "lse", "q_rot", "dq", "dk", "dv"), *out):
+        assert float((x.float() - y.float()).norm()) <= 2.0 ** -6 * float(y.float().norm()), name      # as above, bfloat16
