@@ -112,6 +112,10 @@ int mi_rows_product(const mi_rows_args* args);
  * row_stride multiples of 8 elements (4 for fp32), x 16-byte aligned. */
 int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int dtype, void* stream);
 
+/* out[c * out_stride + r] = x[r * row_stride + c] for 16-bit elements; columns r of out between n_rows and the next multiple of 8 become
+ * zero.  n_cols and both strides multiples of 8, both matrices 16-byte aligned. */
+int mi_transpose16(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int64_t out_stride, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * RMSNorm.  Replaces core/nn/norm/rms_norm.py:47-50:  y = x * rsqrt(mean(x^2, -1) + eps) * weight.
  * Arithmetic in fp32, one rounding to `dtype` on store.  x, y: [n_rows, hidden]; weight: [hidden].

@@ -398,7 +398,51 @@ template <typename T> int launch_column_sum(const void* x, int64_t ld, int64_t r
     return mi_check_launch("column_sum");
 }
 
+// Transposed copy of a 16-bit matrix: 64 x 64 tiles through LDS, 128-bit accesses on both sides, one read and one write of memory.  Columns
+// of the output past the last row (up to the next multiple of 8) become zero.  LDS rows of 33 words: a column's 2-byte reads
+// spread over the banks.
+constexpr int kTransTile = 64;
+
+__global__ __launch_bounds__(256) void transpose_kernel(const uint16_t* __restrict__ x, int64_t ld, int rows, int cols, uint16_t* __restrict__ out,
+                                                        int64_t ldo) {
+    __shared__ uint32_t tile[kTransTile][kTransTile / 2 + 1];
+    const int r0 = blockIdx.y * kTransTile, c0 = blockIdx.x * kTransTile;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int v = (int)threadIdx.x + 256 * j, r = v / 8, u = v % 8;
+        u32x4_t w = {0, 0, 0, 0};
+        if (r0 + r < rows && c0 + 8 * u < cols) w = *reinterpret_cast<const u32x4_t*>(x + (int64_t)(r0 + r) * ld + c0 + 8 * u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tile[r][4 * u + i] = w[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int v = (int)threadIdx.x + 256 * j, c = v / 8, u = v % 8;
+        if (c0 + c >= cols || r0 + 8 * u >= rows) continue;
+        const uint32_t shift = 16u * (c & 1);
+        u32x4_t w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            w[i] = ((tile[8 * u + 2 * i][c / 2] >> shift) & 0xffffu) | ((tile[8 * u + 2 * i + 1][c / 2] >> shift) << 16);
+        *reinterpret_cast<u32x4_t*>(out + (int64_t)(c0 + c) * ldo + r0 + 8 * u) = w;
+    }
+}
+
 }  // namespace
+
+extern "C" int mi_transpose16(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int64_t out_stride, void* stream) {
+    if (n_rows < 0 || n_cols < 0 || n_rows > 0x7fffffc0LL || n_cols > 0x7fffffc0LL) return mi_fail(MI_E_SHAPE, "transpose16: bad shape");
+    if (n_rows == 0 || n_cols == 0) return MI_OK;
+    if (!x || !out) return mi_fail(MI_E_NULL, "transpose16: null pointer");
+    if (n_cols % 8 || row_stride % 8 || out_stride % 8 || !mi_aligned16(x) || !mi_aligned16(out))
+        return mi_fail(MI_E_ALIGN, "transpose16: columns and strides must be multiples of 8, both matrices 16-byte aligned");
+    if (row_stride < n_cols || out_stride < (n_rows + 7) / 8 * 8 || (n_rows + kTransTile - 1) / kTransTile > 65535)
+        return mi_fail(MI_E_SHAPE, "transpose16: bad shape or stride");
+    const dim3 grid((unsigned)((n_cols + kTransTile - 1) / kTransTile), (unsigned)((n_rows + kTransTile - 1) / kTransTile));
+    transpose_kernel<<<grid, dim3(256), 0, (hipStream_t)stream>>>((const uint16_t*)x, row_stride, (int)n_rows, (int)n_cols, (uint16_t*)out, out_stride);
+    return mi_check_launch("transpose16");
+}
 
 extern "C" int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, int64_t n_cols, void* out, int dtype, void* stream) {
     if (!x || !out) return mi_fail(MI_E_NULL, "column_sum: null pointer");

@@ -101,3 +101,33 @@ def test_column_sum(rows, cols, stride, dtype):
     u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
     bound = u * xd.sum(0).abs() + (rows + 1) * 2.0 ** -24 * xd.abs().sum(0) + 2.0 ** -25
     assert bool(((out.double() - xd.sum(0)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows,cols,stride", [(1, 8, 8), (63, 72, 80), (64, 64, 64), (65, 136, 136), (200, 1000, 1008)])
+def test_transpose16(rows, cols, stride):
+    """Exact; one row and column past a tile, one short of it, rows of a wider matrix; the padding of the result becomes zero up to
+    a whole vector and stays as it is behind."""
+    x = torch.randn(rows, stride, generator=torch.Generator().manual_seed(rows)).bfloat16().to(DEV)
+    ld = (rows + 63) // 64 * 64
+    out = torch.full((cols, ld), 7.0, dtype=torch.bfloat16, device=DEV)
+    _lib.check(_lib.load().mi_transpose16(x.data_ptr(), stride, rows, cols, out.data_ptr(), ld, _lib.stream_ptr()), "mi_transpose16")
+    whole = (rows + 7) // 8 * 8
+    assert torch.equal(out[:, :rows], x[:, :cols].t())
+    assert bool((out[:, rows:whole] == 0).all()) and bool((out[:, whole:] == 7).all())
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(4001, 2048, (8192, 4096)), (3001, 8192, (2056,)), (2500, 4096, (5000,))])
+def test_weight_gradients_through_a_transposed_operand(rows, ins, outs):
+    """Wide projections: the input or (one projection that narrows) the output gradient is transposed first; the same products in
+    the same precision, so one rounding of the result and fp32 sums of `rows` terms against float64 on sampled rows."""
+    print(f"case transposed weight gradient rows={rows} {ins}->{outs}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(ins)
+    x = torch.randn(rows, ins, generator=g, device=DEV).bfloat16().requires_grad_()
+    ws = [(torch.randn(o, ins, generator=g, device=DEV) * 0.02).bfloat16().requires_grad_() for o in outs]
+    dys = [torch.randn(rows, o, generator=g, device=DEV).bfloat16() for o in outs]
+    torch.autograd.backward(ops.projections(x, ws, [None] * len(ws)), dys)
+    for w, dy in zip(ws, dys):
+        pick = torch.tensor([0, 7, w.shape[0] // 2, w.shape[0] - 1], device=DEV)
+        a, b = dy[:, pick].double().t().contiguous(), x.detach().double()
+        bound = 2.0 ** -8 * (a @ b).abs() + (rows + 1) * 2.0 ** -24 * (a.abs() @ b.abs())
+        assert bool(((w.grad[pick].double() - a @ b).abs() <= bound * 1.01).all())
