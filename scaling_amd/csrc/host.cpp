@@ -11,7 +11,10 @@
 #include <torch/extension.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/graph_task.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/autocast_mode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
 #include <optional>
@@ -333,9 +336,9 @@ bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
     const double work = 2.0 * (double)m * (double)n * (double)k;
     return n % v == 0 && k % v == 0 && work <= (v == 4 ? 0.75e9 : 3e9);
 }
-bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows that start on 16-byte boundaries
+bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
-    return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+    return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
 void segment(mi_gemm_problem& pr, const Tensor& p, const Tensor& q, int64_t k) {
@@ -396,11 +399,10 @@ struct Projections : Function<Projections> {
         const auto at = bias_at(has_bias);
         const Tensor x2 = x.reshape({-1, in});
         const int64_t rows = x2.size(0);
-        variable_list saved{x2}, out;
+        variable_list saved{x}, out;                      // x itself: what is differentiated again reaches it
         bool small = aligned(x2);
         for (int64_t i = 0; i < n; ++i) {
             const Tensor& w = params[i];
-            TORCH_CHECK(w.dim() == 2 && w.size(1) == in && w.scalar_type() == x.scalar_type(), "linear: input and weight do not match");
             small = small && aligned(w) && small_product(x, rows, w.size(0), in);
             saved.push_back(w);
         }
@@ -418,6 +420,7 @@ struct Projections : Function<Projections> {
             Tensor add;
             if (residual.has_value()) {
                 add = residual->contiguous();
+                if (reinterpret_cast<uintptr_t>(add.data_ptr()) & 15) add = add.clone();
                 pr[0].add = ptr(add);
                 pr[0].ldadd = pr[0].n;
             }
@@ -439,19 +442,21 @@ struct Projections : Function<Projections> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor& x = saved[0];
-        const int64_t n = (int64_t)g.size(), in = x.size(1), rows = x.size(0);
+        const int64_t n = (int64_t)g.size(), in = saved[0].size(-1);
+        const Tensor x = saved[0].reshape({-1, in});
+        const int64_t rows = x.size(0);
+        const bool again = at::GradMode::is_enabled();     // a graph of this pass is wanted: library products, which have one
         const auto has_bias = ctx->saved_data["has_bias"].toIntVector();
         const auto at = bias_at(has_bias);                 // tensor input 1 + at[i] of the node
         const bool need_dx = ctx->needs_input_grad(0);
         const auto need_weight = [&](int64_t i) { return ctx->needs_input_grad(1 + i); };
         const auto need_bias = [&](int64_t i) { return at[i] >= 0 && ctx->needs_input_grad(1 + at[i]); };
         std::vector<Tensor> dy(n), dw(n), db(n);
-        bool small = rows > 0 && aligned(x);
+        bool small = !again && rows > 0 && aligned(x);
         for (int64_t i = 0; i < n; ++i) {
             if (!g[i].defined()) continue;                 // this projection does not reach the loss
             dy[i] = g[i].reshape({rows, saved[1 + i].size(0)});
-            if (!aligned(dy[i])) dy[i] = dy[i].contiguous();
+            if (!again && !aligned(dy[i])) dy[i] = dy[i].contiguous();
             small = small && aligned(dy[i]) && small_product(x, rows, dy[i].size(1), in);
         }
         Tensor dx;
@@ -485,7 +490,7 @@ struct Projections : Function<Projections> {
             for (int64_t i = 0; i < n; ++i)
                 if (dy[i].defined() && need_weight(i)) out += dy[i].size(1);
             Tensor xt, dyt;                                // the smaller of the two operands, where that pays
-            if (out > 0 && transpose_pays(rows, in, out)) {
+            if (!again && out > 0 && transpose_pays(rows, in, out)) {
                 if (in <= out && transposable(x)) xt = transposed(x, l);
                 else if (n == 1 && transposable(dy[0])) dyt = transposed(dy[0], l);
             }
@@ -497,7 +502,7 @@ struct Projections : Function<Projections> {
                     else dx = at::mm(dy[i], w);
                 }
                 if (need_weight(i)) dw[i] = dyt.defined() ? at::mm(dyt, x) : at::mm(dy[i].t(), xt.defined() ? xt.t() : x);
-                if (need_bias(i)) db[i] = bias_gradient(dy[i]);
+                if (need_bias(i)) db[i] = again ? dy[i].sum(0) : bias_gradient(dy[i]);
             }
         }
         variable_list grads{dx.defined() ? dx.view(ctx->saved_data["x_shape"].toIntVector()) : Tensor()};
@@ -511,16 +516,31 @@ struct Projections : Function<Projections> {
     }
 };
 
-// the plain library call where the native nodes do not apply: autocast chooses the dtype, CPU tensors have no kernel
-bool plain_linear(const Tensor& x, const Tensor& w) {
-    return !x.is_cuda() || x.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA) || x.scalar_type() != w.scalar_type() || x.dim() < 1 ||
-           (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat);
+// A transform that has to see library calls: torch.func (grad, vmap, jvp), forward-mode AD, torch.jit tracing, a dispatch mode or a
+// tensor subclass (fake tensors among them)
+bool transformed(const Tensor& t) {
+    return t.unsafeGetTensorImpl()->is_python_dispatch() || t._fw_grad(0).defined();
+}
+bool transforming() {
+    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           torch::jit::tracer::isTracing();
+}
+
+// The plain library call where the native nodes do not apply: autocast chooses the dtype, CPU tensors have no kernel, and operands that
+// do not fit each other in shape, type or device are the library's to broadcast or refuse.
+bool plain_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
+    if (!x.is_cuda() || x.numel() == 0 || w.numel() == 0 || w.dim() != 2 || w.size(1) != x.size(-1) || w.scalar_type() != x.scalar_type() ||
+        w.device() != x.device() || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat))
+        return true;
+    if (b.has_value() && (b->dim() != 1 || b->size(0) != w.size(0) || b->stride(0) != 1 || b->scalar_type() != x.scalar_type() || b->device() != x.device()))
+        return true;
+    return at::autocast::is_autocast_enabled(at::kCUDA) || transforming() || transformed(x) || transformed(w) || (b.has_value() && transformed(*b));
 }
 
 std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases) {
     TORCH_CHECK(weights.size() == biases.size() && weights.size() >= 1 && weights.size() <= 3, "projections: one to three weights");
     bool plain = false;
-    for (const Tensor& w : weights) plain = plain || plain_linear(x, w);
+    for (size_t i = 0; i < weights.size(); ++i) plain = plain || plain_linear(x, weights[i], biases[i]);
     if (plain) {
         std::vector<Tensor> out;
         for (size_t i = 0; i < weights.size(); ++i) out.push_back(at::linear(x, weights[i], biases[i]));
@@ -536,16 +556,18 @@ std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& w
 }
 
 Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b, const OptTensor& residual) {
-    if (plain_linear(x, w)) {
-        const Tensor y = at::linear(x, w, b);
+    const auto residual_fits = [&] {
+        return residual->scalar_type() == x.scalar_type() && residual->device() == x.device() && residual->dim() == x.dim() &&
+               residual->size(-1) == w.size(0) && residual->sizes().slice(0, x.dim() - 1) == x.sizes().slice(0, x.dim() - 1) && !transformed(*residual);
+    };
+    const bool plain = plain_linear(x, w, b);
+    if (plain || (residual.has_value() && !residual_fits())) {
+        const Tensor y = plain ? at::linear(x, w, b) : op_linear(x, w, b, std::nullopt);
         return residual.has_value() ? y + *residual : y;
     }
     variable_list params{w};
     if (b.has_value()) params.push_back(*b);
-    OptTensor add = residual;
-    if (add.has_value() && (add->scalar_type() != x.scalar_type() || add->dim() != x.dim() || add->size(-1) != w.size(0) || add->numel() / w.size(0) != x.numel() / w.size(1)))
-        return Projections::apply(x, at::TensorList(params), OptTensor(), std::vector<int64_t>{b.has_value()})[0] + *residual;
-    return Projections::apply(x, at::TensorList(params), add, std::vector<int64_t>{b.has_value()})[0];
+    return Projections::apply(x, at::TensorList(params), residual, std::vector<int64_t>{b.has_value()})[0];
 }
 
 // ---- attention core ----------------------------------------------------------------------------------------------------

@@ -69,3 +69,52 @@ def test_projection_that_does_not_reach_the_loss():
     odd = torch.randn(7, 64)
     _close("odd", ops.linear(xg.detach(), odd.to(DEV)), x.double() @ odd.double().t(), x.double().abs() @ odd.double().abs().t(), 64, torch.float32)
     assert ops.linear(torch.empty(0, 64, device=DEV), wg[0]).shape == (0, 32)
+
+
+def test_operands_that_do_not_fit_are_the_librarys():
+    """What torch.nn.functional.linear refuses is refused, what it broadcasts is broadcast: no kernel sees such an operand."""
+    x, w, b = torch.randn(4, 64, device=DEV), torch.randn(32, 64, device=DEV), torch.randn(32, device=DEV)
+    for args in ((x, w, b[:16]), (x, w, b.half()), (x, w, b.cpu()), (x, w.cpu(), b), (x, w[:, :32], b), (x, w.half(), b)):
+        with pytest.raises(RuntimeError):
+            ops.linear(*args)
+    _close("broadcast bias", ops.linear(x, w, b[:1]), x.double().cpu() @ w.double().cpu().t() + b[0].double().cpu(),
+           x.double().cpu().abs() @ w.double().cpu().abs().t() + b[0].abs().double().cpu(), 65, torch.float32)
+    # strided bias, residual off the 16-byte boundary, residual of another shape
+    ref = torch.nn.functional.linear(x.double(), w.double(), b[::2].double().repeat(2)).cpu()
+    mag = x.double().cpu().abs() @ w.double().cpu().abs().t() + b.abs().max().double().cpu()
+    _close("strided", ops.linear(x, w, torch.stack([b[::2].repeat(2), b], 1)[:, 0]), ref, mag, 65, torch.float32)
+    res = torch.randn(4 * 32 + 1, device=DEV)[1:].view(4, 32)
+    _close("residual", ops.linear(x, w, None, res), (x.double() @ w.double().t() + res.double()).cpu(), mag + res.abs().double().cpu(), 65, torch.float32)
+    assert ops.linear(x, w, None, res[:1]).shape == (4, 32)
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(6, 16, 8), (2048, 512, 2048)])      # matrix kernel, library product
+def test_gradients_that_lie_on_top_of_each_other(rows, ins, outs):
+    """An output summed over its rows (or altogether) sends back one row for all of them."""
+    x, w, b = (torch.randn(*s, device=DEV, requires_grad=True) for s in ((rows, ins), (outs, ins), (outs,)))
+    v = torch.randn(outs, device=DEV)
+    for loss in (lambda y: (y.sum(0) * v).sum(), lambda y: y.sum()):
+        got = torch.autograd.grad(loss(ops.linear(x, w, b)), (x, w, b))
+        xd, wd, bd = (t.detach().double().requires_grad_() for t in (x, w, b))
+        ref = torch.autograd.grad(loss(torch.nn.functional.linear(xd, wd, bd)), (xd, wd, bd))
+        for name, g, r, mag in zip(("dx", "dw", "db"), got, ref, (v.abs().double() @ wd.abs() + wd.abs().sum(0), (v.abs().double()[:, None] + 1) * xd.abs().sum(0),
+                                                                  rows * (v.abs().double() + 1))):
+            _close(name, g, r.detach().cpu(), mag.detach().expand(r.shape).cpu(), max(rows, outs), torch.float32)
+
+
+def test_transforms_see_a_library_product():
+    """Second derivatives, torch.func and forward-mode AD go through a projection as they do through torch.nn.functional.linear."""
+    x, w = torch.randn(5, 24, device=DEV, requires_grad=True), torch.randn(16, 24, device=DEV, requires_grad=True)
+    f, ref = (lambda a, b: ops.linear(a, b).pow(3).sum()), (lambda a, b: torch.nn.functional.linear(a, b).pow(3).sum())
+
+    def second(fn, a, b):
+        ga, gb = torch.autograd.grad(fn(a, b), (a, b), create_graph=True)
+        return torch.autograd.grad(ga.pow(2).sum() + gb.pow(2).sum(), (a, b))
+    exact = second(ref, x.detach().double().requires_grad_(), w.detach().double().requires_grad_())
+    for got, r in zip(second(f, x, w), exact):             # float32 sums of at most 24 terms in four nested products
+        assert float((got.double() - r).norm() / r.norm()) < 4 * 24 * 2.0 ** -24
+    t = torch.randn_like(x)
+    for a, b in ((torch.func.jvp(lambda q: ops.linear(q, w), (x,), (t,))[1], t @ w.t()),
+                 (torch.func.vmap(lambda q: ops.linear(q, w))(x), x @ w.t()),
+                 (torch.func.grad(lambda q: f(q, w))(x), torch.func.grad(lambda q: ref(q, w))(x))):
+        assert float((a - b).norm() / b.norm()) < 24 * 2.0 ** -23
