@@ -537,10 +537,24 @@ bool plain_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     return at::autocast::is_autocast_enabled(at::kCUDA) || transforming() || transformed(x) || transformed(w) || (b.has_value() && transformed(*b));
 }
 
+// Forward products alone (inference) over a long contraction stay on the library: mi_gemm walks it in one chain per workgroup, the library
+// splits it.  16-bit, 32 rows, us on the device / issued one by one, mi_gemm and library: 2048 -> 2048 10.5 / 10.3 and
+// 8.4 / 17.5; 2816 -> 1024 13.1 / 13.0 and 7.3 / 17.6; 4096 -> 4096 20.6 / 20.1 and 13.2 / 18.2; 8192 -> 1024 35.0 / 34.7 and
+// 15.0 / 17.9.  A training step keeps mi_gemm (4096 -> 4096 60 and 110, 8192 -> 1024 56 and 109: its gradients are one launch), and
+// up to MI_ROWS_MAX rows have a kernel that splits the contraction.
+bool long_chain(const Tensor& x) {
+    return x.scalar_type() != at::kFloat && x.size(-1) >= 3072 && x.numel() / x.size(-1) > MI_ROWS_MAX;
+}
+bool differentiated(const Tensor& t) { return t.requires_grad() && at::GradMode::is_enabled(); }
+
 std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases) {
     TORCH_CHECK(weights.size() == biases.size() && weights.size() >= 1 && weights.size() <= 3, "projections: one to three weights");
     bool plain = false;
     for (size_t i = 0; i < weights.size(); ++i) plain = plain || plain_linear(x, weights[i], biases[i]);
+    if (!plain && long_chain(x)) {
+        plain = !differentiated(x);
+        for (size_t i = 0; i < weights.size(); ++i) plain = plain && !differentiated(weights[i]) && !(biases[i].has_value() && differentiated(*biases[i]));
+    }
     if (plain) {
         std::vector<Tensor> out;
         for (size_t i = 0; i < weights.size(); ++i) out.push_back(at::linear(x, weights[i], biases[i]));
@@ -560,7 +574,8 @@ Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b, const Opt
         return residual->scalar_type() == x.scalar_type() && residual->device() == x.device() && residual->dim() == x.dim() &&
                residual->size(-1) == w.size(0) && residual->sizes().slice(0, x.dim() - 1) == x.sizes().slice(0, x.dim() - 1) && !transformed(*residual);
     };
-    const bool plain = plain_linear(x, w, b);
+    const bool plain = plain_linear(x, w, b) || (long_chain(x) && !differentiated(x) && !differentiated(w) && !(b.has_value() && differentiated(*b)) &&
+                                                 !(residual.has_value() && differentiated(*residual)));
     if (plain || (residual.has_value() && !residual_fits())) {
         const Tensor y = plain ? at::linear(x, w, b) : op_linear(x, w, b, std::nullopt);
         return residual.has_value() ? y + *residual : y;
