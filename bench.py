@@ -310,7 +310,7 @@ def attention_float32_case(steps, warmup):
     flops = 14 * d * nq * (T * (T + 1) // 2)
     return {"ms_step": ms, "ms_fwd": ms_fwd, "tflops_step": flops / (ms * 1e-3) / 1e12,
             "frac_of_fp32_mfma_peak": flops / (ms * 1e-3) / 1e12 / 157.3,
-            "note": "float32 q / k / v / o, fp32 probabilities; completeness path, one wavefront per 32 x 32 tile"}
+            "note": "float32 q / k / v / o, fp32 probabilities"}
 
 
 def bandwidth_cases(steps, warmup):
