@@ -458,6 +458,8 @@ struct Projections : Function<Projections> {
             dy[i] = g[i].reshape({rows, saved[1 + i].size(0)});
             if (!again && !aligned(dy[i])) dy[i] = dy[i].contiguous();
             small = small && aligned(dy[i]) && small_product(x, rows, dy[i].size(1), in);
+            // the forward product may have been the library's, and saved-tensor hooks may bring the weight back in another layout
+            if (need_dx) small = small && aligned(saved[1 + i]);
         }
         Tensor dx;
         if (small) {

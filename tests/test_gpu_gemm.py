@@ -88,6 +88,40 @@ def test_operands_that_do_not_fit_are_the_librarys():
     assert ops.linear(x, w, None, res[:1]).shape == (4, 32)
 
 
+# a weight that the library takes and mi_gemm does not: strided rows, a transposed matrix, rows off the 16-byte boundary
+WEIGHT_VIEWS = {
+    "every second column": lambda w: torch.stack([w, torch.zeros_like(w)], 2)[..., 0],
+    "transposed": lambda w: w.t().contiguous().t(),
+    "off the boundary": lambda w: torch.cat([w.new_zeros(1), w.flatten()])[1:].view_as(w),
+    "rows of an odd stride": lambda w: torch.cat([w, w.new_zeros(w.shape[0], 3)], 1)[:, :-3],
+}
+
+
+@pytest.mark.parametrize("view", list(WEIGHT_VIEWS))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gradients_with_weights_in_other_layouts(view, dtype):
+    """Input, weight and bias gradients of one projection and of two that share their input (one of them in the other layout)."""
+    print(f"case gemm weight view={view} dtype={dtype}", flush=True)
+    x, ws, bs, dys = _case(24, 64, (32, 16), dtype, 11)
+    wg = [WEIGHT_VIEWS[view](ws[0].to(DEV)).detach().requires_grad_(), ws[1].to(DEV).requires_grad_()]
+    assert torch.equal(wg[0].detach().cpu(), ws[0])
+    for n in (1, 2):
+        xg, bg = x.to(DEV).requires_grad_(), bs[0].to(DEV).requires_grad_()
+        for w in wg:
+            w.grad = None
+        ys = [ops.linear(xg, wg[0], bg)] if n == 1 else ops.projections(xg, wg, [bg, None])
+        torch.autograd.backward(ys, [d.to(DEV) for d in dys[:n]])
+        xd, wd, dyd = x.double(), [w.double() for w in ws[:n]], [d.double() for d in dys[:n]]
+        dx, mag = sum(d @ w for d, w in zip(dyd, wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd, wd))
+        # a library product per projection: the first is rounded before the second is added
+        slack = HALF_ULP[dtype] * (dyd[0] @ wd[0]).abs() if n == 2 else torch.zeros_like(dx)
+        err = (xg.grad.double().cpu() - dx).abs()
+        assert bool((err <= (HALF_ULP[dtype] * dx.abs() + slack + 49 * 2.0 ** -24 * mag + 2.0 ** -133) * 1.001).all()), (n, float(err.max()))
+        for i in range(n):
+            _close(f"dw{i}", wg[i].grad, dyd[i].t() @ xd, dyd[i].abs().t() @ xd.abs(), 24, dtype)
+        _close("db", bg.grad, dyd[0].sum(0), dyd[0].abs().sum(0), 24, dtype)
+
+
 @pytest.mark.parametrize("rows,ins,outs", [(6, 16, 8), (2048, 512, 2048)])      # matrix kernel, library product
 def test_gradients_that_lie_on_top_of_each_other(rows, ins, outs):
     """An output summed over its rows (or altogether) sends back one row for all of them."""
