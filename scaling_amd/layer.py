@@ -127,7 +127,11 @@ class TransformerLayer(torch.nn.Module):
             a = self.self_attention(n, cumulative_seq_lengths=x.cumulative_seq_lengths,
                                     attention_scores_manipulation=x.attention_scores_manipulation, position_ids=x.position_ids,
                                     use_cache=use_cache, reset_cache=reset_cache, cache_index=cache_index)
-            h, n = self.post_attention_layernorm.with_residual(self.dropout_attention(a), h)
+            a = self.dropout_attention(a)
+            if a.dtype == h.dtype and a.shape == h.shape:
+                h, n = self.post_attention_layernorm.with_residual(a, h)
+            else:                                        # under autocast: the sum promotes
+                h, n = self.post_attention_layernorm.with_residual(a + h)
             if fuses_residual(self.mlp) and (self.dropout_mlp.p == 0.0 or not self.dropout_mlp.training):
                 h = self.mlp(n, h)
             else:

@@ -5,6 +5,8 @@ import pytest
 import torch
 
 from scaling_amd import _lib, ops
+from scaling_amd.config import TransformerArchitectureConfig
+from scaling_amd.layer import TransformerLayer, TransformerLayerIO
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -64,6 +66,52 @@ def test_norm_outputs_that_do_not_reach_the_loss():
     a = x.detach().clone().requires_grad_()
     ops.rms_norm(a + a, w.detach(), 1e-5).sum().backward()
     assert torch.equal(x.grad, a.grad)
+
+
+def _layer(dtype, default, hidden=256, inter=2.75, heads=4, **options):
+    """The default block (LayerNorm, one QKV projection, GELU MLP, biases) or RMSNorm, grouped heads, SwiGLU without biases."""
+    torch.manual_seed(7)
+    own = dict(mlp_type="default", mlp_factor=4.0) if default else dict(norm_type="rms", mlp_type="swiglu", mlp_factor=inter, attention_bias=False,
+                                                                        mlp_bias=False, attention_qkv_in_one=False, attention_num_kv_heads=heads // 2)
+    cfg = TransformerArchitectureConfig.from_dict(dict(
+        vocab_size=64, hidden_size=hidden, num_layers=1, num_attention_heads=heads, sequence_length=512, precision=dtype,
+        dropout_embedding=0.0, dropout_attention_probs=0.0, dropout_after_attention=0.0, dropout_after_mlp=0.0,
+        masked_softmax={"kernel": "hip"}, **own, **options))
+    return TransformerLayer(cfg, 0, device=torch.device(DEV))
+
+
+def _io(x):
+    b, s, _ = x.shape
+    return TransformerLayerIO(activations=x, position_ids=torch.arange(s, device=DEV).repeat(b, 1),
+                              cumulative_seq_lengths=torch.arange(0, b * s + 1, s, dtype=torch.int32, device=DEV))
+
+
+def _step(layer, forward, x, dy):
+    """Output and every gradient of one step."""
+    layer.zero_grad(set_to_none=True)
+    x = x.clone().requires_grad_()
+    y = forward(x)
+    y.backward(dy)
+    return [y.detach(), x.grad] + [p.grad for p in layer.parameters()]
+
+
+def _blocks(layer, x):
+    """The layer's two blocks, with every residual sum a launch of its own."""
+    io = _io(x)
+    return layer.mlp_block(layer.attention_block(io.activations, io.cumulative_seq_lengths, io.position_ids))
+
+
+@pytest.mark.parametrize("default", [True, False])
+def test_float32_layer_under_autocast(default):
+    """The projections run in bf16 and the residual stream stays float32.  The fused norms' float32 input gradients may differ in the
+    last place, which can turn a bf16 rounding further down: less than one such rounding of a gradient altogether."""
+    layer = _layer("float32", default)
+    x, dy = (torch.randn(2, 100, 256, device=DEV, generator=torch.Generator(DEV).manual_seed(s)) for s in (1, 2))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        want, got = _step(layer, lambda t: _blocks(layer, t), x, dy), _step(layer, lambda t: layer(_io(t)).activations, x, dy)
+    assert got[0].dtype == torch.float32 and torch.equal(want[0], got[0])
+    for a, b in zip(want, got):
+        assert a.dtype == b.dtype and float((a - b).norm()) <= 2.0 ** -8 * float(a.norm())
 
 
 @pytest.mark.parametrize("heads,d,rotary,causal,docs", [(3, 64, True, True, (40,)), (2, 128, True, False, ()), (2, 96, False, True, (7, 100)), (4, 32, False, True, ())])
