@@ -773,10 +773,11 @@ struct AttentionQkv : Function<AttentionQkv> {
         const auto s = ctx->get_saved_variables();
         AttnOptions opts = kept_options(ctx);
         opts.cos = s[7]; opts.sin = s[8]; opts.pos_q = s[9]; opts.pos_k = s[10];
-        const Tensor& q = s[0];
-        const int64_t d = q.size(2);
-        const Tensor dqkv = at::empty({q.size(0), q.size(1), 3 * d}, q.options());
-        attn_backward(g[0], q, s[1], s[2], s[3], s[4], s[5], s[6], opts, dqkv.narrow(2, 0, d), dqkv.narrow(2, d, d), dqkv.narrow(2, 2 * d, d), Tensor());
+        const int64_t d = s[0].size(2);
+        const Tensor dqkv = at::empty({s[0].size(0), s[0].size(1), 3 * d}, s[0].options()), dq = dqkv.narrow(2, 0, d);
+        // saved-tensor hooks (activations kept on the host) may bring q back with rows of its own instead of a slice of qkv's
+        const Tensor q = s[0].strides() == dq.strides() ? s[0] : at::empty_strided(dq.sizes(), dq.strides(), dq.options()).copy_(s[0]);
+        attn_backward(g[0], q, s[1], s[2], s[3], s[4], s[5], s[6], opts, dq, dqkv.narrow(2, d, d), dqkv.narrow(2, 2 * d, d), Tensor());
         return {dqkv, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };

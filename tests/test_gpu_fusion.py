@@ -114,6 +114,21 @@ def test_float32_layer_under_autocast(default):
         assert a.dtype == b.dtype and float((a - b).norm()) <= 2.0 ** -8 * float(a.norm())
 
 
+@pytest.mark.parametrize("default", [True, False])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_layer_with_activations_kept_on_the_host(default, dtype):
+    """What saved-tensor hooks bring back has other addresses and may have other strides; the step is the same to the bit."""
+    layer = _layer(dtype, default)
+    x, dy = (torch.randn(2, 100, 256, device=DEV, generator=torch.Generator(DEV).manual_seed(s)).to(getattr(torch, dtype)) for s in (1, 2))
+
+    def forward(t):
+        return layer(_io(t)).activations
+    want = _step(layer, forward, x, dy)
+    with torch.autograd.graph.save_on_cpu():
+        got = _step(layer, forward, x, dy)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
 @pytest.mark.parametrize("heads,d,rotary,causal,docs", [(3, 64, True, True, (40,)), (2, 128, True, False, ()), (2, 96, False, True, (7, 100)), (4, 32, False, True, ())])
 def test_packed_qkv_attention_matches_three_slices(heads, d, rotary, causal, docs):
     print(f"case attention_qkv heads={heads} d={d} rotary={rotary}", flush=True)
