@@ -12,6 +12,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -888,6 +889,7 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
         ctx->set_materialize_grads(false);
         ctx->mark_non_differentiable({argmax, accuracy});
         ctx->save_for_backward({dh, dw});
+        ctx->saved_data["hooked"] = at::SavedTensorDefaultHooks::get_hooks().has_value();
         ctx->saved_data["dtype"] = (int64_t)weight.scalar_type();
         return {loss, argmax, accuracy};
     }
@@ -896,8 +898,8 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
         if (!g[0].defined()) return grads;
         const auto saved = ctx->get_saved_variables();
         // A graph that is used up by this pass hands its gradients over, scaled in place; one that is kept (or differentiated
-        // further) keeps them.
-        const bool hand_over = !torch::autograd::get_current_graph_task_keep_graph() && !at::GradMode::is_enabled();
+        // further) keeps them, and what a saved-tensor hook returns belongs to the hook.
+        const bool hand_over = !torch::autograd::get_current_graph_task_keep_graph() && !at::GradMode::is_enabled() && !ctx->saved_data["hooked"].toBool();
         const Tensor dloss = g[0].contiguous();
         for (int i = 0; i < 2; ++i) {
             const Tensor& x = saved[i];

@@ -313,3 +313,26 @@ def test_linear_cross_entropy_gradients_are_kept_with_the_graph(chunk):
     two = torch.autograd.grad(loss * 2.0, (h, w))     # the last pass hands the gradients over
     for a, b in zip(kept, two):
         assert torch.equal(a * 2, b)                  # a power of two: exact
+
+
+@pytest.mark.parametrize("chunk", [64, 8192])
+def test_lm_head_gradients_under_saved_tensor_hooks(chunk):
+    """The gradients that the forward pass leaves are handed over scaled in place, but not where a hook holds them."""
+    g = torch.Generator(DEV).manual_seed(2)
+    h, w = torch.randn(100, 64, generator=g, device=DEV).bfloat16(), torch.randn(300, 64, generator=g, device=DEV).bfloat16()
+    targets, weights = torch.randint(0, 300, (100,), generator=g, device=DEV), torch.rand(100, generator=g, device=DEV)
+    held = []
+
+    def step():
+        a, b = h.clone().requires_grad_(), w.clone().requires_grad_()
+        (3.0 * ops.linear_cross_entropy(a, b, targets, weights, chunk)[0]).backward()
+        return a.grad, b.grad
+
+    def pack(t):
+        held.append((t, t.detach().clone()))
+        return t
+    want = step()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        got = step()
+    assert held and all(torch.equal(t, before) for t, before in held)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
