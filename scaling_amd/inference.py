@@ -153,7 +153,7 @@ class TransformerInferenceModule(torch.nn.Module):
         """(cache, arguments of ops.decode_layer) per layer for the next `tokens` cached steps, or None where a layer or this module
         is not the package's own as it is."""
         layers = list(self._layers[1:-2])
-        if type(self).forward is not TransformerInferenceModule.forward or not layers or \
+        if type(self).forward is not TransformerInferenceModule.forward or "forward" in self.__dict__ or not layers or \
                 not all(type(layer) is TransformerLayer and _unhooked(layer) and layer._decodes_natively() for layer in layers):
             return None
         native = [(layer.self_attention.cache.get(0), decode_arguments(layer, batch, tokens, 0)) for layer in layers]

@@ -10,7 +10,7 @@ from typing import Callable, List, Optional
 import torch
 
 from .config import MLPType, TransformerArchitectureConfig
-from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm
+from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm, idle_dropout
 
 
 class InferenceSettings:
@@ -114,13 +114,11 @@ class TransformerLayer(torch.nn.Module):
         s = x.inference_settings
         use_cache, reset_cache, cache_index = (False, False, 0) if s is None else (s.use_cache, s.reset_cache, s.cache_index)
         assert x.cumulative_seq_lengths is not None
-        cls = type(self)
-        blocks_as_here = cls.attention_block is TransformerLayer.attention_block and cls.mlp_block is TransformerLayer.mlp_block
         if use_cache and not reset_cache and x.attention_scores_manipulation is None and self._decodes_natively():
             h = decode_layer(self, x.activations, x.cumulative_seq_lengths, x.position_ids, cache_index)
             if h is not None:
                 return self._next(x, h)
-        if blocks_as_here and fuses_residual(self.input_layernorm) and fuses_residual(self.post_attention_layernorm):
+        if self._own_blocks() and fuses_residual(self.input_layernorm) and fuses_residual(self.post_attention_layernorm):
             # the same arithmetic as attention_block and mlp_block, with the residual stream taken through the norms (and, where
             # nothing comes between, the last projection): its sums and the sums of its gradients need no passes of their own
             h, n = self.input_layernorm.with_residual(x.activations)
@@ -132,7 +130,7 @@ class TransformerLayer(torch.nn.Module):
                 h, n = self.post_attention_layernorm.with_residual(a, h)
             else:                                        # under autocast: the sum promotes
                 h, n = self.post_attention_layernorm.with_residual(a + h)
-            if fuses_residual(self.mlp) and (self.dropout_mlp.p == 0.0 or not self.dropout_mlp.training):
+            if fuses_residual(self.mlp) and idle_dropout(self.dropout_mlp):
                 h = self.mlp(n, h)
             else:
                 h = self.dropout_mlp(self.mlp(n)) + h
@@ -151,18 +149,23 @@ class TransformerLayer(torch.nn.Module):
                                   loss_weights=x.loss_weights, position_ids=x.position_ids,
                                   inference_settings=x.inference_settings, embeddings=x.embeddings)
 
+    def _own_blocks(self) -> bool:
+        cls = type(self)
+        return cls.attention_block is TransformerLayer.attention_block and cls.mlp_block is TransformerLayer.mlp_block and \
+            not ("attention_block" in self.__dict__ or "mlp_block" in self.__dict__)
+
     def _decodes_natively(self) -> bool:
         """Whether a cached step may go through `decode_layer`: inference on this package's own modules that nobody replaced or
         hooked, in the form that function covers (RMSNorm, separate q / k / v, SwiGLU, no biases)."""
-        att, mlp, cls = self.self_attention, self.mlp, type(self)
-        return (cls.attention_block is TransformerLayer.attention_block and cls.mlp_block is TransformerLayer.mlp_block and not self.training and not torch.is_grad_enabled()
-                and not torch.is_autocast_enabled() and type(att) is ParallelSelfAttention and type(mlp) is ParallelSwiGLUMLP and not att.qkv_in_one
-                and att._fusable_rotary and att.causal and not att.key_query_norm
-                and type(self.input_layernorm) is RMSNorm and type(self.post_attention_layernorm) is RMSNorm
-                and all(_unhooked(m) for m in (att, mlp, self.input_layernorm, self.post_attention_layernorm, self.dropout_attention,
-                                               self.dropout_mlp))
-                and _direct(att.query, att.key, att.value, att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out)
-                and att.dense.bias is None and att.query.bias is None and mlp.dense_in.bias is None)
+        att, mlp = self.self_attention, self.mlp
+        if not (self._own_blocks() and not self.training and not torch.is_grad_enabled() and not torch.is_autocast_enabled() and
+                type(att) is ParallelSelfAttention and type(mlp) is ParallelSwiGLUMLP and not att.qkv_in_one and att._fusable_rotary and
+                att.causal and not att.key_query_norm and type(self.input_layernorm) is RMSNorm and
+                type(self.post_attention_layernorm) is RMSNorm and idle_dropout(self.dropout_attention) and idle_dropout(self.dropout_mlp)):
+            return False
+        linears = (att.query, att.key, att.value, att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out)
+        return _direct(*linears) and all(m.bias is None for m in linears) and \
+            all(_unhooked(m) for m in (att, mlp, self.input_layernorm, self.post_attention_layernorm))
 
 
 class LayerNormWrapper(torch.nn.Module):

@@ -73,12 +73,20 @@ class _Linear(torch.nn.Module):
 
 
 def _unhooked(m: torch.nn.Module) -> bool:
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    """Whether calling the module runs its class's forward and nothing else: no hooks on it or on all modules, no forward of the
+    instance's own (as wrapper libraries set it), not compiled."""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__ or
+                m._compiled_call_impl is not None or torch.nn.modules.module._has_any_global_hook())
 
 
 def _direct(*modules: torch.nn.Module) -> bool:
     """Whether calling the modules comes to using their weights: plain projections that nobody replaced or hooked."""
     return all(type(m) is _Linear and _unhooked(m) for m in modules)
+
+
+def idle_dropout(m: torch.nn.Module) -> bool:
+    """Whether the module may be left out: torch's dropout, unhooked, that drops nothing now."""
+    return type(m) is torch.nn.Dropout and _unhooked(m) and (m.p == 0.0 or not m.training)
 
 
 def fuses_residual(m: torch.nn.Module) -> bool:

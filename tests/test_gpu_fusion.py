@@ -6,7 +6,7 @@ import torch
 
 from scaling_amd import _lib, ops
 from scaling_amd.config import TransformerArchitectureConfig
-from scaling_amd.layer import TransformerLayer, TransformerLayerIO
+from scaling_amd.layer import InferenceSettings, TransformerLayer, TransformerLayerIO
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -127,6 +127,76 @@ def test_layer_with_activations_kept_on_the_host(default, dtype):
     with torch.autograd.graph.save_on_cpu():
         got = _step(layer, forward, x, dy)
     assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+def _watch(layer, how, path, calls):
+    """Lets `calls` see every call of the module at `path`; returns what undoes a global registration."""
+    name = path.split(".")[-1]
+    parent = layer.get_submodule(path[:-len(name)].rstrip("."))
+    module = getattr(parent, name)
+    if how == "hook":
+        module.register_forward_hook(lambda m, a, y: calls.append(path))
+    elif how == "global hook":
+        return torch.nn.modules.module.register_module_forward_hook(lambda m, a, y: calls.append(path) if m is module else None)
+    elif how == "own forward":
+        inner = module.forward
+        module.forward = lambda *a, **k: (calls.append(path), inner(*a, **k))[1]
+    else:
+        class Replacement(torch.nn.Module):
+            def __init__(self):
+                super().__init__()
+                self.inner = module
+
+            def forward(self, x):
+                calls.append(path)
+                return self.inner(x)
+        setattr(parent, name, Replacement())
+
+
+WATCHED = ["input_layernorm", "post_attention_layernorm", "dropout_attention", "dropout_mlp", "self_attention.dense", "mlp", "mlp.dense_in",
+           "mlp.siglu_weight", "mlp.dense_out"]
+
+
+@pytest.mark.parametrize("how", ["hook", "global hook", "own forward", "replaced"])
+@pytest.mark.parametrize("path", WATCHED + ["self_attention.query", "self_attention.value"])
+def test_watched_or_replaced_modules_are_called(how, path):
+    """A module that somebody observes or replaces is called in a training step and (but for the stacked q / k / v of inference) in a
+    cached decode step, whose results stay what they were."""
+    print(f"case watched {how} {path}", flush=True)
+    layer = _layer("bfloat16", False)
+    x, dy = (torch.randn(2, 40, 256, device=DEV, generator=torch.Generator(DEV).manual_seed(s)).bfloat16() for s in (1, 2))
+
+    def decode():
+        layer.eval()
+        with torch.no_grad():
+            io = _io(x)
+            io.inference_settings = InferenceSettings(use_cache=True, reset_cache=True)
+            layer(io)
+            calls.clear()
+            one = TransformerLayerIO(activations=x[:, :1].contiguous(), position_ids=torch.full((2, 1), 40, device=DEV),
+                                     cumulative_seq_lengths=torch.arange(3, dtype=torch.int32, device=DEV),
+                                     inference_settings=InferenceSettings(use_cache=True, reset_cache=False))
+            y = layer(one).activations
+        layer.train()
+        return y
+    calls = []
+    want, token = _step(layer, lambda t: layer(_io(t)).activations, x, dy), decode()
+    handle = _watch(layer, how, path, calls)
+    try:
+        calls.clear()
+        got = _step(layer, lambda t: layer(_io(t)).activations, x, dy)
+        assert calls == [path]
+        # the same outputs; gradients of projections that share their input are rounded before they are summed, and the products of a
+        # decode step are summed in another order: one rounding at each of the eight places where either stores a result
+        assert torch.equal(want[0], got[0])
+        assert float((want[1] - got[1]).float().norm()) <= 8 * 2.0 ** -8 * float(want[1].float().norm())
+        if path in WATCHED:
+            y = decode()
+            assert calls == [path]
+            assert float((y - token).float().norm()) <= 8 * 2.0 ** -8 * float(token.float().norm())
+    finally:
+        if handle is not None:
+            handle.remove()
 
 
 @pytest.mark.parametrize("heads,d,rotary,causal,docs", [(3, 64, True, True, (40,)), (2, 128, True, False, ()), (2, 96, False, True, (7, 100)), (4, 32, False, True, ())])
