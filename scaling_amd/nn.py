@@ -570,7 +570,11 @@ class ParallelSelfAttention(torch.nn.Module):
             self._check_positions(pos)
             cu_k = None if cumulative_seq_lengths_key is None else cumulative_seq_lengths_key.to(torch.int32)
             rotary = (*self.rotary_embedding.tables(), pos, pos) if self.rotary_embedding is not None else None
-            ctx = sdpa.forward_qkv(self.query_key_value(x).view(b * s, nq, 3 * d), cu, cu_k, rotary)
+            qkv = self.query_key_value(x).view(b * s, nq, 3 * d)
+            if qkv.is_contiguous() and type(sdpa).forward_tokens is ScaledDotProductAttention.forward_tokens and "forward_tokens" not in sdpa.__dict__:
+                ctx = sdpa.forward_qkv(qkv, cu, cu_k, rotary)
+            else:                                        # a core or a projection that somebody replaced
+                ctx = sdpa.forward_tokens(qkv[..., :d], qkv[..., d:2 * d], qkv[..., 2 * d:], cu, cu_k, rotary=rotary)
             return self.dense(ctx.view(b, s, nq * d))
         q, k, v = self._project(x)
         if self.key_query_norm:

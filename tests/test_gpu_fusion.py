@@ -199,6 +199,52 @@ def test_watched_or_replaced_modules_are_called(how, path):
             handle.remove()
 
 
+class _WideProjection(torch.nn.Module):
+    """The projection `inner` as the first columns of a wider product."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        y = self.inner(x)
+        return torch.cat([y, y[..., :8]], -1)[..., :y.shape[-1]]
+
+
+class _OwnCore(torch.nn.Module):
+    """An attention core with the token-major call alone."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner, self.called = inner, 0
+
+    def forward_tokens(self, *args, **kw):
+        self.called += 1
+        return self.inner.forward_tokens(*args, **kw)
+
+
+@pytest.mark.parametrize("how", ["projection", "core", "core's method"])
+def test_packed_qkv_with_a_replaced_projection_or_core(how):
+    layer = _layer("bfloat16", True)
+    x, dy = (torch.randn(2, 40, 256, device=DEV, generator=torch.Generator(DEV).manual_seed(s)).bfloat16() for s in (1, 2))
+
+    def forward(t):
+        return layer(_io(t)).activations
+    want = _step(layer, forward, x, dy)
+    att = layer.self_attention
+    core, calls = att.scaled_dot_product_attention, []
+    if how == "projection":
+        att.query_key_value = _WideProjection(att.query_key_value)
+    elif how == "core":
+        att.scaled_dot_product_attention = _OwnCore(core)
+    else:
+        own = core.forward_tokens
+        core.forward_tokens = lambda *a, **k: (calls.append(1), own(*a, **k))[1]
+    got = _step(layer, forward, x, dy)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+    assert how == "projection" or (calls or att.scaled_dot_product_attention.called == 1)
+
+
 @pytest.mark.parametrize("heads,d,rotary,causal,docs", [(3, 64, True, True, (40,)), (2, 128, True, False, ()), (2, 96, False, True, (7, 100)), (4, 32, False, True, ())])
 def test_packed_qkv_attention_matches_three_slices(heads, d, rotary, causal, docs):
     print(f"case attention_qkv heads={heads} d={d} rotary={rotary}", flush=True)
