@@ -337,6 +337,16 @@ bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
     const double work = 2.0 * (double)m * (double)n * (double)k;
     return n % v == 0 && k % v == 0 && work <= (v == 4 ? 0.75e9 : 3e9);
 }
+// Forward products of inference (modules in eval mode) over a long contraction stay on the library: mi_gemm walks it in one chain per
+// workgroup, the library splits it.  16-bit, 32 rows, us on the device / issued one by one, mi_gemm and library: 2048 -> 2048
+// 10.5 / 10.3 and 8.4 / 17.5; 2816 -> 1024 13.1 / 13.0 and 7.3 / 17.6; 4096 -> 4096 20.6 / 20.1 and 13.2 / 18.2; 8192 -> 1024
+// 35.0 / 34.7 and 15.0 / 17.9.  A training step, which the host bounds at these sizes, keeps mi_gemm (forward and both gradients,
+// issued one by one, with either forward product: 4096 -> 4096 57 and 74, 8192 -> 1024 54 and 76).  Up to MI_ROWS_MAX rows have a
+// kernel that splits the contraction.  Whether gradients are wanted does not matter: reentrant checkpointing runs a layer without
+// and again with them and counts on the same bits.
+bool long_chain(const Tensor& t, int64_t rows, int64_t k) {
+    return t.scalar_type() != at::kFloat && k >= 3072 && rows > MI_ROWS_MAX;
+}
 bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
@@ -395,13 +405,14 @@ struct Projections : Function<Projections> {
         return at;
     }
     // residual (one projection only): added to the output
-    static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, const OptTensor& residual, const std::vector<int64_t>& has_bias) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, const OptTensor& residual, const std::vector<int64_t>& has_bias,
+                                 bool inference) {
         const int64_t n = (int64_t)has_bias.size(), in = x.size(-1);
         const auto at = bias_at(has_bias);
         const Tensor x2 = x.reshape({-1, in});
         const int64_t rows = x2.size(0);
         variable_list saved{x}, out;                      // x itself: what is differentiated again reaches it
-        bool small = aligned(x2);
+        bool small = aligned(x2) && !(inference && long_chain(x, rows, in));
         for (int64_t i = 0; i < n; ++i) {
             const Tensor& w = params[i];
             small = small && aligned(w) && small_product(x, rows, w.size(0), in);
@@ -514,7 +525,7 @@ struct Projections : Function<Projections> {
             if (at[i] >= 0) grads.push_back(db[i]);
         grads.push_back(g[0]);                             // residual (ignored without one)
         if (!ctx->saved_data["residual"].toBool()) grads.back() = Tensor();
-        grads.emplace_back();                              // has_bias
+        grads.resize(grads.size() + 2);                    // has_bias, inference
         return grads;
     }
 };
@@ -540,24 +551,10 @@ bool plain_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     return at::autocast::is_autocast_enabled(at::kCUDA) || transforming() || transformed(x) || transformed(w) || (b.has_value() && transformed(*b));
 }
 
-// Forward products alone (inference) over a long contraction stay on the library: mi_gemm walks it in one chain per workgroup, the library
-// splits it.  16-bit, 32 rows, us on the device / issued one by one, mi_gemm and library: 2048 -> 2048 10.5 / 10.3 and
-// 8.4 / 17.5; 2816 -> 1024 13.1 / 13.0 and 7.3 / 17.6; 4096 -> 4096 20.6 / 20.1 and 13.2 / 18.2; 8192 -> 1024 35.0 / 34.7 and
-// 15.0 / 17.9.  A training step keeps mi_gemm (4096 -> 4096 60 and 110, 8192 -> 1024 56 and 109: its gradients are one launch), and
-// up to MI_ROWS_MAX rows have a kernel that splits the contraction.
-bool long_chain(const Tensor& x) {
-    return x.scalar_type() != at::kFloat && x.size(-1) >= 3072 && x.numel() / x.size(-1) > MI_ROWS_MAX;
-}
-bool differentiated(const Tensor& t) { return t.requires_grad() && at::GradMode::is_enabled(); }
-
-std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases) {
+std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases, bool inference) {
     TORCH_CHECK(weights.size() == biases.size() && weights.size() >= 1 && weights.size() <= 3, "projections: one to three weights");
     bool plain = false;
     for (size_t i = 0; i < weights.size(); ++i) plain = plain || plain_linear(x, weights[i], biases[i]);
-    if (!plain && long_chain(x)) {
-        plain = !differentiated(x);
-        for (size_t i = 0; i < weights.size(); ++i) plain = plain && !differentiated(weights[i]) && !(biases[i].has_value() && differentiated(*biases[i]));
-    }
     if (plain) {
         std::vector<Tensor> out;
         for (size_t i = 0; i < weights.size(); ++i) out.push_back(at::linear(x, weights[i], biases[i]));
@@ -569,23 +566,22 @@ std::vector<Tensor> op_projections(const Tensor& x, const std::vector<Tensor>& w
         has_bias.push_back(b.has_value());
         if (b.has_value()) params.push_back(*b);
     }
-    return Projections::apply(x, at::TensorList(params), OptTensor(), has_bias);
+    return Projections::apply(x, at::TensorList(params), OptTensor(), has_bias, inference);
 }
 
-Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b, const OptTensor& residual) {
+Tensor op_linear(const Tensor& x, const Tensor& w, const OptTensor& b, const OptTensor& residual, bool inference) {
     const auto residual_fits = [&] {
         return residual->scalar_type() == x.scalar_type() && residual->device() == x.device() && residual->dim() == x.dim() &&
                residual->size(-1) == w.size(0) && residual->sizes().slice(0, x.dim() - 1) == x.sizes().slice(0, x.dim() - 1) && !transformed(*residual);
     };
-    const bool plain = plain_linear(x, w, b) || (long_chain(x) && !differentiated(x) && !differentiated(w) && !(b.has_value() && differentiated(*b)) &&
-                                                 !(residual.has_value() && differentiated(*residual)));
+    const bool plain = plain_linear(x, w, b);
     if (plain || (residual.has_value() && !residual_fits())) {
-        const Tensor y = plain ? at::linear(x, w, b) : op_linear(x, w, b, std::nullopt);
+        const Tensor y = plain ? at::linear(x, w, b) : op_linear(x, w, b, std::nullopt, inference);
         return residual.has_value() ? y + *residual : y;
     }
     variable_list params{w};
     if (b.has_value()) params.push_back(*b);
-    return Projections::apply(x, at::TensorList(params), residual, std::vector<int64_t>{b.has_value()})[0];
+    return Projections::apply(x, at::TensorList(params), residual, std::vector<int64_t>{b.has_value()}, inference)[0];
 }
 
 // ---- attention core ----------------------------------------------------------------------------------------------------

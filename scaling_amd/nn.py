@@ -69,7 +69,7 @@ class _Linear(torch.nn.Module):
             self.register_parameter("bias", None)
 
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
-        return ops.linear(x, self.weight, self.bias, residual)
+        return ops.linear(x, self.weight, self.bias, residual, not self.training)
 
 
 def _unhooked(m: torch.nn.Module) -> bool:
@@ -100,7 +100,7 @@ def fuses_residual(m: torch.nn.Module) -> bool:
 def _project_together(x: torch.Tensor, *modules: torch.nn.Module):
     """The outputs of several projections of one input."""
     if _direct(*modules):
-        return ops.projections(x, [m.weight for m in modules], [m.bias for m in modules])
+        return ops.projections(x, [m.weight for m in modules], [m.bias for m in modules], not any(m.training for m in modules))
     return [m(x) for m in modules]
 
 
@@ -492,7 +492,7 @@ class ParallelSelfAttention(torch.nn.Module):
             # inference (eval mode, so that a no-grad forward that activation checkpointing recomputes with grad takes
             # the same GEMMs both times): one projection GEMM over the row-stacked weights; q, k, v are column slices
             w, bias = self._fused_qkv()
-            out = ops.linear(x, w, bias).view(b * s, (nq + 2 * nkv) * d)
+            out = ops.linear(x, w, bias, inference=True).view(b * s, (nq + 2 * nkv) * d)
             return (out[:, :nq * d].view(b * s, nq, d), out[:, nq * d:(nq + nkv) * d].view(b * s, nkv, d),
                     out[:, (nq + nkv) * d:].view(b * s, nkv, d))
         q, k, v = _project_together(x, self.query, self.key, self.value)

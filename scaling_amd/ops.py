@@ -140,15 +140,16 @@ def swiglu(a: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
 # linear projections
 # ------------------------------------------------------------------------------------------------
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-           residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+           residual: Optional[torch.Tensor] = None, inference: bool = False) -> torch.Tensor:
     """x W^T + b (torch.nn.functional.linear) (+ residual), on the matrix kernel of this package where the product is too small to fill
-    the chip and on the library product elsewhere."""
-    return _lib.host().linear(x, weight, bias, residual)
+    the chip and on the library product elsewhere.  `inference`: no gradients follow, so the forward product alone decides; the same value
+    gives the same bits with and without gradients."""
+    return _lib.host().linear(x, weight, bias, residual, inference)
 
 
-def projections(x: torch.Tensor, weights, biases):
+def projections(x: torch.Tensor, weights, biases, inference: bool = False):
     """[linear(x, w, b) for up to three (w, b)] of one input, whose gradient is then one sum inside the products."""
-    return _lib.host().projections(x, weights, biases)
+    return _lib.host().projections(x, weights, biases, inference)
 
 
 # ------------------------------------------------------------------------------------------------

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from scaling_amd import ops
+from scaling_amd.nn import ParallelSwiGLUMLP
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -54,6 +55,38 @@ def test_projections_and_their_gradients(rows, ins, outs, dtype):
         if bs[i] is not None:
             _close(f"db{i}", bg[i].grad, dyd[i].sum(0), dyd[i].abs().sum(0), rows, dtype)
     _close("dx", xg.grad, sum(d @ w for d, w in zip(dyd, wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd, wd)), sum(outs), dtype)
+
+
+# 16 and 17 rows (the kernel of few rows, the matrix kernel or the library), contractions on both sides of 3072
+@pytest.mark.parametrize("rows,ins,outs", [(16, 4096, (256,)), (17, 3064, (64, 128)), (17, 3072, (64, 128)), (40, 4096, (1024,)), (64, 8192, (512, 256, 256))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_outputs_are_the_same_with_and_without_gradients(rows, ins, outs, dtype):
+    """A forward pass under no_grad that is recomputed with gradients (reentrant checkpointing) has the same bits."""
+    x, ws, bs, dys = _case(rows, ins, outs, dtype, ins)
+    xg, wg, bg = x.to(DEV).requires_grad_(), [w.to(DEV).requires_grad_() for w in ws], [None if b is None else b.to(DEV) for b in bs]
+    res = dys[0].to(DEV)
+    calls = (lambda i: ops.projections(xg, wg, bg, *i), lambda i: [ops.linear(xg, wg[0], bg[0], None, *i)], lambda i: [ops.linear(xg, wg[0], None, res, *i)])
+    for inference in ((), (True,)):
+        for call in calls:
+            with torch.no_grad():
+                want = call(inference)
+            assert all(torch.equal(a, b) for a, b in zip(want, call(inference)))
+
+
+def test_reentrant_checkpoint_over_a_long_contraction():
+    """The MLP of a layer whose second product contracts over 4096 features, 24 rows: loss and gradients of a plain step."""
+    from torch.utils.checkpoint import checkpoint
+    torch.manual_seed(3)
+    mlp = ParallelSwiGLUMLP(io_features=1024, intermediate_feature_factor=4.0, bias=False, device=torch.device(DEV), dtype=torch.bfloat16)
+    x = torch.randn(24, 1024, device=DEV).bfloat16()
+
+    def step(forward):
+        mlp.zero_grad(set_to_none=True)
+        a = x.clone().requires_grad_()
+        y = forward(a)
+        y.float().pow(2).sum().backward()
+        return [y.detach(), a.grad] + [p.grad for p in mlp.parameters()]
+    assert all(torch.equal(a, b) for a, b in zip(step(mlp), step(lambda t: checkpoint(mlp, t, use_reentrant=True))))
 
 
 def test_projection_that_does_not_reach_the_loss():
