@@ -169,6 +169,18 @@ def test_gradients_that_lie_on_top_of_each_other(rows, ins, outs):
             _close(name, g, r.detach().cpu(), mag.detach().expand(r.shape).cpu(), max(rows, outs), torch.float32)
 
 
+@pytest.mark.parametrize("rows,ins,outs", [(6, 16, 8), (2048, 512, 2048), (40, 20, 12)])   # matrix kernel, library products
+@pytest.mark.parametrize("bias", [False, True])
+def test_outputs_can_be_changed_in_place(rows, ins, outs, bias):
+    x, w = torch.randn(2, rows // 2, ins, device=DEV, requires_grad=True), torch.randn(outs, ins, device=DEV, requires_grad=True)
+    b = torch.randn(outs, device=DEV) if bias else None
+    for call in (lambda: ops.linear(x, w, b), lambda: ops.projections(x, [w, w.detach()], [b, None])[0]):
+        y, z = call(), call()
+        y.mul_(2.0).relu_()
+        for got, want in zip(torch.autograd.grad(y.sum(), (x, w)), torch.autograd.grad((2.0 * z).relu().sum(), (x, w))):
+            assert torch.equal(got, want)
+
+
 def test_transforms_see_a_library_product():
     """Second derivatives, torch.func and forward-mode AD go through a projection as they do through torch.nn.functional.linear."""
     x, w = torch.randn(5, 24, device=DEV, requires_grad=True), torch.randn(16, 24, device=DEV, requires_grad=True)
