@@ -392,6 +392,17 @@ Tensor transposed(const Tensor& x, const Launch& l) {
     return t.narrow(1, 0, rows);
 }
 
+// A transform that has to see library calls: torch.func (grad, vmap, jvp), forward-mode AD, torch.jit tracing, a dispatch mode or a
+// tensor subclass (fake tensors among them); in a backward pass also batched gradients (torch.autograd.grad with is_grads_batched)
+bool transformed(const Tensor& t) {
+    return t.unsafeGetTensorImpl()->is_python_dispatch() || t._fw_grad(0).defined() ||
+           t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper}));
+}
+bool transforming() {
+    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           torch::jit::tracer::isTracing();
+}
+
 // Several projections of one input: y_i = x W_i^T + b_i.  Their input gradient is one sum, their forward products and (for small
 // problems) all their gradients are one launch each.
 struct Projections : Function<Projections> {
@@ -460,7 +471,9 @@ struct Projections : Function<Projections> {
         const int64_t n = (int64_t)g.size(), in = saved[0].size(-1);
         const Tensor x = saved[0].reshape({-1, in});
         const int64_t rows = x.size(0);
-        const bool again = at::GradMode::is_enabled();     // a graph of this pass is wanted: library products, which have one
+        // a graph of this pass is wanted, or a transform watches it: library products, out of place
+        bool again = at::GradMode::is_enabled() || transforming() || transformed(saved[0]);
+        for (int64_t i = 0; i < n; ++i) again = again || (g[i].defined() && transformed(g[i])) || transformed(saved[1 + i]);
         const auto has_bias = ctx->saved_data["has_bias"].toIntVector();
         const auto at = bias_at(has_bias);                 // tensor input 1 + at[i] of the node
         const bool need_dx = ctx->needs_input_grad(0);
@@ -515,8 +528,9 @@ struct Projections : Function<Projections> {
                 if (!dy[i].defined()) continue;
                 const Tensor& w = saved[1 + i];
                 if (need_dx) {
-                    if (dx.defined()) dx.addmm_(dy[i], w);  // summed inside the product
-                    else dx = at::mm(dy[i], w);
+                    if (!dx.defined()) dx = at::mm(dy[i], w);
+                    else if (again) dx = dx + at::mm(dy[i], w);
+                    else dx.addmm_(dy[i], w);              // summed inside the product
                 }
                 if (need_weight(i)) dw[i] = dyt.defined() ? at::mm(dyt, x) : at::mm(dy[i].t(), xt.defined() ? xt.t() : x);
                 if (need_bias(i)) db[i] = again ? dy[i].sum(0) : bias_gradient(dy[i]);
@@ -532,16 +546,6 @@ struct Projections : Function<Projections> {
         return grads;
     }
 };
-
-// A transform that has to see library calls: torch.func (grad, vmap, jvp), forward-mode AD, torch.jit tracing, a dispatch mode or a
-// tensor subclass (fake tensors among them)
-bool transformed(const Tensor& t) {
-    return t.unsafeGetTensorImpl()->is_python_dispatch() || t._fw_grad(0).defined();
-}
-bool transforming() {
-    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
-           torch::jit::tracer::isTracing();
-}
 
 // The plain library call where the native nodes do not apply: autocast chooses the dtype, CPU tensors have no kernel, and operands that
 // do not fit each other in shape, type or device are the library's to broadcast or refuse.

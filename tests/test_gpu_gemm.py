@@ -197,3 +197,23 @@ def test_transforms_see_a_library_product():
                  (torch.func.vmap(lambda q: ops.linear(q, w))(x), x @ w.t()),
                  (torch.func.grad(lambda q: f(q, w))(x), torch.func.grad(lambda q: ref(q, w))(x))):
         assert float((a - b).norm() / b.norm()) < 24 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(5, 24, (16,)), (5, 24, (16, 8)), (600, 1024, (1536, 1024))])
+def test_batched_gradients(rows, ins, outs):
+    """torch.autograd.grad with is_grads_batched, and a dispatch mode around the backward pass, see library products."""
+    from torch.utils.flop_counter import FlopCounterMode
+    x, ws, bs, dys = _case(rows, ins, outs, torch.float32, 4)
+    xg, wg, bg = x.to(DEV).requires_grad_(), [w.to(DEV).requires_grad_() for w in ws], bs[0].to(DEV).requires_grad_()
+    inputs = (xg, *wg, bg)
+    gs = [torch.stack([d, d.flip(0), 2 * d]).to(DEV) for d in dys]
+    ys = ops.projections(xg, wg, [bg] + [None] * (len(ws) - 1))
+    got = torch.autograd.grad(ys, inputs, gs, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        one = torch.autograd.grad(ys, inputs, [g[i] for g in gs], retain_graph=True)
+        for a, b in zip(got, one):                         # float32 sums of at most `rows` or sum(outs) terms in another order
+            assert a.shape == (3, *b.shape)
+            assert float((a[i] - b).norm()) <= 2 * max(rows, sum(outs)) ** 0.5 * 2.0 ** -24 * float(b.norm()) * 8
+    with FlopCounterMode(display=False) as counter:
+        torch.autograd.grad(ys, inputs, [g[0] for g in gs])
+    assert counter.get_total_flops() == sum(4 * rows * ins * o for o in outs)
