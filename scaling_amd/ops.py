@@ -12,6 +12,7 @@ import math
 from typing import Optional, Tuple
 
 import torch
+from torch.overrides import has_torch_function      # operands or modes that take over torch functions
 
 from . import _lib
 from ._lib import MiAttnArgs, check, dtype_code, ptr, stream_ptr
@@ -144,11 +145,16 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """x W^T + b (torch.nn.functional.linear) (+ residual), on the matrix kernel of this package where the product is too small to fill
     the chip and on the library product elsewhere.  `inference`: no gradients follow, so the forward product alone decides; the same value
     gives the same bits with and without gradients."""
+    if has_torch_function((x, weight, bias, residual)):
+        y = torch.nn.functional.linear(x, weight, bias)
+        return y if residual is None else y + residual
     return _lib.host().linear(x, weight, bias, residual, inference)
 
 
 def projections(x: torch.Tensor, weights, biases, inference: bool = False):
     """[linear(x, w, b) for up to three (w, b)] of one input, whose gradient is then one sum inside the products."""
+    if has_torch_function((x, *weights, *biases)):
+        return [torch.nn.functional.linear(x, w, b) for w, b in zip(weights, biases)]
     return _lib.host().projections(x, weights, biases, inference)
 
 

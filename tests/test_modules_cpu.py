@@ -126,6 +126,40 @@ def test_scaled_dot_product_attention_and_masked_softmax_mirror_the_reference_cl
     assert not any(k.startswith("scaled_dot_product_attention") for k in att.state_dict())   # no parameters: checkpoints unchanged
 
 
+class _Seen(torch.Tensor):
+    """An operand that takes over torch functions."""
+    functions = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.functions.append(func)
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+def test_projections_are_seen_by_operands_and_modes_that_take_over_torch_functions():
+    from torch.overrides import TorchFunctionMode
+
+    from scaling_amd import ops
+    functions = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            functions.append(func)
+            return func(*args, **(kwargs or {}))
+    x, w, b = torch.randn(3, 8), torch.randn(4, 8), torch.randn(4)
+    want = torch.nn.functional.linear(x, w, b)
+    for call, n in ((lambda v: ops.linear(x, v, b), 1), (lambda v: ops.linear(x, v, b, torch.zeros(3, 4)), 1),
+                    (lambda v: ops.projections(x, [v, w], [b, b])[0], 2)):
+        _Seen.functions.clear()
+        y = call(w.as_subclass(_Seen))
+        assert isinstance(y, _Seen) and torch.nn.functional.linear in _Seen.functions and torch.equal(y.as_subclass(torch.Tensor), want)
+        functions.clear()
+        with Mode():
+            y = call(w)
+        assert functions.count(torch.nn.functional.linear) == n and torch.equal(y, want)
+        assert torch.equal(call(w), want)
+
+
 # ---- module / checkpoint contract ---------------------------------------------------------------------------
 def test_layer_parameter_names_match_reference_checkpoint(golden_dir):
     legacy = torch.load(os.path.join(golden_dir, "legacy_layer_state.pt"), weights_only=True)
