@@ -150,25 +150,27 @@ class TransformerInferenceModule(torch.nn.Module):
         return None if logits is None else logits.unsqueeze(1)
 
     def _native_layers(self, batch: int, tokens: int) -> Optional[list]:
-        """(cache, arguments of ops.decode_layer) per layer for the next `tokens` cached steps, or None where a layer or this module
+        """(layer, cache, arguments of ops.decode_layer) per layer for the next `tokens` cached steps, or None where a layer or this module
         is not the package's own as it is."""
         layers = list(self._layers[1:-2])
         if type(self).forward is not TransformerInferenceModule.forward or "forward" in self.__dict__ or not layers or \
                 not all(type(layer) is TransformerLayer and _unhooked(layer) and layer._decodes_natively() for layer in layers):
             return None
-        native = [(layer.self_attention.cache.get(0), decode_arguments(layer, batch, tokens, 0)) for layer in layers]
-        return native if all(arguments is not None for _, arguments in native) else None
+        native = [(layer, layer.self_attention.cache.get(0), decode_arguments(layer, batch, tokens, 0)) for layer in layers]
+        return native if all(arguments is not None for _, _, arguments in native) else None
 
-    def _native_step(self, native: list, token_ids: torch.Tensor, position_ids: torch.Tensor) -> Optional[torch.Tensor]:
-        """Logits [b, 1, vocab] of one token per sequence; None, with nothing done, where the kernels refuse the first layer (the layers
-        of a model have one shape)."""
+    def _native_step(self, native: list, token_ids: torch.Tensor, position_ids: torch.Tensor, step: dict) -> Optional[torch.Tensor]:
+        """Logits [b, 1, vocab] of one token per sequence; None, with nothing done, where the kernels refuse the first layer.  A later
+        layer that they refuse (a weight of another layout) is called with the arguments `step` of a cached step."""
         h = self._layers[0](token_ids)
-        for i, (cache, arguments) in enumerate(native):
+        for i, (layer, cache, arguments) in enumerate(native):
             y = ops.decode_layer(h, position_ids, arguments)
-            if y is None:
-                assert i == 0, "the layers of a model have one shape"
+            if y is not None:
+                cache.length += 1
+            elif i == 0:
                 return None
-            cache.length += 1
+            else:
+                y = layer(TransformerLayerIO(activations=h, **step)).activations
             h = y
         logits = self._last_logits(h)
         return self._layers[-1].linear(self._layers[-2](TransformerLayerIO(activations=h, position_ids=None)).activations) if logits is None else logits
@@ -291,14 +293,15 @@ class TransformerInferenceModule(torch.nn.Module):
                 tokens.append(nxt)
                 if b == 1 and stop and int(nxt) in stop:
                     break
-                if k + 1 < max_tokens and native is not None:
-                    logits = self._native_step(native, nxt.unsqueeze(1), positions[k].view(-1))
+                if k + 1 == max_tokens:
+                    break
+                step = dict(position_ids=positions[k], cumulative_seq_lengths=one_each, inference_settings=settings)
+                if native is not None:
+                    logits = self._native_step(native, nxt.unsqueeze(1), positions[k].view(-1), step)
                     if logits is not None:
                         continue
                     native = None                        # a shape the kernels do not cover: nothing has been done yet
-                if k + 1 < max_tokens:
-                    logits = self.forward(nxt.unsqueeze(1), position_ids=positions[k], cumulative_seq_lengths=one_each,
-                                          inference_settings=settings, last_token_only=True)
+                logits = self.forward(nxt.unsqueeze(1), last_token_only=True, **step)
             completions = torch.stack(tokens, dim=1).tolist()
         else:
             cur = ids

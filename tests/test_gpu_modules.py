@@ -364,6 +364,23 @@ def test_scaled_dot_product_attention_reference_layout(case):
     check(f"sdpa.forward[{case}]", out, ref(torch.float32), ref(torch.bfloat16), kind="decode" if s_q == 1 else "o")
 
 
+@pytest.mark.parametrize("refused", [0, 1, 2])
+def test_generation_with_a_weight_the_decode_kernels_refuse(refused):
+    """A layer whose weight has another layout (here: stored transposed) takes its modules in a cached step; the layers before and
+    behind it do what they did.  The same values in another order of summation: one rounding where a layer stores a result."""
+    print(f"case generate, layer {refused} transposed", flush=True)
+    model = TransformerInferenceModule(_arch(attention_num_kv_heads=2, num_layers=3, mlp_factor=2.75), device=DEV, seed=4)
+    with torch.no_grad():
+        model._layers[-1].linear.weight.mul_(20.0)
+    prompts = torch.randint(1, 96, (2, 9), generator=torch.Generator().manual_seed(3))
+    want_tokens, want = model.generate(5, prompts)
+    mlp = model._layers[1 + refused].mlp
+    mlp.dense_out.weight = torch.nn.Parameter(mlp.dense_out.weight.detach().t().contiguous().t())
+    tokens, logits = model.generate(5, prompts)
+    assert tokens == want_tokens
+    assert float((logits - want).float().norm()) <= 8 * 2.0 ** -8 * float(want.float().norm())
+
+
 @pytest.mark.parametrize("max_tokens", [1, 2, 3, 9])
 def test_graph_captured_decode_equals_eager_decode(max_tokens):
     """Every replay of the captured per-token step must reproduce the eager step (tokens identical)."""
