@@ -18,6 +18,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
+#include <algorithm>
 #include <optional>
 #include <tuple>
 #include <vector>
@@ -422,13 +423,18 @@ struct Projections : Function<Projections> {
         const auto at = bias_at(has_bias);
         const Tensor x2 = x.reshape({-1, in});
         const int64_t rows = x2.size(0);
-        variable_list saved{x}, out;                      // x itself: what is differentiated again reaches it
+        variable_list saved, out;
         bool small = aligned(x2) && !(inference && long_chain(x, rows, in));
         for (int64_t i = 0; i < n; ++i) {
             const Tensor& w = params[i];
             small = small && aligned(w) && small_product(x, rows, w.size(0), in);
-            saved.push_back(w);
         }
+        // What the gradients read and no more, so that the rest may be changed or freed before the backward pass: x (itself: what is
+        // differentiated again reaches it) for the weights, the weights for x.  The same for a recomputation inside a backward pass.
+        bool any_weight = false;
+        for (int64_t i = 0; i < n; ++i) any_weight = any_weight || params[i].requires_grad();
+        saved.push_back(any_weight ? x : Tensor());
+        for (int64_t i = 0; i < n; ++i) saved.push_back(x.requires_grad() ? params[i] : Tensor());
         std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
         if (small) {
             Launch l(x);
@@ -468,54 +474,61 @@ struct Projections : Function<Projections> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const int64_t n = (int64_t)g.size(), in = saved[0].size(-1);
-        const Tensor x = saved[0].reshape({-1, in});
-        const int64_t rows = x.size(0);
+        const auto x_shape = ctx->saved_data["x_shape"].toIntVector();
+        const int64_t n = (int64_t)g.size(), in = x_shape.back();
+        int64_t rows = 1;
+        for (size_t i = 0; i + 1 < x_shape.size(); ++i) rows *= x_shape[i];
+        const Tensor x = saved[0].defined() ? saved[0].reshape({rows, in}) : Tensor();     // undefined: no weight takes a gradient
         // a graph of this pass is wanted, or a transform watches it: library products, out of place
-        bool again = at::GradMode::is_enabled() || transforming() || transformed(saved[0]);
-        for (int64_t i = 0; i < n; ++i) again = again || (g[i].defined() && transformed(g[i])) || transformed(saved[1 + i]);
+        bool again = at::GradMode::is_enabled() || transforming();
+        for (const Tensor& t : saved) again = again || (t.defined() && transformed(t));
+        for (const Tensor& t : g) again = again || (t.defined() && transformed(t));
         const auto has_bias = ctx->saved_data["has_bias"].toIntVector();
         const auto at = bias_at(has_bias);                 // tensor input 1 + at[i] of the node
         const bool need_dx = ctx->needs_input_grad(0);
         const auto need_weight = [&](int64_t i) { return ctx->needs_input_grad(1 + i); };
         const auto need_bias = [&](int64_t i) { return at[i] >= 0 && ctx->needs_input_grad(1 + at[i]); };
         std::vector<Tensor> dy(n), dw(n), db(n);
-        bool small = !again && rows > 0 && aligned(x);
+        bool small = !again && rows > 0 && (!x.defined() || aligned(x));
         for (int64_t i = 0; i < n; ++i) {
             if (!g[i].defined()) continue;                 // this projection does not reach the loss
-            dy[i] = g[i].reshape({rows, saved[1 + i].size(0)});
+            dy[i] = g[i].reshape({rows, g[i].size(-1)});
             if (!again && !aligned(dy[i])) dy[i] = dy[i].contiguous();
-            small = small && aligned(dy[i]) && small_product(x, rows, dy[i].size(1), in);
+            small = small && aligned(dy[i]) && small_product(dy[i], rows, dy[i].size(1), in);
             // the forward product may have been the library's, and saved-tensor hooks may bring the weight back in another layout
             if (need_dx) small = small && aligned(saved[1 + i]);
         }
-        Tensor dx;
+        Tensor dx, any;                                    // any: a gradient, for device and type
+        for (int64_t i = 0; i < n && !any.defined(); ++i) any = dy[i];
+        if (!any.defined()) return variable_list(n + at.size() - std::count(at.begin(), at.end(), -1) + 4);
+        Launch l(any);
         if (small) {
-            Launch l(x);
             mi_gemm_problem pr[MI_GEMM_MAX_PROBLEMS];
             int count = 0;
             if (need_dx) {
-                dx = at::empty({rows, in}, x.options());
+                dx = at::empty({rows, in}, any.options());
                 mi_gemm_problem p = problem(dx, false, true);
                 for (int64_t i = 0; i < n; ++i)
                     if (dy[i].defined()) segment(p, dy[i], saved[1 + i], dy[i].size(1));
-                if (p.n_segments > 0) pr[count++] = p; else dx = Tensor();
+                pr[count++] = p;
             }
             for (int64_t i = 0; i < n; ++i) {
                 if (!dy[i].defined()) continue;
-                if (!need_weight(i) && !need_bias(i)) continue;
-                dw[i] = at::empty({dy[i].size(1), in}, x.options());
+                if (!need_weight(i)) {
+                    if (need_bias(i)) db[i] = bias_gradient(dy[i]);
+                    continue;
+                }
+                dw[i] = at::empty({dy[i].size(1), in}, any.options());
                 mi_gemm_problem p = problem(dw[i], true, true);
                 segment(p, dy[i], x, rows);
                 if (need_bias(i)) {
-                    db[i] = at::empty({dy[i].size(1)}, x.options());
+                    db[i] = at::empty({dy[i].size(1)}, any.options());
                     p.p_sum = ptr(db[i]);
                 }
                 pr[count++] = p;
             }
-            if (count > 0) check(mi_gemm(pr, count, code_of(x), l.stream), "mi_gemm");
+            if (count > 0) check(mi_gemm(pr, count, code_of(any), l.stream), "mi_gemm");
         } else {
-            Launch l(x);
             int64_t out = 0;
             for (int64_t i = 0; i < n; ++i)
                 if (dy[i].defined() && need_weight(i)) out += dy[i].size(1);
@@ -536,8 +549,8 @@ struct Projections : Function<Projections> {
                 if (need_bias(i)) db[i] = again ? dy[i].sum(0) : bias_gradient(dy[i]);
             }
         }
-        variable_list grads{dx.defined() ? dx.view(ctx->saved_data["x_shape"].toIntVector()) : Tensor()};
-        for (int64_t i = 0; i < n; ++i) grads.push_back(need_weight(i) ? dw[i] : Tensor());
+        variable_list grads{dx.defined() ? dx.view(x_shape) : Tensor()};
+        for (int64_t i = 0; i < n; ++i) grads.push_back(dw[i]);
         for (int64_t i = 0; i < n; ++i)
             if (at[i] >= 0) grads.push_back(db[i]);
         grads.push_back(g[0]);                             // residual (ignored without one)

@@ -104,6 +104,42 @@ def test_projection_that_does_not_reach_the_loss():
     assert ops.linear(torch.empty(0, 64, device=DEV), wg[0]).shape == (0, 32)
 
 
+@pytest.mark.parametrize("rows,ins,outs", [(24, 64, (32, 16)), (2048, 512, (2048, 256))])   # matrix kernel, library products
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_what_no_gradient_reads_may_change_before_the_backward_pass(rows, ins, outs, dtype):
+    """As with torch.nn.functional.linear: the input where no weight is trained, the weights where the input takes no gradient."""
+    print(f"case gemm frozen rows={rows} dtype={dtype}", flush=True)
+    x, ws, bs, dys = _case(rows, ins, outs, dtype, 17)
+    xd, wd, dyd = x.double(), [w.double() for w in ws], [d.double() for d in dys]
+    for n in (1, 2):
+        def forward(xg, wg, bg):
+            return [ops.linear(xg, wg[0], bg)] if n == 1 else ops.projections(xg, wg[:n], [bg, None])
+
+        def backward(ys):
+            torch.autograd.backward(ys, [d.to(DEV) for d in dys[:n]])
+        # frozen weights, a trained bias: the input is a temporary that is overwritten
+        leaf, wg, bg = x.to(DEV).requires_grad_(), [w.to(DEV) for w in ws], bs[0].to(DEV).requires_grad_()
+        xg = leaf * 1
+        ys = forward(xg, wg, bg)
+        xg.detach().zero_()
+        backward(ys)
+        # a library product per projection is rounded before the next is added
+        slack = HALF_ULP[dtype] * (dyd[0] @ wd[0]).abs() if n == 2 else 0.0
+        ref, mag = sum(d @ w for d, w in zip(dyd[:n], wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd[:n], wd))
+        err = (leaf.grad.double().cpu() - ref).abs()
+        assert bool((err <= (HALF_ULP[dtype] * ref.abs() + slack + (sum(outs) + 1) * 2.0 ** -24 * mag + 2.0 ** -133) * 1.001).all()), float(err.max())
+        _close("db", bg.grad, dyd[0].sum(0), dyd[0].abs().sum(0), rows, dtype)
+        # an input without gradients: the weights are stepped between forward and backward
+        wg = [w.to(DEV).requires_grad_() for w in ws]
+        ys = forward(x.to(DEV), wg, None)
+        with torch.no_grad():
+            for w in wg:
+                w.add_(1.0)
+        backward(ys)
+        for i in range(n):
+            _close(f"dw{i}", wg[i].grad, dyd[i].t() @ xd, dyd[i].abs().t() @ xd.abs(), rows, dtype)
+
+
 def test_operands_that_do_not_fit_are_the_librarys():
     """What torch.nn.functional.linear refuses is refused, what it broadcasts is broadcast: no kernel sees such an operand."""
     x, w, b = torch.randn(4, 64, device=DEV), torch.randn(32, 64, device=DEV), torch.randn(32, device=DEV)
