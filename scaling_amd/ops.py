@@ -12,7 +12,8 @@ import math
 from typing import Optional, Tuple
 
 import torch
-from torch.overrides import has_torch_function      # operands or modes that take over torch functions
+from torch.overrides import _get_current_function_mode_stack, has_torch_function
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from ._lib import MiAttnArgs, check, dtype_code, ptr, stream_ptr
@@ -140,12 +141,22 @@ def swiglu(a: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
 # ------------------------------------------------------------------------------------------------
 # linear projections
 # ------------------------------------------------------------------------------------------------
+def _taken_over(operands: tuple) -> bool:
+    """Whether an operand or a mode takes over torch functions, and so has to see them.  A default device (torch.set_default_device,
+    `with torch.device(...)`) is such a mode too, which does nothing to a call on tensors that are there."""
+    if not has_torch_function(operands):
+        return False
+    return any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack()) or \
+        any(t is not None and type(t) is not torch.Tensor and type(t).__torch_function__ is not torch._C._disabled_torch_function_impl
+            for t in operands)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            residual: Optional[torch.Tensor] = None, inference: bool = False) -> torch.Tensor:
     """x W^T + b (torch.nn.functional.linear) (+ residual), on the matrix kernel of this package where the product is too small to fill
     the chip and on the library product elsewhere.  `inference`: no gradients follow, so the forward product alone decides; the same value
     gives the same bits with and without gradients."""
-    if has_torch_function((x, weight, bias, residual)):
+    if _taken_over((x, weight, bias, residual)):
         y = torch.nn.functional.linear(x, weight, bias)
         return y if residual is None else y + residual
     return _lib.host().linear(x, weight, bias, residual, inference)
@@ -153,7 +164,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
 
 def projections(x: torch.Tensor, weights, biases, inference: bool = False):
     """[linear(x, w, b) for up to three (w, b)] of one input, whose gradient is then one sum inside the products."""
-    if has_torch_function((x, *weights, *biases)):
+    if _taken_over((x, *weights, *biases)):
         return [torch.nn.functional.linear(x, w, b) for w, b in zip(weights, biases)]
     return _lib.host().projections(x, weights, biases, inference)
 

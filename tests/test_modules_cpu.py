@@ -161,6 +161,22 @@ def test_projections_are_seen_by_operands_and_modes_that_take_over_torch_functio
 
 
 # ---- module / checkpoint contract ---------------------------------------------------------------------------
+def test_a_default_device_changes_no_projection(monkeypatch):
+    from scaling_amd import _lib, ops
+
+    class Host:
+        @staticmethod
+        def linear(*_):
+            return "native"
+        projections = linear
+    monkeypatch.setattr(_lib, "host", lambda: Host)
+    x, w = torch.randn(3, 8), torch.nn.Parameter(torch.randn(4, 8))
+    for call in (lambda v: ops.linear(x, v), lambda v: ops.projections(x, [v, w], [None, None])):
+        assert call(w) == "native"
+        with torch.device("cpu"):
+            assert call(w) == "native" and call(w.detach().as_subclass(_Seen)) != "native"
+
+
 def test_layer_parameter_names_match_reference_checkpoint(golden_dir):
     legacy = torch.load(os.path.join(golden_dir, "legacy_layer_state.pt"), weights_only=True)
     layer = TransformerLayer(_arch(attention_qkv_in_one=True, attention_num_kv_heads=None), layer_index=0, device=CPU)
