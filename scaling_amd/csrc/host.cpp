@@ -981,15 +981,16 @@ void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v
 
 // ---- a decode step's layer ---------------------------------------------------------------------------------------------
 bool rows_weight(const Tensor& w, const Tensor& x, int64_t k) {
-    return w.dim() == 2 && w.size(0) > 0 && w.size(1) == k && w.scalar_type() == x.scalar_type() && w.device() == x.device() && aligned(w);
+    return !transformed(w) && w.dim() == 2 && w.size(0) > 0 && w.size(1) == k && w.scalar_type() == x.scalar_type() && w.device() == x.device() &&
+           aligned(w);
 }
 bool rows_norm(const Tensor& w, const Tensor& x, int64_t k) {
-    return w.dim() == 1 && w.size(0) == k && w.stride(0) == 1 && w.scalar_type() == x.scalar_type() && w.device() == x.device() &&
+    return !transformed(w) && w.dim() == 1 && w.size(0) == k && w.stride(0) == 1 && w.scalar_type() == x.scalar_type() && w.device() == x.device() &&
            (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0;
 }
-bool rows_input(const Tensor& x) {                         // [rows, k]
-    return x.is_cuda() && x.dim() == 2 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(0) >= 1 &&
-           x.size(0) <= MI_ROWS_MAX && x.size(1) > 0 && x.size(1) % 32 == 0 && aligned(x);
+bool rows_input(const Tensor& x) {                         // [rows, k]; a transform sees the modules' operations instead
+    return !transforming() && !transformed(x) && x.is_cuda() && x.dim() == 2 &&
+           (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(0) >= 1 && x.size(0) <= MI_ROWS_MAX && x.size(1) > 0 && x.size(1) % 32 == 0 && aligned(x);
 }
 
 mi_rows_args rows_args(const Tensor& x, const Tensor& norm, double eps, const Launch& l) {

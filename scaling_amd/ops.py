@@ -533,6 +533,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
 
 def norm_linear_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """rms_norm(x) @ weight.T of up to 16 rows [rows, k] (inference); None where the kernel does not apply."""
+    if _taken_over((x, norm_weight, weight)):
+        return None
     return _lib.host().norm_linear_rows(x, norm_weight, eps, weight)
 
 
@@ -548,4 +550,7 @@ def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w
 def decode_layer(x: torch.Tensor, position_ids: torch.Tensor, arguments: tuple) -> Optional[torch.Tensor]:
     """A cached decode step of a whole layer, x [batch, 1, hidden] of up to 16 sequences, position_ids int64 [batch]: raises the context
     lengths by one, appends to the caches and returns the layer's output.  None, with nothing done, where the kernels do not apply."""
+    norm1, _, qkv_weights, dense, norm2, _, w_in, w_gate, w_out = arguments[:9]
+    if _taken_over((x, position_ids, norm1, *qkv_weights, dense, norm2, w_in, w_gate, w_out)):
+        return None
     return _lib.host().decode_layer(x, position_ids, *arguments)

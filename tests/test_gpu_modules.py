@@ -8,7 +8,7 @@ import oracle
 from scaling_amd import config as C
 from scaling_amd import data as D
 from scaling_amd.inference import TransformerInferenceModule
-from scaling_amd.layer import TransformerLayer, TransformerLayerIO
+from scaling_amd.layer import InferenceSettings, TransformerLayer, TransformerLayerIO
 from tests.parity import check, metrics
 
 pytestmark = pytest.mark.gpu
@@ -362,6 +362,27 @@ def test_scaled_dot_product_attention_reference_layout(case):
                                            softmax_in_fp32=True, softmax_scale=1.5, mask=mask)
 
     check(f"sdpa.forward[{case}]", out, ref(torch.float32), ref(torch.bfloat16), kind="decode" if s_q == 1 else "o")
+
+
+def test_cached_step_is_seen_by_a_dispatch_mode():
+    """A mode around a cached step (here: a flop counter) sees every product of the layers and the head; the same values in another order of
+    summation: one rounding where a layer stores a result."""
+    from torch.utils.flop_counter import FlopCounterMode
+    print("case cached step under a dispatch mode", flush=True)
+    model = TransformerInferenceModule(_arch(attention_num_kv_heads=2, num_layers=2, mlp_factor=2.75), device=DEV, seed=4)
+    prompts = torch.randint(1, 96, (2, 9), generator=torch.Generator().manual_seed(3))
+    settings = dict(position_ids=torch.full((2, 1), 9, device=DEV), cumulative_seq_lengths=torch.arange(3, dtype=torch.int32, device=DEV),
+                    inference_settings=InferenceSettings(use_cache=True, reset_cache=False), last_token_only=True)
+    token = torch.ones(2, 1, dtype=torch.int64, device=DEV)
+    fill = InferenceSettings(use_cache=True, reset_cache=True)
+    model(prompts, inference_settings=fill)
+    want = model(token, **settings)
+    model(prompts, inference_settings=fill)
+    with FlopCounterMode(display=False) as counter:
+        logits = model(token, **settings)
+    weights = sum(p.numel() for n, p in model.named_parameters() if p.dim() == 2 and "embedding" not in n)
+    assert counter.get_total_flops() == 2 * 2 * weights
+    assert float((logits - want).float().norm()) <= 8 * 2.0 ** -8 * float(want.float().norm())
 
 
 @pytest.mark.parametrize("refused", [0, 1, 2])

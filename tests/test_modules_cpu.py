@@ -177,6 +177,36 @@ def test_a_default_device_changes_no_projection(monkeypatch):
             assert call(w) == "native" and call(w.detach().as_subclass(_Seen)) != "native"
 
 
+def test_row_products_leave_operands_and_modes_that_take_over_torch_functions_alone(monkeypatch):
+    from torch.overrides import TorchFunctionMode
+
+    from scaling_amd import _lib, ops
+
+    class Host:
+        @staticmethod
+        def norm_linear_rows(*_):
+            return "native"
+        decode_layer = norm_linear_rows
+    monkeypatch.setattr(_lib, "host", lambda: Host)
+    x, norm, w, ids = torch.randn(3, 8), torch.ones(8), torch.randn(4, 8), torch.zeros(3, dtype=torch.int64)
+
+    def head(i=None):
+        x_, norm_, w_ = (t.as_subclass(_Seen) if j == i else t for j, t in enumerate((x, norm, w)))
+        return ops.norm_linear_rows(x_, norm_, 1e-5, w_)
+
+    def step(i=None):
+        t = [norm, w, w, w, w, norm, w, w, w]
+        if i is not None:
+            t[i] = t[i].as_subclass(_Seen)
+        return ops.decode_layer(x, ids, (t[0], 1e-5, t[1:4], t[4], t[5], 1e-5, *t[6:], 8, *[None] * 8))
+    for call, n in ((head, 3), (step, 9)):
+        assert call() == "native" and all(call(i) is None for i in range(n))
+        with TorchFunctionMode():
+            assert call() is None
+        with torch.device("cpu"):
+            assert call() == "native"
+
+
 def test_layer_parameter_names_match_reference_checkpoint(golden_dir):
     legacy = torch.load(os.path.join(golden_dir, "legacy_layer_state.pt"), weights_only=True)
     layer = TransformerLayer(_arch(attention_qkv_in_one=True, attention_num_kv_heads=None), layer_index=0, device=CPU)
