@@ -539,8 +539,11 @@ def norm_linear_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, wei
 
 
 def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, tables,
-                           softmax_scale, workspace, dtype) -> tuple:
-    """What `decode_layer` takes beside the token: the layer's weights, its caches and rotary tables."""
+                           softmax_scale, workspace, dtype) -> Optional[tuple]:
+    """What `decode_layer` takes beside the token: the layer's weights, its caches and rotary tables.  None for weights that have to see
+    the functions they are used in."""
+    if _taken_over((norm1, *qkv_weights, dense, norm2, w_in, w_gate, w_out)):
+        return None
     cos, sin = tables
     interleaved = _fused_rotary_kind(cos, sin, head_dim, dtype)
     return (norm1, eps1, list(qkv_weights), dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, cos, sin, interleaved,
@@ -550,7 +553,6 @@ def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w
 def decode_layer(x: torch.Tensor, position_ids: torch.Tensor, arguments: tuple) -> Optional[torch.Tensor]:
     """A cached decode step of a whole layer, x [batch, 1, hidden] of up to 16 sequences, position_ids int64 [batch]: raises the context
     lengths by one, appends to the caches and returns the layer's output.  None, with nothing done, where the kernels do not apply."""
-    norm1, _, qkv_weights, dense, norm2, _, w_in, w_gate, w_out = arguments[:9]
-    if _taken_over((x, position_ids, norm1, *qkv_weights, dense, norm2, w_in, w_gate, w_out)):
+    if _taken_over((x, position_ids)):
         return None
     return _lib.host().decode_layer(x, position_ids, *arguments)

@@ -198,7 +198,8 @@ def test_row_products_leave_operands_and_modes_that_take_over_torch_functions_al
         t = [norm, w, w, w, w, norm, w, w, w]
         if i is not None:
             t[i] = t[i].as_subclass(_Seen)
-        return ops.decode_layer(x, ids, (t[0], 1e-5, t[1:4], t[4], t[5], 1e-5, *t[6:], 8, *[None] * 8))
+        arguments = ops.decode_layer_arguments(t[0], 1e-5, t[1:4], t[4], t[5], 1e-5, *t[6:], 8, *[None] * 3, (w, w), 1.0, None, torch.float32)
+        return arguments and ops.decode_layer(x, ids, arguments)
     for call, n in ((head, 3), (step, 9)):
         assert call() == "native" and all(call(i) is None for i in range(n))
         with TorchFunctionMode():
