@@ -309,9 +309,9 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 template <int D>
 __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeParams p) {
     constexpr int kDepth = 8;
-    const int64_t bh = (int64_t)blockIdx.x * (128 / D > 0 ? 128 / D : 1) + (2 * threadIdx.x) / D;
+    const int64_t bh = (int64_t)blockIdx.x * (128 / D) + (2 * threadIdx.x) / D;
     const int d = (2 * threadIdx.x) % D;
-    if (2 * threadIdx.x >= (128 / D > 0 ? 128 / D : 1) * D || bh >= (int64_t)p.batch * p.nq) return;
+    if (2 * threadIdx.x >= (128 / D) * D || bh >= (int64_t)p.batch * p.nq) return;
     const float* ml = p.ws_ml + bh * p.n_splits * 2;
     const float* wo = p.ws_o + bh * p.n_splits * D + d;
     float M = -INFINITY, L = 0.f, O0 = 0.f, O1 = 0.f;
@@ -375,7 +375,7 @@ template <int D, int NWV> int launch_split(const DecodeParams& p, int rot, hipSt
 template <int D> int launch_decode(const DecodeParams& p, int rot, hipStream_t st) {
     const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8>(p, rot, st) : launch_split<D, 4>(p, rot, st);
     if (rc != MI_OK || p.n_splits == 1) return rc;
-    constexpr int kRows = 128 / D > 0 ? 128 / D : 1;
+    constexpr int kRows = 128 / D;
     const int64_t n = (int64_t)p.batch * p.nq;
     decode_merge_kernel<D><<<dim3((unsigned)((n + kRows - 1) / kRows)), dim3(64), 0, st>>>(p);
     return mi_check_launch("decode_merge");

@@ -229,8 +229,8 @@ __device__ __forceinline__ void block_range(int wmin, int wmax, int wave, int la
     bmax = __builtin_amdgcn_readfirstlane(bmax);
 }
 
-// LDS bytes and stages of a kernel that streams two tensors in steps of ROWS rows: two stages where they fit twice into a
-// compute unit's 160 KB together with a second workgroup (FOR_TWO) or alone, else one
+// LDS bytes and stages of a kernel that streams two tensors in steps of ROWS rows: two stages where both take at most 128 KB, however
+// many workgroups that leaves a compute unit, else one
 template <int D, int ROWS> constexpr int stage_bytes() { return 2 * ROWS * 4 * D; }
 template <int D, int ROWS> constexpr int n_stages() { return 2 * stage_bytes<D, ROWS>() <= 128 * 1024 ? 2 : 1; }
 
