@@ -73,6 +73,39 @@ def test_outputs_are_the_same_with_and_without_gradients(rows, ins, outs, dtype)
             assert all(torch.equal(a, b) for a, b in zip(want, call(inference)))
 
 
+@pytest.mark.parametrize("rows,ins,outs", [(16, 2048, (512,)), (17, 2040, (64, 128)), (17, 2048, (64, 128)), (32, 2816, (1024,)), (64, 2048, (2048, 512, 512)),
+                                           (33, 3072, (256,))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_captured_products(rows, ins, outs, dtype):
+    """Products of inference in a captured graph, where a contraction from 2048 on takes the library: every replay on new inputs against
+    float64, with eager work between the replays."""
+    x, ws, bs, dys = _case(rows, ins, outs, dtype, ins)
+    wg, bg = [w.to(DEV) for w in ws], [None if b is None else b.to(DEV) for b in bs]
+    inputs = [x, x.flip(0), 2 * x.roll(1, 1)]
+    xs, res = inputs[0].to(DEV), dys[0].to(DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(side):
+        ops.projections(xs, wg, bg, True), ops.linear(xs, wg[0], None, res, True)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        ys = [*ops.projections(xs, wg, bg, True), ops.linear(xs, wg[0], None, res, True)]
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for new in inputs:
+        xs.copy_(new.to(DEV))
+        graph.replay()
+        (xs.float() @ wg[0].float().t()).sum().item()
+        for i, y in enumerate(ys):
+            last = i == len(ws)
+            w, b = (ws[0], None) if last else (ws[i], bs[i])
+            want = new.double() @ w.double().t() + (0 if b is None else b.double())
+            add = dys[0].double() if last else torch.zeros(())
+            # the product is rounded, and with the residual the sum again
+            err = (y.double().cpu() - want - add).norm()
+            assert err <= 1.01 * eps * (want.norm() + (want + add).norm() * last) + 1e-6
+
+
 def test_reentrant_checkpoint_over_a_long_contraction():
     """The MLP of a layer whose second product contracts over 4096 features, 24 rows: loss and gradients of a plain step."""
     from torch.utils.checkpoint import checkpoint
