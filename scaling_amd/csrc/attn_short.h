@@ -135,24 +135,44 @@ template <int D> __device__ __forceinline__ void short_write(elem_t* row, const 
         *reinterpret_cast<uint2*>(row + 32 * dt) = make_uint2(pack_elem2(x[dt][0] * scale, x[dt][1] * scale), pack_elem2(x[dt][2] * scale, x[dt][3] * scale));
 }
 
-// Host side: whether a call goes to these kernels: up to 2048 workgroups of 32 rows, which is about twice what the chip holds, and 1024
-// in the forward pass above 64 features, where a compute unit holds two.  Tiled / short, us, forward and backward:
-//   12 heads of 64, 3001 tokens in documents of 17 - 400 (1128 workgroups)     20.9 / 12.3   48.4 / 37.1
-//   8 heads of 64, 2048 tokens (512)                                           46.1 / 15.9   90.0 / 44.9
-//   16 heads of 64, 4084 tokens in documents of 16 - 600 (2048)                25.3 / 20.7   62.4 / 59.9
-//   16 heads of 64, 8192 tokens in documents of 1024 (4096)                    42.0 / 50.9    115 / 139
-//   32 / 8 heads of 128, 512 tokens (512)                                      21.8 / 10.7   81.9 / 48.1
-//   32 / 8 heads of 128, 1024 tokens (1024)                                    34.7 / 23.9    145 / 91.8
-//   32 / 8 heads of 128, 2048 tokens (2048)                                    63.6 / 71.5    271 / 206
-//   32 / 8 heads of 128, 4096 tokens in documents of 512 (4096)                45.0 / 73.6    130 / 199
+// Host side: whether a call goes to these kernels, by its workgroups of 32 rows (rows / 32 x query heads).  A compute unit holds eight of them up
+// to 64 features; above, two in the forward pass and one of dK / dV.  The tiled kernels wait for the longest chain of a workgroup, which
+// is what these kernels shorten; they gain where that chain runs alone: few workgroups, and causal documents, whose last rows have
+// twice the average work.  They lose where the tiled kernels have work for every compute unit all along, and the backward pass keeps that
+// up longer with grouped heads (`group` query heads per dK / dV workgroup lengthen the tiled chain).  Ragged documents
+// share tiled workgroups, which then walk the masked tiles of both; documents that are whole blocks of 256 rows cost the tiled
+// kernels nothing, unless there are so few that the chain of one dominates.  Short / tiled, at 512 | 1024 | 1536 | 2048 workgroups:
+//   forward, 64 features:   one causal document .33 - .49 | .37 - .51 | .53 - .64 | .60 - .70     ragged, mean 100 - 800 | | .59 - .80 | .61 - .86
+//                           not causal .41 - .58 | .62 - .73 | .90 - .96 | 1.06 - 1.18            documents of 512 .47 | .70 - .78 | | .91 - 1.06
+//   forward, 128 features:  causal .38 - .53 | .51 - .84 | .72 - 1.06 | .91 - 1.2      not causal .50 - .78 | .87 - 1.10 | 1.3 | 1.5
+//   backward, 64 features:  one causal document .48 - .59 | .56 - .62 | .66 - .76 | .66 - .92     ragged | .57 - .83 | .64 - .88 | .67 - .92
+//                           not causal .57 - .70 | .67 - 1.0 | .79 - .95 | .86 - 1.22             documents of 512 | .96 - 1.03 | | 1.06 - 1.22
+//   backward, 128, no groups:   one causal document .47 - .70 | .75 - .93 | 1.07 - 1.18 | 1.3     ragged, mean 100 - 300 .72 - .96 | 1.1 - 1.2 | 1.3 | 1.5
+//                               not causal .73 - .82 | 1.2 - 1.34 | 1.4 | 1.6                     documents of 512 .87 - .93 | 1.2 - 1.37 | | 1.5 - 1.8
+//   backward, 128, groups of 4: one causal document .59 | .65 | .70 | .79                         ragged .53 | .65 | .70 - .95 | .84 - 1.04
+//                               not causal .63 | .73 | 1.16 | 1.22                                documents of 512 | | | 1.19
+// (4 / 4, 12 / 12, 16 / 4 and 32 / 8 heads, the rows that make up the count; 1 and 2 heads with documents of up to 65536 tokens alike: the
+// length of a context alone does not decide.)  us at some of these, tiled / short: 32 / 8 heads of 128, 1024 tokens 34.7 / 23.9 forward, 145 /
+// 91.8 backward; 16 heads of 128, 8 documents of 512: 29.3 / 41.3 and 80 / 142; 12 heads of 64, 3001 tokens in documents of
+// 17 - 400: 20.9 / 12.3 and 48.4 / 37.1; 1 head of 64, 65536 tokens: 1280 / 762 and 2575 / 2280.  Of 110 calls
+// drawn between 350 and 2300 workgroups none that these kernels take was slower than tiled.
 // Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
 // backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
 static inline bool mi_attn_is_short(const mi_attn_args* a, bool backward) {
     if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return false;
     if (a->flags & MI_ATTN_SHORT) return true;
-    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k;
-    const int per_unit = backward || a->head_dim <= 64 ? 8 : 4;
-    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads <= (int64_t)per_unit * mi_compute_units();
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k, docs = a->n_docs > 1 ? a->n_docs : 1;
+    const bool narrow = a->head_dim <= 64, causal = a->causal != 0;
+    const bool whole = a->total_q == a->total_k && rows % (256 * docs) == 0;                          // may be whole blocks, all of them
+    const bool chains = causal && (whole ? rows >= 1024 * docs * docs : rows >= 512 * docs);        // the chain of a document dominates
+    const int group = a->n_q_heads / a->n_kv_heads / mi_dkdv_head_split(a->n_q_heads, a->n_kv_heads);
+    int64_t per_unit_64;                                   // 64 x workgroups per compute unit
+    if (!backward) per_unit_64 = narrow ? (causal ? 512 : 384) : (causal ? 256 : 192);
+    else if (narrow) per_unit_64 = (!causal ? 320 : whole && !chains ? 256 : 512) + 96 * (group - 1);
+    else per_unit_64 = (chains ? 256 : 128) + (causal ? 96 : 64) * (group - 1);
+    const int most = backward && !narrow && !causal ? 256 : 512;
+    if (per_unit_64 > most) per_unit_64 = most;
+    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads * 64 <= per_unit_64 * mi_compute_units();
 }
 
 // ---- forward: 32 queries of one head --------------------------------------------------------------------------------

@@ -86,3 +86,31 @@ def test_attention_routes_agree_with_rotary(d, interleaved):
     assert torch.equal(out[0][2], out[1][2])               # the same rotation, bit for bit
     for name, x, y in zip(("o", "lse", "q_rot", "dq", "dk", "dv"), *out):
         assert float((x.float() - y.float()).norm()) <= 2.0 ** -6 * float(y.float().norm()), name      # as above, bfloat16
+
+
+# each side of the lines that choose between the two, forward and backward: (heads, KV heads, features, tokens, documents, causal) and the
+# routes of a call that pins none
+@pytest.mark.parametrize("nq,nkv,d,total,docs,causal,fwd,bwd", [
+    (4, 4, 64, 8192, 1, True, SHORT, SHORT), (4, 4, 64, 8192, 1, False, SHORT, SHORT), (8, 8, 64, 8192, 1, False, TILED, TILED),
+    (16, 16, 64, 4096, 8, True, SHORT, TILED),             # documents of whole blocks
+    (16, 16, 64, 4095, 8, True, SHORT, SHORT), (32, 8, 64, 2048, 1, False, TILED, SHORT),
+    (8, 8, 128, 4096, 1, True, SHORT, SHORT), (8, 8, 128, 4096, 8, True, SHORT, TILED), (8, 8, 128, 4090, 20, True, SHORT, TILED),
+    (8, 8, 128, 2048, 4, True, SHORT, SHORT), (4, 4, 128, 8192, 1, False, TILED, TILED), (4, 4, 128, 4096, 1, False, SHORT, SHORT),
+    (4, 4, 128, 16384, 1, True, TILED, TILED), (32, 8, 128, 2048, 1, True, TILED, SHORT), (32, 8, 128, 1056, 1, False, TILED, TILED),
+])
+def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
+    print(f"case route of a call nq={nq} nkv={nkv} d={d} total={total} docs={docs} causal={causal}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are per compute unit; these sizes are for 256")
+    g = torch.Generator(device=DEV).manual_seed(total)
+    q, do = (torch.randn(total, nq, d, generator=g, device=DEV).bfloat16() for _ in range(2))
+    k, v = (torch.randn(total, nkv, d, generator=g, device=DEV).bfloat16() for _ in range(2))
+    cu = torch.tensor([total * i // docs for i in range(docs + 1)], dtype=torch.int32, device=DEV)
+    o, lse = ops.attention_forward(q, k, v, cu, None, causal, None)
+    dq, dk, dv = ops.attention_backward(do, q, k, v, o, lse, cu, None, causal, None)
+    for flags in (SHORT, TILED):
+        o2, _ = ops.attention_forward(q, k, v, cu, None, causal, None, flags=flags)
+        grads = ops.attention_backward(do, q, k, v, o, lse, cu, None, causal, None, flags=flags)
+        # sums in another order: some element of so many rounds the other way
+        assert torch.equal(o, o2) == (flags == fwd)
+        assert all(torch.equal(x, y) == (flags == bwd) for x, y in zip((dq, dk, dv), grads))
