@@ -1009,13 +1009,19 @@ void rows_weight(mi_rows_args& a, const Tensor& w, void* out, int64_t ldo) {
     a.w[i] = ptr(w); a.ldw[i] = w.stride(0); a.n[i] = (int32_t)w.size(0); a.out[i] = out; a.ldo[i] = ldo;
 }
 
-// The norm in front of a product of few rows: inside the product while few workgroups repeat it (3 x 1024 -> 1536: 5.2 us where the two
-// launches take 4.1 + 2.6), a launch of its own in front of wide ones, where normalising the operand in every workgroup
-// outweighs the launch (16 x 4096 -> 28672: 84 us inside, 36 + 3 as two; 3 x 1024 -> 32000: 20 and 12.6 + 3).
+// The norm in front of a product of few rows: inside the product while its workgroups repeat it cheaply, else a launch of its own, after
+// which they load the normalised rows.  Inside each of the features / 16 workgroups walks k values of every row, so the line lies at the product of
+// the two; from 4096 on the walk outlasts the launch with any number of workgroups.  us, inside / as two launches, 1 row and 16, weights
+// from memory, k -> features (x 2: SwiGLU):
+//   1024 -> 4096         6.4 / 7.4     7.4 / 9.2          2048 -> 4096       8.6 / 8.8    9.5 / 10.3       4096 -> 1536     11.1 / 10.5   15.1 / 13.4
+//   1024 -> 8192        11.1 / 10.6   13.0 / 13.7         2048 -> 6144      13.6 / 12.0  16.4 / 14.5       4096 -> 6144     22.3 / 18.5   29.2 / 23.0
+//   1024 -> 12288       15.8 / 14.0   18.5 / 17.8         2048 -> 8192      15.2 / 13.6  17.1 / 15.7       4096 -> 28672    74.8 / 48.6   96.8 / 67.5
+//   1024 -> 8192 x 2    11.2 / 12.2   13.1 / 13.7         2048 -> 4096 x 2  12.9 / 13.5  14.2 / 15.0       4096 -> 3072 x 2 17.9 / 17.3   21.9 / 21.3
+//   1024 -> 14336 x 2   19.2 / 17.2   22.8 / 20.8         2048 -> 6144 x 2  19.7 / 18.3  23.0 / 21.2       4096 -> 8192 x 2 37.2 / 33.4   46.0 / 41.8
 struct RowsNorm {
     Tensor x, weight;
     RowsNorm(const Tensor& x_, const Tensor& weight_, double eps, int64_t features, const Launch& l) : x(x_), weight(weight_) {
-        if (features <= 8192) return;
+        if (x_.size(1) <= 2048 && (features + 15) / 16 * x_.size(1) <= 512 * 1024) return;
         x = x_.is_contiguous() ? at::empty_like(x_) : at::empty(x_.sizes(), x_.options());
         const Tensor in = x_.contiguous();
         check(mi_rmsnorm_fwd(ptr(in), ptr(weight), ptr(x), nullptr, in.size(0), in.size(1), (float)eps, code_of(in), l.stream), "mi_rmsnorm_fwd");
@@ -1085,7 +1091,7 @@ OptTensor op_decode_layer(const Tensor& x, const Tensor& pos, const Tensor& norm
     rows_weight(a, dense, ptr(h), hidden);
     a.add[0] = ptr(x2); a.ldadd[0] = hidden;
     check(mi_rows_product(&a), "mi_rows_product");
-    const RowsNorm in2(h, norm2, eps2, 2 * inter, l);
+    const RowsNorm in2(h, norm2, eps2, inter, l);
     a = rows_args(in2.x, in2.weight, eps2, l);
     a.glu = 1;
     rows_weight(a, w_in, ptr(act), inter);

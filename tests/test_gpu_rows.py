@@ -77,6 +77,28 @@ def test_few_rows_with_norm(rows, k, n, glu, dtype):
     assert _lib.load().mi_rows_product(ctypes.byref(a)) == -3
 
 
+# each side of the lines between the norm inside the product and a launch of its own: (features, k)
+@pytest.mark.parametrize("n,k,inside", [(4096, 2048, True), (4097, 2048, False), (8192, 1024, True), (8200, 1024, False), (16, 2080, False),
+                                        (1536, 4096, False), (1000, 288, True)])
+def test_norm_in_front_of_a_product(n, k, inside):
+    print(f"case norm in front n={n} k={k}", flush=True)
+    x, w = _rand((5, k), torch.bfloat16, 1), _rand((n, k), torch.bfloat16, 2, k ** -0.5)
+    g = (1.0 + _rand((k,), torch.float32, 4, 0.1)).bfloat16()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = ops.norm_linear_rows(x, g, 1e-5, w)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "kernel" in e.key]
+    assert any("rows_kernel" in name for name in names) and any("rmsnorm" in name for name in names) == (not inside), names
+    xd = x.double()
+    normed = (xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-5) * g.double()).bfloat16().double()
+    ref, mag = normed @ w.double().t(), normed.abs() @ w.double().abs().t()
+    u = HALF_ULP[torch.bfloat16]
+    # as in test_few_rows_with_norm: a normalised element may round to the neighbour
+    err = (out.double() - ref).abs()
+    assert bool((err <= (u * ref.abs() + (2 * u + (k + 1) * 2.0 ** -24) * mag) * 1.01).all())
+    assert float(err.norm() / ref.norm()) < 3 * u
+
+
 @pytest.mark.parametrize("batch,heads,kv,dtype", [(1, 4, 2, torch.bfloat16), (3, 8, 8, torch.float16), (16, 4, 1, torch.bfloat16), (17, 4, 2, torch.bfloat16)])
 def test_native_decode_step_equals_the_modules(batch, heads, kv, dtype):
     print(f"case native decode batch={batch} heads={heads}/{kv} dtype={dtype}", flush=True)
