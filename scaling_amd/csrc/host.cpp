@@ -66,6 +66,11 @@ Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 Tensor float_buffer(size_t bytes, const Tensor& like) {
     return at::empty({(int64_t)((bytes + 3) / 4)}, like.options().dtype(at::kFloat));
 }
+// contiguous and on a 16-byte boundary, as the kernels read it
+Tensor vectors(const Tensor& t) {
+    const Tensor c = t.contiguous();
+    return (reinterpret_cast<uintptr_t>(c.data_ptr()) & 15) == 0 ? c : c.clone();
+}
 // x as rows of its last dimension
 int64_t row_count(const Tensor& x) { return x.size(-1) == 0 ? 0 : x.numel() / x.size(-1); }
 
@@ -162,8 +167,8 @@ struct AddNorm : Function<AddNorm> {
         TORCH_CHECK(!residual_.has_value() || (residual_->sizes() == x_.sizes() && residual_->scalar_type() == x_.scalar_type()),
                     "norm: x and residual do not match");
         Launch l(x_);
-        const Tensor x = x_.contiguous(), w = w_.contiguous(), b = b_.has_value() ? b_->contiguous() : Tensor();
-        const Tensor residual = residual_.has_value() ? residual_->contiguous() : Tensor();
+        const Tensor x = residual_.has_value() ? vectors(x_) : x_.contiguous(), w = w_.contiguous(), b = b_.has_value() ? b_->contiguous() : Tensor();
+        const Tensor residual = residual_.has_value() ? vectors(*residual_) : Tensor();
         const int64_t rows = row_count(x), hidden = x.size(-1);
         const Tensor sum = residual.defined() ? at::empty_like(x) : x_;
         Tensor y = at::empty_like(x), stats;
@@ -201,7 +206,7 @@ struct AddNorm : Function<AddNorm> {
             if (bias) db = at::zeros_like(saved[1]);
         } else {
             Launch l(saved[0]);
-            const Tensor x = saved[0].contiguous(), w = saved[1].contiguous(), dy = g[1].contiguous(), dsum = dsum_.defined() ? dsum_.contiguous() : Tensor();
+            const Tensor x = saved[0].contiguous(), w = saved[1].contiguous(), dy = g[1].contiguous(), dsum = dsum_.defined() ? vectors(dsum_) : Tensor();
             const int64_t rows = row_count(x), hidden = x.size(-1);
             const float eps = (float)ctx->saved_data["eps"].toDouble();
             dx = at::empty_like(x);
@@ -453,8 +458,7 @@ struct Projections : Function<Projections> {
             }
             Tensor add;
             if (residual.has_value()) {
-                add = residual->contiguous();
-                if (reinterpret_cast<uintptr_t>(add.data_ptr()) & 15) add = add.clone();
+                add = vectors(*residual);
                 pr[0].add = ptr(add);
                 pr[0].ldadd = pr[0].n;
             }

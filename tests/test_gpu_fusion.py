@@ -68,6 +68,27 @@ def test_norm_outputs_that_do_not_reach_the_loss():
     assert torch.equal(x.grad, a.grad)
 
 
+def _offset(t):
+    """The same values one element off a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
+    return flat.copy_(t.reshape(-1)).view(t.shape)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layer_norm", [False, True])
+def test_residual_stream_off_a_vector_boundary(layer_norm, dtype):
+    """A sum takes its addends and its gradient wherever they lie: the same bits."""
+    g = torch.Generator(DEV).manual_seed(5)
+    x, r, dy, ds = (torch.randn(37, 264, generator=g, device=DEV).to(dtype) for _ in range(4))
+    w = torch.ones(264, dtype=dtype, device=DEV, requires_grad=True)
+    out = []
+    for place in (lambda t: t, _offset):
+        a, c = place(x).requires_grad_(), place(r).requires_grad_()
+        s, y = ops.add_norm(a, c, w, None, 1e-5, layer_norm)
+        out.append([s, y] + list(torch.autograd.grad([s, y], [a, c, w], [place(ds), dy])))
+    assert all(torch.equal(p, q) for p, q in zip(*out))
+
+
 def _layer(dtype, default, hidden=256, inter=2.75, heads=4, **options):
     """The default block (LayerNorm, one QKV projection, GELU MLP, biases) or RMSNorm, grouped heads, SwiGLU without biases."""
     torch.manual_seed(7)
@@ -99,6 +120,15 @@ def _blocks(layer, x):
     """The layer's two blocks, with every residual sum a launch of its own."""
     io = _io(x)
     return layer.mlp_block(layer.attention_block(io.activations, io.cumulative_seq_lengths, io.position_ids))
+
+
+@pytest.mark.parametrize("default", [True, False])
+def test_layer_with_an_output_gradient_off_a_vector_boundary(default):
+    """Every product of that gradient moves to the library: float32 sums in another order."""
+    layer = _layer("float32", default)
+    x, dy = (torch.randn(2, 100, 256, device=DEV, generator=torch.Generator(DEV).manual_seed(s)) for s in (1, 2))
+    for p, q in zip(_step(layer, lambda t: layer(_io(t)).activations, x, dy), _step(layer, lambda t: layer(_io(t)).activations, x, _offset(dy))):
+        assert float((p - q).norm()) <= 1e-5 * float(p.norm()) + 1e-4     # the gradient of a key bias is a sum that cancels to nothing
 
 
 @pytest.mark.parametrize("default", [True, False])
