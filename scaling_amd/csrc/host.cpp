@@ -466,11 +466,9 @@ struct Projections : Function<Projections> {
         } else {
             for (int64_t i = 0; i < n; ++i) {
                 shape.back() = params[i].size(0);
-                const Tensor wt = params[i].t(), y = at::empty(shape, x.options());
-                Tensor y2 = y.view({rows, shape.back()});  // the output itself is no view: a caller may change it in place
-                if (at[i] >= 0) at::addmm_out(y2, params[at[i]], x2, wt);
-                else at::mm_out(y2, x2, wt);
-                out.push_back(y);
+                const Tensor wt = params[i].t();
+                // not a view of the product: a caller may change the output in place
+                out.push_back(at::_unsafe_view(at[i] >= 0 ? at::addmm(params[at[i]], x2, wt) : at::mm(x2, wt), shape));
             }
             if (residual.has_value()) out[0].add_(*residual);
         }
