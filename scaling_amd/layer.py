@@ -10,7 +10,7 @@ from typing import Callable, List, Optional
 import torch
 
 from .config import MLPType, TransformerArchitectureConfig
-from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm, idle_dropout
+from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm, idle_dropout, one_token_each
 
 
 class InferenceSettings:
@@ -114,7 +114,7 @@ class TransformerLayer(torch.nn.Module):
         s = x.inference_settings
         use_cache, reset_cache, cache_index = (False, False, 0) if s is None else (s.use_cache, s.reset_cache, s.cache_index)
         assert x.cumulative_seq_lengths is not None
-        if use_cache and not reset_cache and x.attention_scores_manipulation is None and self._decodes_natively():
+        if use_cache and not reset_cache and x.attention_scores_manipulation is None and one_token_each(x.activations) and self._decodes_natively():
             h = decode_layer(self, x.activations, x.cumulative_seq_lengths, x.position_ids, cache_index)
             if h is not None:
                 return self._next(x, h)

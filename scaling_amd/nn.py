@@ -685,6 +685,12 @@ class ParallelSelfAttention(torch.nn.Module):
                                     self._decode_operand(v), rotary=rotary, softmax_scale=self.softmax_scale, workspace=cache.workspace)
 
 
+def one_token_each(x: torch.Tensor) -> bool:
+    """Whether x [batch, 1, hidden] has no more rows than the kernels of a cached step take.  Asked before anything else: with 17 to 32
+    sequences the step runs in modules, and the checks and arguments of the native one are 20 - 30 us of host time a layer."""
+    return x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= ops.ROWS_MAX
+
+
 def decode_arguments(layer, batch: int, tokens: int, cache_index: int) -> Optional[tuple]:
     """The arguments of `ops.decode_layer` for the next `tokens` tokens of a layer of this package; None where such a step has
     to be refused (the module path raises): no cache, another batch, no room in the cache or the rotary table."""
@@ -706,7 +712,7 @@ def decode_layer(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tensor, p
     """One cached token per sequence through a whole layer (norms, projections, decode attention, MLP, residuals) in one native call.
     None, with nothing changed, where the call has to be refused or the kernels do not apply: the module path then raises or
     computes it."""
-    if position_ids is None or x.dim() != 3 or x.shape[1] != 1 or not x.is_cuda or cumulative_seq_lengths.numel() != x.shape[0] + 1:
+    if position_ids is None or not one_token_each(x) or not x.is_cuda or cumulative_seq_lengths.numel() != x.shape[0] + 1:
         return None
     arguments = decode_arguments(layer, x.shape[0], 1, cache_index)
     y = None if arguments is None else ops.decode_layer(x, position_ids.reshape(-1).contiguous(), arguments)

@@ -531,6 +531,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return out
 
 
+ROWS_MAX = 16   # MI_ROWS_MAX
+
+
 def norm_linear_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """rms_norm(x) @ weight.T of up to 16 rows [rows, k] (inference); None where the kernel does not apply."""
     if _taken_over((x, norm_weight, weight)):
