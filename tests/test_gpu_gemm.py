@@ -1,6 +1,10 @@
 """The matrix kernel of small projections (mi_gemm through ops.linear / ops.projections): forward products, input, weight and
 bias gradients against float64 products of the same rounded operands."""
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -57,8 +61,8 @@ def test_projections_and_their_gradients(rows, ins, outs, dtype):
     _close("dx", xg.grad, sum(d @ w for d, w in zip(dyd, wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd, wd)), sum(outs), dtype)
 
 
-# 16 and 17 rows (the kernel of few rows, the matrix kernel or the library), contractions on both sides of 3072
-@pytest.mark.parametrize("rows,ins,outs", [(16, 4096, (256,)), (17, 3064, (64, 128)), (17, 3072, (64, 128)), (40, 4096, (1024,)), (64, 8192, (512, 256, 256))])
+# 16 and 17 rows (the kernel of few rows, the matrix kernel or the library), contractions on both sides of 2560
+@pytest.mark.parametrize("rows,ins,outs", [(16, 4096, (256,)), (17, 2552, (64, 128)), (17, 2560, (64, 128)), (17, 3064, (64, 128)), (17, 3072, (64, 128)), (40, 4096, (1024,)), (64, 8192, (512, 256, 256))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_outputs_are_the_same_with_and_without_gradients(rows, ins, outs, dtype):
     """A forward pass under no_grad that is recomputed with gradients (reentrant checkpointing) has the same bits."""
@@ -73,12 +77,12 @@ def test_outputs_are_the_same_with_and_without_gradients(rows, ins, outs, dtype)
             assert all(torch.equal(a, b) for a, b in zip(want, call(inference)))
 
 
-@pytest.mark.parametrize("rows,ins,outs", [(16, 2048, (512,)), (17, 2040, (64, 128)), (17, 2048, (64, 128)), (32, 2816, (1024,)), (64, 2048, (2048, 512, 512)),
+@pytest.mark.parametrize("rows,ins,outs", [(16, 2048, (512,)), (17, 2552, (64, 128)), (17, 2560, (64, 128)), (32, 2816, (1024,)), (64, 2048, (2048, 512, 512)),
                                            (33, 3072, (256,))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_captured_products(rows, ins, outs, dtype):
-    """Products of inference in a captured graph, where a contraction from 2048 on takes the library: every replay on new inputs against
-    float64, with eager work between the replays."""
+    """Products of inference in a captured graph, on both sides of the line to the library: every replay on new inputs against float64, with
+    eager work between the replays."""
     x, ws, bs, dys = _case(rows, ins, outs, dtype, ins)
     wg, bg = [w.to(DEV) for w in ws], [None if b is None else b.to(DEV) for b in bs]
     inputs = [x, x.flip(0), 2 * x.roll(1, 1)]
@@ -104,6 +108,31 @@ def test_captured_products(rows, ins, outs, dtype):
             # the product is rounded, and with the residual the sum again
             err = (y.double().cpu() - want - add).norm()
             assert err <= 1.01 * eps * (want.norm() + (want + add).norm() * last) + 1e-6
+
+
+def test_capture_after_one_call():
+    """A first call outside the capture makes whatever the captured one needs, in a process that has used no library product."""
+    code = """
+import torch
+from scaling_amd import ops
+for k in (2048, 2552, 2560, 3072):
+    x, w = torch.ones(17, k, device="cuda", dtype=torch.bfloat16), torch.full((64, k), 0.5, device="cuda", dtype=torch.bfloat16)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(side):
+        ops.linear(x, w, None, None, True)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        y = ops.linear(x, w, None, None, True)
+    for scale in (1.0, 2.0, 4.0):
+        x.fill_(scale)
+        graph.replay()
+        assert bool((y == scale * k / 2).all()), (k, scale)
+print("captured")
+"""
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert run.returncode == 0 and "captured" in run.stdout, run.stderr[-2000:]
 
 
 def test_reentrant_checkpoint_over_a_long_contraction():

@@ -23,7 +23,7 @@ def _rand(shape, dtype, seed, std=1.0):
 # less than a block of 16, ragged, past the line of four (1024 blocks) and of two-block (2048 blocks) workgroups
 @pytest.mark.parametrize("rows,k,outs", [(1, 32, (8,)), (16, 96, (24, 8, 40)), (3, 1056, (1032, 264)), (5, 4096, (72,)), (2, 2816, (16, 16, 16400)),
                                          (16, 544, (33000,)),
-                                         # past 16 rows: the tiled kernel, and the library from 3072 features on
+                                         # past 16 rows: the tiled kernel
                                          (17, 3064, (72, 40)), (17, 3072, (72, 40))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_rows_through_linear(rows, k, outs, dtype):
