@@ -354,7 +354,11 @@ bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
 // issued one by one, with either forward product: 4096 -> 4096 57 and 74, 8192 -> 1024 54 and 76).  Up to MI_ROWS_MAX rows have a
 // kernel that splits the contraction.  Whether gradients are wanted does not matter: reentrant checkpointing runs a layer without
 // and again with them and counts on the same bits.
-bool long_chain(const Tensor& t, int64_t rows, int64_t k) { return t.scalar_type() != at::kFloat && rows > MI_ROWS_MAX && k >= 2560; }
+// float32 has a sixteenth of the matrix rate and no kernel for few rows.  8 - 64 rows, us issued one by one / in a graph, mi_gemm and library:
+// 1024 -> 1024 12.7 / 12.7 and 24.5 / 7.0; 2816 -> 1024 27.5 / 27.5 and 24.5 / 9.5; 4096 -> 1024 38 / 38 and 24.5 / 11.
+bool long_chain(const Tensor& t, int64_t rows, int64_t k) {
+    return t.scalar_type() == at::kFloat ? k >= 1536 : rows > MI_ROWS_MAX && k >= 2560;
+}
 bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
