@@ -347,18 +347,17 @@ bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
 // workgroup, the library splits it.  16-bit, 32 rows, us on the device / issued one by one, mi_gemm and library: 2048 -> 2048
 // 10.5 / 10.3 and 8.4 / 17.5; 2816 -> 1024 13.1 / 13.0 and 7.3 / 17.6; 4096 -> 4096 20.6 / 20.1 and 13.2 / 18.2; 8192 -> 1024
 // 35.0 / 34.7 and 15.0 / 17.9; with the weights from memory, per product of a captured graph: 2816 -> 1024 14.5 and 9.3 - 11.2; 2048 -> 512
-// 10.3 and 7.9; 2048 -> 2048 11.8 and 11.0 - 11.7; 1024 -> 2816 7.6 and 11.  The line lies between 2048, where a graph loses up to 2 us
-// with mi_gemm and a call issued alone 8 with the library, and 2816, where both are 4 - 5.  It is the same for a stream
-// that is being captured: what runs once before the capture has to have made the library's handles and loaded its kernels.
+// 10.3 and 7.9; 2048 -> 2048 11.8 and 11.0 - 11.7; 1024 -> 2816 7.6 and 11.  Below 3072 a graph loses up to 5 us with mi_gemm, and a
+// step that the host issues loses up to 45 with the library (prefill of 175 tokens, 3 layers with 2816 -> 1024: 1.10 and 1.26 ms).  The
+// line is the same for a stream that is being captured: what runs once before the capture has to have made the library's
+// handles and loaded its kernels.
 // A training step, which the host bounds at these sizes, keeps mi_gemm (forward and both gradients,
 // issued one by one, with either forward product: 4096 -> 4096 57 and 74, 8192 -> 1024 54 and 76).  Up to MI_ROWS_MAX rows have a
 // kernel that splits the contraction.  Whether gradients are wanted does not matter: reentrant checkpointing runs a layer without
 // and again with them and counts on the same bits.
-// float32 has a sixteenth of the matrix rate and no kernel for few rows.  8 - 64 rows, us issued one by one / in a graph, mi_gemm and library:
-// 1024 -> 1024 12.7 / 12.7 and 24.5 / 7.0; 2816 -> 1024 27.5 / 27.5 and 24.5 / 9.5; 4096 -> 1024 38 / 38 and 24.5 / 11.
-bool long_chain(const Tensor& t, int64_t rows, int64_t k) {
-    return t.scalar_type() == at::kFloat ? k >= 1536 : rows > MI_ROWS_MAX && k >= 2560;
-}
+// float32 has no kernel for few rows: 8 - 64 rows, us issued one by one, mi_gemm and library: 1024 -> 1024 12.7 and 24.5; 2816 -> 1024 27.5
+// and 24.5; 4096 -> 1024 38 and 24.5.
+bool long_chain(const Tensor& t, int64_t rows, int64_t k) { return k >= 3072 && (t.scalar_type() == at::kFloat || rows > MI_ROWS_MAX); }
 bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
