@@ -26,7 +26,7 @@ EXPORTS = (
     "mi_cross_entropy_padded", "mi_cross_entropy_mean_grad", "mi_loss_reduce", "mi_loss_row_scale", "mi_scale_inplace",
     "mi_swiglu_fwd", "mi_swiglu_bwd", "mi_rotary", "mi_rotary_complex",
     "mi_attn_fwd", "mi_attn_bwd_workspace_bytes", "mi_attn_bwd_workspace_bytes_kv", "mi_attn_bwd",
-    "mi_gemm", "mi_rows_product", "mi_transpose16", "mi_column_sum", "mi_add_rmsnorm_bwd", "mi_add_layernorm_fwd", "mi_add_layernorm_bwd", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
+    "mi_gemm", "mi_gemm_workspace_bytes", "mi_gemm_with_workspace", "mi_rows_product", "mi_transpose16", "mi_column_sum", "mi_add_rmsnorm_bwd", "mi_add_layernorm_fwd", "mi_add_layernorm_bwd", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
 )
 
 
@@ -156,6 +156,10 @@ def _declare(lib):
                                       c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_void_p]
     lib.mi_gemm.restype = c_int
     lib.mi_gemm.argtypes = [POINTER(MiGemmProblem), c_int, c_int, c_void_p]
+    lib.mi_gemm_workspace_bytes.restype = c_size_t
+    lib.mi_gemm_workspace_bytes.argtypes = [POINTER(MiGemmProblem), c_int, c_int]
+    lib.mi_gemm_with_workspace.restype = c_int
+    lib.mi_gemm_with_workspace.argtypes = [POINTER(MiGemmProblem), c_int, c_int, c_void_p, c_size_t, c_void_p]
     lib.mi_rows_product.restype = c_int
     lib.mi_rows_product.argtypes = [POINTER(MiRowsArgs)]
     lib.mi_transpose16.restype = c_int

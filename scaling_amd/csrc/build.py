@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 HOST_NAME = "mi355_host"
 HOST_PATH = os.path.join(HERE, HOST_NAME + ".so")
 SOURCES = ["abi.hip", "rmsnorm.hip", "swiglu.hip", "rotary.hip", "attn_host.hip", "attn_fwd.hip", "attn_bwd.hip",
-           "attn_decode.hip", "attn_f32.hip", "cross_entropy.hip", "gemm.hip", "rows.hip"]
+           "attn_decode.hip", "attn_f32.hip", "cross_entropy.hip", "gemm.hip", "gemm_wide.hip", "rows.hip"]
 F16_SOURCES = ["attn_fwd.hip", "attn_bwd.hip", "attn_decode.hip"]
 # packed fp32 VALU instructions stay disabled for every device translation unit; the kernels never
 # produce NaNs on purpose (masked scores are -inf and every inf - inf is guarded), so NaN-preserving

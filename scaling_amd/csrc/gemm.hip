@@ -16,6 +16,7 @@
 //   fp32:   v_mfma_f32_16x16x4 / 32x32x2, one 128-bit read of a "rows" operand feeds four products (the contraction index is
 //           visited in an order in which a lane's four values are consecutive)
 #include "common.h"
+#include "gemm_wide.h"
 
 #include <type_traits>
 
@@ -288,6 +289,42 @@ template <typename T> bool few_rows(const mi_gemm_problem* in, int count, mi_row
     return true;
 }
 
+// Calls of 16-bit types with a product of more than 3 GFLOP take the larger blocks of gemm_wide.hip: 1024 x 1024 x 1024 alone 9 us here and
+// 11.5 there, 4084 x 1024 x 1024 34 and 13.5.  What follows a ragged extent inside its last vector meets zeros there (rows of Q past the
+// contraction) or unstored results; rows must not overlap and a step of them has to be addressable in 31 bits.
+bool wide(const mi_gemm_problem* in, int count, int dtype) {
+    if (dtype != MI_BF16 && dtype != MI_F16) return false;
+    bool large = false;
+    for (int i = 0; i < count; ++i) {
+        const mi_gemm_problem& a = in[i];
+        if (a.m < 0 || a.n <= 0 || a.n_segments < 1 || a.n_segments > kMaxSegments || !a.c || !mi_aligned16(a.c) || a.ldc % 8 ||
+            (a.add && (!mi_aligned16(a.add) || a.ldadd % 8)) || (a.p_kmajor && !a.q_kmajor) || (a.p_sum && (!a.p_kmajor || a.n_segments > 1 || a.m % 8)))
+            return false;
+        for (int s = 0; s < a.n_segments; ++s) {
+            const auto& g = a.segments[s];
+            const int ep = a.p_kmajor ? a.m : g.k, eq = a.q_kmajor ? a.n : g.k;
+            if (!g.p || !g.q || g.k <= 0 || !mi_aligned16(g.p) || !mi_aligned16(g.q) || g.ldp % 8 || g.ldq % 8 || g.ldp < (ep + 7LL) / 8 * 8 ||
+                g.ldq < (eq + 7LL) / 8 * 8 || g.ldp >= (1 << 22) || g.ldq >= (1 << 22) || (!a.q_kmajor && g.k % 8))
+                return false;
+            large = large || 2.0 * a.m * (double)a.n * g.k > 3e9;
+        }
+    }
+    return large;
+}
+
+int launch_wide(const mi_gemm_problem* in, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
+    if (workspace == nullptr || !mi_aligned16(workspace)) workspace_bytes = 0;
+    const MiGemmPlan plan = mi_gemm_wide_plan(in, count, workspace_bytes, mi_compute_units());
+    const int rc = mi_gemm_wide(in, count, dtype, plan, workspace, st);
+    if (rc != MI_OK) return rc;
+    for (int i = 0; i < count; ++i) {
+        if (in[i].p_sum == nullptr || in[i].m == 0) continue;
+        const auto& g = in[i].segments[0];
+        if (const int e = mi_column_sum(g.p, g.ldp, g.k, in[i].m, in[i].p_sum, dtype, st); e != MI_OK) return e;
+    }
+    return MI_OK;
+}
+
 template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {
     constexpr int V = Elem<T>::kVec;
     Problems ps;
@@ -452,8 +489,18 @@ extern "C" int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, 
     return MI_OK;
 }
 
-extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
+extern "C" int mi_gemm_with_workspace(const mi_gemm_problem* problems, int count, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
     if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
+    if (wide(problems, count, dtype)) return launch_wide(problems, count, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
     return MI_OK;
+}
+
+extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
+    return mi_gemm_with_workspace(problems, count, dtype, nullptr, 0, stream);
+}
+
+extern "C" size_t mi_gemm_workspace_bytes(const mi_gemm_problem* problems, int count, int dtype) {
+    if (!problems || count != 1 || problems[0].m <= 0 || problems[0].n <= 0 || problems[0].n_segments != 1 || !wide(problems, count, dtype)) return 0;
+    return mi_gemm_wide_plan(problems, count, (size_t)1 << 30, mi_compute_units()).workspace_bytes;
 }

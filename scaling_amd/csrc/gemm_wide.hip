@@ -1,0 +1,595 @@
+// Matrix products of 16-bit types with 256 x 256 and 128 x 128 blocks: the projections of a layer, the LM head and their gradients.
+// Same problems as gemm.hip (operands "rows" or "kmajor", up to three segments in one sum, several problems per launch).
+//
+// What bounds them is the matrix pipe and, with all compute units busy, the power it draws: a 8192^3 product that runs 2.0 PFLOP/s on zeros
+// runs 1.5 on random numbers, and every byte an operand is moved costs time.  So
+//   * a wavefront owns 128 x 128 (64 x 64) of the block, four wavefronts per workgroup, one per SIMD: an operand fragment that is read from
+//     LDS feeds eight (four) products.  Eight wavefronts of 128 x 64 read 1.5 x as much and run 0.78 ms where this runs 0.70;
+//   * the products are v_mfma_*_16x16x32, whose accumulator traffic per multiply-add is half that of 32x32x16 (0.74 against 0.77 ms, the
+//     same kernel with eight wavefronts);
+//   * accumulators stay in accumulation registers for the whole kernel.  The products are inline assembly with such operands: left to
+//     itself the compiler moves 64 tuples of four registers around in the loop (1.1 ms);
+//   * tiles pass global -> LDS directly (buffer loads, so that whatever lies outside the matrix arrives as zero and steps past the
+//     contraction cost no memory traffic), one and a half (three) steps of 64 ahead.  A half of a 256 x 256 x 64 stage is refilled as
+//     soon as its fragments are in registers;
+//   * reads and loads are spread evenly between the products (sched_barrier pins the order): with one wavefront per SIMD a clump of more
+//     than three instructions between two products is a hole in the matrix pipe.
+// kmajor operands are read by LDS transpose reads from tiles in memory order, so all three layouts run at the same rate: 8192^3 bf16
+// 0.70 / 0.71 / 0.71 ms (x W^T, dy W, dy^T x), the library 0.68 / 0.79 / 0.91 on the same box.
+//
+// v_mfma_f32_16x16x32 operands, lane = 16 g + l:  A: row l, k = 8 g .. + 7;  B: column l, the same k;  C / D: column l, rows 4 g .. + 3.
+// A = Q (output features), B = P (output rows): a lane holds four consecutive features of one output row.
+#include "common.h"
+#include "gemm_wide.h"
+
+#include <type_traits>
+
+namespace {
+
+typedef short v4i16_t __attribute__((ext_vector_type(4)));
+typedef short v8i16_t __attribute__((ext_vector_type(8)));
+typedef uint32_t srd_t __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256;
+constexpr int kStep = 64;                                  // contraction indices of a stage
+constexpr int kBlockBytes = 64 * 128;                      // 64 x 64 elements
+constexpr int kHalfBytes = 2 * kBlockBytes;                // 128 rows (columns) of one operand
+constexpr int kStages128 = 4;
+constexpr int kQBase = 65536;                              // P stages below, Q stages above
+
+struct Segment { const char* p; const char* q; int64_t ldp, ldq; int k; };
+struct Problem {
+    Segment seg[MI_GEMM_MAX_SEGMENTS];
+    void* c; const void* bias; const void* add;
+    int64_t ldc, ldadd;
+    float* part;                                           // splits > 1: fp32 partial results [splits][tiles_m * tile][tiles_n * tile]
+    int n_seg, p_kmajor, q_kmajor, m, n, tiles_m, tiles_n, first_block, splits;
+};
+struct Problems { Problem p[MI_GEMM_MAX_PROBLEMS]; int count; };
+
+#define PIN() __builtin_amdgcn_sched_barrier(0)
+
+template <int N, int I = 0, class F> __device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
+template <typename T> struct Half16;
+template <> struct Half16<__bf16> {
+    typedef bf16x8_t frag_t;
+    static __device__ __forceinline__ void mma(f32x4_t& c, frag_t a, frag_t b) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
+};
+template <> struct Half16<_Float16> {
+    typedef f16x8_t frag_t;
+    static __device__ __forceinline__ void mma(f32x4_t& c, frag_t a, frag_t b) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
+};
+
+// A 64 x 64 block in LDS: 64 rows (of the matrix as it lies in memory) of eight 16-byte units.  A direct load writes 64 x 16 consecutive
+// bytes, so rows cannot be padded; the unit index of row r is XORed with swizzle(r) instead, which spreads the 16 rows that one pass of a
+// 128-bit read touches over all banks, and likewise the four rows x 32 bytes of two lane groups of a transpose read.
+__device__ __forceinline__ int swizzle(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
+
+// Direct loads of one operand.  A step of 64 contraction indices of `HALVES` x 128 rows is HALVES x 16 instructions, four per wavefront and
+// half.  The lane offsets are fixed, the bases of the buffer descriptors (one per half) move with the steps; their extents cover the present
+// step's rows and columns only (so they never exceed 2^31 bytes) and are 0 past the end.
+template <bool KMAJOR, int HALVES> struct Loader {
+    uint32_t off[4];
+    srd_t srd[HALVES];
+    int step_bytes, left;                                  // contraction indices from the present step on, in this segment
+
+    static __device__ __forceinline__ void source(int j, int wave, int lane, int& block, int& row, int& unit) {
+        const int n = 4 * wave + j;
+        block = n >> 3;
+        row = 8 * (n & 7) + (lane >> 3);
+        unit = (lane & 7) ^ swizzle(row);
+    }
+    __device__ __forceinline__ void open(const char* ptr, int64_t ld, int row0, int rows, int k, int wave, int lane) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            int block, r, u;
+            source(j, wave, lane, block, r, u);
+            off[j] = KMAJOR ? (uint32_t)(r * (int)ld * 2 + (block * 64 + 8 * u) * 2) : (uint32_t)((block * 64 + r) * (int)ld * 2 + u * 16);
+        }
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+            const int first = row0 + h * 128, n = rows - first;
+            const uint64_t base = (uint64_t)(ptr + (KMAJOR ? (int64_t)first * 2 : (int64_t)first * ld * 2));
+            // columns of a kmajor operand in whole vectors: rows of it start on 16-byte boundaries
+            const int extent = n <= 0 ? 0 : KMAJOR ? ((kStep - 1) * (int)ld + (n + 7) / 8 * 8) * 2 : ((min(n, 128) - 1) * (int)ld + kStep) * 2;
+            srd[h][0] = __builtin_amdgcn_readfirstlane((uint32_t)base);
+            srd[h][1] = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32) & 0xffffu);
+            srd[h][2] = __builtin_amdgcn_readfirstlane(extent);
+            srd[h][3] = 0x00020000u;
+        }
+        step_bytes = __builtin_amdgcn_readfirstlane(KMAJOR ? kStep * (int)ld * 2 : kStep * 2);
+        left = k;
+        if (left < kStep) last(wave, lane);
+    }
+    // the step that the contraction ends in
+    __device__ __forceinline__ void last(int wave, int lane) {
+        const int cut = (kStep - left) * (KMAJOR ? step_bytes / kStep : 2);
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) srd[h][2] = (uint32_t)max((int)srd[h][2] - cut, 0);
+        if (!KMAJOR) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                int block, r, u;
+                source(j, wave, lane, block, r, u);
+                if (8 * u >= left) off[j] = 0xfffffff0u;
+            }
+        }
+    }
+    // to the next step; true: this segment has none
+    __device__ __forceinline__ bool advance(int wave, int lane) {
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+            const uint64_t base = ((uint64_t)srd[h][0] | (uint64_t)srd[h][1] << 32) + (uint32_t)step_bytes;
+            srd[h][0] = (uint32_t)base;
+            srd[h][1] = (uint32_t)(base >> 32);
+        }
+        left -= kStep;
+        if (left < kStep) {
+            if (left <= 0) {
+#pragma unroll
+                for (int h = 0; h < HALVES; ++h) srd[h][2] = 0;
+                return true;
+            }
+            last(wave, lane);
+        }
+        return false;
+    }
+    // instruction j of half h to LDS address dst + C; the completion is tracked by the explicit waits of the caller
+    template <int C> __device__ __forceinline__ void load(int h, int j, uint32_t dst) const {
+        asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[j]), "s"(srd[h]), "s"(dst), "n"(C)
+                     : "memory", "m0", "scc");
+    }
+};
+
+// Fragments of 16 rows t of a 64 x 64 block for contraction indices 32 ks ..
+template <typename T, bool KMAJOR> struct Reader {
+    using F = typename Half16<T>::frag_t;
+    int b[4];
+    __device__ __forceinline__ void init(int base, int lane) {
+        const int l = lane & 15, g = lane >> 4;
+        if (!KMAJOR) {
+            b[0] = base + l * 128 + ((g ^ swizzle(l)) << 4);
+            b[1] = base + l * 128 + (((4 + g) ^ swizzle(l)) << 4);
+        } else {
+            // transpose read: lane l of a group of 16 points at contraction row l / 4, columns 4 (l % 4) ..; rows 8 g .. + 3 and 8 g + 4 .. + 7
+            const int r0 = 8 * g + (l >> 2), r1 = r0 + 4, e = (l >> 1) & 1, hb = l & 1;
+            b[0] = base + r0 * 128 + ((e ^ swizzle(r0)) << 4) + 8 * hb;
+            b[1] = base + r1 * 128 + ((e ^ swizzle(r1)) << 4) + 8 * hb;
+            b[2] = b[0] ^ 64;
+            b[3] = b[1] ^ 64;
+        }
+    }
+    __device__ __forceinline__ F get(const char* smem, int off, int t, int ks) const {
+        if constexpr (!KMAJOR) {
+            return *reinterpret_cast<const F*>(smem + b[ks] + off + t * 2048);
+        } else {
+            typedef __attribute__((address_space(3))) v4i16_t lds_v4;
+            const int x = (t & 1) << 5, o = off + ks * 4096;
+            const char *lo = smem + (b[2 * (t >> 1)] ^ x) + o, *hi = smem + (b[2 * (t >> 1) + 1] ^ x) + o;
+            const v4i16_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(__attribute__((address_space(3))) void*)(void*)lo);
+            const v4i16_t c = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(__attribute__((address_space(3))) void*)(void*)hi);
+            return __builtin_bit_cast(F, (v8i16_t)__builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+};
+
+// Results of a wavefront's 64 x 64 quadrant, with the bias, rounded, into 8 KB of LDS as rows.
+template <typename T> __device__ __forceinline__ void stage_quadrant(const Problem& pr, const f32x4_t (&acc)[4][4], char* stage, int n0, int lane) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    const int l = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        f32x4_t bias = {0.f, 0.f, 0.f, 0.f};
+        if (pr.bias != nullptr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bias[i] = Elem<T>::load1((const T*)pr.bias + min(n0 + 16 * nt + 4 * g + i, pr.n - 1));
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const int row = 16 * mt + l;
+            t4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = (T)(acc[mt][nt][i] + bias[i]);
+            *reinterpret_cast<t4*>(stage + row * 128 + (((2 * nt + (g >> 1)) ^ swizzle(row)) << 4) + 8 * (g & 1)) = v;
+        }
+    }
+}
+
+// The staged rows to memory, eight lanes per row of 128 bytes.
+template <typename T> __device__ __forceinline__ void store_quadrant(const Problem& pr, const char* stage, int m0, int n0, int lane) {
+    const int r8 = lane >> 3, u = lane & 7, n = n0 + 8 * u;
+    const char* src = stage + r8 * 128;
+    T* c = (T*)pr.c + (int64_t)(m0 + r8) * pr.ldc + n;
+    if (pr.add == nullptr && m0 + 64 <= pr.m && n0 + 64 <= pr.n) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<u32x4_t*>(c + 8 * i * pr.ldc) = *reinterpret_cast<const u32x4_t*>(src + i * 1024 + ((u ^ swizzle(8 * i + r8)) << 4));
+        return;
+    }
+    const T* add = (const T*)pr.add + (int64_t)(m0 + r8) * pr.ldadd + n;
+#pragma unroll 2
+    for (int i = 0; i < 8; ++i, c += 8 * pr.ldc, add += 8 * pr.ldadd) {
+        if (m0 + r8 + 8 * i >= pr.m || n >= pr.n) continue;
+        u32x4_t v = *reinterpret_cast<const u32x4_t*>(src + i * 1024 + ((u ^ swizzle(8 * i + r8)) << 4));
+        if (n + 8 <= pr.n) {
+            if (pr.add != nullptr) {                       // the product is rounded before it is added, as a separate product and sum would
+                float x[8], y[8];
+                Elem<T>::unpack(make_uint4(v[0], v[1], v[2], v[3]), x);
+                Elem<T>::unpack(*reinterpret_cast<const uint4*>(add), y);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] += y[e];
+                const uint4 s = Elem<T>::pack(x);
+                v = u32x4_t{s.x, s.y, s.z, s.w};
+            }
+            *reinterpret_cast<u32x4_t*>(c) = v;
+        } else {
+            const T* x = reinterpret_cast<const T*>(src + i * 1024 + ((u ^ swizzle(8 * i + r8)) << 4));
+#pragma unroll 1
+            for (int e = 0; e < pr.n - n; ++e) Elem<T>::store1(c + e, pr.add != nullptr ? Elem<T>::load1(x + e) + Elem<T>::load1(add + e) : Elem<T>::load1(x + e));
+        }
+    }
+}
+
+// A quadrant of a split's partial result: 16 rows of 64 bytes per store.
+__device__ __forceinline__ void store_part(const Problem& pr, const f32x4_t (&acc)[4][4], int split, int tile, int m0, int n0, int lane) {
+    const int64_t ld = (int64_t)pr.tiles_n * tile;
+    float* c = pr.part + ((int64_t)split * pr.tiles_m * tile + m0 + (lane & 15)) * ld + n0 + 4 * (lane >> 4);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) *reinterpret_cast<f32x4_t*>(c + 16 * mt * ld + 16 * nt) = acc[mt][nt];
+}
+
+// Both operands of a problem, stepped together; a split of a problem (of one segment) takes the contraction indices k0 .. k0 + k - 1.
+template <bool PK, bool QK, int HALVES> struct Operands {
+    Loader<PK, HALVES> p;
+    Loader<QK, HALVES> q;
+    int seg, k0, k;
+    __device__ __forceinline__ void open(const Problem& pr, int m0, int n0, int wave, int lane) {
+        const Segment& s = pr.seg[seg];
+        const int len = pr.splits > 1 ? k : s.k;
+        p.open(s.p + (PK ? (int64_t)k0 * s.ldp : (int64_t)k0) * 2, s.ldp, m0, pr.m, len, wave, lane);
+        q.open(s.q + (QK ? (int64_t)k0 * s.ldq : (int64_t)k0) * 2, s.ldq, n0, pr.n, len, wave, lane);
+    }
+    // returns the number of steps
+    __device__ __forceinline__ int start(const Problem& pr, int split, int m0, int n0, int wave, int lane) {
+        int steps = 0;
+        for (int i = 0; i < pr.n_seg; ++i) steps += (pr.seg[i].k + kStep - 1) / kStep;
+        seg = 0;
+        k0 = 0;
+        if (pr.splits > 1) {
+            const int first = (int)((int64_t)steps * split / pr.splits), end = (int)((int64_t)steps * (split + 1) / pr.splits);
+            k0 = first * kStep;
+            k = min(end * kStep, pr.seg[0].k) - k0;
+            steps = end - first;
+        }
+        open(pr, m0, n0, wave, lane);
+        return steps;
+    }
+    __device__ __forceinline__ void advance(const Problem& pr, int m0, int n0, int wave, int lane) {
+        const bool end = p.advance(wave, lane);
+        q.advance(wave, lane);
+        if (end && seg + 1 < pr.n_seg) {
+            ++seg;
+            open(pr, m0, n0, wave, lane);
+        }
+    }
+};
+
+template <int VM> __device__ __forceinline__ void wait_and_sync() {
+    PIN();
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
+    PIN();
+}
+
+// 256 x 256: two stages, each of two halves per operand (rows 0 - 127 and 128 - 255; a wavefront takes 64 rows of each).  A step is four
+// quadrants of 32 products in the order (A0, B0), (A0, B1), (A1, B1), (A1, B0), so that each brings one new half; fragments of the next
+// half are read between the products of the present one, and the loads of step s + 2 go out as soon as a half's readers are through.  Two
+// barriers per step, each a quarter of a quadrant after its boundary, where the reads before it have long completed.
+template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(const Problem& pr, int split, int tm, int tn, char* smem) {
+    using H = Half16<T>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+    const int m0 = tm * 256, n0 = tn * 256;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
+    Operands<PK, QK, 2> in;
+    const int steps = in.start(pr, split, m0, n0, wave, lane);
+    Reader<T, PK> rp;
+    Reader<T, QK> rq;
+    rp.init(wm * kBlockBytes, lane);
+    rq.init(kQBase + wn * kBlockBytes, lane);
+    f32x4_t acc[2][2][4][4];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) acc[a][b][c][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    typename H::frag_t pf[2][4][2], qf[2][4][2];           // [half or set][16 rows][32 contraction indices]
+    auto load_p = [&](auto s, auto h, auto j) { in.p.template load<s * 2 * kHalfBytes + h * kHalfBytes + j * 1024>(h, j, dst); PIN(); };
+    auto load_q = [&](auto s, auto h, auto j) { in.q.template load<kQBase + s * 2 * kHalfBytes + h * kHalfBytes + j * 1024>(h, j, dst); PIN(); };
+    auto read_p = [&](int s, int h, int f) { pf[h][f & 3][f >> 2] = rp.get(smem, (2 * s + h) * kHalfBytes, f & 3, f >> 2); PIN(); };
+    auto read_q = [&](int set, int s, int h, int f) { qf[set][f & 3][f >> 2] = rq.get(smem, (2 * s + h) * kHalfBytes, f & 3, f >> 2); PIN(); };
+    auto mma = [&](int h, int q, int set, int i) {         // one operand is the same for four products, the other for the turn of two rows
+        const int ks = i >> 4, mt = (i >> 2) & 3, nt = (mt & 1) ? 3 - (i & 3) : (i & 3);
+        H::mma(acc[h][q][mt][nt], qf[set][nt][ks], pf[h][mt][ks]);
+        PIN();
+    };
+    static_for<2>([&](auto s) {
+        static_for<2>([&](auto h) {
+            static_for<4>([&](auto j) { load_q(s, h, j); });
+            static_for<4>([&](auto j) { load_p(s, h, j); });
+        });
+        in.advance(pr, m0, n0, wave, lane);
+    });
+    wait_and_sync<24>();                                   // A0 and B0 of step 0
+#pragma unroll
+    for (int f = 0; f < 8; ++f) { read_q(0, 0, 0, f); read_p(0, 0, f); }
+    auto step = [&](auto s_c) {
+        constexpr int s = decltype(s_c)::value, X = s, Y = 1 - s;   // X holds B0, Y takes B1 and then the next B0
+        constexpr std::integral_constant<int, 0> h0{};
+        constexpr std::integral_constant<int, 1> h1{};
+        static_for<32>([&](auto i) {
+            if constexpr (i == 8) wait_and_sync<16>();     // A1, B1 of this step are there; A0, B0 are in everybody's registers
+            mma(0, 0, X, i);
+            if constexpr (i >= 8 && i % 3 == 2) read_q(Y, s, 1, i / 3 - 2);
+            if constexpr (i >= 8 && i % 6 == 4) load_q(s_c, h0, std::integral_constant<int, i / 6 - 1>{});
+        });
+        static_for<32>([&](auto i) {
+            mma(0, 1, Y, i);
+            if constexpr (i % 4 == 1) read_p(s, 1, i / 4);
+            if constexpr (i % 8 == 3) load_p(s_c, h0, std::integral_constant<int, i / 8>{});
+        });
+        static_for<32>([&](auto i) {
+            if constexpr (i == 8) wait_and_sync<16>();     // A0, B0 of the next step are there; A1, B1 are in everybody's registers
+            mma(1, 1, Y, i);
+            if constexpr (i >= 8 && i % 3 == 2) read_p(1 - s, 0, i / 3 - 2);
+            if constexpr (i >= 8 && i % 6 == 4) load_q(s_c, h1, std::integral_constant<int, i / 6 - 1>{});
+        });
+        static_for<32>([&](auto i) {
+            mma(1, 0, X, i);
+            if constexpr (i % 4 == 1) read_q(Y, 1 - s, 0, i / 4);
+            if constexpr (i % 8 == 3) load_p(s_c, h1, std::integral_constant<int, i / 8>{});
+            if constexpr (i == 30) in.advance(pr, m0, n0, wave, lane);
+        });
+    };
+    for (int i = 0; i < steps; i += 2) {                   // an odd count ends with a step of zeros
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+    }
+    asm volatile("s_nop 15" ::: "memory");                 // the last products' registers
+    wait_and_sync<0>();
+    if (pr.splits > 1) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) store_part(pr, acc[h][q], split, 256, m0 + h * 128 + wm * 64, n0 + q * 128 + wn * 64, lane);
+        return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            stage_quadrant<T>(pr, acc[h][q], smem + (4 * wave + 2 * h + q) * kBlockBytes, n0 + q * 128 + wn * 64, lane);
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i)
+        store_quadrant<T>(pr, smem + (4 * wave + i) * kBlockBytes, m0 + (i >> 1) * 128 + wm * 64, n0 + (i & 1) * 128 + wn * 64, lane);
+}
+
+// 128 x 128: four stages, loads three steps ahead, one barrier per step a quarter of its products after its start.  The fragments of the
+// next step are read between the products of the present one.
+template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(const Problem& pr, int split, int tm, int tn, char* smem) {
+    using H = Half16<T>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+    const int m0 = tm * 128, n0 = tn * 128;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
+    Operands<PK, QK, 1> in;
+    const int steps = in.start(pr, split, m0, n0, wave, lane);
+    Reader<T, PK> rp;
+    Reader<T, QK> rq;
+    rp.init(wm * kBlockBytes, lane);
+    rq.init(kQBase + wn * kBlockBytes, lane);
+    f32x4_t acc[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) acc[c][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    typename H::frag_t pf[2][4][2], qf[2][4][2];           // [set][16 rows][32 contraction indices]
+    auto load = [&](auto j, uint32_t stage) {
+        if constexpr (j < 4) in.q.template load<kQBase + j * 1024>(0, j, dst + stage);
+        else in.p.template load<(j - 4) * 1024>(0, j - 4, dst + stage);
+        PIN();
+    };
+    auto read = [&](int set, int f, int stage) {           // the fragments of contraction indices 0 .. 31 first
+        const int t = (f >> 1) & 3, ks = f >> 3;
+        if (f & 1) pf[set][t][ks] = rp.get(smem + stage, 0, t, ks);
+        else qf[set][t][ks] = rq.get(smem + stage, 0, t, ks);
+        PIN();
+    };
+    auto mma = [&](int set, int i) {
+        const int ks = i >> 4, mt = (i >> 2) & 3, nt = (mt & 1) ? 3 - (i & 3) : (i & 3);
+        H::mma(acc[mt][nt], qf[set][nt][ks], pf[set][mt][ks]);
+        PIN();
+    };
+#pragma unroll
+    for (int s = 0; s < kStages128; ++s) {
+        static_for<8>([&](auto j) { load(j, s * kHalfBytes); });
+        in.advance(pr, m0, n0, wave, lane);
+    }
+    wait_and_sync<24>();                                   // step 0
+#pragma unroll
+    for (int f = 0; f < 16; ++f) read(0, f, 0);
+    int stage = 0;                                         // of the present step
+    auto step = [&](auto x_c) {
+        constexpr int X = decltype(x_c)::value, Y = 1 - X;
+        const int next = (stage + kHalfBytes) & (kStages128 * kHalfBytes - 1);
+        static_for<32>([&](auto i) {
+            if constexpr (i == 8) wait_and_sync<16>();     // the next step is there; the present one is in everybody's registers
+            mma(X, i);
+            if constexpr (i >= 8 && i < 24) read(Y, i - 8, next);
+            if constexpr (i >= 8 && i % 3 == 2) load(std::integral_constant<int, i / 3 - 2>{}, stage);
+            if constexpr (i == 30) in.advance(pr, m0, n0, wave, lane);
+        });
+        stage = next;
+    };
+    for (int i = 0; i < steps; i += 2) {                   // an odd count ends with a step of zeros
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+    }
+    asm volatile("s_nop 15" ::: "memory");
+    wait_and_sync<0>();
+    if (pr.splits > 1) {
+        store_part(pr, acc, split, 128, m0 + wm * 64, n0 + wn * 64, lane);
+        return;
+    }
+    stage_quadrant<T>(pr, acc, smem + wave * kBlockBytes, n0 + wn * 64, lane);
+    store_quadrant<T>(pr, smem + wave * kBlockBytes, m0 + wm * 64, n0 + wn * 64, lane);
+}
+
+// Blocks of a problem are handed to the XCDs (workgroups modulo 8) in contiguous runs, in groups of four block rows, so that the workgroups
+// that share an L2 read the same rows and columns at the same time.
+template <typename T, int TILE>
+__global__ __launch_bounds__(kThreads, 1) void wide_kernel(const Problems ps) {
+    __shared__ __attribute__((aligned(1024))) char smem[2 * kQBase];
+    int i = 0;
+    while (i + 1 < ps.count && (int)blockIdx.x >= ps.p[i + 1].first_block) ++i;
+    const Problem& pr = ps.p[i];
+    const int tiles = pr.tiles_m * pr.tiles_n, total = tiles * pr.splits;
+    const int b = blockIdx.x - pr.first_block, xcd = b & 7, idx = b >> 3, each = total >> 3, rest = total & 7;
+    if (idx >= each + (xcd < rest)) return;                // first_block is a multiple of eight
+    const int item = xcd * each + min(xcd, rest) + idx, split = item / tiles, t = item - split * tiles;
+    constexpr int kGroup = 4;
+    const int per_group = kGroup * pr.tiles_n, group = t / per_group, first = group * kGroup, height = min(kGroup, pr.tiles_m - first);
+    const int in_group = t - group * per_group, tn = in_group / height, tm = first + in_group - tn * height;
+    if constexpr (TILE == 256) {
+        if (pr.p_kmajor) tile256<T, true, true>(pr, split, tm, tn, smem);
+        else if (pr.q_kmajor) tile256<T, false, true>(pr, split, tm, tn, smem);
+        else tile256<T, false, false>(pr, split, tm, tn, smem);
+    } else {
+        if (pr.p_kmajor) tile128<T, true, true>(pr, split, tm, tn, smem);
+        else if (pr.q_kmajor) tile128<T, false, true>(pr, split, tm, tn, smem);
+        else tile128<T, false, false>(pr, split, tm, tn, smem);
+    }
+}
+
+// Sum of the partial results of a split problem in a fixed order, bias and residual as above: four features per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void split_sum_kernel(const Problem pr, int tile) {
+    const int groups = (pr.n + 3) / 4;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int m = (int)(i / groups), n = 4 * (int)(i - (int64_t)m * groups);
+    if (m >= pr.m) return;
+    const int64_t ld = (int64_t)pr.tiles_n * tile, stride = (int64_t)pr.tiles_m * tile * ld;
+    const float* p = pr.part + (int64_t)m * ld + n;
+    f32x4_t x = *reinterpret_cast<const f32x4_t*>(p);
+    for (int s = 1; s < pr.splits; ++s) x += *reinterpret_cast<const f32x4_t*>(p + s * stride);
+    T* c = (T*)pr.c + (int64_t)m * pr.ldc + n;
+    const T* add = pr.add != nullptr ? (const T*)pr.add + (int64_t)m * pr.ldadd + n : nullptr;
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    t4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int col = min(n + e, pr.n - 1);
+        v[e] = (T)(pr.bias != nullptr ? x[e] + Elem<T>::load1((const T*)pr.bias + col) : x[e]);
+        if (add != nullptr) v[e] = (T)((float)v[e] + Elem<T>::load1(add + col - n));
+    }
+    if (n + 4 <= pr.n) {
+        *reinterpret_cast<t4*>(c) = v;
+    } else {
+        for (int e = 0; e < pr.n - n; ++e) c[e] = v[e];
+    }
+}
+
+int steps_of(const mi_gemm_problem& a) {
+    int steps = 0;
+    for (int s = 0; s < a.n_segments; ++s) steps += (a.segments[s].k + kStep - 1) / kStep;
+    return steps;
+}
+int64_t tiles_of(const mi_gemm_problem& a, int tile) { return (int64_t)((a.m + tile - 1) / tile) * ((a.n + tile - 1) / tile); }
+
+}  // namespace
+
+// Blocks and splits by the time they are expected to take (us): a block costs `fixed` and `per_step` per step of 64, blocks come in rounds of
+// one per compute unit, a split adds the traffic of its partial results and a launch.  Times that the figures come from, 128 / 256, bf16:
+//   4084 x 1024, k 1024 13.4 / 25.2    4084 x 1024, k 4096 34.0 / 70.3    4084 x 4096, k 1024 47.7 / 32.5
+//   2047 x 50257, k 1024 335 / 216     50257 x 1024, k 2047 283 / 198     2048 x 2048, k 2048 20.5 / 39.6    2048 x 5632, k 2048 56.3 / 43.3
+MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t workspace_bytes, int cus) {
+    MiGemmPlan best{};
+    best.us = 1e30;
+    for (int tile = 128; tile <= 256; tile += 128) {
+        const double fixed = tile == 256 ? 7.5 : 5.5, per_step = tile == 256 ? 1.3 : 0.48;
+        double work = 0, longest = 0, rounds_time = 0;
+        int64_t tiles = 0;
+        for (int i = 0; i < count; ++i) {
+            const double t = fixed + per_step * steps_of(in[i]);
+            const int64_t n = tiles_of(in[i], tile);
+            work += n * t;
+            tiles += n;
+            longest = t > longest ? t : longest;
+        }
+        // one problem: whole rounds; several: their blocks fill each other's gaps
+        rounds_time = count == 1 ? longest * (double)((tiles + cus - 1) / cus) : (work / cus + (tiles > cus ? 0.5 * longest : 0));
+        double us = rounds_time > longest ? rounds_time : longest;
+        if (us < best.us) best = MiGemmPlan{us, tile, 1, 0};
+        if (count == 1 && in[0].n_segments == 1) {
+            const int steps = steps_of(in[0]);
+            for (int s = 2; s <= 16 && tiles * s <= cus && steps / s >= 8; ++s) {
+                const size_t bytes = (size_t)tiles * tile * tile * 4 * s;
+                if (bytes > workspace_bytes) break;
+                us = fixed + per_step * ((steps + s - 1) / s) + 3.0 + 2.0 * bytes / 5e6;
+                if (us < best.us) best = MiGemmPlan{us, tile, s, bytes};
+            }
+        }
+    }
+    return best;
+}
+
+int mi_gemm_wide(const mi_gemm_problem* in, int count, int dtype, const MiGemmPlan& plan, void* workspace, hipStream_t st) {
+    const int tile = plan.tile;
+    Problems ps;
+    ps.count = count;
+    int order[MI_GEMM_MAX_PROBLEMS];
+    for (int i = 0; i < count; ++i) {                      // longest contraction first: the launch then ends with short blocks
+        int j = i;
+        for (; j > 0 && steps_of(in[order[j - 1]]) < steps_of(in[i]); --j) order[j] = order[j - 1];
+        order[j] = i;
+    }
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        const mi_gemm_problem& a = in[order[i]];
+        Problem& p = ps.p[i];
+        for (int s = 0; s < a.n_segments; ++s) {
+            const auto& g = a.segments[s];
+            p.seg[s] = Segment{(const char*)g.p, (const char*)g.q, g.ldp, g.ldq, g.k};
+        }
+        p.c = a.c; p.bias = a.bias; p.add = a.add; p.ldc = a.ldc; p.ldadd = a.ldadd; p.n_seg = a.n_segments;
+        p.p_kmajor = a.p_kmajor; p.q_kmajor = a.q_kmajor; p.m = a.m; p.n = a.n;
+        p.tiles_m = (a.m + tile - 1) / tile;
+        p.tiles_n = (a.n + tile - 1) / tile;
+        p.splits = plan.splits;
+        p.part = (float*)workspace;
+        p.first_block = (int)total;
+        total += ((int64_t)p.tiles_m * p.tiles_n * p.splits + 7) / 8 * 8;
+        if (total > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "gemm: too many tiles");
+    }
+    if (total == 0) return MI_OK;
+    const dim3 grid((unsigned)total), block(kThreads);
+    const Problem& p0 = ps.p[0];
+    const dim3 sum_grid((unsigned)(((int64_t)p0.m * ((p0.n + 3) / 4) + 255) / 256));
+    const auto go = [&](auto t) {
+        using T = decltype(t);
+        if (tile == 256) wide_kernel<T, 256><<<grid, block, 0, st>>>(ps);
+        else wide_kernel<T, 128><<<grid, block, 0, st>>>(ps);
+        if (plan.splits > 1) split_sum_kernel<T><<<sum_grid, block, 0, st>>>(p0, tile);
+    };
+    if (dtype == MI_BF16) go(__bf16{});
+    else go(_Float16{});
+    return mi_check_launch("gemm_wide");
+}

@@ -315,3 +315,65 @@ def test_batched_gradients(rows, ins, outs):
     with FlopCounterMode(display=False) as counter:
         torch.autograd.grad(ys, inputs, [g[0] for g in gs])
     assert counter.get_total_flops() == sum(4 * rows * ins * o for o in outs)
+
+
+# products over 3 GFLOP take blocks of 128 or 256: remainders in every direction, one segment and several problems, contractions that
+# are split over the chip (512 x 8200 -> 520, 264 x 16392 -> 520) and that end inside a step
+@pytest.mark.parametrize("rows,ins,outs", [
+    (1031, 1032, (1544,)), (2049, 1096, (1048, 264)), (513, 8200, (520,)), (264, 16392, (520,)), (129, 3080, (4104, 1032, 1032)),
+    (2050, 2056, (5640,)), (4097, 520, (4104,)),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_large_products_and_their_gradients(rows, ins, outs, dtype):
+    print(f"case wide rows={rows} in={ins} out={outs} dtype={dtype}", flush=True)
+    x, ws, bs, dys = (t.to(DEV) if torch.is_tensor(t) else [u if u is None else u.to(DEV) for u in t] for t in _case(rows, ins, outs, dtype, rows + ins))
+    for t in [x, *ws, *(b for b in bs if b is not None)]:
+        t.requires_grad_()
+    ys = ops.projections(x, ws, bs)
+    torch.autograd.backward(ys, dys)
+    xd, wd, dyd = x.detach().double(), [w.detach().double() for w in ws], [d.double() for d in dys]
+    close = lambda name, got, ref, magnitude, k: _close(name, got, ref.cpu(), magnitude.cpu(), k, dtype)
+    for i in range(len(outs)):
+        b = bs[i].detach().double() if bs[i] is not None else torch.zeros(outs[i], dtype=torch.float64, device=DEV)
+        close(f"y{i}", ys[i].detach(), xd @ wd[i].t() + b, xd.abs() @ wd[i].abs().t() + b.abs(), ins)
+        close(f"dw{i}", ws[i].grad, dyd[i].t() @ xd, dyd[i].abs().t() @ xd.abs(), rows)
+        if bs[i] is not None:
+            close(f"db{i}", bs[i].grad, dyd[i].sum(0), dyd[i].abs().sum(0), rows)
+    close("dx", x.grad, sum(d @ w for d, w in zip(dyd, wd)), sum(d.abs() @ w.abs() for d, w in zip(dyd, wd)), sum(outs))
+
+
+def test_large_product_with_residual_and_in_a_graph():
+    """The residual is added to the rounded product; replays with eager work between them give the eager bits."""
+    g = torch.Generator().manual_seed(3)
+    x, w, res = (torch.randn(*s, generator=g).bfloat16().to(DEV) for s in ((1200, 2056), (1032, 2056), (1200, 1032)))
+    with torch.no_grad():
+        want = ops.linear(x, w, None, res)
+        assert torch.equal(want, ops.linear(x, w) + res)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = ops.linear(x, w, None, res)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            (x.float() @ w.float().t()).sum().item()
+            assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("rows,hidden,vocab", [(2047, 1024, 50257), (300, 520, 20003), (1025, 2048, 128)])
+def test_lm_head_products(rows, hidden, vocab):
+    """Loss and gradients of the chunked LM head over ragged vocabularies against float64."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    h = torch.randn(rows, hidden, generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(vocab, hidden, generator=g, device=DEV) * 2 / hidden ** 0.5).bfloat16().requires_grad_()
+    t = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    weights = torch.ones(rows, device=DEV)
+    loss = ops.linear_cross_entropy(h, w, t, weights)[0]
+    loss.backward()
+    hd, wd = h.detach().double().requires_grad_(), w.detach().double().requires_grad_()
+    ref = torch.nn.functional.cross_entropy(hd @ wd.t(), t)
+    ref.backward()
+    assert abs(loss.item() - ref.item()) <= 1e-3 * ref.item()
+    # logits and their gradient are rounded to bfloat16 (2^-9 on average a half of 2^-8 each, over sums with independent errors)
+    for name, a, b in (("dh", h.grad, hd.grad), ("dw", w.grad, wd.grad)):
+        err = ((a.double() - b).norm() / b.norm()).item()
+        assert err <= 2.0 ** -7, f"{name}: {err}"
