@@ -336,3 +336,29 @@ def test_lm_head_gradients_under_saved_tensor_hooks(chunk):
         got = step()
     assert held and all(torch.equal(t, before) for t, before in held)
     assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+@pytest.mark.parametrize("vocab,offset", [(4104, 0), (4099, 3), (37001, 5), (128256, 0), (140007, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_first_index_of_the_maximum_anywhere_in_a_row(vocab, offset, dtype):
+    """The streaming kernel reads again the one vector per thread that raised its maximum: first and last elements, both sides of the
+    steps of a workgroup, rows off a 16-byte boundary, ties between vectors and between a vector and the loose elements, rows of -inf."""
+    print(f"case argmax vocab={vocab} offset={offset} dtype={dtype}", flush=True)
+    v = 16 // torch.finfo(dtype).bits * 8
+    at = sorted({p for p in (0, 1, 7, 8, 9, 512 * v - 1, 512 * v, 512 * v + 9, 4 * 512 * v, 4 * 512 * v + 1, 5 * 512 * v + 3, vocab // 2, vocab - 9, vocab - 2, vocab - 1) if 0 <= p < vocab})
+    rows = len(at)
+    g = torch.Generator().manual_seed(vocab)
+    flat = torch.randn((2 * rows + 1) * vocab + offset, generator=g).clamp_(-4, 4).to(dtype).to(DEV)
+    x = flat[offset:].view(2 * rows + 1, vocab)
+    for r, p in enumerate(at):
+        x[r, p] = 9.0                                      # alone
+        x[rows + r, p] = 9.0                               # with later copies of it
+        for later in (p + 1, p + 8 * 512, vocab - 1):
+            if p < later < vocab:
+                x[rows + r, later] = 9.0
+    x[-1] = -float("inf")
+    targets = torch.tensor(at + at + [0], device=DEV)
+    losses, argmax = ops.cross_entropy_forward(x, targets)
+    assert argmax.tolist() == at + at + [0]
+    ref = torch.nn.functional.cross_entropy(x[:-1].double(), targets[:-1], reduction="none")
+    assert torch.allclose(losses[:-1].double(), ref, rtol=1e-5, atol=1e-5)
