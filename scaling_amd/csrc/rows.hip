@@ -12,7 +12,7 @@
 //
 // What is left is latency: descriptors, then weights and rows, then the norm's barrier, then the sums.  In a decode step of a 4-layer model
 // of hidden 1024 (3 sequences) a product of the tiled kernel took 9.2 us, with 3 us for each norm and activation beside
-// it; a launch here 6.2 with those included (4.1 when the weights are cached: 3 x 1024 x 1024).  Wide products run at the
+// it; a launch here 5.7 - 6.1 with those included (4.1 when the weights are cached: 3 x 1024 x 1024).  Wide products run at the
 // rate of the weights: 16 x 4096 -> 128256 191 us, 5.5 TB/s.
 #include "common.h"
 
@@ -24,15 +24,30 @@ constexpr int kMaxWeights = MI_ROWS_MAX_WEIGHTS, kMaxRows = MI_ROWS_MAX;
 constexpr int kStep = 32;              // contraction indices per product
 constexpr int kRedStride = 20;         // floats per row of partial sums: 16-byte aligned, spread over the banks
 
+// Values that are in registers from here on (the compiler otherwise loads an argument right before its use).
+template <typename V> __device__ __forceinline__ void arrived1(V& v) { asm volatile("" : "+s"(v)); }
+template <typename V> __device__ __forceinline__ void arrived1(V*& v) {   // a pointer to global memory stays one
+    uintptr_t at = (uintptr_t)v;
+    asm volatile("" : "+s"(at));
+    v = (V*)(__attribute__((address_space(1))) V*)at;
+}
+template <typename... V> __device__ __forceinline__ void arrived(V&... v) { (arrived1(v), ...); }
+
+struct Matrix {
+    const void *w, *bias, *add;
+    void* out;
+    int64_t ldw, ldadd, ldo;
+    int n, first_tile;
+    __device__ __forceinline__ void arrive() { arrived(w, bias, add, out, ldw, ldadd, ldo, n, first_tile); }
+};
+
 struct RowsParams {
-    const void* x; const void* norm_weight;
-    const void* w[kMaxWeights]; const void* bias[kMaxWeights]; const void* add[kMaxWeights];
-    void* out[kMaxWeights];
-    int64_t ldx, ldw[kMaxWeights], ldadd[kMaxWeights], ldo[kMaxWeights];
+    const void *x, *norm_weight;
+    int64_t ldx;
     int32_t* count_up;
-    int n[kMaxWeights], first_tile[kMaxWeights];
     int n_weights, rows, k;
     float eps;
+    Matrix m[kMaxWeights];
 };
 
 template <typename T> struct RowsMfma;
@@ -57,25 +72,39 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, G = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    int mat = 0;
-    if constexpr (!GLU)
-        while (mat + 1 < p.n_weights && (int)blockIdx.x >= p.first_tile[mat + 1]) ++mat;
-    const int n0 = ((int)blockIdx.x - p.first_tile[mat]) * FEATURES, n = p.n[mat];
-    if (p.count_up != nullptr && blockIdx.x == 0 && tid < p.rows) p.count_up[tid] += 1;
+    // All arguments at once: read where they are used they are a chain of scalar loads from three or four cache lines, each a trip to memory
+    // on a fresh launch, before the weights are requested and again in front of the results (with the residual and the second chunk requested
+    // up front too, a decode step's five launches per layer at 3 x 1024: 25.0 -> 23.6 us).
+    const void *x = p.x, *norm_weight = p.norm_weight;
+    int64_t ldx = p.ldx;
+    int n_weights = p.n_weights, rows = p.rows, k = p.k;
+    int32_t* count_up = p.count_up;
+    arrived(x, norm_weight, ldx, n_weights, rows, k, count_up);
+    Matrix mx = p.m[0], gate = p.m[1];                     // this workgroup's; GLU: both
+    {
+        Matrix m2 = p.m[2];
+        mx.arrive(); gate.arrive(); m2.arrive();
+        if constexpr (!GLU) {
+            const bool second = n_weights > 1 && (int)blockIdx.x >= gate.first_tile, third = n_weights > 2 && (int)blockIdx.x >= m2.first_tile;
+            if (second) mx = gate;
+            if (third) mx = m2;
+        }
+    }
+    const int n0 = ((int)blockIdx.x - mx.first_tile) * FEATURES, n = mx.n;
 
     // this wavefront's products: an even number, so that it covers whole 128-byte lines
-    const int steps = p.k / kStep;
+    const int steps = k / kStep;
     const int per = ((steps + NW - 1) / NW + 1) & ~1;
     const int s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
 
     // rows past the last one and features past n repeat the last: their results are not stored
-    const T* xr = reinterpret_cast<const T*>(p.x) + (int64_t)min(l16, p.rows - 1) * p.ldx + 8 * G;
-    const T* gr = reinterpret_cast<const T*>(p.norm_weight) + 8 * G;
+    const T* xr = reinterpret_cast<const T*>(x) + (int64_t)min(l16, rows - 1) * ldx + 8 * G;
+    const T* gr = reinterpret_cast<const T*>(norm_weight) + 8 * G;
     const T* wr[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        const int i = GLU ? t : mat;
-        wr[t] = reinterpret_cast<const T*>(p.w[i]) + (int64_t)min(n0 + (GLU ? 0 : 16 * t) + l16, n - 1) * p.ldw[i] + 8 * G;
+        const Matrix& m = GLU && t == 1 ? gate : mx;
+        wr[t] = reinterpret_cast<const T*>(m.w) + (int64_t)min(n0 + (GLU ? 0 : 16 * t) + l16, n - 1) * m.ldw + 8 * G;
     }
     // Weights, rows and norm weights of CH products.  No request is conditional, so that all of them are in flight together: those
     // past this wavefront's last product repeat it and are not used.
@@ -92,6 +121,22 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
     };
     Chunk ca, cb;
     if (s0 < s1) request(ca, s0);
+    if (s0 + CH < s1) request(cb, s0 + CH);                // in front of the loop, where it waits for nothing
+    const bool counts = count_up != nullptr && blockIdx.x == 0;
+    const int32_t count = (counts ? count_up : reinterpret_cast<const int32_t*>(x))[counts ? min(tid, rows - 1) : 0];
+
+    // bias and residual of the results that this thread stores, requested with the weights, clamped like them and without a branch (in its
+    // place the first element of x), which would wait for all that is under way
+    constexpr int kOut = (FEATURES * kMaxRows + 64 * NW - 1) / (64 * NW);
+    T bias[kOut], add[kOut];
+    if constexpr (!GLU) {
+#pragma unroll
+        for (int i = 0; i < kOut; ++i) {
+            const int idx = tid + i * 64 * NW, m = min(idx / FEATURES, rows - 1), f = min(n0 + idx % FEATURES, n - 1);
+            bias[i] = reinterpret_cast<const T*>(mx.bias != nullptr ? mx.bias : x)[mx.bias != nullptr ? f : 0];
+            add[i] = reinterpret_cast<const T*>(mx.add != nullptr ? mx.add : x)[mx.add != nullptr ? (int64_t)m * mx.ldadd + f : 0];
+        }
+    }
 
     float rstd = 1.f;
     if constexpr (NORM) {
@@ -116,7 +161,7 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
         float total = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) total += squares[w][l16];
-        rstd = rsqrtf(total / (float)p.k + p.eps);
+        rstd = rsqrtf(total / (float)k + p.eps);
     }
 
     f32x4v acc[TILES];
@@ -141,11 +186,11 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
         }
     };
     for (int s = s0; s < s1; s += 2 * CH) {
-        if (s + CH < s1) request(cb, s + CH);
         multiply(ca, s);
+        if (s + 2 * CH < s1) request(ca, s + 2 * CH);
         if (s + CH < s1) {
-            if (s + 2 * CH < s1) request(ca, s + 2 * CH);
             multiply(cb, s + CH);
+            if (s + 3 * CH < s1) request(cb, s + 3 * CH);
         }
     }
 
@@ -153,24 +198,26 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
 #pragma unroll
     for (int t = 0; t < TILES; ++t) *reinterpret_cast<f32x4v*>(&red[t][wave][l16][4 * G]) = acc[t];
     __syncthreads();
-    for (int idx = tid; idx < FEATURES * kMaxRows; idx += 64 * NW) {
-        const int m = idx / FEATURES, f = idx % FEATURES;
-        if (m >= p.rows || n0 + f >= n) continue;
+    if (counts && tid < rows) count_up[tid] = count + 1;
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+        const int idx = tid + i * 64 * NW, m = idx / FEATURES, f = idx % FEATURES;
+        if (m >= rows || n0 + f >= n) continue;
         const auto total = [&](int t, int c) {
             float s = 0.f;
 #pragma unroll
             for (int w = 0; w < NW; ++w) s += red[t][w][m][c];
             return s;
         };
-        T* out = reinterpret_cast<T*>(p.out[mat]) + (int64_t)m * p.ldo[mat] + n0 + f;
+        T* out = reinterpret_cast<T*>(mx.out) + (int64_t)m * mx.ldo + n0 + f;
         if constexpr (GLU) {
             // both products are rounded as separate launches would store them
             const float a = (float)(T)total(0, f), g = (float)(T)total(1, f);
             *out = (T)((a * (1.0f / (1.0f + __expf(-a)))) * g);
         } else {
             float v = total(f / 16, f % 16);
-            if (p.bias[mat] != nullptr) v += (float)reinterpret_cast<const T*>(p.bias[mat])[n0 + f];
-            if (p.add[mat] != nullptr) v = (float)(T)v + (float)reinterpret_cast<const T*>(p.add[mat])[(int64_t)m * p.ldadd[mat] + n0 + f];
+            if (mx.bias != nullptr) v += (float)bias[i];
+            if (mx.add != nullptr) v = (float)(T)v + (float)add[i];
             *out = (T)v;
         }
     }
@@ -187,8 +234,7 @@ template <typename T> int launch(const mi_rows_args& a, hipStream_t st) {
     p.n_weights = a.n_weights; p.rows = a.rows; p.k = a.k; p.eps = a.eps;
     int64_t blocks16 = 0;
     for (int i = 0; i < a.n_weights; ++i) {
-        p.w[i] = a.w[i]; p.bias[i] = a.bias[i]; p.add[i] = a.add[i]; p.out[i] = a.out[i];
-        p.ldw[i] = a.ldw[i]; p.ldadd[i] = a.ldadd[i]; p.ldo[i] = a.ldo[i]; p.n[i] = a.n[i];
+        p.m[i] = Matrix{a.w[i], a.bias[i], a.add[i], a.out[i], a.ldw[i], a.ldadd[i], a.ldo[i], a.n[i], 0};
         if (i == 0 || !a.glu) blocks16 += (a.n[i] + 15) / 16;
     }
     // Two blocks per workgroup once that leaves four workgroups per compute unit: the rows are read half as often.  Eight wavefronts
@@ -197,7 +243,7 @@ template <typename T> int launch(const mi_rows_args& a, hipStream_t st) {
     const int features = wide ? 32 : 16;
     int64_t grid = 0;
     for (int i = 0; i < (a.glu ? 1 : a.n_weights); ++i) {
-        p.first_tile[i] = (int)grid;
+        p.m[i].first_tile = (int)grid;
         grid += (a.n[i] + features - 1) / features;
     }
     if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "rows: too many features");
