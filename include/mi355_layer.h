@@ -214,6 +214,8 @@ int mi_cross_entropy(const void* logits, const int64_t* targets, const float* ro
  * kernel.  `lse` as above. */
 int mi_cross_entropy_padded(void* logits, const int64_t* targets, const float* row_scale, float* losses, float* lse, int32_t* argmax,
                             int64_t n_rows, int64_t vocab, int64_t row_stride, int dtype, void* stream);
+/* index[r] = first index of the maximum of row r, in torch.argmax's order (NaN above everything, -0 and +0 equal). */
+int mi_argmax(const void* x, int64_t n_rows, int64_t vocab, int64_t row_stride, int64_t* index, int dtype, void* stream);
 /* The weighted mean of cross_entropy.py:30 and the accuracy of :81-86 in one launch:
  *   loss = sum(losses * weights) / sum(weights),  total = sum(weights),
  *   accuracy = share of the rows with weights > 0 whose argmax is the target

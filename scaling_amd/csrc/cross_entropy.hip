@@ -472,6 +472,76 @@ __global__ __launch_bounds__(BLOCK) void ce_fwd_kernel(const CeArgs a) {
     }
 }
 
+// First index of the maximum of a row (greedy decoding).  Rows are few and latency is all there is to it, so a workgroup of 1024 takes a
+// row with eight vectors in flight per thread: 3 x 32000 bf16 5.1 us, torch's reduction 14.  Elements are compared as integers of the
+// same order, in which -0 is +0 and NaN above everything, as torch.argmax has it.
+constexpr int kArgDepth = 8;
+
+template <typename T> __device__ __forceinline__ uint32_t order_key(uint32_t bits) {
+    constexpr int W = 8 * sizeof(T);
+    constexpr uint32_t kSign = 1u << (W - 1), kMask = kSign | (kSign - 1);
+    constexpr uint32_t kInf = std::is_same_v<T, float> ? 0x7f800000u : std::is_same_v<T, _Float16> ? 0x7c00u : 0x7f80u;
+    const uint32_t magnitude = bits & (kSign - 1);
+    if (magnitude > kInf) return 0xffffffffu;
+    return (bits & kSign) != 0 && magnitude != 0 ? ~bits & kMask : magnitude | kSign;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kCeBlock) void argmax_kernel(const void* rows, int64_t stride, int vocab, int64_t* out) {
+    constexpr int V = Elem<T>::kVec;
+    __shared__ uint64_t lds[kCeWaves];
+    const T* x = reinterpret_cast<const T*>(rows) + (int64_t)blockIdx.x * stride;
+    const RowSplit rs = split_row<T>(x, vocab);
+    const uint4* xr = reinterpret_cast<const uint4*>(x + rs.head);
+    const auto element = [](const uint4& u, int i) {
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+        return sizeof(T) == 4 ? w[i] : (w[i >> 1] >> (16 * (i & 1))) & 0xffffu;
+    };
+    uint32_t best_key = 0;                                 // of the whole vectors, in ascending order
+    int best_index = 0x7fffffff;
+    for (int v0 = threadIdx.x; v0 < rs.vecs; v0 += kArgDepth * kCeBlock) {
+        uint4 buf[kArgDepth];
+#pragma unroll
+        for (int d = 0; d < kArgDepth; ++d) buf[d] = xr[min(v0 + d * kCeBlock, rs.vecs - 1)];
+#pragma unroll
+        for (int d = 0; d < kArgDepth; ++d) {
+            const int v = v0 + d * kCeBlock;
+            if (v >= rs.vecs) break;
+            uint32_t top = 0;
+#pragma unroll
+            for (int i = 0; i < V; ++i) top = max(top, order_key<T>(element(buf[d], i)));
+            if (top > best_key) {                          // rare after the first vectors
+                best_key = top;
+                best_index = rs.head + v * V;
+#pragma unroll
+                for (int i = V - 1; i >= 0; --i)
+                    if (order_key<T>(element(buf[d], i)) == top) best_index = rs.head + v * V + i;
+            }
+        }
+    }
+    // key, then the complement of the index: the first one of equals is the largest
+    uint64_t best = (uint64_t)best_key << 32 | (uint32_t)~best_index;
+    const int sc = rs.scalar_index(threadIdx.x);
+    if (sc >= 0) {
+        uint32_t bits = 0;
+        __builtin_memcpy(&bits, x + sc, sizeof(T));
+        const uint64_t other = (uint64_t)order_key<T>(bits) << 32 | (uint32_t)~sc;
+        best = other > best ? other : best;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const uint64_t other = __shfl_xor((unsigned long long)best, off, MI_WAVE);
+        best = other > best ? other : best;
+    }
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < kCeWaves; ++w) best = lds[w] > best ? lds[w] : best;
+        out[blockIdx.x] = (int64_t)(int32_t)~(uint32_t)best;
+    }
+}
+
 // Any vocabulary size, stride and alignment: three passes over the row with scalar accesses.
 template <typename T>
 __global__ __launch_bounds__(kCeBlock) void ce_stream_kernel(const CeArgs a) {
@@ -809,3 +879,13 @@ int mi_scale_inplace(void* x, int64_t n_elem, const float* scale, int dtype, voi
 }
 
 }  // extern "C"
+
+extern "C" int mi_argmax(const void* x, int64_t n_rows, int64_t vocab, int64_t row_stride, int64_t* index, int dtype, void* stream) {
+    if (n_rows == 0) return MI_OK;
+    if (!x || !index) return mi_fail(MI_E_NULL, "argmax: null pointer");
+    if (n_rows < 0 || n_rows > 0x7fffffffLL || vocab < 1 || vocab > 0x7fffffffLL - kArgDepth * kCeBlock || row_stride < 0)
+        return mi_fail(MI_E_SHAPE, "argmax: bad shape");
+    const dim3 grid((unsigned)n_rows), block(kCeBlock);
+    MI_DISPATCH_DTYPE(dtype, (argmax_kernel<T><<<grid, block, 0, (hipStream_t)stream>>>(x, row_stride, (int)vocab, index)));
+    return mi_check_launch("argmax");
+}

@@ -1084,6 +1084,18 @@ OptTensor op_norm_linear_rows(const Tensor& x, const Tensor& norm, double eps, c
     return out;
 }
 
+// Index of the maximum of each row of x [rows, n]; nothing where mi_argmax does not apply or a transform has to see the operation.
+OptTensor op_argmax_rows(const Tensor& x) {
+    if (transforming() || transformed(x) || !x.is_cuda() || x.dim() != 2 || x.size(0) < 1 || x.size(1) < 1 || x.size(1) > (1 << 30) ||
+        (x.size(1) > 1 && x.stride(1) != 1) || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat))
+        return std::nullopt;
+    need_gpu(x);
+    Launch l(x);
+    const Tensor out = at::empty({x.size(0)}, x.options().dtype(at::kLong));
+    check(mi_argmax(ptr(x), x.size(0), x.size(1), x.stride(0), out.data_ptr<int64_t>(), code_of(x), l.stream), "mi_argmax");
+    return out;
+}
+
 // One token per sequence through a pre-norm layer (RMSNorm, separate q / k / v, SwiGLU, no biases): five launches, plus the merge of
 // the decode attention and the norms in front of wide products.  x [batch, 1, hidden]; raises ctx_len by one and appends to the caches.  Nothing happens, and nothing
 // is returned, where a shape, type or alignment does not suit the kernels.
@@ -1178,5 +1190,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("linear_cross_entropy", &op_linear_cross_entropy);
     def("decode_attention", &op_decode_attention);
     def("norm_linear_rows", &op_norm_linear_rows);
+    def("argmax_rows", &op_argmax_rows);
     def("decode_layer", &op_decode_layer);
 }

@@ -541,6 +541,12 @@ def norm_linear_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, wei
     return _lib.host().norm_linear_rows(x, norm_weight, eps, weight)
 
 
+def argmax_rows(x: torch.Tensor) -> torch.Tensor:
+    """torch.argmax(x, dim=-1) of x [rows, n]."""
+    index = None if _taken_over((x,)) or not x.is_cuda else _lib.host().argmax_rows(x)
+    return torch.argmax(x, dim=-1) if index is None else index
+
+
 def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, tables,
                            softmax_scale, workspace, dtype) -> Optional[tuple]:
     """What `decode_layer` takes beside the token: the layer's weights, its caches and rotary tables.  None for weights that have to see

@@ -128,3 +128,21 @@ def test_native_decode_step_equals_the_modules(batch, heads, kv, dtype):
             assert float((x.float() - y.float()).norm() / x.float().norm()) < tol
     short, _ = model.generate(6, ids[:1], stop_tokens=[tokens[0][2]])
     assert short[0] == tokens[0][:tokens[0].index(tokens[0][2]) + 1]
+
+
+# one vector, less than a wavefront, both sides of a round of 1024 threads x 8 vectors, rows off a 16-byte boundary
+@pytest.mark.parametrize("rows,n,offset", [(1, 1, 0), (3, 7, 1), (4, 1000, 3), (16, 32000, 0), (5, 65537, 2), (2, 131072 + 9, 0), (300, 515, 5)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_argmax_of_rows(rows, n, offset, dtype):
+    print(f"case argmax rows={rows} n={n} offset={offset} dtype={dtype}", flush=True)
+    x = _rand((rows * (n + offset) + offset,), dtype, n)[offset:].view(rows, n + offset)[:, :n]
+    cases = [x, x.clone().clamp_(max=0.0), torch.full_like(x, -float("inf")), -torch.zeros_like(x)]     # ties from clamping, at -inf and at -0
+    if n > 8:
+        at = torch.randint(0, n, (rows, 2), generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+        cases += [x.scatter(1, at, float("inf")), x.scatter(1, at, float("nan")), cases[3].scatter(1, at, 0.0)]
+    for i, c in enumerate(cases):
+        ref = torch.argmax(c.float().cpu(), dim=-1)
+        if i == 6:
+            assert ref.tolist() == [0] * rows              # -0 and +0 are equal
+        assert torch.equal(ops.argmax_rows(c).cpu(), ref), i
+    assert ops.argmax_rows(x[:0]).numel() == 0
