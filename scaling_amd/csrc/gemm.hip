@@ -315,14 +315,7 @@ bool wide(const mi_gemm_problem* in, int count, int dtype) {
 int launch_wide(const mi_gemm_problem* in, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
     if (workspace == nullptr || !mi_aligned16(workspace)) workspace_bytes = 0;
     const MiGemmPlan plan = mi_gemm_wide_plan(in, count, workspace_bytes, mi_compute_units());
-    const int rc = mi_gemm_wide(in, count, dtype, plan, workspace, st);
-    if (rc != MI_OK) return rc;
-    for (int i = 0; i < count; ++i) {
-        if (in[i].p_sum == nullptr || in[i].m == 0) continue;
-        const auto& g = in[i].segments[0];
-        if (const int e = mi_column_sum(g.p, g.ldp, g.k, in[i].m, in[i].p_sum, dtype, st); e != MI_OK) return e;
-    }
-    return MI_OK;
+    return mi_gemm_wide(in, count, dtype, plan, workspace, st);
 }
 
 template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {

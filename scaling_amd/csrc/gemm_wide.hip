@@ -43,9 +43,10 @@ struct Problem {
     void* c; const void* bias; const void* add;
     int64_t ldc, ldadd;
     float* part;                                           // splits > 1: fp32 partial results [splits][tiles_m * tile][tiles_n * tile]
-    int n_seg, p_kmajor, q_kmajor, m, n, tiles_m, tiles_n, first_block, splits;
+    void* p_sum;                                           // column sums of a contraction-major P
+    int n_seg, p_kmajor, q_kmajor, m, n, tiles_m, tiles_n, first_block, splits, sum_blocks;
 };
-struct Problems { Problem p[MI_GEMM_MAX_PROBLEMS]; int count; };
+struct Problems { Problem p[MI_GEMM_MAX_PROBLEMS]; int count, first_sum; };
 
 #define PIN() __builtin_amdgcn_sched_barrier(0)
 
@@ -453,12 +454,62 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
     store_quadrant<T>(pr, smem + wave * kBlockBytes, m0 + wm * 64, n0 + wn * 64, lane);
 }
 
+// Bias gradients: sums over the rows of P, 64 columns per workgroup, behind the blocks of the products, where they run on compute units that
+// the last round leaves idle and find most of P in the caches.  A launch of its own for each took 11 - 13 us at 4084 rows of 1024 .. 4096,
+// with 16 .. 64 workgroups; here that is the cost only where the blocks are whole rounds (4084 x 4096 -> 1024, 75.7 -> 86.7 us), and nothing
+// elsewhere (1024 -> 4096 86.6 -> 84.5, 1024 -> 3072 64.5 -> 64.6, 1024 -> 1024 35.2 -> 34.8).
+constexpr int kSumColumns = 64;
+template <typename T> __device__ __forceinline__ void sum_columns(const Problem& pr, int block, char* smem) {
+    constexpr int V = 8, GROUPS = kThreads / 8, DEPTH = 8;
+    const int lane = threadIdx.x & 63, u = threadIdx.x & 7, rows = pr.seg[0].k, col = block * kSumColumns + u * V;
+    const int64_t ld = pr.seg[0].ldp;
+    const T* base = (const T*)pr.seg[0].p + (col < pr.m ? col : 0);   // m is a whole number of vectors
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    const auto add = [&](const uint4& v) {
+        float f[V];
+        Elem<T>::unpack(v, f);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] += f[i];
+    };
+    int r = threadIdx.x >> 3;
+    for (; r + (DEPTH - 1) * GROUPS < rows; r += DEPTH * GROUPS) {
+        uint4 v[DEPTH];
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) v[d] = *reinterpret_cast<const uint4*>(base + (int64_t)(r + d * GROUPS) * ld);
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) add(v[d]);
+    }
+    for (; r < rows; r += GROUPS) add(*reinterpret_cast<const uint4*>(base + (int64_t)r * ld));
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        acc[i] += __shfl_xor(acc[i], 8, MI_WAVE);
+        acc[i] += __shfl_xor(acc[i], 16, MI_WAVE);
+        acc[i] += __shfl_xor(acc[i], 32, MI_WAVE);
+    }
+    float* part = reinterpret_cast<float*>(smem);          // [wavefront][column]
+    if (lane < 8) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) part[(threadIdx.x >> 6) * kSumColumns + u * V + i] = acc[i];
+    }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c < kSumColumns && block * kSumColumns + c < pr.m)
+        Elem<T>::store1((T*)pr.p_sum + block * kSumColumns + c, (part[c] + part[kSumColumns + c]) + (part[2 * kSumColumns + c] + part[3 * kSumColumns + c]));
+}
+
 // Blocks of a problem are handed to the XCDs (workgroups modulo 8) in contiguous runs, in groups of four block rows, so that the workgroups
 // that share an L2 read the same rows and columns at the same time.
 template <typename T, int TILE>
 __global__ __launch_bounds__(kThreads, 1) void wide_kernel(const Problems ps) {
     __shared__ __attribute__((aligned(1024))) char smem[2 * kQBase];
     int i = 0;
+    if ((int)blockIdx.x >= ps.first_sum) {
+        int b = blockIdx.x - ps.first_sum;
+        while (b >= ps.p[i].sum_blocks) b -= ps.p[i++].sum_blocks;
+        return sum_columns<T>(ps.p[i], b, smem);
+    }
     while (i + 1 < ps.count && (int)blockIdx.x >= ps.p[i + 1].first_block) ++i;
     const Problem& pr = ps.p[i];
     const int tiles = pr.tiles_m * pr.tiles_n, total = tiles * pr.splits;
@@ -575,10 +626,14 @@ int mi_gemm_wide(const mi_gemm_problem* in, int count, int dtype, const MiGemmPl
         p.tiles_n = (a.n + tile - 1) / tile;
         p.splits = plan.splits;
         p.part = (float*)workspace;
+        p.p_sum = a.p_sum;
+        p.sum_blocks = a.p_sum != nullptr ? (a.m + kSumColumns - 1) / kSumColumns : 0;
         p.first_block = (int)total;
         total += ((int64_t)p.tiles_m * p.tiles_n * p.splits + 7) / 8 * 8;
         if (total > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "gemm: too many tiles");
     }
+    ps.first_sum = (int)total;
+    for (int i = 0; i < count; ++i) total += ps.p[i].sum_blocks;
     if (total == 0) return MI_OK;
     const dim3 grid((unsigned)total), block(kThreads);
     const Problem& p0 = ps.p[0];
