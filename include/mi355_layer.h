@@ -390,6 +390,10 @@ size_t mi_attn_bwd_workspace_bytes(int64_t total_q, int32_t n_q_heads, int32_t h
  * mi_attn_bwd_workspace_bytes() for 8 or more KV heads. */
 size_t mi_attn_bwd_workspace_bytes_kv(int64_t total_q, int64_t total_k, int32_t n_q_heads, int32_t n_kv_heads,
                                       int32_t head_dim);
+/* Workspace with which the backward of this call is fastest, for calls of all its stages.  float32 at head_dim 64 and more, large enough to
+ * fill the chip: with this much the dK/dV kernel leaves dS in the workspace (at most 1.25 GiB, a number of KV heads at a time) and the dQ
+ * kernel has one product to do instead of three; the same bits.  Otherwise mi_attn_bwd_workspace_bytes_kv(). */
+size_t mi_attn_bwd_workspace_bytes_for(const mi_attn_args* args);
 int mi_attn_bwd(const mi_attn_bwd_args* args);
 
 /* ------------------------------------------------------------------------------------------

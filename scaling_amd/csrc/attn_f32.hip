@@ -22,7 +22,9 @@
 //     with F32Tile::f(row), which spreads the 16 rows that one pass of a 128-bit read touches over all banks.
 // One wavefront per workgroup with synchronous staging, the earlier form of these kernels, kept three of the four SIMDs
 // of a compute unit busy at most and each of them waiting for its own loads: 19.1 ms for a forward + backward at 32 / 8
-// heads of 128 and 4096 causal tokens (25 TFLOP/s), now 5.3 ms (91 TFLOP/s; forward 1.18, dK/dV 2.49, dQ 1.71 ms).
+// heads of 128 and 4096 causal tokens (25 TFLOP/s).  With the backward as dK/dV and a dQ kernel that forms S and dP again 5.3 ms (forward
+// 1.14, dK/dV 2.62, dQ 1.80); where the products are a sixteenth of the 16-bit rate a byte of memory costs a sixteenth as much beside
+// them, so dK/dV leaves dS in a workspace and dQ reads it: 4.25 ms, 113 TFLOP/s (dK/dV 2.75, dQ 0.62).
 #include "attn_common.h"
 
 namespace {
@@ -41,6 +43,31 @@ struct F32Params {
     const float* q; const float* k; const float* v; float* o; float* lse;
     const float* d_o; float* dq; float* dk; float* dv; float* delta;
     AttnParams m;     // masks, sizes, strides (the pointer members of m are not used)
+    // backward, all of it in one call with room for dS: the dK/dV kernel leaves dS there and the dQ kernel reads it, for the KV heads
+    // kv0 .. kv0 + kv_count - 1 at a time
+    float* ds;
+    int kv0, kv_count;
+    bool ds_triangle;
+};
+
+// Where dS lies: tiles of 32 keys x 32 queries, [query head of the present KV heads][tile], each key's 32 queries contiguous.  Under a
+// causal mask with the same documents on both axes no tile has its keys behind its queries, and the tiles form a triangle.
+constexpr int kDsTile = 32 * 32;
+inline bool ds_triangle(const mi_attn_args* a) {
+    return a->causal && (a->cu_seqlens_k == nullptr || a->cu_seqlens_k == a->cu_seqlens_q) && a->total_q == a->total_k;
+}
+struct DsLayout {
+    int64_t per_head;
+    int k_tiles;                                           // 0: triangle
+    __host__ __device__ DsLayout(int total_q, int total_k, bool triangle) {
+        const int64_t nq = ((int64_t)total_q + 31) / 32, nk = ((int64_t)total_k + 31) / 32;
+        per_head = triangle ? nq * (nq + 1) / 2 : nq * nk;
+        k_tiles = triangle ? 0 : (int)nk;
+    }
+    __device__ __forceinline__ int64_t tile(int head, int q, int k) const {    // q, k: first token of the tile
+        const int64_t i = q >> 5, j = k >> 5;
+        return (head * per_head + (k_tiles == 0 ? i * (i + 1) / 2 : i * k_tiles) + j) * kDsTile;
+    }
 };
 
 // ---- LDS tile of D floats per row ------------------------------------------------------------------------------------
@@ -381,7 +408,7 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(const F32Params fp)
 // ---- dK / dV: KGRP groups of 32 keys of one KV head (K, V rows in registers), 4 / KGRP wavefronts per group that take
 // different 32-query tiles of a step; loops over the group's query heads and over the query steps: S = Q K^T, dP = dO V^T
 // (lane = key), dV^T += dO^T P, dK^T += Q^T dS.  One wavefront per SIMD: K, V and both accumulators take 256 registers. ----
-template <int D, int KGRP>
+template <int D, int KGRP, bool KEEP>
 __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const F32Params fp) {
     constexpr int DT = D / 32, QS = kF32Waves / KGRP, BQ = 32 * QS, BK = 32 * KGRP;
     constexpr int NS = n_stages<D, BQ>(), TILE = BQ * 4 * D;
@@ -395,8 +422,9 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
     const int nkb = (p.total_k + BK - 1) / BK;
     // (KV head, split of its query heads) groups; the workgroup takes query heads kvh * n_rep + hs * hpw .. + hpw
     int group, rank;
-    head_and_rank(blockIdx.x, p.nkv * p.hsplit, group, rank);
-    const int kvh = group / p.hsplit, hs = group - kvh * p.hsplit, hpw = p.n_rep / p.hsplit;
+    head_and_rank(blockIdx.x, (KEEP ? fp.kv_count : p.nkv) * p.hsplit, group, rank);
+    const int first_kv = KEEP ? fp.kv0 : 0;
+    const int kvh = first_kv + group / p.hsplit, hs = group - (kvh - first_kv) * p.hsplit, hpw = p.n_rep / p.hsplit;
     const int kb = block_for_rank(rank, nkb, p.n_docs, 0, false);
     const int key = kb * BK + kgrp * 32 + l32;
     int qlo, qhi;
@@ -441,14 +469,15 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
 #pragma unroll
         for (int r = 0; r < 16; ++r) { dk_acc[dt][r] = 0.f; dv_acc[dt][r] = 0.f; }
     const float c2 = p.scale_log2;
-    int tile = 0;
+    const DsLayout ds(p.total_q, p.total_k, fp.ds_triangle);
+    int tile = 0, rep = 0;
     for (int step = 0; step < n_steps; ++step) {
         put_stat(step);
         wait_vmcnt<0>();
         __syncthreads();                  // the step has landed, and the readers of the one before are done
         if constexpr (NS == 2) issue();
-        const int qt = qt0 + tile * BQ + 32 * qs;
-        if (++tile == n_tiles) tile = 0;
+        const int qt = qt0 + tile * BQ + 32 * qs, head = kvh * p.n_rep + hs * hpw + rep;
+        if (++tile == n_tiles) { tile = 0; ++rep; }
         if (qt < wmax && qt + 32 > wmin) {
             const char* q_s = smem + (step % NS) * 2 * TILE;
             const char* do_s = q_s + TILE;
@@ -470,6 +499,11 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
                     s[r] = pv;
                     dp[r] = pv * (dp[r] - d4[c]);
                 }
+            }
+            if constexpr (KEEP) {
+                float* out = fp.ds + ds.tile(head - first_kv * p.n_rep, qt, kb * BK + kgrp * 32) + l32 * 32 + 4 * g;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) *reinterpret_cast<f32x4_t*>(out + 8 * a) = f32x4_t{dp[4 * a], dp[4 * a + 1], dp[4 * a + 2], dp[4 * a + 3]};
             }
             cols_product<D>(dv_acc, do_s, 32 * qs, s, l32, g);
             cols_product<D>(dk_acc, q_s, 32 * qs, dp, l32, g);
@@ -594,6 +628,77 @@ __global__ __launch_bounds__(64 * kF32Waves, D == 128 ? 1 : 2) void attn_f32_dq_
     sum_and_store<D, KG>(dq_acc, slot, kg, lane, g, fp.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh, tq < p.total_q, p.scale);
 }
 
+// ---- dQ from the dS that the dK/dV kernel left: one product instead of three.  The key tiles of a step as above, the dS of the next one in
+// registers: lane = query, one 128-byte line per key and half.  What no query may see was not written, or not by this call, and counts as zero. ----
+template <int D, int QG>
+__global__ __launch_bounds__(64 * kF32Waves, 2) void attn_f32_dq_kept_kernel(const F32Params fp) {
+    constexpr int DT = D / 32, KG = kF32Waves / QG, BN = 32 * KG, BM = 32 * QG;
+    constexpr int NS = 2, TILE = BN * 4 * D;
+    __shared__ __attribute__((aligned(1024))) char smem[NS * TILE];
+    __shared__ int range_lds[2 * kF32Waves];
+    const AttnParams& p = fp.m;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qg = wave % QG, kg = wave / QG;
+    const int nqb = (p.total_q + BM - 1) / BM;
+    int head, rank;
+    head_and_rank(blockIdx.x, fp.kv_count * p.n_rep, head, rank);
+    const int qb = block_for_rank(rank, nqb, p.n_docs, 0, true);
+    const int kvh = fp.kv0 + head / p.n_rep;
+    const int q0 = qb * BM + qg * 32, tq = q0 + l32;
+    int klo, khi;
+    key_range(p, tq, klo, khi);
+    const int wmin = __builtin_amdgcn_readfirstlane(group_min<64>(khi > klo ? klo : 0x7fffffff));
+    const int wmax = __builtin_amdgcn_readfirstlane(group_max<64>(khi > klo ? khi : 0));
+    int bmin, bmax;
+    block_range(wmin, wmax, wave, lane, range_lds, bmin, bmax);
+    const int kt0 = bmin & ~31, n_steps = (bmax - kt0 + BN - 1) / BN;
+    const float* kbase = fp.k + (int64_t)kvh * p.k_sh;
+    F32Dma<D, BN> k_dma;
+    k_dma.init(wave, lane, p.k_st);
+    const float* ds = fp.ds + DsLayout(p.total_q, p.total_k, fp.ds_triangle).tile(head, q0, 0) + l32;
+    f32x16_t next;
+    auto issue = [&](int t) {
+        if (t >= n_steps) return;
+        const int kt = kt0 + t * BN + 32 * kg;
+        if (kt < wmax && kt + 32 > wmin) {
+            const float* from = ds + (int64_t)(kt >> 5) * kDsTile;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) next[r] = from[acc_row(r, g) * 32];
+        }
+        k_dma.issue(kbase, p.k_st, kt0 + t * BN, p.total_k - 1, smem + (t % NS) * TILE);
+    };
+#pragma unroll
+    for (int r = 0; r < 16; ++r) next[r] = 0.f;
+    issue(0);
+    f32x16_t dq_acc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dq_acc[dt][r] = 0.f;
+    for (int t = 0; t < n_steps; ++t) {
+        wait_vmcnt<0>();
+        f32x16_t x = next;
+        asm volatile("" : "+v"(x));           // arrived: the loads below are not waited for
+        __syncthreads();
+        issue(t + 1);
+        const int kt = kt0 + t * BN + 32 * kg;
+        if (kt < wmax && kt + 32 > wmin) {
+            if (__any(kt < klo || kt + 32 > khi)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = kt + acc_row(r, g);
+                    if (key < klo || key >= khi) x[r] = 0.f;
+                }
+            }
+            cols_product<D>(dq_acc, smem + (t % NS) * TILE, 32 * kg, x, l32, g);
+        }
+    }
+    float* slot = reinterpret_cast<float*>(smem) + (size_t)qg * KG * DT * 16 * 64;
+    static_assert(QG * KG * DT * 16 * 64 * 4 <= NS * TILE || KG == 1, "the exchange reuses the tile stages");
+    sum_and_store<D, KG>(dq_acc, slot, kg, lane, g, fp.dq + (int64_t)tq * p.q_st + (int64_t)(fp.kv0 * p.n_rep + head) * p.q_sh, tq < p.total_q, p.scale);
+}
+
 int validate_f32(const mi_attn_args* a, const char* who) {
     int rc = mi_attn_validate(a, who, MI_F32, 4);
     if (rc != MI_OK) return rc;
@@ -643,6 +748,57 @@ int mi_attn_fwd_impl_f32(const mi_attn_args* a) {
     }
 }
 
+// Backward with dS kept: five products instead of seven, the same bits.  Bytes of dS are bounded; what does not fit at once goes a number of
+// KV heads at a time, each of them two workgroups per compute unit.  us, recomputed / kept (query heads / KV heads, head_dim, causal unless said):
+//   32/32  64  1101 tokens  258 / 191     32/32 128  1101  443 / 336     12/12 128  14 x 300  334 / 252     16/16 128  8192  8199 / 6628 (2 passes)
+//   16/16  64  8192        4310 / 3658    32/8  128  4096 4221 / 3167    32/32  64  64 x 64   167 / 131     32/32  64  1100, not causal  489 / 361
+// At head_dim 32 the products that are saved take less time than the bytes.
+static constexpr int64_t kDsBytes = (int64_t)5 << 28;             // 1.25 GiB
+
+// KV heads per pass, 0: not at all
+static int ds_heads(const mi_attn_args* a) {
+    if (a->head_dim < 64 || a->total_q <= 0 || a->total_k <= 0 || a->n_kv_heads <= 0 || a->n_q_heads % a->n_kv_heads != 0 || a->total_q > 0x7fffff00LL ||
+        a->total_k > 0x7fffff00LL)
+        return 0;
+    const DsLayout l((int)a->total_q, (int)a->total_k, ds_triangle(a));
+    const int64_t each = l.per_head * kDsTile * (int64_t)sizeof(float) * (a->n_q_heads / a->n_kv_heads), fit = kDsBytes / each;
+    if (fit < 1) return 0;
+    const int passes = (int)((a->n_kv_heads + fit - 1) / fit), heads = (a->n_kv_heads + passes - 1) / passes;
+    const int64_t blocks = (a->total_k + 63) / 64 * heads * mi_dkdv_head_split(a->n_q_heads, a->n_kv_heads);
+    return blocks >= 2 * mi_compute_units() ? heads : 0;
+}
+
+template <int D> static int launch_reduce_f32(const F32Params& fp, hipStream_t st) {
+    const AttnParams& p = fp.m;
+    if (p.hsplit == 1) return MI_OK;
+    const int64_t n = (int64_t)p.total_k * p.nkv * (D / 4);
+    attn_f32_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(fp);
+    return mi_check_launch("attn_bwd_dkdv_reduce (f32)");
+}
+
+template <int D> static int launch_kept_f32(const F32Params& all, hipStream_t st) {
+    if constexpr (D < 64) return mi_fail(MI_E_SHAPE, "attn_bwd: dS is not kept at head_dim %d", D);
+    else {
+        F32Params fp = all;
+        const AttnParams& p = fp.m;
+        const dim3 block(64 * kF32Waves);
+        const int step = all.kv_count;
+        for (fp.kv0 = 0; fp.kv0 < p.nkv; fp.kv0 += step) {
+            fp.kv_count = step < p.nkv - fp.kv0 ? step : p.nkv - fp.kv0;
+            const int64_t keys = (((int64_t)p.total_k + 63) / 64) * fp.kv_count * p.hsplit, heads = (int64_t)fp.kv_count * p.n_rep;
+            attn_f32_dkdv_kernel<D, 2, true><<<dim3((unsigned)keys), block, 0, st>>>(fp);
+            int rc = mi_check_launch("attn_bwd_dkdv (f32)");
+            if (rc != MI_OK) return rc;
+            const int64_t wide = (((int64_t)p.total_q + 127) / 128) * heads, narrow = (((int64_t)p.total_q + 31) / 32) * heads;
+            if (wide >= 2 * mi_compute_units()) attn_f32_dq_kept_kernel<D, 4><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+            else attn_f32_dq_kept_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
+            rc = mi_check_launch("attn_bwd_dq (f32)");
+            if (rc != MI_OK) return rc;
+        }
+        return launch_reduce_f32<D>(fp, st);
+    }
+}
+
 template <int D> static int launch_bwd_f32(const F32Params& fp, int flags, hipStream_t st) {
     const AttnParams& p = fp.m;
     const int stages = flags & (MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ);
@@ -659,18 +815,15 @@ template <int D> static int launch_bwd_f32(const F32Params& fp, int flags, hipSt
         // on, which a causal mask needs to pair long key blocks with short ones; below that, one key group whose four
         // wavefronts split the queries.  Measured (head_dim 128, two groups / one): 512 blocks of 64 keys 331 / 377 us,
         // 384 blocks 1751 / 1656 us, 256 blocks 1168 / 700 us
+        if (all && fp.ds != nullptr) return launch_kept_f32<D>(fp, st);
         const int64_t groups = (int64_t)p.nkv * p.hsplit;
         const int64_t wide = (((int64_t)p.total_k + 63) / 64) * groups, narrow = (((int64_t)p.total_k + 31) / 32) * groups;
-        if (wide >= 2 * mi_compute_units()) attn_f32_dkdv_kernel<D, 2><<<dim3((unsigned)wide), block, 0, st>>>(fp);
-        else attn_f32_dkdv_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
+        if (wide >= 2 * mi_compute_units()) attn_f32_dkdv_kernel<D, 2, false><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+        else attn_f32_dkdv_kernel<D, 1, false><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
         int rc = mi_check_launch("attn_bwd_dkdv (f32)");
         if (rc != MI_OK) return rc;
-        if (p.hsplit > 1) {
-            const int64_t n = (int64_t)p.total_k * p.nkv * (D / 4);
-            attn_f32_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(fp);
-            rc = mi_check_launch("attn_bwd_dkdv_reduce (f32)");
-            if (rc != MI_OK) return rc;
-        }
+        rc = launch_reduce_f32<D>(fp, st);
+        if (rc != MI_OK) return rc;
     }
     if (all || (stages & MI_ATTN_BWD_DQ)) {
         const int64_t wide = (((int64_t)p.total_q + 127) / 128) * p.nq, narrow = (((int64_t)p.total_q + 31) / 32) * p.nq;
@@ -680,6 +833,14 @@ template <int D> static int launch_bwd_f32(const F32Params& fp, int flags, hipSt
         return mi_check_launch("attn_bwd_dq (f32)");
     }
     return MI_OK;
+}
+
+size_t mi_attn_bwd_workspace_bytes_f32(const mi_attn_args* a) {
+    const int heads = ds_heads(a);
+    if (heads == 0) return 0;
+    const DsLayout l((int)a->total_q, (int)a->total_k, ds_triangle(a));
+    const size_t base = mi_attn_bwd_workspace_bytes_kv(a->total_q, a->total_k, a->n_q_heads, a->n_kv_heads, a->head_dim);
+    return (base + 255) / 256 * 256 + (size_t)l.per_head * kDsTile * sizeof(float) * heads * (a->n_q_heads / a->n_kv_heads);
 }
 
 int mi_attn_bwd_impl_f32(const mi_attn_bwd_args* b) {
@@ -706,6 +867,12 @@ int mi_attn_bwd_impl_f32(const mi_attn_bwd_args* b) {
     fp.m.dv_st = b->dv_stride_token; fp.m.dv_sh = b->dv_stride_head;
     fp.delta = (float*)b->workspace;
     mi_set_head_split(a, b, &fp.m);
+    const size_t kept = mi_attn_bwd_workspace_bytes_f32(a), base = mi_attn_bwd_workspace_bytes_kv(a->total_q, a->total_k, a->n_q_heads, a->n_kv_heads, a->head_dim);
+    if (kept > 0 && b->workspace_bytes >= kept) {
+        fp.ds = (float*)((char*)b->workspace + (base + 255) / 256 * 256);
+        fp.kv_count = ds_heads(a);
+        fp.ds_triangle = ds_triangle(a);
+    }
     hipStream_t st = (hipStream_t)a->stream;
     switch (a->head_dim) {
         case 32: return launch_bwd_f32<32>(fp, a->flags, st);

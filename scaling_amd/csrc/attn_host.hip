@@ -10,6 +10,7 @@ int mi_attn_bwd_impl_bf16(const mi_attn_bwd_args* b);
 int mi_attn_bwd_impl_f16(const mi_attn_bwd_args* b);
 int mi_attn_fwd_impl_f32(const mi_attn_args* a);
 int mi_attn_bwd_impl_f32(const mi_attn_bwd_args* b);
+size_t mi_attn_bwd_workspace_bytes_f32(const mi_attn_args* a);
 int mi_attn_decode_impl_bf16(const mi_decode_args* a, bool static_ws);
 int mi_attn_decode_impl_f16(const mi_decode_args* a, bool static_ws);
 
@@ -25,6 +26,12 @@ extern "C" int mi_attn_bwd(const mi_attn_bwd_args* b) {
     if (b->fwd.total_q == 0 && b->fwd.total_k == 0) return MI_OK;
     if (b->fwd.dtype == MI_F32) return mi_attn_bwd_impl_f32(b);
     return b->fwd.dtype == MI_F16 ? mi_attn_bwd_impl_f16(b) : mi_attn_bwd_impl_bf16(b);
+}
+
+extern "C" size_t mi_attn_bwd_workspace_bytes_for(const mi_attn_args* a) {
+    if (!a) return 0;
+    const size_t kept = a->dtype == MI_F32 ? mi_attn_bwd_workspace_bytes_f32(a) : 0;
+    return kept > 0 ? kept : mi_attn_bwd_workspace_bytes_kv(a->total_q, a->total_k, a->n_q_heads, a->n_kv_heads, a->head_dim);
 }
 
 extern "C" int mi_attn_decode(const mi_decode_args* a) {

@@ -694,9 +694,18 @@ void attn_backward(const Tensor& d_o_, const Tensor& q, const Tensor& k, const T
     TORCH_CHECK(dq.strides() == q.strides(), "attention backward: dq needs the layout of q");
     Tensor d_o = d_o_;
     if (d_o.strides() != o.strides()) d_o = at::empty_strided(o.sizes(), o.strides(), o.options()).copy_(d_o_);
-    if (!ws.defined()) ws = float_buffer(std::max<size_t>(16, mi_attn_bwd_workspace_bytes_kv(q.size(0), k.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2))), q);
     mi_attn_bwd_args b{};
     fill_args(b.fwd, q, k, v, o, lse, cu_q, cu_k, opts, l.stream);
+    if (!ws.defined()) {
+        const size_t least = std::max<size_t>(16, mi_attn_bwd_workspace_bytes_kv(q.size(0), k.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2)));
+        const size_t best = std::max(least, mi_attn_bwd_workspace_bytes_for(&b.fwd));
+        try {
+            ws = float_buffer(best, q);
+        } catch (const c10::OutOfMemoryError&) {           // does with less, as it did
+            if (best == least) throw;
+            ws = float_buffer(least, q);
+        }
+    }
     b.d_o = ptr(d_o); b.dq = ptr(dq); b.dk = ptr(dk); b.dv = ptr(dv);
     b.dk_stride_token = dk.stride(0); b.dk_stride_head = dk.stride(1);
     b.dv_stride_token = dv.stride(0); b.dv_stride_head = dv.stride(1);

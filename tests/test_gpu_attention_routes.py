@@ -114,3 +114,34 @@ def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
         # sums in another order: some element of so many rounds the other way
         assert torch.equal(o, o2) == (flags == fwd)
         assert all(torch.equal(x, y) == (flags == bwd) for x, y in zip((dq, dk, dv), grads))
+
+
+# float32 backward with dS kept by the dK/dV kernel (a workspace that has room for it) against the dQ kernel that recomputes it: the same
+# bits.  Triangle and whole plane, documents that end inside tiles, keys and queries of different lengths (rows that see nothing among
+# them), few KV heads, several passes over the heads (4128 tokens of 64 heads), each head_dim.
+@pytest.mark.parametrize("nq,nkv,d,causal,lens_q,lens_k", [
+    (32, 32, 128, True, [1101], None), (32, 32, 64, False, [500, 37, 590], None), (64, 32, 96, True, [33, 1, 700, 331], None),
+    (16, 16, 128, True, [1000, 1200, 3], [900, 1300, 2]), (16, 16, 64, False, [700, 900], [1500, 617]), (16, 1, 128, True, [4099], None),
+    (64, 64, 64, True, [4128], None),
+])
+def test_float32_backward_with_kept_scores(nq, nkv, d, causal, lens_q, lens_k):
+    print(f"case f32 kept nq={nq} nkv={nkv} d={d} causal={causal} q={lens_q} k={lens_k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(d + nq)
+    cu = lambda lens: torch.tensor([0] + lens, dtype=torch.int32, device="cuda").cumsum(0, dtype=torch.int32)
+    cu_q, cu_k = cu(lens_q), None if lens_k is None else cu(lens_k)
+    tq, tk = sum(lens_q), sum(lens_k or lens_q)
+    rand = lambda n, h: torch.randn(n, h, d, generator=g, device="cuda")
+    q, k, v, do = rand(tq, nq), rand(tk, nkv), rand(tk, nkv), rand(tq, nq)
+    o, lse = ops.attention_forward(q, k, v, cu_q, cu_k, causal)
+    from scaling_amd import _lib
+    least = _lib.load().mi_attn_bwd_workspace_bytes_kv(tq, tk, nq, nkv, d)
+    small = [torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty((least + 3) // 4, device="cuda")]
+    want = [t.clone() for t in ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, buffers=tuple(small))]
+    junk = torch.full((1 << 28,), float("nan"), device="cuda")   # what the kept scores are written into holds no zeros
+    del junk
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal)
+    assert torch.cuda.max_memory_allocated() - before > 4 * least + (32 << 20), "the kept route was not taken"
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        assert torch.equal(a, b), f"{name}: {(a - b).abs().max().item()}"
