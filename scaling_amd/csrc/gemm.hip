@@ -291,8 +291,8 @@ template <typename T> bool few_rows(const mi_gemm_problem* in, int count, mi_row
 
 // Calls of 16-bit types with a product of more than 3 GFLOP take the larger blocks of gemm_wide.hip: 1024 x 1024 x 1024 alone 9 us here and
 // 11.5 there, 4084 x 1024 x 1024 34 and 13.5.  What follows a ragged extent inside its last vector meets zeros there (rows of Q past the
-// contraction) or unstored results; rows must not overlap and a step of them has to be addressable in 31 bits.
-bool wide(const mi_gemm_problem* in, int count, int dtype) {
+// contraction) or unstored results (`ragged`: the entry point allows it); rows must not overlap and a step of them has to be addressable in 31 bits.
+bool wide(const mi_gemm_problem* in, int count, int dtype, bool ragged) {
     if (dtype != MI_BF16 && dtype != MI_F16) return false;
     bool large = false;
     for (int i = 0; i < count; ++i) {
@@ -304,7 +304,7 @@ bool wide(const mi_gemm_problem* in, int count, int dtype) {
             const auto& g = a.segments[s];
             const int ep = a.p_kmajor ? a.m : g.k, eq = a.q_kmajor ? a.n : g.k;
             if (!g.p || !g.q || g.k <= 0 || !mi_aligned16(g.p) || !mi_aligned16(g.q) || g.ldp % 8 || g.ldq % 8 || g.ldp < (ep + 7LL) / 8 * 8 ||
-                g.ldq < (eq + 7LL) / 8 * 8 || g.ldp >= (1 << 22) || g.ldq >= (1 << 22) || (!a.q_kmajor && g.k % 8))
+                g.ldq < (eq + 7LL) / 8 * 8 || g.ldp >= (1 << 22) || g.ldq >= (1 << 22) || (!a.q_kmajor && g.k % 8) || (!ragged && (a.n % 4 || ep % 8 || eq % 8)))
                 return false;
             large = large || 2.0 * a.m * (double)a.n * g.k > 3e9;
         }
@@ -484,16 +484,19 @@ extern "C" int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, 
 
 extern "C" int mi_gemm_with_workspace(const mi_gemm_problem* problems, int count, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
     if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
-    if (wide(problems, count, dtype)) return launch_wide(problems, count, dtype, workspace, workspace_bytes, (hipStream_t)stream);
+    if (wide(problems, count, dtype, true)) return launch_wide(problems, count, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
     return MI_OK;
 }
 
 extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
-    return mi_gemm_with_workspace(problems, count, dtype, nullptr, 0, stream);
+    if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
+    if (wide(problems, count, dtype, false)) return launch_wide(problems, count, dtype, nullptr, 0, (hipStream_t)stream);
+    MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
+    return MI_OK;
 }
 
 extern "C" size_t mi_gemm_workspace_bytes(const mi_gemm_problem* problems, int count, int dtype) {
-    if (!problems || count != 1 || problems[0].m <= 0 || problems[0].n <= 0 || problems[0].n_segments != 1 || !wide(problems, count, dtype)) return 0;
+    if (!problems || count != 1 || problems[0].m <= 0 || problems[0].n <= 0 || problems[0].n_segments != 1 || !wide(problems, count, dtype, true)) return 0;
     return mi_gemm_wide_plan(problems, count, (size_t)1 << 30, mi_compute_units()).workspace_bytes;
 }

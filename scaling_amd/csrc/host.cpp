@@ -359,11 +359,19 @@ bool small_product(const Tensor& t, int64_t m, int64_t n, int64_t k) {
 // and 24.5; 4096 -> 1024 38 and 24.5.
 bool long_chain(const Tensor& t, int64_t rows, int64_t k) { return k >= 3072 && (t.scalar_type() == at::kFloat || rows > MI_ROWS_MAX); }
 // Larger products of 16-bit types with whole vectors in every direction: blocks of 128 or 256 rows and columns in mi_gemm, all layouts at the rate
-// of the library's fastest.  us on the device, mi_gemm and library: 4084 x 1024 -> 4096 forward 32.6 / 29.0, input gradient 34.6 / 40.0,
+// of the library's fastest.  us on the device, mi_gemm and library: 4084 x 1024 -> 4096 forward 34.4 / 30.5, input gradient 34.6 / 40.0,
 // weight gradient 32.7 / 37.5; 1024 -> 1024 13.8 / 13.4, 13.7 / 15.0, 22.4 / 33.0; 8192 x 4096 -> 14336 649 / 618, 629 / 693, 660 / 827 (767 + 24
-// with x transposed first).  Forward products of 100 GFLOP and more stay on the library; fewer than 128 rows fill no block.
-bool wide_product(const Tensor& t, int64_t rows, int64_t n, int64_t k, bool forward) {
-    return t.scalar_type() != at::kFloat && rows >= 128 && n % 8 == 0 && k % 8 == 0 && !(forward && 2.0 * (double)rows * (double)n * (double)k >= 1e11);
+// with x transposed first).  Fewer than 128 rows fill no block.
+//   Training (forward and gradients, here and with the library): 2048 x 1024 -> 1024 33 / 78, 2048 x 4096 -> 4096 177 / 193, 301 x 4096 -> 14336
+// 188 / 227; forward products of 100 GFLOP and more stay on the library.
+//   Inference keeps the library where its own time exceeds what it costs the host, or nearly: issued one by one (on the device alone) 2048 x 1024 ->
+// 1024 12.2 / 19.7 (11.8 / 10.2), 1024 x 1024 -> 4096 13.7 / 19.9 (14.2 / 13.4), 2048 x 1024 -> 4096 26.5 / 21.8, 1024 x 2816 -> 1024 22.5 / 19.8 (22.5 /
+// 13.4), 513 x 2048 -> 2048 19.2 / 19.8 (19.7 / 12.3), 4084 x 2048 -> 2048 41 / 35, 301 x 4096 -> 14336 59 / 40.
+enum class Pass { kInference, kForward, kBackward };
+bool wide_product(const Tensor& t, int64_t rows, int64_t n, int64_t k, Pass pass) {
+    const double work = 2.0 * (double)rows * (double)n * (double)k;
+    if (pass == Pass::kInference ? k > 1536 || work > 1e10 : pass == Pass::kForward && work >= 1e11) return false;
+    return t.scalar_type() != at::kFloat && rows >= 128 && n % 8 == 0 && k % 8 == 0;
 }
 bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
@@ -452,7 +460,7 @@ struct Projections : Function<Projections> {
             const Tensor& w = params[i];
             fit = fit && aligned(w);
             small = small && small_product(x, rows, w.size(0), in);
-            wide = wide && wide_product(x, rows, w.size(0), in, true);
+            wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward);
         }
         // What the gradients read and no more, so that the rest may be changed or freed before the backward pass: x (itself: what is
         // differentiated again reaches it) for the weights, the weights for x.  The same for a recomputation inside a backward pass.
@@ -518,7 +526,7 @@ struct Projections : Function<Projections> {
             if (!again && !aligned(dy[i])) dy[i] = dy[i].contiguous();
             fit = fit && aligned(dy[i]);
             small = small && small_product(dy[i], rows, dy[i].size(1), in);
-            wide = wide && wide_product(dy[i], rows, dy[i].size(1), in, false);
+            wide = wide && wide_product(dy[i], rows, dy[i].size(1), in, Pass::kBackward);
             // the forward product may have been the library's, and saved-tensor hooks may bring the weight back in another layout
             if (need_dx) fit = fit && aligned(saved[1 + i]);
         }
@@ -910,7 +918,7 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
             const Tensor hc = h.narrow(0, r0, r);
             Tensor logits = buffer.narrow(0, 0, r).narrow(1, 0, vocab);
             // 2047 x 50257 x 1024, us, mi_gemm and library: logits 216 / 257, dh 161 / 291, dW 197 / 252
-            const bool wide = wide_product(h, r, 8, h.size(1), false) && 2.0 * (double)r * (double)vocab * (double)h.size(1) > 3e9 && aligned(hc) &&
+            const bool wide = wide_product(h, r, 8, h.size(1), Pass::kBackward) && 2.0 * (double)r * (double)vocab * (double)h.size(1) > 3e9 && aligned(hc) &&
                               aligned(weight);
             if (wide) {
                 mi_gemm_problem p = problem(logits, false, false);

@@ -8,7 +8,7 @@ import sys
 import pytest
 import torch
 
-from scaling_amd import ops
+from scaling_amd import _lib, ops
 from scaling_amd.nn import ParallelSwiGLUMLP
 
 pytestmark = pytest.mark.gpu
@@ -114,7 +114,7 @@ def test_capture_after_one_call():
     """A first call outside the capture makes whatever the captured one needs, in a process that has used no library product."""
     code = """
 import torch
-from scaling_amd import ops
+from scaling_amd import _lib, ops
 for k in (2048, 2816, 3064, 3072):
     x, w = torch.ones(17, k, device="cuda", dtype=torch.bfloat16), torch.full((64, k), 0.5, device="cuda", dtype=torch.bfloat16)
     side = torch.cuda.Stream()
@@ -377,3 +377,18 @@ def test_lm_head_products(rows, hidden, vocab):
     for name, a, b in (("dh", h.grad, hd.grad), ("dw", w.grad, wd.grad)):
         err = ((a.double() - b).norm() / b.norm()).item()
         assert err <= 2.0 ** -7, f"{name}: {err}"
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(512, 1024, 4101), (512, 4100, 1024)])
+def test_ragged_extents_need_the_entry_with_a_workspace(rows, ins, outs):
+    """mi_gemm takes whole vectors whatever the size of the product; the other entry takes any n of a large one, and no ragged contraction
+    between operands that are both contiguous along it."""
+    lib = _lib.load()
+    x, c = (torch.zeros(rows, 4104, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    w = torch.zeros(outs, 4104, dtype=torch.bfloat16, device=DEV)
+    p = _lib.MiGemmProblem(c=c.data_ptr(), ldc=4104, n_segments=1, m=rows, n=outs)
+    p.segments[0] = _lib.MiGemmSegment(x.data_ptr(), w.data_ptr(), 4104, 4104, ins)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.mi_gemm(p, 1, 0, stream) != 0
+    assert (lib.mi_gemm_with_workspace(p, 1, 0, None, 0, stream) == 0) == (ins % 8 == 0)
+    torch.cuda.synchronize()
