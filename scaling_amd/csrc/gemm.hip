@@ -315,7 +315,7 @@ bool wide(const mi_gemm_problem* in, int count, int dtype, bool ragged) {
 int launch_wide(const mi_gemm_problem* in, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
     if (workspace == nullptr || !mi_aligned16(workspace)) workspace_bytes = 0;
     const MiGemmPlan plan = mi_gemm_wide_plan(in, count, workspace_bytes, mi_compute_units());
-    return mi_gemm_wide(in, count, dtype, plan, workspace, st);
+    return mi_gemm_wide(in, count, dtype, plan, workspace, mi_compute_units(), st);
 }
 
 template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {

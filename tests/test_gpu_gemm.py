@@ -318,10 +318,11 @@ def test_batched_gradients(rows, ins, outs):
 
 
 # products over 3 GFLOP take blocks of 128 or 256: remainders in every direction, one segment and several problems, contractions that
-# are split over the chip (512 x 8200 -> 520, 264 x 16392 -> 520) and that end inside a step
+# are split over the chip (512 x 8200 -> 520, 264 x 16392 -> 520) and that end inside a step, launches of whole rounds with the rest behind
+# them, by rows (4097 x 520 -> 4104; weight gradient of 600 x 1040 -> 13320) and by columns (2047 x 520 -> 16904)
 @pytest.mark.parametrize("rows,ins,outs", [
     (1031, 1032, (1544,)), (2049, 1096, (1048, 264)), (513, 8200, (520,)), (264, 16392, (520,)), (129, 3080, (4104, 1032, 1032)),
-    (2050, 2056, (5640,)), (4097, 520, (4104,)),
+    (2050, 2056, (5640,)), (4097, 520, (4104,)), (2047, 520, (16904,)), (600, 1040, (13320,)),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_large_products_and_their_gradients(rows, ins, outs, dtype):
@@ -357,6 +358,17 @@ def test_large_product_with_residual_and_in_a_graph():
             graph.replay()
             (x.float() @ w.float().t()).sum().item()
             assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(2047, 520, 16904), (4097, 520, 4104)])
+def test_bias_and_residual_of_a_product_in_two_launches(rows, ins, outs):
+    g = torch.Generator().manual_seed(outs)
+    x, w, b, res = (torch.randn(*s, generator=g).bfloat16().to(DEV) for s in ((rows, ins), (outs, ins), (outs,), (rows, outs)))
+    with torch.no_grad():
+        y = ops.linear(x, w, b)
+        ref, magnitude = x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs()
+        _close("y", y, ref.cpu(), magnitude.cpu(), ins, torch.bfloat16)
+        assert torch.equal(ops.linear(x, w, b, res), y + res)
 
 
 @pytest.mark.parametrize("rows,hidden,vocab", [(2047, 1024, 50257), (300, 520, 20003), (1025, 2048, 128)])
