@@ -32,7 +32,7 @@ LEGACY_CLASS_NAMES = {"LuminousEmbeddingInput": "EmbeddingInput", "LuminousLayer
 
 def sample_argmax(logits: torch.Tensor) -> torch.Tensor:
     """transformer/inference/sample.py:5-6: greedy choice at the last position, one id per batch row."""
-    return ops.argmax_rows(logits[:, -1])
+    return ops.argmax_rows(logits[:, -1, :])
 
 
 class EmbeddingInput(torch.nn.Module):

@@ -300,3 +300,12 @@ def test_checked_once_handles_inference_tensors_and_caches_by_version():
             att._check_positions(torch.arange(17))
         assert att._rows_are_single_documents(torch.tensor([0, 8, 16], dtype=torch.int32), 2, 8)
         assert not att._rows_are_single_documents(torch.tensor([0, 5, 16], dtype=torch.int32), 2, 8)
+
+
+def test_greedy_choice_takes_batch_position_vocabulary():
+    from scaling_amd.inference import sample_argmax
+
+    logits = torch.tensor([[[5.0, 1.0, 2.0], [0.0, 3.0, 3.0]], [[1.0, 0.0, 9.0], [4.0, -1.0, float("nan")]]])
+    assert sample_argmax(logits).tolist() == [1, 2]
+    with pytest.raises(IndexError):
+        sample_argmax(logits[0])
