@@ -5,8 +5,8 @@
 // The row kernels:
 //   ce_row_kernel     gradient asked for: 1024-thread workgroups (one per compute unit) walk the rows; a row stays in
 //                     registers (up to 16 x 128-bit vectors per thread, i.e. 131072 16-bit or 65536 fp32 logits), so
-//                     max, sum of exponentials and the gradient all come from the single read; of rows longer than
-//                     9216 vectors the first 9 vectors per thread of the next row are fetched into LDS meanwhile
+//                     max, sum of exponentials and the gradient all come from the single read; of rows of more than 2
+//                     vectors per thread all whole ones (at most 9) of the next row are fetched into LDS meanwhile
 //   ce_fwd_kernel     no gradient: 512-thread workgroups stream a row once with a running (max, sum)
 //   ce_grad_kernel    gradient from a log-sum-exp that is already known, elementwise
 //   ce_stream_kernel  anything else (rows that do not fit, unaligned rows, vocab not a multiple of the vector width):
@@ -633,17 +633,36 @@ __global__ __launch_bounds__(kGradBlock) void ce_grad_kernel(const CeArgs a) {
     }
 }
 
-// The register-resident kernel: one resident workgroup per compute unit, each walking its share of the rows.
+// The register-resident kernel: one resident workgroup per compute unit, each walking its share of the rows.  From three vectors per thread
+// on all whole ones of the next row are staged (nine at most: the LDS), with as many registers as the row has vectors up to nine: a fifth to
+// eighth vector that is not there costs its exponentials all the same.  In place, us, nothing staged and 4, 8 or 16 registers / as it is, bf16:
+//   8192 x 20000 153 / 133     8192 x 32000 197 / 186     4096 x 40001 136 / 114     2047 x 50257 82 / 74     1024 x 65536 49 / 47
+//   4096 x 66000 225 / 193     2047 x 70000 123 / 106     fp32: 8192 x 10000 127 / 113     4096 x 25152 154 / 147     4096 x 33000 204 / 191
+// Rows of four whose logits stay in the cache are short and wait for their reads too little to make up for the staging: 2047 x 32000 46.7 /
+// 48.1, 2047 x 24999 41.4 / 43.5.  Beyond nine fewer than 16 registers are level (2047 x 76000 112 / 112, 4096 x 84000 250 / 247).
+constexpr int64_t kCacheBytes = (int64_t)256 << 20;
+
+template <int N> using Count = std::integral_constant<int, N>;
+
 template <typename T, bool RAGGED>
 void launch_rows(const CeArgs& a, int64_t n_rows, int64_t vecs, hipStream_t st) {
     const int nv = (int)((vecs + kCeBlock - 1) / kCeBlock), nr = (int)n_rows;
     const dim3 grid((unsigned)(n_rows < kCeResident ? n_rows : kCeResident)), block(kCeBlock);
-    if (nv <= 1) ce_row_kernel<T, 1, 0, RAGGED><<<grid, block, 0, st>>>(a, nr);
-    else if (nv <= 2) ce_row_kernel<T, 2, 0, RAGGED><<<grid, block, 0, st>>>(a, nr);
-    else if (nv <= 4) ce_row_kernel<T, 4, 0, RAGGED><<<grid, block, 0, st>>>(a, nr);
-    else if (nv <= 8) ce_row_kernel<T, 8, 0, RAGGED><<<grid, block, 0, st>>>(a, nr);
-    else if (vecs >= 9 * kCeBlock) ce_row_kernel<T, 16, 9, RAGGED><<<grid, block, 0, st>>>(a, nr);
-    else ce_row_kernel<T, 16, 0, RAGGED><<<grid, block, 0, st>>>(a, nr);
+    const bool cached = n_rows * vecs * 16 <= kCacheBytes;
+    const auto go = [&](auto regs, auto staged) { ce_row_kernel<T, decltype(regs)::value, decltype(staged)::value, RAGGED><<<grid, block, 0, st>>>(a, nr); };
+    switch (nv) {
+        case 0:
+        case 1: return go(Count<1>{}, Count<0>{});
+        case 2: return go(Count<2>{}, Count<0>{});
+        case 3: return go(Count<3>{}, Count<2>{});
+        case 4: return cached ? go(Count<4>{}, Count<0>{}) : go(Count<4>{}, Count<3>{});
+        case 5: return go(Count<5>{}, Count<4>{});
+        case 6: return go(Count<6>{}, Count<5>{});
+        case 7: return go(Count<7>{}, Count<6>{});
+        case 8: return go(Count<8>{}, Count<7>{});
+        case 9: return go(Count<9>{}, Count<8>{});
+        default: return go(Count<16>{}, Count<9>{});
+    }
 }
 
 // A row of at most kShortRow vectors is one wavefront's: with 512 threads most of them hold nothing and the block's merges are all

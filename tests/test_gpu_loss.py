@@ -362,3 +362,40 @@ def test_first_index_of_the_maximum_anywhere_in_a_row(vocab, offset, dtype):
     assert argmax.tolist() == at + at + [0]
     ref = torch.nn.functional.cross_entropy(x[:-1].double(), targets[:-1], reduction="none")
     assert torch.allclose(losses[:-1].double(), ref, rtol=1e-5, atol=1e-5)
+
+
+# Vectors of a row at the edges of the row kernel's register counts, where rows after a workgroup's first come through LDS but for their last
+# vectors; 4000 with logits beyond the cache too.  Every row against float64; a gradient of g rounds to half a unit of its type, and before
+# that carries the float32 evaluation of the exponent, |x - lse| < 32, to 32 x 2^-23 relative.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,vectors", [(600, 2049), (600, 3072), (600, 3073), (600, 4096), (4300, 4000), (600, 4097), (600, 5120), (530, 5121),
+                                          (530, 6144), (530, 6145), (530, 7169), (530, 8192), (530, 8193), (530, 9216), (530, 9217)])
+def test_cross_entropy_staged_rows(rows, vectors, dtype):
+    per = 4 if dtype == torch.float32 else 8
+    for vocab in (vectors * per, vectors * per - 3):
+        print(f"case cross_entropy staged rows={rows} vocab={vocab} dtype={dtype}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(vectors)
+        logits = torch.randn(rows, vectors * per, generator=g, device=DEV).mul_(3).to(dtype)
+        x = logits[:, :vocab].clone()
+        targets = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+        scale = torch.rand(rows, generator=g, device=DEV) + 0.1
+        losses, lse = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+        argmax = torch.empty(rows, dtype=torch.int32, device=DEV)
+        _lib.check(_lib.load().mi_cross_entropy_padded(logits.data_ptr(), targets.data_ptr(), scale.data_ptr(), losses.data_ptr(), lse.data_ptr(),
+                                                       argmax.data_ptr(), rows, vocab, vectors * per, ops.dtype_code(dtype), ops.stream_ptr()),
+                   "mi_cross_entropy_padded")
+        assert int(logits[:, vocab:].float().abs().sum()) == 0
+        unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+        least = {torch.bfloat16: 0.0, torch.float16: 2.0 ** -24, torch.float32: 0.0}[dtype]           # subnormals of fp16
+        for part in torch.arange(rows, device=DEV).split(64):
+            d = x[part].double()
+            ref_lse = torch.logsumexp(d, -1)
+            assert torch.allclose(lse[part].double(), ref_lse, rtol=1e-6, atol=1e-6)
+            at_target = d.gather(1, targets[part, None])[:, 0]
+            assert torch.allclose(losses[part].double(), ref_lse - at_target, rtol=1e-5, atol=1e-5)
+            assert torch.equal(d.gather(1, argmax[part].long()[:, None])[:, 0], d.max(-1).values)
+            ref = torch.exp(d - ref_lse[:, None])
+            ref.scatter_add_(1, targets[part, None], -torch.ones_like(targets[part, None], dtype=torch.float64))
+            ref *= scale[part, None].double()
+            error = (logits[part, :vocab].double() - ref).abs()
+            assert bool((error <= ref.abs() * (unit + 64 * 2.0 ** -23) + least + 1e-9).all()), float(error.max())
