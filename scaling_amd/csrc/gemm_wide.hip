@@ -115,9 +115,10 @@ template <bool KMAJOR, int HALVES> struct Loader {
         left = k;
         if (left < kStep) last(wave, lane);
     }
-    // the step that the contraction ends in
+    // The step that the contraction ends in.  Contiguous contraction indices end with a whole vector: an extent of an odd number of elements would
+    // end inside the word that holds the last one.
     __device__ __forceinline__ void last(int wave, int lane) {
-        const int cut = (kStep - left) * (KMAJOR ? step_bytes / kStep : 2);
+        const int cut = KMAJOR ? (kStep - left) * (step_bytes / kStep) : (kStep - (left + 7) / 8 * 8) * 2;
 #pragma unroll
         for (int h = 0; h < HALVES; ++h) srd[h][2] = (uint32_t)max((int)srd[h][2] - cut, 0);
         if (!KMAJOR) {

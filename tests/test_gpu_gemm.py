@@ -404,3 +404,43 @@ def test_ragged_extents_need_the_entry_with_a_workspace(rows, ins, outs):
     assert lib.mi_gemm(p, 1, 0, stream) != 0
     assert (lib.mi_gemm_with_workspace(p, 1, 0, None, 0, stream) == 0) == (ins % 8 == 0)
     torch.cuda.synchronize()
+
+
+# contractions that end inside a 32-bit word and at either end of a vector, of an operand contiguous along them; rows at the end of a block
+# (127, 255, 383 and the last), where nothing lies behind the row that may be read, take nearly all of their result from the last index
+@pytest.mark.parametrize("k", [16385, 16387, 16391, 16390, 65, 16384 + 63])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_last_index_of_a_ragged_contraction(k, dtype):
+    print(f"case ragged contraction k={k} dtype={dtype}", flush=True)
+    rows, n = (389, 520) if k > 1000 else (12293, 2056)
+    ld = (k + 7) // 8 * 8
+    g = torch.Generator(device=DEV).manual_seed(k)
+    p = torch.zeros(rows, ld, dtype=dtype, device=DEV)
+    p[:, :k] = (torch.randn(rows, k, generator=g, device=DEV) * 2.0 ** -6).to(dtype)
+    q = torch.randn(k, n, generator=g, device=DEV).to(dtype)
+    ends = sorted({*range(127, rows, 128), rows - 1})
+    p[ends, k - 1] = 8.0
+    q[k - 1] = 4.0
+    c = torch.full((rows, n), float("nan"), dtype=dtype, device=DEV)
+    pr = _lib.MiGemmProblem(c=c.data_ptr(), ldc=n, n_segments=1, m=rows, n=n, q_kmajor=1)
+    pr.segments[0] = _lib.MiGemmSegment(p.data_ptr(), q.data_ptr(), ld, n, k)
+    lib, code = _lib.load(), ops.dtype_code(dtype)
+    bytes_ = lib.mi_gemm_workspace_bytes(pr, 1, code)
+    ws = torch.empty(max(bytes_, 16) // 4, device=DEV)
+    _lib.check(lib.mi_gemm_with_workspace(pr, 1, code, ws.data_ptr(), bytes_, ops.stream_ptr()), "mi_gemm_with_workspace")
+    pd, qd = p[:, :k].double(), q.double()
+    _close("c", c, (pd @ qd).cpu(), (pd.abs() @ qd.abs()).cpu(), k, dtype)
+
+
+def test_lm_head_rows_whose_target_is_the_last_entry():
+    """dh over an odd vocabulary, row by row: where the target is the last entry, the last index of the contraction is half of the row."""
+    rows, hidden, vocab = 519, 256, 20003
+    g = torch.Generator(device=DEV).manual_seed(1)
+    h = torch.randn(rows, hidden, generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(vocab, hidden, generator=g, device=DEV) * 2 / hidden ** 0.5).bfloat16().requires_grad_()
+    t = torch.full((rows,), vocab - 1, device=DEV)
+    ops.linear_cross_entropy(h, w, t, torch.ones(rows, device=DEV))[0].backward()
+    hd, wd = h.detach().double().requires_grad_(), w.detach().double()
+    torch.nn.functional.cross_entropy(hd @ wd.t(), t).backward()
+    err = (h.grad.double() - hd.grad).norm(dim=1) / hd.grad.norm(dim=1)
+    assert float(err.max()) <= 2.0 ** -6, (int(err.argmax()), float(err.max()))   # logits, their gradient and dh rounded to bfloat16
