@@ -789,8 +789,9 @@ template <int D> static int launch_kept_f32(const F32Params& all, hipStream_t st
             attn_f32_dkdv_kernel<D, 2, true><<<dim3((unsigned)keys), block, 0, st>>>(fp);
             int rc = mi_check_launch("attn_bwd_dkdv (f32)");
             if (rc != MI_OK) return rc;
+            // by all heads, as where dS is not kept: the split of the keys is the order of the sums, which the room for dS must not decide
             const int64_t wide = (((int64_t)p.total_q + 127) / 128) * heads, narrow = (((int64_t)p.total_q + 31) / 32) * heads;
-            if (wide >= 2 * mi_compute_units()) attn_f32_dq_kept_kernel<D, 4><<<dim3((unsigned)wide), block, 0, st>>>(fp);
+            if (wide / heads * p.nq >= 2 * mi_compute_units()) attn_f32_dq_kept_kernel<D, 4><<<dim3((unsigned)wide), block, 0, st>>>(fp);
             else attn_f32_dq_kept_kernel<D, 1><<<dim3((unsigned)narrow), block, 0, st>>>(fp);
             rc = mi_check_launch("attn_bwd_dq (f32)");
             if (rc != MI_OK) return rc;

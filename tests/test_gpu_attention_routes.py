@@ -118,11 +118,12 @@ def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
 
 # float32 backward with dS kept by the dK/dV kernel (a workspace that has room for it) against the dQ kernel that recomputes it: the same
 # bits.  Triangle and whole plane, documents that end inside tiles, keys and queries of different lengths (rows that see nothing among
-# them), few KV heads, several passes over the heads (4128 tokens of 64 heads), each head_dim.
+# them), few KV heads, several passes over the heads (4128 tokens of 64 heads; 8192 of 12 and 16384 of 8, whose passes alone have fewer
+# query blocks than decide for a split of the keys), each head_dim.
 @pytest.mark.parametrize("nq,nkv,d,causal,lens_q,lens_k", [
     (32, 32, 128, True, [1101], None), (32, 32, 64, False, [500, 37, 590], None), (64, 32, 96, True, [33, 1, 700, 331], None),
     (16, 16, 128, True, [1000, 1200, 3], [900, 1300, 2]), (16, 16, 64, False, [700, 900], [1500, 617]), (16, 1, 128, True, [4099], None),
-    (64, 64, 64, True, [4128], None),
+    (64, 64, 64, True, [4128], None), (12, 12, 64, True, [8192], None), (12, 12, 96, False, [8190], None), (8, 8, 64, True, [16384], None),
 ])
 def test_float32_backward_with_kept_scores(nq, nkv, d, causal, lens_q, lens_k):
     print(f"case f32 kept nq={nq} nkv={nkv} d={d} causal={causal} q={lens_q} k={lens_k}", flush=True)
