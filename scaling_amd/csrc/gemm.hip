@@ -497,6 +497,6 @@ extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, vo
 }
 
 extern "C" size_t mi_gemm_workspace_bytes(const mi_gemm_problem* problems, int count, int dtype) {
-    if (!problems || count != 1 || problems[0].m <= 0 || problems[0].n <= 0 || problems[0].n_segments != 1 || !wide(problems, count, dtype, true)) return 0;
+    if (!problems || count < 1 || count > kMaxProblems || !wide(problems, count, dtype, true)) return 0;
     return mi_gemm_wide_plan(problems, count, (size_t)1 << 30, mi_compute_units()).workspace_bytes;
 }

@@ -5,7 +5,7 @@
 
 struct MiGemmPlan {
     double us;              // expected time
-    int tile;               // blocks of 128 or 256 rows and columns
+    int tile;               // blocks of 128 or 256 rows and columns; 0: several problems, each in a launch (and with a plan) of its own
     int splits;             // of the contraction (a single problem of one segment)
     size_t workspace_bytes;
     int cut;                // rows, or columns, that go in a launch of whole rounds, in front of the rest; 0: all in one launch

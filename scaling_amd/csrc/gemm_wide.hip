@@ -22,6 +22,7 @@
 #include "common.h"
 #include "gemm_wide.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -643,9 +644,25 @@ MiGemmPlan plan_in_one(const mi_gemm_problem* in, int count, size_t workspace_by
 // A problem whose last round is nearly empty goes in two launches: the rows or columns that make whole rounds, and the rest with a plan of its
 // own.  It waits for the first to drain, so it has to promise 7 %.  Loss and gradients of an LM head, us: 2047 x 1024 x 50257 680 -> 652 (logits in
 // 6 rounds and 160 small blocks instead of 7, weight gradient in 3 and 72 instead of 4), 8192 x 2048 x 9973 897 -> 820, 4096 x 4096 x 9973 level.
+// Several problems go in one launch, where short blocks fill the gaps that long ones leave, unless one of them is a long chain of few blocks
+// (tokens of a narrow layer: its weight gradient; few tokens before a wide output: its input gradient): it can be split over the chip only in a
+// launch of its own.  Both gradients, us, one launch / a launch each: 131072 x 256 -> 256 819 / 99, 32768 x 1024 -> 1024 213 / 131, 257 x 1024 ->
+// 16384 97 / 43, 2090 x 1536 -> 128256 1906 / 1277, 1976 x 2048 -> 8192 142 / 113; 4084 x 1024 -> 4096 65 / 68, 300 x 4096 -> 14336 and 14336 273 / 352,
+// 1468 x 4096 -> 4096 81 / 99.  A launch each is expected to take too little, mostly (of these 0.10, 0.45, 0.32, 0.57, 0.64 of one launch; 0.80, 0.80, 0.89), hence 0.65.
 MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t workspace_bytes, int cus) {
     MiGemmPlan best = plan_in_one(in, count, workspace_bytes, cus);
-    if (count > 1) return best;
+    if (count > 1) {
+        double us = 0;
+        size_t bytes = 0;
+        for (int i = 0; i < count && us < best.us * 0.65; ++i) {
+            if (in[i].m == 0) continue;
+            const MiGemmPlan p = mi_gemm_wide_plan(in + i, 1, workspace_bytes, cus);
+            us += p.us;
+            bytes = std::max(bytes, p.workspace_bytes);
+        }
+        if (us < best.us * 0.65) best = MiGemmPlan{us, 0, 1, bytes, 0, false};
+        return best;
+    }
     const mi_gemm_problem& a = in[0];
     double us = best.us * 0.93;
     for (int tile = 128; tile <= 256; tile += 128) {
@@ -667,6 +684,12 @@ MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t worksp
 }
 
 int mi_gemm_wide(const mi_gemm_problem* in, int count, int dtype, const MiGemmPlan& plan, void* workspace, int cus, hipStream_t st) {
+    if (plan.tile == 0) {                                  // one after the other, with the same workspace
+        int rc = MI_OK;
+        for (int i = 0; i < count && rc == MI_OK; ++i)
+            if (in[i].m > 0) rc = mi_gemm_wide(in + i, 1, dtype, mi_gemm_wide_plan(in + i, 1, plan.workspace_bytes, cus), workspace, cus, st);
+        return rc;
+    }
     if (plan.cut == 0) return launch_in_one(in, count, dtype, plan, workspace, st);
     const mi_gemm_problem first = part(in[0], plan.columns, plan.cut, true), rest = part(in[0], plan.columns, plan.cut, false);
     const int rc = launch_in_one(&first, 1, dtype, MiGemmPlan{plan.us, plan.tile, 1, 0, 0, false}, nullptr, st);

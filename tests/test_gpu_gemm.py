@@ -444,3 +444,45 @@ def test_lm_head_rows_whose_target_is_the_last_entry():
     torch.nn.functional.cross_entropy(hd @ wd.t(), t).backward()
     err = (h.grad.double() - hd.grad).norm(dim=1) / hd.grad.norm(dim=1)
     assert float(err.max()) <= 2.0 ** -6, (int(err.argmax()), float(err.max()))   # logits, their gradient and dh rounded to bfloat16
+
+
+# both gradients of a projection where one of them is a long chain of few blocks: many tokens of a narrow layer (weight gradient; with the
+# bias gradient beside a split), few tokens before a wide output (input gradient).  Each gets the plan that it has alone, splits included.
+@pytest.mark.parametrize("rows,ins,outs,bias", [(32768, 256, 256, True), (20000, 264, 520, False), (257, 1024, 16384, True), (130, 776, 40960, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gradients_of_which_one_is_a_long_chain(rows, ins, outs, bias, dtype):
+    print(f"case chain rows={rows} in={ins} out={outs} dtype={dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w, dy = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((rows, ins), (outs, ins), (rows, outs)))
+    lib, code = _lib.load(), ops.dtype_code(dtype)
+
+    def problems(dx, dw, db):
+        a = _lib.MiGemmProblem(c=dx.data_ptr(), ldc=ins, n_segments=1, m=rows, n=ins, q_kmajor=1)
+        a.segments[0] = _lib.MiGemmSegment(dy.data_ptr(), w.data_ptr(), outs, ins, outs)
+        b = _lib.MiGemmProblem(c=dw.data_ptr(), ldc=ins, n_segments=1, m=outs, n=ins, p_kmajor=1, q_kmajor=1, p_sum=db.data_ptr() if bias else None)
+        b.segments[0] = _lib.MiGemmSegment(dy.data_ptr(), x.data_ptr(), outs, ins, rows)
+        return (_lib.MiGemmProblem * 2)(a, b)
+
+    def run(p, count):
+        bytes_ = lib.mi_gemm_workspace_bytes(p, count, code)
+        ws = torch.full((max(bytes_, 16) // 4,), float("nan"), device=DEV)
+        _lib.check(lib.mi_gemm_with_workspace(p, count, code, ws.data_ptr(), bytes_, ops.stream_ptr()), "mi_gemm_with_workspace")
+        torch.cuda.synchronize()
+        return bytes_
+
+    new = lambda: (torch.empty_like(x), torch.empty_like(w), torch.empty(outs, dtype=dtype, device=DEV))
+    both, each = new(), new()
+    need = run(problems(*both), 2)
+    single = problems(*each)
+    assert need == max(run(_lib.MiGemmProblem.from_buffer_copy(bytes(single[i])), 1) for i in range(2)) > 0
+    xd, wd, dyd = x.double(), w.double(), dy.double()
+    _close("dx", both[0], (dyd @ wd).cpu(), (dyd.abs() @ wd.abs()).cpu(), outs, dtype)
+    _close("dw", both[1], (dyd.t() @ xd).cpu(), (dyd.abs().t() @ xd.abs()).cpu(), rows, dtype)
+    assert torch.equal(both[0], each[0]) and torch.equal(both[1], each[1])
+    if bias:
+        _close("db", both[2], dyd.sum(0).cpu(), dyd.abs().sum(0).cpu(), rows, dtype)
+        assert torch.equal(both[2], each[2])
+    xg, wg = x.clone().requires_grad_(), w.clone().requires_grad_()
+    bg = torch.zeros(outs, dtype=dtype, device=DEV, requires_grad=True) if bias else None
+    ops.linear(xg, wg, bg).backward(dy)
+    assert torch.equal(xg.grad, both[0]) and torch.equal(wg.grad, both[1]) and (not bias or torch.equal(bg.grad, both[2]))
