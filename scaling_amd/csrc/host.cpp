@@ -361,7 +361,7 @@ bool long_chain(const Tensor& t, int64_t rows, int64_t k) { return k >= 3072 && 
 // Larger products of 16-bit types with whole vectors in every direction: blocks of 128 or 256 rows and columns in mi_gemm, all layouts at the rate
 // of the library's fastest.  us on the device, mi_gemm and library: 4084 x 1024 -> 4096 forward 34.4 / 30.5, input gradient 34.6 / 40.0,
 // weight gradient 32.7 / 37.5; 1024 -> 1024 13.8 / 13.4, 13.7 / 15.0, 22.4 / 33.0; 8192 x 4096 -> 14336 649 / 618, 629 / 693, 660 / 827 (767 + 24
-// with x transposed first).  Fewer than 128 rows fill no block.
+// with x transposed first).  Fewer than 128 rows, or 32 features on either side, fill no block (8192 x 32768 -> 16, forward and gradients, 409 / 442).
 //   Training (forward and gradients, here and with the library): 2048 x 1024 -> 1024 33 / 78, 2048 x 4096 -> 4096 177 / 193, 301 x 4096 -> 14336
 // 188 / 227; forward products of 100 GFLOP and more stay on the library.
 //   Inference keeps the library where its own time exceeds what it costs the host, or nearly: issued one by one (on the device alone) 2048 x 1024 ->
@@ -371,8 +371,15 @@ enum class Pass { kInference, kForward, kBackward };
 bool wide_product(const Tensor& t, int64_t rows, int64_t n, int64_t k, Pass pass) {
     const double work = 2.0 * (double)rows * (double)n * (double)k;
     if (pass == Pass::kInference ? k > 1536 || work > 1e10 : pass == Pass::kForward && work >= 1e11) return false;
-    return t.scalar_type() != at::kFloat && rows >= 128 && n % 8 == 0 && k % 8 == 0;
+    return t.scalar_type() != at::kFloat && rows >= 128 && n >= 32 && k >= 32 && n % 8 == 0 && k % 8 == 0;
 }
+// Short contractions into large outputs: a block spends more on its fill and its results than on products, and the library's kernels for whole
+// blocks do that part better.  us, mi_gemm and library, forward / input gradient / weight gradient layout:
+//   8192 x 8192, k 32  51 30 / 51 32 / 49 32   k 192  65 50 / 65 51 / 61 50   k 320  83 62 / 81 66 / 75 65   k 448  91 78 / 88 80 / 85 80   k 512  89 84 / 88 86 / 85 87
+//   4096 x 4096, k 256  29 20 / 19 18 / 18 19        2048 x 4096, k 256  15 18 / 16 18 / 15 19        8192 x 32768, forward, k 96  226 145   k 144  279 240
+// Where the library's blocks are not whole, mi_gemm stays: 8192 x 8256, k 256  78 87 / 78 90 / 74 91;  16001 x 3072, k 360  67 67 / 64 66;  4096 x 14920, k 64
+// 51 56 / 51 58 / 50 59;  8192 x 32768, forward, k 200  248 250.
+bool thin(int64_t m, int64_t n, int64_t k) { return k < 512 && k % 16 == 0 && n % 256 == 0 && (double)m * (double)n >= 33554432.0; }
 bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous rows, none on top of another, that start on 16-byte boundaries
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
@@ -460,7 +467,7 @@ struct Projections : Function<Projections> {
             const Tensor& w = params[i];
             fit = fit && aligned(w);
             small = small && small_product(x, rows, w.size(0), in);
-            wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward);
+            wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward) && !thin(rows, w.size(0), in);
         }
         // What the gradients read and no more, so that the rest may be changed or freed before the backward pass: x (itself: what is
         // differentiated again reaches it) for the weights, the weights for x.  The same for a recomputation inside a backward pass.
@@ -534,52 +541,51 @@ struct Projections : Function<Projections> {
         for (int64_t i = 0; i < n && !any.defined(); ++i) any = dy[i];
         if (!any.defined()) return variable_list(n + at.size() - std::count(at.begin(), at.end(), -1) + 4);
         Launch l(any);
-        if (fit && (small || wide)) {
-            mi_gemm_problem pr[MI_GEMM_MAX_PROBLEMS];
-            int count = 0;
-            if (need_dx) {
-                dx = at::empty({rows, in}, any.options());
-                mi_gemm_problem p = problem(dx, false, true);
-                for (int64_t i = 0; i < n; ++i)
-                    if (dy[i].defined()) segment(p, dy[i], saved[1 + i], dy[i].size(1));
-                pr[count++] = p;
-            }
-            for (int64_t i = 0; i < n; ++i) {
-                if (!dy[i].defined()) continue;
-                if (!need_weight(i)) {
-                    if (need_bias(i)) db[i] = bias_gradient(dy[i]);
-                    continue;
-                }
-                dw[i] = at::empty({dy[i].size(1), in}, any.options());
-                mi_gemm_problem p = problem(dw[i], true, true);
-                segment(p, dy[i], x, rows);
-                if (need_bias(i)) {
-                    db[i] = at::empty({dy[i].size(1)}, any.options());
-                    p.p_sum = ptr(db[i]);
-                }
-                pr[count++] = p;
-            }
-            if (count > 0) run_gemm(pr, count, any, l);
-        } else {
-            int64_t out = 0;
+        int64_t sum_out = 0;
+        for (const Tensor& t : dy) sum_out += t.defined() ? t.size(1) : 0;
+        const auto mine = [&](int64_t m, int64_t k) { return fit && (small || (wide && !thin(m, in, k))); };
+        mi_gemm_problem pr[MI_GEMM_MAX_PROBLEMS];
+        int count = 0;
+        if (need_dx && mine(rows, sum_out)) {
+            dx = at::empty({rows, in}, any.options());
+            mi_gemm_problem p = problem(dx, false, true);
             for (int64_t i = 0; i < n; ++i)
-                if (dy[i].defined() && need_weight(i)) out += dy[i].size(1);
-            Tensor xt, dyt;                                // the smaller of the two operands, where that pays
-            if (!again && out > 0 && transpose_pays(rows, in, out)) {
-                if (in <= out && transposable(x)) xt = transposed(x, l);
-                else if (n == 1 && transposable(dy[0])) dyt = transposed(dy[0], l);
+                if (dy[i].defined()) segment(p, dy[i], saved[1 + i], dy[i].size(1));
+            pr[count++] = p;
+        }
+        int64_t out = 0;                                   // of the weight gradients that the library makes
+        for (int64_t i = 0; i < n; ++i) {
+            if (!dy[i].defined() || !need_weight(i)) continue;
+            if (!mine(dy[i].size(1), rows)) {
+                out += dy[i].size(1);
+                continue;
             }
-            for (int64_t i = 0; i < n; ++i) {
-                if (!dy[i].defined()) continue;
+            dw[i] = at::empty({dy[i].size(1), in}, any.options());
+            mi_gemm_problem p = problem(dw[i], true, true);
+            segment(p, dy[i], x, rows);
+            if (need_bias(i)) {
+                db[i] = at::empty({dy[i].size(1)}, any.options());
+                p.p_sum = ptr(db[i]);
+            }
+            pr[count++] = p;
+        }
+        if (count > 0) run_gemm(pr, count, any, l);
+        Tensor xt, dyt;                                    // the smaller of the two operands, where that pays
+        if (!again && out > 0 && transpose_pays(rows, in, out)) {
+            if (in <= out && transposable(x)) xt = transposed(x, l);
+            else if (n == 1 && transposable(dy[0])) dyt = transposed(dy[0], l);
+        }
+        const bool library_dx = need_dx && !dx.defined();
+        for (int64_t i = 0; i < n; ++i) {
+            if (!dy[i].defined()) continue;
+            if (library_dx) {
                 const Tensor& w = saved[1 + i];
-                if (need_dx) {
-                    if (!dx.defined()) dx = at::mm(dy[i], w);
-                    else if (again) dx = dx + at::mm(dy[i], w);
-                    else dx.addmm_(dy[i], w);              // summed inside the product
-                }
-                if (need_weight(i)) dw[i] = dyt.defined() ? at::mm(dyt, x) : at::mm(dy[i].t(), xt.defined() ? xt.t() : x);
-                if (need_bias(i)) db[i] = again ? dy[i].sum(0) : bias_gradient(dy[i]);
+                if (!dx.defined()) dx = at::mm(dy[i], w);
+                else if (again) dx = dx + at::mm(dy[i], w);
+                else dx.addmm_(dy[i], w);                  // summed inside the product
             }
+            if (need_weight(i) && !dw[i].defined()) dw[i] = dyt.defined() ? at::mm(dyt, x) : at::mm(dy[i].t(), xt.defined() ? xt.t() : x);
+            if (need_bias(i) && !db[i].defined()) db[i] = again ? dy[i].sum(0) : bias_gradient(dy[i]);
         }
         variable_list grads{dx.defined() ? dx.view(x_shape) : Tensor()};
         for (int64_t i = 0; i < n; ++i) grads.push_back(dw[i]);
@@ -918,9 +924,9 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
             const Tensor hc = h.narrow(0, r0, r);
             Tensor logits = buffer.narrow(0, 0, r).narrow(1, 0, vocab);
             // 2047 x 50257 x 1024, us, mi_gemm and library: logits 216 / 257, dh 161 / 291, dW 197 / 252
-            const bool wide = wide_product(h, r, 8, h.size(1), Pass::kBackward) && 2.0 * (double)r * (double)vocab * (double)h.size(1) > 3e9 && aligned(hc) &&
+            const bool wide = wide_product(h, r, 32, h.size(1), Pass::kBackward) && 2.0 * (double)r * (double)vocab * (double)h.size(1) > 3e9 && aligned(hc) &&
                               aligned(weight);
-            if (wide) {
+            if (wide && !thin(r, vocab, h.size(1))) {
                 mi_gemm_problem p = problem(logits, false, false);
                 segment(p, hc, weight, h.size(1));
                 run_gemm(&p, 1, h, l);
@@ -949,7 +955,7 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
             }
             if (need_dw) {
                 Tensor product;
-                if (wide) {
+                if (wide && !thin(vocab, h.size(1), r)) {
                     product = at::empty({vocab, h.size(1)}, h.options());
                     mi_gemm_problem p = problem(product, true, true);
                     segment(p, logits, hc, r);
