@@ -13,6 +13,7 @@
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/SavedTensorHooks.h>
+#include <ATen/hip/HIPContext.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -366,7 +367,10 @@ bool long_chain(const Tensor& t, int64_t rows, int64_t k) { return k >= 3072 && 
 // 188 / 227; forward products of 100 GFLOP and more stay on the library.
 //   Inference keeps the library where its own time exceeds what it costs the host, or nearly: issued one by one (on the device alone) 2048 x 1024 ->
 // 1024 12.2 / 19.7 (11.8 / 10.2), 1024 x 1024 -> 4096 13.7 / 19.9 (14.2 / 13.4), 2048 x 1024 -> 4096 26.5 / 21.8, 1024 x 2816 -> 1024 22.5 / 19.8 (22.5 /
-// 13.4), 513 x 2048 -> 2048 19.2 / 19.8 (19.7 / 12.3), 4084 x 2048 -> 2048 41 / 35, 301 x 4096 -> 14336 59 / 40.
+// 13.4), 513 x 2048 -> 2048 19.2 / 19.8 (19.7 / 12.3), 4084 x 2048 -> 2048 41 / 35, 301 x 4096 -> 14336 59 / 40.  So does a second round of blocks, beyond
+// 512 contraction indices (issued one by one, where the library is 20.2): one round 1078 x 1024 -> 3072 12.8, 2897 x 1536 -> 1024 15.8,
+// two 1163 x 1024 -> 4096 22.0, 739 x 800 -> 6912 23.2, 1142 x 640 -> 5632 21.8, 1982 x 552 -> 2544 22.4, 1785 x 512 -> 4224 19.7, 1450 x 384 -> 3072 16.5, three
+// 1350 x 384 -> 8192 18.2.  Of several projections, which are a library call each, the average decides.
 enum class Pass { kInference, kForward, kBackward };
 bool wide_product(const Tensor& t, int64_t rows, int64_t n, int64_t k, Pass pass) {
     const double work = 2.0 * (double)rows * (double)n * (double)k;
@@ -463,12 +467,15 @@ struct Projections : Function<Projections> {
         const int64_t rows = x2.size(0);
         variable_list saved, out;
         bool small = !(inference && long_chain(x, rows, in)), wide = true, fit = aligned(x2);
+        int64_t blocks = 0;
         for (int64_t i = 0; i < n; ++i) {
             const Tensor& w = params[i];
+            blocks += (rows + 127) / 128 * ((w.size(0) + 127) / 128);
             fit = fit && aligned(w);
             small = small && small_product(x, rows, w.size(0), in);
             wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward) && !thin(rows, w.size(0), in);
         }
+        if (inference && in > 512 && blocks > n * at::cuda::getDeviceProperties(x.device().index())->multiProcessorCount) wide = false;
         // What the gradients read and no more, so that the rest may be changed or freed before the backward pass: x (itself: what is
         // differentiated again reaches it) for the weights, the weights for x.  The same for a recomputation inside a backward pass.
         bool any_weight = false;

@@ -522,3 +522,22 @@ def test_short_contractions_into_large_outputs(rows, ins, outs, library):
     for name, t in (("dx", xg), ("dw", wg)):
         assert float((t.grad.float() - ref[name].float()).norm() / ref[name].float().norm()) < eps
     _close("db", b.grad, dy.double().sum(0).cpu(), dy.double().abs().sum(0).cpu(), rows, torch.bfloat16)
+
+
+# inference: one round of 128 x 128 blocks, or short contractions, on the package's kernel; a second round beyond 512 contraction indices is the
+# library's, by the average of projections that share their input
+@pytest.mark.parametrize("rows,ins,outs,own", [
+    (1078, 1024, (3072,), True), (1024, 1024, (4096,), True), (1025, 1024, (4096,), False), (1450, 520, (3072,), False), (1450, 512, (3072,), True),
+    (1163, 1024, (4096, 256), True), (1163, 1024, (4096, 4096), False), (1000, 1544, (1024,), False),
+])
+def test_route_of_inference_products(rows, ins, outs, own):
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, ins, generator=g, device=DEV).bfloat16()
+    ws = [torch.randn(o, ins, generator=g, device=DEV).bfloat16() for o in outs]
+    with torch.no_grad():
+        call = lambda: ops.projections(x, ws, [None] * len(ws), True)
+        for y, w in zip(call(), ws):
+            ref = x.double() @ w.double().t()
+            assert float((y.double() - ref).norm() / ref.norm()) < 2.0 ** -8
+        names = launched(call)
+    assert any("wide_kernel" in k for k in names) == own and any("wide_kernel" not in k for k in names) != own, names
