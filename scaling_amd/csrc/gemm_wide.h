@@ -5,11 +5,12 @@
 
 struct MiGemmPlan {
     double us;              // expected time
-    int tile;               // blocks of 128 or 256 rows and columns; 0: several problems, each in a launch (and with a plan) of its own
+    int tile;               // blocks of 128 or 256 rows and columns
     int splits;             // of the contraction (a single problem of one segment)
     size_t workspace_bytes;
     int cut;                // rows, or columns, that go in a launch of whole rounds, in front of the rest; 0: all in one launch
     bool columns;
+    int apart;              // several problems: 0 in one launch, -1 in a launch (and with a plan) each, i + 1 problem i alone and the rest in one
 };
 // the fastest plan that takes no more than workspace_bytes
 MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* problems, int count, size_t workspace_bytes, int compute_units);

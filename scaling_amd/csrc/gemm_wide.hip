@@ -599,6 +599,14 @@ mi_gemm_problem part(const mi_gemm_problem& a, bool columns, int at, bool first)
     return r;
 }
 
+// all problems but one; returns how many
+int others(const mi_gemm_problem* in, int count, int but, mi_gemm_problem* out) {
+    int n = 0;
+    for (int i = 0; i < count; ++i)
+        if (i != but) out[n++] = in[i];
+    return n;
+}
+
 MiGemmPlan plan_in_one(const mi_gemm_problem* in, int count, size_t workspace_bytes, int cus);
 int launch_in_one(const mi_gemm_problem* in, int count, int dtype, const MiGemmPlan& plan, void* workspace, hipStream_t st);
 
@@ -625,14 +633,14 @@ MiGemmPlan plan_in_one(const mi_gemm_problem* in, int count, size_t workspace_by
         // one problem: whole rounds; several: their blocks fill each other's gaps
         rounds_time = count == 1 ? longest * (double)((tiles + cus - 1) / cus) : (work / cus + (tiles > cus ? 0.5 * longest : 0));
         double us = rounds_time > longest ? rounds_time : longest;
-        if (us < best.us) best = MiGemmPlan{us, tile, 1, 0, 0, false};
+        if (us < best.us) best = MiGemmPlan{us, tile, 1, 0, 0, false, 0};
         if (count == 1 && in[0].n_segments == 1) {
             const int steps = steps_of(in[0]);
             for (int s = 2; s <= 16 && tiles * s <= cus && steps / s >= 8; ++s) {
                 const size_t bytes = (size_t)tiles * tile * tile * 4 * s;
                 if (bytes > workspace_bytes) break;
                 us = block_us(tile, (steps + s - 1) / s) + 3.0 + 2.0 * bytes / 5e6;
-                if (us < best.us) best = MiGemmPlan{us, tile, s, bytes, 0, false};
+                if (us < best.us) best = MiGemmPlan{us, tile, s, bytes, 0, false, 0};
             }
         }
     }
@@ -646,21 +654,30 @@ MiGemmPlan plan_in_one(const mi_gemm_problem* in, int count, size_t workspace_by
 // 6 rounds and 160 small blocks instead of 7, weight gradient in 3 and 72 instead of 4), 8192 x 2048 x 9973 897 -> 820, 4096 x 4096 x 9973 level.
 // Several problems go in one launch, where short blocks fill the gaps that long ones leave, unless one of them is a long chain of few blocks
 // (tokens of a narrow layer: its weight gradient; few tokens before a wide output: its input gradient): it can be split over the chip only in a
-// launch of its own.  Both gradients, us, one launch / a launch each: 131072 x 256 -> 256 819 / 99, 32768 x 1024 -> 1024 213 / 131, 257 x 1024 ->
+// launch of its own.  All gradients, us, one launch / a launch each: 131072 x 256 -> 256 819 / 99, 32768 x 1024 -> 1024 213 / 131, 257 x 1024 ->
 // 16384 97 / 43, 2090 x 1536 -> 128256 1906 / 1277, 1976 x 2048 -> 8192 142 / 113; 4084 x 1024 -> 4096 65 / 68, 300 x 4096 -> 14336 and 14336 273 / 352,
-// 1468 x 4096 -> 4096 81 / 99.  A launch each is expected to take too little, mostly (of these 0.10, 0.45, 0.32, 0.57, 0.64 of one launch; 0.80, 0.80, 0.89), hence 0.65.
+// 1468 x 4096 -> 4096 81 / 99.  A launch each is expected to take too little, mostly (of these 0.10, 0.45, 0.32, 0.57, 0.64 of one launch; 0.80, 0.80, 0.89), hence
+// 0.65; the longest chain alone and the rest in one launch 0.70: 1024 x 4096 -> 14336 and 14336 573 / 476 (0.68), 32768 x 1024 -> three of 1024 425 / 430 (0.72).
 MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t workspace_bytes, int cus) {
     MiGemmPlan best = plan_in_one(in, count, workspace_bytes, cus);
     if (count > 1) {
-        double us = 0;
-        size_t bytes = 0;
-        for (int i = 0; i < count && us < best.us * 0.65; ++i) {
+        double each = 0, longest_us = 0;
+        size_t bytes = 0, longest_bytes = 0;
+        int longest = 0;
+        for (int i = 0; i < count; ++i) {
             if (in[i].m == 0) continue;
             const MiGemmPlan p = mi_gemm_wide_plan(in + i, 1, workspace_bytes, cus);
-            us += p.us;
+            each += p.us;
             bytes = std::max(bytes, p.workspace_bytes);
+            if (i > 0 && steps_of(in[i]) <= steps_of(in[longest])) continue;
+            longest = i;
+            longest_us = p.us;
+            longest_bytes = p.workspace_bytes;
         }
-        if (us < best.us * 0.65) best = MiGemmPlan{us, 0, 1, bytes, 0, false};
+        if (each < best.us * 0.65) return MiGemmPlan{each, 0, 1, bytes, 0, false, -1};
+        mi_gemm_problem rest[MI_GEMM_MAX_PROBLEMS];
+        const double two = longest_us + plan_in_one(rest, others(in, count, longest, rest), 0, cus).us;
+        if (count > 2 && two < best.us * 0.70) return MiGemmPlan{two, 0, 1, longest_bytes, 0, false, longest + 1};
         return best;
     }
     const mi_gemm_problem& a = in[0];
@@ -676,7 +693,7 @@ MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t worksp
             const double both = rounds * block_us(tile, steps_of(a)) + p.us;
             if (both < us) {
                 us = both;
-                best = MiGemmPlan{both, tile, 1, p.workspace_bytes, (int)cut, columns != 0};
+                best = MiGemmPlan{both, tile, 1, p.workspace_bytes, (int)cut, columns != 0, 0};
             }
         }
     }
@@ -684,15 +701,19 @@ MiGemmPlan mi_gemm_wide_plan(const mi_gemm_problem* in, int count, size_t worksp
 }
 
 int mi_gemm_wide(const mi_gemm_problem* in, int count, int dtype, const MiGemmPlan& plan, void* workspace, int cus, hipStream_t st) {
-    if (plan.tile == 0) {                                  // one after the other, with the same workspace
+    if (plan.apart != 0) {                                 // one after the other, with the same workspace
         int rc = MI_OK;
         for (int i = 0; i < count && rc == MI_OK; ++i)
-            if (in[i].m > 0) rc = mi_gemm_wide(in + i, 1, dtype, mi_gemm_wide_plan(in + i, 1, plan.workspace_bytes, cus), workspace, cus, st);
-        return rc;
+            if (in[i].m > 0 && (plan.apart < 0 || plan.apart == i + 1))
+                rc = mi_gemm_wide(in + i, 1, dtype, mi_gemm_wide_plan(in + i, 1, plan.workspace_bytes, cus), workspace, cus, st);
+        if (plan.apart < 0 || rc != MI_OK) return rc;
+        mi_gemm_problem rest[MI_GEMM_MAX_PROBLEMS];
+        const int left = others(in, count, plan.apart - 1, rest);
+        return launch_in_one(rest, left, dtype, plan_in_one(rest, left, 0, cus), nullptr, st);
     }
     if (plan.cut == 0) return launch_in_one(in, count, dtype, plan, workspace, st);
     const mi_gemm_problem first = part(in[0], plan.columns, plan.cut, true), rest = part(in[0], plan.columns, plan.cut, false);
-    const int rc = launch_in_one(&first, 1, dtype, MiGemmPlan{plan.us, plan.tile, 1, 0, 0, false}, nullptr, st);
+    const int rc = launch_in_one(&first, 1, dtype, MiGemmPlan{plan.us, plan.tile, 1, 0, 0, false, 0}, nullptr, st);
     if (rc != MI_OK) return rc;
     return launch_in_one(&rest, 1, dtype, plan_in_one(&rest, 1, plan.workspace_bytes, cus), workspace, st);
 }

@@ -26,6 +26,15 @@ def _close(name, got, ref, magnitude, k, dtype):
     assert bool((err <= bound * 1.001).all()), f"{name}: {float((err / bound).max()):.2f} x the bound"
 
 
+def launched(call):
+    """Names of the kernels that a call launches."""
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+
+
 def _case(rows, ins, outs, dtype, seed):
     g = torch.Generator().manual_seed(seed)
     x = torch.randn(rows, ins, generator=g).to(dtype)
@@ -488,13 +497,23 @@ def test_gradients_of_which_one_is_a_long_chain(rows, ins, outs, bias, dtype):
     assert torch.equal(xg.grad, both[0]) and torch.equal(wg.grad, both[1]) and (not bias or torch.equal(bg.grad, both[2]))
 
 
-def launched(call):
-    """Names of the kernels that a call launches."""
-    torch.cuda.synchronize()
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
-        call()
-        torch.cuda.synchronize()
-    return [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+def test_chain_alone_and_the_rest_in_one_launch():
+    """1024 rows of two wide projections: the input gradient (one sum over both) in a launch of its own, both weight gradients in another."""
+    rows, ins, outs = 1024, 4096, 14336
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(rows, ins, generator=g, device=DEV).bfloat16().requires_grad_()
+    ws = [torch.randn(outs, ins, generator=g, device=DEV).bfloat16().requires_grad_() for _ in range(2)]
+    dys = [torch.randn(rows, outs, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    ys = ops.projections(x, ws, [None, None])
+    names = launched(lambda: torch.autograd.backward(ys, dys))
+    assert sum("wide_kernel" in k for k in names) == 2, names
+    rows_ = torch.tensor([0, 127, 128, 700, rows - 1], device=DEV)
+    dyd, wd, xd = [d.double() for d in dys], [w.detach().double() for w in ws], x.detach().double()
+    _close("dx", x.grad[rows_], sum(d[rows_] @ w for d, w in zip(dyd, wd)).cpu(), sum(d[rows_].abs() @ w.abs() for d, w in zip(dyd, wd)).cpu(), 2 * outs, torch.bfloat16)
+    cols = torch.tensor([0, 255, 256, 9000, outs - 1], device=DEV)
+    for w, d in zip(ws, dyd):
+        a = d[:, cols].t().contiguous()
+        _close("dw", w.grad[cols], (a @ xd).cpu(), (a.abs() @ xd.abs()).cpu(), rows, torch.bfloat16)
 
 
 # short contractions into large outputs are the library's, each product by itself: forward (k = ins), input gradient (k = outs) and weight
