@@ -318,6 +318,18 @@ int launch_wide(const mi_gemm_problem* in, int count, int dtype, void* workspace
     return mi_gemm_wide(in, count, dtype, plan, workspace, mi_compute_units(), st);
 }
 
+// Without a workspace no contraction is split, and large blocks on a quarter of the chip walk it in one chain: the small ones (or mi_rows_product) keep
+// what leaves them less than that or fits one round of 32 x 32.  us, small and large: 64 x 14336 -> 4096 (32 large blocks) 52 / 82, 127 x 4096 -> 4096 (32)
+// 21 / 28, 32 x 8192 -> 8192 (64, one round) 37 / 50, 96 x 8192 -> 8192 (64) 64 / 50, 64 x 4096 -> 14336 (112) 53 / 29, 16 x 4096 -> 128256 244 / 181.
+bool few_blocks(const mi_gemm_problem* in, int count) {
+    int64_t large = 0, small = 0;
+    for (int i = 0; i < count; ++i) {
+        large += (int64_t)((in[i].m + 127) / 128) * ((in[i].n + 127) / 128);
+        small += (int64_t)((in[i].m + 31) / 32) * ((in[i].n + 31) / 32);
+    }
+    return 4 * large < mi_compute_units() || small <= mi_compute_units();
+}
+
 template <typename T> int launch(const mi_gemm_problem* in, int count, hipStream_t st) {
     constexpr int V = Elem<T>::kVec;
     Problems ps;
@@ -491,7 +503,7 @@ extern "C" int mi_gemm_with_workspace(const mi_gemm_problem* problems, int count
 
 extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
     if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
-    if (wide(problems, count, dtype, false)) return launch_wide(problems, count, dtype, nullptr, 0, (hipStream_t)stream);
+    if (wide(problems, count, dtype, false) && !few_blocks(problems, count)) return launch_wide(problems, count, dtype, nullptr, 0, (hipStream_t)stream);
     MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
     return MI_OK;
 }

@@ -560,3 +560,22 @@ def test_route_of_inference_products(rows, ins, outs, own):
             assert float((y.double() - ref).norm() / ref.norm()) < 2.0 ** -8
         names = launched(call)
     assert any("wide_kernel" in k for k in names) == own and any("wide_kernel" not in k for k in names) != own, names
+
+
+@pytest.mark.parametrize("rows,ins,outs,large", [(64, 14336, 4096, False), (96, 4096, 4096, False), (32, 8192, 8192, False), (16, 12288, 8192, False), (96, 8192, 8192, True),
+                                                 (16, 4096, 32000, True), (64, 4096, 14336, True)])
+def test_few_blocks_without_a_workspace(rows, ins, outs, large):
+    """mi_gemm has nothing to split a long contraction with: few large blocks are left to the small ones; with a workspace they are split."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w = (torch.randn(n, ins, generator=g, device=DEV).bfloat16() for n in (rows, outs))
+    c = torch.empty(rows, outs, dtype=torch.bfloat16, device=DEV)
+    p = _lib.MiGemmProblem(c=c.data_ptr(), ldc=outs, n_segments=1, m=rows, n=outs)
+    p.segments[0] = _lib.MiGemmSegment(x.data_ptr(), w.data_ptr(), ins, ins, ins)
+    lib, ws = _lib.load(), torch.empty(1 << 26, device=DEV)
+    ref, magnitude = (x.double() @ w.double().t()).cpu(), (x.double().abs() @ w.double().abs().t()).cpu()
+    for call, wide in ((lambda: lib.mi_gemm(p, 1, 0, ops.stream_ptr()), large),
+                       (lambda: lib.mi_gemm_with_workspace(p, 1, 0, ws.data_ptr(), 1 << 28, ops.stream_ptr()), True)):
+        c.fill_(float("nan"))
+        names = launched(lambda: _lib.check(call(), "mi_gemm"))
+        assert any("wide_kernel" in k for k in names) == wide, names
+        _close("c", c, ref, magnitude, ins, torch.bfloat16)
