@@ -375,6 +375,7 @@ enum class Pass { kInference, kForward, kBackward };
 bool wide_product(const Tensor& t, int64_t rows, int64_t n, int64_t k, Pass pass) {
     const double work = 2.0 * (double)rows * (double)n * (double)k;
     if (pass == Pass::kInference ? k > 1536 || work > 1e10 : pass == Pass::kForward && work >= 1e11) return false;
+    if (std::max({rows, n, k}) > 0x7fffffff) return false;
     return t.scalar_type() != at::kFloat && rows >= 128 && n >= 32 && k >= 32 && n % 8 == 0 && k % 8 == 0;
 }
 // Short contractions into large outputs: a block spends more on its fill and its results than on products, and the library's kernels for whole
@@ -388,6 +389,8 @@ bool aligned(const Tensor& t) {        // as an operand of mi_gemm: contiguous r
     const int64_t v = t.scalar_type() == at::kFloat ? 4 : 8;
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % v == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
+// rows that the large blocks of mi_gemm reach: 128 of them within 2^31 bytes
+bool in_reach(const Tensor& t) { return t.stride(0) < (1 << 22); }
 
 void segment(mi_gemm_problem& pr, const Tensor& p, const Tensor& q, int64_t k) {
     mi_gemm_segment& s = pr.segments[pr.n_segments++];
@@ -473,7 +476,8 @@ struct Projections : Function<Projections> {
             blocks += (rows + 127) / 128 * ((w.size(0) + 127) / 128);
             fit = fit && aligned(w);
             small = small && small_product(x, rows, w.size(0), in);
-            wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward) && !thin(rows, w.size(0), in);
+            wide = wide && wide_product(x, rows, w.size(0), in, inference ? Pass::kInference : Pass::kForward) && !thin(rows, w.size(0), in) && in_reach(x2) &&
+                   in_reach(w);
         }
         if (inference && in > 512 && blocks > n * at::cuda::getDeviceProperties(x.device().index())->multiProcessorCount) wide = false;
         // What the gradients read and no more, so that the rest may be changed or freed before the backward pass: x (itself: what is
@@ -540,7 +544,8 @@ struct Projections : Function<Projections> {
             if (!again && !aligned(dy[i])) dy[i] = dy[i].contiguous();
             fit = fit && aligned(dy[i]);
             small = small && small_product(dy[i], rows, dy[i].size(1), in);
-            wide = wide && wide_product(dy[i], rows, dy[i].size(1), in, Pass::kBackward);
+            wide = wide && wide_product(dy[i], rows, dy[i].size(1), in, Pass::kBackward) && in_reach(dy[i]) && (!x.defined() || in_reach(x)) &&
+                   (!need_dx || in_reach(saved[1 + i]));
             // the forward product may have been the library's, and saved-tensor hooks may bring the weight back in another layout
             if (need_dx) fit = fit && aligned(saved[1 + i]);
         }
@@ -932,7 +937,7 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
             Tensor logits = buffer.narrow(0, 0, r).narrow(1, 0, vocab);
             // 2047 x 50257 x 1024, us, mi_gemm and library: logits 216 / 257, dh 161 / 291, dW 197 / 252
             const bool wide = wide_product(h, r, 32, h.size(1), Pass::kBackward) && 2.0 * (double)r * (double)vocab * (double)h.size(1) > 3e9 && aligned(hc) &&
-                              aligned(weight);
+                              aligned(weight) && in_reach(hc) && in_reach(weight) && ld < (1 << 22);
             if (wide && !thin(r, vocab, h.size(1))) {
                 mi_gemm_problem p = problem(logits, false, false);
                 segment(p, hc, weight, h.size(1));

@@ -579,3 +579,35 @@ def test_few_blocks_without_a_workspace(rows, ins, outs, large):
         names = launched(lambda: _lib.check(call(), "mi_gemm"))
         assert any("wide_kernel" in k for k in names) == wide, names
         _close("c", c, ref, magnitude, ins, torch.bfloat16)
+
+
+def test_lm_head_over_more_entries_than_large_blocks_reach():
+    """2^22 + 1 entries (a row of logits is longer than the blocks address): the library's products, as for any operand they do not take."""
+    rows, hidden, vocab = 128, 64, (1 << 22) + 1
+    g = torch.Generator(device=DEV).manual_seed(1)
+    h = torch.randn(rows, hidden, generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(vocab, hidden, generator=g, device=DEV) * 0.25).bfloat16().requires_grad_()
+    t = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    loss = ops.linear_cross_entropy(h, w, t, torch.ones(rows, device=DEV))[0]
+    loss.backward()
+    hd, wd = h.detach().double().requires_grad_(), w.detach().double().requires_grad_()
+    ref = torch.nn.functional.cross_entropy(hd @ wd.t(), t)
+    ref.backward()
+    assert abs(loss.item() - ref.item()) <= 1e-3 * ref.item()
+    for name, a, b in (("dh", h.grad, hd.grad), ("dw", w.grad, wd.grad)):
+        err = ((a.double() - b).norm() / b.norm()).item()
+        assert err <= 2.0 ** -7, f"{name}: {err}"          # logits and their gradient are rounded to bfloat16
+
+
+def test_projection_of_rows_that_lie_far_apart():
+    """Rows 2^22 elements apart go to the library, forward and backward, at any size of the product that is not a small one."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.zeros(128, 1 << 22, dtype=torch.bfloat16, device=DEV)[:, :4096].copy_(torch.randn(128, 4096, generator=g, device=DEV))
+    w = torch.randn(4096, 4096, generator=g, device=DEV).bfloat16().requires_grad_()
+    dy = torch.randn(128, 4096, generator=g, device=DEV).bfloat16()
+    out = []
+    names = launched(lambda: out.append(ops.linear(x, w)) or out[0].backward(dy))
+    assert not any("wide_kernel" in k or "gemm_kernel" in k for k in names), names
+    xd, wd, dyd = x.double(), w.detach().double(), dy.double()
+    _close("y", out[0].detach(), (xd @ wd.t()).cpu(), (xd.abs() @ wd.abs().t()).cpu(), 4096, torch.bfloat16)
+    _close("dw", w.grad, (dyd.t() @ xd).cpu(), (dyd.abs().t() @ xd.abs()).cpu(), 128, torch.bfloat16)
