@@ -973,7 +973,8 @@ struct LinearCrossEntropy : Function<LinearCrossEntropy> {
                     segment(p, logits, hc, r);
                     run_gemm(&p, 1, h, l);
                 } else {
-                    product = at::mm(logits.t(), hc);
+                    const bool turn = transpose_pays(r, h.size(1), vocab) && h.size(1) <= vocab && transposable(hc);
+                    product = at::mm(logits.t(), turn ? transposed(hc, l).t() : hc);
                 }
                 if (n <= chunk) dw = product;
                 else if (!dw.defined()) dw = product.to(at::kFloat);

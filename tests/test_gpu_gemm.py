@@ -611,3 +611,20 @@ def test_projection_of_rows_that_lie_far_apart():
     xd, wd, dyd = x.double(), w.detach().double(), dy.double()
     _close("y", out[0].detach(), (xd @ wd.t()).cpu(), (xd.abs() @ wd.abs().t()).cpu(), 4096, torch.bfloat16)
     _close("dw", w.grad, (dyd.t() @ xd).cpu(), (dyd.abs().t() @ xd.abs()).cpu(), 128, torch.bfloat16)
+
+
+def test_lm_head_with_a_weight_that_is_stored_transposed():
+    """The library's products; the weight gradient of 107 GFLOP with the activations transposed first."""
+    rows, hidden, vocab = 2048, 2048, 12800
+    g = torch.Generator(device=DEV).manual_seed(1)
+    h = torch.randn(rows, hidden, generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(hidden, vocab, generator=g, device=DEV) * 2 / hidden ** 0.5).bfloat16().t().requires_grad_()
+    t = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    grads = []
+    names = launched(lambda: grads.extend(torch.autograd.grad(ops.linear_cross_entropy(h, w, t, torch.ones(rows, device=DEV))[0], (h, w))))
+    assert any("transpose_kernel" in k for k in names) and not any("wide_kernel" in k for k in names), names
+    hd, wd = h.detach().double().requires_grad_(), w.detach().double().requires_grad_()
+    ref = torch.autograd.grad(torch.nn.functional.cross_entropy(hd @ wd.t(), t), (hd, wd))
+    for name, a, b in zip(("dh", "dw"), grads, ref):
+        err = ((a.double() - b).norm() / b.norm()).item()
+        assert err <= 2.0 ** -7, f"{name}: {err}"          # logits and their gradient are rounded to bfloat16
