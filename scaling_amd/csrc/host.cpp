@@ -17,8 +17,11 @@
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
+#include <hip/hip_runtime_api.h>
 #include <algorithm>
 #include <optional>
 #include <tuple>
@@ -713,6 +716,23 @@ std::tuple<Tensor, Tensor> attn_forward(const Tensor& q, const Tensor& k, const 
     return {o, lse};
 }
 
+// Whether the allocator has so many bytes without giving its cache back first: in a free block of the cache, or on the device within the process's
+// share.  (Nothing asks the device while a graph is captured, and not every allocator answers.)
+bool has_room(size_t bytes, const Tensor& like) {
+    namespace allocator = c10::hip::HIPCachingAllocator;
+    const auto device = like.device().index();
+    try {
+        size_t block = 1, free = 0, total = 0;             // not 0, which would ask the device for a first guess
+        allocator::cacheInfo(device, &block);
+        if (block >= bytes || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return true;
+        if (hipMemGetInfo(&free, &total) != hipSuccess) return true;
+        const double share = allocator::getMemoryFraction(device) * (double)total - (double)allocator::getDeviceStats(device).reserved_bytes[0].current;
+        return std::min((double)free, share) >= (double)bytes;
+    } catch (const c10::Error&) {
+        return true;
+    }
+}
+
 // dq must have the strides of q; `ws` may be undefined
 void attn_backward(const Tensor& d_o_, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& cu_q,
                    const Tensor& cu_k, const AttnOptions& opts, const Tensor& dq, const Tensor& dk, const Tensor& dv, Tensor ws) {
@@ -724,7 +744,8 @@ void attn_backward(const Tensor& d_o_, const Tensor& q, const Tensor& k, const T
     fill_args(b.fwd, q, k, v, o, lse, cu_q, cu_k, opts, l.stream);
     if (!ws.defined()) {
         const size_t least = std::max<size_t>(16, mi_attn_bwd_workspace_bytes_kv(q.size(0), k.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2)));
-        const size_t best = std::max(least, mi_attn_bwd_workspace_bytes_for(&b.fwd));
+        size_t best = std::max(least, mi_attn_bwd_workspace_bytes_for(&b.fwd));
+        if (best > least && !has_room(best, q)) best = least;
         try {
             ws = float_buffer(best, q);
         } catch (const c10::OutOfMemoryError&) {           // does with less, as it did

@@ -146,3 +146,31 @@ def test_float32_backward_with_kept_scores(nq, nkv, d, causal, lens_q, lens_k):
     assert torch.cuda.max_memory_allocated() - before > 4 * least + (32 << 20), "the kept route was not taken"
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
         assert torch.equal(a, b), f"{name}: {(a - b).abs().max().item()}"
+
+
+def test_float32_backward_in_a_program_near_its_limit():
+    """Where the room for dS is not there the pass takes the small workspace at once: nothing is thrown out of the allocator's cache, the bits stay."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, do = (torch.randn(4096, 32, 64, generator=g, device="cuda") for _ in range(2))
+    k, v = (torch.randn(4096, 32, 64, generator=g, device="cuda") for _ in range(2))
+    cu = torch.tensor([0, 4096], dtype=torch.int32, device="cuda")
+    for t in (q, k, v):
+        t.requires_grad_()
+    o = ops.attention(q, k, v, cu)
+    grads = lambda: torch.autograd.grad(o, (q, k, v), do, retain_graph=True)
+    want = grads()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (512 << 20)) / total)
+        cached = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")        # a block of the cache, for the next step
+        del cached
+        before = torch.cuda.memory_stats()
+        for _ in range(3):
+            got = grads()
+        after = torch.cuda.memory_stats()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert all(after[n] == before[n] for n in ("num_alloc_retries", "num_ooms")), (before["num_alloc_retries"], after["num_alloc_retries"])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
