@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from scaling_amd import ops
+from scaling_amd import _lib, ops
 from tests import attn_utils as U
 from tests.parity import check
 from tests.test_gpu_attention import CASES
@@ -134,16 +134,19 @@ def test_float32_backward_with_kept_scores(nq, nkv, d, causal, lens_q, lens_k):
     rand = lambda n, h: torch.randn(n, h, d, generator=g, device="cuda")
     q, k, v, do = rand(tq, nq), rand(tk, nkv), rand(tk, nkv), rand(tq, nq)
     o, lse = ops.attention_forward(q, k, v, cu_q, cu_k, causal)
-    from scaling_amd import _lib
-    least = _lib.load().mi_attn_bwd_workspace_bytes_kv(tq, tk, nq, nkv, d)
-    small = [torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty((least + 3) // 4, device="cuda")]
-    want = [t.clone() for t in ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, buffers=tuple(small))]
-    junk = torch.full((1 << 28,), float("nan"), device="cuda")   # what the kept scores are written into holds no zeros
-    del junk
-    torch.cuda.reset_peak_memory_stats()
-    before = torch.cuda.memory_allocated()
-    got = ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal)
-    assert torch.cuda.max_memory_allocated() - before > 4 * least + (32 << 20), "the kept route was not taken"
+    lib = _lib.load()
+    least = lib.mi_attn_bwd_workspace_bytes_kv(tq, tk, nq, nkv, d)
+    best = lib.mi_attn_bwd_workspace_bytes_for(ops._fill_attn_args(q, k, v, o, lse, cu_q, cu_k, causal, 1.0 / d ** 0.5))
+    room = (least + 255) // 256 * 64                       # dS lies behind what the smaller workspace holds
+    assert best > least
+    run = lambda bytes_: (torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.full(((bytes_ + 3) // 4,), float("nan"), device="cuda"))
+    small, large = run(least), run(best)
+    want = ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, buffers=small)
+    got = ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, buffers=large)
+    kept = large[3][room:]
+    assert bool((kept == kept).any()), "the kept route was not taken"
+    own = ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal)
+    assert all(torch.equal(a, b) for a, b in zip(got, own))
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
         assert torch.equal(a, b), f"{name}: {(a - b).abs().max().item()}"
 

@@ -10,6 +10,7 @@ import torch
 
 from scaling_amd import _lib, ops
 from scaling_amd.nn import ParallelSwiGLUMLP
+from tests.kernels import launched
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -24,15 +25,6 @@ def _close(name, got, ref, magnitude, k, dtype):
     bound = HALF_ULP[dtype] * ref.abs() + (k + 1) * 2.0 ** -24 * magnitude + tiny
     err = (got.double().cpu() - ref).abs()
     assert bool((err <= bound * 1.001).all()), f"{name}: {float((err / bound).max()):.2f} x the bound"
-
-
-def launched(call):
-    """Names of the kernels that a call launches."""
-    torch.cuda.synchronize()
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
-        call()
-        torch.cuda.synchronize()
-    return [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA]
 
 
 def _case(rows, ins, outs, dtype, seed):
@@ -123,7 +115,7 @@ def test_capture_after_one_call():
     """A first call outside the capture makes whatever the captured one needs, in a process that has used no library product."""
     code = """
 import torch
-from scaling_amd import _lib, ops
+from scaling_amd import ops
 for k in (2048, 2816, 3064, 3072):
     x, w = torch.ones(17, k, device="cuda", dtype=torch.bfloat16), torch.full((64, k), 0.5, device="cuda", dtype=torch.bfloat16)
     side = torch.cuda.Stream()
@@ -175,12 +167,14 @@ def test_projection_that_does_not_reach_the_loss():
     assert ops.linear(torch.empty(0, 64, device=DEV), wg[0]).shape == (0, 32)
 
 
-@pytest.mark.parametrize("rows,ins,outs", [(24, 64, (32, 16)), (2048, 512, (2048, 256))])   # matrix kernel, library products
+@pytest.mark.parametrize("rows,ins,outs", [(24, 64, (32, 16)), (2048, 512, (2048, 256)), (2048, 516, (2044, 252))])   # small and large blocks, library products
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_what_no_gradient_reads_may_change_before_the_backward_pass(rows, ins, outs, dtype):
     """As with torch.nn.functional.linear: the input where no weight is trained, the weights where the input takes no gradient."""
     print(f"case gemm frozen rows={rows} dtype={dtype}", flush=True)
     x, ws, bs, dys = _case(rows, ins, outs, dtype, 17)
+    own = any("gemm_kernel" in k or "wide_kernel" in k for k in launched(lambda: ops.linear(x.to(DEV), ws[0].to(DEV))))
+    assert own == (rows < 2048 or dtype != torch.float32 and ins % 8 == 0)
     xd, wd, dyd = x.double(), [w.double() for w in ws], [d.double() for d in dys]
     for n in (1, 2):
         def forward(xg, wg, bg):
@@ -380,7 +374,7 @@ def test_bias_and_residual_of_a_product_in_two_launches(rows, ins, outs):
         assert torch.equal(ops.linear(x, w, b, res), y + res)
 
 
-@pytest.mark.parametrize("rows,hidden,vocab", [(2047, 1024, 50257), (300, 520, 20003), (1025, 2048, 128)])
+@pytest.mark.parametrize("rows,hidden,vocab", [(2047, 1024, 50257), (300, 520, 20003), (1025, 2048, 1000), (1025, 2048, 128)])   # the last: library
 def test_lm_head_products(rows, hidden, vocab):
     """Loss and gradients of the chunked LM head over ragged vocabularies against float64."""
     g = torch.Generator(device=DEV).manual_seed(rows)
@@ -405,14 +399,47 @@ def test_ragged_extents_need_the_entry_with_a_workspace(rows, ins, outs):
     """mi_gemm takes whole vectors whatever the size of the product; the other entry takes any n of a large one, and no ragged contraction
     between operands that are both contiguous along it."""
     lib = _lib.load()
-    x, c = (torch.zeros(rows, 4104, dtype=torch.bfloat16, device=DEV) for _ in range(2))
-    w = torch.zeros(outs, 4104, dtype=torch.bfloat16, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(ins)
+    x, w = (torch.randn(n, 4104, generator=g, device=DEV).bfloat16() for n in (rows, outs))
+    c = torch.full((rows, 4104), 7.0, dtype=torch.bfloat16, device=DEV)
     p = _lib.MiGemmProblem(c=c.data_ptr(), ldc=4104, n_segments=1, m=rows, n=outs)
     p.segments[0] = _lib.MiGemmSegment(x.data_ptr(), w.data_ptr(), 4104, 4104, ins)
-    stream = torch.cuda.current_stream().cuda_stream
-    assert lib.mi_gemm(p, 1, 0, stream) != 0
-    assert (lib.mi_gemm_with_workspace(p, 1, 0, None, 0, stream) == 0) == (ins % 8 == 0)
+    assert lib.mi_gemm(p, 1, 0, ops.stream_ptr()) != 0
+    assert (lib.mi_gemm_with_workspace(p, 1, 0, None, 0, ops.stream_ptr()) == 0) == (ins % 8 == 0)
     torch.cuda.synchronize()
+    if ins % 8 == 0:
+        xd, wd = x[:, :ins].double(), w[:, :ins].double()
+        _close("c", c[:, :outs], (xd @ wd.t()).cpu(), (xd.abs() @ wd.abs().t()).cpu(), ins, torch.bfloat16)
+    assert bool((c[:, outs if ins % 8 == 0 else 0:] == 7).all())
+
+
+# results of whole and ragged rows: blocks of 128 and 256, one launch, two launches by rows and by columns, and contractions that are split;
+# with bias and residual (a wider matrix, or the result itself), whatever lies behind a row of the result left as it is
+@pytest.mark.parametrize("rows,ins,outs", [(513, 8200, 520), (264, 16392, 517), (512, 1032, 4101), (2050, 2056, 5633), (2047, 520, 16903), (4097, 520, 4101), (130, 4104, 4099)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_results_bias_and_residual_of_ragged_rows(rows, ins, outs, dtype):
+    print(f"case wide epilogue rows={rows} in={ins} out={outs} dtype={dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(outs)
+    lib, code, ld = _lib.load(), ops.dtype_code(dtype), (outs + 15) // 8 * 8
+    x, w, b, res = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((rows, ins), (outs, ins), (outs,), (rows, ld)))
+    xd, wd = x.double(), w.double()
+    ref, magnitude = xd @ wd.t() + b.double(), xd.abs() @ wd.abs().t() + b.double().abs()
+
+    def run(c, add):
+        p = _lib.MiGemmProblem(c=c.data_ptr(), ldc=ld, n_segments=1, m=rows, n=outs, bias=b.data_ptr(), add=None if add is None else add.data_ptr(), ldadd=ld)
+        p.segments[0] = _lib.MiGemmSegment(x.data_ptr(), w.data_ptr(), ins, ins, ins)
+        bytes_ = lib.mi_gemm_workspace_bytes(p, 1, code)
+        ws = torch.full((max(bytes_, 16) // 4,), float("nan"), device=DEV)
+        _lib.check(lib.mi_gemm_with_workspace(p, 1, code, ws.data_ptr(), bytes_, ops.stream_ptr()), "mi_gemm_with_workspace")
+        return bytes_ > 0
+
+    c, d, e = torch.full((rows, ld), 7.0, dtype=dtype, device=DEV), torch.full((rows, ld), 7.0, dtype=dtype, device=DEV), res.clone()
+    split = [run(c, None), run(d, res), run(e, e)]
+    assert split == [(rows, ins, outs) in ((513, 8200, 520), (264, 16392, 517), (130, 4104, 4099))] * 3
+    _close("product", c[:, :outs], ref.cpu(), magnitude.cpu(), ins, dtype)
+    assert torch.equal(d[:, :outs], c[:, :outs] + res[:, :outs]) and torch.equal(e[:, :outs], d[:, :outs])   # the rounded product, then the sum
+    assert bool((c[:, outs:] == 7).all() and (d[:, outs:] == 7).all()) and torch.equal(e[:, outs:], res[:, outs:])
+
 
 
 # contractions that end inside a 32-bit word and at either end of a vector, of an operand contiguous along them; rows at the end of a block
