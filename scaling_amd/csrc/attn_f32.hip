@@ -22,9 +22,9 @@
 //     with F32Tile::f(row), which spreads the 16 rows that one pass of a 128-bit read touches over all banks.
 // One wavefront per workgroup with synchronous staging, the earlier form of these kernels, kept three of the four SIMDs
 // of a compute unit busy at most and each of them waiting for its own loads: 19.1 ms for a forward + backward at 32 / 8
-// heads of 128 and 4096 causal tokens (25 TFLOP/s).  With the backward as dK/dV and a dQ kernel that forms S and dP again 5.3 ms (forward
-// 1.14, dK/dV 2.62, dQ 1.80); where the products are a sixteenth of the 16-bit rate a byte of memory costs a sixteenth as much beside
-// them, so dK/dV leaves dS in a workspace and dQ reads it: 4.25 ms, 113 TFLOP/s (dK/dV 2.75, dQ 0.62).
+// heads of 128 and 4096 causal tokens (25 TFLOP/s).  With the backward as dK/dV and a dQ kernel that forms S and dP again 5.28 ms, 91 TFLOP/s (forward
+// 1.08, delta 0.02, dK/dV 2.49, dQ 1.73 under the profiler, 5.33 together); where the products are a sixteenth of the 16-bit rate a byte of memory costs a
+// sixteenth as much beside them, so dK/dV leaves dS in a workspace and dQ reads it: 4.24 ms, 113 TFLOP/s (dK/dV 2.60, dQ 0.58, 4.29 together).
 #include "attn_common.h"
 
 namespace {

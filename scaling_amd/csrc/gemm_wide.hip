@@ -15,7 +15,7 @@
 //   * reads and loads are spread evenly between the products (sched_barrier pins the order): with one wavefront per SIMD a clump of more
 //     than three instructions between two products is a hole in the matrix pipe.
 // kmajor operands are read by LDS transpose reads from tiles in memory order, so all three layouts run at the same rate: 8192^3 bf16
-// 0.70 / 0.71 / 0.71 ms (x W^T, dy W, dy^T x), the library 0.68 / 0.79 / 0.91 on the same box.
+// 0.70 / 0.71 / 0.71 ms (x W^T, dy W, dy^T x), the library 0.67 / 0.78 / 0.90 on the same box (another box: 0.71 / 0.72 / 0.73, 0.69 / 0.79 / 0.92).
 //
 // v_mfma_f32_16x16x32 operands, lane = 16 g + l:  A: row l, k = 8 g .. + 7;  B: column l, the same k;  C / D: column l, rows 4 g .. + 3.
 // A = Q (output features), B = P (output rows): a lane holds four consecutive features of one output row.

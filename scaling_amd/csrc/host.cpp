@@ -6,8 +6,8 @@
 // torch.cuda.current_stream() per launch, a Python autograd node per operation whose backward waits for the interpreter).
 // Here an operation costs its allocations and launches, and a backward pass runs without the interpreter.
 //
-// Linear projections run on the library product (at::mm) or, where they are too small to fill the chip, on mi_gemm; see
-// small_product for the line between the two.
+// Linear projections run on mi_gemm or on the library product (at::mm); see small_product, long_chain, wide_product and thin for the lines
+// between the two.
 #include <torch/extension.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/graph_task.h>
@@ -425,10 +425,10 @@ Tensor bias_gradient(const Tensor& dy) {
 // Weight gradients dW = dY^T X contract over the rows of both operands, which is the library's slowest layout for 16-bit types; with one of
 // them transposed first it runs a fifth faster, which pays for the transposed copy once the other side is wide.  us, product as it is /
 // with X or dY transposed + the copy:
-//   8192 x 4096 -> 14336   967 / 767 + 24        8192 x 14336 -> 4096 (dY)   972 / 755 + 24
-//   8192 x 4096 -> 4096    239 / 197 + 24        4096 x 2048 -> 8192         120 / 104 + 7
-//   4096 x 2048 -> 32000   509 / 410 + 7
-// and not where the copy or the product is small: 4084 x 1024 -> 4096 55 / 51 + 5, 2047 x 1024 -> 50257 271 / 256 + 5.
+//   8192 x 4096 -> 14340   972 / 732 + 24        8192 x 14340 -> 4096 (dY)   1006 / 766 + 24
+//   8192 x 4096 -> 4100    424 / 261 + 24        4096 x 2048 -> 8196          169 / 155 + 7
+//   4096 x 2048 -> 32004   474 / 409 + 6         3001 x 8196 -> 2056 (dY)     165 / 140 + 7
+// and not where the copy or the product is small: 4084 x 1024 -> 4096 55 / 51 + 5, 2047 x 1024 -> 50257 271 / 256 + 5 (2047 x 2048 -> 50257 471 / 476 + 6).
 bool transpose_pays(int64_t rows, int64_t in, int64_t out) {
     return 2.0 * (double)rows * (double)in * (double)out >= 1e11 && std::max(in, out) >= 4096 && std::min(in, out) >= 2048;
 }

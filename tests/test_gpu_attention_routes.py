@@ -177,3 +177,28 @@ def test_float32_backward_in_a_program_near_its_limit():
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert all(after[n] == before[n] for n in ("num_alloc_retries", "num_ooms")), (before["num_alloc_retries"], after["num_alloc_retries"])
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_float32_step_with_kept_scores_in_a_graph():
+    """The room for dS comes from the graph's own pool: replays between eager steps give the eager bits."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v, do = (torch.randn(1101, 32, 64, generator=g, device="cuda") for _ in range(4))
+    cu = torch.tensor([0, 600, 1101], dtype=torch.int32, device="cuda")
+    for t in (q, k, v):
+        t.requires_grad_()
+    step = lambda: torch.autograd.grad(ops.attention(q, k, v, cu), (q, k, v), do)
+    want = step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(step(), want))
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -655,3 +655,27 @@ def test_lm_head_with_a_weight_that_is_stored_transposed():
     for name, a, b in zip(("dh", "dw"), grads, ref):
         err = ((a.double() - b).norm() / b.norm()).item()
         assert err <= 2.0 ** -7, f"{name}: {err}"          # logits and their gradient are rounded to bfloat16
+
+
+def test_gradients_with_workspaces_in_a_graph():
+    """A split product of one projection and a chain with a launch of its own, captured: every replay, with eager work that reuses the allocator
+    between them, gives the eager bits."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, w, dy = (torch.randn(*s, generator=g, device=DEV).bfloat16() for s in ((257, 1024), (16384, 1024), (257, 16384)))
+    x.requires_grad_(), w.requires_grad_()
+    step = lambda: torch.autograd.grad(ops.linear(x, w), (x, w), dy)
+    want = step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(step(), want))
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
