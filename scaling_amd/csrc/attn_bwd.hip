@@ -1,6 +1,7 @@
 // Attention backward for gfx950 (bf16 MFMA, fp32 softmax recomputation from the saved log-sum-exp).
 //
-// Long contexts: three kernels (four with fewer than 8 KV heads; short contexts: attn_short.h), no atomics, fixed summation order (bit-reproducible):
+// Long contexts: two launches (three with fewer than 8 KV heads; short contexts: attn_short.h), no atomics, fixed summation order (bit-reproducible).
+// The second launch holds the blocks of 2 and of 3:
 //   1. delta[h][t] = sum_d dO[t][h][d] * O[t][h][d]
 //   2. dK/dV: a workgroup owns 128 keys of one KV head (K and V rows stay in LDS), loops over the query
 //      heads of the group and over 64-query tiles staged in LDS:
@@ -49,6 +50,19 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_delta_kernel(const AttnPara
     if (ok && c == 0) p.delta[(int64_t)h * p.total_q + t] = acc;
 }
 
+// LDS of a backward workgroup, which is a dK / dV block or a dQ block: arrays of the kernel's own (as members of one struct
+// the same code had ten more waits in the dV / dK products of a step and dK / dV took 3 % longer).
+template <int D> struct BwdShared {
+    static constexpr int kStageBytes = 8 * LdsTile<D>::kBytes;        // dK/dV: K, V (two tiles each), Q, dO (two stages each); dQ: four stages of K and V
+    static constexpr int kExchangeBytes = 8 * 16 * (D / 32) * 64 * 4; // dK/dV: one accumulator set (dK or dV) of each of the 8 wavefronts
+    static constexpr int kTileBytes = kStageBytes > kExchangeBytes ? kStageBytes : kExchangeBytes;
+    char* tiles;
+    float (*lse)[64];
+    float (*delta)[64];
+    int* range;
+    int* lpt;                             // work estimates and hand-out order of the blocks (packed documents)
+};
+
 // ---------------------------------------------------------------------------------------------
 // 2. dK / dV
 // ---------------------------------------------------------------------------------------------
@@ -57,10 +71,8 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_delta_kernel(const AttnPara
 // (32 of the 64 queries staged per iteration), so the pair (w, w + 4) accumulates the same dK / dV
 // rows and is summed once at the end.  The first four wavefronts stage Q, the last four dO; the staged
 // tiles are double buffered (one barrier per iteration).
-// __launch_bounds__(512, 2): the second argument is wavefronts per SIMD, i.e. the two that one 512-thread workgroup
-// brings; the kernel takes 250 - 254 of the 256 registers each of them can have (no AGPRs, no scratch).
 template <int D, bool DROP, bool SPLIT>
-__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_kernel(const AttnParams p) {
+__device__ __forceinline__ void dkdv_block(const AttnParams& p, const BwdShared<D>& sh, int block) {
     constexpr int BNK = 128;              // keys per workgroup
     constexpr int BQ = 64;                // queries per tile
     constexpr int KS = D / 16;
@@ -69,15 +81,12 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_kernel(const AttnParams 
     constexpr int RB = Tile::RB;
     constexpr int TILE = Tile::kBytes;    // one 64-token tile
     constexpr int IPW = Tile::kInstrs / 4;   // direct-load instructions per loader wavefront and 64-token tile
-    constexpr int STAGE_BYTES = 4 * TILE + 4 * TILE;  // K, V (two tiles each) + Q, dO (two stages each)
-    constexpr int RED_BYTES = 8 * 16 * DT * 64 * 4;   // the pair exchange: one accumulator set (dK or dV) of each of the 8 wavefronts
-    constexpr int SMEM_BYTES = STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES;
 
-    __shared__ __attribute__((aligned(1024))) char smem[SMEM_BYTES];
-    __shared__ __attribute__((aligned(16))) float lse_lds[2][BQ];
-    __shared__ __attribute__((aligned(16))) float delta_lds[2][BQ];
-    __shared__ int range_lds[16];
-    __shared__ int lpt_lds[2 * kLptMax];  // work estimates and hand-out order of the key blocks (packed documents)
+    char* smem = sh.tiles;                // K, V (two tiles each) + Q, dO (two stages each), then the pair exchange
+    float(*lse_lds)[BQ] = sh.lse;
+    float(*delta_lds)[BQ] = sh.delta;
+    int* range_lds = sh.range;
+    int* lpt_lds = sh.lpt;
     // The streamed tiles come first: with the stage index a compile-time constant (the tile loop is unrolled by two)
     // their LDS addresses are a per-lane register plus an immediate offset, which reaches 64 KB.
     char* q_t = smem;                     // [2 stages]
@@ -98,12 +107,12 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_kernel(const AttnParams 
     const int n_groups = p.nkv * p.hsplit;
     int kb_rank, group;
     if ((n_groups & 7) == 0) {
-        const int work = xcd_remap(blockIdx.x, gridDim.x);
+        const int work = xcd_remap(block, nkb * n_groups);
         kb_rank = work % nkb;
         group = work / nkb;
     } else {
-        kb_rank = blockIdx.x / n_groups;
-        group = blockIdx.x - kb_rank * n_groups;
+        kb_rank = block / n_groups;
+        group = block - kb_rank * n_groups;
     }
     int kb = block_for_rank(kb_rank, nkb, p.n_docs, p.across_k, false);   // key blocks with the most queries first
     if (p.lpt_k) {                        // documents of different lengths: by the work each key block really has
@@ -315,7 +324,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_kernel(const AttnParams 
     // One exchange: the second wavefront of a pair hands its dK to the first and receives the first's dV, so each of them
     // sums and stores one of the two tensors (half the LDS traffic and half the stores per wavefront of a one-way sum).
     constexpr int kAccFloats = 16 * DT * 64;          // one accumulator set of one wavefront
-    static_assert(2 * 4 * kAccFloats * 4 <= SMEM_BYTES, "the exchange reuses the tile stages");
+    static_assert(2 * 4 * kAccFloats * 4 <= BwdShared<D>::kTileBytes, "the exchange reuses the tile stages");
     float* red_k = reinterpret_cast<float*>(smem) + (size_t)kgp * kAccFloats + lane;
     float* red_v = reinterpret_cast<float*>(smem) + (size_t)(4 + kgp) * kAccFloats + lane;
     {
@@ -449,7 +458,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_reduce_kernel(const At
 // token-major tile read both as row operand and transposed), the last four stage V.  Double-buffered
 // LDS, one barrier per 64-key tile.
 template <int D, bool DROP, bool SPLIT>
-__global__ __launch_bounds__(512, 2) void attn_bwd_dq_kernel(const AttnParams p) {
+__device__ __forceinline__ void dq_block(const AttnParams& p, const BwdShared<D>& sh, int block) {
     constexpr int BM = 256;
     constexpr int BN = 64;
     constexpr int KS = D / 16;
@@ -460,10 +469,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_kernel(const AttnParams p)
     constexpr int TILE = Tile::kBytes;
     constexpr int IPW = Tile::kInstrs / 4;   // direct-load instructions per loader wavefront and tile
 
-    __shared__ __attribute__((aligned(1024))) char k_t[NS * TILE];   // row operand and transposed operand
-    __shared__ __attribute__((aligned(1024))) char v_t[NS * TILE];   // row operand
-    __shared__ int range_lds[16];
-    __shared__ int lpt_lds[2 * kLptMax];  // work estimates and hand-out order of the query blocks (packed documents)
+    static_assert(2 * NS * TILE <= BwdShared<D>::kTileBytes, "two rings");
+    char* k_t = sh.tiles;                 // row operand and transposed operand
+    char* v_t = sh.tiles + NS * TILE;     // row operand
+    int* range_lds = sh.range;
+    int* lpt_lds = sh.lpt;
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -471,7 +481,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_kernel(const AttnParams p)
 
     const int nqb = (p.total_q + BM - 1) / BM;
     int head, q_rank;
-    head_and_rank(blockIdx.x, p.nq, head, q_rank);
+    head_and_rank(block, p.nq, head, q_rank);
     const int kvh = head / p.n_rep;
     int qb = block_for_rank(q_rank, nqb, p.n_docs, p.across_q, true);
     if (p.lpt_q) {                        // documents of different lengths: by the work each query block really has
@@ -670,6 +680,25 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dq_kernel(const AttnParams p)
     }
 }
 
+// Both in one launch: blocks [0, n_dkdv) of the grid are dK / dV blocks, the others dQ blocks.  Both kinds take a compute unit each and
+// neither number is a multiple of 256, so as launches of their own each of them ended with compute units that had nothing left to do; now
+// the dQ blocks start where dK / dV blocks, the longer ones, have ended.  One launch each / together, us with delta, head_dim 128, bf16:
+//   8192 tokens 32 / 8 heads 1704 / 1687      the same in documents of 256 - 2048 380 / 359      4 x 2048, 16 / 16 279 / 272
+//   2445, 32 / 32 234 / 203                   4397, 16 / 2, no mask 830 / 621                   4 x 538, 32 / 8 of 64, no mask 129 / 95
+// The second argument of __launch_bounds__ is wavefronts per SIMD: the two that one 512-thread workgroup brings, where the
+// kernel takes 253 of the 256 registers each of them can have (no AGPRs, no scratch), or two workgroups' at head_dim 32.
+template <int D, bool DROP, bool SPLIT>
+__global__ __launch_bounds__(512, D == 32 ? 4 : 2) void attn_bwd_kernel(const AttnParams p, int n_dkdv) {
+    __shared__ __attribute__((aligned(1024))) char tiles[BwdShared<D>::kTileBytes];
+    __shared__ __attribute__((aligned(16))) float lse[2][64];
+    __shared__ __attribute__((aligned(16))) float delta[2][64];
+    __shared__ int range[16];
+    __shared__ int lpt[2 * kLptMax];
+    const BwdShared<D> sh{tiles, lse, delta, range, lpt};
+    if ((int)blockIdx.x < n_dkdv) dkdv_block<D, DROP, SPLIT>(p, sh, blockIdx.x);
+    else dq_block<D, DROP, SPLIT>(p, sh, blockIdx.x - n_dkdv);
+}
+
 template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) {
     const int stages = flags & (MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ);
     const bool split = (flags & MI_ATTN_SPLIT_P) != 0;     // accuracy mode (no dropout: checked by the entry point)
@@ -682,26 +711,20 @@ template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) 
         int rc = mi_check_launch("attn_bwd_delta");
         if (rc != MI_OK) return rc;
     }
-    if (all || (stages & MI_ATTN_BWD_DKDV)) {
-        const int64_t grid = (((int64_t)p.total_k + 127) / 128) * p.nkv * p.hsplit;
-        if (split) attn_bwd_dkdv_kernel<D, false, true><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        else if (p.drop_thr != 0) attn_bwd_dkdv_kernel<D, true, false><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        else attn_bwd_dkdv_kernel<D, false, false><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        int rc = mi_check_launch("attn_bwd_dkdv");
+    const bool dkdv = all || (stages & MI_ATTN_BWD_DKDV) != 0, dq = all || (stages & MI_ATTN_BWD_DQ) != 0;
+    if (dkdv || dq) {
+        const int64_t n_dkdv = dkdv ? (((int64_t)p.total_k + 127) / 128) * p.nkv * p.hsplit : 0;
+        const int64_t grid = n_dkdv + (dq ? (((int64_t)p.total_q + 255) / 256) * p.nq : 0);
+        if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+        const auto kernel = split ? attn_bwd_kernel<D, false, true> : p.drop_thr != 0 ? attn_bwd_kernel<D, true, false> : attn_bwd_kernel<D, false, false>;
+        kernel<<<dim3((unsigned)grid), dim3(512), 0, st>>>(p, (int)n_dkdv);
+        const int rc = mi_check_launch("attn_bwd");
         if (rc != MI_OK) return rc;
-        if (p.hsplit > 1) {
-            const int64_t n = (int64_t)p.total_k * p.nkv * (D / 8);
-            attn_bwd_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>(p);
-            rc = mi_check_launch("attn_bwd_dkdv_reduce");
-            if (rc != MI_OK) return rc;
-        }
     }
-    if (all || (stages & MI_ATTN_BWD_DQ)) {
-        const int64_t grid = (((int64_t)p.total_q + 255) / 256) * p.nq;
-        if (split) attn_bwd_dq_kernel<D, false, true><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        else if (p.drop_thr != 0) attn_bwd_dq_kernel<D, true, false><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        else attn_bwd_dq_kernel<D, false, false><<<dim3((unsigned)grid), dim3(512), 0, st>>>(p);
-        return mi_check_launch("attn_bwd_dq");
+    if (dkdv && p.hsplit > 1) {
+        const int64_t n = (int64_t)p.total_k * p.nkv * (D / 8);
+        attn_bwd_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>(p);
+        return mi_check_launch("attn_bwd_dkdv_reduce");
     }
     return MI_OK;
 }

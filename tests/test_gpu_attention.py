@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from scaling_amd import ops
+from scaling_amd import _lib, ops
 from tests import attn_utils as U
 from tests.golden import known_answers as KA
 from tests.parity import check
@@ -406,6 +406,34 @@ def test_attention_is_bit_reproducible_and_gqa_equals_repeated_heads():
         lse_ref.append(torch.logsumexp(sc, 0))
     got = lse1[1, [0, 99, 100, 319]].double().cpu()
     assert torch.allclose(got, torch.stack(lse_ref), atol=2e-3)
+
+
+# ends of key and query blocks that do not coincide, one block of either kind, groups that are split over workgroups (their number
+# of dK / dV blocks is no multiple of 8), keys without queries, and the orders of a packed batch
+@pytest.mark.parametrize("q_lens,k_lens,nq,nkv,d,causal,precise", [
+    ((700,), (700,), 8, 8, 128, True, False), ((1,), (1,), 1, 1, 64, True, False), ((257,), (129,), 6, 3, 96, False, False),
+    ((300, 1, 555, 30), (300, 1, 555, 30), 8, 2, 128, True, False), ((513,), (1025,), 12, 12, 32, True, False),
+    ((260, 130), (0, 390), 4, 1, 64, False, False), ((385, 385), (385, 385), 16, 16, 64, True, True),
+])
+def test_backward_blocks_in_one_launch_equal_launches_of_their_own(q_lens, k_lens, nq, nkv, d, causal, precise):
+    """dK / dV and dQ blocks share a launch: the same bits as from one launch of either kind (flags 16: delta, 32: dK / dV, 64: dQ)."""
+    g = torch.Generator().manual_seed(17)
+    tq, tk = sum(q_lens), sum(k_lens)
+    q, do = (torch.randn(tq, nq, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    k, v = (torch.randn(tk, nkv, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    cu_q, cu_k = (torch.tensor([0] + list(x), dtype=torch.int32).cumsum(0).int().to(DEV) for x in (q_lens, k_lens))
+    o, lse = ops.attention_forward(q, k, v, cu_q, cu_k, causal, precise=precise)
+    words = _lib.load().mi_attn_bwd_workspace_bytes_kv(tq, tk, nq, nkv, d) // 4
+
+    def run(flag_sets):
+        bufs = tuple(torch.full_like(t, float("nan")) for t in (q, k, v)) + (torch.full((words,), float("nan"), device=DEV),)
+        for flags in flag_sets:
+            ops.attention_backward(do, q, k, v, o, lse, cu_q, cu_k, causal, flags=flags, buffers=bufs, precise=precise)
+        return bufs[:3]
+
+    joint, single = run([16 | 32 | 64]), run([16, 32, 64])
+    for name, a, b in zip(("dq", "dk", "dv"), joint, single):
+        assert not torch.isnan(a).any() and torch.equal(a, b), name
 
 
 def test_attention_strided_views_of_fused_qkv():
