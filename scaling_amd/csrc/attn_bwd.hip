@@ -699,16 +699,19 @@ __global__ __launch_bounds__(512, D == 32 ? 4 : 2) void attn_bwd_kernel(const At
     else dq_block<D, DROP, SPLIT>(p, sh, blockIdx.x - n_dkdv);
 }
 
+template <int D> int launch_delta(const AttnParams& p, hipStream_t st) {
+    const int64_t blocks = ((int64_t)p.total_q * p.nq * 16 + kThreads - 1) / kThreads;
+    if (blocks > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+    attn_bwd_delta_kernel<D><<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(p);
+    return mi_check_launch("attn_bwd_delta");
+}
+
 template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) {
     const int stages = flags & (MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ);
     const bool split = (flags & MI_ATTN_SPLIT_P) != 0;     // accuracy mode (no dropout: checked by the entry point)
     const bool all = stages == 0;
     if (all || (stages & MI_ATTN_BWD_DELTA)) {
-        const int64_t rows = (int64_t)p.total_q * p.nq;
-        const int64_t blocks = (rows * 16 + kThreads - 1) / kThreads;
-        if (blocks > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
-        attn_bwd_delta_kernel<D><<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(p);
-        int rc = mi_check_launch("attn_bwd_delta");
+        const int rc = launch_delta<D>(p, st);
         if (rc != MI_OK) return rc;
     }
     const bool dkdv = all || (stages & MI_ATTN_BWD_DKDV) != 0, dq = all || (stages & MI_ATTN_BWD_DQ) != 0;
@@ -729,16 +732,30 @@ template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) 
     return MI_OK;
 }
 
-// dQ first: it leaves delta for dK / dV
-template <int D> int launch_short(const AttnParams& p, hipStream_t st) {
+template <int D> int launch_short(const AttnParams& p, ShortBwd route, hipStream_t st) {
     const int64_t grid_q = ((int64_t)p.total_q + kShortRows - 1) / kShortRows * p.nq;
     const int64_t grid_k = ((int64_t)p.total_k + kShortRows - 1) / kShortRows * p.nkv * p.hsplit;
-    if (grid_q > 0x7fffffffLL || grid_k > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
-    attn_short_dq_kernel<D><<<dim3((unsigned)grid_q), dim3(64 * kShortWaves), 0, st>>>(p);
-    int rc = mi_check_launch("attn_short_dq");
-    if (rc != MI_OK) return rc;
-    attn_short_dkdv_kernel<D><<<dim3((unsigned)grid_k), dim3(64 * kShortWaves), 0, st>>>(p);
-    rc = mi_check_launch("attn_short_dkdv");
+    if (grid_q + grid_k > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+    const dim3 block(64 * kShortWaves);
+    int rc = MI_OK;
+    if (D > 64 && route == ShortBwd::kApart) {
+        if constexpr (D > 64) attn_short_dq_kernel<D><<<dim3((unsigned)grid_q), block, 0, st>>>(p);
+        rc = mi_check_launch("attn_short_dq");
+        if (rc != MI_OK) return rc;
+        attn_short_bwd_kernel<D, false><<<dim3((unsigned)grid_k), block, 0, st>>>(p, (int)grid_k);
+    } else {
+        // delta inside the dK / dV blocks, or a launch of its own in front: that costs 4 us, forming it anew for every key block a tenth of
+        // the time of a chain (queries of a document x query heads of a block).  Inside / in front, us, bf16, 4 heads, chains of 512 | 1024 | 1626 |
+        // 2600:  32 features 7.4 / 8.6 | 11.3 / 11.5 | 17.3 / 16.1 | 26.3 / 22.9     64 features 10.9 / 12.1 | 17.4 / 16.8 | 27.4 / 24.9 | 41.4 / 35.7
+        //        128 features 16.7 / 16.1 | 25.5 / 22.8 | 37.5 / 32.3
+        const int64_t chain = (int64_t)p.total_q / p.n_docs * (p.n_rep / p.hsplit);
+        const bool own_delta = chain < (D <= 64 ? 1024 : 512);
+        if (!own_delta) rc = launch_delta<D>(p, st);
+        if (rc != MI_OK) return rc;
+        const auto kernel = own_delta ? attn_short_bwd_kernel<D, true> : attn_short_bwd_kernel<D, false>;
+        kernel<<<dim3((unsigned)(grid_k + grid_q)), block, 0, st>>>(p, (int)grid_k);
+    }
+    rc = mi_check_launch("attn_short_bwd");
     if (rc != MI_OK || p.hsplit == 1) return rc;
     const int64_t n = (int64_t)p.total_k * p.nkv * (D / 8);
     attn_bwd_dkdv_reduce_kernel<D><<<dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>(p);
@@ -794,12 +811,13 @@ int MI_ENTRY(mi_attn_bwd_impl)(const mi_attn_bwd_args* b) {
     p.delta = (float*)b->workspace;
     p.unrotate = a->rotary_cos == nullptr ? 0 : (a->rotary_interleaved ? 2 : 1);
     mi_set_head_split(a, b, &p);
-    if (mi_attn_is_short(a, true) && !(a->flags & (MI_ATTN_SPLIT_P | MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ)) && p.drop_thr == 0) {
+    const ShortBwd route = mi_attn_bwd_short(a, p.hsplit);
+    if (route != ShortBwd::kNo && !(a->flags & (MI_ATTN_SPLIT_P | MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ)) && p.drop_thr == 0) {
         switch (a->head_dim) {
-            case 32: return launch_short<32>(p, (hipStream_t)a->stream);
-            case 64: return launch_short<64>(p, (hipStream_t)a->stream);
-            case 96: return launch_short<96>(p, (hipStream_t)a->stream);
-            default: return launch_short<128>(p, (hipStream_t)a->stream);
+            case 32: return launch_short<32>(p, route, (hipStream_t)a->stream);
+            case 64: return launch_short<64>(p, route, (hipStream_t)a->stream);
+            case 96: return launch_short<96>(p, route, (hipStream_t)a->stream);
+            default: return launch_short<128>(p, route, (hipStream_t)a->stream);
         }
     }
     {                                                                                               // dQ: 256-query blocks

@@ -521,7 +521,7 @@ int MI_ENTRY(mi_attn_fwd_impl)(const mi_attn_args* a) {
         if (!mi_aligned16(a->q_rot_out)) return mi_fail(MI_E_ALIGN, "attn_fwd: q_rot_out must be 16-byte aligned");
         p.q_rot = (elem_t*)a->q_rot_out;
     }
-    if (mi_attn_is_short(a, false) && !(a->flags & MI_ATTN_SPLIT_P) && p.drop_thr == 0) {
+    if (mi_attn_fwd_is_short(a) && !(a->flags & MI_ATTN_SPLIT_P) && p.drop_thr == 0) {
         switch (a->head_dim) {
             case 32: return launch_short<32>(p, rot, q_only, (hipStream_t)a->stream);
             case 64: return launch_short<64>(p, rot, q_only, (hipStream_t)a->stream);

@@ -7,7 +7,7 @@
 // LDS at the end, in a fixed order.  A document of 512 tokens is a chain of at most four tiles.  The mask interval of a row comes from one
 // load of the cumulative lengths and a search in registers.
 // The price is operand traffic: a tile serves 32 rows instead of 128 or 256, so long contexts stay with the tiled kernels
-// (see mi_attn_is_short).
+// (see mi_attn_fwd_is_short and mi_attn_bwd_short).
 #pragma once
 #include "attn_common.h"
 
@@ -66,17 +66,18 @@ __device__ __forceinline__ void short_tiles(int lo, int hi, int& wmin, int& wmax
     n_tiles = __builtin_amdgcn_readfirstlane(any ? (wmax - t0 + 31) / 32 : 0);
 }
 
-// One wavefront's two tiles of 32 tokens, in STAGES stages.  The chains are short, so what hides the loads is the other workgroups of the
+// One wavefront's two (three) tiles of 32 tokens, in STAGES stages.  The chains are short, so what hides the loads is the other workgroups of the
 // compute unit: one stage (8192 tokens x 32 heads of 128 in documents of 512: forward 240 us with two, 137 with one), except for dK / dV
 // of 96 and 128 features, whose registers leave room for one workgroup anyway.
-template <int D, int STAGES = 1> struct ShortStages {
+template <int D, int STAGES = 1, int TILES = 2> struct ShortStages {
     using Tile = LdsTile<D>;
     static constexpr int kTile = 32 * Tile::RB, kLoads = Tile::kInstrs / 2;
-    static constexpr int kBytes = 2 * STAGES * kTile;
+    static constexpr int kBytes = TILES * STAGES * kTile;
     static constexpr int kSmem = kShortWaves * kBytes;
     char* base;
-    __device__ __forceinline__ char* first(int buf = 0) const { return base + buf * 2 * kTile; }
-    __device__ __forceinline__ char* second(int buf = 0) const { return base + buf * 2 * kTile + kTile; }
+    __device__ __forceinline__ char* first(int buf = 0) const { return base + buf * TILES * kTile; }
+    __device__ __forceinline__ char* second(int buf = 0) const { return base + buf * TILES * kTile + kTile; }
+    __device__ __forceinline__ char* third(int buf = 0) const { return base + buf * TILES * kTile + 2 * kTile; }
     // Before a stage is loaded again its reads must have returned.
     static __device__ __forceinline__ void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 };
@@ -135,44 +136,63 @@ template <int D> __device__ __forceinline__ void short_write(elem_t* row, const 
         *reinterpret_cast<uint2*>(row + 32 * dt) = make_uint2(pack_elem2(x[dt][0] * scale, x[dt][1] * scale), pack_elem2(x[dt][2] * scale, x[dt][3] * scale));
 }
 
-// Host side: whether a call goes to these kernels, by its workgroups of 32 rows (rows / 32 x query heads).  A compute unit holds eight of them up
-// to 64 features; above, two in the forward pass and one of dK / dV.  The tiled kernels wait for the longest chain of a workgroup, which
-// is what these kernels shorten; they gain where that chain runs alone: few workgroups, and causal documents, whose last rows have
-// twice the average work.  They lose where the tiled kernels have work for every compute unit all along, and the backward pass keeps that
-// up longer with grouped heads (`group` query heads per dK / dV workgroup lengthen the tiled chain).  Ragged documents
-// share tiled workgroups, which then walk the masked tiles of both; documents that are whole blocks of 256 rows cost the tiled
-// kernels nothing, unless there are so few that the chain of one dominates.  Short / tiled, at 512 | 1024 | 1536 | 2048 workgroups:
-//   forward, 64 features:   one causal document .33 - .49 | .37 - .51 | .53 - .64 | .60 - .70     ragged, mean 100 - 800 | | .59 - .80 | .61 - .86
-//                           not causal .41 - .58 | .62 - .73 | .90 - .96 | 1.06 - 1.18            documents of 512 .47 | .70 - .78 | | .91 - 1.06
-//   forward, 128 features:  causal .38 - .53 | .51 - .84 | .72 - 1.06 | .91 - 1.2      not causal .50 - .78 | .87 - 1.10 | 1.3 | 1.5
-//   backward, 64 features:  one causal document .48 - .59 | .56 - .62 | .66 - .76 | .66 - .92     ragged | .57 - .83 | .64 - .88 | .67 - .92
-//                           not causal .57 - .70 | .67 - 1.0 | .79 - .95 | .86 - 1.22             documents of 512 | .96 - 1.03 | | 1.06 - 1.22
-//   backward, 128, no groups:   one causal document .47 - .70 | .75 - .93 | 1.07 - 1.18 | 1.3     ragged, mean 100 - 300 .72 - .96 | 1.1 - 1.2 | 1.3 | 1.5
-//                               not causal .73 - .82 | 1.2 - 1.34 | 1.4 | 1.6                     documents of 512 .87 - .93 | 1.2 - 1.37 | | 1.5 - 1.8
-//   backward, 128, groups of 4: one causal document .59 | .65 | .70 | .79                         ragged .53 | .65 | .70 - .95 | .84 - 1.04
-//                               not causal .63 | .73 | 1.16 | 1.22                                documents of 512 | | | 1.19
+// Host side: whether a forward pass goes to these kernels, by its workgroups of 32 rows (rows / 32 x query heads).  A compute unit holds eight of
+// them up to 64 features, two above.  The tiled kernels wait for the longest chain of a workgroup, which is what these kernels shorten; they
+// gain where that chain runs alone: few workgroups, and causal documents, whose last rows have twice the average work.  They lose where the
+// tiled kernels have work for every compute unit all along.  Short / tiled, at 512 | 1024 | 1536 | 2048 workgroups:
+//   64 features:   one causal document .33 - .49 | .37 - .51 | .53 - .64 | .60 - .70     ragged, mean 100 - 800 | | .59 - .80 | .61 - .86
+//                  not causal .41 - .58 | .62 - .73 | .90 - .96 | 1.06 - 1.18            documents of 512 .47 | .70 - .78 | | .91 - 1.06
+//   128 features:  causal .38 - .53 | .51 - .84 | .72 - 1.06 | .91 - 1.2      not causal .50 - .78 | .87 - 1.10 | 1.3 | 1.5
 // (4 / 4, 12 / 12, 16 / 4 and 32 / 8 heads, the rows that make up the count; 1 and 2 heads with documents of up to 65536 tokens alike: the
-// length of a context alone does not decide.)  us at some of these, tiled / short: 32 / 8 heads of 128, 1024 tokens 34.7 / 23.9 forward, 145 /
-// 91.8 backward; 16 heads of 128, 8 documents of 512: 29.3 / 41.3 and 80 / 142; 12 heads of 64, 3001 tokens in documents of
-// 17 - 400: 20.9 / 12.3 and 48.4 / 37.1; 1 head of 64, 65536 tokens: 1280 / 762 and 2575 / 2280.  Of 110 calls
-// drawn between 350 and 2300 workgroups none that these kernels take was slower than tiled.
+// length of a context alone does not decide.)  us at some of these, tiled / short: 32 / 8 heads of 128, 1024 tokens 34.7 / 23.9; 16 heads of
+// 128, 8 documents of 512: 29.3 / 41.3; 12 heads of 64, 3001 tokens in documents of 17 - 400: 20.9 / 12.3; 1 head of 64, 65536 tokens: 1280 / 762.
 // Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
 // backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
-static inline bool mi_attn_is_short(const mi_attn_args* a, bool backward) {
+static inline bool mi_attn_fwd_is_short(const mi_attn_args* a) {
     if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return false;
     if (a->flags & MI_ATTN_SHORT) return true;
-    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k, docs = a->n_docs > 1 ? a->n_docs : 1;
-    const bool narrow = a->head_dim <= 64, causal = a->causal != 0;
-    const bool whole = a->total_q == a->total_k && rows % (256 * docs) == 0;                          // may be whole blocks, all of them
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k;
+    const int64_t per_unit = a->head_dim <= 64 ? (a->causal ? 8 : 6) : (a->causal ? 4 : 3);
+    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads <= per_unit * mi_compute_units();
+}
+
+// The same for a backward pass, whose blocks of either kind (dQ: rows / 32 x query heads, dK / dV: rows / 32 x KV heads x head split)
+// share a launch here as they do in the tiled kernels.  Short / tiled, over 510 calls of 1 - 32 heads drawn between 130 and 16384 tokens:
+//   up to 64 features, where a compute unit holds three blocks of either kind, by dQ blocks:
+//     up to 1500 .35 - .97          1500 - 2600 .71 - .99 (not causal 1.02 - 1.07, 8 documents of 256 1.26)
+//     2600 - 4100: one document .93 - 1.13, ragged documents of 30 - 500 .78 - .94          4100 - 7000: 1.02 - 1.12, ragged .78 - .90
+//   above, where one block fills it, by blocks of both kinds, causal, without | with groups of 4 query heads:
+//     350 .63 - .88 | .60       500 .67 - .96 | .61       576 .77 - 1.0 | .65      640 .95 - 1.15 | .62 - .68     760 .97 - 1.15 | .79 - .84     1120 1.1 | .97
+//     one causal document, whose chain the tiled kernels walk alone: 700 .89, 770 .74, 900 .86, 1060 1.11
+// Of the 510 the rule takes 12 to the slower side, by 2 - 8 %.  us, tiled / short: 12 heads of 64, 3001 tokens in documents of 17 - 400:
+// 35.9 / 31.3; 32 / 8 heads of 128, 512 tokens 57.4 / 35.5; 4 heads of 64, 1024 tokens 29.2 / 17.0.
+// Longer chains above 64 features are a band of their own: there dQ blocks are better off two to a compute unit, in a launch in front of the
+// dK / dV blocks (tiled / together / apart, us: 16 / 4 heads of 128, 1664 tokens 95 / 105 / 90; 32 / 8, 1316 tokens 137 / 134 / 124; 32 / 1,
+// 3 documents of 312 64 / 64 / 59).
+enum class ShortBwd { kNo, kTogether, kApart };
+static inline ShortBwd mi_attn_bwd_short(const mi_attn_args* a, int hsplit) {
+    if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return ShortBwd::kNo;
+    if (a->flags & MI_ATTN_SHORT) return ShortBwd::kTogether;
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k, docs = a->n_docs > 1 ? a->n_docs : 1, units = mi_compute_units();
+    if (rows <= 128) return ShortBwd::kNo;
+    const int64_t row_blocks = (rows + kShortRows - 1) / kShortRows, dq = row_blocks * a->n_q_heads, both = dq + row_blocks * a->n_kv_heads * hsplit;
+    const int64_t group = a->n_q_heads / a->n_kv_heads / hsplit;                                      // query heads of a dK / dV block
+    const bool causal = a->causal != 0;
+    const bool whole = a->total_q == a->total_k && rows % (256 * docs) == 0;                          // may be whole tiled blocks, all of them
     const bool chains = causal && (whole ? rows >= 1024 * docs * docs : rows >= 512 * docs);        // the chain of a document dominates
-    const int group = a->n_q_heads / a->n_kv_heads / mi_dkdv_head_split(a->n_q_heads, a->n_kv_heads);
-    int64_t per_unit_64;                                   // 64 x workgroups per compute unit
-    if (!backward) per_unit_64 = narrow ? (causal ? 512 : 384) : (causal ? 256 : 192);
-    else if (narrow) per_unit_64 = (!causal ? 320 : whole && !chains ? 256 : 512) + 96 * (group - 1);
-    else per_unit_64 = (chains ? 256 : 128) + (causal ? 96 : 64) * (group - 1);
-    const int most = backward && !narrow && !causal ? 256 : 512;
-    if (per_unit_64 > most) per_unit_64 = most;
-    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads * 64 <= per_unit_64 * mi_compute_units();
+    if (a->head_dim <= 64) {
+        int64_t per_unit_8;                                                                           // 8 x dQ blocks per compute unit
+        if (!whole && docs > 1 && rows <= 512 * docs) per_unit_8 = 192;
+        else if (causal && (!whole || chains)) per_unit_8 = 80 + 12 * (group - 1) < 96 ? 80 + 12 * (group - 1) : 96;
+        else per_unit_8 = (causal ? 32 : 40) + 12 * (group - 1) < 64 ? (causal ? 32 : 40) + 12 * (group - 1) : 64;
+        return dq * 8 <= per_unit_8 * units ? ShortBwd::kTogether : ShortBwd::kNo;
+    }
+    const bool alone = chains && rows >= 1024 * docs * docs;                                         // few documents, long ones
+    int64_t eighths = whole && docs > 1 && !chains ? 16 : 18 + 9 * (group - 1) / 2;                              // of a block of either kind per compute unit
+    if (alone && eighths < 28) eighths = 28;
+    if (both * 8 <= eighths * units) return ShortBwd::kTogether;
+    if (causal && rows * group >= (group < 4 ? 1536 : 1024) * docs && (alone || group >= 4) && both <= (3 + group) * units) return ShortBwd::kApart;
+    return ShortBwd::kNo;
 }
 
 // ---- forward: 32 queries of one head --------------------------------------------------------------------------------
@@ -340,20 +360,32 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
         p.lse[(int64_t)head * p.total_q + tq] = L > 0.f ? (M + __log2f(L)) * 0.6931471805599453f : INFINITY;
 }
 
-// ---- backward: dQ and delta of 32 queries of one head ------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 2) void attn_short_dq_kernel(const AttnParams p) {
+// acc + the products of eight features of an O row and a dO row: delta = sum of them over the features, in the same order wherever it is formed
+__device__ __forceinline__ float short_dot(const elem8_t& o, const elem8_t& d_o, float acc) {
+    float a[8], b[8];
+    Elem<elem_t>::unpack(__builtin_bit_cast(uint4, o), a);
+    Elem<elem_t>::unpack(__builtin_bit_cast(uint4, d_o), b);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc += a[i] * b[i];
+    return acc;
+}
+
+// ---- backward: dQ of 32 queries of one head ------------------------------------------------------------------
+template <int D> constexpr int kShortRed = kShortWaves * 16 * (D / 32) * 64 * 4;      // an accumulator set of every wavefront
+
+template <int D> constexpr int kShortDqSmem = ShortStages<D>::kSmem > kShortRed<D> ? ShortStages<D>::kSmem : kShortRed<D>;
+
+template <int D, bool KEEP_DELTA>
+__device__ __forceinline__ void short_dq_block(const AttnParams& p, char* smem, int block) {
     constexpr int KS = D / 16, DT = D / 32;
     using Stages = ShortStages<D>;
     using Tile = LdsTile<D>;
     constexpr int RB = Tile::RB;
-    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
-    __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nqb = (p.total_q + 31) / 32;
     int head, rank;
-    head_and_rank(blockIdx.x, p.nq, head, rank);
+    head_and_rank(block, p.nq, head, rank);
     const int qb = nqb - 1 - rank, kvh = head / p.n_rep;
     const int tq = qb * 32 + l32, tl = min(tq, p.total_q - 1);
 
@@ -371,15 +403,9 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 2) void attn_short_
             o_raw[ks] = ld128(orow + 16 * ks);
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            float a[8], b[8];
-            Elem<elem_t>::unpack(o_raw[ks], a);
-            Elem<elem_t>::unpack(__builtin_bit_cast(uint4, dof[ks]), b);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) delta += a[i] * b[i];
-        }
+        for (int ks = 0; ks < KS; ++ks) delta = short_dot(__builtin_bit_cast(elem8_t, o_raw[ks]), dof[ks], delta);
         delta = pair_sum(delta);
-        if (wave == 0 && g == 0 && tq < p.total_q) p.delta[(int64_t)head * p.total_q + tq] = delta;
+        if (KEEP_DELTA && wave == 0 && g == 0 && tq < p.total_q) p.delta[(int64_t)head * p.total_q + tq] = delta;
     }
     const float lse2 = p.lse[(int64_t)head * p.total_q + tl] * 1.4426950408889634f;
     int klo, khi, wmin, wmax, kt0, n_tiles;
@@ -454,21 +480,25 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 2) void attn_short_
 }
 
 // ---- backward: dK and dV of 32 keys of one KV head (of one share of its query heads: hsplit) ------------------------------
-// The wavefronts take (query tile, query head) pairs in turn; delta has been written by the dQ launch.
-template <int D>
-__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_dkdv_kernel(const AttnParams p) {
+// The wavefronts take (query tile, query head) pairs in turn.  OWN_DELTA: they form delta themselves, from the fragments of the dO tile and of
+// an O tile (up to 64 features) or of O rows in registers, which a compute unit's only workgroup has enough of; otherwise a launch in front has left it.
+template <int D, bool OWN_DELTA> using ShortDkdvStages = ShortStages<D, D <= 64 ? 1 : 2, OWN_DELTA && D <= 64 ? 3 : 2>;
+template <int D, bool OWN_DELTA>
+constexpr int kShortDkdvSmem = ShortDkdvStages<D, OWN_DELTA>::kSmem > kShortRed<D> ? ShortDkdvStages<D, OWN_DELTA>::kSmem : kShortRed<D>;
+
+// stat_lds: 32 log-sum-exps, 32 deltas of each wavefront's tile
+template <int D, bool OWN_DELTA>
+__device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem, float (*stat_lds)[64], int block) {
     constexpr int KS = D / 16, DT = D / 32;
     constexpr int STAGES = D <= 64 ? 1 : 2;
-    using Stages = ShortStages<D, STAGES>;
+    constexpr bool O_TILE = OWN_DELTA && D <= 64, O_ROWS = OWN_DELTA && D > 64;
+    using Stages = ShortDkdvStages<D, OWN_DELTA>;
     using Tile = LdsTile<D>;
     constexpr int RB = Tile::RB;
-    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
-    __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
-    __shared__ __attribute__((aligned(16))) float stat_lds[kShortWaves][64];      // 32 log-sum-exps, 32 deltas of the wavefront's tile
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int group, kb;
-    head_and_rank(blockIdx.x, p.nkv * p.hsplit, group, kb);       // key blocks with the most queries come first
+    head_and_rank(block, p.nkv * p.hsplit, group, kb);            // key blocks with the most queries come first
     const int kvh = group / p.hsplit, hs = group - kvh * p.hsplit, hpw = p.n_rep / p.hsplit;
     const int key = kb * 32 + l32, kl = min(key, p.total_k - 1);
 
@@ -495,30 +525,61 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_
     DmaPlan<D, Stages::kLoads> q_plan, do_plan;
     q_plan.init(0, lane, p.q_st);
     do_plan.init(0, lane, p.o_st);
-    const float* stat_base = g == 0 ? p.lse : p.delta;
-    const float stat_scale = g == 0 ? 1.4426950408889634f : 1.0f;
     const int iters = n_tiles * hpw;
+    const float* stat_base = OWN_DELTA || g == 0 ? p.lse : p.delta;
+    const float stat_scale = OWN_DELTA || g == 0 ? 1.4426950408889634f : 1.0f;
     float stat = 0.f;
+    elem8_t o_raw[O_ROWS ? KS : 1];
     auto issue = [&](int iter, int buf) {
         const int tile = iter / hpw, head = kvh * p.n_rep + hs * hpw + (iter - tile * hpw), qt = qt0 + 32 * tile;
         stat = stat_base[(int64_t)head * p.total_q + min(qt + l32, p.total_q - 1)];
         q_plan.issue(p.q + (int64_t)head * p.q_sh, p.q_st, qt, p.total_q - 1, st.first(buf));
         do_plan.issue(p.d_o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, st.second(buf));
+        if constexpr (O_TILE) do_plan.issue(p.o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, st.third(buf));
+    };
+    auto load_o = [&](int iter) {
+        const int tile = iter / hpw, head = kvh * p.n_rep + hs * hpw + (iter - tile * hpw);
+        const elem_t* row = p.o + (int64_t)min(qt0 + 32 * tile + l32, p.total_q - 1) * p.o_st + (int64_t)head * p.o_sh + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) o_raw[ks] = *reinterpret_cast<const elem8_t*>(row + 16 * ks);
     };
     int h0, h1;
     Tile::tr_bases(lane, h0, h1);
     const int a_row = Tile::row_base(l32, g);
-    if (wave < iters) issue(wave, 0);
+    if (wave < iters) {
+        issue(wave, 0);
+        if constexpr (O_ROWS) load_o(wave);
+    }
     int buf = 0;
     for (int iter = wave; iter < iters; iter += kShortWaves) {
         const bool next = iter + kShortWaves < iters;
-        stat_lds[wave][lane] = stat * stat_scale;
+        if (!OWN_DELTA || g == 0) stat_lds[wave][lane] = stat * stat_scale;
+        if constexpr (O_ROWS) {                           // waited for here, or the wait would take the next step's tiles along
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(o_raw[ks]));
+        }
         const char *qs_ = st.first(buf), *ds_ = st.second(buf);
         if (STAGES == 2 && next) {
             issue(iter + kShortWaves, buf ^ 1);
-            wait_vmcnt<2 * Stages::kLoads>();             // this step's tiles have landed, the next one's may be in flight
+            wait_vmcnt<2 * Stages::kLoads>();             // this step's tiles and rows have landed, the next one's tiles may be in flight
         } else {
             wait_vmcnt<0>();
+        }
+        if constexpr (OWN_DELTA) {
+            float delta = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const int at = a_row ^ (ks << 5);
+                const elem8_t d_o = *reinterpret_cast<const elem8_t*>(ds_ + at);
+                if constexpr (O_TILE) delta = short_dot(*reinterpret_cast<const elem8_t*>(st.third(buf) + at), d_o, delta);
+                else delta = short_dot(o_raw[ks], d_o, delta);
+            }
+            delta = pair_sum(delta);
+            if (g == 1) stat_lds[wave][lane] = delta;
+            __builtin_amdgcn_sched_barrier(0);            // before the accumulators are live: 168 registers at 64 features
+            if constexpr (O_ROWS) {
+                if (next) load_o(iter + kShortWaves);
+            }
         }
         const int qs = qt0 + 32 * (iter / hpw);
         f32x16_t s_acc, dp_acc;
@@ -592,6 +653,22 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_
     }
     short_write<D>(p.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh + 8 * wave + 4 * g, dk, 1.0f);
     short_write<D>(p.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh + 8 * wave + 4 * g, dv, 1.0f);
+}
+
+// Both in one launch: dK / dV blocks, the longer ones, in the first n_dkdv workgroups, dQ blocks in the others.
+template <int D, bool OWN_DELTA>
+__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_bwd_kernel(const AttnParams p, int n_dkdv) {
+    __shared__ __attribute__((aligned(1024))) char smem[kShortDqSmem<D> > kShortDkdvSmem<D, OWN_DELTA> ? kShortDqSmem<D> : kShortDkdvSmem<D, OWN_DELTA>];
+    __shared__ __attribute__((aligned(16))) float stat_lds[kShortWaves][64];
+    if ((int)blockIdx.x < n_dkdv) short_dkdv_block<D, OWN_DELTA>(p, smem, stat_lds, blockIdx.x);
+    else short_dq_block<D, false>(p, smem, blockIdx.x - n_dkdv);
+}
+
+// dQ blocks alone, two to a compute unit; they leave delta for dK / dV
+template <int D>
+__global__ __launch_bounds__(64 * kShortWaves, 2) void attn_short_dq_kernel(const AttnParams p) {
+    __shared__ __attribute__((aligned(1024))) char smem[kShortDqSmem<D>];
+    short_dq_block<D, true>(p, smem, blockIdx.x);
 }
 
 }  // namespace

@@ -10,6 +10,7 @@ import oracle
 from scaling_amd import _lib, ops
 from tests import attn_utils as U
 from tests.parity import check
+from tests.kernels import launched
 from tests.test_gpu_attention import CASES
 
 pytestmark = pytest.mark.gpu
@@ -94,9 +95,11 @@ def test_attention_routes_agree_with_rotary(d, interleaved):
     (4, 4, 64, 8192, 1, True, SHORT, SHORT), (4, 4, 64, 8192, 1, False, SHORT, SHORT), (8, 8, 64, 8192, 1, False, TILED, TILED),
     (16, 16, 64, 4096, 8, True, SHORT, TILED),             # documents of whole blocks
     (16, 16, 64, 4095, 8, True, SHORT, SHORT), (32, 8, 64, 2048, 1, False, TILED, SHORT),
-    (8, 8, 128, 4096, 1, True, SHORT, SHORT), (8, 8, 128, 4096, 8, True, SHORT, TILED), (8, 8, 128, 4090, 20, True, SHORT, TILED),
-    (8, 8, 128, 2048, 4, True, SHORT, SHORT), (4, 4, 128, 8192, 1, False, TILED, TILED), (4, 4, 128, 4096, 1, False, SHORT, SHORT),
-    (4, 4, 128, 16384, 1, True, TILED, TILED), (32, 8, 128, 2048, 1, True, TILED, SHORT), (32, 8, 128, 1056, 1, False, TILED, TILED),
+    (8, 8, 128, 4096, 1, True, SHORT, TILED), (8, 8, 128, 4096, 8, True, SHORT, TILED), (8, 8, 128, 4090, 20, True, SHORT, TILED),
+    (8, 8, 128, 2048, 4, True, SHORT, TILED), (4, 4, 128, 8192, 1, False, TILED, TILED), (4, 4, 128, 4096, 1, False, SHORT, TILED),
+    (4, 4, 128, 16384, 1, True, TILED, TILED), (32, 8, 128, 2048, 1, True, TILED, TILED), (32, 8, 128, 1056, 1, False, TILED, TILED),
+    (8, 8, 128, 1152, 4, True, SHORT, SHORT), (4, 4, 128, 3584, 1, True, SHORT, SHORT), (32, 8, 128, 768, 1, False, SHORT, SHORT),
+    (8, 8, 64, 16380, 40, True, TILED, SHORT),
 ])
 def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
     print(f"case route of a call nq={nq} nkv={nkv} d={d} total={total} docs={docs} causal={causal}", flush=True)
@@ -114,6 +117,30 @@ def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
         # sums in another order: some element of so many rounds the other way
         assert torch.equal(o, o2) == (flags == fwd)
         assert all(torch.equal(x, y) == (flags == bwd) for x, y in zip((dq, dk, dv), grads))
+
+
+# where a launch in front of the dK / dV blocks leaves delta: one of its own for long chains, or the dQ blocks' (single long documents above
+# 64 features, by the size of the call)
+@pytest.mark.parametrize("nq,nkv,d,lens,flags,kernel", [
+    (1, 1, 64, (1100,), SHORT, "attn_bwd_delta"), (8, 1, 32, (1021,), SHORT, None), (2, 1, 128, (530,), SHORT, "attn_bwd_delta"),
+    (2, 1, 96, (500, 17), SHORT, None), (4, 4, 128, (3601,), 0, "attn_short_dq"), (16, 4, 128, (1663,), 0, "attn_short_dq"),
+])
+def test_backward_with_delta_of_another_launch(nq, nkv, d, lens, flags, kernel):
+    print(f"case delta nq={nq} nkv={nkv} d={d} lens={lens} flags={flags}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are per compute unit; these sizes are for 256")
+    g = torch.Generator(device=DEV).manual_seed(d)
+    q, do = (torch.randn(sum(lens), nq, d, generator=g, device=DEV).half() for _ in range(2))
+    k, v = (torch.randn(sum(lens), nkv, d, generator=g, device=DEV).half() for _ in range(2))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    o, lse = ops.attention_forward(q, k, v, cu, None, True, None)
+    run = lambda f: ops.attention_backward(do, q, k, v, o, lse, cu, None, True, None, flags=f)
+    grads, tiled, names = run(flags), run(TILED), launched(lambda: run(flags))
+    assert any("attn_short_bwd" in n for n in names)
+    assert [n for n in ("attn_bwd_delta", "attn_short_dq") if any(n in x for x in names)] == ([kernel] if kernel else [])
+    for name, x, y in zip(("dq", "dk", "dv"), grads, tiled):
+        # P and dS round the same values to float16 but for the last bits of delta and of their exponents: two roundings each way
+        assert float((x.float() - y.float()).norm()) <= 2.0 ** -9 * float(y.float().norm()), name
 
 
 # float32 backward with dS kept by the dK/dV kernel (a workspace that has room for it) against the dQ kernel that recomputes it: the same
