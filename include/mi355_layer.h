@@ -449,6 +449,13 @@ typedef struct mi_decode_args {
 size_t mi_attn_decode_workspace_bytes(int32_t batch, int32_t n_q_heads, int32_t head_dim, int32_t max_ctx);
 int mi_attn_decode(const mi_decode_args* args);
 
+/* mi_attn_decode whose splits, where they are few and short, are merged by the workgroup that arrives last instead of by a second launch
+ * (which the host takes longer to issue than such a call takes): same arguments, same bits.
+ * tickets: n_tickets >= batch * n_kv_heads * ceil(n_q_heads / n_kv_heads / 16) (never more than batch * n_q_heads) int32 of device memory,
+ * all zero before the first call; every call leaves them zero.  Like the workspace they belong to one call at a time: calls that may
+ * overlap (different streams) need tickets of their own. */
+int mi_attn_decode_with_tickets(const mi_decode_args* args, int32_t* tickets, int64_t n_tickets);
+
 /* mi_attn_decode for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments, kernels and results
  * as mi_attn_decode, except that `workspace` / `workspace_bytes` are ignored: the per-split partial results go to

@@ -7,7 +7,8 @@
 //                                   memory in operand layout, B = Q^T (heads of the group, zero padded)
 //     online softmax over keys      the lane's column is a head; 8 in-lane keys + 2 lane exchanges
 //     O^T[d][head]   += V^T * P^T   A = V^T read from a transposed per-wavefront LDS copy of the chunk
-// Partial (max, sum, O) per split go to a workspace and are merged by a second kernel (none with a single split).
+// Partial (max, sum, O) per split go to a workspace and are merged by the last workgroup of the splits to arrive (with tickets) or by a
+// second kernel (none of it with a single split).
 // The wavefront whose keys include the new token first appends the new K/V row in place (instead of the
 // reference's torch.cat), rotated, and then reads it back with the rest of its chunk; the query is rotated while its
 // fragments are loaded.  (A launch of its own for the append took 3 - 5 us: a third of a step at batch 1.)
@@ -33,6 +34,7 @@ struct DecodeParams {
     float scale_log2;
     float* ws_o;   // [batch][nq][n_splits][D]
     float* ws_ml;  // [batch][nq][n_splits][2]
+    int32_t* tickets;   // nullable: one arrival count per (batch, KV head, head chunk), zero between launches
 };
 
 __device__ __forceinline__ f32x4v mfma_16x16x32(elem8_t a, elem8_t b, f32x4v c) {
@@ -72,6 +74,60 @@ __device__ __forceinline__ void append_row(const DecodeParams& p, int b, int kvh
     st128(p.vc + dst + D / 2, vhi);
 }
 
+// ---- merge of the splits ------------------------------------------------------------------------------
+// SHARED: the partial results pass between workgroups of one launch, past the L2s (those of the XCDs are not coherent; writing back and
+// invalidating them, as a release and an acquire do, took 2 - 10 us of a launch of 104 - 256 workgroups).
+template <bool SHARED> __device__ __forceinline__ float2 load_partial(const float* at) {
+    if constexpr (!SHARED) return *reinterpret_cast<const float2*>(at);
+    const uint64_t x = __hip_atomic_load(reinterpret_cast<const uint64_t*>(at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((uint32_t)x), __uint_as_float((uint32_t)(x >> 32)));
+}
+template <bool SHARED> __device__ __forceinline__ void store_partial(float* at, float x) {
+    if constexpr (SHARED) __hip_atomic_store(at, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *at = x;
+}
+
+// Features d and d + 1 of row bh = (batch, head), in steps of eight splits, the partial results of two steps requested before the first is
+// used: 16 splits are one latency.
+template <int D, bool SHARED>
+__device__ __forceinline__ void merge_splits(const DecodeParams& p, int64_t bh, int d) {
+    constexpr int kStep = 8, kSteps = 2;
+    const float* ml = p.ws_ml + bh * p.n_splits * 2;
+    const float* wo = p.ws_o + bh * p.n_splits * D + d;
+    float M = -INFINITY, L = 0.f, O0 = 0.f, O1 = 0.f;
+    for (int s0 = 0; s0 < p.n_splits; s0 += kSteps * kStep) {
+        float2 mls[kSteps][kStep], os[kSteps][kStep];
+#pragma unroll
+        for (int h = 0; h < kSteps; ++h) {
+            if (s0 + h * kStep >= p.n_splits) break;
+#pragma unroll
+            for (int i = 0; i < kStep; ++i) {              // past the last split: its values again, with no weight below
+                const int s = min(s0 + h * kStep + i, p.n_splits - 1);
+                mls[h][i] = load_partial<SHARED>(ml + 2 * s);
+                os[h][i] = load_partial<SHARED>(wo + (int64_t)s * D);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < kSteps; ++h) {
+            if (s0 + h * kStep >= p.n_splits) break;
+            float m = M;
+#pragma unroll
+            for (int i = 0; i < kStep; ++i) m = fmaxf(m, mls[h][i].x);
+            const float a = M == -INFINITY ? 0.f : fast_exp2(M - m);
+            L *= a; O0 *= a; O1 *= a;
+            M = m;
+#pragma unroll
+            for (int i = 0; i < kStep; ++i) {
+                const float f = s0 + h * kStep + i >= p.n_splits || mls[h][i].x == -INFINITY ? 0.f : fast_exp2(mls[h][i].x - M);
+                L += f * mls[h][i].y;
+                O0 += f * os[h][i].x;
+                O1 += f * os[h][i].y;
+            }
+        }
+    }
+    *reinterpret_cast<uint32_t*>(p.o + bh * D + d) = pack_elem2(L > 0.f ? O0 / L : 0.f, L > 0.f ? O1 / L : 0.f);
+}
+
 // ---- split kernel ----------------------------------------------------------------------------------
 // NWV wavefronts (4 or 8) share the keys of one (batch, KV head, split); with a single split the merged result
 // is the attention output and goes straight to `o`, otherwise the partial goes to the workspace.
@@ -89,6 +145,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     __shared__ float wm_lds[NWV][16];
     __shared__ float wl_lds[NWV][16];
     __shared__ float wo_lds[NWV][16][D + 1];
+    __shared__ int last_lds;
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, G = lane >> 4;
@@ -296,48 +353,51 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
             p.o[bh * D + d] = (elem_t)(L > 0.f ? O / L : 0.f);
         } else {
             const int64_t slot = bh * p.n_splits + split;
-            p.ws_o[slot * D + d] = O;
-            if (d == 0) { p.ws_ml[slot * 2] = M; p.ws_ml[slot * 2 + 1] = L; }
+            if (p.tickets != nullptr) {
+                store_partial<true>(p.ws_o + slot * D + d, O);
+                if (d == 0) { store_partial<true>(p.ws_ml + slot * 2, M); store_partial<true>(p.ws_ml + slot * 2 + 1, L); }
+            } else {
+                store_partial<false>(p.ws_o + slot * D + d, O);
+                if (d == 0) { store_partial<false>(p.ws_ml + slot * 2, M); store_partial<false>(p.ws_ml + slot * 2 + 1, L); }
+            }
         }
     }
+    // With tickets the last workgroup of a (batch, KV head) to get here merges its splits; nobody waits for anybody.  The partial results are
+    // stored past the L2 and every wavefront has waited for its own before the barrier, so the count that thread 0 raises behind it
+    // comes after them in memory, and the loads of the workgroup that reads the highest count come after all.
+    if (p.n_splits == 1 || p.tickets == nullptr) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        int32_t* ticket = p.tickets + blockIdx.x / p.n_splits;
+        const int arrived = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_lds = arrived == p.n_splits - 1;
+        if (arrived == p.n_splits - 1) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
+    }
+    __syncthreads();
+    if (last_lds == 0) return;
+    for (int idx = tid; idx < n_heads * (D / 2); idx += kThreads)
+        merge_splits<D, true>(p, (int64_t)b * p.nq + head0 + idx / (D / 2), 2 * (idx % (D / 2)));
 }
 
-// ---- merge of the splits ------------------------------------------------------------------------------
-// One thread per (batch, head, two features), its partial results requested eight splits at a time before the first is
-// used: a launch of 16 splits is two latencies, not sixteen.  (With the append's launch gone as well, batch 1 over a cache of
+// Where the caller has no tickets: one thread per (batch, head, two features).  (With the append's launch gone as well, batch 1 over a cache of
 // 1,024: 21.5 -> 11.2 us for a call; batch 32: 83.8 -> 81.6.)
 template <int D>
 __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeParams p) {
-    constexpr int kDepth = 8;
     const int64_t bh = (int64_t)blockIdx.x * (128 / D) + (2 * threadIdx.x) / D;
     const int d = (2 * threadIdx.x) % D;
     if (2 * threadIdx.x >= (128 / D) * D || bh >= (int64_t)p.batch * p.nq) return;
-    const float* ml = p.ws_ml + bh * p.n_splits * 2;
-    const float* wo = p.ws_o + bh * p.n_splits * D + d;
-    float M = -INFINITY, L = 0.f, O0 = 0.f, O1 = 0.f;
-    for (int s0 = 0; s0 < p.n_splits; s0 += kDepth) {
-        float2 mls[kDepth], os[kDepth];
-#pragma unroll
-        for (int i = 0; i < kDepth; ++i) {                 // past the last split: its values again, with no weight below
-            const int s = min(s0 + i, p.n_splits - 1);
-            mls[i] = *reinterpret_cast<const float2*>(ml + 2 * s);
-            os[i] = *reinterpret_cast<const float2*>(wo + (int64_t)s * D);
-        }
-        float m = M;
-#pragma unroll
-        for (int i = 0; i < kDepth; ++i) m = fmaxf(m, mls[i].x);
-        const float a = M == -INFINITY ? 0.f : fast_exp2(M - m);
-        L *= a; O0 *= a; O1 *= a;
-        M = m;
-#pragma unroll
-        for (int i = 0; i < kDepth; ++i) {
-            const float f = s0 + i >= p.n_splits || mls[i].x == -INFINITY ? 0.f : fast_exp2(mls[i].x - M);
-            L += f * mls[i].y;
-            O0 += f * os[i].x;
-            O1 += f * os[i].y;
-        }
-    }
-    *reinterpret_cast<uint32_t*>(p.o + bh * D + d) = pack_elem2(L > 0.f ? O0 / L : 0.f, L > 0.f ? O1 / L : 0.f);
+    merge_splits<D, false>(p, bh, d);
+}
+
+// Whether the last workgroup merges, given tickets.  On the device that is no gain: its one workgroup per (batch, KV head) loads past the caches what
+// the merge launch spreads over more of them, with a thread for every two features of its heads and up to 16 splits 0 - 1 us more than that
+// launch, beyond 2 - 9.  But a call of so few bytes is over before the host has issued two launches: batch 1, 32 / 8 heads of 128, a cache of 1,564, one call
+// after the other 10.9 -> 8.8 us.
+bool merges_in_launch(const DecodeParams& p, int head_dim) {
+    const int heads = p.n_rep < 16 ? p.n_rep : 16;
+    return p.n_splits > 1 && p.n_splits <= 16 && heads * head_dim <= 512 &&
+           (int64_t)p.batch * p.nkv * p.max_ctx * head_dim * 4 <= (int64_t)32 << 20;
 }
 
 // 8-wavefront workgroups (one per compute unit) once there is a (batch, KV head) pair for most of the 256
@@ -374,7 +434,7 @@ template <int D, int NWV> int launch_split(const DecodeParams& p, int rot, hipSt
 
 template <int D> int launch_decode(const DecodeParams& p, int rot, hipStream_t st) {
     const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8>(p, rot, st) : launch_split<D, 4>(p, rot, st);
-    if (rc != MI_OK || p.n_splits == 1) return rc;
+    if (rc != MI_OK || p.n_splits == 1 || p.tickets != nullptr) return rc;
     constexpr int kRows = 128 / D;
     const int64_t n = (int64_t)p.batch * p.nq;
     decode_merge_kernel<D><<<dim3((unsigned)((n + kRows - 1) / kRows)), dim3(64), 0, st>>>(p);
@@ -394,7 +454,7 @@ extern "C" size_t mi_attn_decode_workspace_bytes(int32_t batch, int32_t n_q_head
 namespace {
 // Validation and launches shared by the two entry points; `ws` / `ws_bytes` is the scratch for the per-split partial
 // results (the caller's workspace, or the library's own static array for mi_attn_decode_static).
-int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static_ws) {
+int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static_ws, int32_t* tickets, int64_t n_tickets) {
     if (!a) return mi_fail(MI_E_NULL, "attn_decode: args is null");
     if (!a->q || !a->k_cache || !a->v_cache || !a->o || !a->ctx_len) return mi_fail(MI_E_NULL, "attn_decode: q, caches, o and ctx_len are required");
     if (a->dtype != MI_ELEM_DTYPE) return mi_fail(MI_E_DTYPE, "attn_decode: the decode kernels take bf16 or f16 tensors (dtype code %d)", a->dtype);
@@ -430,7 +490,10 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
                        a->batch, a->n_q_heads, splits, a->head_dim, need, ws_bytes);
     if (!ws || ws_bytes < need || !mi_aligned16(ws))
         return mi_fail(MI_E_WORKSPACE, "attn_decode: workspace needs %zu bytes (16-byte aligned), got %zu", need, ws_bytes);
+    if (tickets && (n_tickets < (int64_t)a->batch * a->n_kv_heads * n_hc || (reinterpret_cast<uintptr_t>(tickets) & 3u) != 0))
+        return mi_fail(MI_E_WORKSPACE, "attn_decode: %lld tickets (4-byte aligned), got %lld", (long long)a->batch * a->n_kv_heads * n_hc, (long long)n_tickets);
     DecodeParams p{};
+    p.tickets = tickets;
     p.q = (const elem_t*)a->q; p.kc = (elem_t*)a->k_cache; p.vc = (elem_t*)a->v_cache; p.o = (elem_t*)a->o;
     p.ctx_len = a->ctx_len; p.k_new = (const elem_t*)a->k_new; p.v_new = (const elem_t*)a->v_new;
     if (a->rotary_interleaved) {
@@ -447,6 +510,7 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
     p.kn_sb = a->k_new_stride_batch ? a->k_new_stride_batch : (int64_t)a->n_kv_heads * a->head_dim;
     p.vn_sb = a->v_new_stride_batch ? a->v_new_stride_batch : (int64_t)a->n_kv_heads * a->head_dim;
     p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
+    if (p.tickets != nullptr && !merges_in_launch(p, a->head_dim)) p.tickets = nullptr;
     p.ws_o = (float*)ws;
     p.ws_ml = p.ws_o + (size_t)a->batch * a->n_q_heads * splits * a->head_dim;
     hipStream_t st = (hipStream_t)a->stream;
@@ -460,13 +524,13 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
 }
 }  // namespace
 
-int MI_ENTRY(mi_attn_decode_impl)(const mi_decode_args* a, bool static_ws) {
+int MI_ENTRY(mi_attn_decode_impl)(const mi_decode_args* a, bool static_ws, int32_t* tickets, int64_t n_tickets) {
     if (!a) return mi_fail(MI_E_NULL, "attn_decode: args is null");
-    if (!static_ws) return decode_entry(a, a->workspace, a->workspace_bytes, false);
+    if (!static_ws) return decode_entry(a, a->workspace, a->workspace_bytes, false, tickets, n_tickets);
     // the entry point that allocates nothing: partial results go to the library's static device array
     void* ws = nullptr;
     size_t bytes = 0;
     const int rc = mi_static_scratch(&ws, &bytes);
     if (rc != MI_OK) return rc;
-    return decode_entry(a, ws, bytes, true);
+    return decode_entry(a, ws, bytes, true, nullptr, 0);
 }

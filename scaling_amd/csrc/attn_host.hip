@@ -11,8 +11,8 @@ int mi_attn_bwd_impl_f16(const mi_attn_bwd_args* b);
 int mi_attn_fwd_impl_f32(const mi_attn_args* a);
 int mi_attn_bwd_impl_f32(const mi_attn_bwd_args* b);
 size_t mi_attn_bwd_workspace_bytes_f32(const mi_attn_args* a);
-int mi_attn_decode_impl_bf16(const mi_decode_args* a, bool static_ws);
-int mi_attn_decode_impl_f16(const mi_decode_args* a, bool static_ws);
+int mi_attn_decode_impl_bf16(const mi_decode_args* a, bool static_ws, int32_t* tickets, int64_t n_tickets);
+int mi_attn_decode_impl_f16(const mi_decode_args* a, bool static_ws, int32_t* tickets, int64_t n_tickets);
 
 extern "C" int mi_attn_fwd(const mi_attn_args* a) {
     if (!a) return mi_fail(MI_E_NULL, "attn_fwd: args is null");
@@ -36,12 +36,17 @@ extern "C" size_t mi_attn_bwd_workspace_bytes_for(const mi_attn_args* a) {
 
 extern "C" int mi_attn_decode(const mi_decode_args* a) {
     if (!a) return mi_fail(MI_E_NULL, "attn_decode: args is null");
-    return a->dtype == MI_F16 ? mi_attn_decode_impl_f16(a, false) : mi_attn_decode_impl_bf16(a, false);
+    return a->dtype == MI_F16 ? mi_attn_decode_impl_f16(a, false, nullptr, 0) : mi_attn_decode_impl_bf16(a, false, nullptr, 0);
+}
+
+extern "C" int mi_attn_decode_with_tickets(const mi_decode_args* a, int32_t* tickets, int64_t n_tickets) {
+    if (!a || !tickets) return mi_fail(MI_E_NULL, "attn_decode: args or tickets are null");
+    return a->dtype == MI_F16 ? mi_attn_decode_impl_f16(a, false, tickets, n_tickets) : mi_attn_decode_impl_bf16(a, false, tickets, n_tickets);
 }
 
 extern "C" int mi_attn_decode_static(const mi_decode_args* a) {
     if (!a) return mi_fail(MI_E_NULL, "attn_decode_static: args is null");
-    return a->dtype == MI_F16 ? mi_attn_decode_impl_f16(a, true) : mi_attn_decode_impl_bf16(a, true);
+    return a->dtype == MI_F16 ? mi_attn_decode_impl_f16(a, true, nullptr, 0) : mi_attn_decode_impl_bf16(a, true, nullptr, 0);
 }
 
 // ---- scratch of the entry point that allocates nothing -----------------------------------------------------------

@@ -1052,7 +1052,7 @@ std::tuple<Tensor, Tensor, Tensor> op_linear_cross_entropy(const Tensor& h, cons
 // ---- decode ------------------------------------------------------------------------------------------------------------
 void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, const OptTensor& k_new,
                       const OptTensor& v_new, const OptTensor& cos, const OptTensor& sin, const OptTensor& pos, bool interleaved, double scale,
-                      const OptTensor& workspace, int n_splits, const Tensor& out, bool static_scratch) {
+                      const OptTensor& workspace, const OptTensor& tickets, int n_splits, const Tensor& out, bool static_scratch) {
     need_gpu(q); need_gpu(k_cache); need_gpu(v_cache); need_gpu(ctx_len);
     Launch l(q);
     mi_decode_args a{};
@@ -1080,7 +1080,12 @@ void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v
     }
     a.workspace = ptr(*workspace);
     a.workspace_bytes = (size_t)workspace->numel() * 4;
-    check(mi_attn_decode(&a), "mi_attn_decode");
+    // One launch less where the tickets that came with the workspace are enough; a graph issues the second one for nothing.
+    const bool merge = tickets.has_value() && tickets->scalar_type() == at::kInt && tickets->is_contiguous() && tickets->device() == out.device() &&
+                       tickets->numel() >= (int64_t)a.batch * a.n_q_heads &&
+                       c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+    if (merge) check(mi_attn_decode_with_tickets(&a, static_cast<int32_t*>(ptr(*tickets)), tickets->numel()), "mi_attn_decode_with_tickets");
+    else check(mi_attn_decode(&a), "mi_attn_decode");
 }
 
 // ---- a decode step's layer ---------------------------------------------------------------------------------------------

@@ -483,9 +483,18 @@ def attention_qkv(qkv: torch.Tensor, cu_seqlens_q: torch.Tensor, cu_seqlens_k: O
 # ------------------------------------------------------------------------------------------------
 # decode attention over a pre-allocated KV cache
 # ------------------------------------------------------------------------------------------------
-def decode_workspace(batch: int, n_q_heads: int, head_dim: int, max_ctx: int, device) -> torch.Tensor:
+def _decode_scratch(batch: int, n_q_heads: int, head_dim: int, max_ctx: int, device) -> torch.Tensor:
     nbytes = _lib.load().mi_attn_decode_workspace_bytes(batch, n_q_heads, head_dim, max_ctx)
     return torch.empty(nbytes // 4, dtype=torch.float32, device=device)
+
+
+def decode_workspace(batch: int, n_q_heads: int, head_dim: int, max_ctx: int, device) -> torch.Tensor:
+    """Scratch of `decode_attention` for calls that do not overlap.  With it come the arrival counts (attribute `tickets`, int32, zero
+    between calls) by which the last workgroup of a small call merges the splits of the keys in the same launch; a workspace without them (a
+    slice, a tensor of the caller's own) takes a second launch for the same result."""
+    workspace = _decode_scratch(batch, n_q_heads, head_dim, max_ctx, device)
+    workspace.tickets = torch.zeros(max(batch * n_q_heads, 0), dtype=torch.int32, device=device)
+    return workspace
 
 
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx_len: torch.Tensor,
@@ -512,7 +521,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     if workspace is None and not static_scratch:
-        workspace = decode_workspace(B, nq, d, k_cache.shape[1], q.device)
+        workspace = _decode_scratch(B, nq, d, k_cache.shape[1], q.device)
     if out is None:
         out = torch.empty((B, nq, d), dtype=q.dtype, device=q.device)
     _check_rows(q)
@@ -527,7 +536,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         interleaved = _fused_rotary_kind(cos, sin, d, q.dtype)
         assert pos.dtype == torch.int64 and pos.numel() == B and pos.is_contiguous()
     _lib.host().decode_attention(q, k_cache, v_cache, ctx_len, k_new, v_new, cos, sin, pos, interleaved, float(softmax_scale),
-                                 None if static_scratch else workspace, int(n_splits), out, bool(static_scratch))
+                                 None if static_scratch else workspace, None if static_scratch else getattr(workspace, "tickets", None),
+                                 int(n_splits), out, bool(static_scratch))
     return out
 
 

@@ -7,7 +7,8 @@ import pytest
 import torch
 
 import oracle
-from scaling_amd import ops
+from scaling_amd import _lib, ops
+from tests.kernels import launched
 from tests.parity import check
 
 pytestmark = pytest.mark.gpu
@@ -239,3 +240,50 @@ def test_decode_append_at_chunk_and_split_edges(B, nq, nkv, d, max_ctx, n_splits
     check("decode.o(append edges)", out, _oracle_decode(q, kc_ref, vc_ref, ctx, scale, torch.float32),
           _oracle_decode(q, kc_ref, vc_ref, ctx, scale, torch.bfloat16), kind="decode")
     assert torch.equal(out, present) and torch.equal(kcd.cpu(), kc_ref) and torch.equal(vcd.cpu(), vc_ref)
+
+
+# splits that are empty (short contexts, none at all), one and every count of head chunks, the most splits, both sizes of workgroups
+@pytest.mark.parametrize("B,nq,nkv,d,max_ctx,lens,n_splits", [
+    (1, 32, 8, 128, 1564, [1500], 0), (3, 8, 2, 128, 4000, [4000, 1, 0], 13), (2, 24, 1, 32, 700, [700, 129], 0), (1, 4, 4, 96, 4096, [4096], 16),
+    (2, 6, 3, 32, 300, [300, 299], 2), (48, 8, 4, 64, 330, [330, 256, 255, 7, 300, 1] * 8, 3), (1, 16, 4, 128, 2000, [33], 9),
+])
+def test_decode_merged_by_the_last_workgroup(B, nq, nkv, d, max_ctx, lens, n_splits):
+    """With the tickets of a `decode_workspace` the splits of a small call are merged inside the launch: the bits of the two launches, tickets zero
+    again after every call; through the C entry in a graph too, where the Python one takes two launches."""
+    g = torch.Generator().manual_seed(B + d)
+    kc, vc = (torch.randn(B, max_ctx, nkv, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    qs = [torch.randn(B, nq, d, generator=g).bfloat16().to(DEV) for _ in range(3)]
+    ctx = torch.tensor(lens, dtype=torch.int32).to(DEV)
+    ws = ops.decode_workspace(B, nq, d, max_ctx, DEV)
+    plain = torch.empty_like(ws)
+    call = lambda q, workspace, out: ops.decode_attention(q, kc, vc, ctx, workspace=workspace, n_splits=n_splits, out=out)
+    want = [call(q, plain, torch.empty_like(q)) for q in qs]
+    out, q = torch.empty_like(qs[0]), qs[0].clone()
+    assert not any("decode_merge" in n for n in launched(lambda: call(q, ws, out)))
+    for i in (1, 2, 0):
+        out.fill_(float("nan"))
+        call(qs[i], ws, out)
+        assert torch.equal(out, want[i]) and not ws.tickets.any()
+    args = _lib.MiDecodeArgs()
+    args.q, args.o, args.k_cache, args.v_cache, args.ctx_len = (t.data_ptr() for t in (q, out, kc, vc, ctx))
+    args.batch, args.max_ctx, args.n_q_heads, args.n_kv_heads, args.head_dim, args.n_splits = B, max_ctx, nq, nkv, d, n_splits
+    args.softmax_scale = 1.0 / math.sqrt(d)
+    args.cache_stride_batch, args.cache_stride_token, args.cache_stride_head = kc.stride()[:3]
+    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel() * 4
+
+    def entry(n_tickets):
+        args.stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(_lib.load().mi_attn_decode_with_tickets(args, ws.tickets.data_ptr(), n_tickets), "mi_attn_decode_with_tickets")
+
+    with pytest.raises(RuntimeError, match="ticket"):
+        entry(B * nkv - 1)
+    for capture in (lambda: entry(B * nq), lambda: call(q, ws, out)):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            capture()
+        for i in (0, 1, 2):
+            q.copy_(qs[i])
+            out.fill_(float("nan"))
+            graph.replay()
+            assert torch.equal(out, want[i]) and not ws.tickets.any()
+    assert getattr(ws[:1], "tickets", None) is None
