@@ -446,6 +446,28 @@ typedef struct mi_decode_args {
     int32_t rotary_interleaved;    /* fused rotary: 0 = rotate-half, 1 = interleaved pairs with fp32 tables */
 } mi_decode_args;
 
+/* What a prefill of `batch` sequences of `seq` tokens leaves in a KV cache (the layout of mi_decode_args): k rotated and v of its
+ * [batch * seq, n_kv_heads, head_dim] rows at positions 0 .. seq - 1, ctx_len[b] = seq; the rotated k also packed in k_rot, for mi_attn_fwd with
+ * position_ids_k == NULL.  Replaces attention.py:836-845 (k) and :861-862 of the reference.  16-bit types, head_dim 64 or 128; table
+ * formats and rotary_interleaved as in mi_attn_args, the arithmetic of mi_rotary / mi_rotary_complex. */
+typedef struct mi_fill_cache_args {
+    const void* k;
+    const void* v;
+    void* k_rot;
+    void* k_cache;
+    void* v_cache;
+    int32_t* ctx_len;
+    const void* rotary_cos;
+    const void* rotary_sin;
+    const int64_t* position_ids;   /* [batch * seq] */
+    int64_t table_rows;
+    int64_t k_stride_token, k_stride_head, v_stride_token, v_stride_head;
+    int64_t cache_stride_batch, cache_stride_token, cache_stride_head;
+    int32_t batch, seq, max_ctx, n_kv_heads, head_dim, dtype, rotary_interleaved;
+    void* stream;
+} mi_fill_cache_args;
+int mi_fill_cache(const mi_fill_cache_args* args);
+
 size_t mi_attn_decode_workspace_bytes(int32_t batch, int32_t n_q_heads, int32_t head_dim, int32_t max_ctx);
 int mi_attn_decode(const mi_decode_args* args);
 

@@ -886,6 +886,86 @@ Tensor op_attention_qkv(const Tensor& qkv, const Tensor& cu_q, const OptTensor& 
     return AttentionQkv::apply(qkv, cu_q, cu_k, &o, at::GradMode::is_enabled() && qkv.requires_grad());
 }
 
+// ---- a layer in one call -----------------------------------------------------------------------------------------------
+// Attention over the rows of a prefill [batch * seq, heads, head_dim] (inference), which leaves rotated k and v in the caches
+// [batch, max_ctx, KV heads, head_dim] and raises ctx_len to seq: two launches.
+Tensor op_prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const Tensor& pos, const Tensor& cos, const Tensor& sin,
+                            bool interleaved, double scale, int64_t batch, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len) {
+    check_qkv(q, k, v, cu, Tensor());
+    TORCH_CHECK(batch > 0 && k.size(0) % batch == 0 && k.size(0) == q.size(0) && k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
+                    k_cache.strides() == v_cache.strides() && k_cache.stride(3) == 1 && k_cache.size(0) == batch && k_cache.size(2) == k.size(1) &&
+                    k_cache.size(3) == k.size(2) && k_cache.scalar_type() == k.scalar_type() && v_cache.scalar_type() == k.scalar_type() &&
+                    ctx_len.scalar_type() == at::kInt && ctx_len.is_contiguous() && ctx_len.numel() == batch && pos.scalar_type() == at::kLong &&
+                    pos.is_contiguous() && pos.numel() == k.size(0) && cos.is_contiguous() && sin.is_contiguous(),
+                "prefill attention: caches, lengths and position ids have to fit the rows");
+    for (const Tensor* t : {&k_cache, &v_cache, &ctx_len, &pos, &cos, &sin}) need_gpu(*t);
+    Launch l(q);
+    const Tensor k_rot = at::empty(k.sizes(), k.options());
+    mi_fill_cache_args a{};
+    a.k = ptr(k); a.v = ptr(v); a.k_rot = ptr(k_rot); a.k_cache = ptr(k_cache); a.v_cache = ptr(v_cache); a.ctx_len = static_cast<int32_t*>(ptr(ctx_len));
+    a.rotary_cos = ptr(cos); a.rotary_sin = ptr(sin); a.position_ids = static_cast<const int64_t*>(ptr(pos)); a.table_rows = cos.size(0);
+    a.k_stride_token = k.stride(0); a.k_stride_head = k.stride(1); a.v_stride_token = v.stride(0); a.v_stride_head = v.stride(1);
+    a.cache_stride_batch = k_cache.stride(0); a.cache_stride_token = k_cache.stride(1); a.cache_stride_head = k_cache.stride(2);
+    a.batch = (int32_t)batch; a.seq = (int32_t)(k.size(0) / batch); a.max_ctx = (int32_t)k_cache.size(1); a.n_kv_heads = (int32_t)k.size(1);
+    a.head_dim = (int32_t)k.size(2); a.dtype = code_of(k); a.rotary_interleaved = interleaved; a.stream = l.stream;
+    check(mi_fill_cache(&a), "mi_fill_cache");
+    return std::get<0>(attn_forward(q, k_rot, v, cu, Tensor(), options(true, scale, 0, 0.0, 0, cos, sin, pos, std::nullopt, interleaved), Tensor()));
+}
+
+// A pre-norm layer on x [batch, seq, hidden]: the same operations, one after the other, as the modules of the layer issue them, with their autograd
+// nodes where gradients are recorded; what it saves is the way through those modules (half of a small layer's forward pass).
+//   norms    [weight, bias (RMSNorm: none)] of either norm
+//   qkv      one weight: per head q, k, v (in_one) or the rows of q, of k and of v; or three.  dense, and in, (gate,) out of the MLP follow.
+//   rotary   0 none, 1 inside the attention core, 2 in front of it; caches: [k, v, ctx_len] of a prefill (rotary 1, inference) or empty
+Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, const std::vector<OptTensor>& norms, double eps1, double eps2, bool layer_norm1,
+                bool layer_norm2, const std::vector<Tensor>& qkv_w, const std::vector<OptTensor>& qkv_b, bool in_one, const std::vector<Tensor>& rest_w,
+                const std::vector<OptTensor>& rest_b, int64_t nq, int64_t nkv, int64_t d, bool causal, double scale, int rotary, bool interleaved,
+                const OptTensor& cos, const OptTensor& sin, const std::vector<Tensor>& caches, bool inference) {
+    TORCH_CHECK(x.dim() == 3 && norms.size() == 4 && norms[0].has_value() && norms[2].has_value() && (qkv_w.size() == 1 || qkv_w.size() == 3) &&
+                    qkv_b.size() == qkv_w.size() && (rest_w.size() == 3 || rest_w.size() == 4) && rest_b.size() == rest_w.size() &&
+                    (caches.empty() || caches.size() == 3),
+                "layer: bad arguments");
+    const int64_t b = x.size(0), s = x.size(1), tokens = b * s;
+    auto [h, n] = op_add_norm(x, std::nullopt, *norms[0], norms[1], eps1, layer_norm1);
+    Tensor ctx;
+    const OptTensor fused_cos = rotary == 1 ? cos : OptTensor(), fused_sin = rotary == 1 ? sin : OptTensor(), fused_pos = rotary == 1 ? pos : OptTensor();
+    if (in_one && rotary != 2) {
+        const Tensor qkv = op_linear(n, qkv_w[0], qkv_b[0], std::nullopt, inference).view({tokens, nq, 3 * d});
+        ctx = op_attention_qkv(qkv, cu, std::nullopt, causal, scale, 0.0, 0, fused_cos, fused_sin, fused_pos, fused_pos, interleaved);
+    } else {
+        Tensor q, k, v;
+        if (in_one) {
+            const Tensor qkv = op_linear(n, qkv_w[0], qkv_b[0], std::nullopt, inference).view({tokens, nq, 3 * d});
+            q = qkv.narrow(2, 0, d); k = qkv.narrow(2, d, d); v = qkv.narrow(2, 2 * d, d);
+        } else if (qkv_w.size() == 1) {
+            const Tensor qkv = op_linear(n, qkv_w[0], qkv_b[0], std::nullopt, inference).view({tokens, nq + 2 * nkv, d});
+            q = qkv.narrow(1, 0, nq); k = qkv.narrow(1, nq, nkv); v = qkv.narrow(1, nq + nkv, nkv);
+        } else {
+            const auto out = op_projections(n, qkv_w, qkv_b, inference);
+            q = out[0].view({tokens, nq, d}); k = out[1].view({tokens, nkv, d}); v = out[2].view({tokens, nkv, d});
+        }
+        if (!caches.empty()) {
+            ctx = op_prefill_attention(q, k, v, cu, *pos, *cos, *sin, interleaved, scale, b, caches[0], caches[1], caches[2]);
+        } else {
+            if (rotary == 2) {
+                q = Rotary::apply(q, *cos, *sin, pos, s, interleaved);
+                k = Rotary::apply(k, *cos, *sin, pos, s, interleaved);
+            }
+            ctx = op_attention(q, k, v, cu, std::nullopt, causal, scale, 0.0, 0, fused_cos, fused_sin, fused_pos, fused_pos, interleaved, false);
+        }
+    }
+    const Tensor a = op_linear(ctx.view({b, s, nq * d}), rest_w[0], rest_b[0], std::nullopt, inference);
+    std::tie(h, n) = op_add_norm(a, h, *norms[2], norms[3], eps2, layer_norm2);
+    Tensor act;
+    if (rest_w.size() == 4) {
+        const auto out = op_projections(n, {rest_w[1], rest_w[2]}, {rest_b[1], rest_b[2]}, inference);
+        act = SwiGlu::apply(out[0], out[1]);
+    } else {
+        act = Gelu::apply(op_linear(n, rest_w[1], rest_b[1], std::nullopt, inference));
+    }
+    return op_linear(act, rest_w.back(), rest_b.back(), h, inference);
+}
+
 // ---- loss --------------------------------------------------------------------------------------------------------------
 // Weighted mean of the cross entropy of logits [rows, vocab], and the accuracy.  The gradient takes the log-sum-exp of the forward
 // pass, so it reads the logits once.
@@ -1248,6 +1328,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("attention", &op_attention);
     def("attention_qkv", &op_attention_qkv);
     def("add_norm", &op_add_norm);
+    def("layer", &op_layer);
+    def("prefill_attention", &op_prefill_attention);
     def("weighted_cross_entropy", &op_weighted_cross_entropy);
     def("linear_cross_entropy", &op_linear_cross_entropy);
     def("decode_attention", &op_decode_attention);

@@ -77,6 +77,72 @@ __global__ __launch_bounds__(kBlock) void rotary_vec_kernel(RotaryParams p) {
     stg_nt(reinterpret_cast<uint4*>(orow + c1), Elem<T>::pack(o1));
 }
 
+// What a prefill leaves in a KV cache, in one launch: k rotated (whole head, rotate-half or interleaved pairs, as the two kernels around this one)
+// into the cache and, packed, for the attention launch that follows; v into the cache; the context lengths.  A thread owns a vector of the
+// first half of a k row and its partner (interleaved: one of either half) or the same two of a v row.  As two rotary launches (q and k; q is now
+// rotated where the attention kernel loads it), two copies and a fill it was five launches a layer.
+struct FillParams {
+    const void *k, *v, *cos, *sin;
+    const int64_t* pos;
+    void *k_out, *k_cache, *v_cache;
+    int32_t* ctx_len;
+    int64_t n_tokens, k_st, k_sh, v_st, v_sh, c_sb, c_st, c_sh, table_rows;
+    int seq, n_heads, batch;
+};
+
+template <typename T, int D, bool PAIRS>
+__global__ __launch_bounds__(kBlock) void fill_cache_kernel(const FillParams p) {
+    constexpr int V = Elem<T>::kVec, HALF = D / 2 / V;
+    const uint32_t item = blockIdx.x * (uint32_t)kBlock + threadIdx.x;        // fewer than 2^32: checked by the entry point
+    if (item < (uint32_t)p.batch) p.ctx_len[item] = p.seq;
+    const uint32_t per_token = 2u * HALF * p.n_heads, token = item / per_token;
+    if (token >= (uint32_t)p.n_tokens) return;
+    const uint32_t rem = item - token * per_token, b = token / (uint32_t)p.seq;
+    const int h = rem / (2 * HALF), c = rem % HALF;
+    const bool value = rem % (2 * HALF) >= HALF;
+    const int64_t t = token, at = (int64_t)b * p.c_sb + (int64_t)(token - b * p.seq) * p.c_st + (int64_t)h * p.c_sh + V * c;
+    const T* src = value ? (const T*)p.v + t * p.v_st + (int64_t)h * p.v_sh + V * c : (const T*)p.k + t * p.k_st + (int64_t)h * p.k_sh + V * c;
+    uint4 lo = *reinterpret_cast<const uint4*>(src), hi = *reinterpret_cast<const uint4*>(src + D / 2);
+    if (value) {
+        T* dst = (T*)p.v_cache + at;
+        *reinterpret_cast<uint4*>(dst) = lo;
+        *reinterpret_cast<uint4*>(dst + D / 2) = hi;
+        return;
+    }
+    int64_t r = p.pos[t];
+    r = r < 0 ? 0 : (r >= p.table_rows ? p.table_rows - 1 : r);
+    float x0[V], x1[V];
+    Elem<T>::unpack(lo, x0);
+    Elem<T>::unpack(hi, x1);
+    if constexpr (PAIRS) {
+        const float *cr = (const float*)p.cos + r * (D / 2) + V / 2 * c, *sr = (const float*)p.sin + r * (D / 2) + V / 2 * c;
+#pragma unroll
+        for (int i = 0; i < V / 2; ++i) {
+            rotate_complex_pair(x0[2 * i], x0[2 * i + 1], cr[i], sr[i]);
+            rotate_complex_pair(x1[2 * i], x1[2 * i + 1], cr[D / 4 + i], sr[D / 4 + i]);
+        }
+    } else {
+        float cA[V], sA[V], cB[V], sB[V];
+        load_table<T, V>((const T*)p.cos + r * D + V * c, cA);
+        load_table<T, V>((const T*)p.sin + r * D + V * c, sA);
+        load_table<T, V>((const T*)p.cos + r * D + D / 2 + V * c, cB);
+        load_table<T, V>((const T*)p.sin + r * D + D / 2 + V * c, sB);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const float a = __builtin_fmaf(x0[i], cA[i], -(x1[i] * sA[i])), d = __builtin_fmaf(x1[i], cB[i], x0[i] * sB[i]);
+            x0[i] = a;
+            x1[i] = d;
+        }
+    }
+    lo = Elem<T>::pack(x0);
+    hi = Elem<T>::pack(x1);
+    T *dst = (T*)p.k_cache + at, *out = (T*)p.k_out + (t * p.n_heads + h) * D + V * c;
+    *reinterpret_cast<uint4*>(dst) = lo;
+    *reinterpret_cast<uint4*>(dst + D / 2) = hi;
+    *reinterpret_cast<uint4*>(out) = lo;
+    *reinterpret_cast<uint4*>(out + D / 2) = hi;
+}
+
 template <typename T, typename TT>
 __global__ __launch_bounds__(kBlock) void rotary_scalar_kernel(RotaryParams p) {
     const int half = p.rot_dim / 2;
@@ -193,4 +259,36 @@ extern "C" int mi_rotary_complex(const void* x, void* out, const float* cos, con
         rotary_complex_kernel<T><<<dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream>>>(p);
     });
     return mi_check_launch("rotary_complex");
+}
+
+extern "C" int mi_fill_cache(const mi_fill_cache_args* a) {
+    if (!a) return mi_fail(MI_E_NULL, "fill_cache: args is null");
+    if (a->batch <= 0 || a->seq <= 0 || a->n_kv_heads <= 0 || (a->head_dim != 64 && a->head_dim != 128) || a->max_ctx < a->seq ||
+        (int64_t)a->batch * a->seq > 0x7fffffffLL || a->table_rows <= 0)
+        return mi_fail(MI_E_SHAPE, "fill_cache: batch %d x %d tokens, %d heads of %d (64 or 128), a cache of %d", a->batch, a->seq, a->n_kv_heads, a->head_dim, a->max_ctx);
+    if (a->dtype != MI_BF16 && a->dtype != MI_F16) return mi_fail(MI_E_DTYPE, "fill_cache: bf16 or f16 tensors (dtype code %d)", a->dtype);
+    if (!a->k || !a->v || !a->k_rot || !a->k_cache || !a->v_cache || !a->ctx_len || !a->rotary_cos || !a->rotary_sin || !a->position_ids)
+        return mi_fail(MI_E_NULL, "fill_cache: null pointer");
+    if (!mi_aligned16(a->k) || !mi_aligned16(a->v) || !mi_aligned16(a->k_rot) || !mi_aligned16(a->k_cache) || !mi_aligned16(a->v_cache) ||
+        !mi_aligned16(a->rotary_cos) || !mi_aligned16(a->rotary_sin))
+        return mi_fail(MI_E_ALIGN, "fill_cache: tensors must be 16-byte aligned");
+    for (const int64_t s : {a->k_stride_token, a->k_stride_head, a->v_stride_token, a->v_stride_head, a->cache_stride_batch, a->cache_stride_token, a->cache_stride_head})
+        if (s % 8 != 0) return mi_fail(MI_E_ALIGN, "fill_cache: strides must be multiples of 8 elements");
+    FillParams p{};
+    p.k = a->k; p.v = a->v; p.cos = a->rotary_cos; p.sin = a->rotary_sin; p.pos = a->position_ids;
+    p.k_out = a->k_rot; p.k_cache = a->k_cache; p.v_cache = a->v_cache; p.ctx_len = a->ctx_len;
+    p.seq = a->seq; p.batch = a->batch; p.n_heads = a->n_kv_heads; p.n_tokens = (int64_t)a->batch * a->seq; p.table_rows = a->table_rows;
+    p.k_st = a->k_stride_token; p.k_sh = a->k_stride_head; p.v_st = a->v_stride_token; p.v_sh = a->v_stride_head;
+    p.c_sb = a->cache_stride_batch; p.c_st = a->cache_stride_token; p.c_sh = a->cache_stride_head;
+    const int64_t items = p.n_tokens * a->n_kv_heads * (a->head_dim / 8), blocks = (items + kBlock - 1) / kBlock;     // more items than sequences
+    if (items > 0xffffff00LL) return mi_fail(MI_E_SHAPE, "fill_cache: more than 2^32 vectors");
+    const auto go = [&](auto t) {
+        using T = decltype(t);
+        const auto kernel = a->head_dim == 64 ? (a->rotary_interleaved ? fill_cache_kernel<T, 64, true> : fill_cache_kernel<T, 64, false>)
+                                              : (a->rotary_interleaved ? fill_cache_kernel<T, 128, true> : fill_cache_kernel<T, 128, false>);
+        kernel<<<dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)a->stream>>>(p);
+    };
+    if (a->dtype == MI_BF16) go(__bf16{});
+    else go(_Float16{});
+    return mi_check_launch("fill_cache");
 }

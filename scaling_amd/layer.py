@@ -10,7 +10,7 @@ from typing import Callable, List, Optional
 import torch
 
 from .config import MLPType, TransformerArchitectureConfig
-from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm, idle_dropout, one_token_each
+from .nn import ParallelMLP, ParallelSelfAttention, ParallelSwiGLUMLP, RMSNorm, _direct, _unhooked, decode_layer, fuses_residual, get_norm, idle_dropout, layer_in_one_call, one_token_each
 
 
 class InferenceSettings:
@@ -119,6 +119,10 @@ class TransformerLayer(torch.nn.Module):
             if h is not None:
                 return self._next(x, h)
         if self._own_blocks() and fuses_residual(self.input_layernorm) and fuses_residual(self.post_attention_layernorm):
+            if x.attention_scores_manipulation is None:
+                h = layer_in_one_call(self, x.activations, x.cumulative_seq_lengths, x.position_ids, use_cache, reset_cache, cache_index)
+                if h is not None:
+                    return self._next(x, h)
             # the same arithmetic as attention_block and mlp_block, with the residual stream taken through the norms (and, where
             # nothing comes between, the last projection): its sums and the sums of its gradients need no passes of their own
             h, n = self.input_layernorm.with_residual(x.activations)

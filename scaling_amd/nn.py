@@ -620,13 +620,18 @@ class ParallelSelfAttention(torch.nn.Module):
             return self.rotary_embedding.max_seq_length
         raise ValueError("set max_cache_length when the module has no rotary table to size the cache from")
 
-    def _fill_cache(self, k: torch.Tensor, v: torch.Tensor, b: int, s: int, cache_index: int) -> None:
-        nkv, d = self.num_kv_heads_per_partition, self.hidden_size_per_attention_head
+    def _cache_for(self, b: int, s: int, dtype: torch.dtype, device: torch.device, cache_index: int) -> KVCache:
+        """The cache that a prefill of b sequences of s tokens fills: the one that is there, if it suits."""
         cap = max(self._cache_capacity(), s)
         cache = self.cache.get(cache_index)
         if cache is None or cache.k.shape[0] != b or cache.max_ctx < cap:
-            cache = KVCache(b, cap, nkv, d, k.dtype, k.device)
+            cache = KVCache(b, cap, self.num_kv_heads_per_partition, self.hidden_size_per_attention_head, dtype, device)
             self.cache[cache_index] = cache
+        return cache
+
+    def _fill_cache(self, k: torch.Tensor, v: torch.Tensor, b: int, s: int, cache_index: int) -> None:
+        nkv, d = self.num_kv_heads_per_partition, self.hidden_size_per_attention_head
+        cache = self._cache_for(b, s, k.dtype, k.device, cache_index)
         cache.k[:, :s].copy_(k.detach().view(b, s, nkv, d))
         cache.v[:, :s].copy_(v.detach().view(b, s, nkv, d))
         cache.length = s
@@ -683,6 +688,64 @@ class ParallelSelfAttention(torch.nn.Module):
             cache.workspace = ops.decode_workspace(b, nq, d, cache.max_ctx, q.device)
         return ops.decode_attention(self._decode_operand(q), cache.k, cache.v, cache.ctx_len, self._decode_operand(k),
                                     self._decode_operand(v), rotary=rotary, softmax_scale=self.softmax_scale, workspace=cache.workspace)
+
+
+def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tensor, position_ids: Optional[torch.Tensor], use_cache: bool,
+                      reset_cache: bool, cache_index: int) -> Optional[torch.Tensor]:
+    """The output of a layer whose norms and MLP may be passed by (`fuses_residual`) in one native call of the operations its modules would
+    issue; with a cache: of a prefill.  None, with nothing done, where a module below is not the package's own as it is or the operands are not what
+    the kernels take: the modules then compute or refuse it."""
+    att, mlp, norm1, norm2 = layer.self_attention, layer.mlp, layer.input_layernorm, layer.post_attention_layernorm
+    sdpa, rot, dtype, training = att.scaled_dot_product_attention, att.rotary_embedding, att.dtype, layer.training
+    if not (x.is_cuda and x.dim() == 3 and x.dtype == dtype and x.numel() > 0 and not torch.is_autocast_enabled() and type(att) is ParallelSelfAttention and
+            _unhooked(att) and fuses_residual(mlp) and idle_dropout(layer.dropout_attention) and idle_dropout(layer.dropout_mlp) and
+            not att.key_query_norm and type(sdpa) is ScaledDotProductAttention and "forward_tokens" not in sdpa.__dict__ and
+            "forward_qkv" not in sdpa.__dict__ and not (training and sdpa.dropout_p > 0.0) and
+            (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex))):
+        return None
+    swiglu = type(mlp) is ParallelSwiGLUMLP
+    rest = (att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out) if swiglu else (att.dense, mlp.dense_in, mlp.dense_out)
+    into = (att.query_key_value,) if att.qkv_in_one else (att.query, att.key, att.value)
+    if not (_direct(*into, *rest) and all(m.training == training for m in (att, sdpa, mlp, *into, *rest))):
+        return None
+    b, s, hidden = x.shape
+    pos = None if position_ids is None else position_ids.reshape(-1).contiguous()
+    cu = cumulative_seq_lengths.to(torch.int32)
+    inference = not torch.is_grad_enabled() and not training
+    if not (cu.is_cuda and cu.is_contiguous() and (pos is None or (pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == b * s))):
+        return None
+    if use_cache and not (inference and reset_cache and att.causal and not att.qkv_in_one and att._fusable_rotary and pos is not None):
+        return None
+    if inference and not att.qkv_in_one:
+        w, bias = att._fused_qkv()
+        qkv_w, qkv_b = [w], [bias]
+    else:
+        qkv_w, qkv_b = [m.weight for m in into], [m.bias for m in into]
+    norms = [p for n in (norm1, norm2) for p in (n.weight, n.bias if type(n) is LayerNorm else None)]
+    rest_w, rest_b = [m.weight for m in rest], [m.bias for m in rest]
+    if ops._taken_over((x, *norms, *qkv_w, *qkv_b, *rest_w, *rest_b)) or any(p is not None and (p.dtype != dtype or not p.is_cuda) for p in (*norms, *qkv_w, *rest_w)) or \
+            norm1.weight.shape[0] != hidden or norm2.weight.shape[0] != hidden:
+        return None
+    if use_cache:
+        assert att._rows_are_single_documents(cu, b, s), "sequence packing is not supported with cache"
+    elif reset_cache:
+        att.cache[cache_index] = None
+    att._check_positions(pos)
+    nq, nkv, d = att.num_attention_heads, att.num_kv_heads_per_partition, att.hidden_size_per_attention_head
+    cos = sin = None
+    kind, interleaved = 0, False
+    if rot is not None:
+        cos, sin = rot.tables()
+        kind, interleaved = (1 if att._fusable_rotary and pos is not None else 2), type(rot) is RotaryEmbeddingComplex
+    caches = []
+    if use_cache:
+        cache = att._cache_for(b, s, dtype, x.device, cache_index)
+        caches = [cache.k, cache.v, cache.ctx_len]
+    h = ops.layer(x, cu, pos, norms, norm1.eps, norm2.eps, type(norm1) is LayerNorm, type(norm2) is LayerNorm, qkv_w, qkv_b, att.qkv_in_one, rest_w, rest_b,
+                  nq, nkv, d, att.causal, sdpa.softmax_scale, kind, interleaved, cos, sin, caches, not training)
+    if use_cache:
+        cache.length = s
+    return h
 
 
 def one_token_each(x: torch.Tensor) -> bool:

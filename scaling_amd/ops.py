@@ -541,6 +541,11 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return out
 
 
+def layer(*arguments) -> torch.Tensor:
+    """A pre-norm layer in one native call (csrc/host.cpp op_layer); the callers check what it takes."""
+    return _lib.host().layer(*arguments)
+
+
 ROWS_MAX = 16   # MI_ROWS_MAX
 
 

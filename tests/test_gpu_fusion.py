@@ -343,3 +343,70 @@ def test_weight_gradients_through_a_transposed_operand(rows, ins, outs):
         a, b = dy[:, pick].double().t().contiguous(), x.detach().double()
         bound = 2.0 ** -8 * (a @ b).abs() + (rows + 1) * 2.0 ** -24 * (a.abs() @ b.abs())
         assert bool(((w.grad[pick].double() - a @ b).abs() <= bound * 1.01).all())
+
+
+# norms, MLPs, projections, types and rotaries of a layer; a step, and the two forms of a pass without gradients
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("default,options", [
+    (True, {}), (False, {}), (True, dict(relative_position_embedding_type="none")), (False, dict(rotary_percentage=0.5)),
+    (False, dict(relative_position_embedding_type="rotary_complex")), (True, dict(relative_position_embedding_type="rotary_complex")),
+    (False, dict(causal=False)),
+])
+def test_layer_in_one_call_equals_its_modules(dtype, default, options):
+    layer = _layer(dtype, default, **options)
+    x = torch.randn(2, 93, 256, generator=torch.Generator().manual_seed(5)).to(layer.self_attention.dtype).to(DEV)
+    dy = torch.randn(2, 93, 256, generator=torch.Generator().manual_seed(6)).to(x.dtype).to(DEV)
+    io = TransformerLayerIO(activations=x, position_ids=(torch.arange(93, device=DEV) % 60).repeat(2, 1),
+                            cumulative_seq_lengths=torch.tensor([0, 60, 93, 153, 186], dtype=torch.int32, device=DEV))
+
+    def run(train, grad):
+        layer.train(train)
+        x.grad = None
+        x.requires_grad_(grad)
+        for p in layer.parameters():
+            p.grad = None
+        with torch.set_grad_enabled(grad):
+            out = layer(io).activations
+        if not grad:
+            return [out]
+        out.backward(dy)
+        return [out.detach(), x.grad] + [p.grad for p in layer.parameters()]
+
+    for train, grad in ((True, True), (False, True), (True, False), (False, False)):
+        native = run(train, grad)
+        seen = []
+        handle = layer.self_attention.register_forward_hook(lambda *a: seen.append(1))      # whoever watches a module sees it called
+        modules = run(train, grad)
+        handle.remove()
+        assert seen == [1]
+        for i, (a, b) in enumerate(zip(native, modules)):
+            assert torch.equal(a, b), (train, grad, i)
+
+
+@pytest.mark.parametrize("b,s,max_ctx,nkv,d", [(1, 1, 1, 1, 64), (3, 67, 80, 2, 64), (2, 130, 130, 8, 128)])
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prefill_attention_fills_the_cache(b, s, max_ctx, nkv, d, interleaved, dtype):
+    """The rotated rows and the rest of the cache, the lengths and the attention of the launches that it replaces."""
+    nq, g = 2 * nkv, torch.Generator().manual_seed(s)
+    qkv = torch.randn(b * s, nq + 2 * nkv, d, generator=g).to(dtype).to(DEV)
+    q, k, v = qkv[:, :nq], qkv[:, nq:nq + nkv], qkv[:, nq + nkv:]
+    pos = torch.arange(s, device=DEV).repeat(b) + 3
+    ang = torch.outer(torch.arange(max_ctx + 3).float(), 1.0 / (10000.0 ** (torch.arange(0, d, 2).float() / d))).to(DEV)
+    cos, sin = (t if interleaved else torch.cat((t, t), -1).to(dtype) for t in (ang.cos(), ang.sin()))
+    cu = torch.arange(0, b * s + 1, s, dtype=torch.int32, device=DEV)
+    kc, vc = (torch.full((b, nkv, max_ctx, d), 7.0, dtype=dtype, device=DEV).transpose(1, 2) for _ in range(2))
+    ctx = torch.zeros(b, dtype=torch.int32, device=DEV)
+    o = _lib.host().prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, d ** -0.5, b, kc, vc, ctx)
+    rotate = ops.rotary_embedding_complex if interleaved else ops.rotary_embedding
+    k_rot = rotate(k, cos, sin, pos)
+    got = kc[:, :s].reshape(b * s, nkv, d)
+    if dtype == torch.float16:
+        # the rotary kernel rounds some of its float32 sums twice (float32, float16) and some once (mixed-precision fma): one ulp apart
+        assert torch.allclose(got.float(), k_rot.float(), rtol=2.0 ** -10, atol=2.0 ** -24)
+        k_rot = got.contiguous()
+    assert torch.equal(got, k_rot) and torch.equal(vc[:, :s].reshape(b * s, nkv, d), v)
+    assert bool((kc[:, s:] == 7).all()) and bool((vc[:, s:] == 7).all()) and ctx.tolist() == [s] * b
+    assert torch.equal(o, ops.attention_forward(q, k_rot, v, cu, None, True, d ** -0.5, rotary=(cos, sin, pos, None))[0])
+    with pytest.raises(RuntimeError, match="fit the rows"):
+        _lib.host().prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, d ** -0.5, b, kc, vc, ctx[:0])
