@@ -9,9 +9,9 @@
 //     O^T[d][head]   += V^T * P^T   A = V^T read from a transposed per-wavefront LDS copy of the chunk
 // Partial (max, sum, O) per split go to a workspace and are merged by the last workgroup of the splits to arrive (with tickets) or by a
 // second kernel (none of it with a single split).
-// The wavefront whose keys include the new token first appends the new K/V row in place (instead of the
-// reference's torch.cat), rotated, and then reads it back with the rest of its chunk; the query is rotated while its
-// fragments are loaded.  (A launch of its own for the append took 3 - 5 us: a third of a step at batch 1.)
+// The wavefront whose keys include the new token appends the new K/V row in place (instead of the
+// reference's torch.cat), rotated, and puts the same bits into its operands of that chunk; the query is rotated while the
+// first chunk is on its way.  (A launch of its own for the append took 3 - 5 us: a third of a step at batch 1.)
 #include "attn_common.h"
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
@@ -29,6 +29,7 @@ struct DecodeParams {
     const float* cos32; const float* sin32;   // interleaved-pair rotary: fp32 tables [table_rows, D / 2]
     int batch, max_ctx, nq, nkv, n_rep, n_splits;
     int n_hc;      // chunks of up to 16 query heads per KV head (a workgroup serves one chunk)
+    uint32_t splits_m, groups_m, hc_m;   // for divide(): by n_splits, nkv * n_hc and n_hc
     int64_t c_sb, c_st, c_sh;
     int64_t q_sb, kn_sb, vn_sb;   // element strides between sequences of q / k_new / v_new
     float scale_log2;
@@ -43,35 +44,6 @@ __device__ __forceinline__ f32x4v mfma_16x16x32(elem8_t a, elem8_t b, f32x4v c) 
 #else
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 #endif
-}
-
-// ---- in-place append of the new K/V row (optionally rotated) by one wavefront -------------------------
-template <int D>
-__device__ __forceinline__ void append_row(const DecodeParams& p, int b, int kvh, int ctx, int lane) {
-    // one lane per 8-feature vector of the first half
-    if (lane >= D / 16) return;
-    const int c = lane;
-    const int64_t src = (int64_t)b * p.kn_sb + (int64_t)kvh * D + 8 * c;
-    const int64_t src_v = (int64_t)b * p.vn_sb + (int64_t)kvh * D + 8 * c;
-    const int64_t dst = (int64_t)b * p.c_sb + (int64_t)(ctx - 1) * p.c_st + (int64_t)kvh * p.c_sh + 8 * c;
-    uint4 lo = ld128(p.k_new + src), hi = ld128(p.k_new + src + D / 2);
-    const uint4 vlo = ld128(p.v_new + src_v), vhi = ld128(p.v_new + src_v + D / 2);
-    if (p.cos != nullptr) {
-        int64_t pos = p.pos[b];
-        pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
-        rotate_pair(lo, hi, ld128(p.cos + pos * D + 8 * c), ld128(p.sin + pos * D + 8 * c), 1.0f);
-    } else if (p.cos32 != nullptr) {
-        int64_t pos = p.pos[b];
-        pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
-        const float* cr = p.cos32 + pos * (D / 2) + 4 * c;   // features 8 c .. + 8 = pairs 4 c .. + 4
-        const float* sr = p.sin32 + pos * (D / 2) + 4 * c;
-        rotate_interleaved(lo, ld128(cr), ld128(sr), 1.0f);
-        rotate_interleaved(hi, ld128(cr + D / 4), ld128(sr + D / 4), 1.0f);
-    }
-    st128(p.kc + dst, lo);
-    st128(p.kc + dst + D / 2, hi);
-    st128(p.vc + dst, vlo);
-    st128(p.vc + dst + D / 2, vhi);
 }
 
 // ---- merge of the splits ------------------------------------------------------------------------------
@@ -133,7 +105,7 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, int64_t bh, 
 // is the attention output and goes straight to `o`, otherwise the partial goes to the workspace.
 // ROT: 0 = q as it is, 1 = rotate-half rotary on the q load, 2 = interleaved-pair rotary on the q load.
 template <int D, int ROT, int NWV>
-__global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeParams p) {
+__global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeParams args) {
     constexpr int kThreads = 64 * NWV;
     constexpr int KS = D / 32;          // contraction steps of Q K^T (32 features each)
     constexpr int DT = D / 16;          // 16-row tiles of O^T
@@ -150,63 +122,74 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, G = lane >> 4;
 
-    const int split = blockIdx.x % p.n_splits;
-    const int kv_hc = (blockIdx.x / p.n_splits) % (p.nkv * p.n_hc);
-    const int kvh = kv_hc / p.n_hc, hc = kv_hc - kvh * p.n_hc;
-    const int b = blockIdx.x / (p.n_splits * p.nkv * p.n_hc);
+    // All arguments at once: read where they are used they are four trips of the scalar cache, one after the other, in front of the first load.
+    DecodeParams p = args;
+    arrived(p.q, p.kc, p.vc, p.o, p.ctx_len, p.k_new, p.v_new, p.max_ctx, p.nq, p.nkv, p.n_rep, p.n_splits, p.n_hc, p.splits_m, p.groups_m, p.hc_m);
+    arrived(p.c_sb, p.c_st, p.c_sh, p.q_sb, p.kn_sb, p.vn_sb, p.scale_log2, p.ws_o, p.ws_ml, p.tickets);
+    if constexpr (ROT == 1) arrived(p.cos, p.sin, p.pos, p.table_rows);
+    if constexpr (ROT == 2) arrived(p.cos32, p.sin32, p.pos, p.table_rows);
+
+    const int split = blockIdx.y;
+    const int b = divide(blockIdx.x, p.nkv * p.n_hc, p.groups_m), kv_hc = blockIdx.x - b * p.nkv * p.n_hc;
+    const int kvh = divide(kv_hc, p.n_hc, p.hc_m), hc = kv_hc - kvh * p.n_hc;
     // this workgroup's query heads: head0 .. head0 + n_heads of the group (groups of more than 16 heads take
     // several workgroups, each reading the group's K / V once)
     const int head0 = kvh * p.n_rep + 16 * hc;
     const int n_heads = min(16, p.n_rep - 16 * hc);
 
     int ctx = p.ctx_len[b];
+    int64_t pos = 0;                    // requested with ctx: the rows of the rotary tables need not wait for anything else
+    if constexpr (ROT != 0) {
+        pos = p.pos[b];
+        pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+    }
     const bool append = p.k_new != nullptr && ctx >= 1 && ctx <= p.max_ctx;
     ctx = ctx < 0 ? 0 : (ctx > p.max_ctx ? p.max_ctx : ctx);
     // keys of this split: [s0, s1), split length rounded up to whole workgroup iterations
-    int per = (ctx + p.n_splits - 1) / p.n_splits;
+    int per = divide(ctx + p.n_splits - 1, p.n_splits, p.splits_m);
     per = (per + NWV * kChunk - 1) / (NWV * kChunk) * (NWV * kChunk);
     const int s0 = split * per;
     const int s1 = min(ctx, s0 + per);
     const int n_iter = s1 > s0 ? (s1 - s0 + NWV * kChunk - 1) / (NWV * kChunk) : 0;
 
-    // The last key of this split is the new token: the wavefront whose chunk (iteration it_new) holds it writes it now and waits
-    // for its own stores before that chunk is requested.  (Groups of more than 16 heads: each of their workgroups does,
-    // with the same bytes, since each reads the row.)
+    // The last key of this split is the new token: the wavefront whose chunk (iteration it_new) holds it writes it to the cache and
+    // replaces that key's operands, whose loads do not wait for the store and may bring what the row held before.  (Groups of more than 16 heads: each of
+    // their workgroups does, with the same bytes, since each reads the row.)
     const int c_new = (ctx - 1 - s0) / kChunk;
     const int it_new = append && ctx - 1 >= s0 && ctx - 1 < s1 && c_new % NWV == wave ? c_new / NWV : -1;   // wave-uniform
-    if (it_new >= 0) append_row<D>(p, b, kvh, ctx, lane);
 
-    // Q^T fragments: column = head slot l16 (valid when < n_rep), contraction = features 32*ks + 8*G + i
-    elem8_t qf[KS];
+    // A small call is a chain of trips to memory.  Whatever depends on nothing but ctx and pos is requested before the first of it is used, in the order of
+    // use: q, the new row, rows of the rotary tables, the first chunk.  (With the arguments in one trip too, us in a graph, before / after: batch 1, 32 / 8
+    // heads of 128, 1500 keys 7.9 / 7.3, 200 keys 6.7 / 5.9; batch 3, 16 / 4 of 64, 224 keys 5.1 / 4.3; batch 32, 32 / 8 of 128, 4096 keys 80.6 / 79.7.)
+    // Q^T fragments: column = head slot l16 (valid when < n_rep), contraction = features 32*ks + 8*G + i; the new K row alike, in every column
+    uint4 raw[KS], kn[KS] = {}, vn[V_PER_LANE] = {};
     {
         const int hs = l16 < n_heads ? l16 : 0;
         const elem_t* qr = p.q + (int64_t)b * p.q_sb + (int64_t)(head0 + hs) * D + 8 * G;
-        uint4 raw[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) raw[ks] = *reinterpret_cast<const uint4*>(qr + 32 * ks);
-        if constexpr (ROT == 1) {
-            int64_t pos = p.pos[b];
-            pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+    }
+    if (it_new >= 0) {
+        const elem_t* kr = p.k_new + (int64_t)b * p.kn_sb + (int64_t)kvh * D + 8 * G;
+        const elem_t* vr = p.v_new + (int64_t)b * p.vn_sb + (int64_t)kvh * D;
 #pragma unroll
-            for (int ks = 0; ks < KS / 2; ++ks) {
-                const uint4 cv = *reinterpret_cast<const uint4*>(p.cos + pos * D + 32 * ks + 8 * G);
-                const uint4 sv = *reinterpret_cast<const uint4*>(p.sin + pos * D + 32 * ks + 8 * G);
-                rotate_pair(raw[ks], raw[ks + KS / 2], cv, sv, 1.0f);
-            }
-        } else if constexpr (ROT == 2) {
-            int64_t pos = p.pos[b];
-            pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+        for (int ks = 0; ks < KS; ++ks) kn[ks] = ld128(kr + 32 * ks);
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {   // features 32 ks + 8 G .. + 8 = pairs 16 ks + 4 G .. + 4
-                const float* cr = p.cos32 + pos * (D / 2) + 16 * ks + 4 * G;
-                const float* sr = p.sin32 + pos * (D / 2) + 16 * ks + 4 * G;
-                rotate_interleaved(raw[ks], ld128(cr), ld128(sr), 1.0f);
-            }
+        for (int j = 0; j < V_PER_LANE; ++j) vn[j] = ld128(vr + 8 * ((lane + 64 * j) % (D / 8)));
+    }
+    uint4 cv[KS / 2 + 1], sv[KS / 2 + 1];              // rotate-half: features 32 ks + 8 G .. + 8 of the first half
+    uint4 ci[KS], si[KS];                              // interleaved: pairs 16 ks + 4 G .. + 4
+    if constexpr (ROT == 1) {
+#pragma unroll
+        for (int ks = 0; ks < KS / 2; ++ks) {
+            cv[ks] = ld128(p.cos + pos * D + 32 * ks + 8 * G);
+            sv[ks] = ld128(p.sin + pos * D + 32 * ks + 8 * G);
         }
+    } else if constexpr (ROT == 2) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            if (l16 >= n_heads) raw[ks] = make_uint4(0, 0, 0, 0);
-            qf[ks] = __builtin_bit_cast(elem8_t, raw[ks]);
+            ci[ks] = ld128(p.cos32 + pos * (D / 2) + 16 * ks + 4 * G);
+            si[ks] = ld128(p.sin32 + pos * (D / 2) + 16 * ks + 4 * G);
         }
     }
 
@@ -227,11 +210,9 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
         elem8_t kf[2][KS];
         uint4 vraw[V_PER_LANE][4];
     };
-    auto load_chunk = [&](ChunkRegs& c, int it) {
-        const int key0 = s0 + (NWV * it + wave) * kChunk;
-        if (key0 >= s1) return;
-        if (it == it_new) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the appended row is in the cache
-        const int last = s1 - 1;
+    // (a wavefront without keys asks for the last row or, of an empty cache, the first)
+    auto request = [&](ChunkRegs& c, int it) {
+        const int key0 = s0 + (NWV * it + wave) * kChunk, last = max(s1 - 1, 0);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int tok = min(key0 + 16 * t + l16, last);
@@ -251,9 +232,28 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
             }
         }
     };
-    auto process_chunk = [&](const ChunkRegs& c, int it) {
+    elem8_t qf[KS];
+    // the new row in place of what its key (and keys past it, which read the same row) brought
+    auto put_new = [&](ChunkRegs& c, int it) {
+        const int key0 = s0 + (NWV * it + wave) * kChunk, last = s1 - 1;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                if (key0 + 16 * t + l16 >= last) c.kf[t][ks] = __builtin_bit_cast(elem8_t, kn[ks]);
+#pragma unroll
+        for (int j = 0; j < V_PER_LANE; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (key0 + 4 * ((lane + 64 * j) / (D / 8)) + r >= last) c.vraw[j][r] = vn[j];
+    };
+    auto load_chunk = [&](ChunkRegs& c, int it) {
+        if (s0 + (NWV * it + wave) * kChunk < s1) request(c, it);
+    };
+    auto process_chunk = [&](ChunkRegs& c, int it) {
         const int key0 = s0 + (NWV * it + wave) * kChunk;
         const bool active = key0 < s1;          // wave-uniform
+        if (it == it_new) put_new(c, it);
         // Each wavefront owns its LDS chunk; the LDS pipeline executes one wavefront's accesses in program
         // order, so wavefront-scope fences (compiler ordering only) are enough and the wavefronts of a
         // workgroup never wait for each other inside the loop.
@@ -314,7 +314,34 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     };
 
     ChunkRegs ra, rb;
-    if (n_iter > 0) load_chunk(ra, 0);
+    request(ra, 0);                                    // without a branch, behind which q's arrival would be waited for as if this had not been sent
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ROT == 1) {
+#pragma unroll
+        for (int ks = 0; ks < KS / 2; ++ks) {
+            rotate_pair(raw[ks], raw[ks + KS / 2], cv[ks], sv[ks], 1.0f);
+            if (it_new >= 0) rotate_pair(kn[ks], kn[ks + KS / 2], cv[ks], sv[ks], 1.0f);
+        }
+    } else if constexpr (ROT == 2) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            rotate_interleaved(raw[ks], ci[ks], si[ks], 1.0f);
+            if (it_new >= 0) rotate_interleaved(kn[ks], ci[ks], si[ks], 1.0f);
+        }
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        if (l16 >= n_heads) raw[ks] = make_uint4(0, 0, 0, 0);
+        qf[ks] = __builtin_bit_cast(elem8_t, raw[ks]);
+    }
+    if (it_new >= 0) {
+        const int64_t dst = (int64_t)b * p.c_sb + (int64_t)(ctx - 1) * p.c_st + (int64_t)kvh * p.c_sh;
+        if (l16 == 0) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) st128(p.kc + dst + 32 * ks + 8 * G, kn[ks]);
+        }
+        if (lane < D / 8) st128(p.vc + dst + 8 * lane, vn[0]);
+    }
     for (int it = 0; it < n_iter; it += 2) {
         if (it + 1 < n_iter) load_chunk(rb, it + 1);
         process_chunk(ra, it);
@@ -326,7 +353,6 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 
     // ---- merge the four wavefronts, emit the split partial -----------------------------------------
     l_i = quad_sum(l_i);
-    __syncthreads();
     if (G == 0) { wm_lds[wave][l16] = m_i; wl_lds[wave][l16] = l_i; }
     if (l16 < n_heads) {
 #pragma unroll
@@ -369,7 +395,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        int32_t* ticket = p.tickets + blockIdx.x / p.n_splits;
+        int32_t* ticket = p.tickets + blockIdx.x;
         const int arrived = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last_lds = arrived == p.n_splits - 1;
         if (arrived == p.n_splits - 1) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
@@ -422,13 +448,13 @@ int choose_splits(int batch, int nkv, int max_ctx) {
 
 // rot: 0 = none, 1 = rotate-half, 2 = interleaved pairs
 template <int D, int NWV> int launch_split(const DecodeParams& p, int rot, hipStream_t st) {
-    const unsigned grid = (unsigned)p.batch * p.nkv * p.n_hc * p.n_splits;
-    if (rot == 2) decode_split_kernel<D, 2, NWV><<<dim3(grid), dim3(64 * NWV), 0, st>>>(p);
+    const dim3 grid((unsigned)p.batch * p.nkv * p.n_hc, p.n_splits);
+    if (rot == 2) decode_split_kernel<D, 2, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
     else if (rot == 1) {
         // rotate-half pairs feature i with i + D / 2: the same lane holds both only when D / 32 is even
-        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV><<<dim3(grid), dim3(64 * NWV), 0, st>>>(p);
+        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
         else return mi_fail(MI_E_SHAPE, "attn_decode: fused rotate-half rotary needs head_dim 64 or 128");
-    } else decode_split_kernel<D, 0, NWV><<<dim3(grid), dim3(64 * NWV), 0, st>>>(p);
+    } else decode_split_kernel<D, 0, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
     return mi_check_launch("decode_split");
 }
 
@@ -505,6 +531,7 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
     p.table_rows = (int)a->rotary_table_rows;
     p.batch = a->batch; p.max_ctx = a->max_ctx; p.nq = a->n_q_heads; p.nkv = a->n_kv_heads;
     p.n_rep = a->n_q_heads / a->n_kv_heads; p.n_splits = splits; p.n_hc = n_hc;
+    p.splits_m = divide_m(splits); p.groups_m = divide_m((uint32_t)(p.nkv * n_hc)); p.hc_m = divide_m(n_hc);
     p.c_sb = a->cache_stride_batch; p.c_st = a->cache_stride_token; p.c_sh = a->cache_stride_head;
     p.q_sb = a->q_stride_batch ? a->q_stride_batch : (int64_t)a->n_q_heads * a->head_dim;
     p.kn_sb = a->k_new_stride_batch ? a->k_new_stride_batch : (int64_t)a->n_kv_heads * a->head_dim;

@@ -168,6 +168,23 @@ template <int WIDTH> __device__ __forceinline__ int group_max(int v) {
     return (int)group_reduce_bits<WIDTH>((uint32_t)v, [](uint32_t a, uint32_t b) { return (uint32_t)max((int)a, (int)b); });
 }
 
+// Values that are in registers from here on (the compiler otherwise loads an argument right before its use).
+template <typename V> __device__ __forceinline__ void arrived1(V& v) { asm volatile("" : "+s"(v)); }
+template <typename V> __device__ __forceinline__ void arrived1(V*& v) {   // a pointer to global memory stays one
+    uintptr_t at = (uintptr_t)v;
+    asm volatile("" : "+s"(at));
+    v = (V*)(__attribute__((address_space(1))) V*)at;
+}
+template <typename... V> __device__ __forceinline__ void arrived(V&... v) { (arrived1(v), ...); }
+
+// u / d for u < 2^31 by the high half of u * m with m = 2^32 / d + 1, which is the quotient or one more: five scalar instructions in a row, where the
+// compiler's division is about forty.
+inline uint32_t divide_m(uint32_t d) { return d > 1 ? (uint32_t)((1ull << 32) / d + 1) : 0; }
+__device__ __forceinline__ int divide(uint32_t u, uint32_t d, uint32_t m) {
+    const uint32_t q = __umulhi(u, m);
+    return (int)(m == 0 ? u : q * d > u ? q - 1 : q);
+}
+
 #define MI_DISPATCH_DTYPE(dtype, ...)                                       \
     switch (dtype) {                                                        \
         case MI_BF16: { using T = __bf16; __VA_ARGS__; break; }             \

@@ -24,15 +24,6 @@ constexpr int kMaxWeights = MI_ROWS_MAX_WEIGHTS, kMaxRows = MI_ROWS_MAX;
 constexpr int kStep = 32;              // contraction indices per product
 constexpr int kRedStride = 20;         // floats per row of partial sums: 16-byte aligned, spread over the banks
 
-// Values that are in registers from here on (the compiler otherwise loads an argument right before its use).
-template <typename V> __device__ __forceinline__ void arrived1(V& v) { asm volatile("" : "+s"(v)); }
-template <typename V> __device__ __forceinline__ void arrived1(V*& v) {   // a pointer to global memory stays one
-    uintptr_t at = (uintptr_t)v;
-    asm volatile("" : "+s"(at));
-    v = (V*)(__attribute__((address_space(1))) V*)at;
-}
-template <typename... V> __device__ __forceinline__ void arrived(V&... v) { (arrived1(v), ...); }
-
 struct Matrix {
     const void *w, *bias, *add;
     void* out;

@@ -287,3 +287,41 @@ def test_decode_merged_by_the_last_workgroup(B, nq, nkv, d, max_ctx, lens, n_spl
             graph.replay()
             assert torch.equal(out, want[i]) and not ws.tickets.any()
     assert getattr(ws[:1], "tickets", None) is None
+
+
+@pytest.mark.parametrize("nq,nkv,d,max_ctx,n_splits", [
+    (32, 8, 128, 256, 0), (4, 2, 128, 600, 0), (4, 4, 64, 300, 3), (6, 3, 96, 257, 0), (40, 2, 32, 256, 0), (24, 1, 64, 700, 7),
+])
+@pytest.mark.parametrize("kind", ["plain", "half", "interleaved"])
+def test_decode_append_over_what_the_row_held(nq, nkv, d, max_ctx, n_splits, kind):
+    """The new key's operands come from `k_new` and `v_new`: the same bits as with the row in the cache before the call, whatever the row held,
+    where the new key is first, in the middle or last of a chunk, and for sequences without any key, whose rows stay as they are."""
+    if kind == "half" and d not in (64, 128):
+        pytest.skip("rotate-half rotary inside the kernel is for heads of 64 and 128")
+    lens = [0, 1, 17, 32, 33, 128, 129, 255, max_ctx]
+    g = torch.Generator().manual_seed(nq + d)
+    normal = lambda *shape: torch.randn(*shape, generator=g).bfloat16().to(DEV)
+    B = len(lens)
+    q, k_new, v_new, kc, vc = normal(B, nq, d), normal(B, nkv, d), normal(B, nkv, d), normal(B, max_ctx, nkv, d), normal(B, max_ctx, nkv, d)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    rotary = None
+    if kind != "plain":
+        angle = torch.rand(max_ctx, d // 2, generator=g) * 6
+        cos, sin = (angle.cos().to(DEV), angle.sin().to(DEV))
+        if kind == "half":
+            cos, sin = (torch.cat([t, t], 1).bfloat16() for t in (cos, sin))
+        rotary = (cos, sin, torch.tensor([max(n - 1, 0) for n in lens], device=DEV))
+    for b, n in enumerate(lens):
+        kc[b, max(n - 1, 0):], vc[b, max(n - 1, 0):] = float("nan"), float("inf")
+    before = kc.clone(), vc.clone()
+    out = ops.decode_attention(q, kc, vc, ctx, k_new, v_new, rotary=rotary, n_splits=n_splits)
+    present = ops.decode_attention(q, kc, vc, ctx, rotary=rotary, n_splits=n_splits)
+    assert torch.equal(out, present) and out.isfinite().all() and not out[0].any()
+    for b, n in enumerate(lens):
+        if n > 0:
+            assert torch.equal(vc[b, n - 1], v_new[b]) and kc[b, n - 1].isfinite().all()
+            if kind == "plain":
+                assert torch.equal(kc[b, n - 1], k_new[b])
+        for now, held in zip((kc, vc), before):            # nothing but the new row was written
+            now[b, max(n - 1, 0):n] = held[b, max(n - 1, 0):n]
+            assert torch.equal(now[b].view(torch.int16), held[b].view(torch.int16))
