@@ -13,7 +13,11 @@
 //     contraction cost no memory traffic), one and a half (three) steps of 64 ahead.  A half of a 256 x 256 x 64 stage is refilled as
 //     soon as its fragments are in registers;
 //   * reads and loads are spread evenly between the products (sched_barrier pins the order): with one wavefront per SIMD a clump of more
-//     than three instructions between two products is a hole in the matrix pipe.
+//     than three instructions between two products is a hole in the matrix pipe;
+//   * with 16 steps of contraction a quarter of a block is what comes before and after them, so arguments come in two trips (ten, one after the other,
+//     before), accumulators are cleared and the bias is fetched under the first tiles, and results are read, staged and stored a quadrant
+//     at a time (all at once they did not fit the registers).  bf16, k 1024, before / after: 4084 x 4096 33.1 / 31.7 us, with bias 36.4 / 33.2;
+//     4084 x 3072 with bias 34.0 / 30.7; 4084 x 1024 with bias, blocks of 128, 15.5 / 14.9; 8192 x 14336, k 4096 601 / 601.
 // kmajor operands are read by LDS transpose reads from tiles in memory order, so all three layouts run at the same rate: 8192^3 bf16
 // 0.70 / 0.71 / 0.71 ms (x W^T, dy W, dy^T x), the library 0.67 / 0.78 / 0.90 on the same box (another box: 0.71 / 0.72 / 0.73, 0.69 / 0.79 / 0.92).
 //
@@ -40,14 +44,20 @@ constexpr int kQBase = 65536;                              // P stages below, Q 
 
 struct Segment { const char* p; const char* q; int64_t ldp, ldq; int k; };
 struct Problem {
+    int m, n, n_seg, p_kmajor, q_kmajor, first_block, tiles_m, tiles_n, splits, steps;
+    uint32_t tiles_by, group_by;                           // for divide(): by tiles_m * tiles_n and kGroup * tiles_n
     Segment seg[MI_GEMM_MAX_SEGMENTS];
     void* c; const void* bias; const void* add;
     int64_t ldc, ldadd;
     float* part;                                           // splits > 1: fp32 partial results [splits][tiles_m * tile][tiles_n * tile]
     void* p_sum;                                           // column sums of a contraction-major P
-    int n_seg, p_kmajor, q_kmajor, m, n, tiles_m, tiles_n, first_block, splits, sum_blocks;
+    int sum_blocks;
 };
-struct Problems { Problem p[MI_GEMM_MAX_PROBLEMS]; int count, first_sum; };
+struct Problems { int first_sum, first_block[MI_GEMM_MAX_PROBLEMS]; Problem p[MI_GEMM_MAX_PROBLEMS]; };   // no problem: first_block INT_MAX
+// What a block needs before its first loads, and what it needs for its results
+struct Block { Segment s; const void* bias; int m, n, n_seg, steps, splits; };
+struct Out { void* c; const void* add; int64_t ldc, ldadd; int m, n; };
+constexpr int kGroup = 4;                                  // block rows that are gone through together
 
 #define PIN() __builtin_amdgcn_sched_barrier(0)
 
@@ -73,6 +83,13 @@ template <> struct Half16<_Float16> {
 __device__ __forceinline__ void clear(f32x4_t& c) {
     c = f32x4_t{0.f, 0.f, 0.f, 0.f};
     asm volatile("" : "+a"(c));
+}
+
+// Results that are in accumulation registers up to here: left to itself the compiler reads all of them behind the last product, into registers that
+// it has to clear first.
+__device__ __forceinline__ f32x4_t fetch(f32x4_t c) {
+    asm volatile("" : "+a"(c));
+    return c;
 }
 
 // A 64 x 64 block in LDS: 64 rows (of the matrix as it lies in memory) of eight 16-byte units.  A direct load writes 64 x 16 consecutive
@@ -189,30 +206,59 @@ template <typename T, bool KMAJOR> struct Reader {
     }
 };
 
+// The bias of a lane's features in 64 columns from n0 on.  Where four of them are a word of eight bytes they are requested in front of the tiles (and so
+// are there with them); elsewhere when they are needed.
+template <typename T> struct Bias {
+    const T* at;                                           // nullable
+    int n, n0;
+    bool whole;
+    uint2 raw[4];
+    __device__ __forceinline__ void request(const Block& b, int first, int lane) {
+        at = (const T*)b.bias;
+        n = b.n;
+        n0 = first + 4 * (lane >> 4);
+        whole = at != nullptr && (n & 3) == 0 && ((uintptr_t)at & 7) == 0;
+        if (whole) {
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) raw[nt] = *reinterpret_cast<const uint2*>(at + min(n0 + 16 * nt, n - 4));
+        }
+    }
+    __device__ __forceinline__ f32x4_t get(int nt) const {
+        f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+        if (whole) {
+            typedef T t4 __attribute__((ext_vector_type(4)));
+            const t4 v = __builtin_bit_cast(t4, raw[nt]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = (float)v[i];
+        } else if (at != nullptr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = Elem<T>::load1(at + min(n0 + 16 * nt + i, n - 1));
+        }
+        return x;
+    }
+};
+
 // Results of a wavefront's 64 x 64 quadrant, with the bias, rounded, into 8 KB of LDS as rows.
-template <typename T> __device__ __forceinline__ void stage_quadrant(const Problem& pr, const f32x4_t (&acc)[4][4], char* stage, int n0, int lane) {
+template <typename T> __device__ __forceinline__ void stage_quadrant(const Bias<T>& bias, const f32x4_t (&acc)[4][4], char* stage, int lane) {
     typedef T t4 __attribute__((ext_vector_type(4)));
     const int l = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-        f32x4_t bias = {0.f, 0.f, 0.f, 0.f};
-        if (pr.bias != nullptr) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bias[i] = Elem<T>::load1((const T*)pr.bias + min(n0 + 16 * nt + 4 * g + i, pr.n - 1));
-        }
+        const f32x4_t add = bias.get(nt);
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             const int row = 16 * mt + l;
+            const f32x4_t x = fetch(acc[mt][nt]);
             t4 v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = (T)(acc[mt][nt][i] + bias[i]);
+            for (int i = 0; i < 4; ++i) v[i] = (T)(x[i] + add[i]);
             *reinterpret_cast<t4*>(stage + row * 128 + (((2 * nt + (g >> 1)) ^ swizzle(row)) << 4) + 8 * (g & 1)) = v;
         }
     }
 }
 
 // The staged rows to memory, eight lanes per row of 128 bytes.
-template <typename T> __device__ __forceinline__ void store_quadrant(const Problem& pr, const char* stage, int m0, int n0, int lane) {
+template <typename T> __device__ __forceinline__ void store_quadrant(const Out& pr, const char* stage, int m0, int n0, int lane) {
     const int r8 = lane >> 3, u = lane & 7, n = n0 + 8 * u;
     const char* src = stage + r8 * 128;
     T* c = (T*)pr.c + (int64_t)(m0 + r8) * pr.ldc + n;
@@ -253,7 +299,7 @@ __device__ __forceinline__ void store_part(const Problem& pr, const f32x4_t (&ac
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) *reinterpret_cast<f32x4_t*>(c + 16 * mt * ld + 16 * nt) = acc[mt][nt];
+        for (int nt = 0; nt < 4; ++nt) *reinterpret_cast<f32x4_t*>(c + 16 * mt * ld + 16 * nt) = fetch(acc[mt][nt]);
 }
 
 // Both operands of a problem, stepped together; a split of a problem (of one segment) takes the contraction indices k0 .. k0 + k - 1.
@@ -261,36 +307,41 @@ template <bool PK, bool QK, int HALVES> struct Operands {
     Loader<PK, HALVES> p;
     Loader<QK, HALVES> q;
     int seg, k0, k;
-    __device__ __forceinline__ void open(const Problem& pr, int m0, int n0, int wave, int lane) {
-        const Segment& s = pr.seg[seg];
-        const int len = pr.splits > 1 ? k : s.k;
-        p.open(s.p + (PK ? (int64_t)k0 * s.ldp : (int64_t)k0) * 2, s.ldp, m0, pr.m, len, wave, lane);
-        q.open(s.q + (QK ? (int64_t)k0 * s.ldq : (int64_t)k0) * 2, s.ldq, n0, pr.n, len, wave, lane);
+    __device__ __forceinline__ void open(const Segment& s, const Block& b, int m0, int n0, int wave, int lane) {
+        const int len = b.splits > 1 ? k : s.k;
+        p.open(s.p + (PK ? (int64_t)k0 * s.ldp : (int64_t)k0) * 2, s.ldp, m0, b.m, len, wave, lane);
+        q.open(s.q + (QK ? (int64_t)k0 * s.ldq : (int64_t)k0) * 2, s.ldq, n0, b.n, len, wave, lane);
     }
     // returns the number of steps
-    __device__ __forceinline__ int start(const Problem& pr, int split, int m0, int n0, int wave, int lane) {
-        int steps = 0;
-        for (int i = 0; i < pr.n_seg; ++i) steps += (pr.seg[i].k + kStep - 1) / kStep;
+    __device__ __forceinline__ int start(const Block& b, int split, int m0, int n0, int wave, int lane) {
+        int steps = b.steps;
         seg = 0;
         k0 = 0;
-        if (pr.splits > 1) {
-            const int first = (int)((int64_t)steps * split / pr.splits), end = (int)((int64_t)steps * (split + 1) / pr.splits);
+        if (b.splits > 1) {
+            const unsigned first = (unsigned)steps * split / b.splits, end = (unsigned)steps * (split + 1) / b.splits;
             k0 = first * kStep;
-            k = min(end * kStep, pr.seg[0].k) - k0;
+            k = min((int)end * kStep, b.s.k) - k0;
             steps = end - first;
         }
-        open(pr, m0, n0, wave, lane);
+        open(b.s, b, m0, n0, wave, lane);
         return steps;
     }
-    __device__ __forceinline__ void advance(const Problem& pr, int m0, int n0, int wave, int lane) {
+    __device__ __forceinline__ void advance(const Problem& pr, const Block& b, int m0, int n0, int wave, int lane) {
         const bool end = p.advance(wave, lane);
         q.advance(wave, lane);
-        if (end && seg + 1 < pr.n_seg) {
+        if (end && seg + 1 < b.n_seg) {
             ++seg;
-            open(pr, m0, n0, wave, lane);
+            open(pr.seg[seg], b, m0, n0, wave, lane);
         }
     }
 };
+
+// Requested between the first loads and the first products, not at the end.
+__device__ __forceinline__ Out results(const Problem& pr, const Block& b) {
+    Out out{pr.c, pr.add, pr.ldc, pr.ldadd, b.m, b.n};
+    arrived(out.c, out.add, out.ldc, out.ldadd);
+    return out;
+}
 
 template <int VM> __device__ __forceinline__ void wait_and_sync() {
     PIN();
@@ -302,26 +353,21 @@ template <int VM> __device__ __forceinline__ void wait_and_sync() {
 // quadrants of 32 products in the order (A0, B0), (A0, B1), (A1, B1), (A1, B0), so that each brings one new half; fragments of the next
 // half are read between the products of the present one, and the loads of step s + 2 go out as soon as a half's readers are through.  Two
 // barriers per step, each a quarter of a quadrant after its boundary, where the reads before it have long completed.
-template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(const Problem& pr, int split, int tm, int tn, char* smem) {
+template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(const Problem& pr, const Block& blk, int split, int tm, int tn, char* smem) {
     using H = Half16<T>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
     const int m0 = tm * 256, n0 = tn * 256;
     const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
     Operands<PK, QK, 2> in;
-    const int steps = in.start(pr, split, m0, n0, wave, lane);
+    const int steps = in.start(blk, split, m0, n0, wave, lane);
+    Bias<T> bias[2];
+    bias[0].request(blk, n0 + wn * 64, lane);
+    bias[1].request(blk, n0 + 128 + wn * 64, lane);
     Reader<T, PK> rp;
     Reader<T, QK> rq;
     rp.init(wm * kBlockBytes, lane);
     rq.init(kQBase + wn * kBlockBytes, lane);
     f32x4_t acc[2][2][4][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int d = 0; d < 4; ++d) clear(acc[a][b][c][d]);
     typename H::frag_t pf[2][4][2], qf[2][4][2];           // [half or set][16 rows][32 contraction indices]
     auto load_p = [&](auto s, auto h, auto j) { in.p.template load<s * 2 * kHalfBytes + h * kHalfBytes + j * 1024>(h, j, dst); PIN(); };
     auto load_q = [&](auto s, auto h, auto j) { in.q.template load<kQBase + s * 2 * kHalfBytes + h * kHalfBytes + j * 1024>(h, j, dst); PIN(); };
@@ -337,8 +383,18 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(
             static_for<4>([&](auto j) { load_q(s, h, j); });
             static_for<4>([&](auto j) { load_p(s, h, j); });
         });
-        in.advance(pr, m0, n0, wave, lane);
+        in.advance(pr, blk, m0, n0, wave, lane);
     });
+    Out out = results(pr, blk);
+    // while the first tiles are on their way
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) clear(acc[a][b][c][d]);
     wait_and_sync<24>();                                   // A0 and B0 of step 0
 #pragma unroll
     for (int f = 0; f < 8; ++f) { read_q(0, 0, 0, f); read_p(0, 0, f); }
@@ -367,7 +423,7 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(
             mma(1, 0, X, i);
             if constexpr (i % 4 == 1) read_q(Y, 1 - s, 0, i / 4);
             if constexpr (i % 8 == 3) load_p(s_c, h1, std::integral_constant<int, i / 8>{});
-            if constexpr (i == 30) in.advance(pr, m0, n0, wave, lane);
+            if constexpr (i == 30) in.advance(pr, blk, m0, n0, wave, lane);
         });
     };
     for (int i = 0; i < steps; i += 2) {                   // an odd count ends with a step of zeros
@@ -376,41 +432,45 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(
     }
     asm volatile("s_nop 15" ::: "memory");                 // the last products' registers
     wait_and_sync<0>();
-    if (pr.splits > 1) {
+    if (blk.splits > 1) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int q = 0; q < 2; ++q) store_part(pr, acc[h][q], split, 256, m0 + h * 128 + wm * 64, n0 + q * 128 + wn * 64, lane);
         return;
     }
+    // a quadrant is staged while the one before it is read back and stored
+    const auto stage = [&](int i) { stage_quadrant<T>(bias[i & 1], acc[i >> 1][i & 1], smem + (4 * wave + i) * kBlockBytes, lane); };
+    const auto store = [&](int i) {
+        store_quadrant<T>(out, smem + (4 * wave + i) * kBlockBytes, m0 + (i >> 1) * 128 + wm * 64, n0 + (i & 1) * 128 + wn * 64, lane);
+    };
+    stage(0);
+    PIN();
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            stage_quadrant<T>(pr, acc[h][q], smem + (4 * wave + 2 * h + q) * kBlockBytes, n0 + q * 128 + wn * 64, lane);
-#pragma unroll 1
-    for (int i = 0; i < 4; ++i)
-        store_quadrant<T>(pr, smem + (4 * wave + i) * kBlockBytes, m0 + (i >> 1) * 128 + wm * 64, n0 + (i & 1) * 128 + wn * 64, lane);
+    for (int i = 1; i < 4; ++i) {
+        stage(i);
+        store(i - 1);
+        PIN();
+    }
+    store(3);
 }
 
 // 128 x 128: four stages, loads three steps ahead, one barrier per step a quarter of its products after its start.  The fragments of the
 // next step are read between the products of the present one.
-template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(const Problem& pr, int split, int tm, int tn, char* smem) {
+template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(const Problem& pr, const Block& blk, int split, int tm, int tn, char* smem) {
     using H = Half16<T>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
     const int m0 = tm * 128, n0 = tn * 128;
     const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
     Operands<PK, QK, 1> in;
-    const int steps = in.start(pr, split, m0, n0, wave, lane);
+    const int steps = in.start(blk, split, m0, n0, wave, lane);
+    Bias<T> bias;
+    bias.request(blk, n0 + wn * 64, lane);
     Reader<T, PK> rp;
     Reader<T, QK> rq;
     rp.init(wm * kBlockBytes, lane);
     rq.init(kQBase + wn * kBlockBytes, lane);
     f32x4_t acc[4][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) clear(acc[c][d]);
     typename H::frag_t pf[2][4][2], qf[2][4][2];           // [set][16 rows][32 contraction indices]
     auto load = [&](auto j, uint32_t stage) {
         if constexpr (j < 4) in.q.template load<kQBase + j * 1024>(0, j, dst + stage);
@@ -431,8 +491,13 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
 #pragma unroll
     for (int s = 0; s < kStages128; ++s) {
         static_for<8>([&](auto j) { load(j, s * kHalfBytes); });
-        in.advance(pr, m0, n0, wave, lane);
+        in.advance(pr, blk, m0, n0, wave, lane);
     }
+    Out out = results(pr, blk);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) clear(acc[c][d]);
     wait_and_sync<24>();                                   // step 0
 #pragma unroll
     for (int f = 0; f < 16; ++f) read(0, f, 0);
@@ -445,7 +510,7 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
             mma(X, i);
             if constexpr (i >= 8 && i < 24) read(Y, i - 8, next);
             if constexpr (i >= 8 && i % 3 == 2) load(std::integral_constant<int, i / 3 - 2>{}, stage);
-            if constexpr (i == 30) in.advance(pr, m0, n0, wave, lane);
+            if constexpr (i == 30) in.advance(pr, blk, m0, n0, wave, lane);
         });
         stage = next;
     };
@@ -455,12 +520,12 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
     }
     asm volatile("s_nop 15" ::: "memory");
     wait_and_sync<0>();
-    if (pr.splits > 1) {
+    if (blk.splits > 1) {
         store_part(pr, acc, split, 128, m0 + wm * 64, n0 + wn * 64, lane);
         return;
     }
-    stage_quadrant<T>(pr, acc, smem + wave * kBlockBytes, n0 + wn * 64, lane);
-    store_quadrant<T>(pr, smem + wave * kBlockBytes, m0 + wm * 64, n0 + wn * 64, lane);
+    stage_quadrant<T>(bias, acc, smem + wave * kBlockBytes, lane);
+    store_quadrant<T>(out, smem + wave * kBlockBytes, m0 + wm * 64, n0 + wn * 64, lane);
 }
 
 // Bias gradients: sums over the rows of P, 64 columns per workgroup, behind the blocks of the products, where they run on compute units that
@@ -513,29 +578,42 @@ template <typename T> __device__ __forceinline__ void sum_columns(const Problem&
 template <typename T, int TILE>
 __global__ __launch_bounds__(kThreads, 1) void wide_kernel(const Problems ps) {
     __shared__ __attribute__((aligned(1024))) char smem[2 * kQBase];
-    int i = 0;
-    if ((int)blockIdx.x >= ps.first_sum) {
-        int b = blockIdx.x - ps.first_sum;
+    // Arguments in two trips, first which problem, then all that comes before the first loads: read where each is used they are ten in a row.
+    int first_sum = ps.first_sum, i = 0;
+    int first[MI_GEMM_MAX_PROBLEMS];
+#pragma unroll
+    for (int j = 1; j < MI_GEMM_MAX_PROBLEMS; ++j) first[j] = ps.first_block[j];
+    arrived(first_sum, first[1], first[2], first[3], first[4], first[5]);
+    static_assert(MI_GEMM_MAX_PROBLEMS == 6);
+    if ((int)blockIdx.x >= first_sum) {
+        int b = blockIdx.x - first_sum;
         while (b >= ps.p[i].sum_blocks) b -= ps.p[i++].sum_blocks;
         return sum_columns<T>(ps.p[i], b, smem);
     }
-    while (i + 1 < ps.count && (int)blockIdx.x >= ps.p[i + 1].first_block) ++i;
+#pragma unroll
+    for (int j = 1; j < MI_GEMM_MAX_PROBLEMS; ++j) i += (int)blockIdx.x >= first[j];
     const Problem& pr = ps.p[i];
-    const int tiles = pr.tiles_m * pr.tiles_n, total = tiles * pr.splits;
-    const int b = blockIdx.x - pr.first_block, xcd = b & 7, idx = b >> 3, each = total >> 3, rest = total & 7;
+    Block blk{pr.seg[0], pr.bias, pr.m, pr.n, pr.n_seg, pr.steps, pr.splits};
+    int p_kmajor = pr.p_kmajor, q_kmajor = pr.q_kmajor, first_block = pr.first_block, tiles_m = pr.tiles_m, tiles_n = pr.tiles_n;
+    uint32_t tiles_by = pr.tiles_by, group_by = pr.group_by;
+    arrived(blk.s.p, blk.s.q, blk.s.ldp, blk.s.ldq, blk.s.k, blk.bias, blk.m, blk.n, blk.n_seg, blk.steps, blk.splits, p_kmajor, q_kmajor, first_block, tiles_m,
+            tiles_n, tiles_by, group_by);
+    const int tiles = tiles_m * tiles_n, total = tiles * blk.splits;
+    const int b = blockIdx.x - first_block, xcd = b & 7, idx = b >> 3, each = total >> 3, rest = total & 7;
     if (idx >= each + (xcd < rest)) return;                // first_block is a multiple of eight
-    const int item = xcd * each + min(xcd, rest) + idx, split = item / tiles, t = item - split * tiles;
-    constexpr int kGroup = 4;
-    const int per_group = kGroup * pr.tiles_n, group = t / per_group, first = group * kGroup, height = min(kGroup, pr.tiles_m - first);
-    const int in_group = t - group * per_group, tn = in_group / height, tm = first + in_group - tn * height;
+    const int item = xcd * each + min(xcd, rest) + idx, split = divide(item, tiles, tiles_by), t = item - split * tiles;
+    const int per_group = kGroup * tiles_n, group = divide(t, per_group, group_by), row = group * kGroup, height = min(kGroup, tiles_m - row);
+    const int in_group = t - group * per_group;
+    const int tn = height == 4 ? in_group >> 2 : height == 3 ? divide(in_group, 3, 0x55555556u) : height == 2 ? in_group >> 1 : in_group;
+    const int tm = row + in_group - tn * height;
     if constexpr (TILE == 256) {
-        if (pr.p_kmajor) tile256<T, true, true>(pr, split, tm, tn, smem);
-        else if (pr.q_kmajor) tile256<T, false, true>(pr, split, tm, tn, smem);
-        else tile256<T, false, false>(pr, split, tm, tn, smem);
+        if (p_kmajor) tile256<T, true, true>(pr, blk, split, tm, tn, smem);
+        else if (q_kmajor) tile256<T, false, true>(pr, blk, split, tm, tn, smem);
+        else tile256<T, false, false>(pr, blk, split, tm, tn, smem);
     } else {
-        if (pr.p_kmajor) tile128<T, true, true>(pr, split, tm, tn, smem);
-        else if (pr.q_kmajor) tile128<T, false, true>(pr, split, tm, tn, smem);
-        else tile128<T, false, false>(pr, split, tm, tn, smem);
+        if (p_kmajor) tile128<T, true, true>(pr, blk, split, tm, tn, smem);
+        else if (q_kmajor) tile128<T, false, true>(pr, blk, split, tm, tn, smem);
+        else tile128<T, false, false>(pr, blk, split, tm, tn, smem);
     }
 }
 
@@ -722,7 +800,7 @@ namespace {
 int launch_in_one(const mi_gemm_problem* in, int count, int dtype, const MiGemmPlan& plan, void* workspace, hipStream_t st) {
     const int tile = plan.tile;
     Problems ps;
-    ps.count = count;
+    for (int& f : ps.first_block) f = 0x7fffffff;
     int order[MI_GEMM_MAX_PROBLEMS];
     for (int i = 0; i < count; ++i) {                      // longest contraction first: the launch then ends with short blocks
         int j = i;
@@ -741,11 +819,14 @@ int launch_in_one(const mi_gemm_problem* in, int count, int dtype, const MiGemmP
         p.p_kmajor = a.p_kmajor; p.q_kmajor = a.q_kmajor; p.m = a.m; p.n = a.n;
         p.tiles_m = (a.m + tile - 1) / tile;
         p.tiles_n = (a.n + tile - 1) / tile;
+        p.tiles_by = divide_m((uint32_t)(p.tiles_m * p.tiles_n));
+        p.group_by = divide_m((uint32_t)(kGroup * p.tiles_n));
+        p.steps = steps_of(a);
         p.splits = plan.splits;
         p.part = (float*)workspace;
         p.p_sum = a.p_sum;
         p.sum_blocks = a.p_sum != nullptr ? (a.m + kSumColumns - 1) / kSumColumns : 0;
-        p.first_block = (int)total;
+        p.first_block = ps.first_block[i] = (int)total;
         total += ((int64_t)p.tiles_m * p.tiles_n * p.splits + 7) / 8 * 8;
         if (total > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "gemm: too many tiles");
     }

@@ -679,3 +679,27 @@ def test_gradients_with_workspaces_in_a_graph():
         graph.replay()
         assert all(torch.equal(a, b) for a, b in zip(step(), want))
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("rows,ins,outs", [(4097, 520, 4104), (2050, 2056, 5632), (512, 1032, 4104), (513, 8200, 520), (1030, 1544, 1028)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_bias_off_the_boundaries_of_vectors(rows, ins, outs, dtype):
+    """Blocks of 256 and 128 and split contractions: a bias that starts between words of eight bytes gives the bits of one that does not."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    lib, code = _lib.load(), ops.dtype_code(dtype)
+    ld = (outs + 7) // 8 * 8
+    x, w, b = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((rows, ins), (outs, ins), (outs,)))
+    results = []
+    for shift in range(4):
+        bias = torch.empty(outs + 4, dtype=dtype, device=DEV)[shift:shift + outs].copy_(b)
+        c = torch.full((rows, ld), 7.0, dtype=dtype, device=DEV)
+        p = _lib.MiGemmProblem(c=c.data_ptr(), ldc=ld, n_segments=1, m=rows, n=outs, bias=bias.data_ptr())
+        p.segments[0] = _lib.MiGemmSegment(x.data_ptr(), w.data_ptr(), ins, ins, ins)
+        bytes_ = lib.mi_gemm_workspace_bytes(p, 1, code)
+        ws = torch.empty(max(bytes_, 16) // 4, device=DEV)
+        names = launched(lambda: _lib.check(lib.mi_gemm_with_workspace(p, 1, code, ws.data_ptr(), bytes_, ops.stream_ptr()), "mi_gemm_with_workspace"))
+        assert any("wide_kernel" in n for n in names), names
+        results.append(c)
+    xd, wd, bd = x.double(), w.double(), b.double()
+    _close("c", results[0][:, :outs], (xd @ wd.t() + bd).cpu(), (xd.abs() @ wd.abs().t() + bd.abs()).cpu(), ins, dtype)
+    assert all(torch.equal(c, results[0]) for c in results[1:]) and bool((results[0][:, outs:] == 7).all())
