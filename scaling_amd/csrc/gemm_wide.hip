@@ -3,7 +3,7 @@
 //
 // What bounds them is the matrix pipe and, with all compute units busy, the power it draws: a 8192^3 product that runs 2.0 PFLOP/s on zeros
 // runs 1.5 on random numbers, and every byte an operand is moved costs time.  So
-//   * a wavefront owns 128 x 128 (64 x 64) of the block, four wavefronts per workgroup, one per SIMD: an operand fragment that is read from
+//   * a wavefront owns 128 x 128 (64 x 64) of the block, four such wavefronts per workgroup, one per SIMD: an operand fragment that is read from
 //     LDS feeds eight (four) products.  Eight wavefronts of 128 x 64 read 1.5 x as much and run 0.78 ms where this runs 0.70;
 //   * the products are v_mfma_*_16x16x32, whose accumulator traffic per multiply-add is half that of 32x32x16 (0.74 against 0.77 ms, the
 //     same kernel with eight wavefronts);
@@ -348,6 +348,12 @@ template <int VM> __device__ __forceinline__ void wait_and_sync() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
     PIN();
 }
+// of a wavefront whose loads are for nobody else
+__device__ __forceinline__ void wait_and_sync() {
+    PIN();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    PIN();
+}
 
 // 256 x 256: two stages, each of two halves per operand (rows 0 - 127 and 128 - 255; a wavefront takes 64 rows of each).  A step is four
 // quadrants of 32 products in the order (A0, B0), (A0, B1), (A1, B1), (A1, B0), so that each brings one new half; fragments of the next
@@ -456,14 +462,33 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile256(
 }
 
 // 128 x 128: four stages, loads three steps ahead, one barrier per step a quarter of its products after its start.  The fragments of the
-// next step are read between the products of the present one.
+// next step are read between the products of the present one.  Each of the four wavefronts has a neighbour on its SIMD that does nothing but load: a wavefront
+// takes about 100 cycles to get rid of a direct load, and eight of them between 32 products of 16 cycles held the products up.  bf16, one wavefront
+// per SIMD / two: 4084 x 1024, k 1024 with bias 15.2 / 13.8 us, k 4096 36.2 / 33.7; 2048 x 2048, k 8192 67.9 / 61.3; forward and backward of 4084 x 1024 -> 1024
+// with bias 49.4 / 42.3.  (A fifth stage in place of the neighbour: level, 36.9 / 36.2.  A block of 256 has no registers for one.)
 template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(const Problem& pr, const Block& blk, int split, int tm, int tn, char* smem) {
     using H = Half16<T>;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3, wm = wave >> 1, wn = wave & 1;
     const int m0 = tm * 128, n0 = tn * 128;
-    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
     Operands<PK, QK, 1> in;
     const int steps = in.start(blk, split, m0, n0, wave, lane);
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= kThreads) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 4096);
+        const auto load = [&](int stage) {
+            static_for<4>([&](auto j) { in.q.template load<kQBase + j * 1024>(0, j, dst + stage); });
+            static_for<4>([&](auto j) { in.p.template load<j * 1024>(0, j, dst + stage); });
+            in.advance(pr, blk, m0, n0, wave, lane);
+        };
+#pragma unroll
+        for (int s = 0; s < kStages128; ++s) load(s * kHalfBytes);
+        wait_and_sync<24>();                               // step 0
+        for (int i = 0; i < (steps + 1) / 2 * 2; ++i) {
+            wait_and_sync<16>();                           // the next step is there; the present one is in everybody's registers
+            load((i & (kStages128 - 1)) * kHalfBytes);
+        }
+        wait_and_sync<0>();
+        return;
+    }
     Bias<T> bias;
     bias.request(blk, n0 + wn * 64, lane);
     Reader<T, PK> rp;
@@ -472,11 +497,6 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
     rq.init(kQBase + wn * kBlockBytes, lane);
     f32x4_t acc[4][4];
     typename H::frag_t pf[2][4][2], qf[2][4][2];           // [set][16 rows][32 contraction indices]
-    auto load = [&](auto j, uint32_t stage) {
-        if constexpr (j < 4) in.q.template load<kQBase + j * 1024>(0, j, dst + stage);
-        else in.p.template load<(j - 4) * 1024>(0, j - 4, dst + stage);
-        PIN();
-    };
     auto read = [&](int set, int f, int stage) {           // the fragments of contraction indices 0 .. 31 first
         const int t = (f >> 1) & 3, ks = f >> 3;
         if (f & 1) pf[set][t][ks] = rp.get(smem + stage, 0, t, ks);
@@ -488,17 +508,12 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
         H::mma(acc[mt][nt], qf[set][nt][ks], pf[set][mt][ks]);
         PIN();
     };
-#pragma unroll
-    for (int s = 0; s < kStages128; ++s) {
-        static_for<8>([&](auto j) { load(j, s * kHalfBytes); });
-        in.advance(pr, blk, m0, n0, wave, lane);
-    }
     Out out = results(pr, blk);
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int d = 0; d < 4; ++d) clear(acc[c][d]);
-    wait_and_sync<24>();                                   // step 0
+    wait_and_sync();                                       // step 0
 #pragma unroll
     for (int f = 0; f < 16; ++f) read(0, f, 0);
     int stage = 0;                                         // of the present step
@@ -506,11 +521,9 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
         constexpr int X = decltype(x_c)::value, Y = 1 - X;
         const int next = (stage + kHalfBytes) & (kStages128 * kHalfBytes - 1);
         static_for<32>([&](auto i) {
-            if constexpr (i == 8) wait_and_sync<16>();     // the next step is there; the present one is in everybody's registers
+            if constexpr (i == 8) wait_and_sync();
             mma(X, i);
             if constexpr (i >= 8 && i < 24) read(Y, i - 8, next);
-            if constexpr (i >= 8 && i % 3 == 2) load(std::integral_constant<int, i / 3 - 2>{}, stage);
-            if constexpr (i == 30) in.advance(pr, blk, m0, n0, wave, lane);
         });
         stage = next;
     };
@@ -519,7 +532,7 @@ template <typename T, bool PK, bool QK> __device__ __forceinline__ void tile128(
         step(std::integral_constant<int, 1>{});
     }
     asm volatile("s_nop 15" ::: "memory");
-    wait_and_sync<0>();
+    wait_and_sync();
     if (blk.splits > 1) {
         store_part(pr, acc, split, 128, m0 + wm * 64, n0 + wn * 64, lane);
         return;
@@ -576,7 +589,7 @@ template <typename T> __device__ __forceinline__ void sum_columns(const Problem&
 // Blocks of a problem are handed to the XCDs (workgroups modulo 8) in contiguous runs, in groups of four block rows, so that the workgroups
 // that share an L2 read the same rows and columns at the same time.
 template <typename T, int TILE>
-__global__ __launch_bounds__(kThreads, 1) void wide_kernel(const Problems ps) {
+__global__ __launch_bounds__(TILE == 256 ? kThreads : 2 * kThreads, TILE == 256 ? 1 : 2) void wide_kernel(const Problems ps) {
     __shared__ __attribute__((aligned(1024))) char smem[2 * kQBase];
     // Arguments in two trips, first which problem, then all that comes before the first loads: read where each is used they are ten in a row.
     int first_sum = ps.first_sum, i = 0;
@@ -586,6 +599,7 @@ __global__ __launch_bounds__(kThreads, 1) void wide_kernel(const Problems ps) {
     arrived(first_sum, first[1], first[2], first[3], first[4], first[5]);
     static_assert(MI_GEMM_MAX_PROBLEMS == 6);
     if ((int)blockIdx.x >= first_sum) {
+        if (TILE != 256 && threadIdx.x >= kThreads) return;
         int b = blockIdx.x - first_sum;
         while (b >= ps.p[i].sum_blocks) b -= ps.p[i++].sum_blocks;
         return sum_columns<T>(ps.p[i], b, smem);
@@ -839,7 +853,7 @@ int launch_in_one(const mi_gemm_problem* in, int count, int dtype, const MiGemmP
     const auto go = [&](auto t) {
         using T = decltype(t);
         if (tile == 256) wide_kernel<T, 256><<<grid, block, 0, st>>>(ps);
-        else wide_kernel<T, 128><<<grid, block, 0, st>>>(ps);
+        else wide_kernel<T, 128><<<grid, dim3(2 * kThreads), 0, st>>>(ps);
         if (plan.splits > 1) split_sum_kernel<T><<<sum_grid, block, 0, st>>>(p0, tile);
     };
     if (dtype == MI_BF16) go(__bf16{});
