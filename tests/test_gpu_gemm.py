@@ -703,3 +703,25 @@ def test_bias_off_the_boundaries_of_vectors(rows, ins, outs, dtype):
     xd, wd, bd = x.double(), w.double(), b.double()
     _close("c", results[0][:, :outs], (xd @ wd.t() + bd).cpu(), (xd.abs() @ wd.abs().t() + bd.abs()).cpu(), ins, dtype)
     assert all(torch.equal(c, results[0]) for c in results[1:]) and bool((results[0][:, outs:] == 7).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_chains_shorter_than_the_stages_of_a_block(dtype):
+    """Contractions of 1, 2, 3, 4 and 5 steps, in every layout, beside a long one in a launch of blocks of 128."""
+    lib, code, g = _lib.load(), ops.dtype_code(dtype), torch.Generator(device=DEV).manual_seed(3)
+    normal = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
+    for layout in range(3):                                # rows and rows; rows and contraction-major; contraction-major both
+        ks, problems, results = (2048, 8, 72, 136, 200, 264), (_lib.MiGemmProblem * 6)(), []
+        for i, k in enumerate(ks):
+            m, n = (2048, 2048) if i == 0 else (136, 264)
+            p, q = normal(m, k), normal(n, k)
+            c = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+            pm, qm = p.t().contiguous() if layout == 2 else p, q.t().contiguous() if layout > 0 else q
+            problems[i] = _lib.MiGemmProblem(c=c.data_ptr(), ldc=n, n_segments=1, m=m, n=n, p_kmajor=int(layout == 2), q_kmajor=int(layout > 0))
+            problems[i].segments[0] = _lib.MiGemmSegment(pm.data_ptr(), qm.data_ptr(), pm.stride(0), qm.stride(0), k)
+            results.append((p, q, c, pm, qm))
+        names = launched(lambda: _lib.check(lib.mi_gemm_with_workspace(problems, 6, code, None, 0, ops.stream_ptr()), "mi_gemm_with_workspace"))
+        assert sum("wide_kernel" in n and "128" in n for n in names) == len(names) == 1, names
+        for k, (p, q, c, _, _) in zip(ks, results):
+            pd, qd = p.double(), q.double()
+            _close(f"layout {layout} k {k}", c, (pd @ qd.t()).cpu(), (pd.abs() @ qd.abs().t()).cpu(), k, dtype)
