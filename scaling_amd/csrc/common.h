@@ -111,6 +111,21 @@ __device__ __forceinline__ void rotate_complex_pair(float& x0, float& x1, float 
     x1 = im;
 }
 
+// float16 results of a rotate-half rotary.  Their products are exact in float32, so the mixed-precision fma rounds a sum once, an fma and a conversion
+// round it twice (float32, float16), and one sum in some thousands comes out an ulp apart.  Left to the compiler the choice moves with the code around it, and
+// with it what a cache holds; kernels that have to leave the same bits name it: a pair of sums rounded once ...
+__device__ __forceinline__ uint32_t fma_pair_f16(float a0, float b0, float c0, float a1, float b1, float c1) {
+    uint32_t d;
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3\n\tv_fma_mixhi_f16 %0, %4, %5, %6" : "=&v"(d) : "v"(a0), "v"(b0), "v"(c0), "v"(a1), "v"(b1), "v"(c1));
+    return d;
+}
+// ... and a sum that is rounded to float32 first.
+__device__ __forceinline__ float sum_f32(float a, float b, float c) {
+    float x = __builtin_fmaf(a, b, c);
+    asm("" : "+v"(x));
+    return x;
+}
+
 // ---- wavefront reductions (64 lanes) -------------------------------------------------------
 // Sum over aligned groups of WIDTH lanes, every lane receiving the total, without going through the LDS crossbar
 // (six dependent ds_bpermute round trips per 64-lane sum otherwise): DPP lane selects inside a row of 16 lanes

@@ -888,9 +888,9 @@ Tensor op_attention_qkv(const Tensor& qkv, const Tensor& cu_q, const OptTensor& 
 
 // ---- a layer in one call -----------------------------------------------------------------------------------------------
 // Attention over the rows of a prefill [batch * seq, heads, head_dim] (inference), which leaves rotated k and v in the caches
-// [batch, max_ctx, KV heads, head_dim] and raises ctx_len to seq: two launches.
-Tensor op_prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const Tensor& pos, const Tensor& cos, const Tensor& sin,
-                            bool interleaved, double scale, int64_t batch, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len) {
+// [batch, max_ctx, KV heads, head_dim] and raises ctx_len to seq: two launches, or with q_first one more that rotates q in front of the attention kernel.
+Tensor prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const Tensor& pos, const Tensor& cos, const Tensor& sin,
+                         bool interleaved, double scale, int64_t batch, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len, bool q_first) {
     check_qkv(q, k, v, cu, Tensor());
     TORCH_CHECK(batch > 0 && k.size(0) % batch == 0 && k.size(0) == q.size(0) && k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
                     k_cache.strides() == v_cache.strides() && k_cache.stride(3) == 1 && k_cache.size(0) == batch && k_cache.size(2) == k.size(1) &&
@@ -909,7 +909,17 @@ Tensor op_prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, c
     a.batch = (int32_t)batch; a.seq = (int32_t)(k.size(0) / batch); a.max_ctx = (int32_t)k_cache.size(1); a.n_kv_heads = (int32_t)k.size(1);
     a.head_dim = (int32_t)k.size(2); a.dtype = code_of(k); a.rotary_interleaved = interleaved; a.stream = l.stream;
     check(mi_fill_cache(&a), "mi_fill_cache");
+    if (q_first) {
+        const Tensor q_rot = rotary_launch(q, cos, sin, pos, 0, false, interleaved);
+        const auto plain = options(true, scale, 0, 0.0, 0, std::nullopt, std::nullopt, std::nullopt, std::nullopt, false);
+        return std::get<0>(attn_forward(q_rot, k_rot, v, cu, Tensor(), plain, Tensor()));
+    }
     return std::get<0>(attn_forward(q, k_rot, v, cu, Tensor(), options(true, scale, 0, 0.0, 0, cos, sin, pos, std::nullopt, interleaved), Tensor()));
+}
+
+Tensor op_prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const Tensor& pos, const Tensor& cos, const Tensor& sin,
+                            bool interleaved, double scale, int64_t batch, const Tensor& k_cache, const Tensor& v_cache, const Tensor& ctx_len) {
+    return prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, scale, batch, k_cache, v_cache, ctx_len, false);
 }
 
 // A pre-norm layer on x [batch, seq, hidden]: the same operations, one after the other, as the modules of the layer issue them, with their autograd
@@ -945,7 +955,8 @@ Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, const s
             q = out[0].view({tokens, nq, d}); k = out[1].view({tokens, nkv, d}); v = out[2].view({tokens, nkv, d});
         }
         if (!caches.empty()) {
-            ctx = op_prefill_attention(q, k, v, cu, *pos, *cos, *sin, interleaved, scale, b, caches[0], caches[1], caches[2]);
+            // float16: the stand-alone kernel rounds some sums of q otherwise than the attention kernel does on its loads, and the modules take that kernel
+            ctx = prefill_attention(q, k, v, cu, *pos, *cos, *sin, interleaved, scale, b, caches[0], caches[1], caches[2], q.scalar_type() == at::kHalf);
         } else {
             if (rotary == 2) {
                 q = Rotary::apply(q, *cos, *sin, pos, s, interleaved);

@@ -34,6 +34,30 @@ template <typename TT, int N> __device__ __forceinline__ void load_table(const T
     }
 }
 
+// One vector of either half of a head, rotated: what every kernel here leaves for a data type and 16-bit tables of the same type.
+template <typename T>
+__device__ __forceinline__ void rotate_half(const float* x0, const float* x1, const float* cA, const float* sA, const float* cB, const float* sB, uint4& lo, uint4& hi) {
+    constexpr int V = Elem<T>::kVec;
+    float o0[V], o1[V];
+    if constexpr (std::is_same_v<T, _Float16>) {           // first half rounded twice, second half once
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < V; ++i) o0[i] = sum_f32(x0[i], cA[i], -(x1[i] * sA[i]));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = fma_pair_f16(x1[2 * i], cB[2 * i], x0[2 * i] * sB[2 * i], x1[2 * i + 1], cB[2 * i + 1], x0[2 * i + 1] * sB[2 * i + 1]);
+        lo = Elem<T>::pack(o0);
+        hi = make_uint4(h[0], h[1], h[2], h[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            o0[i] = x0[i] * cA[i] - x1[i] * sA[i];
+            o1[i] = x1[i] * cB[i] + x0[i] * sB[i];
+        }
+        lo = Elem<T>::pack(o0);
+        hi = Elem<T>::pack(o1);
+    }
+}
+
 // T: data type, TT: table type.  Work item = (token, head, vec) with vec over half the rotated span
 // followed by the vectors of the unrotated tail.
 template <typename T, typename TT>
@@ -61,25 +85,38 @@ __global__ __launch_bounds__(kBlock) void rotary_vec_kernel(RotaryParams p) {
     const int64_t r = table_row(p, t);
     const TT* cr = (const TT*)p.cos + r * p.rot_dim;
     const TT* sr = (const TT*)p.sin + r * p.rot_dim;
-    float x0[V], x1[V], o0[V], o1[V], cA[V], sA[V], cB[V], sB[V];
+    float x0[V], x1[V], cA[V], sA[V], cB[V], sB[V];
     Elem<T>::unpack(ldg_nt(reinterpret_cast<const uint4*>(xrow + c0)), x0);
     Elem<T>::unpack(ldg_nt(reinterpret_cast<const uint4*>(xrow + c1)), x1);
     load_table<TT, V>(cr + c0, cA);
     load_table<TT, V>(sr + c0, sA);
     load_table<TT, V>(cr + c1, cB);
     load_table<TT, V>(sr + c1, sB);
+    uint4 lo, hi;
+    if constexpr (sizeof(TT) == 2) {
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-        o0[i] = x0[i] * cA[i] - x1[i] * (p.sign * sA[i]);
-        o1[i] = x1[i] * cB[i] + x0[i] * (p.sign * sB[i]);
+        for (int i = 0; i < V; ++i) {
+            sA[i] *= p.sign;
+            sB[i] *= p.sign;
+        }
+        rotate_half<T>(x0, x1, cA, sA, cB, sB, lo, hi);
+    } else {
+        float o0[V], o1[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            o0[i] = x0[i] * cA[i] - x1[i] * (p.sign * sA[i]);
+            o1[i] = x1[i] * cB[i] + x0[i] * (p.sign * sB[i]);
+        }
+        lo = Elem<T>::pack(o0);
+        hi = Elem<T>::pack(o1);
     }
-    stg_nt(reinterpret_cast<uint4*>(orow + c0), Elem<T>::pack(o0));
-    stg_nt(reinterpret_cast<uint4*>(orow + c1), Elem<T>::pack(o1));
+    stg_nt(reinterpret_cast<uint4*>(orow + c0), lo);
+    stg_nt(reinterpret_cast<uint4*>(orow + c1), hi);
 }
 
 // What a prefill leaves in a KV cache, in one launch: k rotated (whole head, rotate-half or interleaved pairs, as the two kernels around this one)
 // into the cache and, packed, for the attention launch that follows; v into the cache; the context lengths.  A thread owns a vector of the
-// first half of a k row and its partner (interleaved: one of either half) or the same two of a v row.  As two rotary launches (q and k; q is now
+// first half of a k row and its partner (interleaved: one of either half) or the same two of a v row.  As two rotary launches (q and k; bfloat16 q is now
 // rotated where the attention kernel loads it), two copies and a fill it was five launches a layer.
 struct FillParams {
     const void *k, *v, *cos, *sin;
@@ -121,21 +158,16 @@ __global__ __launch_bounds__(kBlock) void fill_cache_kernel(const FillParams p) 
             rotate_complex_pair(x0[2 * i], x0[2 * i + 1], cr[i], sr[i]);
             rotate_complex_pair(x1[2 * i], x1[2 * i + 1], cr[D / 4 + i], sr[D / 4 + i]);
         }
+        lo = Elem<T>::pack(x0);
+        hi = Elem<T>::pack(x1);
     } else {
         float cA[V], sA[V], cB[V], sB[V];
         load_table<T, V>((const T*)p.cos + r * D + V * c, cA);
         load_table<T, V>((const T*)p.sin + r * D + V * c, sA);
         load_table<T, V>((const T*)p.cos + r * D + D / 2 + V * c, cB);
         load_table<T, V>((const T*)p.sin + r * D + D / 2 + V * c, sB);
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const float a = __builtin_fmaf(x0[i], cA[i], -(x1[i] * sA[i])), d = __builtin_fmaf(x1[i], cB[i], x0[i] * sB[i]);
-            x0[i] = a;
-            x1[i] = d;
-        }
+        rotate_half<T>(x0, x1, cA, sA, cB, sB, lo, hi);
     }
-    lo = Elem<T>::pack(x0);
-    hi = Elem<T>::pack(x1);
     T *dst = (T*)p.k_cache + at, *out = (T*)p.k_out + (t * p.n_heads + h) * D + V * c;
     *reinterpret_cast<uint4*>(dst) = lo;
     *reinterpret_cast<uint4*>(dst + D / 2) = hi;

@@ -410,3 +410,58 @@ def test_prefill_attention_fills_the_cache(b, s, max_ctx, nkv, d, interleaved, d
     assert torch.equal(o, ops.attention_forward(q, k_rot, v, cu, None, True, d ** -0.5, rotary=(cos, sin, pos, None))[0])
     with pytest.raises(RuntimeError, match="fit the rows"):
         _lib.host().prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, d ** -0.5, b, kc, vc, ctx[:0])
+
+
+@pytest.mark.parametrize("d,b,s", [(64, 1, 1), (64, 3, 67), (128, 2, 130), (128, 1, 509)])
+@pytest.mark.parametrize("kind", ["rotary", "rotary_complex"])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_prefill_in_one_call_equals_its_modules(dtype, kind, d, b, s):
+    """Output, cache and lengths of a prefill, a prefill into a cache that is there and longer, and the step that follows, in every bit: float16
+    too, whose rotary sums the kernels round once or twice."""
+    layer = _layer(dtype, False, hidden=4 * d, relative_position_embedding_type=kind).eval()
+    g = torch.Generator().manual_seed(s)
+    normal = lambda *shape: torch.randn(*shape, generator=g).to(layer.self_attention.dtype).to(DEV)
+    x, x2, x3, step = normal(b, s, 4 * d), normal(b, s, 4 * d), normal(b, max(s - 1, 1), 4 * d), normal(b, 1, 4 * d)
+
+    def io(x, position, reset):
+        io = _io(x)
+        io.position_ids, io.inference_settings = io.position_ids + position, InferenceSettings(use_cache=True, reset_cache=reset)
+        return io
+
+    def run(watched):
+        layer.self_attention.cache.clear()
+        seen, out = [], []
+        for x_ in (x, x2, x3):
+            handle = layer.self_attention.register_forward_hook(lambda *a: seen.append(1)) if watched else None
+            with torch.no_grad():
+                out.append(layer(io(x_, 0, True)).activations)
+            if handle is not None:
+                handle.remove()
+            cache = layer.self_attention.cache[0]
+            assert cache.length == x_.shape[1]
+            out += [cache.k.clone(), cache.v.clone(), cache.ctx_len.clone()]
+        with torch.no_grad():
+            out.append(layer(io(step, x3.shape[1], False)).activations)
+        return out + [cache.k, cache.v], seen
+
+    native, _ = run(False)
+    modules, seen = run(True)
+    assert len(seen) == 3
+    for i, (a, c) in enumerate(zip(native, modules)):
+        assert torch.equal(a, c), i
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+def test_cached_keys_are_those_of_the_rotary_kernel(d, interleaved, dtype):
+    """The rounding of float16 sums included: 131072 rotated features."""
+    nkv, s, g = 8, 16384 // d, torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(s, nkv, d, generator=g).to(dtype).to(DEV) for _ in range(3))
+    pos = torch.arange(s, device=DEV)
+    ang = torch.outer(torch.arange(s).float(), 1.0 / (10000.0 ** (torch.arange(0, d, 2).float() / d))).to(DEV)
+    cos, sin = (t if interleaved else torch.cat((t, t), -1).to(dtype) for t in (ang.cos(), ang.sin()))
+    cu = torch.tensor([0, s], dtype=torch.int32, device=DEV)
+    kc, vc = (torch.zeros(1, s, nkv, d, dtype=dtype, device=DEV) for _ in range(2))
+    _lib.host().prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, d ** -0.5, 1, kc, vc, torch.zeros(1, dtype=torch.int32, device=DEV))
+    assert torch.equal(kc[0], (ops.rotary_embedding_complex if interleaved else ops.rotary_embedding)(k, cos, sin, pos)) and torch.equal(vc[0], v)
