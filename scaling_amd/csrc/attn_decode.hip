@@ -46,6 +46,31 @@ __device__ __forceinline__ f32x4v mfma_16x16x32(elem8_t a, elem8_t b, f32x4v c) 
 #endif
 }
 
+// Rotate-half rotary of a query or of the new key.  float16: sums are rounded once, but for features 2 - 7 of every eight of a key's second half, which are
+// rounded to float32 first.  That is what the compiler once made of `rotate_pair` in either place, and what caches hold; it is named so that it no longer
+// depends on the code around it.
+template <bool KEY> __device__ __forceinline__ void rotate_row(uint4& lo, uint4& hi, const uint4& c, const uint4& s) {
+#ifdef MI_ELEM_F16
+    float x0[8], x1[8], cs[8], sn[8];
+    Elem<elem_t>::unpack(lo, x0);
+    Elem<elem_t>::unpack(hi, x1);
+    Elem<elem_t>::unpack(c, cs);
+    Elem<elem_t>::unpack(s, sn);
+    uint32_t l[4], h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int a = 2 * i, b = a + 1;
+        l[i] = fma_pair_f16(x0[a], cs[a], -(x1[a] * sn[a]), x0[b], cs[b], -(x1[b] * sn[b]));
+        h[i] = KEY && i > 0 ? pack_elem2(sum_f32(x1[a], cs[a], x0[a] * sn[a]), sum_f32(x1[b], cs[b], x0[b] * sn[b]))
+                            : fma_pair_f16(x1[a], cs[a], x0[a] * sn[a], x1[b], cs[b], x0[b] * sn[b]);
+    }
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+#else
+    rotate_pair(lo, hi, c, s, 1.0f);
+#endif
+}
+
 // ---- merge of the splits ------------------------------------------------------------------------------
 // SHARED: the partial results pass between workgroups of one launch, past the L2s (those of the XCDs are not coherent; writing back and
 // invalidating them, as a release and an acquire do, took 2 - 10 us of a launch of 104 - 256 workgroups).
@@ -319,8 +344,8 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     if constexpr (ROT == 1) {
 #pragma unroll
         for (int ks = 0; ks < KS / 2; ++ks) {
-            rotate_pair(raw[ks], raw[ks + KS / 2], cv[ks], sv[ks], 1.0f);
-            if (it_new >= 0) rotate_pair(kn[ks], kn[ks + KS / 2], cv[ks], sv[ks], 1.0f);
+            rotate_row<false>(raw[ks], raw[ks + KS / 2], cv[ks], sv[ks]);
+            if (it_new >= 0) rotate_row<true>(kn[ks], kn[ks + KS / 2], cv[ks], sv[ks]);
         }
     } else if constexpr (ROT == 2) {
 #pragma unroll

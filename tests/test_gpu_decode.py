@@ -325,3 +325,27 @@ def test_decode_append_over_what_the_row_held(nq, nkv, d, max_ctx, n_splits, kin
         for now, held in zip((kc, vc), before):            # nothing but the new row was written
             now[b, max(n - 1, 0):n] = held[b, max(n - 1, 0):n]
             assert torch.equal(now[b].view(torch.int16), held[b].view(torch.int16))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_float16_keys_are_rounded_as_they_always_were(d):
+    """The sums of a rotated float16 key are exact in float64.  Features 2 - 7 of every eight of the second half are rounded to float32 and then to
+    float16, the others once.  The smaller product of each sum lies below the last bit of float32 and the larger one, of 22 bits, is a tie between two
+    float16 values in one of 2000 sums, so that the two differ often enough."""
+    B, nkv, g = 64, 32, torch.Generator().manual_seed(d)
+    size = torch.where(torch.arange(d) < d // 2, 64.0, 2.0 ** -8)
+    k, v, q = (((1 + torch.rand(B, nkv, d, generator=g)) * torch.randn(B, nkv, d, generator=g).sign()).half() for _ in range(3))
+    k[::2], k[1::2] = k[::2] * size, k[1::2] * size.flip(0)
+    cos, sin = (torch.cat([t, t], 1).half() for t in (0.5 + 0.5 * torch.rand(B, d // 2, generator=g), 2.0 ** -14 * (1 + torch.rand(B, d // 2, generator=g))))
+    kc, vc = (torch.zeros(B, 4, nkv, d, dtype=torch.float16, device=DEV) for _ in range(2))
+    ctx = torch.full((B,), 3, dtype=torch.int32, device=DEV)
+    ops.decode_attention(q.to(DEV), kc, vc, ctx, k.to(DEV), v.to(DEV), rotary=(cos.to(DEV), sin.to(DEV), torch.arange(B, device=DEV)))
+    x0, x1 = k.double().chunk(2, -1)
+    c, s = (t[:, None, :d // 2].double() for t in (cos, sin))
+    exact = torch.cat([x0 * c - x1 * s, x1 * c + x0 * s], -1)
+    once = torch.from_numpy(exact.numpy().astype("float16"))
+    twice = torch.from_numpy(exact.numpy().astype("float32").astype("float16"))
+    feature = torch.arange(d)
+    want = torch.where((feature >= d // 2) & (feature % 8 >= 2), twice, once)
+    assert torch.equal(kc[:, 2].cpu(), want) and torch.equal(vc[:, 2].cpu(), v)
+    assert int((want != once).sum()) > 10 and int((want != twice).sum()) > 10
