@@ -699,19 +699,15 @@ __global__ __launch_bounds__(512, D == 32 ? 4 : 2) void attn_bwd_kernel(const At
     else dq_block<D, DROP, SPLIT>(p, sh, blockIdx.x - n_dkdv);
 }
 
-template <int D> int launch_delta(const AttnParams& p, hipStream_t st) {
-    const int64_t blocks = ((int64_t)p.total_q * p.nq * 16 + kThreads - 1) / kThreads;
-    if (blocks > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
-    attn_bwd_delta_kernel<D><<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(p);
-    return mi_check_launch("attn_bwd_delta");
-}
-
 template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) {
     const int stages = flags & (MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ);
     const bool split = (flags & MI_ATTN_SPLIT_P) != 0;     // accuracy mode (no dropout: checked by the entry point)
     const bool all = stages == 0;
     if (all || (stages & MI_ATTN_BWD_DELTA)) {
-        const int rc = launch_delta<D>(p, st);
+        const int64_t blocks = ((int64_t)p.total_q * p.nq * 16 + kThreads - 1) / kThreads;
+        if (blocks > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+        attn_bwd_delta_kernel<D><<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(p);
+        const int rc = mi_check_launch("attn_bwd_delta");
         if (rc != MI_OK) return rc;
     }
     const bool dkdv = all || (stages & MI_ATTN_BWD_DKDV) != 0, dq = all || (stages & MI_ATTN_BWD_DQ) != 0;
@@ -750,8 +746,13 @@ template <int D> int launch_short(const AttnParams& p, ShortBwd route, hipStream
         //        128 features 16.7 / 16.1 | 25.5 / 22.8 | 37.5 / 32.3
         const int64_t chain = (int64_t)p.total_q / p.n_docs * (p.n_rep / p.hsplit);
         const bool own_delta = chain < (D <= 64 ? 1024 : 512);
-        if (!own_delta) rc = launch_delta<D>(p, st);
-        if (rc != MI_OK) return rc;
+        if (!own_delta) {
+            const int64_t blocks = ((int64_t)p.total_q * p.nq * 2 + 255) / 256;
+            if (blocks > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
+            attn_bwd_delta_short_kernel<D><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(p);
+            rc = mi_check_launch("attn_bwd_delta_short");
+            if (rc != MI_OK) return rc;
+        }
         const auto kernel = own_delta ? attn_short_bwd_kernel<D, true> : attn_short_bwd_kernel<D, false>;
         kernel<<<dim3((unsigned)(grid_k + grid_q)), block, 0, st>>>(p, (int)grid_k);
     }

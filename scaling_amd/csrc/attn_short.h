@@ -360,7 +360,8 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
         p.lse[(int64_t)head * p.total_q + tq] = L > 0.f ? (M + __log2f(L)) * 0.6931471805599453f : INFINITY;
 }
 
-// acc + the products of eight features of an O row and a dO row: delta = sum of them over the features, in the same order wherever it is formed
+// acc + the products of eight features of an O row and a dO row: delta = sum of them over the features, in the same order wherever
+// these kernels form it
 __device__ __forceinline__ float short_dot(const elem8_t& o, const elem8_t& d_o, float acc) {
     float a[8], b[8];
     Elem<elem_t>::unpack(__builtin_bit_cast(uint4, o), a);
@@ -368,6 +369,28 @@ __device__ __forceinline__ float short_dot(const elem8_t& o, const elem8_t& d_o,
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc += a[i] * b[i];
     return acc;
+}
+
+// delta for the dK / dV blocks of long chains, in a launch in front: two lanes per (token, head) row, its sums in the order of the blocks that form
+// their own, so that a gradient does not depend on who formed its delta.  (The tiled kernels' 16 lanes sum in another order.)
+template <int D>
+__global__ __launch_bounds__(256) void attn_bwd_delta_short_kernel(const AttnParams p) {
+    const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x, row = item >> 1;
+    if (row >= (int64_t)p.total_q * p.nq) return;          // both lanes of a row
+    const int64_t t = row / p.nq;
+    const int h = (int)(row - t * p.nq), g = (int)(item & 1);
+    const elem_t *o = p.o + t * p.o_st + (int64_t)h * p.o_sh + 8 * g, *d_o = p.d_o + t * p.o_st + (int64_t)h * p.o_sh + 8 * g;
+    elem8_t a[D / 16], b[D / 16];
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+        a[ks] = *reinterpret_cast<const elem8_t*>(o + 16 * ks);
+        b[ks] = *reinterpret_cast<const elem8_t*>(d_o + 16 * ks);
+    }
+    float delta = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) delta = short_dot(a[ks], b[ks], delta);
+    delta = group_sum<2>(delta);
+    if (g == 0) p.delta[(int64_t)h * p.total_q + t] = delta;
 }
 
 // ---- backward: dQ of 32 queries of one head ------------------------------------------------------------------

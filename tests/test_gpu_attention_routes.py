@@ -143,6 +143,28 @@ def test_backward_with_delta_of_another_launch(nq, nkv, d, lens, flags, kernel):
         assert float((x.float() - y.float()).norm()) <= 2.0 ** -9 * float(y.float().norm()), name
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("nq,nkv,dtype", [(2, 2, torch.float16), (3, 1, torch.bfloat16)])
+def test_delta_is_the_same_whoever_forms_it(nq, nkv, d, dtype):
+    """A document of 35 blocks of 32 rows: its gradients alone, where a launch in front leaves delta, have the bits they have beside seven short
+    documents, where the blocks of the second launch form it."""
+    g = torch.Generator(device=DEV).manual_seed(d)
+    lens = (1120,) + 7 * (16,)
+    q, do = (torch.randn(sum(lens), nq, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    k, v = (torch.randn(sum(lens), nkv, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    results = []
+    for docs in (1, 8):
+        n = sum(lens[:docs])
+        cu = torch.tensor([0] + list(torch.tensor(lens[:docs]).cumsum(0)), dtype=torch.int32, device=DEV)
+        rows = [t[:n].contiguous() for t in (do, q, k, v)]
+        o, lse = ops.attention_forward(*rows[1:], cu, None, True, None, flags=SHORT)
+        run = lambda: ops.attention_backward(*rows, o, lse, cu, None, True, None, flags=SHORT)
+        assert any("attn_bwd_delta" in x for x in launched(run)) == (docs == 1)
+        results.append([t[:lens[0]] for t in (o, *run())])
+    for name, x, y in zip(("o", "dq", "dk", "dv"), *results):
+        assert torch.equal(x, y), name
+
+
 # float32 backward with dS kept by the dK/dV kernel (a workspace that has room for it) against the dQ kernel that recomputes it: the same
 # bits.  Triangle and whole plane, documents that end inside tiles, keys and queries of different lengths (rows that see nothing among
 # them), few KV heads, several passes over the heads (4128 tokens of 64 heads; 8192 of 12 and 16384 of 8, whose passes alone have fewer
