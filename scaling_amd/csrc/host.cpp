@@ -887,6 +887,18 @@ Tensor op_attention_qkv(const Tensor& qkv, const Tensor& cu_q, const OptTensor& 
 }
 
 // ---- a layer in one call -----------------------------------------------------------------------------------------------
+// The kernels take the tables' bytes for what `interleaved` and the type of the rows say: float32 [rows, head_dim / 2], or [rows, head_dim] of x's type where
+// the attention kernel rotates (whole), or any part of a head, of x's type or float32.
+void check_tables(const Tensor& x, int64_t head_dim, const OptTensor& cos, const OptTensor& sin, bool interleaved, bool whole) {
+    const auto fits = [&](at::ScalarType type, int64_t width) { return cos->scalar_type() == type && cos->size(1) == width; };
+    TORCH_CHECK(cos.has_value() && sin.has_value() && cos->dim() == 2 && cos->sizes() == sin->sizes() && cos->scalar_type() == sin->scalar_type() &&
+                    cos->device() == x.device() && sin->device() == x.device() && cos->is_contiguous() && sin->is_contiguous() &&
+                    (interleaved ? fits(at::kFloat, head_dim / 2)
+                     : whole     ? fits(x.scalar_type(), head_dim)
+                                 : cos->size(1) <= head_dim && (cos->scalar_type() == x.scalar_type() || cos->scalar_type() == at::kFloat)),
+                "rotary: tables have to fit the type and the features of the rows");
+}
+
 // Attention over the rows of a prefill [batch * seq, heads, head_dim] (inference), which leaves rotated k and v in the caches
 // [batch, max_ctx, KV heads, head_dim] and raises ctx_len to seq: two launches, or with q_first one more that rotates q in front of the attention kernel.
 Tensor prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const Tensor& pos, const Tensor& cos, const Tensor& sin,
@@ -896,9 +908,10 @@ Tensor prefill_attention(const Tensor& q, const Tensor& k, const Tensor& v, cons
                     k_cache.strides() == v_cache.strides() && k_cache.stride(3) == 1 && k_cache.size(0) == batch && k_cache.size(2) == k.size(1) &&
                     k_cache.size(3) == k.size(2) && k_cache.scalar_type() == k.scalar_type() && v_cache.scalar_type() == k.scalar_type() &&
                     ctx_len.scalar_type() == at::kInt && ctx_len.is_contiguous() && ctx_len.numel() == batch && pos.scalar_type() == at::kLong &&
-                    pos.is_contiguous() && pos.numel() == k.size(0) && cos.is_contiguous() && sin.is_contiguous(),
+                    pos.is_contiguous() && pos.numel() == k.size(0),
                 "prefill attention: caches, lengths and position ids have to fit the rows");
-    for (const Tensor* t : {&k_cache, &v_cache, &ctx_len, &pos, &cos, &sin}) need_gpu(*t);
+    check_tables(k, k.size(2), cos, sin, interleaved, true);
+    for (const Tensor* t : {&k_cache, &v_cache, &ctx_len, &pos}) need_gpu(*t);
     Launch l(q);
     const Tensor k_rot = at::empty(k.sizes(), k.options());
     mi_fill_cache_args a{};
@@ -935,6 +948,7 @@ Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, const s
                     qkv_b.size() == qkv_w.size() && (rest_w.size() == 3 || rest_w.size() == 4) && rest_b.size() == rest_w.size() &&
                     (caches.empty() || caches.size() == 3),
                 "layer: bad arguments");
+    if (rotary != 0) check_tables(x, d, cos, sin, interleaved, rotary == 1);
     const int64_t b = x.size(0), s = x.size(1), tokens = b * s;
     auto [h, n] = op_add_norm(x, std::nullopt, *norms[0], norms[1], eps1, layer_norm1);
     Tensor ctx;

@@ -690,6 +690,17 @@ class ParallelSelfAttention(torch.nn.Module):
                                     self._decode_operand(v), rotary=rotary, softmax_scale=self.softmax_scale, workspace=cache.workspace)
 
 
+def _tables_fit(rot: torch.nn.Module, cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int, fused: bool) -> bool:
+    """Whether the kernels of a layer in one call read these tables as they are: float32 halves of a head (interleaved pairs), or as many features as
+    are rotated, of x's type (inside the attention core: the whole head) or float32."""
+    if not (cos.dim() == 2 and cos.shape == sin.shape and cos.dtype == sin.dtype and cos.device == sin.device == x.device and
+            cos.is_contiguous() and sin.is_contiguous()):
+        return False
+    if type(rot) is RotaryEmbeddingComplex:
+        return cos.dtype == torch.float32 and cos.shape[1] * 2 == head_dim
+    return (cos.dtype == x.dtype and cos.shape[1] == head_dim) if fused else (cos.dtype in (x.dtype, torch.float32) and cos.shape[1] <= head_dim)
+
+
 def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tensor, position_ids: Optional[torch.Tensor], use_cache: bool,
                       reset_cache: bool, cache_index: int) -> Optional[torch.Tensor]:
     """The output of a layer whose norms and MLP may be passed by (`fuses_residual`) in one native call of the operations its modules would
@@ -716,6 +727,13 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
         return None
     if use_cache and not (inference and reset_cache and att.causal and not att.qkv_in_one and att._fusable_rotary and pos is not None):
         return None
+    cos = sin = None
+    kind, interleaved = 0, False
+    if rot is not None:
+        cos, sin = rot.tables()
+        kind, interleaved = (1 if att._fusable_rotary and pos is not None else 2), type(rot) is RotaryEmbeddingComplex
+        if not _tables_fit(rot, cos, sin, x, att.hidden_size_per_attention_head, kind == 1):
+            return None
     if inference and not att.qkv_in_one:
         w, bias = att._fused_qkv()
         qkv_w, qkv_b = [w], [bias]
@@ -732,11 +750,6 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
         att.cache[cache_index] = None
     att._check_positions(pos)
     nq, nkv, d = att.num_attention_heads, att.num_kv_heads_per_partition, att.hidden_size_per_attention_head
-    cos = sin = None
-    kind, interleaved = 0, False
-    if rot is not None:
-        cos, sin = rot.tables()
-        kind, interleaved = (1 if att._fusable_rotary and pos is not None else 2), type(rot) is RotaryEmbeddingComplex
     caches = []
     if use_cache:
         cache = att._cache_for(b, s, dtype, x.device, cache_index)

@@ -5,8 +5,9 @@ import pytest
 import torch
 
 from scaling_amd import _lib, ops
-from scaling_amd.config import TransformerArchitectureConfig
+from scaling_amd.config import RotaryConfig, TransformerArchitectureConfig
 from scaling_amd.layer import InferenceSettings, TransformerLayer, TransformerLayerIO
+from scaling_amd.nn import RotaryEmbedding
 from tests.kernels import launched
 
 pytestmark = pytest.mark.gpu
@@ -465,3 +466,53 @@ def test_cached_keys_are_those_of_the_rotary_kernel(d, interleaved, dtype):
     kc, vc = (torch.zeros(1, s, nkv, d, dtype=dtype, device=DEV) for _ in range(2))
     _lib.host().prefill_attention(q, k, v, cu, pos, cos, sin, interleaved, d ** -0.5, 1, kc, vc, torch.zeros(1, dtype=torch.int32, device=DEV))
     assert torch.equal(kc[0], (ops.rotary_embedding_complex if interleaved else ops.rotary_embedding)(k, cos, sin, pos)) and torch.equal(vc[0], v)
+
+
+def _watched(layer, io):
+    """The layer's activations from its modules, which a hook keeps from being passed by."""
+    handle = layer.self_attention.register_forward_hook(lambda *a: None)
+    try:
+        return layer(io).activations
+    finally:
+        handle.remove()
+
+
+@pytest.mark.parametrize("default", [False, True])
+@pytest.mark.parametrize("tables", ["float32", "other16", "narrow"])
+def test_rotary_tables_that_the_kernels_cannot_read(tables, default):
+    """Tables of another type or of fewer features than a head, as casts and replaced modules leave them: refused where the attention core rotates, as
+    the modules refuse them; a prefill with float32 tables is computed, as the modules compute it."""
+    layer = _layer("bfloat16", default)
+    att, x = layer.self_attention, torch.randn(2, 40, 256, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+    if tables == "narrow":
+        att.rotary_embedding = RotaryEmbedding(RotaryConfig(dimensions=32, max_seq_length=512, base=10000), torch.device(DEV), torch.bfloat16)
+    else:
+        att.rotary_embedding.to(torch.float32 if tables == "float32" else torch.float16)
+    for train in (True, False):
+        layer.train(train)
+        with torch.set_grad_enabled(train), pytest.raises(AssertionError, match="fused rotary"):
+            layer(_io(x))
+    if default:
+        return
+    io = _io(x)
+    io.inference_settings = InferenceSettings(use_cache=True, reset_cache=True)
+    with torch.no_grad():
+        if tables == "other16":
+            with pytest.raises(RuntimeError, match="table dtype"):
+                layer(io)
+            return
+        y, cache = layer(io).activations, att.cache[0]
+        y, k, n = y.clone(), cache.k.clone(), cache.ctx_len.tolist()
+        assert torch.equal(y, _watched(layer, io)) and torch.equal(k, cache.k) and n == [40, 40] and y.isfinite().all()
+
+
+@pytest.mark.parametrize("cos_dtype,width,interleaved", [(torch.float32, 64, False), (torch.float16, 64, False), (torch.bfloat16, 32, False),
+                                                         (torch.bfloat16, 32, True), (torch.float32, 64, True)])
+def test_prefill_attention_refuses_tables_that_do_not_fit(cos_dtype, width, interleaved):
+    q, k, v = (torch.zeros(8, 2, 64, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    cos, sin = (torch.zeros(16, width, dtype=cos_dtype, device=DEV) for _ in range(2))
+    kc, vc = (torch.full((1, 8, 2, 64), 3.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    cu, ctx = torch.tensor([0, 8], dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="tables have to fit"):
+        _lib.host().prefill_attention(q, k, v, cu, torch.arange(8, device=DEV), cos, sin, interleaved, 0.125, 1, kc, vc, ctx)
+    assert bool((kc == 3).all()) and int(ctx) == 0
