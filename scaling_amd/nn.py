@@ -725,7 +725,8 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
     inference = not torch.is_grad_enabled() and not training
     if not (cu.is_cuda and cu.is_contiguous() and (pos is None or (pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == b * s))):
         return None
-    if use_cache and not (inference and reset_cache and att.causal and not att.qkv_in_one and att._fusable_rotary and pos is not None):
+    if use_cache and not (inference and reset_cache and att.causal and sdpa.causal and not att.qkv_in_one and att._fusable_rotary and
+                          pos is not None):
         return None
     cos = sin = None
     kind, interleaved = 0, False
@@ -755,7 +756,7 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
         cache = att._cache_for(b, s, dtype, x.device, cache_index)
         caches = [cache.k, cache.v, cache.ctx_len]
     h = ops.layer(x, cu, pos, norms, norm1.eps, norm2.eps, type(norm1) is LayerNorm, type(norm2) is LayerNorm, qkv_w, qkv_b, att.qkv_in_one, rest_w, rest_b,
-                  nq, nkv, d, att.causal, sdpa.softmax_scale, kind, interleaved, cos, sin, caches, not training)
+                  nq, nkv, d, sdpa.causal, sdpa.softmax_scale, kind, interleaved, cos, sin, caches, not training)
     if use_cache:
         cache.length = s
     return h

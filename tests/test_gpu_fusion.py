@@ -516,3 +516,25 @@ def test_prefill_attention_refuses_tables_that_do_not_fit(cos_dtype, width, inte
     with pytest.raises(RuntimeError, match="tables have to fit"):
         _lib.host().prefill_attention(q, k, v, cu, torch.arange(8, device=DEV), cos, sin, interleaved, 0.125, 1, kc, vc, ctx)
     assert bool((kc == 3).all()) and int(ctx) == 0
+
+
+@pytest.mark.parametrize("default", [False, True])
+@pytest.mark.parametrize("owner", ["attention", "core"])
+def test_mask_of_a_layer_is_its_cores(owner, default):
+    """`causal` of the attention module decides whether a cache may be filled, that of its core what is masked."""
+    layer, x = _layer("bfloat16", default).eval(), torch.randn(2, 70, 256, generator=torch.Generator().manual_seed(2)).bfloat16().to(DEV)
+    with torch.no_grad():
+        y = layer(_io(x)).activations
+        target = layer.self_attention if owner == "attention" else layer.self_attention.scaled_dot_product_attention
+        target.causal = False
+        changed = layer(_io(x)).activations
+        assert torch.equal(changed, _watched(layer, _io(x))) and torch.equal(changed, y) == (owner == "attention")
+        if default:
+            return
+        io = _io(x)
+        io.inference_settings = InferenceSettings(use_cache=True, reset_cache=True)
+        if owner == "attention":
+            with pytest.raises(ValueError, match="causal"):
+                layer(io)
+        else:
+            assert torch.equal(layer(io).activations, _watched(layer, io))
