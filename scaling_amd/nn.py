@@ -690,6 +690,19 @@ class ParallelSelfAttention(torch.nn.Module):
                                     self._decode_operand(v), rotary=rotary, softmax_scale=self.softmax_scale, workspace=cache.workspace)
 
 
+# What the modules of a layer call by name, with the functions that this package put there: a layer in one call passes them by.
+_PASSED_BY = tuple((cls, name, cls.__dict__[name]) for cls, names in (
+    (RMSNorm, ("with_residual",)), (LayerNorm, ("with_residual",)), (_Linear, ("forward",)), (ParallelMLP, ("forward",)),
+    (ParallelSwiGLUMLP, ("forward",)), (RotaryEmbedding, ("rotate_tokens",)), (RotaryEmbeddingComplex, ("rotate_tokens",)),
+    (ScaledDotProductAttention, ("forward_tokens", "forward_qkv")), (ParallelSelfAttention, ("forward", "_project", "_fill_cache"))) for name in names)
+_PASSED_BY_NAMES = frozenset(name for _, name, _ in _PASSED_BY)
+
+
+def _nothing_overridden(*modules: torch.nn.Module) -> bool:
+    """Whether nobody set one of those functions anew, on its class or on one of the modules."""
+    return all(getattr(cls, name) is own for cls, name, own in _PASSED_BY) and all(_PASSED_BY_NAMES.isdisjoint(m.__dict__) for m in modules)
+
+
 def _tables_fit(rot: torch.nn.Module, cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int, fused: bool) -> bool:
     """Whether the kernels of a layer in one call read these tables as they are: float32 halves of a head (interleaved pairs), or as many features as
     are rotated, of x's type (inside the attention core: the whole head) or float32."""
@@ -710,9 +723,9 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
     sdpa, rot, dtype, training = att.scaled_dot_product_attention, att.rotary_embedding, att.dtype, layer.training
     if not (x.is_cuda and x.dim() == 3 and x.dtype == dtype and x.numel() > 0 and not torch.is_autocast_enabled() and type(att) is ParallelSelfAttention and
             _unhooked(att) and fuses_residual(mlp) and idle_dropout(layer.dropout_attention) and idle_dropout(layer.dropout_mlp) and
-            not att.key_query_norm and type(sdpa) is ScaledDotProductAttention and "forward_tokens" not in sdpa.__dict__ and
-            "forward_qkv" not in sdpa.__dict__ and not (training and sdpa.dropout_p > 0.0) and
-            (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex))):
+            not att.key_query_norm and type(sdpa) is ScaledDotProductAttention and not (training and sdpa.dropout_p > 0.0) and
+            (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex)) and
+            _nothing_overridden(att, sdpa, mlp, norm1, norm2, *(() if rot is None else (rot,)))):
         return None
     swiglu = type(mlp) is ParallelSwiGLUMLP
     rest = (att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out) if swiglu else (att.dense, mlp.dense_in, mlp.dense_out)

@@ -538,3 +538,35 @@ def test_mask_of_a_layer_is_its_cores(owner, default):
                 layer(io)
         else:
             assert torch.equal(layer(io).activations, _watched(layer, io))
+
+
+@pytest.mark.parametrize("on_class", [False, True])
+@pytest.mark.parametrize("default,where,name", [
+    (False, "self_attention", "_project"), (True, "self_attention", "_fill_cache"), (False, "self_attention", "_fill_cache"),
+    (False, "self_attention.rotary_embedding", "rotate_tokens"), (True, "self_attention.scaled_dot_product_attention", "forward_qkv"),
+    (False, "self_attention.scaled_dot_product_attention", "forward_tokens"), (False, "input_layernorm", "with_residual"),
+    (True, "post_attention_layernorm", "with_residual"), (False, "mlp", "forward"), (True, "mlp", "forward"), (True, "self_attention.dense", "forward"),
+])
+def test_functions_that_somebody_set_anew_are_called(where, name, default, on_class, monkeypatch):
+    """A function of the layer's modules that is replaced, on the module or on its class, is called wherever the modules call it: in a pass without a
+    cache or in a prefill (which only the layer without one QKV projection can take here)."""
+    layer = _layer("bfloat16", default).eval()
+    x = torch.randn(2, 30, 256, generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)
+    module = layer.get_submodule(where)
+    calls, own = [], getattr(type(module), name)
+    io = _io(x)
+    with torch.no_grad():
+        y = layer(io).activations
+        if name in ("_fill_cache", "rotate_tokens"):       # called in a prefill alone
+            io.inference_settings = InferenceSettings(use_cache=True, reset_cache=True)
+            y = layer(io).activations
+
+        def replaced(self, *args, **kwargs):
+            calls.append(name)
+            return own(self, *args, **kwargs)
+
+        if on_class:
+            monkeypatch.setattr(type(module), name, replaced)
+        else:
+            monkeypatch.setattr(module, name, lambda *args, **kwargs: replaced(module, *args, **kwargs))
+        assert torch.equal(layer(io).activations, y) and calls
