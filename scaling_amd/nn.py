@@ -741,6 +741,9 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
     if use_cache and not (inference and reset_cache and att.causal and sdpa.causal and not att.qkv_in_one and att._fusable_rotary and
                           pos is not None):
         return None
+    held = att.cache.get(cache_index) if use_cache else None
+    if held is not None and not (held.k.dtype == held.v.dtype == dtype and held.k.device == held.v.device == x.device and held.k.stride() == held.v.stride()):
+        return None                                        # a cache that is there is kept, and copies convert
     cos = sin = None
     kind, interleaved = 0, False
     if rot is not None:

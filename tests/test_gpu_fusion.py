@@ -7,7 +7,7 @@ import torch
 from scaling_amd import _lib, ops
 from scaling_amd.config import RotaryConfig, TransformerArchitectureConfig
 from scaling_amd.layer import InferenceSettings, TransformerLayer, TransformerLayerIO
-from scaling_amd.nn import RotaryEmbedding
+from scaling_amd.nn import KVCache, RotaryEmbedding
 from tests.kernels import launched
 
 pytestmark = pytest.mark.gpu
@@ -570,3 +570,21 @@ def test_functions_that_somebody_set_anew_are_called(where, name, default, on_cl
         else:
             monkeypatch.setattr(module, name, lambda *args, **kwargs: replaced(module, *args, **kwargs))
         assert torch.equal(layer(io).activations, y) and calls
+
+
+@pytest.mark.parametrize("case", ["float16", "strides"])
+def test_prefill_into_a_cache_of_another_kind(case):
+    """A cache that is there and long enough is filled, whatever its type (a model that was cast in between) and strides, as the modules fill it."""
+    layer = _layer("bfloat16", False).eval()
+    att, x = layer.self_attention, torch.randn(2, 30, 256, generator=torch.Generator().manual_seed(4)).bfloat16().to(DEV)
+    io = _io(x)
+    io.inference_settings = InferenceSettings(use_cache=True, reset_cache=True)
+    results = []
+    for run in (lambda: layer(io).activations, lambda: _watched(layer, io)):
+        cache = att.cache[0] = KVCache(2, 512, 2, 64, torch.float16 if case == "float16" else torch.bfloat16, torch.device(DEV))
+        if case == "strides":
+            cache.v = cache.v.contiguous()
+        with torch.no_grad():
+            results.append([run(), cache.k, cache.v, cache.ctx_len])
+        assert att.cache[0] is cache and cache.length == 30
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and results[0][1].any()
