@@ -119,6 +119,27 @@ def test_route_of_a_call(nq, nkv, d, total, docs, causal, fwd, bwd):
         assert all(torch.equal(x, y) == (flags == bwd) for x, y in zip((dq, dk, dv), grads))
 
 
+# sizes around the lines between the routes, which lie where measurements put them: whichever is taken is one of the two, bit for bit, and the
+# two agree to the rounding of P and dS
+@pytest.mark.parametrize("nq,nkv,d,total,docs,causal", [
+    (8, 8, 128, 4096, 1, True), (8, 8, 128, 2048, 4, True), (4, 4, 128, 4096, 1, False), (32, 8, 128, 2048, 1, True), (12, 12, 96, 2560, 4, True),
+    (16, 16, 64, 4190, 1, True), (32, 1, 64, 2520, 3, True), (12, 12, 128, 877, 16, True), (8, 8, 64, 6000, 20, False),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_backward_takes_one_of_two_routes_that_agree(nq, nkv, d, total, docs, causal, dtype):
+    g = torch.Generator(device=DEV).manual_seed(total)
+    q, do = (torch.randn(total, nq, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    k, v = (torch.randn(total, nkv, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    cu = torch.tensor([i * total // docs for i in range(docs + 1)], dtype=torch.int32, device=DEV)
+    o, lse = ops.attention_forward(q, k, v, cu, None, causal, None)
+    run = lambda flags: ops.attention_backward(do, q, k, v, o, lse, cu, None, causal, None, flags=flags)
+    taken, short, tiled = run(0), run(SHORT), run(TILED)
+    assert any(all(torch.equal(a, b) for a, b in zip(taken, route)) for route in (short, tiled))
+    for name, a, b in zip(("dq", "dk", "dv"), short, tiled):
+        # both round the same P and dS but for the last bits of their float32 sums, and each its own results: two roundings each way
+        assert float((a.float() - b.float()).norm()) <= 2.0 ** (-6 if dtype == torch.bfloat16 else -9) * float(b.float().norm()), name
+
+
 # where a launch in front of the dK / dV blocks leaves delta: one of its own for long chains, or the dQ blocks' (single long documents above
 # 64 features, by the size of the call)
 @pytest.mark.parametrize("nq,nkv,d,lens,flags,kernel", [

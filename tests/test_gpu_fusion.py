@@ -1,6 +1,8 @@
 """Fused launches of the layer step against the separate launches they replace: residual add + norm (forward and
 backward), the packed-QKV attention node, column sums."""
 
+from unittest import mock
+
 import pytest
 import torch
 
@@ -346,6 +348,13 @@ def test_weight_gradients_through_a_transposed_operand(rows, ins, outs):
         assert bool(((w.grad[pick].double() - a @ b).abs() <= bound * 1.01).all())
 
 
+def _native_calls(call):
+    """How many layers of a call go through the native layer."""
+    with mock.patch.object(ops, "layer", wraps=ops.layer) as native:
+        call()
+    return native.call_count
+
+
 # norms, MLPs, projections, types and rotaries of a layer; a step, and the two forms of a pass without gradients
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 @pytest.mark.parametrize("default,options", [
@@ -374,6 +383,7 @@ def test_layer_in_one_call_equals_its_modules(dtype, default, options):
         return [out.detach(), x.grad] + [p.grad for p in layer.parameters()]
 
     for train, grad in ((True, True), (False, True), (True, False), (False, False)):
+        assert _native_calls(lambda: run(train, grad)) == 1
         native = run(train, grad)
         seen = []
         handle = layer.self_attention.register_forward_hook(lambda *a: seen.append(1))      # whoever watches a module sees it called
@@ -445,6 +455,7 @@ def test_prefill_in_one_call_equals_its_modules(dtype, kind, d, b, s):
             out.append(layer(io(step, x3.shape[1], False)).activations)
         return out + [cache.k, cache.v], seen
 
+    assert _native_calls(lambda: run(False)) == 3 and _native_calls(lambda: run(True)) == 0
     native, _ = run(False)
     modules, seen = run(True)
     assert len(seen) == 3
