@@ -691,16 +691,22 @@ class ParallelSelfAttention(torch.nn.Module):
 
 
 # What the modules of a layer call by name, with the functions that this package put there: a layer in one call passes them by.
-_PASSED_BY = tuple((cls, name, cls.__dict__[name]) for cls, names in (
+_PASSED_BY = [(cls, name) for cls, names in (
     (RMSNorm, ("with_residual",)), (LayerNorm, ("with_residual",)), (_Linear, ("forward",)), (ParallelMLP, ("forward",)),
     (ParallelSwiGLUMLP, ("forward",)), (RotaryEmbedding, ("rotate_tokens",)), (RotaryEmbeddingComplex, ("rotate_tokens",)),
-    (ScaledDotProductAttention, ("forward_tokens", "forward_qkv")), (ParallelSelfAttention, ("forward", "_project", "_fill_cache"))) for name in names)
-_PASSED_BY_NAMES = frozenset(name for _, name, _ in _PASSED_BY)
+    (ScaledDotProductAttention, ("forward_tokens", "forward_qkv")), (ParallelSelfAttention, ("forward", "_project", "_fill_cache"))) for name in names]
+_OWN_FUNCTIONS = [getattr(cls, name) for cls, name in _PASSED_BY]
 
 
 def _nothing_overridden(*modules: torch.nn.Module) -> bool:
-    """Whether nobody set one of those functions anew, on its class or on one of the modules."""
-    return all(getattr(cls, name) is own for cls, name, own in _PASSED_BY) and all(_PASSED_BY_NAMES.isdisjoint(m.__dict__) for m in modules)
+    """Whether nobody set one of those functions anew, on its class or on one of the modules (their `forward`s: see _unhooked)."""
+    if [getattr(cls, name) for cls, name in _PASSED_BY] != _OWN_FUNCTIONS:
+        return False
+    for m in modules:
+        d = m.__dict__
+        if "with_residual" in d or "rotate_tokens" in d or "forward_tokens" in d or "forward_qkv" in d or "_project" in d or "_fill_cache" in d:
+            return False
+    return True
 
 
 def _tables_fit(rot: torch.nn.Module, cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int, fused: bool) -> bool:
@@ -725,7 +731,7 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
             _unhooked(att) and fuses_residual(mlp) and idle_dropout(layer.dropout_attention) and idle_dropout(layer.dropout_mlp) and
             not att.key_query_norm and type(sdpa) is ScaledDotProductAttention and not (training and sdpa.dropout_p > 0.0) and
             (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex)) and
-            _nothing_overridden(att, sdpa, mlp, norm1, norm2, *(() if rot is None else (rot,)))):
+            _nothing_overridden(att, sdpa, norm1, norm2, *(() if rot is None else (rot,)))):
         return None
     swiglu = type(mlp) is ParallelSwiGLUMLP
     rest = (att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out) if swiglu else (att.dense, mlp.dense_in, mlp.dense_out)
