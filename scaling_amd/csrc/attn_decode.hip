@@ -14,6 +14,8 @@
 // first chunk is on its way.  (A launch of its own for the append took 3 - 5 us: a third of a step at batch 1.)
 #include "attn_common.h"
 
+#include <limits.h>
+
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 namespace {
@@ -30,6 +32,7 @@ struct DecodeParams {
     int batch, max_ctx, nq, nkv, n_rep, n_splits;
     int n_hc;      // chunks of up to 16 query heads per KV head (a workgroup serves one chunk)
     uint32_t splits_m, groups_m, hc_m;   // for divide(): by n_splits, nkv * n_hc and n_hc
+    int by_length; // sequences that are handed out by their lengths (see order_by_length), or 0
     int64_t c_sb, c_st, c_sh;
     int64_t q_sb, kn_sb, vn_sb;   // element strides between sequences of q / k_new / v_new
     float scale_log2;
@@ -149,25 +152,42 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 
     // All arguments at once: read where they are used they are four trips of the scalar cache, one after the other, in front of the first load.
     DecodeParams p = args;
-    arrived(p.q, p.kc, p.vc, p.o, p.ctx_len, p.k_new, p.v_new, p.max_ctx, p.nq, p.nkv, p.n_rep, p.n_splits, p.n_hc, p.splits_m, p.groups_m, p.hc_m);
+    arrived(p.q, p.kc, p.vc, p.o, p.ctx_len, p.k_new, p.v_new, p.max_ctx, p.nq, p.nkv, p.n_rep, p.n_splits, p.n_hc, p.splits_m, p.groups_m, p.hc_m, p.by_length);
     arrived(p.c_sb, p.c_st, p.c_sh, p.q_sb, p.kn_sb, p.vn_sb, p.scale_log2, p.ws_o, p.ws_ml, p.tickets);
     if constexpr (ROT == 1) arrived(p.cos, p.sin, p.pos, p.table_rows);
     if constexpr (ROT == 2) arrived(p.cos32, p.sin32, p.pos, p.table_rows);
 
     const int split = blockIdx.y;
-    const int b = divide(blockIdx.x, p.nkv * p.n_hc, p.groups_m), kv_hc = blockIdx.x - b * p.nkv * p.n_hc;
+    int b = divide(blockIdx.x, p.nkv * p.n_hc, p.groups_m);
+    const int kv_hc = blockIdx.x - b * p.nkv * p.n_hc;
     const int kvh = divide(kv_hc, p.n_hc, p.hc_m), hc = kv_hc - kvh * p.n_hc;
     // this workgroup's query heads: head0 .. head0 + n_heads of the group (groups of more than 16 heads take
     // several workgroups, each reading the group's K / V once)
     const int head0 = kvh * p.n_rep + 16 * hc;
     const int n_heads = min(16, p.n_rep - 16 * hc);
 
-    int ctx = p.ctx_len[b];
+    int ctx;
     int64_t pos = 0;                    // requested with ctx: the rows of the rotary tables need not wait for anything else
-    if constexpr (ROT != 0) {
-        pos = p.pos[b];
-        pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+    if (p.by_length == 0) {
+        ctx = p.ctx_len[b];
+        if constexpr (ROT != 0) pos = p.pos[b];
+    } else {                            // lane i: sequence i; of different lengths the b-th shortest, in the last split the b-th longest
+        const int i = min(lane, p.by_length - 1), len = p.ctx_len[i];
+        int64_t at = 0;
+        if constexpr (ROT != 0) at = p.pos[i];
+        if (__ballot(len != __builtin_amdgcn_readfirstlane(len)) != 0) {
+            const int key = lane < p.by_length ? min(max(len, 0), p.max_ctx) * 64 + lane : INT_MAX;
+            int rank = 0;
+            for (int j = 0; j < p.by_length; j += 8)
+#pragma unroll
+                for (int u = 0; u < 8; ++u) rank += __builtin_amdgcn_readlane(key, j + u) < key;
+            b = __builtin_ctzll(__ballot(lane < p.by_length && rank == (split == p.n_splits - 1 ? p.by_length - 1 - b : b)));
+        }
+        ctx = __builtin_amdgcn_readlane(len, b);
+        if constexpr (ROT != 0)
+            pos = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(at >> 32), b) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)at, b));
     }
+    if constexpr (ROT != 0) pos = pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
     const bool append = p.k_new != nullptr && ctx >= 1 && ctx <= p.max_ctx;
     ctx = ctx < 0 ? 0 : (ctx > p.max_ctx ? p.max_ctx : ctx);
     // keys of this split: [s0, s1), split length rounded up to whole workgroup iterations
@@ -420,7 +440,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        int32_t* ticket = p.tickets + blockIdx.x;
+        int32_t* ticket = p.tickets + b * p.nkv * p.n_hc + kv_hc;
         const int arrived = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last_lds = arrived == p.n_splits - 1;
         if (arrived == p.n_splits - 1) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
@@ -469,6 +489,21 @@ int choose_splits(int batch, int nkv, int max_ctx) {
     if (s > kMaxSplits) s = kMaxSplits;
     if (s < 1) s = 1;
     return (int)s;
+}
+
+// Workgroups go to the compute units in the order of the grid: split 0 of every (sequence, KV head), then split 1 and so on.  Where there are more of them
+// than compute units, the last, which are of the last split, join the first.  Splits are rounded up to whole iterations, so the last is the shortest, and
+// sequences of one length gain from that order; of different lengths, long ones met by chance, and such a call lost more than it had gained.  So where
+// workgroups share a compute unit, splits take the sequences from the shortest to the longest and the last split from the longest on: the units that get
+// two of them get short ones.  us in a graph, bf16, splits of a sequence side by side / split by split / by length:
+//   17 sequences of 2979 - 5956 keys, 32 / 8 heads of 128, 69.2 / 85.1 / 66.7     18 of 5977 - 11953 154 / 175 / 128     9 of 2979 - 5956 46.9 / 48.6 / 35.0
+//   10 of up to 12472, 8 / 8 of 64, 33.8 / 39.8 / 33.1                            36 of up to 13740, 16 / 4 of 128, 171 / 189 / 119
+//   17 of 4000, all of one length, 32 / 8 of 128, 76.9 / 75.8 / 75.6
+// A workgroup finds its sequence among the lengths of all, one per lane, which is 0.3 us; with fewer than 512 keys a split there is no more than that
+// to gain (344 keys: 12.7 split by split, 13.2 by length; 627: 15.4 / 13.3).  More than 64 sequences, with one or two KV heads, keep their order.
+int order_by_length(const DecodeParams& p) {
+    const int64_t blocks = (int64_t)p.batch * p.nkv * p.n_hc * p.n_splits;
+    return p.n_splits > 1 && p.batch > 1 && p.batch <= 64 && p.max_ctx >= 512 * p.n_splits && p.max_ctx < (1 << 24) && blocks > mi_compute_units() ? p.batch : 0;
 }
 
 // rot: 0 = none, 1 = rotate-half, 2 = interleaved pairs
@@ -563,6 +598,7 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
     p.vn_sb = a->v_new_stride_batch ? a->v_new_stride_batch : (int64_t)a->n_kv_heads * a->head_dim;
     p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
     if (p.tickets != nullptr && !merges_in_launch(p, a->head_dim)) p.tickets = nullptr;
+    p.by_length = order_by_length(p);
     p.ws_o = (float*)ws;
     p.ws_ml = p.ws_o + (size_t)a->batch * a->n_q_heads * splits * a->head_dim;
     hipStream_t st = (hipStream_t)a->stream;

@@ -349,3 +349,40 @@ def test_float16_keys_are_rounded_as_they_always_were(d):
     want = torch.where((feature >= d // 2) & (feature % 8 >= 2), twice, once)
     assert torch.equal(kc[:, 2].cpu(), want) and torch.equal(vc[:, 2].cpu(), v)
     assert int((want != once).sum()) > 10 and int((want != twice).sum()) > 10
+
+
+# more workgroups than compute units, with sequences of different lengths, of equal ones, without keys; the most sequences that are handed out by
+# length, and one more; one key too few for it; splits that are merged by the last workgroup and by a launch of their own
+@pytest.mark.parametrize("B,nq,nkv,d,max_ctx,n_splits,kind", [
+    (17, 32, 8, 128, 1100, 2, "half"), (17, 32, 8, 128, 1023, 2, "half"), (10, 8, 8, 64, 2048, 4, "half"), (64, 4, 1, 128, 2600, 5, "plain"),
+    (65, 4, 1, 128, 2600, 5, "plain"), (5, 16, 16, 64, 2100, 4, "pairs"), (3, 24, 2, 96, 16384, 32, "plain"), (5, 40, 2, 32, 16400, 16, "pairs"),
+    (63, 2, 2, 64, 1600, 3, "half"),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_decode_of_more_workgroups_than_compute_units(B, nq, nkv, d, max_ctx, n_splits, kind, dtype):
+    """Workgroups find their sequence by its length: every sequence has the bits it has in a call of its own."""
+    g = torch.Generator().manual_seed(B)
+    normal = lambda *shape: torch.randn(*shape, generator=g).to(dtype).to(DEV)
+    q, k_new, v_new, kc, vc = normal(B, nq, d), normal(B, nkv, d), normal(B, nkv, d), normal(B, max_ctx, nkv, d), normal(B, max_ctx, nkv, d)
+    lens = torch.randint(1, max_ctx + 1, (B,), generator=g)
+    lens[B // 2:] = lens[B // 2:].clamp(max=max_ctx // 3)  # several of one length
+    lens[0], lens[-1] = max_ctx, 0
+    ctx, pos, rotary = lens.int().to(DEV), (lens - 1).clamp(min=0).to(DEV), None
+    if kind != "plain":
+        angle = torch.rand(max_ctx, d // 2, generator=g) * 6
+        cos, sin = (angle.cos().to(DEV), angle.sin().to(DEV))
+        if kind == "half":
+            cos, sin = (torch.cat([t, t], 1).to(dtype) for t in (cos, sin))
+        rotary = (cos, sin, pos)
+    alone = []
+    for b in range(B):
+        one = [t[b:b + 1].clone() for t in (kc, vc)]
+        row = None if rotary is None else (*rotary[:2], pos[b:b + 1].contiguous())
+        alone.append([ops.decode_attention(q[b:b + 1], *one, ctx[b:b + 1], k_new[b:b + 1], v_new[b:b + 1], rotary=row, n_splits=n_splits), *one])
+    want = [torch.cat(t) for t in zip(*alone)]
+    for workspace in (None, ops.decode_workspace(B, nq, d, max_ctx, DEV)):
+        caches = kc.clone(), vc.clone()
+        for _ in range(2):
+            out = ops.decode_attention(q, *caches, ctx, k_new, v_new, rotary=rotary, n_splits=n_splits, workspace=workspace)
+            assert all(torch.equal(a, c) for a, c in zip((out, *caches), want))
+    assert not workspace.tickets.any()
