@@ -32,7 +32,6 @@ struct DecodeParams {
     int batch, max_ctx, nq, nkv, n_rep, n_splits;
     int n_hc;      // chunks of up to 16 query heads per KV head (a workgroup serves one chunk)
     uint32_t splits_m, groups_m, hc_m;   // for divide(): by n_splits, nkv * n_hc and n_hc
-    int by_length; // sequences that are handed out by their lengths (see order_by_length), or 0
     int64_t c_sb, c_st, c_sh;
     int64_t q_sb, kn_sb, vn_sb;   // element strides between sequences of q / k_new / v_new
     float scale_log2;
@@ -132,7 +131,8 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, int64_t bh, 
 // NWV wavefronts (4 or 8) share the keys of one (batch, KV head, split); with a single split the merged result
 // is the attention output and goes straight to `o`, otherwise the partial goes to the workspace.
 // ROT: 0 = q as it is, 1 = rotate-half rotary on the q load, 2 = interleaved-pair rotary on the q load.
-template <int D, int ROT, int NWV>
+// BY_LENGTH: sequences are handed out by their lengths (order_by_length).
+template <int D, int ROT, int NWV, bool BY_LENGTH>
 __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeParams args) {
     constexpr int kThreads = 64 * NWV;
     constexpr int KS = D / 32;          // contraction steps of Q K^T (32 features each)
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 
     // All arguments at once: read where they are used they are four trips of the scalar cache, one after the other, in front of the first load.
     DecodeParams p = args;
-    arrived(p.q, p.kc, p.vc, p.o, p.ctx_len, p.k_new, p.v_new, p.max_ctx, p.nq, p.nkv, p.n_rep, p.n_splits, p.n_hc, p.splits_m, p.groups_m, p.hc_m, p.by_length);
+    arrived(p.q, p.kc, p.vc, p.o, p.ctx_len, p.k_new, p.v_new, p.max_ctx, p.nq, p.nkv, p.n_rep, p.n_splits, p.n_hc, p.splits_m, p.groups_m, p.hc_m);
     arrived(p.c_sb, p.c_st, p.c_sh, p.q_sb, p.kn_sb, p.vn_sb, p.scale_log2, p.ws_o, p.ws_ml, p.tickets);
     if constexpr (ROT == 1) arrived(p.cos, p.sin, p.pos, p.table_rows);
     if constexpr (ROT == 2) arrived(p.cos32, p.sin32, p.pos, p.table_rows);
@@ -168,20 +168,20 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
 
     int ctx;
     int64_t pos = 0;                    // requested with ctx: the rows of the rotary tables need not wait for anything else
-    if (p.by_length == 0) {
+    if constexpr (!BY_LENGTH) {
         ctx = p.ctx_len[b];
         if constexpr (ROT != 0) pos = p.pos[b];
     } else {                            // lane i: sequence i; of different lengths the b-th shortest, in the last split the b-th longest
-        const int i = min(lane, p.by_length - 1), len = p.ctx_len[i];
+        const int n = args.batch, i = min(lane, n - 1), len = p.ctx_len[i];
         int64_t at = 0;
         if constexpr (ROT != 0) at = p.pos[i];
         if (__ballot(len != __builtin_amdgcn_readfirstlane(len)) != 0) {
-            const int key = lane < p.by_length ? min(max(len, 0), p.max_ctx) * 64 + lane : INT_MAX;
+            const int key = lane < n ? min(max(len, 0), p.max_ctx) * 64 + lane : INT_MAX;
             int rank = 0;
-            for (int j = 0; j < p.by_length; j += 8)
+            for (int j = 0; j < n; j += 8)
 #pragma unroll
                 for (int u = 0; u < 8; ++u) rank += __builtin_amdgcn_readlane(key, j + u) < key;
-            b = __builtin_ctzll(__ballot(lane < p.by_length && rank == (split == p.n_splits - 1 ? p.by_length - 1 - b : b)));
+            b = __builtin_ctzll(__ballot(lane < n && rank == (split == p.n_splits - 1 ? n - 1 - b : b)));
         }
         ctx = __builtin_amdgcn_readlane(len, b);
         if constexpr (ROT != 0)
@@ -359,6 +359,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     };
 
     ChunkRegs ra, rb;
+    __builtin_amdgcn_sched_barrier(0);                 // q, the new row and the tables first: their arrival is waited for alone
     request(ra, 0);                                    // without a branch, behind which q's arrival would be waited for as if this had not been sent
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (ROT == 1) {
@@ -501,25 +502,27 @@ int choose_splits(int batch, int nkv, int max_ctx) {
 //   17 of 4000, all of one length, 32 / 8 of 128, 76.9 / 75.8 / 75.6
 // A workgroup finds its sequence among the lengths of all, one per lane, which is 0.3 us; with fewer than 512 keys a split there is no more than that
 // to gain (344 keys: 12.7 split by split, 13.2 by length; 627: 15.4 / 13.3).  More than 64 sequences, with one or two KV heads, keep their order.
-int order_by_length(const DecodeParams& p) {
+bool order_by_length(const DecodeParams& p) {
     const int64_t blocks = (int64_t)p.batch * p.nkv * p.n_hc * p.n_splits;
-    return p.n_splits > 1 && p.batch > 1 && p.batch <= 64 && p.max_ctx >= 512 * p.n_splits && p.max_ctx < (1 << 24) && blocks > mi_compute_units() ? p.batch : 0;
+    return p.n_splits > 1 && p.batch > 1 && p.batch <= 64 && p.max_ctx >= 512 * p.n_splits && p.max_ctx < (1 << 24) && blocks > mi_compute_units();
 }
 
 // rot: 0 = none, 1 = rotate-half, 2 = interleaved pairs
-template <int D, int NWV> int launch_split(const DecodeParams& p, int rot, hipStream_t st) {
-    const dim3 grid((unsigned)p.batch * p.nkv * p.n_hc, p.n_splits);
-    if (rot == 2) decode_split_kernel<D, 2, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
+template <int D, int NWV, bool BY_LENGTH> int launch_split(const DecodeParams& p, int rot, hipStream_t st) {
+    const dim3 grid((unsigned)p.batch * p.nkv * p.n_hc, p.n_splits), block(64 * NWV);
+    if (rot == 2) decode_split_kernel<D, 2, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
     else if (rot == 1) {
         // rotate-half pairs feature i with i + D / 2: the same lane holds both only when D / 32 is even
-        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
+        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
         else return mi_fail(MI_E_SHAPE, "attn_decode: fused rotate-half rotary needs head_dim 64 or 128");
-    } else decode_split_kernel<D, 0, NWV><<<grid, dim3(64 * NWV), 0, st>>>(p);
+    } else decode_split_kernel<D, 0, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
     return mi_check_launch("decode_split");
 }
 
 template <int D> int launch_decode(const DecodeParams& p, int rot, hipStream_t st) {
-    const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8>(p, rot, st) : launch_split<D, 4>(p, rot, st);
+    const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8, false>(p, rot, st)
+                   : order_by_length(p)                          ? launch_split<D, 4, true>(p, rot, st)
+                                                                 : launch_split<D, 4, false>(p, rot, st);
     if (rc != MI_OK || p.n_splits == 1 || p.tickets != nullptr) return rc;
     constexpr int kRows = 128 / D;
     const int64_t n = (int64_t)p.batch * p.nq;
@@ -598,7 +601,6 @@ int decode_entry(const mi_decode_args* a, void* ws, size_t ws_bytes, bool static
     p.vn_sb = a->v_new_stride_batch ? a->v_new_stride_batch : (int64_t)a->n_kv_heads * a->head_dim;
     p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
     if (p.tickets != nullptr && !merges_in_launch(p, a->head_dim)) p.tickets = nullptr;
-    p.by_length = order_by_length(p);
     p.ws_o = (float*)ws;
     p.ws_ml = p.ws_o + (size_t)a->batch * a->n_q_heads * splits * a->head_dim;
     hipStream_t st = (hipStream_t)a->stream;
