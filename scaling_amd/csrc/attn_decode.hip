@@ -131,8 +131,8 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, int64_t bh, 
 // NWV wavefronts (4 or 8) share the keys of one (batch, KV head, split); with a single split the merged result
 // is the attention output and goes straight to `o`, otherwise the partial goes to the workspace.
 // ROT: 0 = q as it is, 1 = rotate-half rotary on the q load, 2 = interleaved-pair rotary on the q load.
-// BY_LENGTH: sequences are handed out by their lengths (order_by_length).
-template <int D, int ROT, int NWV, bool BY_LENGTH>
+// BY_LENGTH: sequences are handed out by their lengths (order_by_length).  NEW_IN_LDS: the new row waits in LDS for its chunk (two_per_unit).
+template <int D, int ROT, int NWV, bool BY_LENGTH, bool NEW_IN_LDS>
 __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeParams args) {
     constexpr int kThreads = 64 * NWV;
     constexpr int KS = D / 32;          // contraction steps of Q K^T (32 features each)
@@ -145,6 +145,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     __shared__ float wm_lds[NWV][16];
     __shared__ float wl_lds[NWV][16];
     __shared__ float wo_lds[NWV][16][D + 1];
+    __shared__ __attribute__((aligned(16))) elem_t new_lds[2][NEW_IN_LDS ? D : 8];
     __shared__ int last_lds;
 
     const int tid = threadIdx.x;
@@ -281,6 +282,13 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
     // the new row in place of what its key (and keys past it, which read the same row) brought
     auto put_new = [&](ChunkRegs& c, int it) {
         const int key0 = s0 + (NWV * it + wave) * kChunk, last = s1 - 1;
+        if constexpr (NEW_IN_LDS) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) kn[ks] = *reinterpret_cast<const uint4*>(new_lds[0] + 32 * ks + 8 * G);
+#pragma unroll
+            for (int j = 0; j < V_PER_LANE; ++j) vn[j] = *reinterpret_cast<const uint4*>(new_lds[1] + 8 * ((lane + 64 * j) % (D / 8)));
+        }
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -387,6 +395,14 @@ __global__ __launch_bounds__(64 * NWV, 2) void decode_split_kernel(const DecodeP
             for (int ks = 0; ks < KS; ++ks) st128(p.kc + dst + 32 * ks + 8 * G, kn[ks]);
         }
         if (lane < D / 8) st128(p.vc + dst + 8 * lane, vn[0]);
+        if constexpr (NEW_IN_LDS) {                        // read back by the same wavefront
+            if (l16 == 0) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<uint4*>(new_lds[0] + 32 * ks + 8 * G) = kn[ks];
+            }
+            if (lane < D / 8) *reinterpret_cast<uint4*>(new_lds[1] + 8 * lane) = vn[0];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
     }
     for (int it = 0; it < n_iter; it += 2) {
         if (it + 1 < n_iter) load_chunk(rb, it + 1);
@@ -507,22 +523,32 @@ bool order_by_length(const DecodeParams& p) {
     return p.n_splits > 1 && p.batch > 1 && p.batch <= 64 && p.max_ctx >= 512 * p.n_splits && p.max_ctx < (1 << 24) && blocks > mi_compute_units();
 }
 
+// Whether 8-wavefront workgroups of 64 features, of which there are more than compute units, share these.  Two fit by LDS, but by registers only where the new row
+// (K rotated, V) waits for its chunk in LDS instead: 119 registers, else 138.  One more trip through LDS is 0.1 - 0.2 us.  Long sequences are better off
+// alone, the next one starting where the shortest has ended.  us in a graph, bf16, alone / shared:
+//   57 sequences of 100 keys, 8 / 8 heads 7.3 / 6.7       30 of 800, 32 / 32 38.9 / 33.6       40 of 1200, 16 / 16 42.4 / 37.1
+//   64 of 851 - 1700, 32 / 32 111.2 / 104.9               20 of 601 - 1200, 16 / 16 21.4 / 22.5   40 of 2500, 16 / 16 77.4 / 72.4
+//   20 of up to 2500, 16 / 16 29.2 / 34.8                  57 of up to 4000, 8 / 8 62.5 / 66.4
+template <int D> bool two_per_unit(const DecodeParams& p) {
+    return D == 64 && (int64_t)p.batch * p.nkv * p.n_hc * p.n_splits > mi_compute_units() && p.max_ctx <= 2048;
+}
+
 // rot: 0 = none, 1 = rotate-half, 2 = interleaved pairs
-template <int D, int NWV, bool BY_LENGTH> int launch_split(const DecodeParams& p, int rot, hipStream_t st) {
+template <int D, int NWV, bool BY_LENGTH, bool NEW_IN_LDS = false> int launch_split(const DecodeParams& p, int rot, hipStream_t st) {
     const dim3 grid((unsigned)p.batch * p.nkv * p.n_hc, p.n_splits), block(64 * NWV);
-    if (rot == 2) decode_split_kernel<D, 2, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
+    if (rot == 2) decode_split_kernel<D, 2, NWV, BY_LENGTH, NEW_IN_LDS><<<grid, block, 0, st>>>(p);
     else if (rot == 1) {
         // rotate-half pairs feature i with i + D / 2: the same lane holds both only when D / 32 is even
-        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
+        if constexpr (D == 64 || D == 128) decode_split_kernel<D, 1, NWV, BY_LENGTH, NEW_IN_LDS><<<grid, block, 0, st>>>(p);
         else return mi_fail(MI_E_SHAPE, "attn_decode: fused rotate-half rotary needs head_dim 64 or 128");
-    } else decode_split_kernel<D, 0, NWV, BY_LENGTH><<<grid, block, 0, st>>>(p);
+    } else decode_split_kernel<D, 0, NWV, BY_LENGTH, NEW_IN_LDS><<<grid, block, 0, st>>>(p);
     return mi_check_launch("decode_split");
 }
 
 template <int D> int launch_decode(const DecodeParams& p, int rot, hipStream_t st) {
-    const int rc = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx) ? launch_split<D, 8, false>(p, rot, st)
-                   : order_by_length(p)                          ? launch_split<D, 4, true>(p, rot, st)
-                                                                 : launch_split<D, 4, false>(p, rot, st);
+    const bool wide = wide_blocks(p.batch, p.nkv * p.n_hc, p.max_ctx);
+    const int rc = wide ? (two_per_unit<D>(p) ? launch_split<D, 8, false, D == 64>(p, rot, st) : launch_split<D, 8, false>(p, rot, st))
+                        : (order_by_length(p) ? launch_split<D, 4, true>(p, rot, st) : launch_split<D, 4, false>(p, rot, st));
     if (rc != MI_OK || p.n_splits == 1 || p.tickets != nullptr) return rc;
     constexpr int kRows = 128 / D;
     const int64_t n = (int64_t)p.batch * p.nq;

@@ -386,3 +386,39 @@ def test_decode_of_more_workgroups_than_compute_units(B, nq, nkv, d, max_ctx, n_
             out = ops.decode_attention(q, *caches, ctx, k_new, v_new, rotary=rotary, n_splits=n_splits, workspace=workspace)
             assert all(torch.equal(a, c) for a, c in zip((out, *caches), want))
     assert not workspace.tickets.any()
+
+
+@pytest.mark.parametrize("kind", ["plain", "half", "pairs"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,nq,nkv,n_splits", [(33, 16, 8, 0), (48, 6, 6, 0), (24, 8, 8, 2)])
+def test_workgroups_that_share_a_compute_unit(B, nq, nkv, n_splits, dtype, kind):
+    """Up to 2048 keys the new row of heads of 64 waits for its chunk in LDS, with one more in registers: the same bits, and the oracle's values."""
+    g, d, lens = torch.Generator().manual_seed(B + nq), 64, [1, 31, 32, 33, 255, 256, 257, 600, 2048, 0]
+    normal = lambda *shape: torch.randn(*shape, generator=g).to(dtype).to(DEV)
+    q, k_new, v_new, kc, vc = normal(B, nq, d), normal(B, nkv, d), normal(B, nkv, d), normal(B, 2049, nkv, d), normal(B, 2049, nkv, d)
+    ctx = torch.tensor((lens * 5)[:B], dtype=torch.int32, device=DEV)
+    pos, rotary = (ctx.long() - 1).clamp(min=0), None
+    if kind != "plain":
+        angle = torch.rand(2048, d // 2, generator=g) * 6
+        cos, sin = (angle.cos().to(DEV), angle.sin().to(DEV))
+        if kind == "half":
+            cos, sin = (torch.cat([t, t], 1).to(dtype) for t in (cos, sin))
+        rotary = (cos, sin, pos)
+    results = []
+    for max_ctx in (2048, 2049):
+        caches = kc.clone(), vc.clone()
+        call = lambda: results.append([ops.decode_attention(q, *(c[:, :max_ctx] for c in caches), ctx, k_new, v_new, rotary=rotary, n_splits=n_splits), *caches])
+        call()
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    for b in range(min(B, 10)):
+        assert torch.equal(vc[b, lens[b]:], results[0][2][b, lens[b]:]) and torch.equal(kc[b, :max(lens[b] - 1, 0)], results[0][1][b, :max(lens[b] - 1, 0)])
+        if lens[b] > 0:
+            assert torch.equal(results[0][2][b, lens[b] - 1], v_new[b])
+    rotated = q if rotary is None else (ops.rotary_embedding if kind == "half" else ops.rotary_embedding_complex)(q, cos, sin, pos)
+    some = [b for b in range(10) if lens[b] > 0]
+    for b in some:
+        keys, values = (t[b, :lens[b]].float().repeat_interleave(nq // nkv, 1) for t in results[0][1:])
+        p = torch.einsum("hd,thd->ht", rotated[b].float().cpu(), keys.cpu()).mul(d ** -0.5).softmax(-1)
+        want = torch.einsum("ht,thd->hd", p, values.cpu())
+        # P is rounded to 16 bits before it meets V, the result once more; q by the rotary, once or twice
+        assert float((results[0][0][b].float().cpu() - want).norm()) <= (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10) * float(want.norm()), b
