@@ -449,7 +449,7 @@ typedef struct mi_decode_args {
 /* What a prefill of `batch` sequences of `seq` tokens leaves in a KV cache (the layout of mi_decode_args): k rotated and v of its
  * [batch * seq, n_kv_heads, head_dim] rows at positions 0 .. seq - 1, ctx_len[b] = seq; the rotated k also packed in k_rot, for mi_attn_fwd with
  * position_ids_k == NULL.  Replaces attention.py:836-845 (k) and :861-862 of the reference.  16-bit types, head_dim 64 or 128; table
- * formats and rotary_interleaved as in mi_attn_args, the arithmetic of mi_rotary / mi_rotary_complex. */
+ * formats and rotary_interleaved as in mi_attn_args, the bits of mi_rotary / mi_rotary_complex. */
 typedef struct mi_fill_cache_args {
     const void* k;
     const void* v;
@@ -475,7 +475,8 @@ int mi_attn_decode(const mi_decode_args* args);
  * (which the host takes longer to issue than such a call takes): same arguments, same bits.
  * tickets: n_tickets >= batch * n_kv_heads * ceil(n_q_heads / n_kv_heads / 16) (never more than batch * n_q_heads) int32 of device memory,
  * all zero before the first call; every call leaves them zero.  Like the workspace they belong to one call at a time: calls that may
- * overlap (different streams) need tickets of their own. */
+ * overlap (different streams) need tickets of their own.  Unlike the workspace they outlive a mistake: after calls that overlapped on them they
+ * may not be zero, and calls then merge too early or never until they are cleared. */
 int mi_attn_decode_with_tickets(const mi_decode_args* args, int32_t* tickets, int64_t n_tickets);
 
 /* mi_attn_decode for callers that cannot allocate device memory (code under HIP graph capture, tight serving

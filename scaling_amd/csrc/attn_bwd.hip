@@ -685,8 +685,12 @@ __device__ __forceinline__ void dq_block(const AttnParams& p, const BwdShared<D>
 // the dQ blocks start where dK / dV blocks, the longer ones, have ended.  One launch each / together, us with delta, head_dim 128, bf16:
 //   8192 tokens 32 / 8 heads 1704 / 1687      the same in documents of 256 - 2048 380 / 359      4 x 2048, 16 / 16 279 / 272
 //   2445, 32 / 32 234 / 203                   4397, 16 / 2, no mask 830 / 621                   4 x 538, 32 / 8 of 64, no mask 129 / 95
-// The second argument of __launch_bounds__ is wavefronts per SIMD: the two that one 512-thread workgroup brings, where the
-// kernel takes 253 of the 256 registers each of them can have (no AGPRs, no scratch), or two workgroups' at head_dim 32.
+// The second argument of __launch_bounds__ is wavefronts per SIMD, the two of one 512-thread workgroup or, at head_dim 32, the four of two.  Registers and
+// scratch bytes as compiled, default / dropout / accuracy mode: head_dim 128 255, none / 256, 16 / 249 (float16 256), none; 96 207 / 213 / 229 (224),
+// 64 169 / 174 / 176 (177), none; 32 128, 20 / 128, 44 / 128, 36 (68).  With one workgroup per compute unit head_dim 32 takes 135 - 141 and no scratch, which is
+// faster where there are few blocks only.  us of a backward pass, one / two workgroups per compute unit, bf16: 8192 tokens, 32 / 8 heads 763 / 636, dropout 1239 /
+// 981, accuracy 1084 / 909 (float16 1102 / 967); 4397, 16 / 2, no mask 274 / 275, 454 / 432, 387 / 392; 4096, 16 / 16 141 / 132, 229 / 247, 198 / 192; 3001,
+// 12 / 12 80 / 85, 119 / 150, 102 / 128.
 template <int D, bool DROP, bool SPLIT>
 __global__ __launch_bounds__(512, D == 32 ? 4 : 2) void attn_bwd_kernel(const AttnParams p, int n_dkdv) {
     __shared__ __attribute__((aligned(1024))) char tiles[BwdShared<D>::kTileBytes];

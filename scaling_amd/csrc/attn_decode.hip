@@ -481,7 +481,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeParams p) 
 // Whether the last workgroup merges, given tickets.  On the device that is no gain: its one workgroup per (batch, KV head) loads past the caches what
 // the merge launch spreads over more of them, with a thread for every two features of its heads and up to 16 splits 0 - 1 us more than that
 // launch, beyond 2 - 9.  But a call of so few bytes is over before the host has issued two launches: batch 1, 32 / 8 heads of 128, a cache of 1,564, one call
-// after the other 10.9 -> 8.8 us.
+// after the other 9.1 -> 7.6 us from C, 10.9 -> 8.8 from Python.
 bool merges_in_launch(const DecodeParams& p, int head_dim) {
     const int heads = p.n_rep < 16 ? p.n_rep : 16;
     return p.n_splits > 1 && p.n_splits <= 16 && heads * head_dim <= 512 &&

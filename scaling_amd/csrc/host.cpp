@@ -1185,7 +1185,8 @@ void op_decode_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v
     }
     a.workspace = ptr(*workspace);
     a.workspace_bytes = (size_t)workspace->numel() * 4;
-    // One launch less where the tickets that came with the workspace are enough; a graph issues the second one for nothing.
+    // One launch less where the tickets that came with the workspace are enough.  A graph issues the second one for nothing, and on the device two are level or
+    // ahead (us in a graph, one / two launches: 1500 keys, 32 / 8 heads of 128 7.4 / 6.7; 2 x 960, 16 / 16 of 64 6.1 / 5.3; 536, 32 / 8 of 128 6.2 / 6.4).
     const bool merge = tickets.has_value() && tickets->scalar_type() == at::kInt && tickets->is_contiguous() && tickets->device() == out.device() &&
                        tickets->numel() >= (int64_t)a.batch * a.n_q_heads &&
                        c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;

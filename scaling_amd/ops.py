@@ -491,7 +491,9 @@ def _decode_scratch(batch: int, n_q_heads: int, head_dim: int, max_ctx: int, dev
 def decode_workspace(batch: int, n_q_heads: int, head_dim: int, max_ctx: int, device) -> torch.Tensor:
     """Scratch of `decode_attention` for calls that do not overlap.  With it come the arrival counts (attribute `tickets`, int32, zero
     between calls) by which the last workgroup of a small call merges the splits of the keys in the same launch; a workspace without them (a
-    slice, a tensor of the caller's own) takes a second launch for the same result."""
+    slice, a tensor of the caller's own) takes a second launch for the same result.  The counts are cleared on the current stream, so a first call
+    on another stream waits for this one; and where calls on one workspace overlapped all the same, not these calls alone are spoilt: counts
+    that are not zero again make later ones merge too early or never, until `tickets` is cleared (`workspace.tickets.zero_()`)."""
     workspace = _decode_scratch(batch, n_q_heads, head_dim, max_ctx, device)
     workspace.tickets = torch.zeros(max(batch * n_q_heads, 0), dtype=torch.int32, device=device)
     return workspace
