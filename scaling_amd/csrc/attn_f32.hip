@@ -126,6 +126,10 @@ template <int D, int ROWS> struct F32Dma {
             off[j] = (uint32_t)(row * (int)row_stride * 4 + byte);
         }
     }
+    // instruction j of that alone, of a tile that is whole
+    __device__ __forceinline__ void issue_whole(int j, const float* tile_base, char* tile) const {
+        DmaPlan<D, 1>::issue_one(off[j], tile_base, tile + 1024 * (n0 + j));
+    }
     // rows row0 .. row0 + ROWS - 1 of `base` (rows past last_row repeat it) into `tile`
     __device__ __forceinline__ void issue(const float* base, int64_t row_stride, int row0, int last_row, char* tile) const {
         char* dst = tile + 1024 * n0;
@@ -186,6 +190,60 @@ __device__ __forceinline__ void cols_product(f32x16_t (&acc)[D / 32], const char
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[dt] = mfma_f32(a[r & 1][dt], x[r], acc[dt]);
     }
+}
+
+// The two products of a kernel whose wavefronts have a SIMD each, with the rest of its work between them: between(j) behind every fourth product of rows
+// and behind the DT products of a row of columns.  They are inline assembly because the compiler keeps the gradients' accumulators in vector registers otherwise
+// and moves all of them to accumulation registers and back in every step; C tiles that vector instructions read are in vector registers.  What the compiler
+// does not see then are waits between a product and whoever reads its result: between() may read the C tile of the product before this one
+// (four products of 64 cycles lie between), and `settled` is for the end.
+__device__ __forceinline__ void mma_v(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
+__device__ __forceinline__ void mma_v0(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b)); }
+__device__ __forceinline__ void mma_acc(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
+__device__ __forceinline__ void clear_acc(f32x16_t& c) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[r] = 0.f;
+    asm volatile("" : "+a"(c));
+}
+__device__ __forceinline__ void settled() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+
+// a0, x0: the first operand, read ahead; then(): reads the one of the product behind this
+template <int D, class F, class G>
+__device__ __forceinline__ void rows_product_with(f32x16_t& c, const char* tile, int row, int g, const f32x4_t& a0, const f32x4_t (&b)[D / 8], F&& between, G&& then) {
+    f32x4_t a[2];
+    a[0] = a0;
+    static_for<D / 8>([&](auto j_c) {
+        constexpr int j = decltype(j_c)::value;
+        if constexpr (j + 1 < D / 8) a[(j + 1) & 1] = F32Tile<D>::row4(tile, row, j + 1, g);
+        else then();
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<4>([&](auto i_c) {
+            constexpr int i = decltype(i_c)::value;
+            if constexpr (j == 0 && i == 0) mma_v0(c, a[0][0], b[0][0]);
+            else mma_v(c, a[j & 1][i], b[j][i]);
+        });
+        between(j_c);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
+template <int D, class F, class G>
+__device__ __forceinline__ void cols_product_with(f32x16_t (&acc)[D / 32], const char* tile, int row0, const float (&x0)[D / 32], const f32x16_t& x, int l32, int g,
+                                                  F&& between, G&& then) {
+    constexpr int DT = D / 32;
+    float a[2][DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) a[0][dt] = x0[dt];
+    static_for<16>([&](auto r_c) {
+        constexpr int r = decltype(r_c)::value;
+        if constexpr (r + 1 < 16) F32Tile<D>::cols(tile, row0 + acc_row(r + 1, g), l32, a[(r + 1) & 1]);
+        else then();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) mma_acc(acc[dt], a[r & 1][dt], x[r]);
+        between(r_c);
+        __builtin_amdgcn_sched_barrier(0);
+    });
 }
 
 // stores the features that accumulator registers r0 .. r0 + N - 1 hold of one token's row
@@ -412,6 +470,12 @@ template <int D, int KGRP, bool KEEP>
 __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const F32Params fp) {
     constexpr int DT = D / 32, QS = kF32Waves / KGRP, BQ = 32 * QS, BK = 32 * KGRP;
     constexpr int NS = n_stages<D, BQ>(), TILE = BQ * 4 * D;
+    // A wavefront has its SIMD to itself and a product takes the matrix pipe 64 cycles, so loads, softmax and moves between two stages of a step cost what they
+    // take: the pipe was busy 0.68 of the time, 0.74 with all of them between products (the rest: a clock of 2.07 GHz instead of 2.17, the barrier of a step, the last
+    // blocks of the launch).  us, before / after: 32 / 8 heads of 128, 4096 tokens 2600 / 2380, 32 / 32, 1101 245 / 230, 8 / 8, 700 (KGRP 1) 70.2 / 66.9; of 96, 32 / 32, 1101
+    // 201 / 186.  Where stages are short or one tile deep it does not pay: of 96, KGRP 1 564 / 583, of 64, KGRP 1 100.0 / 101.1 and 11.1 / 11.7, of 32 358 / 359.
+    constexpr bool kBetween = D == 128 || (D == 96 && KGRP == 2);
+    static_assert(!kBetween || DT >= 2, "dS is formed one row of products behind dP");
     __shared__ __attribute__((aligned(1024))) char smem[NS * 2 * TILE];
     __shared__ __attribute__((aligned(16))) float lse_lds[2][BQ], delta_lds[2][BQ];
     __shared__ int range_lds[2 * kF32Waves];
@@ -440,7 +504,18 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
     do_dma.init(wave, lane, p.o_st);
     // (query head of the group, query tile) of the next step; heads outermost, in a fixed order: bit-reproducible sums
     int nxt_rep = 0, nxt_tile = 0, nxt = 0;
-    float stat = 0.f;
+    // log-sum-exp and delta of a step's queries, straight into LDS like the tiles: a load into a register would make the compiler wait for the stores of dS
+    // behind it as well
+    auto issue_stat = [&](int head, int qt, int buf) {
+        if (wave >= 2 * BQ / 64) return;
+        const bool first = wave < BQ / 64;
+        const int at = 64 * (first ? wave : wave - BQ / 64);
+        const float* row = (first ? fp.lse : fp.delta) + (int64_t)head * p.total_q + qt;   // qt < total_q
+        const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(char*)((first ? lse_lds[buf] : delta_lds[buf]) + at);
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                     ::"v"(4u * (uint32_t)min(at + lane, p.total_q - 1 - qt)), "s"(row), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+    };
+    float stat = 0.f;                     // without kBetween they pass through a register of threads 0 .. 2 BQ - 1
     const float* stat_base = tid < BQ ? fp.lse : fp.delta;
     auto issue = [&]() {
         if (nxt >= n_steps) return;
@@ -448,7 +523,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
         char* st = smem + (nxt % NS) * 2 * TILE;
         q_dma.issue(fp.q + (int64_t)head * p.q_sh, p.q_st, qt, p.total_q - 1, st);
         do_dma.issue(fp.d_o + (int64_t)head * p.o_sh, p.o_st, qt, p.total_q - 1, st + TILE);
-        if (tid < 2 * BQ) stat = stat_base[(int64_t)head * p.total_q + min(qt + (tid & (BQ - 1)), p.total_q - 1)];
+        if constexpr (kBetween) issue_stat(head, qt, nxt & 1);
+        else if (tid < 2 * BQ) stat = stat_base[(int64_t)head * p.total_q + min(qt + (tid & (BQ - 1)), p.total_q - 1)];
         if (++nxt_tile == n_tiles) { nxt_tile = 0; ++nxt_rep; }
         ++nxt;
     };
@@ -465,52 +541,145 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
     issue();
     f32x16_t dk_acc[DT], dv_acc[DT];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt) {
+        if constexpr (kBetween) {
+            clear_acc(dk_acc[dt]);
+            clear_acc(dv_acc[dt]);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) { dk_acc[dt][r] = 0.f; dv_acc[dt][r] = 0.f; }
+            for (int r = 0; r < 16; ++r) { dk_acc[dt][r] = 0.f; dv_acc[dt][r] = 0.f; }
+        }
+    }
     const float c2 = p.scale_log2;
     const DsLayout ds(p.total_q, p.total_k, fp.ds_triangle);
     int tile = 0, rep = 0;
-    for (int step = 0; step < n_steps; ++step) {
-        put_stat(step);
-        wait_vmcnt<0>();
-        __syncthreads();                  // the step has landed, and the readers of the one before are done
-        if constexpr (NS == 2) issue();
-        const int qt = qt0 + tile * BQ + 32 * qs, head = kvh * p.n_rep + hs * hpw + rep;
-        if (++tile == n_tiles) { tile = 0; ++rep; }
-        if (qt < wmax && qt + 32 > wmin) {
-            const char* q_s = smem + (step % NS) * 2 * TILE;
-            const char* do_s = q_s + TILE;
-            f32x16_t s = rows_product<D>(q_s, 32 * qs + l32, g, kf);         // rows = queries, column = this lane's key
-            f32x16_t dp = rows_product<D>(do_s, 32 * qs + l32, g, vf);
-            const bool edge = __any(qt < qlo || qt + 32 > qhi);
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&lse_lds[step & 1][32 * qs + 8 * a + 4 * g]);
-                const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&delta_lds[step & 1][32 * qs + 8 * a + 4 * g]);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const int r = 4 * a + c;
-                    float pv = fast_exp2(s[r] * c2 - l4[c]);
-                    if (edge) {
-                        const int q = qt + 8 * a + 4 * g + c;
-                        if (q < qlo || q >= qhi) pv = 0.f;
+    if constexpr (kBetween) {
+        // What is not a product goes between products: the direct loads of the next step between those of S, P between those of dP, dS between those of dV.
+        constexpr int kLoads = F32Dma<D, BQ>::kCount, kParts = D / 8;
+        bool stored = false;                  // by the step before, behind its loads: four stores that need not have arrived
+        for (int step = 0; step < n_steps; ++step) {
+            if (KEEP && NS == 2 && stored) wait_vmcnt<4>(); else wait_vmcnt<0>();
+            __syncthreads();                  // the step has landed, and the readers of the one before are done
+            const int qt = qt0 + tile * BQ + 32 * qs, head = kvh * p.n_rep + hs * hpw + rep;
+            if (++tile == n_tiles) { tile = 0; ++rep; }
+            const bool wanted = qt < wmax && qt + 32 > wmin;
+            // the next step's tiles, if they are whole: as issue() requests them
+            const int next_qt = qt0 + nxt_tile * BQ, next_head = kvh * p.n_rep + hs * hpw + nxt_rep;
+            const bool between = NS == 2 && wanted && nxt < n_steps && next_qt + BQ <= p.total_q;
+            const float* next_q = fp.q + (int64_t)next_head * p.q_sh + (int64_t)next_qt * p.q_st;
+            const float* next_do = fp.d_o + (int64_t)next_head * p.o_sh + (int64_t)next_qt * p.o_st;
+            char* next_stage = smem + (nxt % NS) * 2 * TILE;
+            if (between) {
+                issue_stat(next_head, next_qt, nxt & 1);
+                if (++nxt_tile == n_tiles) { nxt_tile = 0; ++nxt_rep; }
+                ++nxt;
+            } else if constexpr (NS == 2) {
+                issue();
+            }
+            stored = wanted;
+            if (wanted) {
+                const char* q_s = smem + (step % NS) * 2 * TILE;
+                const char* do_s = q_s + TILE;
+                int l = l32, h = g;
+                asm volatile("" : "+v"(l), "+v"(h));   // opaque: the swizzled LDS addresses are made where they are used, not kept in registers over the steps
+                f32x16_t s, dp;                   // rows = queries, column = this lane's key
+                f32x4_t row0;
+                float col0[2][DT];
+                rows_product_with<D>(s, q_s, 32 * qs + l, h, F32Tile<D>::row4(q_s, 32 * qs + l, 0, h), kf, [&](auto j) {
+                    if (between) {
+                        static_for<2 * kLoads>([&](auto n_c) {
+                            constexpr int n = decltype(n_c)::value;
+                            if constexpr (n * kParts / (2 * kLoads) == decltype(j)::value) {
+                                if constexpr (n < kLoads) q_dma.issue_whole(n, next_q, next_stage);
+                                else do_dma.issue_whole(n - kLoads, next_do, next_stage + TILE);
+                            }
+                        });
                     }
-                    s[r] = pv;
-                    dp[r] = pv * (dp[r] - d4[c]);
-                }
+                }, [&] { row0 = F32Tile<D>::row4(do_s, 32 * qs + l, 0, h); });
+                const unsigned seen = (unsigned)(qhi - qlo);
+                const int rel0 = qt + 4 * h - qlo;
+                const float* lse_row = &lse_lds[step & 1][32 * qs + 4 * h];
+                const float* delta_row = &delta_lds[step & 1][32 * qs + 4 * h];
+                auto log2_sums = [&](int a) {     // rounded before they are subtracted, as a product of their own
+                    f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(lse_row + 8 * a) * kLog2eF;
+                    asm volatile("" : "+v"(l4));
+                    return l4;
+                };
+                f32x4_t l4 = log2_sums(0);
+                rows_product_with<D>(dp, do_s, 32 * qs + l, h, row0, vf, [&](auto j) {
+                    static_for<16>([&](auto r_c) {
+                        constexpr int r = decltype(r_c)::value, a = r >> 2, c = r & 3;
+                        if constexpr (r * kParts / 16 == decltype(j)::value) {
+                            float pv = fast_exp2(s[r] * c2 - l4[c]);
+                            pv = (unsigned)(rel0 + 8 * a + c) < seen ? pv : 0.f;
+                            asm volatile("" : "+v"(pv));   // here, not where it is used
+                            s[r] = pv;
+                            if constexpr (c == 3 && a < 3) l4 = log2_sums(a + 1);
+                        }
+                    });
+                }, [&] { F32Tile<D>::cols(do_s, 32 * qs + acc_row(0, h), l, col0[0]); });
+                f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(delta_row);
+                float* out = KEEP ? fp.ds + ds.tile(head - first_kv * p.n_rep, qt, kb * BK + kgrp * 32) + l32 * 32 + 4 * g : nullptr;
+                cols_product_with<D>(dv_acc, do_s, 32 * qs, col0[0], s, l, h, [&](auto r_c) {
+                    constexpr int r = decltype(r_c)::value, a = r >> 2, c = r & 3;
+                    float dsv = s[r] * (dp[r] - d4[c]);
+                    asm volatile("" : "+v"(dsv));
+                    dp[r] = dsv;
+                    if constexpr (c == 3) {
+                        if constexpr (KEEP) *reinterpret_cast<f32x4_t*>(out + 8 * a) = f32x4_t{dp[4 * a], dp[4 * a + 1], dp[4 * a + 2], dp[4 * a + 3]};
+                        if constexpr (a < 3) d4 = *reinterpret_cast<const f32x4_t*>(delta_row + 8 * (a + 1));
+                    }
+                }, [&] { F32Tile<D>::cols(q_s, 32 * qs + acc_row(0, h), l, col0[1]); });
+                cols_product_with<D>(dk_acc, q_s, 32 * qs, col0[1], dp, l, h, [](auto) {}, [] {});
             }
-            if constexpr (KEEP) {
-                float* out = fp.ds + ds.tile(head - first_kv * p.n_rep, qt, kb * BK + kgrp * 32) + l32 * 32 + 4 * g;
-#pragma unroll
-                for (int a = 0; a < 4; ++a) *reinterpret_cast<f32x4_t*>(out + 8 * a) = f32x4_t{dp[4 * a], dp[4 * a + 1], dp[4 * a + 2], dp[4 * a + 3]};
+            if constexpr (NS == 1) {
+                __syncthreads();
+                issue();
             }
-            cols_product<D>(dv_acc, do_s, 32 * qs, s, l32, g);
-            cols_product<D>(dk_acc, q_s, 32 * qs, dp, l32, g);
         }
-        if constexpr (NS == 1) {
-            __syncthreads();
-            issue();
+        settled();
+    } else {
+        for (int step = 0; step < n_steps; ++step) {
+            put_stat(step);
+            wait_vmcnt<0>();
+            __syncthreads();                  // the step has landed, and the readers of the one before are done
+            if constexpr (NS == 2) issue();
+            const int qt = qt0 + tile * BQ + 32 * qs, head = kvh * p.n_rep + hs * hpw + rep;
+            if (++tile == n_tiles) { tile = 0; ++rep; }
+            if (qt < wmax && qt + 32 > wmin) {
+                const char* q_s = smem + (step % NS) * 2 * TILE;
+                const char* do_s = q_s + TILE;
+                f32x16_t s = rows_product<D>(q_s, 32 * qs + l32, g, kf);         // rows = queries, column = this lane's key
+                f32x16_t dp = rows_product<D>(do_s, 32 * qs + l32, g, vf);
+                const bool edge = __any(qt < qlo || qt + 32 > qhi);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&lse_lds[step & 1][32 * qs + 8 * a + 4 * g]);
+                    const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&delta_lds[step & 1][32 * qs + 8 * a + 4 * g]);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const int r = 4 * a + c;
+                        float pv = fast_exp2(s[r] * c2 - l4[c]);
+                        if (edge) {
+                            const int q = qt + 8 * a + 4 * g + c;
+                            if (q < qlo || q >= qhi) pv = 0.f;
+                        }
+                        s[r] = pv;
+                        dp[r] = pv * (dp[r] - d4[c]);
+                    }
+                }
+                if constexpr (KEEP) {
+                    float* out = fp.ds + ds.tile(head - first_kv * p.n_rep, qt, kb * BK + kgrp * 32) + l32 * 32 + 4 * g;
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) *reinterpret_cast<f32x4_t*>(out + 8 * a) = f32x4_t{dp[4 * a], dp[4 * a + 1], dp[4 * a + 2], dp[4 * a + 3]};
+                }
+                cols_product<D>(dv_acc, do_s, 32 * qs, s, l32, g);
+                cols_product<D>(dk_acc, q_s, 32 * qs, dp, l32, g);
+            }
+            if constexpr (NS == 1) {
+                __syncthreads();
+                issue();
+            }
         }
     }
     const bool live = key < p.total_k;

@@ -663,6 +663,28 @@ def test_attention_float32_wide_tilings(b, s, nq, nkv, d, causal, cuts):
         check(f"attn.f32.wide.{name}", got, r, literal=True, max_abs_tol=1e-4, mean_rel_tol=1e-5)
 
 
+@pytest.mark.parametrize("b,s,nq,nkv,d,causal,cuts", [
+    (1, 192, 256, 256, 128, True, ()),            # whole steps only: every one after the first is requested between products
+    (1, 193, 256, 256, 96, False, ()),            # the last step is one query
+    (1, 130, 512, 256, 128, True, (64, 65)),      # steps that some wavefronts have nothing to do in, two query heads per group
+    (1, 256, 2, 1, 128, True, ()),                # one key group per workgroup, one stage
+    (1, 129, 4, 2, 128, False, (128,)),
+])
+def test_attention_float32_backward_steps(b, s, nq, nkv, d, causal, cuts):
+    """dK / dV with loads and softmax between the products: steps that are whole, ragged, or not for every wavefront.  Sums of as many terms as in the
+    parity test above, hence its gates."""
+    print(f"case attn f32 steps b={b} s={s} nq={nq} nkv={nkv} d={d} causal={causal} cuts={cuts}", flush=True)
+    q, k, v, do = U.make_qkv(b, s, nq, nkv, d, seed=11 + s + d, dtype=torch.float32)
+    cu = U.make_cu(b, s, cuts)
+    scale = 1.0 / math.sqrt(d)
+    ref = U.oracle_attention(q, k, v, cu, b, s, causal, scale, torch.float32, do)
+    qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    ops.attention(qg, kg, vg, cu.to(DEV), None, causal, scale).backward(do.to(DEV))
+    torch.cuda.synchronize()
+    for name, got, r in (("dq", qg.grad, ref[1]), ("dk", kg.grad, ref[2]), ("dv", vg.grad, ref[3])):
+        check(f"attn.f32.steps.{name}", got, r, literal=True, max_abs_tol=1e-4, mean_rel_tol=1e-5)
+
+
 def test_attention_float32_cross_length_and_rotary():
     """fp32: keys longer than queries (causal diagonal aligned to the end of the keys), and the rotary embedding applied
     by the stand-alone kernel in front of the fp32 core when ops.attention is handed fp32 tables."""
