@@ -5,6 +5,9 @@
 // from HBM exactly once.  Rows handled by a wavefront need no block barrier, so the memory pipeline
 // stays full.  The weight gradient is accumulated in registers across a block's rows, combined in
 // LDS in a fixed order, written as one fp32 partial row per block and reduced by a second kernel.
+// Rows narrower than 256 vectors, backward, in a row of launches with the reduction, us, one row at a time and LDS summed in turn / as it is, bf16:
+//   RMSNorm    4084 x 1024 11.1 / 9.9    8192 x 1024 15.7 / 14.1    700 x 2040 10.7 / 8.9    2048 x 64 6.2 / 5.0
+//   LayerNorm  4084 x 1024 17.0 / 12.3   8192 x 1024 22.1 / 17.3    700 x 2040 21.4 / 10.9   2048 x 64 13.2 / 5.8
 #include "common.h"
 
 namespace {
@@ -24,6 +27,33 @@ template <int TPR> __device__ __forceinline__ float row_sum(float v, float* lds)
         if ((threadIdx.x & 63) == 0) lds[wave] = v;
         __syncthreads();
         return lds[0] + lds[1] + lds[2] + lds[3];
+    }
+}
+
+// Sums the accumulators that the RPB row groups of a block hold for the columns, in the order of the groups, into one row of partial sums.  Each group has a
+// row of `lds` to itself (RPB * hidden floats; with one group none is needed), written and read as 128-bit vectors: one row that the groups add to in turn costs a
+// barrier each and eight lanes meet on a bank.
+template <int TPR, int CH, int V>
+__device__ __forceinline__ void store_partial(const float (&acc)[CH][V], float* lds, float* out, int hidden) {
+    constexpr int RPB = kBlock / TPR;
+    const int tr = threadIdx.x % TPR, rg = threadIdx.x / TPR, vecs = hidden / V;
+    float* own = RPB == 1 ? out : lds + rg * hidden;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int v = c * TPR + tr;
+        if (v < vecs) {
+#pragma unroll
+            for (int i = 0; i < V; i += 4) *reinterpret_cast<f32x4_t*>(own + v * V + i) = f32x4_t{acc[c][i], acc[c][i + 1], acc[c][i + 2], acc[c][i + 3]};
+        }
+    }
+    if constexpr (RPB > 1) {
+        __syncthreads();
+        for (int i = 4 * threadIdx.x; i < hidden; i += 4 * kBlock) {
+            f32x4_t sum = *reinterpret_cast<const f32x4_t*>(lds + i);
+#pragma unroll
+            for (int g = 1; g < RPB; ++g) sum += *reinterpret_cast<const f32x4_t*>(lds + g * hidden + i);
+            *reinterpret_cast<f32x4_t*>(out + i) = sum;
+        }
     }
 }
 
@@ -98,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
                                                               int hidden, float eps) {
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kBlock / TPR;
-    extern __shared__ float dw_lds[];  // [hidden]
+    extern __shared__ __attribute__((aligned(16))) float dw_lds[];  // [RPB][hidden], nothing with one row group
     __shared__ float lds[4];
     const int tr = threadIdx.x % TPR;
     const int rg = threadIdx.x / TPR;
@@ -120,19 +150,31 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
     const int64_t row_step = (int64_t)gridDim.x * RPB;
     // every thread of the block runs the same number of iterations (barriers inside row_sum for TPR=256)
     const int64_t iters = (n_rows + row_step - 1) / row_step;
-    for (int64_t it = 0; it < iters; ++it) {
+    // the next row is requested before this one is reduced, where the registers hold both
+    constexpr bool kAhead = CH <= 4;
+    constexpr int NX = kAhead ? CH : 1;
+    uint4 xraw[CH], graw[CH], rraw[CH], xnext[NX], gnext[NX], rnext[NX];
+    auto fetch = [&](int64_t it, uint4 (&xv)[CH], uint4 (&gv)[CH], uint4 (&rv)[CH]) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
         const bool row_ok = row < n_rows;
-        const uint4* xr = reinterpret_cast<const uint4*>(x + (row_ok ? row : 0) * hidden);
-        const uint4* gr = reinterpret_cast<const uint4*>(dy + (row_ok ? row : 0) * hidden);
-        uint4 xraw[CH], graw[CH], rraw[CH];
+        const int64_t at = (row_ok ? row : 0) * hidden;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const int v = c * TPR + tr;
             const bool ok = row_ok && v < vecs;
-            xraw[c] = ok ? xr[v] : make_uint4(0, 0, 0, 0);
-            graw[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
-            rraw[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
+            xv[c] = ok ? reinterpret_cast<const uint4*>(x + at)[v] : make_uint4(0, 0, 0, 0);
+            gv[c] = ok ? reinterpret_cast<const uint4*>(dy + at)[v] : make_uint4(0, 0, 0, 0);
+            rv[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + at)[v] : make_uint4(0, 0, 0, 0);
+        }
+    };
+    if (kAhead && iters > 0) fetch(0, xraw, graw, rraw);
+    for (int64_t it = 0; it < iters; ++it) {
+        const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
+        const bool row_ok = row < n_rows;
+        if constexpr (kAhead) {
+            if (it + 1 < iters) fetch(it + 1, xnext, gnext, rnext);
+        } else {
+            fetch(it, xraw, graw, rraw);
         }
         float ss = 0.f, dot = 0.f;
 #pragma unroll
@@ -169,26 +211,13 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
                 }
             }
         }
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) { xraw[c] = xnext[c]; graw[c] = gnext[c]; rraw[c] = rnext[c]; }
+        }
     }
 
-    // combine the row groups of this block in a fixed order, then emit one partial row
-    for (int i = threadIdx.x; i < hidden; i += kBlock) dw_lds[i] = 0.f;
-    __syncthreads();
-    for (int g = 0; g < RPB; ++g) {
-        if (rg == g) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int v = c * TPR + tr;
-                if (v < vecs) {
-#pragma unroll
-                    for (int i = 0; i < V; ++i) dw_lds[v * V + i] += acc[c][i];
-                }
-            }
-        }
-        __syncthreads();
-    }
-    float* out = dw_partial + (int64_t)blockIdx.x * hidden;
-    for (int i = threadIdx.x; i < hidden; i += kBlock) out[i] = dw_lds[i];
+    store_partial<TPR, CH, V>(acc, dw_lds, dw_partial + (int64_t)blockIdx.x * hidden, hidden);
 }
 
 // Backward for wide rows: 1024 threads per block, TPR (256 or 512) threads per row, so 4 or 2 rows are in
@@ -209,7 +238,7 @@ __global__ __launch_bounds__(kRmsWideBlock) void rmsnorm_bwd_wide_kernel(const T
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kRmsWideBlock / TPR;
     constexpr int WPR = TPR / 64;      // wavefronts per row
-    extern __shared__ float dw_lds[];  // [hidden] dweight combine buffer, then [hidden] fp32 copy of the weight
+    extern __shared__ __attribute__((aligned(16))) float dw_lds[];  // [hidden] dweight combine buffer, then [hidden] fp32 copy of the weight
     __shared__ float2 part[2][16];     // [parity][wavefront]
     float* w_lds = dw_lds + hidden;
     const int tr = threadIdx.x % TPR;
@@ -528,7 +557,8 @@ int launch_bwd(const void* x, const void* w, const void* dy, const void* dres, v
     const bool launched = dispatch_plan(plan, [&](auto tag) {
         constexpr int TPR = decltype(tag)::TPR;
         constexpr int CH = decltype(tag)::CH;
-        rmsnorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), hidden * sizeof(float), st>>>(
+        constexpr int RPB = kBlock / TPR;
+        rmsnorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), RPB == 1 ? 0 : RPB * hidden * sizeof(float), st>>>(
             (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
     });
     if (!launched) return mi_fail(MI_E_SHAPE, "rmsnorm: no kernel for hidden=%lld", (long long)hidden);
@@ -620,7 +650,7 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
                                                                 float eps) {
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kBlock / TPR;
-    extern __shared__ float comb_lds[];  // [2][hidden]
+    extern __shared__ __attribute__((aligned(16))) float comb_lds[];  // [2][RPB][hidden], nothing with one row group
     __shared__ float lds[4];
     const int tr = threadIdx.x % TPR;
     const int rg = threadIdx.x / TPR;
@@ -636,22 +666,37 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
 
     const int64_t row_step = (int64_t)gridDim.x * RPB;
     const int64_t iters = (n_rows + row_step - 1) / row_step;   // same count in every thread (barriers in row_sum)
-    for (int64_t it = 0; it < iters; ++it) {
+    // the next row is requested before this one is reduced, where the registers hold both
+    constexpr bool kAhead = CH <= 4;
+    constexpr int NX = kAhead ? CH : 1;
+    uint4 xraw[CH], graw[CH], rraw[CH], xnext[NX], gnext[NX], rnext[NX];
+    auto fetch = [&](int64_t it, uint4 (&xv)[CH], uint4 (&gv)[CH], uint4 (&rv)[CH]) {
         const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
         const bool row_ok = row < n_rows;
-        const uint4* xr = reinterpret_cast<const uint4*>(x + (row_ok ? row : 0) * hidden);
-        const uint4* gr = reinterpret_cast<const uint4*>(dy + (row_ok ? row : 0) * hidden);
-        float xf[CH][V], gw[CH][V];
-        uint4 graw[CH], rraw[CH];
-        float sum = 0.f;
+        const int64_t at = (row_ok ? row : 0) * hidden;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const int v = c * TPR + tr;
             const bool ok = row_ok && v < vecs;
-            const uint4 xraw = ok ? xr[v] : make_uint4(0, 0, 0, 0);
-            graw[c] = ok ? gr[v] : make_uint4(0, 0, 0, 0);
-            rraw[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + row * hidden)[v] : make_uint4(0, 0, 0, 0);
-            Elem<T>::unpack(xraw, xf[c]);
+            xv[c] = ok ? reinterpret_cast<const uint4*>(x + at)[v] : make_uint4(0, 0, 0, 0);
+            gv[c] = ok ? reinterpret_cast<const uint4*>(dy + at)[v] : make_uint4(0, 0, 0, 0);
+            rv[c] = ok && dres != nullptr ? reinterpret_cast<const uint4*>(dres + at)[v] : make_uint4(0, 0, 0, 0);
+        }
+    };
+    if (kAhead && iters > 0) fetch(0, xraw, graw, rraw);
+    for (int64_t it = 0; it < iters; ++it) {
+        const int64_t row = it * row_step + (int64_t)blockIdx.x * RPB + rg;
+        const bool row_ok = row < n_rows;
+        if constexpr (kAhead) {
+            if (it + 1 < iters) fetch(it + 1, xnext, gnext, rnext);
+        } else {
+            fetch(it, xraw, graw, rraw);
+        }
+        float xf[CH][V], gw[CH][V];
+        float sum = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            Elem<T>::unpack(xraw[c], xf[c]);
 #pragma unroll
             for (int i = 0; i < V; ++i) sum += xf[c][i];
         }
@@ -700,30 +745,15 @@ __global__ __launch_bounds__(kBlock) void layernorm_bwd_kernel(const T* __restri
                 }
             }
         }
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) { xraw[c] = xnext[c]; graw[c] = gnext[c]; rraw[c] = rnext[c]; }
+        }
     }
 
-    // combine the row groups of this block in a fixed order, then emit one partial row each for dw and db
-    for (int i = threadIdx.x; i < 2 * hidden; i += kBlock) comb_lds[i] = 0.f;
-    __syncthreads();
-    for (int g = 0; g < RPB; ++g) {
-        if (rg == g) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int v = c * TPR + tr;
-                if (v < vecs) {
-#pragma unroll
-                    for (int i = 0; i < V; ++i) {
-                        comb_lds[v * V + i] += acc_w[c][i];
-                        comb_lds[hidden + v * V + i] += acc_b[c][i];
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    float* out_w = partial + (int64_t)blockIdx.x * hidden;
-    float* out_b = partial + ((int64_t)gridDim.x + blockIdx.x) * hidden;
-    for (int i = threadIdx.x; i < hidden; i += kBlock) { out_w[i] = comb_lds[i]; out_b[i] = comb_lds[hidden + i]; }
+    // one partial row each for dw and db
+    store_partial<TPR, CH, V>(acc_w, comb_lds, partial + (int64_t)blockIdx.x * hidden, hidden);
+    store_partial<TPR, CH, V>(acc_b, comb_lds + RPB * hidden, partial + ((int64_t)gridDim.x + blockIdx.x) * hidden, hidden);
 }
 
 // Backward for wide rows, laid out like rmsnorm_bwd_wide_kernel: 512 threads per block, TPR (256 or 512)
@@ -738,7 +768,7 @@ __global__ __launch_bounds__(kWideBlock, 4) void layernorm_bwd_wide_kernel(const
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kWideBlock / TPR;
     constexpr int WPR = TPR / 64;
-    extern __shared__ float comb_lds[];   // [hidden] dweight, [hidden] dbias, then [hidden] fp32 copy of the weight
+    extern __shared__ __attribute__((aligned(16))) float comb_lds[];   // [hidden] dweight, [hidden] dbias, then [hidden] fp32 copy of the weight
     __shared__ float part_mean[2][8];
     __shared__ float part_sq[2][8], part_s1[2][8], part_s2[2][8];
     float* w_lds = comb_lds + 2 * hidden;
@@ -887,7 +917,7 @@ __global__ __launch_bounds__(kRmsWideBlock) void layernorm_bwd_stats_kernel(cons
     constexpr int V = Elem<T>::kVec;
     constexpr int RPB = kRmsWideBlock / TPR;
     constexpr int WPR = TPR / 64;
-    extern __shared__ float comb_lds[];   // [hidden] dweight, [hidden] dbias, then [hidden] fp32 copy of the weight
+    extern __shared__ __attribute__((aligned(16))) float comb_lds[];   // [hidden] dweight, [hidden] dbias, then [hidden] fp32 copy of the weight
     __shared__ float2 part[2][16];        // [parity][wavefront]: sum g*w, sum g*w*xhat
     float* w_lds = comb_lds + 2 * hidden;
     const int tr = threadIdx.x % TPR;
@@ -1089,7 +1119,8 @@ int launch_ln_bwd(const void* x, const void* w, const void* dy, const void* dres
         launched = dispatch_plan(plan, [&](auto tag) {
             constexpr int TPR = decltype(tag)::TPR;
             constexpr int CH = decltype(tag)::CH;
-            layernorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), 2 * hidden * sizeof(float), st>>>(
+            constexpr int RPB = kBlock / TPR;
+            layernorm_bwd_kernel<T, TPR, CH><<<dim3(blocks), dim3(kBlock), RPB == 1 ? 0 : 2 * RPB * hidden * sizeof(float), st>>>(
                 (const T*)x, (const T*)w, (const T*)dy, (const T*)dres, (T*)dx, (float*)ws, n_rows, (int)hidden, eps);
         });
     }

@@ -322,3 +322,31 @@ def test_empty_tensors_pass_through_every_elementwise_op():
     q = torch.zeros(0, 4, 64, dtype=torch.bfloat16, device=DEV)
     tables = torch.zeros(16, 64, dtype=torch.bfloat16, device=DEV)
     assert ops.rotary_embedding(q, tables, tables, torch.zeros(0, dtype=torch.int64, device=DEV)).shape == q.shape
+
+
+@pytest.mark.parametrize("layer_norm", [False, True])
+@pytest.mark.parametrize("rows,hidden,dtype", [
+    (4099, 1000, torch.bfloat16), (2060, 2040, torch.float16), (2049, 8, torch.bfloat16), (1, 1024, torch.bfloat16), (9000, 128, torch.float16),
+    (2050, 1016, torch.float32), (2050, 12, torch.float32),
+])
+def test_norm_backward_of_narrow_rows(rows, hidden, dtype, layer_norm):
+    """Row groups that walk several rows (more than 2048 of 64 lanes, 8192 of 16) or have none, the last row a group's second or third, rows that are not
+    whole vectors of the lanes; with the gradient that goes past the norm.  Against float64: dx is rounded twice, the weight gradients once, each
+    by at most half a unit in the last place (relative 2^-8 with the 8 bits of bf16, 2^-11 with the 11 of fp16); float32 sums of up to 9000 terms stay below 1e-5."""
+    print(f"case narrow norm backward rows={rows} hidden={hidden} dtype={dtype} layer_norm={layer_norm}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows + hidden)
+    x, dy, dsum = (torch.randn(rows, hidden, generator=g, device=DEV).to(dtype) for _ in range(3))
+    w, b = (torch.randn(hidden, generator=g, device=DEV).to(dtype) for _ in range(2))
+    leaves = [t.clone().requires_grad_() for t in ((x, w, b) if layer_norm else (x, w))]
+    s, y = ops.add_norm(leaves[0], None, leaves[1], leaves[2] if layer_norm else None, 1e-5, layer_norm)
+    torch.autograd.backward([s, y], [dsum, dy])
+    exact = [t.double().requires_grad_() for t in ((x, w, b) if layer_norm else (x, w))]
+    if layer_norm:
+        ye = torch.nn.functional.layer_norm(exact[0], (hidden,), exact[1], exact[2], 1e-5)
+    else:
+        ye = exact[0] * torch.rsqrt(exact[0].square().mean(-1, keepdim=True) + 1e-5) * exact[1]
+    torch.autograd.backward([exact[0] * 1.0, ye], [dsum.double(), dy.double()])
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 5e-6}[dtype]
+    for name, got, want, bound in zip(("dx", "dw", "db"), leaves, exact, (2 * unit, unit, unit)):
+        error = ((got.grad.double() - want.grad).norm() / want.grad.norm()).item()
+        assert error <= bound, (name, error, bound)
