@@ -72,16 +72,31 @@ class _Linear(torch.nn.Module):
         return ops.linear(x, self.weight, self.bias, residual, not self.training)
 
 
-def _unhooked(m: torch.nn.Module) -> bool:
-    """Whether calling the module runs its class's forward and nothing else: no hooks on it or on all modules, no forward of the
+def _unhooked(*modules: torch.nn.Module) -> bool:
+    """Whether calling the modules runs their class's forward and nothing else: no hooks on them or on all modules, no forward of the
     instance's own (as wrapper libraries set it), not compiled."""
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__ or
-                m._compiled_call_impl is not None or torch.nn.modules.module._has_any_global_hook())
+    if torch.nn.modules.module._has_any_global_hook():
+        return False
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__ or \
+                m._compiled_call_impl is not None:
+            return False
+    return True
 
 
 def _direct(*modules: torch.nn.Module) -> bool:
     """Whether calling the modules comes to using their weights: plain projections that nobody replaced or hooked."""
-    return all(type(m) is _Linear and _unhooked(m) for m in modules)
+    for m in modules:
+        if type(m) is not _Linear:
+            return False
+    return _unhooked(*modules)
+
+
+def _weights(modules) -> Tuple[list, list]:
+    """Weights and biases (RMSNorm: none) of this package's projections and norms."""
+    kept = [(m._parameters, m) for m in modules]
+    return [p["weight"] if "weight" in p else m.weight for p, m in kept], \
+        [None if type(m) is RMSNorm else p["bias"] if "bias" in p else m.bias for p, m in kept]
 
 
 def idle_dropout(m: torch.nn.Module) -> bool:
@@ -725,18 +740,24 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
     """The output of a layer whose norms and MLP may be passed by (`fuses_residual`) in one native call of the operations its modules would
     issue; with a cache: of a prefill.  None, with nothing done, where a module below is not the package's own as it is or the operands are not what
     the kernels take: the modules then compute or refuse it."""
-    att, mlp, norm1, norm2 = layer.self_attention, layer.mlp, layer.input_layernorm, layer.post_attention_layernorm
-    sdpa, rot, dtype, training = att.scaled_dot_product_attention, att.rotary_embedding, att.dtype, layer.training
-    if not (x.is_cuda and x.dim() == 3 and x.dtype == dtype and x.numel() > 0 and not torch.is_autocast_enabled() and type(att) is ParallelSelfAttention and
-            _unhooked(att) and fuses_residual(mlp) and idle_dropout(layer.dropout_attention) and idle_dropout(layer.dropout_mlp) and
-            not att.key_query_norm and type(sdpa) is ScaledDotProductAttention and not (training and sdpa.dropout_p > 0.0) and
+    # Modules and parameters come from their dictionaries: as some 40 attributes they took half of the time spent here
+    parts = layer._modules
+    att, mlp, norm1, norm2 = parts["self_attention"], parts["mlp"], parts["input_layernorm"], parts["post_attention_layernorm"]
+    if not (type(att) is ParallelSelfAttention and type(mlp) in (ParallelSwiGLUMLP, ParallelMLP)):
+        return None
+    own = att._modules
+    sdpa, rot, dtype, training = own["scaled_dot_product_attention"], att.rotary_embedding, att.dtype, layer.training
+    if not (x.is_cuda and x.dim() == 3 and x.dtype == dtype and x.numel() > 0 and not torch.is_autocast_enabled() and _unhooked(att, mlp) and
+            idle_dropout(parts["dropout_attention"]) and idle_dropout(parts["dropout_mlp"]) and not att.key_query_norm and
+            type(sdpa) is ScaledDotProductAttention and not (training and sdpa.dropout_p > 0.0) and
             (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex)) and
             _nothing_overridden(att, sdpa, norm1, norm2, *(() if rot is None else (rot,)))):
         return None
     swiglu = type(mlp) is ParallelSwiGLUMLP
-    rest = (att.dense, mlp.dense_in, mlp.siglu_weight, mlp.dense_out) if swiglu else (att.dense, mlp.dense_in, mlp.dense_out)
-    into = (att.query_key_value,) if att.qkv_in_one else (att.query, att.key, att.value)
-    if not (_direct(*into, *rest) and all(m.training == training for m in (att, sdpa, mlp, *into, *rest))):
+    inner = mlp._modules
+    rest = [own["dense"], inner["dense_in"], inner["siglu_weight"], inner["dense_out"]] if swiglu else [own["dense"], inner["dense_in"], inner["dense_out"]]
+    into = [own["query_key_value"]] if att.qkv_in_one else [own["query"], own["key"], own["value"]]
+    if not _direct(*into, *rest) or [True for m in (att, sdpa, mlp, *into, *rest) if m.training != training]:
         return None
     b, s, hidden = x.shape
     pos = None if position_ids is None else position_ids.reshape(-1).contiguous()
@@ -761,11 +782,12 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
         w, bias = att._fused_qkv()
         qkv_w, qkv_b = [w], [bias]
     else:
-        qkv_w, qkv_b = [m.weight for m in into], [m.bias for m in into]
-    norms = [p for n in (norm1, norm2) for p in (n.weight, n.bias if type(n) is LayerNorm else None)]
-    rest_w, rest_b = [m.weight for m in rest], [m.bias for m in rest]
+        qkv_w, qkv_b = _weights(into)
+    norm_w, norm_b = _weights((norm1, norm2))
+    norms = [norm_w[0], norm_b[0], norm_w[1], norm_b[1]]
+    rest_w, rest_b = _weights(rest)
     if ops._taken_over((x, *norms, *qkv_w, *qkv_b, *rest_w, *rest_b)) or any(p is not None and (p.dtype != dtype or not p.is_cuda) for p in (*norms, *qkv_w, *rest_w)) or \
-            norm1.weight.shape[0] != hidden or norm2.weight.shape[0] != hidden:
+            norm_w[0].shape[0] != hidden or norm_w[1].shape[0] != hidden:
         return None
     if use_cache:
         assert att._rows_are_single_documents(cu, b, s), "sequence packing is not supported with cache"

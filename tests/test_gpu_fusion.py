@@ -599,3 +599,35 @@ def test_prefill_into_a_cache_of_another_kind(case):
             results.append([run(), cache.k, cache.v, cache.ctx_len])
         assert att.cache[0] is cache and cache.length == 30
     assert all(torch.equal(a, b) for a, b in zip(*results)) and results[0][1].any()
+
+
+# on the line up to which a layer is one autograd node, above it, and with rows that end inside a tile
+@pytest.mark.parametrize("default,dtype,options,b,s", [
+    (True, "float32", {}, 2, 93), (True, "bfloat16", dict(relative_position_embedding_type="none"), 1, 1), (False, "bfloat16", {}, 8, 256),
+    (False, "bfloat16", {}, 9, 228), (False, "float16", dict(rotary_percentage=0.5), 3, 67),
+])
+def test_gradients_of_a_layer_that_is_one_node(default, dtype, options, b, s):
+    """Any choice of gradients, a kept graph and a graph of the gradients: to the bit what the nodes of the modules give."""
+    layer = _layer(dtype, default, **options)
+    x = torch.randn(b, s, 256, generator=torch.Generator().manual_seed(5)).to(getattr(torch, dtype)).to(DEV).requires_grad_()
+    io, parameters = _io(x), dict(layer.named_parameters())
+    first = "self_attention.query_key_value.weight" if default else "self_attention.key.weight"
+
+    def gradients(forward, inputs, **how):
+        y = forward()
+        return [torch.autograd.grad(y, inputs, torch.cos(y.detach()), **how) for _ in range(2 if how else 1)]
+
+    def native():
+        y = layer(io).activations
+        assert y.grad_fn.name().endswith("::Layer>") == (b * s * 256 <= 2 ** 19)
+        return y
+    for names in (["x"], ["input_layernorm.weight"], [first], ["self_attention.dense.weight", "x"], ["post_attention_layernorm.weight"],
+                  ["mlp.dense_in.weight"], ["mlp.dense_out.weight"], ["x", *parameters]):
+        inputs = [x if n == "x" else parameters[n] for n in names]
+        for how in ({}, dict(retain_graph=True), dict(create_graph=True)):
+            for got, want in zip(gradients(native, inputs, **how), gradients(lambda: _watched(layer, io), inputs, **how)):
+                assert all(torch.equal(p, q) for p, q in zip(got, want)), (names, how)
+    for n, p in parameters.items():                        # frozen: everything but one
+        p.requires_grad_(n == first)
+    io.activations = x.detach()
+    assert all(torch.equal(p, q) for p, q in zip(gradients(native, [parameters[first]])[0], gradients(lambda: _watched(layer, io), [parameters[first]])[0]))
