@@ -12,8 +12,12 @@
 //
 // What is left is latency: descriptors, then weights and rows, then the norm's barrier, then the sums.  In a decode step of a 4-layer model
 // of hidden 1024 (3 sequences) a product of the tiled kernel took 9.2 us, with 3 us for each norm and activation beside
-// it; a launch here 5.7 - 6.1 with those included (4.1 when the weights are cached: 3 x 1024 x 1024).  Wide products run at the
-// rate of the weights: 16 x 4096 -> 128256 191 us, 5.5 TB/s.
+// it.  Wide products run at the rate of the weights: 16 x 4096 -> 128256 191 us, 5.5 TB/s.
+//
+// Few features leave compute units without a workgroup, and the rest wait for what each of them fetches (1024 features: 64 workgroups, of 16 x k
+// weights).  So up to 8 (4) rows may be folded: a workgroup owns 8 (4) features, and a wavefront takes two (four) slices of the contraction at
+// once.  Of an operand's 16 rows the first 8 (4) are those of one slice, the next those of the next; of the 16 x 16 results the parts on the
+// diagonal count.  The slices and the order that their sums meet in are what they are without, so the results are the same to the bit.
 #include "common.h"
 
 namespace {
@@ -52,14 +56,18 @@ template <> struct RowsMfma<_Float16> {
 };
 
 // TILES: blocks of 16 weight rows per workgroup (2 with GLU: the same 16 rows of both matrices)
-template <typename T, int NW, int TILES, bool NORM, bool GLU>
+// FOLD: slices of the contraction per wavefront; up to 16 / FOLD rows, and 16 / FOLD features of a block
+template <typename T, int NW, int TILES, bool NORM, bool GLU, int FOLD>
 __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
     static_assert(!GLU || TILES == 2, "two matrices");
+    static_assert(FOLD == 1 || GLU || TILES == 1, "a part of a block");
     using F = typename RowsMfma<T>::frag_t;
     constexpr int CH = TILES == 2 ? 4 : 8;                 // products ahead
-    constexpr int FEATURES = GLU ? 16 : 16 * TILES;
-    __shared__ __attribute__((aligned(16))) float red[TILES][NW][kMaxRows][kRedStride];
-    __shared__ float squares[NW][kMaxRows];
+    constexpr int SLICES = FOLD * NW, ROWS = kMaxRows / FOLD;     // rows of a slice
+    constexpr int FEATURES = (GLU ? 16 : 16 * TILES) / FOLD;
+    constexpr int RED = FOLD == 1 ? kRedStride : 16 / FOLD + 4;
+    __shared__ __attribute__((aligned(16))) float red[TILES][SLICES][ROWS][RED];
+    __shared__ float squares[SLICES][ROWS];
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, G = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -83,27 +91,30 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
     }
     const int n0 = ((int)blockIdx.x - mx.first_tile) * FEATURES, n = mx.n;
 
-    // this wavefront's products: an even number, so that it covers whole 128-byte lines
+    // this slice's products: an even number, so that it covers whole 128-byte lines
     const int steps = k / kStep;
-    const int per = ((steps + NW - 1) / NW + 1) & ~1;
-    const int s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
+    const int per = ((steps + SLICES - 1) / SLICES + 1) & ~1;
+    const int part = l16 / ROWS, slice = FOLD * wave + part, row = l16 % ROWS;
+    const int s0 = min(slice * per, steps), s1 = min(s0 + per, steps), mine = s1 - s0;
+    const int count = __builtin_amdgcn_readfirstlane(mine);                // of the first slice: the others have no more
+    const int all = __builtin_amdgcn_readlane(mine, 15);                  // of the last
 
     // rows past the last one and features past n repeat the last: their results are not stored
-    const T* xr = reinterpret_cast<const T*>(x) + (int64_t)min(l16, rows - 1) * ldx + 8 * G;
+    const T* xr = reinterpret_cast<const T*>(x) + (int64_t)min(row, rows - 1) * ldx + 8 * G;
     const T* gr = reinterpret_cast<const T*>(norm_weight) + 8 * G;
     const T* wr[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         const Matrix& m = GLU && t == 1 ? gate : mx;
-        wr[t] = reinterpret_cast<const T*>(m.w) + (int64_t)min(n0 + (GLU ? 0 : 16 * t) + l16, n - 1) * m.ldw + 8 * G;
+        wr[t] = reinterpret_cast<const T*>(m.w) + (int64_t)min(n0 + (GLU ? 0 : 16 * t) + row, n - 1) * m.ldw + 8 * G;
     }
     // Weights, rows and norm weights of CH products.  No request is conditional, so that all of them are in flight together: those
-    // past this wavefront's last product repeat it and are not used.
+    // past this slice's last product repeat it and are not used.
     struct Chunk { u32x4_t w[TILES][CH], x[CH], g[NORM ? CH : 1]; };
-    auto request = [&](Chunk& c, int s) {
+    auto request = [&](Chunk& c, int i) {
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
-            const int64_t at = (int64_t)kStep * min(s + j, s1 - 1);
+            const int64_t at = (int64_t)kStep * min(s0 + i + j, s1 - 1);
             c.x[j] = *reinterpret_cast<const u32x4_t*>(xr + at);
             if constexpr (NORM) c.g[j] = *reinterpret_cast<const u32x4_t*>(gr + at);
 #pragma unroll
@@ -111,14 +122,14 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
         }
     };
     Chunk ca, cb;
-    if (s0 < s1) request(ca, s0);
-    if (s0 + CH < s1) request(cb, s0 + CH);                // in front of the loop, where it waits for nothing
+    if (0 < count) request(ca, 0);
+    if (CH < count) request(cb, CH);                       // in front of the loop, where it waits for nothing
     const bool counts = count_up != nullptr && blockIdx.x == 0;
-    const int32_t count = (counts ? count_up : reinterpret_cast<const int32_t*>(x))[counts ? min(tid, rows - 1) : 0];
+    const int32_t length = (counts ? count_up : reinterpret_cast<const int32_t*>(x))[counts ? min(tid, rows - 1) : 0];
 
     // bias and residual of the results that this thread stores, requested with the weights, clamped like them and without a branch (in its
     // place the first element of x), which would wait for all that is under way
-    constexpr int kOut = (FEATURES * kMaxRows + 64 * NW - 1) / (64 * NW);
+    constexpr int kOut = (FEATURES * ROWS + 64 * NW - 1) / (64 * NW);
     T bias[kOut], add[kOut];
     if constexpr (!GLU) {
 #pragma unroll
@@ -138,27 +149,27 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
         };
-        if (s0 < s1) {
+        if (0 < count) {
 #pragma unroll
             for (int j = 0; j < CH; ++j)
-                if (s0 + j < s1) add_squares(ca.x[j]);
+                if (j < mine) add_squares(ca.x[j]);
         }
 #pragma unroll 8
-        for (int s = s0 + CH; s < s1; ++s) add_squares(*reinterpret_cast<const u32x4_t*>(xr + kStep * s));
+        for (int i = CH; i < mine; ++i) add_squares(*reinterpret_cast<const u32x4_t*>(xr + kStep * (s0 + i)));
         ss += __shfl_xor(ss, 16, MI_WAVE);
         ss += __shfl_xor(ss, 32, MI_WAVE);
-        if (G == 0) squares[wave][l16] = ss;
+        if (G == 0) squares[slice][row] = ss;
         __syncthreads();
         float total = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) total += squares[w][l16];
+        for (int w = 0; w < SLICES; ++w) total += squares[w][row];
         rstd = rsqrtf(total / (float)k + p.eps);
     }
 
     f32x4v acc[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const Chunk& c, int s) {
+    auto multiply = [&](const Chunk& c, int i) {
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             uint4 xv = make_uint4(c.x[j][0], c.x[j][1], c.x[j][2], c.x[j][3]);
@@ -167,29 +178,39 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
                 Elem<T>::unpack(xv, f);
                 Elem<T>::unpack(make_uint4(c.g[j][0], c.g[j][1], c.g[j][2], c.g[j][3]), g);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) f[i] = (f[i] * rstd) * g[i];
+                for (int e = 0; e < 8; ++e) f[e] = (f[e] * rstd) * g[e];
                 xv = Elem<T>::pack(f);
             }
-            if (s + j < s1) {                              // the same for the whole wavefront
+            if (i + j < count) {                           // the same for the whole wavefront
+                u32x4_t w[TILES];
 #pragma unroll
-                for (int t = 0; t < TILES; ++t) acc[t] = RowsMfma<T>::mma(__builtin_bit_cast(F, c.w[t][j]), __builtin_bit_cast(F, xv), acc[t]);
+                for (int t = 0; t < TILES; ++t) w[t] = c.w[t][j];
+                if (FOLD > 1 && i + j >= all && i + j >= mine) {   // nothing more of this slice
+                    xv = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t) w[t] = u32x4_t{0, 0, 0, 0};
+                }
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) acc[t] = RowsMfma<T>::mma(__builtin_bit_cast(F, w[t]), __builtin_bit_cast(F, xv), acc[t]);
             }
         }
     };
-    for (int s = s0; s < s1; s += 2 * CH) {
-        multiply(ca, s);
-        if (s + 2 * CH < s1) request(ca, s + 2 * CH);
-        if (s + CH < s1) {
-            multiply(cb, s + CH);
-            if (s + 3 * CH < s1) request(cb, s + 3 * CH);
+    for (int i = 0; i < count; i += 2 * CH) {
+        multiply(ca, i);
+        if (i + 2 * CH < count) request(ca, i + 2 * CH);
+        if (i + CH < count) {
+            multiply(cb, i + CH);
+            if (i + 3 * CH < count) request(cb, i + 3 * CH);
         }
     }
 
-    // a lane holds four consecutive features of row l16
+    // a lane holds four consecutive features of a row
+    if (FOLD == 1 || G * FOLD / 4 == part) {
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) *reinterpret_cast<f32x4v*>(&red[t][wave][l16][4 * G]) = acc[t];
+        for (int t = 0; t < TILES; ++t) *reinterpret_cast<f32x4v*>(&red[t][slice][row][4 * (G % (4 / FOLD))]) = acc[t];
+    }
     __syncthreads();
-    if (counts && tid < rows) count_up[tid] = count + 1;
+    if (counts && tid < rows) count_up[tid] = length + 1;
 #pragma unroll
     for (int i = 0; i < kOut; ++i) {
         const int idx = tid + i * 64 * NW, m = idx / FEATURES, f = idx % FEATURES;
@@ -197,7 +218,7 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
         const auto total = [&](int t, int c) {
             float s = 0.f;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) s += red[t][w][m][c];
+            for (int w = 0; w < SLICES; ++w) s += red[t][w][m][c];
             return s;
         };
         T* out = reinterpret_cast<T*>(mx.out) + (int64_t)m * mx.ldo + n0 + f;
@@ -214,9 +235,9 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(const RowsParams p) {
     }
 }
 
-template <typename T, int NW, int TILES, bool GLU> void launch_one(const RowsParams& p, int grid, hipStream_t st) {
-    if (p.norm_weight != nullptr) rows_kernel<T, NW, TILES, true, GLU><<<dim3((unsigned)grid), dim3(64 * NW), 0, st>>>(p);
-    else rows_kernel<T, NW, TILES, false, GLU><<<dim3((unsigned)grid), dim3(64 * NW), 0, st>>>(p);
+template <typename T, int NW, int TILES, bool GLU, int FOLD> void launch_one(const RowsParams& p, int grid, hipStream_t st) {
+    if (p.norm_weight != nullptr) rows_kernel<T, NW, TILES, true, GLU, FOLD><<<dim3((unsigned)grid), dim3(64 * NW), 0, st>>>(p);
+    else rows_kernel<T, NW, TILES, false, GLU, FOLD><<<dim3((unsigned)grid), dim3(64 * NW), 0, st>>>(p);
 }
 
 template <typename T> int launch(const mi_rows_args& a, hipStream_t st) {
@@ -231,16 +252,23 @@ template <typename T> int launch(const mi_rows_args& a, hipStream_t st) {
     // Two blocks per workgroup once that leaves four workgroups per compute unit: the rows are read half as often.  Eight wavefronts
     // while there is less than one workgroup of four per SIMD, to have more of the weights in flight.
     const bool wide = !a.glu && blocks16 >= 2048, many = blocks16 >= 1024;
-    const int features = wide ? 32 : 16;
+    // Folded where a compute unit is left with less: 256 workgroups of a quarter or of half a block instead of as many whole ones or fewer, or three halves on
+    // a compute unit instead of two blocks.  us, one / two / four slices, weights from memory: 3 rows, k 1024 -> 1024 4.53 / 3.60 / 3.16, 2816 -> 1024 7.09 / 5.59 /
+    // 4.44, 4096 -> 1024 with norm and glu 14.9 / 11.2 / 9.1; 1024 -> 1536 4.77 / 3.90 / 4.20; 4096 -> 6144 15.3 / 13.6 / 14.6 (8 rows 17.2 / 16.3); elsewhere
+    // the rows are only read more often: 1024 -> 2816 4.87 / 5.23 / 4.96, 4096 -> 4096 9.00 / 10.0 / 10.7, 8 rows, 4096 -> 10240 25.5 / 27.2.
+    const int fold = a.rows <= 4 && blocks16 <= 64 ? 4 : a.rows <= 8 && (blocks16 <= 128 || (blocks16 > 256 && blocks16 <= 384)) ? 2 : 1;
+    const int features = (wide ? 32 : 16) / fold;
     int64_t grid = 0;
     for (int i = 0; i < (a.glu ? 1 : a.n_weights); ++i) {
         p.m[i].first_tile = (int)grid;
         grid += (a.n[i] + features - 1) / features;
     }
     if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "rows: too many features");
-    if (a.glu) many ? launch_one<T, 4, 2, true>(p, (int)grid, st) : launch_one<T, 8, 2, true>(p, (int)grid, st);
-    else if (wide) launch_one<T, 4, 2, false>(p, (int)grid, st);
-    else many ? launch_one<T, 4, 1, false>(p, (int)grid, st) : launch_one<T, 8, 1, false>(p, (int)grid, st);
+    if (fold == 4) a.glu ? launch_one<T, 2, 2, true, 4>(p, (int)grid, st) : launch_one<T, 2, 1, false, 4>(p, (int)grid, st);
+    else if (fold == 2) a.glu ? launch_one<T, 4, 2, true, 2>(p, (int)grid, st) : launch_one<T, 4, 1, false, 2>(p, (int)grid, st);
+    else if (a.glu) many ? launch_one<T, 4, 2, true, 1>(p, (int)grid, st) : launch_one<T, 8, 2, true, 1>(p, (int)grid, st);
+    else if (wide) launch_one<T, 4, 2, false, 1>(p, (int)grid, st);
+    else many ? launch_one<T, 4, 1, false, 1>(p, (int)grid, st) : launch_one<T, 8, 1, false, 1>(p, (int)grid, st);
     return mi_check_launch("rows");
 }
 

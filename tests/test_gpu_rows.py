@@ -78,6 +78,34 @@ def test_few_rows_with_norm(rows, k, n, glu, dtype):
 
 
 # each side of the lines between the norm inside the product and a launch of its own: (features, k)
+# both sides of the lines between whole, half and quarter blocks (64, 128, 256 and 384 of 16 features); slices that are shorter than others or empty
+@pytest.mark.parametrize("rows,k,n,glu", [(1, 32, 5, False), (4, 2816, 1024, True), (4, 544, 1025, False), (5, 544, 1024, False), (8, 1056, 2048, True),
+                                          (8, 96, 2049, False), (3, 64, 4097, False), (8, 2080, 6144, True), (2, 352, 6145, False)])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_folded_rows_equal_whole_blocks(rows, k, n, glu, norm, dtype):
+    """More than 8 rows are not folded, and a row's results do not depend on the others: the same to the bit, infinite weights included."""
+    x, g = _rand((16, k), dtype, 3), (1.0 + _rand((k,), torch.float32, 4, 0.1)).to(dtype)
+    ws = [_rand((n, k), dtype, 5 + i, k ** -0.5) for i in range(2)]
+    ws[0][n // 2, k - 1] = float("inf")
+    bias, add = _rand((n,), dtype, 7), _rand((16, n), dtype, 8)
+
+    def product(count):
+        out = torch.full((count, n), 3.0, dtype=dtype, device=DEV)
+        a = _lib.MiRowsArgs()
+        a.x, a.norm_weight, a.ldx, a.k, a.rows, a.eps, a.glu = x.data_ptr(), g.data_ptr() if norm else None, k, k, count, 1e-5, int(glu)
+        a.n_weights, a.dtype, a.stream = 1 + int(glu), _lib.dtype_code(dtype), _lib.stream_ptr()
+        for i in range(1 + int(glu)):
+            a.w[i], a.n[i], a.ldw[i], a.out[i], a.ldo[i] = ws[i].data_ptr(), n, k, out.data_ptr(), n
+        if not glu:
+            a.bias[0], a.add[0], a.ldadd[0] = bias.data_ptr(), add.data_ptr(), n
+        _lib.check(_lib.load().mi_rows_product(ctypes.byref(a)), "mi_rows_product")
+        return out
+    got, want = product(rows), product(16)[:rows]
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+    assert int((~want.isfinite()).sum()) <= rows
+
+
 @pytest.mark.parametrize("n,k,inside", [(4096, 2048, True), (4097, 2048, False), (8192, 1024, True), (8200, 1024, False), (16, 2080, False),
                                         (1536, 4096, False), (1000, 288, True)])
 def test_norm_in_front_of_a_product(n, k, inside):
