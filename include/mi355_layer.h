@@ -218,6 +218,10 @@ int mi_cross_entropy_padded(void* logits, const int64_t* targets, const float* r
                             int64_t n_rows, int64_t vocab, int64_t row_stride, int dtype, void* stream);
 /* index[r] = first index of the maximum of row r, in torch.argmax's order (NaN above everything, -0 and +0 equal). */
 int mi_argmax(const void* x, int64_t n_rows, int64_t vocab, int64_t row_stride, int64_t* index, int dtype, void* stream);
+/* The same, and out[r] = table[index[r]] in one launch: table [table_rows >= vocab, hidden] of the same type, out [n_rows, hidden], both 16-byte aligned,
+ * hidden and table_stride multiples of 8 elements (4 for fp32). */
+int mi_argmax_embed(const void* x, int64_t n_rows, int64_t vocab, int64_t row_stride, int64_t* index, const void* table, int64_t table_rows,
+                    int64_t table_stride, int64_t hidden, void* out, int dtype, void* stream);
 /* The weighted mean of cross_entropy.py:30 and the accuracy of :81-86 in one launch:
  *   loss = sum(losses * weights) / sum(weights),  total = sum(weights),
  *   accuracy = share of the rows with weights > 0 whose argmax is the target

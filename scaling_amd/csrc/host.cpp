@@ -1527,15 +1527,32 @@ OptTensor op_norm_linear_rows(const Tensor& x, const Tensor& norm, double eps, c
 }
 
 // Index of the maximum of each row of x [rows, n]; nothing where mi_argmax does not apply or a transform has to see the operation.
+bool argmax_applies(const Tensor& x) {
+    return !(transforming() || transformed(x) || !x.is_cuda() || x.dim() != 2 || x.size(0) < 1 || x.size(1) < 1 || x.size(1) > (1 << 30) ||
+             (x.size(1) > 1 && x.stride(1) != 1) || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat));
+}
 OptTensor op_argmax_rows(const Tensor& x) {
-    if (transforming() || transformed(x) || !x.is_cuda() || x.dim() != 2 || x.size(0) < 1 || x.size(1) < 1 || x.size(1) > (1 << 30) ||
-        (x.size(1) > 1 && x.stride(1) != 1) || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf && x.scalar_type() != at::kFloat))
-        return std::nullopt;
+    if (!argmax_applies(x)) return std::nullopt;
     need_gpu(x);
     Launch l(x);
     const Tensor out = at::empty({x.size(0)}, x.options().dtype(at::kLong));
     check(mi_argmax(ptr(x), x.size(0), x.size(1), x.stride(0), out.data_ptr<int64_t>(), code_of(x), l.stream), "mi_argmax");
     return out;
+}
+
+// The same and those rows of a table [at least n, hidden] (inference); nothing where mi_argmax_embed does not apply.
+std::optional<std::tuple<Tensor, Tensor>> op_argmax_embed(const Tensor& x, const Tensor& table) {
+    if (!argmax_applies(x) || transformed(table) || table.scalar_type() != x.scalar_type() || table.device() != x.device() || !aligned(table) ||
+        table.size(0) < x.size(1) || table.size(1) < 1 || table.size(1) % (x.scalar_type() == at::kFloat ? 4 : 8) != 0 ||
+        (at::GradMode::is_enabled() && table.requires_grad()))
+        return std::nullopt;
+    need_gpu(x);
+    Launch l(x);
+    const Tensor index = at::empty({x.size(0)}, x.options().dtype(at::kLong)), out = at::empty({x.size(0), table.size(1)}, table.options());
+    check(mi_argmax_embed(ptr(x), x.size(0), x.size(1), x.stride(0), index.data_ptr<int64_t>(), ptr(table), table.size(0), table.stride(0), table.size(1),
+                          ptr(out), code_of(x), l.stream),
+          "mi_argmax_embed");
+    return std::make_tuple(index, out);
 }
 
 // One token per sequence through a pre-norm layer (RMSNorm, separate q / k / v, SwiGLU, no biases): five launches, plus the merge of
@@ -1635,5 +1652,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     def("decode_attention", &op_decode_attention);
     def("norm_linear_rows", &op_norm_linear_rows);
     def("argmax_rows", &op_argmax_rows);
+    def("argmax_embed", &op_argmax_embed);
     def("decode_layer", &op_decode_layer);
 }

@@ -44,6 +44,9 @@ class EmbeddingInput(torch.nn.Module):
         return self.embedding(token_ids)
 
 
+_CHOOSE_AND_EMBED = (sample_argmax, EmbeddingInput.forward, torch.nn.Embedding.forward)
+
+
 class TransformerInferenceModule(torch.nn.Module):
     """`_layers[i]` holds the i-th layer in the reference's order, so checkpoint indices line up."""
 
@@ -159,10 +162,18 @@ class TransformerInferenceModule(torch.nn.Module):
         native = [(layer, layer.self_attention.cache.get(0), decode_arguments(layer, batch, tokens, 0)) for layer in layers]
         return native if all(arguments is not None for _, _, arguments in native) else None
 
-    def _native_step(self, native: list, token_ids: torch.Tensor, position_ids: torch.Tensor, step: dict) -> Optional[torch.Tensor]:
-        """Logits [b, 1, vocab] of one token per sequence; None, with nothing done, where the kernels refuse the first layer.  A later
+    def _own_embedding(self) -> Optional[torch.Tensor]:
+        """The embedding's weight where choosing a token and embedding it come to one look at each; None where somebody replaced or hooked either."""
+        first = self._layers[0]
+        if type(first) is not EmbeddingInput or type(first.embedding) is not torch.nn.Embedding or not _unhooked(first, first.embedding) or \
+                first.embedding.max_norm is not None or (sample_argmax, EmbeddingInput.forward, torch.nn.Embedding.forward) != _CHOOSE_AND_EMBED:
+            return None
+        return first.embedding.weight
+
+    def _native_step(self, native: list, token_ids: torch.Tensor, h: Optional[torch.Tensor], position_ids: torch.Tensor, step: dict) -> Optional[torch.Tensor]:
+        """Logits [b, 1, vocab] of one token per sequence (h: already embedded); None, with nothing done, where the kernels refuse the first layer.  A later
         layer that they refuse (a weight of another layout) is called with the arguments `step` of a cached step."""
-        h = self._layers[0](token_ids)
+        h = self._layers[0](token_ids) if h is None else h
         for i, (layer, cache, arguments) in enumerate(native):
             y = ops.decode_layer(h, position_ids, arguments)
             if y is not None:
@@ -288,7 +299,9 @@ class TransformerInferenceModule(torch.nn.Module):
             native = self._native_layers(b, max_tokens - 1)
             tokens = []
             for k in range(max_tokens):
-                nxt = sample_argmax(logits)
+                table = self._own_embedding() if native is not None and k + 1 < max_tokens else None
+                both = None if table is None else ops.argmax_embed(logits[:, -1, :], table)
+                nxt, h = (sample_argmax(logits), None) if both is None else (both[0], both[1].unsqueeze(1))
                 step_logits.append(logits[:, -1, :])
                 tokens.append(nxt)
                 if b == 1 and stop and int(nxt) in stop:
@@ -297,7 +310,7 @@ class TransformerInferenceModule(torch.nn.Module):
                     break
                 step = dict(position_ids=positions[k], cumulative_seq_lengths=one_each, inference_settings=settings)
                 if native is not None:
-                    logits = self._native_step(native, nxt.unsqueeze(1), positions[k].view(-1), step)
+                    logits = self._native_step(native, nxt.unsqueeze(1), h, positions[k].view(-1), step)
                     if logits is not None:
                         continue
                     native = None                        # a shape the kernels do not cover: nothing has been done yet

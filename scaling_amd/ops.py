@@ -564,6 +564,11 @@ def argmax_rows(x: torch.Tensor) -> torch.Tensor:
     return torch.argmax(x, dim=-1) if index is None else index
 
 
+def argmax_embed(x: torch.Tensor, table: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """(argmax_rows(x), table[argmax_rows(x)]) of x [rows, n] and table [at least n, hidden] in one launch (inference); None where the kernel does not apply."""
+    return None if _taken_over((x, table)) or not x.is_cuda else _lib.host().argmax_embed(x, table)
+
+
 def decode_layer_arguments(norm1, eps1, qkv_weights, dense, norm2, eps2, w_in, w_gate, w_out, head_dim, k_cache, v_cache, ctx_len, tables,
                            softmax_scale, workspace, dtype) -> Optional[tuple]:
     """What `decode_layer` takes beside the token: the layer's weights, its caches and rotary tables.  None for weights that have to see

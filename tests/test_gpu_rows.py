@@ -174,3 +174,29 @@ def test_argmax_of_rows(rows, n, offset, dtype):
             assert ref.tolist() == [0] * rows              # -0 and +0 are equal
         assert torch.equal(ops.argmax_rows(c).cpu(), ref), i
     assert ops.argmax_rows(x[:0]).numel() == 0
+
+
+# one vector, more of them than threads, a padded table with more rows than are chosen from
+@pytest.mark.parametrize("rows,n,hidden,pad", [(1, 1, 8, 0), (3, 32000, 1024, 0), (5, 1001, 12288, 8), (300, 515, 264, 16)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_argmax_with_its_embedding(rows, n, hidden, pad, dtype):
+    x, table = _rand((rows, n), dtype, n), _rand((n + 3, hidden + pad), dtype, 2)[:, :hidden]
+    x[0, n // 2] = float("nan")                            # above everything
+    with torch.no_grad():
+        index, out = ops.argmax_embed(x, table)
+        assert torch.equal(index, ops.argmax_rows(x)) and int(index[0]) == n // 2 and torch.equal(out, table[index])
+        for refused in (table[:n - 1], table[:, :hidden - 1], table.double(), table.t()):
+            assert ops.argmax_embed(x, refused) is None
+    assert ops.argmax_embed(x, table.clone().requires_grad_()) is None
+
+
+def test_generation_calls_a_watched_embedding():
+    cfg = TransformerArchitectureConfig.from_dict(dict(
+        vocab_size=512, hidden_size=256, num_layers=2, num_attention_heads=4, attention_num_kv_heads=2, sequence_length=64, precision="bfloat16", norm_type="rms",
+        mlp_type="swiglu", mlp_factor=2.75, attention_bias=False, mlp_bias=False, attention_qkv_in_one=False, masked_softmax={"kernel": "hip"}))
+    model, ids, calls = TransformerInferenceModule(cfg, DEV, seed=3), torch.arange(1, 21).view(2, 10), []
+    tokens, logits = model.generate(6, ids)
+    handle = model._layers[0].embedding.register_forward_hook(lambda *a: calls.append(1))
+    tokens2, logits2 = model.generate(6, ids)
+    handle.remove()
+    assert len(calls) == 6 and tokens == tokens2 and torch.equal(logits, logits2)
