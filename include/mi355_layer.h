@@ -270,6 +270,16 @@ int mi_rotary_complex(const void* x, void* out, const float* cos, const float* s
                       int64_t x_stride_token, int64_t x_stride_head, int64_t out_stride_token, int64_t out_stride_head,
                       int64_t table_rows, int64_t seq_len_for_null_ids, int inverse, int dtype, void* stream);
 
+/* mi_rotary (interleaved: mi_rotary_complex, rot_dim = head_dim) of two tensors of the same tokens, in one launch where both are whole vectors. */
+typedef struct mi_rotary_rows {
+    const void* x;
+    void* out;
+    int64_t x_stride_token, x_stride_head, out_stride_token, out_stride_head;
+    int32_t n_heads;
+} mi_rotary_rows;
+int mi_rotary_two(const mi_rotary_rows* rows, const void* cos, const void* sin, const int64_t* position_ids, int64_t n_tokens, int32_t head_dim,
+                  int32_t rot_dim, int64_t table_rows, int64_t seq_len_for_null_ids, int inverse, int interleaved, int dtype, int table_dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Attention core.  Replaces core/nn/attention/attention.py:108-213 (multi_head_attention) with
  * core/nn/masked_softmax/masked_softmax.py:14-34 as softmax and :76-105 as mask, plus repeat_kv

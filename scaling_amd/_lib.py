@@ -24,7 +24,7 @@ EXPORTS = (
     "mi_rmsnorm_fwd", "mi_add_rmsnorm_fwd", "mi_rmsnorm_bwd_workspace_bytes", "mi_rmsnorm_bwd",
     "mi_layernorm_fwd", "mi_layernorm_bwd_workspace_bytes", "mi_layernorm_bwd", "mi_gelu_fwd", "mi_gelu_bwd", "mi_cross_entropy",
     "mi_cross_entropy_padded", "mi_argmax", "mi_argmax_embed", "mi_cross_entropy_mean_grad", "mi_loss_reduce", "mi_loss_row_scale", "mi_scale_inplace",
-    "mi_swiglu_fwd", "mi_swiglu_bwd", "mi_rotary", "mi_rotary_complex",
+    "mi_swiglu_fwd", "mi_swiglu_bwd", "mi_rotary", "mi_rotary_complex", "mi_rotary_two",
     "mi_attn_fwd", "mi_attn_bwd_workspace_bytes", "mi_attn_bwd_workspace_bytes_kv", "mi_attn_bwd_workspace_bytes_for", "mi_attn_bwd",
     "mi_gemm", "mi_gemm_workspace_bytes", "mi_gemm_with_workspace", "mi_rows_product", "mi_transpose16", "mi_column_sum", "mi_add_rmsnorm_bwd", "mi_add_layernorm_fwd", "mi_add_layernorm_bwd", "mi_attn_decode_workspace_bytes", "mi_attn_decode", "mi_attn_decode_with_tickets", "mi_fill_cache", "mi_attn_decode_static_scratch_bytes", "mi_attn_decode_static",
 )
@@ -99,6 +99,11 @@ class MiRowsArgs(Structure):
     ]
 
 
+class MiRotaryRows(Structure):
+    _fields_ = [("x", c_void_p), ("out", c_void_p), ("x_stride_token", c_int64), ("x_stride_head", c_int64), ("out_stride_token", c_int64),
+                ("out_stride_head", c_int64), ("n_heads", c_int32)]
+
+
 _lib = None
 _host = None
 _device_checked = False
@@ -138,6 +143,9 @@ def _declare(lib):
     lib.mi_cross_entropy_padded.argtypes = [c_void_p] * 6 + [c_int64, c_int64, c_int64, c_int, c_void_p]
     lib.mi_cross_entropy_mean_grad.restype = c_int
     lib.mi_cross_entropy_mean_grad.argtypes = [c_void_p] * 7 + [c_int64, c_int64, c_int64, c_int64, c_int, c_void_p]
+    lib.mi_rotary_two.restype = c_int
+    lib.mi_rotary_two.argtypes = [POINTER(MiRotaryRows), c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_int64, c_int64, c_int, c_int, c_int, c_int,
+                                  c_void_p]
     lib.mi_argmax.restype = c_int
     lib.mi_argmax.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p]
     lib.mi_argmax_embed.restype = c_int

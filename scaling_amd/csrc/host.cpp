@@ -346,21 +346,75 @@ Tensor rotary_launch(const Tensor& x, const Tensor& cos, const Tensor& sin, cons
     return out;
 }
 
+// The same of two tensors of the same tokens
+std::tuple<Tensor, Tensor> rotary_launch_two(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const OptTensor& ids,
+                                             int64_t seq_len_for_null_ids, bool inverse, bool interleaved) {
+    for (const Tensor* t : {&q, &k}) {
+        need_gpu(*t);
+        TORCH_CHECK(t->dim() == 3 && t->stride(2) == 1 && t->size(0) == q.size(0) && t->size(2) == q.size(2) && t->scalar_type() == q.scalar_type() &&
+                        t->device() == q.device(),
+                    "rotary: bad layout");
+    }
+    TORCH_CHECK(cos.is_contiguous() && sin.is_contiguous(), "rotary: bad layout");
+    Launch l(q);
+    const Tensor q_out = at::empty(q.sizes(), q.options()), k_out = at::empty(k.sizes(), k.options());
+    const Tensor pos = ids.has_value() && ids->defined() ? ids->contiguous() : Tensor();
+    TORCH_CHECK(!pos.defined() || (pos.scalar_type() == at::kLong && pos.numel() == q.size(0)), "rotary: one int64 position id per token");
+    const auto rows = [](const Tensor& x, const Tensor& out) {
+        return mi_rotary_rows{ptr(x), ptr(out), x.stride(0), x.stride(1), out.stride(0), out.stride(1), (int32_t)x.size(1)};
+    };
+    const mi_rotary_rows both[2] = {rows(q, q_out), rows(k, k_out)};
+    check(mi_rotary_two(both, ptr(cos), ptr(sin), (const int64_t*)ptr(pos), q.size(0), (int)q.size(2), interleaved ? (int)q.size(2) : (int)cos.size(1),
+                        cos.size(0), seq_len_for_null_ids, inverse, interleaved, code_of(q), code_of(cos), l.stream),
+          "mi_rotary_two");
+    return {q_out, k_out};
+}
+
 struct Rotary : Function<Rotary> {
-    template <class Context> static Tensor run(Context* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len, bool interleaved) {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len, bool interleaved) {
         ctx->save_for_backward({cos, sin, opt(ids)});
         ctx->saved_data["seq_len"] = seq_len;
         ctx->saved_data["interleaved"] = interleaved;
         return rotary_launch(x, cos, sin, ids, seq_len, false, interleaved);
     }
-    template <class Context> static variable_list gradients(Context* ctx, const variable_list& g) {
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
         const variable_list saved = ctx->get_saved_variables();
         const Tensor dout = g[0].stride(-1) == 1 ? g[0] : g[0].contiguous();
         return {rotary_launch(dout, saved[0], saved[1], saved[2], ctx->saved_data["seq_len"].toInt(), true, ctx->saved_data["interleaved"].toBool()),
                 Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
-    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len, bool interleaved) {
-        return run(ctx, x, cos, sin, ids, seq_len, interleaved);
+};
+
+// q and k of a layer
+struct RotaryTwo : Function<RotaryTwo> {
+    template <class Context> static variable_list run(Context* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const OptTensor& ids,
+                                                      int64_t seq_len, bool interleaved) {
+        ctx->set_materialize_grads(false);
+        ctx->save_for_backward({cos, sin, opt(ids)});
+        ctx->saved_data["seq_len"] = seq_len;
+        ctx->saved_data["interleaved"] = interleaved;
+        auto [q_rot, k_rot] = rotary_launch_two(q, k, cos, sin, ids, seq_len, false, interleaved);
+        return {q_rot, k_rot};
+    }
+    template <class Context> static variable_list gradients(Context* ctx, const variable_list& g) {
+        const variable_list saved = ctx->get_saved_variables();
+        const int64_t seq_len = ctx->saved_data["seq_len"].toInt();
+        const bool interleaved = ctx->saved_data["interleaved"].toBool();
+        variable_list d(7);
+        Tensor in[2];
+        for (int i : {0, 1})
+            if (g[i].defined()) in[i] = g[i].stride(-1) == 1 ? g[i] : g[i].contiguous();
+        if (in[0].defined() && in[1].defined()) {
+            std::tie(d[0], d[1]) = rotary_launch_two(in[0], in[1], saved[0], saved[1], saved[2], seq_len, true, interleaved);
+        } else {
+            for (int i : {0, 1})
+                if (in[i].defined()) d[i] = rotary_launch(in[i], saved[0], saved[1], saved[2], seq_len, true, interleaved);
+        }
+        return d;
+    }
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const OptTensor& ids, int64_t seq_len,
+                                 bool interleaved) {
+        return run(ctx, q, k, cos, sin, ids, seq_len, interleaved);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) { return gradients(ctx, g); }
 };
@@ -988,7 +1042,7 @@ struct LayerCall : torch::CustomClassHolder {
     int64_t nq, nkv, d;
     int rotary;                                            // 0 none, 1 inside the attention core, 2 in front of it
     std::vector<Tensor> caches;                            // [k, v, ctx_len] of a prefill (rotary 1, inference) or empty
-    enum Part { kNorm1, kQkv, kRotaryQ, kRotaryK, kAttention, kDense, kNorm2, kIn, kActivation, kOut, kParts };
+    enum Part { kNorm1, kQkv, kRotary, kAttention, kDense, kNorm2, kIn, kActivation, kOut, kParts };
     Kept parts[kParts];                                    // of a layer that is one node
     bool split() const { return !in_one || rotary == 2; }  // q, k and v reach the attention core as three
 };
@@ -1003,7 +1057,7 @@ struct Apart {
         if (w.size() > 1) return op_projections(x, w, b, c.inference);
         return {op_linear(x, w[0], b[0], residual, c.inference)};
     }
-    Tensor rotary(LayerCall::Part, const Tensor& x, int64_t s) { return Rotary::apply(x, *c.cos, *c.sin, c.pos, s, c.interleaved); }
+    variable_list rotary(const Tensor& q, const Tensor& k, int64_t s) { return RotaryTwo::apply(q, k, *c.cos, *c.sin, c.pos, s, c.interleaved); }
     Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const AttnOptions& o) {
         return Attention::apply(q, k, v, c.cu, OptTensor(), &o, at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()));
     }
@@ -1037,7 +1091,9 @@ struct Together {
         for (const Tensor& t : params) reaches(t);
         return Projections::run(&c.parts[p], x, params, residual, has_bias, c.inference, need_dx);
     }
-    Tensor rotary(LayerCall::Part p, const Tensor& x, int64_t s) { return Rotary::run(&c.parts[p], x, *c.cos, *c.sin, c.pos, s, c.interleaved); }
+    variable_list rotary(const Tensor& q, const Tensor& k, int64_t s) {
+        return RotaryTwo::run(&c.parts[LayerCall::kRotary], q, k, *c.cos, *c.sin, c.pos, s, c.interleaved);
+    }
     Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const AttnOptions& o) {
         return attention_node_forward(&c.parts[LayerCall::kAttention], q, k, v, c.cu, Tensor(), o, grad);
     }
@@ -1075,8 +1131,9 @@ template <class Operations> Tensor layer_forward(const LayerCall& c, Operations 
                                     q.scalar_type() == at::kHalf);
         } else {
             if (c.rotary == 2) {
-                q = ops.rotary(LayerCall::kRotaryQ, q, s);
-                k = ops.rotary(LayerCall::kRotaryK, k, s);
+                const auto both = ops.rotary(q, k, s);
+                q = both[0];
+                k = both[1];
             }
             ctx = ops.attention(q, k, v, rotated());
         }
@@ -1199,9 +1256,9 @@ struct Layer : Function<Layer> {
         variable_list dqkv = c.split() ? Attention::gradients(&att, dout) : AttentionQkv::gradients(&att, dout);
         dqkv.resize(c.split() ? 3 : 1);
         if (c.rotary == 2) {
-            Replayed q = part(LayerCall::kRotaryQ), k = part(LayerCall::kRotaryK);
-            dqkv[0] = Rotary::gradients(&q, {dqkv[0]})[0];
-            dqkv[1] = Rotary::gradients(&k, {dqkv[1]})[0];
+            Replayed rotary = part(LayerCall::kRotary);
+            const variable_list d = RotaryTwo::gradients(&rotary, {dqkv[0], dqkv[1]});
+            std::copy(d.begin(), d.begin() + 2, dqkv.begin());
         }
         if (c.in_one && c.split()) dqkv = {at::cat(dqkv, 2)};
         for (Tensor& t : dqkv) t = t.reshape({tokens, -1});

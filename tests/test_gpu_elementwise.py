@@ -350,3 +350,30 @@ def test_norm_backward_of_narrow_rows(rows, hidden, dtype, layer_norm):
     for name, got, want, bound in zip(("dx", "dw", "db"), leaves, exact, (2 * unit, unit, unit)):
         error = ((got.grad.double() - want.grad).norm() / want.grad.norm()).item()
         assert error <= bound, (name, error, bound)
+
+
+# whole vectors in one launch; rotated spans, strides or a second tensor that are not
+@pytest.mark.parametrize("tokens,heads,kv,d,rot,pad,interleaved", [(1, 1, 1, 64, 64, 0, False), (67, 4, 2, 64, 32, 8, False), (300, 3, 5, 128, 128, 0, True),
+                                                                   (33, 2, 2, 64, 36, 0, False), (50, 4, 2, 96, 96, 3, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("table,inverse,ids", [("own", 0, True), ("float32", 1, False)])
+def test_rotary_of_two_tensors(tokens, heads, kv, d, rot, pad, interleaved, dtype, table, inverse, ids):
+    """To the bit what a launch for each gives."""
+    g = torch.Generator().manual_seed(d + rot)
+    own = torch.float32 if interleaved or table == "float32" else dtype
+    cos, sin = (_rand(g, 40, d // 2 if interleaved else rot, dtype=own).to(DEV) for _ in range(2))
+    pos = torch.randint(0, 40, (tokens,), generator=g).to(DEV) if ids else None
+    q = _rand(g, tokens, heads, d, dtype=dtype).to(DEV)
+    k = _rand(g, tokens, kv, d + pad, dtype=dtype).to(DEV)[:, :, pad:]
+    if pad == 3:
+        assert k.data_ptr() % 16 != 0
+    lib, outs = _lib.load(), [torch.empty(tokens, heads, d, dtype=dtype, device=DEV), torch.empty(tokens, kv, d, dtype=dtype, device=DEV)]
+    rows = (_lib.MiRotaryRows * 2)(*[_lib.MiRotaryRows(x.data_ptr(), o.data_ptr(), x.stride(0), x.stride(1), o.stride(0), o.stride(1), x.shape[1])
+                                     for x, o in zip((q, k), outs)])
+    code, at = _lib.dtype_code(dtype), 0 if pos is None else pos.data_ptr()
+    status = lib.mi_rotary_two(rows, cos.data_ptr(), sin.data_ptr(), at, tokens, d, d if interleaved else rot, 40, 40, inverse, int(interleaved), code,
+                               _lib.dtype_code(own), _lib.stream_ptr())
+    assert status == 0
+    for x, o in zip((q, k), outs):
+        want = _lib.host().rotary_launch(x, cos, sin, pos, 40, bool(inverse), interleaved)
+        assert torch.equal(o, want)
