@@ -732,17 +732,17 @@ template <int D> int launch_bwd(const AttnParams& p, int flags, hipStream_t st) 
     return MI_OK;
 }
 
-template <int D> int launch_short(const AttnParams& p, ShortBwd route, hipStream_t st) {
+template <int D> int launch_short(const AttnParams& p, ShortBwd route, bool pairs, hipStream_t st) {
     const int64_t grid_q = ((int64_t)p.total_q + kShortRows - 1) / kShortRows * p.nq;
     const int64_t grid_k = ((int64_t)p.total_k + kShortRows - 1) / kShortRows * p.nkv * p.hsplit;
     if (grid_q + grid_k > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_bwd: grid too large");
-    const dim3 block(64 * kShortWaves);
+    const dim3 block(256);
     int rc = MI_OK;
     if (D > 64 && route == ShortBwd::kApart) {
         if constexpr (D > 64) attn_short_dq_kernel<D><<<dim3((unsigned)grid_q), block, 0, st>>>(p);
         rc = mi_check_launch("attn_short_dq");
         if (rc != MI_OK) return rc;
-        attn_short_bwd_kernel<D, false><<<dim3((unsigned)grid_k), block, 0, st>>>(p, (int)grid_k);
+        attn_short_bwd_kernel<D, 4, false><<<dim3((unsigned)grid_k), block, 0, st>>>(p, (int)grid_k);
     } else {
         // delta inside the dK / dV blocks, or a launch of its own in front: that costs 4 us, forming it anew for every key block a tenth of
         // the time of a chain (queries of a document x query heads of a block).  Inside / in front, us, bf16, 4 heads, chains of 512 | 1024 | 1626 |
@@ -757,8 +757,16 @@ template <int D> int launch_short(const AttnParams& p, ShortBwd route, hipStream
             rc = mi_check_launch("attn_bwd_delta_short");
             if (rc != MI_OK) return rc;
         }
-        const auto kernel = own_delta ? attn_short_bwd_kernel<D, true> : attn_short_bwd_kernel<D, false>;
-        kernel<<<dim3((unsigned)(grid_k + grid_q)), block, 0, st>>>(p, (int)grid_k);
+        const dim3 grid((unsigned)(grid_k + grid_q));
+        if (D <= 64 && pairs) {
+            if constexpr (D <= 64) {
+                const auto kernel = own_delta ? attn_short_bwd_kernel<D, 2, true> : attn_short_bwd_kernel<D, 2, false>;
+                kernel<<<grid, dim3(128), 0, st>>>(p, (int)grid_k);
+            }
+        } else {
+            const auto kernel = own_delta ? attn_short_bwd_kernel<D, 4, true> : attn_short_bwd_kernel<D, 4, false>;
+            kernel<<<grid, block, 0, st>>>(p, (int)grid_k);
+        }
     }
     rc = mi_check_launch("attn_short_bwd");
     if (rc != MI_OK || p.hsplit == 1) return rc;
@@ -818,11 +826,12 @@ int MI_ENTRY(mi_attn_bwd_impl)(const mi_attn_bwd_args* b) {
     mi_set_head_split(a, b, &p);
     const ShortBwd route = mi_attn_bwd_short(a, p.hsplit);
     if (route != ShortBwd::kNo && !(a->flags & (MI_ATTN_SPLIT_P | MI_ATTN_BWD_DELTA | MI_ATTN_BWD_DKDV | MI_ATTN_BWD_DQ)) && p.drop_thr == 0) {
+        const bool pairs = mi_attn_short_pairs(a, true, mi_attn_short_blocks(a, a->n_q_heads + (int64_t)a->n_kv_heads * p.hsplit));
         switch (a->head_dim) {
-            case 32: return launch_short<32>(p, route, (hipStream_t)a->stream);
-            case 64: return launch_short<64>(p, route, (hipStream_t)a->stream);
-            case 96: return launch_short<96>(p, route, (hipStream_t)a->stream);
-            default: return launch_short<128>(p, route, (hipStream_t)a->stream);
+            case 32: return launch_short<32>(p, route, pairs, (hipStream_t)a->stream);
+            case 64: return launch_short<64>(p, route, pairs, (hipStream_t)a->stream);
+            case 96: return launch_short<96>(p, route, pairs, (hipStream_t)a->stream);
+            default: return launch_short<128>(p, route, pairs, (hipStream_t)a->stream);
         }
     }
     {                                                                                               // dQ: 256-query blocks

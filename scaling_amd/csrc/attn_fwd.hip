@@ -486,19 +486,19 @@ template <int D> int launch_d(const AttnParams& p, int rot, bool q_only, int nw,
     return nw == 8 ? launch<D, 8, 0, false>(p, st) : launch<D, 4, 0, false>(p, st);
 }
 
-template <int D> int launch_short(const AttnParams& p, int rot, bool q_only, hipStream_t st) {
+template <int D, int W> int launch_short(const AttnParams& p, int rot, bool q_only, hipStream_t st) {
     const int64_t grid = ((int64_t)p.total_q + kShortRows - 1) / kShortRows * p.nq;
     if (grid > 0x7fffffffLL) return mi_fail(MI_E_SHAPE, "attn_fwd: too many work items");
-    const dim3 g((unsigned)grid), b(64 * kShortWaves);
+    const dim3 g((unsigned)grid), b(64 * W);
     if constexpr (D == 64 || D == 128) {
-        if (rot == 2 && q_only) attn_short_fwd_kernel<D, 2, false><<<g, b, 0, st>>>(p);
-        else if (rot == 2) attn_short_fwd_kernel<D, 2, true><<<g, b, 0, st>>>(p);
-        else if (rot == 1 && q_only) attn_short_fwd_kernel<D, 1, false><<<g, b, 0, st>>>(p);
-        else if (rot == 1) attn_short_fwd_kernel<D, 1, true><<<g, b, 0, st>>>(p);
-        else attn_short_fwd_kernel<D, 0, false><<<g, b, 0, st>>>(p);
+        if (rot == 2 && q_only) attn_short_fwd_kernel<D, 2, false, W><<<g, b, 0, st>>>(p);
+        else if (rot == 2) attn_short_fwd_kernel<D, 2, true, W><<<g, b, 0, st>>>(p);
+        else if (rot == 1 && q_only) attn_short_fwd_kernel<D, 1, false, W><<<g, b, 0, st>>>(p);
+        else if (rot == 1) attn_short_fwd_kernel<D, 1, true, W><<<g, b, 0, st>>>(p);
+        else attn_short_fwd_kernel<D, 0, false, W><<<g, b, 0, st>>>(p);
     } else {
         if (rot) return mi_fail(MI_E_SHAPE, "attn_fwd: fused rotary needs head_dim 64 or 128");
-        attn_short_fwd_kernel<D, 0, false><<<g, b, 0, st>>>(p);
+        attn_short_fwd_kernel<D, 0, false, W><<<g, b, 0, st>>>(p);
     }
     return mi_check_launch("attn_short_fwd");
 }
@@ -522,11 +522,16 @@ int MI_ENTRY(mi_attn_fwd_impl)(const mi_attn_args* a) {
         p.q_rot = (elem_t*)a->q_rot_out;
     }
     if (mi_attn_fwd_is_short(a) && !(a->flags & MI_ATTN_SPLIT_P) && p.drop_thr == 0) {
+        const bool pairs = mi_attn_short_pairs(a, false, mi_attn_short_blocks(a, a->n_q_heads));
+        const auto go = [&](auto d) {
+            constexpr int D = decltype(d)::value;
+            return pairs ? launch_short<D, 2>(p, rot, q_only, (hipStream_t)a->stream) : launch_short<D, 4>(p, rot, q_only, (hipStream_t)a->stream);
+        };
         switch (a->head_dim) {
-            case 32: return launch_short<32>(p, rot, q_only, (hipStream_t)a->stream);
-            case 64: return launch_short<64>(p, rot, q_only, (hipStream_t)a->stream);
-            case 96: return launch_short<96>(p, rot, q_only, (hipStream_t)a->stream);
-            default: return launch_short<128>(p, rot, q_only, (hipStream_t)a->stream);
+            case 32: return go(std::integral_constant<int, 32>{});
+            case 64: return go(std::integral_constant<int, 64>{});
+            case 96: return go(std::integral_constant<int, 96>{});
+            default: return go(std::integral_constant<int, 128>{});
         }
     }
     // 256-query workgroups (two groups of wavefronts a phase apart) beat 128-query ones at every size measured,

@@ -2,8 +2,8 @@
 //
 // The tiled kernels give a workgroup 128 - 256 rows and walk its keys (queries) in one chain of barriers; with short documents that
 // chain is most of the launch, its workgroups leave compute units idle, and 256 rows span several documents.  Here a workgroup of
-// four wavefronts owns 32 rows, and the wavefronts split the other axis: wavefront w takes tiles w, w + 4, ... of 32 tokens,
-// each through its own LDS stages with direct global -> LDS loads and no barrier, and the four partial results meet in
+// four (two: mi_attn_short_pairs) wavefronts owns 32 rows, and the wavefronts split the other axis: wavefront w takes tiles w, w + 4, ... of 32 tokens,
+// each through its own LDS stages with direct global -> LDS loads and no barrier, and the partial results meet in
 // LDS at the end, in a fixed order.  A document of 512 tokens is a chain of at most four tiles.  The mask interval of a row comes from one
 // load of the cumulative lengths and a search in registers.
 // The price is operand traffic: a tile serves 32 rows instead of 128 or 256, so long contexts stay with the tiled kernels
@@ -13,7 +13,7 @@
 
 namespace {
 
-constexpr int kShortWaves = 4, kShortRows = 32;
+constexpr int kShortRows = 32;
 
 // Largest j < n_docs with cu[j] <= t and the bounds of that document on both axes, as find_doc gives them; for up to 63 documents the
 // lengths sit one per lane.
@@ -69,11 +69,11 @@ __device__ __forceinline__ void short_tiles(int lo, int hi, int& wmin, int& wmax
 // One wavefront's two (three) tiles of 32 tokens, in STAGES stages.  The chains are short, so what hides the loads is the other workgroups of the
 // compute unit: one stage (8192 tokens x 32 heads of 128 in documents of 512: forward 240 us with two, 137 with one), except for dK / dV
 // of 96 and 128 features, whose registers leave room for one workgroup anyway.
-template <int D, int STAGES = 1, int TILES = 2> struct ShortStages {
+template <int D, int WAVES, int STAGES = 1, int TILES = 2> struct ShortStages {
     using Tile = LdsTile<D>;
     static constexpr int kTile = 32 * Tile::RB, kLoads = Tile::kInstrs / 2;
     static constexpr int kBytes = TILES * STAGES * kTile;
-    static constexpr int kSmem = kShortWaves * kBytes;
+    static constexpr int kSmem = WAVES * kBytes;
     char* base;
     __device__ __forceinline__ char* first(int buf = 0) const { return base + buf * TILES * kTile; }
     __device__ __forceinline__ char* second(int buf = 0) const { return base + buf * TILES * kTile + kTile; }
@@ -82,7 +82,8 @@ template <int D, int STAGES = 1, int TILES = 2> struct ShortStages {
     static __device__ __forceinline__ void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 };
 
-// Sum over the wavefronts of quad a = wave of every feature tile, from the per-wavefront copies in LDS ([wave][16 DT][64] floats).
+template <int D, int WAVES> constexpr int kShortRed = WAVES * 16 * (D / 32) * 64 * 4;      // an accumulator set of every wavefront
+// Sums over the wavefronts meet in LDS ([wave][16 DT][64] floats); then each of them takes 4 / WAVES of the quads of every feature tile (rows 8 a + 4 g + c).
 template <int D> __device__ __forceinline__ void short_store(float* red, int wave, int lane, const f32x16_t (&acc)[D / 32]) {
     float* mine = red + wave * (16 * (D / 32) * 64) + lane;
 #pragma unroll
@@ -90,15 +91,18 @@ template <int D> __device__ __forceinline__ void short_store(float* red, int wav
 #pragma unroll
         for (int r = 0; r < 16; ++r) mine[(dt * 16 + r) * 64] = acc[dt][r];
 }
-template <int D> __device__ __forceinline__ void short_sum(const float* red, int wave, int lane, float (&x)[D / 32][4]) {
+template <int D, int WAVES> __device__ __forceinline__ void short_sums(const float* red, int wave, int lane, float (&x)[4 / WAVES][D / 32][4]) {
     constexpr int kSet = 16 * (D / 32) * 64;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int j = 0; j < 4 / WAVES; ++j)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const float* at = red + (dt * 16 + 4 * wave + c) * 64 + lane;
-            x[dt][c] = (at[0] + at[kSet]) + (at[2 * kSet] + at[3 * kSet]);
-        }
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float* at = red + (dt * 16 + 4 * (wave * (4 / WAVES) + j) + c) * 64 + lane;
+                if constexpr (WAVES == 4) x[j][dt][c] = (at[0] + at[kSet]) + (at[2 * kSet] + at[3 * kSet]);
+                else x[j][dt][c] = at[0] + at[kSet];
+            }
 }
 // Rotation by minus the position's angles of features 32 dt + 8 a + 4 g + c (see unrotate_acc)
 template <int D> __device__ __forceinline__ void short_unrotate(float (&x)[D / 32][4], const AttnParams& p, int64_t pos, int a, int g) {
@@ -148,12 +152,42 @@ template <int D> __device__ __forceinline__ void short_write(elem_t* row, const 
 // 128, 8 documents of 512: 29.3 / 41.3; 12 heads of 64, 3001 tokens in documents of 17 - 400: 20.9 / 12.3; 1 head of 64, 65536 tokens: 1280 / 762.
 // Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
 // backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
+
+// Two wavefronts to a block instead of four.  What comes before and after a chain of tiles costs every wavefront of a block alike, and of four the short
+// chains of packed documents leave some without a tile; so two do a block in half as many turns of the chip again, as long as there are blocks
+// enough for it to wait for all of them and not for the longest chain.  That is twice as long now, and its length is not known here, only
+// the mean: hence enough heads, so that one document of half the tokens among 16 small ones is level too (8 heads of 64: 1.25 forward, 1.28
+// backward).  Two / four, over 691 calls of 4 - 32 heads of 32 - 128, 1024 - 16384 tokens, documents ragged, whole, with a long tail and with one long one among
+// short ones: forward .67 - 1.02, mean .85, backward .65 - 1.03, mean .79, where the rule takes two.  us: 16 heads of 64, 4096 tokens, documents of 20 - 380:
+// here four / two: backward 50.3 / 38.4; 32 heads: 92.2 / 68.5, forward 30.2 / 24.2; 16 heads of 128 35.0 / 25.4.
+// `blocks`: of 32 rows, of both kinds in a backward pass
+static inline bool mi_attn_short_pairs(const mi_attn_args* a, bool backward, int64_t blocks) {
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k, units = mi_compute_units(), d = a->head_dim;
+    if (a->n_docs <= 1) return false;
+    const int64_t chain = (a->causal ? 1 : 2) * rows / a->n_docs;
+    if (backward)
+        return d <= 64 && a->n_q_heads == a->n_kv_heads && a->n_q_heads >= 12 && blocks >= (d == 64 ? 6 : 7) * units && blocks * (d == 64 ? 64 : 40) >= chain * units;
+    if (d <= 64) return a->n_q_heads >= 24 && blocks >= 4 * units && blocks * (d == 64 ? 56 : 28) >= chain * units;
+    return a->n_q_heads >= 16 && blocks >= (a->n_q_heads >= 24 ? 4 : 5) * units && blocks * 96 >= chain * units;
+}
+
+static inline int64_t mi_attn_short_blocks(const mi_attn_args* a, int64_t heads) {
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k;
+    return (rows + kShortRows - 1) / kShortRows * heads;
+}
+
 static inline bool mi_attn_fwd_is_short(const mi_attn_args* a) {
     if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return false;
     if (a->flags & MI_ATTN_SHORT) return true;
-    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k;
+    const int64_t rows = a->total_q > a->total_k ? a->total_q : a->total_k, blocks = mi_attn_short_blocks(a, a->n_q_heads), units = mi_compute_units();
     const int64_t per_unit = a->head_dim <= 64 ? (a->causal ? 8 : 6) : (a->causal ? 4 : 3);
-    return rows > 128 && (rows + kShortRows - 1) / kShortRows * a->n_q_heads <= per_unit * mi_compute_units();
+    if (rows <= 128) return false;
+    if (blocks <= per_unit * units) return true;
+    // More blocks, of short documents and with two wavefronts each: two / tiled .42 - 1.01, mean .76 (32 heads of 64, 8192 tokens, documents of 20 - 380 47.1 / 64.2 us; 16 heads of
+    // 128 43.9 / 50.3).  Not where k is rotated here: these blocks rotate a tile more often.
+    const int64_t chain = (a->causal ? 1 : 2) * rows / (a->n_docs > 1 ? a->n_docs : 1);
+    return mi_attn_short_pairs(a, false, blocks) && (a->rotary_cos == nullptr || a->position_ids_k == nullptr) &&
+           (a->head_dim <= 64 ? chain <= (a->causal ? 600 : 400) : chain <= 250 && blocks <= 32 * units);
 }
 
 // The same for a backward pass, whose blocks of either kind (dQ: rows / 32 x query heads, dK / dV: rows / 32 x KV heads x head split)
@@ -185,7 +219,9 @@ static inline ShortBwd mi_attn_bwd_short(const mi_attn_args* a, int hsplit) {
         if (!whole && docs > 1 && rows <= 512 * docs) per_unit_8 = 192;
         else if (causal && (!whole || chains)) per_unit_8 = 80 + 12 * (group - 1) < 96 ? 80 + 12 * (group - 1) : 96;
         else per_unit_8 = (causal ? 32 : 40) + 12 * (group - 1) < 64 ? (causal ? 32 : 40) + 12 * (group - 1) : 64;
-        return dq * 8 <= per_unit_8 * units ? ShortBwd::kTogether : ShortBwd::kNo;
+        if (dq * 8 <= per_unit_8 * units) return ShortBwd::kTogether;
+        // two wavefronts / tiled .68 - 1.00, mean .81: 32 heads of 64, documents of 20 - 380, 4096 tokens 68.5 / 101 us, 8192 144 / 181
+        return mi_attn_short_pairs(a, true, both) && a->n_q_heads >= 16 && (causal ? 1 : 2) * rows <= 400 * docs ? ShortBwd::kTogether : ShortBwd::kNo;
     }
     const bool alone = chains && rows >= 1024 * docs * docs;                                         // few documents, long ones
     int64_t eighths = whole && docs > 1 && !chains ? 16 : 18 + 9 * (group - 1) / 2;                              // of a block of either kind per compute unit
@@ -198,15 +234,15 @@ static inline ShortBwd mi_attn_bwd_short(const mi_attn_args* a, int hsplit) {
 // ---- forward: 32 queries of one head --------------------------------------------------------------------------------
 // QROT: 0 = q as it is, 1 = rotate-half, 2 = interleaved rotary on the q load; KROT: k is rotated too, in its LDS tile (otherwise it
 // arrives rotated, as training passes it)
-template <int D, int QROT, bool KROT>
-__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_fwd_kernel(const AttnParams p) {
+template <int D, int QROT, bool KROT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, D <= 64 ? 4 : 2) void attn_short_fwd_kernel(const AttnParams p) {
     constexpr int KS = D / 16, DT = D / 32;
-    using Stages = ShortStages<D>;
+    using Stages = ShortStages<D, WAVES>;
     using Tile = LdsTile<D>;
     constexpr int RB = Tile::RB;
-    constexpr int kRed = kShortWaves * 16 * DT * 64 * 4;
+    constexpr int kRed = kShortRed<D, WAVES>;
     __shared__ __attribute__((aligned(1024))) char smem[Stages::kSmem > kRed ? Stages::kSmem : kRed];
-    __shared__ float m_lds[kShortWaves][32], l_lds[kShortWaves][32];
+    __shared__ float m_lds[WAVES][32], l_lds[WAVES][32];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nqb = (p.total_q + 31) / 32;
@@ -266,8 +302,8 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
     Tile::tr_bases(lane, h0, h1);
     const int k_row = Tile::row_base(l32, g);
     if (wave < n_tiles) { issue_k(wave); issue_v(wave); }
-    for (int tile = wave; tile < n_tiles; tile += kShortWaves) {
-        const bool next = tile + kShortWaves < n_tiles;
+    for (int tile = wave; tile < n_tiles; tile += WAVES) {
+        const bool next = tile + WAVES < n_tiles;
         const int kt = kt0 + 32 * tile;
         wait_vmcnt<Stages::kLoads>();     // K has landed, V may still be in flight
         if constexpr (KROT) {
@@ -296,7 +332,7 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) s_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(ks_ + (k_row ^ (ks << 5))), qf[ks], s_acc);
         Stages::reads_done();
-        if (next) issue_k(tile + kShortWaves);
+        if (next) issue_k(tile + WAVES);
         // rows of the accumulator are keys kt + 8 a + 4 g + c, the column is this lane's query
         if (__any((kt < klo) || (kt + 32 > khi))) {
             const int rel0 = kt + 4 * g - klo;
@@ -333,7 +369,7 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
             for (int dt = 0; dt < DT; ++dt)
                 o_acc[dt] = mfma_32x32x16(tr_pair(vs_ + (h0 ^ (dt << 6)) + 16 * m * RB, vs_ + (h1 ^ (dt << 6)) + 16 * m * RB), pf[m], o_acc[dt]);
         Stages::reads_done();
-        if (next) issue_v(tile + kShortWaves);
+        if (next) issue_v(tile + WAVES);
     }
     // ---- merge
     l_i = pair_sum(l_i);
@@ -341,9 +377,9 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
     __syncthreads();
     float M = -INFINITY, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < kShortWaves; ++w) M = fmaxf(M, m_lds[w][l32]);
+    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, m_lds[w][l32]);
 #pragma unroll
-    for (int w = 0; w < kShortWaves; ++w) L += m_lds[w][l32] == -INFINITY ? 0.f : l_lds[w][l32] * fast_exp2(m_lds[w][l32] - M);
+    for (int w = 0; w < WAVES; ++w) L += m_lds[w][l32] == -INFINITY ? 0.f : l_lds[w][l32] * fast_exp2(m_lds[w][l32] - M);
     const float f = m_i == -INFINITY ? 0.f : fast_exp2(m_i - M);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -353,9 +389,11 @@ __global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 4 : 2) void attn_short_
     short_store<D>(red, wave, lane, o_acc);
     __syncthreads();
     if (tq >= p.total_q) return;
-    float x[DT][4];
-    short_sum<D>(red, wave, lane, x);
-    short_write<D>(p.o + (int64_t)tq * p.o_st + (int64_t)head * p.o_sh + 8 * wave + 4 * g, x, L > 0.f ? 1.0f / L : 0.f);
+    float x[4 / WAVES][DT][4];
+    short_sums<D, WAVES>(red, wave, lane, x);
+#pragma unroll
+    for (int j = 0; j < 4 / WAVES; ++j)
+        short_write<D>(p.o + (int64_t)tq * p.o_st + (int64_t)head * p.o_sh + 8 * (wave * (4 / WAVES) + j) + 4 * g, x[j], L > 0.f ? 1.0f / L : 0.f);
     if (wave == 0 && g == 0 && p.lse != nullptr)
         p.lse[(int64_t)head * p.total_q + tq] = L > 0.f ? (M + __log2f(L)) * 0.6931471805599453f : INFINITY;
 }
@@ -394,14 +432,12 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_short_kernel(const AttnPar
 }
 
 // ---- backward: dQ of 32 queries of one head ------------------------------------------------------------------
-template <int D> constexpr int kShortRed = kShortWaves * 16 * (D / 32) * 64 * 4;      // an accumulator set of every wavefront
+template <int D, int WAVES> constexpr int kShortDqSmem = ShortStages<D, WAVES>::kSmem < kShortRed<D, WAVES> ? kShortRed<D, WAVES> : ShortStages<D, WAVES>::kSmem;
 
-template <int D> constexpr int kShortDqSmem = ShortStages<D>::kSmem > kShortRed<D> ? ShortStages<D>::kSmem : kShortRed<D>;
-
-template <int D, bool KEEP_DELTA>
+template <int D, int WAVES, bool KEEP_DELTA>
 __device__ __forceinline__ void short_dq_block(const AttnParams& p, char* smem, int block) {
     constexpr int KS = D / 16, DT = D / 32;
-    using Stages = ShortStages<D>;
+    using Stages = ShortStages<D, WAVES>;
     using Tile = LdsTile<D>;
     constexpr int RB = Tile::RB;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
@@ -453,8 +489,8 @@ __device__ __forceinline__ void short_dq_block(const AttnParams& p, char* smem, 
     Tile::tr_bases(lane, h0, h1);
     const int a_row = Tile::row_base(l32, g);
     if (wave < n_tiles) { issue_v(wave); issue_k(wave); }
-    for (int tile = wave; tile < n_tiles; tile += kShortWaves) {
-        const bool next = tile + kShortWaves < n_tiles;
+    for (int tile = wave; tile < n_tiles; tile += WAVES) {
+        const bool next = tile + WAVES < n_tiles;
         const int kt = kt0 + 32 * tile;
         wait_vmcnt<0>();
         f32x16_t s_acc, dp_acc;
@@ -466,7 +502,7 @@ __device__ __forceinline__ void short_dq_block(const AttnParams& p, char* smem, 
             dp_acc = mfma_32x32x16(*reinterpret_cast<const elem8_t*>(vs_ + (a_row ^ (ks << 5))), dof[ks], dp_acc);
         }
         Stages::reads_done();
-        if (next) issue_v(tile + kShortWaves);
+        if (next) issue_v(tile + WAVES);
         if (__any((kt < klo) || (kt + 32 > khi))) {
             const int rel0 = kt + 4 * g - klo;
             const unsigned len = (unsigned)(khi - klo);
@@ -483,39 +519,44 @@ __device__ __forceinline__ void short_dq_block(const AttnParams& p, char* smem, 
             for (int dt = 0; dt < DT; ++dt)
                 dq_acc[dt] = mfma_32x32x16(tr_pair(ks_ + (h0 ^ (dt << 6)) + 16 * m * RB, ks_ + (h1 ^ (dt << 6)) + 16 * m * RB), dsf[m], dq_acc[dt]);
         Stages::reads_done();
-        if (next) issue_k(tile + kShortWaves);
+        if (next) issue_k(tile + WAVES);
     }
     __syncthreads();                      // every wavefront is done with its stages
     float* red = reinterpret_cast<float*>(smem);
     short_store<D>(red, wave, lane, dq_acc);
     __syncthreads();
     if (tq >= p.total_q) return;
-    float x[DT][4];
-    short_sum<D>(red, wave, lane, x);
+    float x[4 / WAVES][DT][4];
+    short_sums<D, WAVES>(red, wave, lane, x);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int j = 0; j < 4 / WAVES; ++j) {
+        const int a = wave * (4 / WAVES) + j;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) x[dt][c] *= p.scale;
-    if constexpr (D == 64 || D == 128) {
-        if (p.unrotate != 0) short_unrotate<D>(x, p, p.pos_q[tq], wave, g);
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[j][dt][c] *= p.scale;
+        if constexpr (D == 64 || D == 128) {
+            if (p.unrotate != 0) short_unrotate<D>(x[j], p, p.pos_q[tq], a, g);
+        }
+        short_write<D>(p.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh + 8 * a + 4 * g, x[j], 1.0f);
     }
-    short_write<D>(p.dq + (int64_t)tq * p.q_st + (int64_t)head * p.q_sh + 8 * wave + 4 * g, x, 1.0f);
 }
 
 // ---- backward: dK and dV of 32 keys of one KV head (of one share of its query heads: hsplit) ------------------------------
 // The wavefronts take (query tile, query head) pairs in turn.  OWN_DELTA: they form delta themselves, from the fragments of the dO tile and of
 // an O tile (up to 64 features) or of O rows in registers, which a compute unit's only workgroup has enough of; otherwise a launch in front has left it.
-template <int D, bool OWN_DELTA> using ShortDkdvStages = ShortStages<D, D <= 64 ? 1 : 2, OWN_DELTA && D <= 64 ? 3 : 2>;
-template <int D, bool OWN_DELTA>
-constexpr int kShortDkdvSmem = ShortDkdvStages<D, OWN_DELTA>::kSmem > kShortRed<D> ? ShortDkdvStages<D, OWN_DELTA>::kSmem : kShortRed<D>;
+template <int D, int WAVES, bool OWN_DELTA> using ShortDkdvStages = ShortStages<D, WAVES, D <= 64 ? 1 : 2, OWN_DELTA && D <= 64 ? 3 : 2>;
+template <int D, int WAVES, bool OWN_DELTA>
+constexpr int kShortDkdvSmem = ShortDkdvStages<D, WAVES, OWN_DELTA>::kSmem < kShortRed<D, WAVES> ? kShortRed<D, WAVES>
+                                                                                                          : ShortDkdvStages<D, WAVES, OWN_DELTA>::kSmem;
 
 // stat_lds: 32 log-sum-exps, 32 deltas of each wavefront's tile
-template <int D, bool OWN_DELTA>
+template <int D, int WAVES, bool OWN_DELTA>
 __device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem, float (*stat_lds)[64], int block) {
     constexpr int KS = D / 16, DT = D / 32;
     constexpr int STAGES = D <= 64 ? 1 : 2;
     constexpr bool O_TILE = OWN_DELTA && D <= 64, O_ROWS = OWN_DELTA && D > 64;
-    using Stages = ShortDkdvStages<D, OWN_DELTA>;
+    using Stages = ShortDkdvStages<D, WAVES, OWN_DELTA>;
     using Tile = LdsTile<D>;
     constexpr int RB = Tile::RB;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
@@ -574,8 +615,8 @@ __device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem
         if constexpr (O_ROWS) load_o(wave);
     }
     int buf = 0;
-    for (int iter = wave; iter < iters; iter += kShortWaves) {
-        const bool next = iter + kShortWaves < iters;
+    for (int iter = wave; iter < iters; iter += WAVES) {
+        const bool next = iter + WAVES < iters;
         if (!OWN_DELTA || g == 0) stat_lds[wave][lane] = stat * stat_scale;
         if constexpr (O_ROWS) {                           // waited for here, or the wait would take the next step's tiles along
 #pragma unroll
@@ -583,7 +624,7 @@ __device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem
         }
         const char *qs_ = st.first(buf), *ds_ = st.second(buf);
         if (STAGES == 2 && next) {
-            issue(iter + kShortWaves, buf ^ 1);
+            issue(iter + WAVES, buf ^ 1);
             wait_vmcnt<2 * Stages::kLoads>();             // this step's tiles and rows have landed, the next one's tiles may be in flight
         } else {
             wait_vmcnt<0>();
@@ -601,7 +642,7 @@ __device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem
             if (g == 1) stat_lds[wave][lane] = delta;
             __builtin_amdgcn_sched_barrier(0);            // before the accumulators are live: 168 registers at 64 features
             if constexpr (O_ROWS) {
-                if (next) load_o(iter + kShortWaves);
+                if (next) load_o(iter + WAVES);
             }
         }
         const int qs = qt0 + 32 * (iter / hpw);
@@ -645,53 +686,58 @@ __device__ __forceinline__ void short_dkdv_block(const AttnParams& p, char* smem
             }
         Stages::reads_done();
         if (STAGES == 2) buf ^= 1;
-        else if (next) issue(iter + kShortWaves, 0);
+        else if (next) issue(iter + WAVES, 0);
     }
     __syncthreads();                      // every wavefront is done with its stages
     float* red = reinterpret_cast<float*>(smem);
     short_store<D>(red, wave, lane, dk_acc);
     __syncthreads();
-    float dk[DT][4], dv[DT][4];
-    short_sum<D>(red, wave, lane, dk);
+    float dk[4 / WAVES][DT][4], dv[4 / WAVES][DT][4];
+    short_sums<D, WAVES>(red, wave, lane, dk);
     __syncthreads();
     short_store<D>(red, wave, lane, dv_acc);
     __syncthreads();
     if (key >= p.total_k) return;
-    short_sum<D>(red, wave, lane, dv);
+    short_sums<D, WAVES>(red, wave, lane, dv);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int j = 0; j < 4 / WAVES; ++j) {
+        const int a = wave * (4 / WAVES) + j;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) dk[dt][c] *= p.scale;
-    if (p.hsplit > 1) {
-        const int64_t row = (((int64_t)hs * p.total_k + key) * p.nkv + kvh) * D + 8 * wave + 4 * g;
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            *reinterpret_cast<f32x4_t*>(p.dk_part + row + 32 * dt) = f32x4_t{dk[dt][0], dk[dt][1], dk[dt][2], dk[dt][3]};
-            *reinterpret_cast<f32x4_t*>(p.dv_part + row + 32 * dt) = f32x4_t{dv[dt][0], dv[dt][1], dv[dt][2], dv[dt][3]};
+            for (int c = 0; c < 4; ++c) dk[j][dt][c] *= p.scale;
+        if (p.hsplit > 1) {
+            const int64_t row = (((int64_t)hs * p.total_k + key) * p.nkv + kvh) * D + 8 * a + 4 * g;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                *reinterpret_cast<f32x4_t*>(p.dk_part + row + 32 * dt) = f32x4_t{dk[j][dt][0], dk[j][dt][1], dk[j][dt][2], dk[j][dt][3]};
+                *reinterpret_cast<f32x4_t*>(p.dv_part + row + 32 * dt) = f32x4_t{dv[j][dt][0], dv[j][dt][1], dv[j][dt][2], dv[j][dt][3]};
+            }
+            continue;
         }
-        return;
+        if constexpr (D == 64 || D == 128) {
+            if (p.unrotate != 0) short_unrotate<D>(dk[j], p, p.pos_k[key], a, g);
+        }
+        short_write<D>(p.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh + 8 * a + 4 * g, dk[j], 1.0f);
+        short_write<D>(p.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh + 8 * a + 4 * g, dv[j], 1.0f);
     }
-    if constexpr (D == 64 || D == 128) {
-        if (p.unrotate != 0) short_unrotate<D>(dk, p, p.pos_k[key], wave, g);
-    }
-    short_write<D>(p.dk + (int64_t)key * p.dk_st + (int64_t)kvh * p.dk_sh + 8 * wave + 4 * g, dk, 1.0f);
-    short_write<D>(p.dv + (int64_t)key * p.dv_st + (int64_t)kvh * p.dv_sh + 8 * wave + 4 * g, dv, 1.0f);
 }
 
 // Both in one launch: dK / dV blocks, the longer ones, in the first n_dkdv workgroups, dQ blocks in the others.
-template <int D, bool OWN_DELTA>
-__global__ __launch_bounds__(64 * kShortWaves, D <= 64 ? 3 : 1) void attn_short_bwd_kernel(const AttnParams p, int n_dkdv) {
-    __shared__ __attribute__((aligned(1024))) char smem[kShortDqSmem<D> > kShortDkdvSmem<D, OWN_DELTA> ? kShortDqSmem<D> : kShortDkdvSmem<D, OWN_DELTA>];
-    __shared__ __attribute__((aligned(16))) float stat_lds[kShortWaves][64];
-    if ((int)blockIdx.x < n_dkdv) short_dkdv_block<D, OWN_DELTA>(p, smem, stat_lds, blockIdx.x);
-    else short_dq_block<D, false>(p, smem, blockIdx.x - n_dkdv);
+template <int D, int WAVES, bool OWN_DELTA>
+__global__ __launch_bounds__(64 * WAVES, D <= 64 ? 3 : 1) void attn_short_bwd_kernel(const AttnParams p, int n_dkdv) {
+    constexpr int kDq = kShortDqSmem<D, WAVES>, kDkdv = kShortDkdvSmem<D, WAVES, OWN_DELTA>;
+    __shared__ __attribute__((aligned(1024))) char smem[kDq > kDkdv ? kDq : kDkdv];
+    __shared__ __attribute__((aligned(16))) float stat_lds[WAVES][64];
+    if ((int)blockIdx.x < n_dkdv) short_dkdv_block<D, WAVES, OWN_DELTA>(p, smem, stat_lds, blockIdx.x);
+    else short_dq_block<D, WAVES, false>(p, smem, blockIdx.x - n_dkdv);
 }
 
 // dQ blocks alone, two to a compute unit; they leave delta for dK / dV
 template <int D>
-__global__ __launch_bounds__(64 * kShortWaves, 2) void attn_short_dq_kernel(const AttnParams p) {
-    __shared__ __attribute__((aligned(1024))) char smem[kShortDqSmem<D>];
-    short_dq_block<D, true>(p, smem, blockIdx.x);
+__global__ __launch_bounds__(256, 2) void attn_short_dq_kernel(const AttnParams p) {
+    __shared__ __attribute__((aligned(1024))) char smem[kShortDqSmem<D, 4>];
+    short_dq_block<D, 4, true>(p, smem, blockIdx.x);
 }
 
 }  // namespace

@@ -2,6 +2,7 @@
 each pinned by its flag: against the oracle, and with the rotary inside against each other."""
 
 import math
+import random
 
 import pytest
 import torch
@@ -272,3 +273,47 @@ def test_float32_step_with_kept_scores_in_a_graph():
         graph.replay()
         assert all(torch.equal(a, b) for a, b in zip(step(), want))
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# blocks of two wavefronts, and which way goes to them: a last block that is not whole, empty documents, one much longer than the others, q of another
+# length than k, rotary on the load of q
+@pytest.mark.parametrize("nq,nkv,d,total,docs,causal,fwd,bwd", [
+    (24, 24, 64, 2081, 9, True, 2, 2), (24, 24, 64, 2049, 9, False, 4, 2), (16, 4, 128, 2600, 13, True, 2, 4), (12, 12, 32, 2500, 20, False, 4, 2),
+    (12, 12, 64, 2047, 6, True, 4, 2), (12, 12, 64, 2047, 5, True, 4, 4), (16, 16, 96, 2561, 30, True, 2, 4), (32, 32, 64, 4096, 40, True, 2, 2),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["self", "cross", "rotary"])
+def test_blocks_of_two_wavefronts(nq, nkv, d, total, docs, causal, fwd, bwd, dtype, kind):
+    print(f"case two wavefronts nq={nq} nkv={nkv} d={d} total={total} docs={docs} causal={causal} {dtype} {kind}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are per compute unit; these sizes are for 256")
+    if kind == "rotary" and d not in (64, 128):
+        pytest.skip("rotary inside: 64 and 128 features")
+    g = torch.Generator(device=DEV).manual_seed(total)
+    cut = [0] + sorted(random.Random(docs).sample(range(1, total), docs - 2)) + [total, total]              # the last document is empty
+    cu = torch.tensor(cut, dtype=torch.int32, device=DEV)
+    cu_k = torch.clamp(cu, max=total - 40) if kind == "cross" else cu
+    total_k = int(cu_k[-1])
+    q, do = (torch.randn(total, nq, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    k, v = (torch.randn(total_k, nkv, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    forward = backward = {}
+    if kind == "rotary":
+        tabs = oracle.rotary_tables(d, total, 10000, dtype)
+        cos, sin, pos = tabs.cos.to(DEV).view(total, d), tabs.sin.to(DEV).view(total, d), torch.arange(total, device=DEV)
+        k = ops.rotary_embedding(k, cos, sin, pos, total)
+        forward, backward = dict(rotary=(cos, sin, pos, None), return_rotated_q=True), dict(rotary=(cos, sin, pos, pos))
+    out = []
+    for flags in (SHORT, TILED):
+        names = []
+        run = lambda: ops.attention_forward(q, k, v, cu, cu_k, causal, None, flags=flags, **forward)
+        o, lse, *rotated = run()
+        qr = rotated[0] if rotated else q
+        grads = lambda: ops.attention_backward(do, qr, k, v, o, lse, cu, cu_k, causal, None, flags=flags, **backward)
+        out.append([o, *rotated, *grads()])
+        if flags == SHORT:
+            names = launched(lambda: (run(), grads()))
+            assert any(f"attn_short_fwd_kernel<{d}, {1 if kind == 'rotary' else 0}, false, {fwd}>" in n for n in names), names
+            assert any(f"attn_short_bwd_kernel<{d}, {bwd}, " in n for n in names), names
+    for i, (a, b) in enumerate(zip(*out)):
+        # as above: the two round the same P and dS and their own results
+        assert float((a.float() - b.float()).norm()) <= 2.0 ** (-6 if dtype == torch.bfloat16 else -9) * float(b.float().norm()) + 1e-6, i
