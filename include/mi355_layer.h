@@ -63,7 +63,7 @@ int mi_check_device(void);
  * computed by one call, mostly in one launch.  Pointers 16-byte aligned, leading dimensions and the contiguous extent of every operand
  * multiples of 8 elements (4 for fp32), n a multiple of 4.  m == 0 is not an error.
  * A call of 16-bit types with a product of more than 3 GFLOP whose ldc and ldadd are multiples of 8 takes larger blocks (mi_gemm, which
- * cannot split a contraction, if they are enough for the chip).  In such a call of
+ * cannot split a contraction, if they are enough for the chip), and so do smaller ones that they serve better.  In a call of more than 3 GFLOP of
  * mi_gemm_with_workspace n may be anything, the extents of contraction-major operands too (leading dimensions cover whole vectors), and with q_kmajor the k of a P with
  * contiguous contraction indices, if the elements up to the next multiple of 8 in its rows are finite.  With a workspace (16-byte
  * aligned, mi_gemm_workspace_bytes) a product of few blocks and a long contraction is split over the chip; of several problems only

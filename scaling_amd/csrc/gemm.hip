@@ -289,12 +289,22 @@ template <typename T> bool few_rows(const mi_gemm_problem* in, int count, mi_row
     return true;
 }
 
-// Calls of 16-bit types with a product of more than 3 GFLOP take the larger blocks of gemm_wide.hip: 1024 x 1024 x 1024 alone 9 us here and
-// 11.5 there, 4084 x 1024 x 1024 34 and 13.5.  What follows a ragged extent inside its last vector meets zeros there (rows of Q past the
+// Calls of 16-bit types with a product of more than 3 GFLOP take the larger blocks of gemm_wide.hip, and below, of 128 rows and more:
+//   * gradients, once there are 64 x 64 blocks of weight and input gradient for every compute unit: a block here walks its contraction (tokens; output
+//     features) at half the speed.  us, here and there, input and weight gradient of rows x in -> out: 2048 x 768 -> 768 22.7 / 15.7, 512 x 1024 -> 1024 11.5 / 9.7,
+//     1024 x 1024 -> 512 12.2 / 9.9, 4096 x 256 -> 256 34 / 18; with fewer blocks level or slower (2048 x 256 -> 512 13.0 / 14.7, 512 x 512 -> 1024 9.0 / 9.4), and with
+//     nothing but short contractions (256 x 2048 -> 256 5.7 / 6.2).  Of 212 pairs of 0.1 - 3 GFLOP the rule takes 131, 1.03 - 3.2 x, mean 1.36, and one of .95;
+//   * forward products from 1.6 GFLOP on that give three quarters of the compute units such a block: 2048 x 768 -> 768 10.2 / 8.6, 1024 x 1024 -> 1024 10.3 / 9.6, 512 x 768 -> 2048
+//     8.7 / 8.4 (below: 512 x 1024 -> 1024 7.8 / 9.4; few long chains: 1024 x 2048 -> 512 13.3 / 14.9);
+//   * one forward product over 4096 and more with room to split it: 512 x 4096 -> 512 17.9 / 15.4, 256 x 4096 -> 256 16.6 / 12.4.
+// Only whole extents there, as the kernels of this file take them.  What follows a ragged extent inside its last vector meets zeros there (rows of Q past the
 // contraction) or unstored results (`ragged`: the entry point allows it); rows must not overlap and a step of them has to be addressable in 31 bits.
-bool wide(const mi_gemm_problem* in, int count, int dtype, bool ragged) {
+bool wide(const mi_gemm_problem* in, int count, int dtype, bool ragged, bool can_split) {
     if (dtype != MI_BF16 && dtype != MI_F16) return false;
-    bool large = false;
+    bool large = false, plain = true, forward = true, weights = false, long_chain = can_split && count == 1;     // plain: at least 128 rows, whole extents
+    double work = 0;
+    int longest = 0;
+    int64_t blocks = 0;                                    // of 64 x 64
     for (int i = 0; i < count; ++i) {
         const mi_gemm_problem& a = in[i];
         if (a.m < 0 || a.n <= 0 || a.n_segments < 1 || a.n_segments > kMaxSegments || !a.c || !mi_aligned16(a.c) || a.ldc % 8 ||
@@ -306,10 +316,21 @@ bool wide(const mi_gemm_problem* in, int count, int dtype, bool ragged) {
             if (!g.p || !g.q || g.k <= 0 || !mi_aligned16(g.p) || !mi_aligned16(g.q) || g.ldp % 8 || g.ldq % 8 || g.ldp < (ep + 7LL) / 8 * 8 ||
                 g.ldq < (eq + 7LL) / 8 * 8 || g.ldp >= (1 << 22) || g.ldq >= (1 << 22) || (!a.q_kmajor && g.k % 8) || (!ragged && (a.n % 4 || ep % 8 || eq % 8)))
                 return false;
-            large = large || 2.0 * a.m * (double)a.n * g.k > 3e9;
+            const double part = 2.0 * a.m * (double)a.n * g.k;
+            large = large || part > 3e9;
+            work += part;
+            longest = std::max(longest, g.k);
+            plain = plain && a.n % 4 == 0 && ep % 8 == 0 && eq % 8 == 0;
         }
+        plain = plain && (a.p_kmajor ? a.segments[0].k : a.m) >= 128;
+        forward = forward && !a.q_kmajor;
+        weights = weights || a.p_kmajor;
+        long_chain = long_chain && a.n_segments == 1 && a.segments[0].k >= 4096;
+        blocks += (int64_t)((a.m + 63) / 64) * ((a.n + 63) / 64);
     }
-    return large;
+    if (large || !plain) return large;
+    const int64_t units = mi_compute_units();
+    return weights ? blocks >= units && longest >= 512 : (work >= 1.6e9 && 4 * blocks >= 3 * units) || (forward && long_chain);
 }
 
 int launch_wide(const mi_gemm_problem* in, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
@@ -496,19 +517,19 @@ extern "C" int mi_column_sum(const void* x, int64_t row_stride, int64_t n_rows, 
 
 extern "C" int mi_gemm_with_workspace(const mi_gemm_problem* problems, int count, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
     if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
-    if (wide(problems, count, dtype, true)) return launch_wide(problems, count, dtype, workspace, workspace_bytes, (hipStream_t)stream);
+    if (wide(problems, count, dtype, true, workspace != nullptr && workspace_bytes > 0)) return launch_wide(problems, count, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
     return MI_OK;
 }
 
 extern "C" int mi_gemm(const mi_gemm_problem* problems, int count, int dtype, void* stream) {
     if (!problems || count < 1 || count > kMaxProblems) return mi_fail(MI_E_NULL, "gemm: 1 .. %d problems, got %d", kMaxProblems, count);
-    if (wide(problems, count, dtype, false) && !few_blocks(problems, count)) return launch_wide(problems, count, dtype, nullptr, 0, (hipStream_t)stream);
+    if (wide(problems, count, dtype, false, false) && !few_blocks(problems, count)) return launch_wide(problems, count, dtype, nullptr, 0, (hipStream_t)stream);
     MI_DISPATCH_DTYPE(dtype, return launch<T>(problems, count, (hipStream_t)stream));
     return MI_OK;
 }
 
 extern "C" size_t mi_gemm_workspace_bytes(const mi_gemm_problem* problems, int count, int dtype) {
-    if (!problems || count < 1 || count > kMaxProblems || !wide(problems, count, dtype, true)) return 0;
+    if (!problems || count < 1 || count > kMaxProblems || !wide(problems, count, dtype, true, true)) return 0;
     return mi_gemm_wide_plan(problems, count, (size_t)1 << 30, mi_compute_units()).workspace_bytes;
 }

@@ -725,3 +725,31 @@ def test_chains_shorter_than_the_stages_of_a_block(dtype):
         for k, (p, q, c, _, _) in zip(ks, results):
             pd, qd = p.double(), q.double()
             _close(f"layout {layout} k {k}", c, (pd @ qd.t()).cpu(), (pd.abs() @ qd.abs().t()).cpu(), k, dtype)
+
+
+# both sides of the lines between the two kernels below 3 GFLOP: blocks of gradients, work and blocks of a forward product, a contraction that is split,
+# rows that end inside a block
+@pytest.mark.parametrize("rows,ins,outs,forward,backward", [
+    (2048, 256, 512, "gemm", "gemm"), (2048, 512, 256, "gemm", "wide"), (1000, 768, 1032, "gemm", "wide"), (1028, 1024, 768, "wide", "wide"), (256, 2048, 256, "gemm", "gemm"),
+    (300, 4096, 520, "wide", "wide"), (300, 4088, 520, "gemm", "wide"), (120, 4096, 520, "gemm", "gemm"), (1021, 520, 1048, "gemm", "wide"),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_large_blocks_below_three_gflop(rows, ins, outs, forward, backward, dtype):
+    print(f"case large blocks rows={rows} in={ins} out={outs} {dtype}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are per compute unit; these sizes are for 256")
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w, dy = (torch.randn(s, generator=g, device=DEV).to(dtype).requires_grad_() for s in ((rows, ins), (outs, ins), (rows, outs)))
+    b = torch.randn(outs, generator=g, device=DEV).to(dtype).requires_grad_()
+    y = ops.linear(x, w, b)
+    got = [y, *torch.autograd.grad(y, (x, w, b), dy.detach(), retain_graph=True)]
+    for kind, call in ((forward, lambda: ops.linear(x, w, b)), (backward, lambda: torch.autograd.grad(y, (x, w, b), dy.detach(), retain_graph=True))):
+        names = launched(call)
+        assert any(f"{kind}_kernel" in n for n in names) and not any(("gemm" if kind == "wide" else "wide") + "_kernel" in n for n in names), names
+    xd, wd, dyd = (t.detach().double() for t in (x, w, dy))
+    half_ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for name, a, p, q, k, add in (("y", got[0], xd, wd.t(), ins, b.detach().double()), ("dx", got[1], dyd, wd, outs, 0.0), ("dw", got[2], dyd.t(), xd, rows, 0.0),
+                                  ("db", got[3], dyd.t(), torch.ones(rows, 1, dtype=torch.float64, device=DEV), rows, 0.0)):
+        ref, mag = (p @ q).reshape(a.shape) + add, (p.abs() @ q.abs()).reshape(a.shape)
+        # one rounding of the result, k + 1 of float32 sums, the smallest step of float16
+        assert bool(((a.detach().double() - ref).abs() <= half_ulp * ref.abs() + (k + 1) * 2.0 ** -24 * (mag + abs(add)) + 2.0 ** -25).all()), name
