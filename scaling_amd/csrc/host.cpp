@@ -10,6 +10,8 @@
 // between the two.
 #include <torch/extension.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/SavedTensorHooks.h>
@@ -1154,8 +1156,8 @@ constexpr int64_t kOneNode = 1 << 19;                      // elements of x
 
 // The layer as one autograd node.  Inputs: x and the parameters in the order of `parameters`.
 struct Layer : Function<Layer> {
-    template <class F> static void parameters(const LayerCall& c, F f) {
-        const auto all = [&](const std::vector<Tensor>& w, const std::vector<OptTensor>& b, size_t first, size_t last) {
+    template <class Call, class F> static void parameters(Call& c, F f) {
+        const auto all = [&](auto& w, auto& b, size_t first, size_t last) {
             for (size_t i = first; i < last; ++i) f(w[i]);
             for (size_t i = first; i < last; ++i)
                 if (b[i].has_value()) f(*b[i]);
@@ -1186,16 +1188,30 @@ struct Layer : Function<Layer> {
         using Part = LayerCall::Part;
         const auto held = ctx->saved_data["call"].toCapsule();
         LayerCall& c = static_cast<LayerCall&>(*held);
-        variable_list grads{Tensor()};
-        std::vector<Tensor> inputs{Tensor()};
-        parameters(c, [&](const Tensor& p) { inputs.push_back(p); });
-        grads.resize(inputs.size() + 1);                   // the call
+        size_t n_inputs = 1;
+        parameters(c, [&](const Tensor&) { ++n_inputs; });
+        variable_list grads(n_inputs + 1), inputs;         // of the inputs and the call
         if (!g[0].defined()) return grads;
         const variable_list saved = ctx->get_saved_variables();
         const Tensor x = saved[0];                         // the first norm's sum
         if (at::GradMode::is_enabled()) {                  // this pass is to be differentiated again: the graph of many nodes
+            // On an alias of each input at each of its places, differentiated with respect to these alone: hooks and retained gradients of the inputs themselves,
+            // their other uses and what x was made of belong to the pass that is under way.  An alias leads to where this node's gradient of it goes.
+            const auto node = torch::autograd::get_current_node();
+            const auto alias = [&](const Tensor& t) {
+                const Tensor a = t.detach();
+                const auto& edge = node->next_edge(inputs.size());
+                if (edge.is_valid()) {
+                    const auto way = std::make_shared<torch::autograd::Identity>();
+                    way->add_next_edge(edge);
+                    torch::autograd::set_history(a, way);
+                }
+                inputs.push_back(a);
+                return a;
+            };
             LayerCall again = c;
-            again.x = inputs[0] = x;
+            again.x = alias(x);
+            parameters(again, [&](Tensor& p) { p = alias(p); });
             const Tensor y = layer_forward(again, Apart{again});
             variable_list wanted;
             for (size_t i = 0; i < inputs.size(); ++i)

@@ -631,3 +631,54 @@ def test_gradients_of_a_layer_that_is_one_node(default, dtype, options, b, s):
         p.requires_grad_(n == first)
     io.activations = x.detach()
     assert all(torch.equal(p, q) for p, q in zip(gradients(native, [parameters[first]])[0], gradients(lambda: _watched(layer, io), [parameters[first]])[0]))
+
+
+@pytest.mark.parametrize("case", ["retained", "hooks", "shared", "twice", "frozen since"])
+def test_graph_of_gradients_of_a_layer_that_is_one_node(case):
+    """Gradients with a graph of their own meet hooks, retained gradients and parameters in several places as often as those of the modules' nodes, and
+    that graph is theirs: to the bit, and where it is differentiated again up to the order of float32 sums of a few terms."""
+    layer = _layer("float32", True)
+    if case == "shared":
+        layer.post_attention_layernorm.weight = layer.input_layernorm.weight
+        layer.mlp.dense_out.bias = layer.self_attention.dense.bias
+    leaf = torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(8)).to(DEV).requires_grad_()
+    parameters = dict(layer.named_parameters())
+    dy = torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(9)).to(DEV).requires_grad_()
+    where = ["self_attention.query_key_value.weight", "mlp.dense_in.bias", "post_attention_layernorm.weight"]
+
+    def gradients(forward):
+        layer.zero_grad(set_to_none=True)
+        leaf.grad = None
+        x = leaf * layer.input_layernorm.weight if case in ("retained", "twice") else leaf
+        handles = [p.register_hook(lambda g: 2 * g) for p in (x, *(parameters[n] for n in where))] if case == "hooks" else []
+        if case == "retained":
+            x.retain_grad()
+        y = forward(x)
+        if case == "twice":
+            y = forward(y)
+        if case == "frozen since":                         # its gradient is wanted all the same: what the graph was made with counts
+            parameters[where[1]].requires_grad_(False)
+        if case in ("retained", "frozen since"):
+            torch.autograd.backward(y, dy, create_graph=True)
+            got = [x.grad, *(p.grad for p in (leaf, *parameters.values()) if p.requires_grad)]
+        else:
+            got = list(torch.autograd.grad(y, [leaf, *parameters.values()], dy, create_graph=True))
+        parameters[where[1]].requires_grad_(True)
+        connected = [g for g in got if g.requires_grad]
+        again = torch.autograd.grad(sum((g * torch.cos(g.detach())).sum() for g in connected), [leaf, dy, *parameters.values()], allow_unused=True)
+        for handle in handles:
+            handle.remove()
+        for p in (x, leaf, *parameters.values()):
+            p.grad = None
+        return [g.detach() for g in got], [g.requires_grad for g in got], again
+
+    def native(x):
+        y = layer(_io(x)).activations
+        assert y.grad_fn.name().endswith("::Layer>")
+        return y
+    (got, graph, again), (want, want_graph, want_again) = gradients(native), gradients(lambda x: _watched(layer, _io(x)))
+    assert all(torch.equal(p, q) for p, q in zip(got, want)) and graph == want_graph and any(graph)
+    assert [g is None for g in again] == [g is None for g in want_again]
+    for p, q in zip(again, want_again):
+        if q is not None:
+            assert (p - q).abs().max() <= 1e-5 * q.abs().max()
