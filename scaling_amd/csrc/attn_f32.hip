@@ -195,8 +195,9 @@ __device__ __forceinline__ void cols_product(f32x16_t (&acc)[D / 32], const char
 // The two products of a kernel whose wavefronts have a SIMD each, with the rest of its work between them: between(j) behind every fourth product of rows
 // and behind the DT products of a row of columns.  They are inline assembly because the compiler keeps the gradients' accumulators in vector registers otherwise
 // and moves all of them to accumulation registers and back in every step; C tiles that vector instructions read are in vector registers.  What the compiler
-// does not see then are waits between a product and whoever reads its result: between() may read the C tile of the product before this one
-// (four products of 64 cycles lie between), and `settled` is for the end.
+// does not see then are waits between a product and whoever reads its result (18 states): between() may read the C tile of the stage before, `last`, which
+// passes through an empty statement behind the first products of this stage (four, or DT, of 16 states each), so that no read of it moves in front of them; and
+// the gradients pass through `settled` at the end.
 __device__ __forceinline__ void mma_v(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
 __device__ __forceinline__ void mma_v0(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b)); }
 __device__ __forceinline__ void mma_acc(f32x16_t& c, float a, float b) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
@@ -205,11 +206,19 @@ __device__ __forceinline__ void clear_acc(f32x16_t& c) {
     for (int r = 0; r < 16; ++r) c[r] = 0.f;
     asm volatile("" : "+a"(c));
 }
-__device__ __forceinline__ void settled() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+struct NoTile {};
+__device__ __forceinline__ void behind(f32x16_t& last) { asm volatile("" : "+v"(last)); }
+__device__ __forceinline__ void behind(NoTile) {}
+template <int DT> __device__ __forceinline__ void settled(f32x16_t (&x)[DT], f32x16_t (&y)[DT]) {
+    asm volatile("s_nop 15\n\ts_nop 15" : "+a"(x[0]), "+a"(y[0]));
+#pragma unroll
+    for (int dt = 1; dt < DT; ++dt) asm volatile("" : "+a"(x[dt]), "+a"(y[dt]));
+}
 
 // a0, x0: the first operand, read ahead; then(): reads the one of the product behind this
-template <int D, class F, class G>
-__device__ __forceinline__ void rows_product_with(f32x16_t& c, const char* tile, int row, int g, const f32x4_t& a0, const f32x4_t (&b)[D / 8], F&& between, G&& then) {
+template <int D, class Last, class F, class G>
+__device__ __forceinline__ void rows_product_with(f32x16_t& c, const char* tile, int row, int g, const f32x4_t& a0, const f32x4_t (&b)[D / 8], Last&& last, F&& between,
+                                                  G&& then) {
     f32x4_t a[2];
     a[0] = a0;
     static_for<D / 8>([&](auto j_c) {
@@ -222,14 +231,15 @@ __device__ __forceinline__ void rows_product_with(f32x16_t& c, const char* tile,
             if constexpr (j == 0 && i == 0) mma_v0(c, a[0][0], b[0][0]);
             else mma_v(c, a[j & 1][i], b[j][i]);
         });
+        if constexpr (j == 0) behind(last);
         between(j_c);
         __builtin_amdgcn_sched_barrier(0);
     });
 }
 
-template <int D, class F, class G>
+template <int D, class Last, class F, class G>
 __device__ __forceinline__ void cols_product_with(f32x16_t (&acc)[D / 32], const char* tile, int row0, const float (&x0)[D / 32], const f32x16_t& x, int l32, int g,
-                                                  F&& between, G&& then) {
+                                                  Last&& last, F&& between, G&& then) {
     constexpr int DT = D / 32;
     float a[2][DT];
 #pragma unroll
@@ -241,6 +251,7 @@ __device__ __forceinline__ void cols_product_with(f32x16_t (&acc)[D / 32], const
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) mma_acc(acc[dt], a[r & 1][dt], x[r]);
+        if constexpr (r == 0) behind(last);
         between(r_c);
         __builtin_amdgcn_sched_barrier(0);
     });
@@ -585,7 +596,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
                 f32x16_t s, dp;                   // rows = queries, column = this lane's key
                 f32x4_t row0;
                 float col0[2][DT];
-                rows_product_with<D>(s, q_s, 32 * qs + l, h, F32Tile<D>::row4(q_s, 32 * qs + l, 0, h), kf, [&](auto j) {
+                rows_product_with<D>(s, q_s, 32 * qs + l, h, F32Tile<D>::row4(q_s, 32 * qs + l, 0, h), kf, NoTile{}, [&](auto j) {
                     if (between) {
                         static_for<2 * kLoads>([&](auto n_c) {
                             constexpr int n = decltype(n_c)::value;
@@ -606,7 +617,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
                     return l4;
                 };
                 f32x4_t l4 = log2_sums(0);
-                rows_product_with<D>(dp, do_s, 32 * qs + l, h, row0, vf, [&](auto j) {
+                rows_product_with<D>(dp, do_s, 32 * qs + l, h, row0, vf, s, [&](auto j) {
                     static_for<16>([&](auto r_c) {
                         constexpr int r = decltype(r_c)::value, a = r >> 2, c = r & 3;
                         if constexpr (r * kParts / 16 == decltype(j)::value) {
@@ -620,7 +631,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
                 }, [&] { F32Tile<D>::cols(do_s, 32 * qs + acc_row(0, h), l, col0[0]); });
                 f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(delta_row);
                 float* out = KEEP ? fp.ds + ds.tile(head - first_kv * p.n_rep, qt, kb * BK + kgrp * 32) + l32 * 32 + 4 * g : nullptr;
-                cols_product_with<D>(dv_acc, do_s, 32 * qs, col0[0], s, l, h, [&](auto r_c) {
+                cols_product_with<D>(dv_acc, do_s, 32 * qs, col0[0], s, l, h, dp, [&](auto r_c) {
                     constexpr int r = decltype(r_c)::value, a = r >> 2, c = r & 3;
                     float dsv = s[r] * (dp[r] - d4[c]);
                     asm volatile("" : "+v"(dsv));
@@ -630,14 +641,14 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
                         if constexpr (a < 3) d4 = *reinterpret_cast<const f32x4_t*>(delta_row + 8 * (a + 1));
                     }
                 }, [&] { F32Tile<D>::cols(q_s, 32 * qs + acc_row(0, h), l, col0[1]); });
-                cols_product_with<D>(dk_acc, q_s, 32 * qs, col0[1], dp, l, h, [](auto) {}, [] {});
+                cols_product_with<D>(dk_acc, q_s, 32 * qs, col0[1], dp, l, h, NoTile{}, [](auto) {}, [] {});
             }
             if constexpr (NS == 1) {
                 __syncthreads();
                 issue();
             }
         }
-        settled();
+        settled(dk_acc, dv_acc);
     } else {
         for (int step = 0; step < n_steps; ++step) {
             put_stat(step);
