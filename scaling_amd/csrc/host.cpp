@@ -1046,6 +1046,7 @@ struct LayerCall : torch::CustomClassHolder {
     std::vector<Tensor> caches;                            // [k, v, ctx_len] of a prefill (rotary 1, inference) or empty
     enum Part { kNorm1, kQkv, kRotary, kAttention, kDense, kNorm2, kIn, kActivation, kOut, kParts };
     Kept parts[kParts];                                    // of a layer that is one node
+    std::vector<uint32_t> versions;                        // the same: of what a graph of its gradients is made from
     bool split() const { return !in_one || rotary == 2; }  // q, k and v reach the attention core as three
 };
 
@@ -1170,6 +1171,17 @@ struct Layer : Function<Layer> {
         all(c.rest_w, c.rest_b, 1, out);
         all(c.rest_w, c.rest_b, out, out + 1);
     }
+    static std::vector<uint32_t> versions(const LayerCall& c) {
+        std::vector<uint32_t> v;
+        const auto add = [&](const Tensor& t) {
+            if (t.defined() && !t.is_inference()) v.push_back(t._version());
+        };
+        parameters(c, add);
+        add(c.cu);
+        if (c.rotary != 0)
+            for (const OptTensor* t : {&c.pos, &c.cos, &c.sin}) add(opt(*t));
+        return v;
+    }
     static Tensor forward(AutogradContext* ctx, at::TensorList, const c10::intrusive_ptr<LayerCall>& c) {
         const Tensor y = layer_forward(*c, Together(*c, true));
         variable_list saved;
@@ -1179,6 +1191,7 @@ struct Layer : Function<Layer> {
             part.saved.clear();
         }
         c->x = Tensor();
+        c->versions = versions(*c);
         ctx->set_materialize_grads(false);
         ctx->save_for_backward(saved);
         ctx->saved_data["call"] = at::IValue::make_capsule(c);
@@ -1197,6 +1210,9 @@ struct Layer : Function<Layer> {
         if (at::GradMode::is_enabled()) {                  // this pass is to be differentiated again: the graph of many nodes
             // On an alias of each input at each of its places, differentiated with respect to these alone: hooks and retained gradients of the inputs themselves,
             // their other uses and what x was made of belong to the pass that is under way.  An alias leads to where this node's gradient of it goes.
+            // The forward pass is gone through again, so what it reads has to be what it was: biases, say, are not among what the node saves.
+            TORCH_CHECK(versions(c) == c.versions, "layer: one of the variables needed for gradient computation has been modified by an inplace operation: "
+                                                   "a parameter, the lengths, the positions or a rotary table, all of which a graph of the gradients is made from");
             const auto node = torch::autograd::get_current_node();
             const auto alias = [&](const Tensor& t) {
                 const Tensor a = t.detach();

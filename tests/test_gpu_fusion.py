@@ -682,3 +682,27 @@ def test_graph_of_gradients_of_a_layer_that_is_one_node(case):
     for p, q in zip(again, want_again):
         if q is not None:
             assert (p - q).abs().max() <= 1e-5 * q.abs().max()
+
+
+@pytest.mark.parametrize("name", ["mlp.dense_out.bias", "input_layernorm.bias", "self_attention.dense.bias", "self_attention.query_key_value.weight", "lengths"])
+def test_graph_of_gradients_of_a_layer_changed_since(name):
+    """What the forward pass read and nothing saved, changed in place before the backward pass: a graph of the gradients, which is made from it, is refused,
+    and gradients without one are those of the pass that was."""
+    layer = _layer("float32", True)
+    for n, p in layer.named_parameters():                  # nothing in front of the first projection takes a gradient: its weight is not saved
+        p.requires_grad_(not n.startswith("input_layernorm"))
+    io = _io(torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(8)).to(DEV))
+    wanted = [layer.mlp.dense_in.weight, layer.self_attention.query_key_value.bias]
+    y = layer(io).activations
+    assert y.grad_fn.name().endswith("::Layer>")
+    before = torch.autograd.grad(y.sum(), wanted, retain_graph=True)
+    torch.autograd.grad(y.sum(), wanted, create_graph=True)
+    with torch.no_grad():
+        if name == "lengths":
+            io.cumulative_seq_lengths[1] += 1
+        else:
+            layer.get_parameter(name).add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y.sum(), wanted, create_graph=True)
+    if name != "lengths":
+        assert all(torch.equal(p, q) for p, q in zip(before, torch.autograd.grad(y.sum(), wanted)))
