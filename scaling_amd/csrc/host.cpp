@@ -1228,7 +1228,10 @@ struct Layer : Function<Layer> {
             LayerCall again = c;
             again.x = alias(x);
             parameters(again, [&](Tensor& p) { p = alias(p); });
-            const Tensor y = layer_forward(again, Apart{again});
+            const Tensor y = [&] {                         // in the types of the pass that was, whatever this one is under
+                const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+                return layer_forward(again, Apart{again});
+            }();
             variable_list wanted;
             for (size_t i = 0; i < inputs.size(); ++i)
                 if (ctx->needs_input_grad(i)) wanted.push_back(inputs[i]);

@@ -706,3 +706,18 @@ def test_graph_of_gradients_of_a_layer_changed_since(name):
         torch.autograd.grad(y.sum(), wanted, create_graph=True)
     if name != "lengths":
         assert all(torch.equal(p, q) for p, q in zip(before, torch.autograd.grad(y.sum(), wanted)))
+
+
+@pytest.mark.parametrize("to", [torch.bfloat16, torch.float16])
+def test_graph_of_gradients_of_a_layer_under_autocast(to):
+    """Autocast around the backward pass alone: what the modules' nodes give under it, to the bit, and no forward pass in another type."""
+    layer = _layer("float32", True)
+    x = torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(8)).to(DEV).requires_grad_()
+    inputs = [x, *layer.parameters()]
+
+    def gradients(y):
+        with torch.autocast("cuda", dtype=to):
+            return torch.autograd.grad(y, inputs, torch.cos(y.detach()), create_graph=True)
+    y = layer(_io(x)).activations
+    assert y.grad_fn.name().endswith("::Layer>")
+    assert all(torch.equal(p, q) for p, q in zip(gradients(y), gradients(_watched(layer, _io(x)))))
