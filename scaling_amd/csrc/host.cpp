@@ -13,6 +13,7 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/graph_task.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/SavedTensorHooks.h>
 #include <ATen/hip/HIPContext.h>
@@ -81,12 +82,16 @@ int64_t row_count(const Tensor& x) { return x.size(-1) == 0 ? 0 : x.numel() / x.
 
 // Where an operation is a part of a larger node, of AutogradContext what the nodes below use of it: in the forward pass, and in the backward pass.
 struct Kept {
-    bool keeps = false;                                    // there will be a backward pass
-    size_t count = 0;
-    variable_list saved;
+    bool keeps = false;                                    // a gradient will come by here
+    std::vector<torch::autograd::SavedVariable> saved;
     decltype(AutogradContext::saved_data) saved_data;
-    void save_for_backward(variable_list t) { if (keeps) saved = std::move(t); }
+    void save_for_backward(const variable_list& tensors) {
+        if (!keeps) return;
+        saved.reserve(tensors.size());
+        for (const Tensor& t : tensors) saved.emplace_back(t, false);
+    }
     void set_materialize_grads(bool) {}
+    void give_back() { for (auto& t : saved) t.reset_data(); }
 };
 struct Replayed {
     variable_list saved;
@@ -1045,9 +1050,18 @@ struct LayerCall : torch::CustomClassHolder {
     int rotary;                                            // 0 none, 1 inside the attention core, 2 in front of it
     std::vector<Tensor> caches;                            // [k, v, ctx_len] of a prefill (rotary 1, inference) or empty
     enum Part { kNorm1, kQkv, kRotary, kAttention, kDense, kNorm2, kIn, kActivation, kOut, kParts };
-    Kept parts[kParts];                                    // of a layer that is one node
-    std::vector<uint32_t> versions;                        // the same: of what a graph of its gradients is made from
     bool split() const { return !in_one || rotary == 2; }  // q, k and v reach the attention core as three
+};
+// Of a layer that is one node, with what its gradients need: as in nodes of their own, each part looks at its tensors when its turn comes (whether they were
+// changed in place), gives them back then, and keeps none where no gradient comes by.
+struct LayerKept : LayerCall {
+    Kept parts[kParts];
+    torch::autograd::SavedVariable input;                  // x, and versions of the rest: what a graph of the gradients is made from
+    std::vector<uint32_t> versions;
+    void give_back() {
+        for (Kept& part : parts) part.give_back();
+        input.reset_data();
+    }
 };
 
 // The operations of a layer, each with a node of its own
@@ -1073,14 +1087,18 @@ struct Apart {
 
 // The same with no node of their own: what the gradients need stays in the call.  `grad`: something up to here takes a gradient
 struct Together {
-    LayerCall& c;
+    LayerKept& c;
     bool recorded, grad;
-    Together(LayerCall& call, bool recorded_) : c(call), recorded(recorded_), grad(recorded_ && call.x.requires_grad()) {}
+    Together(LayerKept& call, bool recorded_) : c(call), recorded(recorded_), grad(recorded_ && call.x.requires_grad()) {}
     void reaches(const Tensor& p) { grad = grad || (recorded && p.requires_grad()); }
+    Kept* kept(LayerCall::Part p) {
+        c.parts[p].keeps = grad;
+        return &c.parts[p];
+    }
     std::tuple<Tensor, Tensor> norm(LayerCall::Part p, const Tensor& x, const OptTensor& residual, const Tensor& w, const OptTensor& b, double eps, bool layer_norm) {
         reaches(w);
         if (b.has_value()) reaches(*b);
-        auto out = AddNorm::run(&c.parts[p], x, residual, w, b, eps, layer_norm);
+        auto out = AddNorm::run(kept(p), x, residual, w, b, eps, layer_norm);
         return {out[0], out[1]};
     }
     std::vector<Tensor> projections(LayerCall::Part p, const Tensor& x, const std::vector<Tensor>& w, const std::vector<OptTensor>& b, const OptTensor& residual) {
@@ -1092,17 +1110,17 @@ struct Together {
         }
         const bool need_dx = grad;
         for (const Tensor& t : params) reaches(t);
-        return Projections::run(&c.parts[p], x, params, residual, has_bias, c.inference, need_dx);
+        return Projections::run(kept(p), x, params, residual, has_bias, c.inference, need_dx);
     }
     variable_list rotary(const Tensor& q, const Tensor& k, int64_t s) {
-        return RotaryTwo::run(&c.parts[LayerCall::kRotary], q, k, *c.cos, *c.sin, c.pos, s, c.interleaved);
+        return RotaryTwo::run(kept(LayerCall::kRotary), q, k, *c.cos, *c.sin, c.pos, s, c.interleaved);
     }
     Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const AttnOptions& o) {
-        return attention_node_forward(&c.parts[LayerCall::kAttention], q, k, v, c.cu, Tensor(), o, grad);
+        return attention_node_forward(kept(LayerCall::kAttention), q, k, v, c.cu, Tensor(), o, grad);
     }
-    Tensor attention_qkv(const Tensor& qkv, const AttnOptions& o) { return AttentionQkv::run(&c.parts[LayerCall::kAttention], qkv, c.cu, OptTensor(), o, grad); }
-    Tensor gelu(const Tensor& x) { return Gelu::run(&c.parts[LayerCall::kActivation], x); }
-    Tensor swiglu(const Tensor& a, const Tensor& gate) { return SwiGlu::run(&c.parts[LayerCall::kActivation], a, gate); }
+    Tensor attention_qkv(const Tensor& qkv, const AttnOptions& o) { return AttentionQkv::run(kept(LayerCall::kAttention), qkv, c.cu, OptTensor(), o, grad); }
+    Tensor gelu(const Tensor& x) { return Gelu::run(kept(LayerCall::kActivation), x); }
+    Tensor swiglu(const Tensor& a, const Tensor& gate) { return SwiGlu::run(kept(LayerCall::kActivation), a, gate); }
 };
 
 template <class Operations> Tensor layer_forward(const LayerCall& c, Operations ops) {
@@ -1182,31 +1200,29 @@ struct Layer : Function<Layer> {
             for (const OptTensor* t : {&c.pos, &c.cos, &c.sin}) add(opt(*t));
         return v;
     }
-    static Tensor forward(AutogradContext* ctx, at::TensorList, const c10::intrusive_ptr<LayerCall>& c) {
+    static Tensor forward(AutogradContext* ctx, at::TensorList, const c10::intrusive_ptr<LayerKept>& c) {
         const Tensor y = layer_forward(*c, Together(*c, true));
-        variable_list saved;
-        for (Kept& part : c->parts) {                      // from here on the node alone holds them: it sees changes in place, and gives them back
-            part.count = part.saved.size();
-            saved.insert(saved.end(), part.saved.begin(), part.saved.end());
-            part.saved.clear();
-        }
+        c->input = torch::autograd::SavedVariable(c->x, false);
         c->x = Tensor();
         c->versions = versions(*c);
         ctx->set_materialize_grads(false);
-        ctx->save_for_backward(saved);
         ctx->saved_data["call"] = at::IValue::make_capsule(c);
         return y;
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         using Part = LayerCall::Part;
+        ctx->get_saved_variables();                        // raises where the graph is used up
         const auto held = ctx->saved_data["call"].toCapsule();
-        LayerCall& c = static_cast<LayerCall&>(*held);
+        LayerKept& c = static_cast<LayerKept&>(*held);
+        struct UsedUp {                                    // a pass that keeps the graph leaves everything, any other nothing
+            LayerKept& c;
+            bool kept;
+            ~UsedUp() { if (!kept) c.give_back(); }
+        } const graph{c, torch::autograd::get_current_graph_task_keep_graph()};
         size_t n_inputs = 1;
         parameters(c, [&](const Tensor&) { ++n_inputs; });
         variable_list grads(n_inputs + 1), inputs;         // of the inputs and the call
         if (!g[0].defined()) return grads;
-        const variable_list saved = ctx->get_saved_variables();
-        const Tensor x = saved[0];                         // the first norm's sum
         if (at::GradMode::is_enabled()) {                  // this pass is to be differentiated again: the graph of many nodes
             // On an alias of each input at each of its places, differentiated with respect to these alone: hooks and retained gradients of the inputs themselves,
             // their other uses and what x was made of belong to the pass that is under way.  An alias leads to where this node's gradient of it goes.
@@ -1226,7 +1242,7 @@ struct Layer : Function<Layer> {
                 return a;
             };
             LayerCall again = c;
-            again.x = alias(x);
+            again.x = alias(c.input.unpack());
             parameters(again, [&](Tensor& p) { p = alias(p); });
             const Tensor y = [&] {                         // in the types of the pass that was, whatever this one is under
                 const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
@@ -1259,9 +1275,12 @@ struct Layer : Function<Layer> {
         // Whether a gradient goes on from each operation to what comes before it
         const bool from_qkv = ctx->needs_input_grad(0) || norm1.any, from_dense = from_qkv || qkv.any, from_in = from_dense || dense.any || norm2.any,
                    from_out = from_in || in.any;
-        size_t offsets[LayerCall::kParts + 1] = {0};
-        for (int p = 0; p < LayerCall::kParts; ++p) offsets[p + 1] = offsets[p] + c.parts[p].count;
-        const auto part = [&](Part p) { return Replayed{variable_list(saved.begin() + offsets[p], saved.begin() + offsets[p + 1]), c.parts[p].saved_data, {}}; };
+        const auto part = [&](Part p) {
+            Replayed r{{}, c.parts[p].saved_data, {}};
+            for (const auto& t : c.parts[p].saved) r.saved.push_back(t.unpack());
+            if (!graph.kept) c.parts[p].give_back();
+            return r;
+        };
         const auto projections = [&](Part p, const Group& own, bool on, const variable_list& dy) {
             Replayed r = part(p);
             r.needs = own.needs;
@@ -1276,30 +1295,40 @@ struct Layer : Function<Layer> {
             std::copy(d.begin() + 2, d.begin() + 2 + own.needs.size(), grads.begin() + own.first);
             return d[0];
         };
-        const Tensor dact = projections(LayerCall::kOut, out, from_out, g);
+        Tensor d = projections(LayerCall::kOut, out, from_out, g);
         if (!from_out) return grads;
-        Replayed act = part(LayerCall::kActivation);
-        const Tensor dn2 = projections(LayerCall::kIn, in, from_in, mlp_in == 2 ? SwiGlu::gradients(&act, {dact}) : Gelu::gradients(&act, {dact}));
+        const auto activation = [&](Tensor dy) {
+            Replayed r = part(LayerCall::kActivation);
+            return mlp_in == 2 ? SwiGlu::gradients(&r, {dy}) : Gelu::gradients(&r, {dy});
+        };
+        variable_list dmany = activation(std::move(d));
+        d = projections(LayerCall::kIn, in, from_in, dmany);
+        dmany.clear();
         if (!from_in) return grads;
-        const Tensor dh = norm(LayerCall::kNorm2, norm2, g[0], dn2);
+        const Tensor dh = norm(LayerCall::kNorm2, norm2, g[0], d);
         if (!from_dense && !dense.any) return grads;
-        const Tensor dctx = projections(LayerCall::kDense, dense, from_dense, {dh});
+        d = projections(LayerCall::kDense, dense, from_dense, {dh});
         if (!from_dense) return grads;
-        const int64_t tokens = x.size(0) * x.size(1), nq = c.nq, d = c.d;
-        Replayed att = part(LayerCall::kAttention);
-        const variable_list dout{dctx.view({tokens, nq, d})};
-        variable_list dqkv = c.split() ? Attention::gradients(&att, dout) : AttentionQkv::gradients(&att, dout);
-        dqkv.resize(c.split() ? 3 : 1);
+        const int64_t tokens = dh.numel() / dh.size(-1);
+        const auto attention = [&](Tensor dctx) {
+            Replayed r = part(LayerCall::kAttention);
+            const variable_list dout{dctx.view({tokens, c.nq, c.d})};
+            variable_list dqkv = c.split() ? Attention::gradients(&r, dout) : AttentionQkv::gradients(&r, dout);
+            dqkv.resize(c.split() ? 3 : 1);
+            return dqkv;
+        };
+        dmany = attention(std::move(d));
         if (c.rotary == 2) {
             Replayed rotary = part(LayerCall::kRotary);
-            const variable_list d = RotaryTwo::gradients(&rotary, {dqkv[0], dqkv[1]});
-            std::copy(d.begin(), d.begin() + 2, dqkv.begin());
+            const variable_list two = RotaryTwo::gradients(&rotary, {dmany[0], dmany[1]});
+            std::copy(two.begin(), two.begin() + 2, dmany.begin());
         }
-        if (c.in_one && c.split()) dqkv = {at::cat(dqkv, 2)};
-        for (Tensor& t : dqkv) t = t.reshape({tokens, -1});
-        const Tensor dn1 = projections(LayerCall::kQkv, qkv, from_qkv, dqkv);
+        if (c.in_one && c.split()) dmany = {at::cat(dmany, 2)};
+        for (Tensor& t : dmany) t = t.reshape({tokens, -1});
+        d = projections(LayerCall::kQkv, qkv, from_qkv, dmany);
+        dmany.clear();
         if (!from_qkv) return grads;
-        grads[0] = norm(LayerCall::kNorm1, norm1, dh, dn1);
+        grads[0] = norm(LayerCall::kNorm1, norm1, dh, d);
         return grads;
     }
 };
@@ -1336,7 +1365,7 @@ Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, std::ve
                     (caches.empty() || caches.size() == 3),
                 "layer: bad arguments");
     if (rotary != 0) check_tables(x, d, cos, sin, interleaved, rotary == 1);
-    auto c = c10::make_intrusive<LayerCall>();
+    auto c = c10::make_intrusive<LayerKept>();
     c->x = x; c->cu = cu; c->pos = pos; c->cos = cos; c->sin = sin; c->norms = std::move(norms);
     c->eps1 = eps1; c->eps2 = eps2; c->scale = scale; c->layer_norm1 = layer_norm1; c->layer_norm2 = layer_norm2; c->in_one = in_one; c->causal = causal;
     c->interleaved = interleaved; c->inference = inference; c->qkv_w = std::move(qkv_w); c->qkv_b = std::move(qkv_b); c->rest_w = std::move(rest_w);
@@ -1351,9 +1380,8 @@ Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, std::ve
     if (!recorded || !at::GradMode::is_enabled()) return layer_forward(*c, Together(*c, false));
     // One node instead of 9 to 14, views included: the engine takes 4 us for a node beside its launches, and a small step waits for the host.  Forward and backward
     // of 256 x 256, float32: 354 us with nodes of their own, 286 so; 512 x 1024, bf16: 430 and 380 (on a slower host); 1000 x 1024, where the device is what a step
-    // waits for: 370 and 370.  Nodes of their own give back what they keep one by one (512 x 1024: 6 MiB above the start of the step at the most, 28 so).
+    // waits for: 370 and 370.  What the parts keep is given back one by one either way.
     if (x.numel() > kOneNode || (c->qkv_w.size() == 1 && !in_one)) return layer_forward(*c, Apart{*c});
-    for (Kept& part : c->parts) part.keeps = true;
     return Layer::apply(at::TensorList(inputs), c);
 }
 

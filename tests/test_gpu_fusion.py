@@ -721,3 +721,53 @@ def test_graph_of_gradients_of_a_layer_under_autocast(to):
     y = layer(_io(x)).activations
     assert y.grad_fn.name().endswith("::Layer>")
     assert all(torch.equal(p, q) for p, q in zip(gradients(y), gradients(_watched(layer, _io(x)))))
+
+
+@pytest.mark.parametrize("default", [False, True])
+@pytest.mark.parametrize("trained", ["everything", "mlp.dense_out.weight", "mlp.dense_in.weight"])
+def test_memory_of_a_layer_that_is_one_node(default, trained):
+    """What is kept for the backward pass, and the most that is held during it, beside the modules' nodes: no more than x, which a graph of the gradients would
+    need, and the gradient that goes past the MLP."""
+    layer = _layer("bfloat16", default)
+    if trained != "everything":
+        layer.requires_grad_(False).get_parameter(trained).requires_grad_()
+    x = torch.randn(8, 256, 256, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(DEV)
+    io, dy = _io(x), torch.randn(8, 256, 256, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(DEV)
+
+    def held(forward):
+        layer.zero_grad(set_to_none=True)
+        torch.cuda.synchronize()
+        start = torch.cuda.memory_allocated()
+        y = forward()
+        kept = torch.cuda.memory_allocated() - start
+        torch.cuda.reset_peak_memory_stats()
+        torch.autograd.backward(y, dy)
+        return kept, torch.cuda.max_memory_allocated() - start
+
+    def native():
+        y = layer(io).activations
+        assert y.grad_fn.name().endswith("::Layer>")
+        return y
+    for forward in (native, lambda: _watched(layer, io)):  # workspaces
+        held(forward)
+    (kept, most), (want, want_most) = held(native), held(lambda: _watched(layer, io))
+    size = x.numel() * x.element_size()
+    assert kept <= want + size and most <= want_most + 2 * size, (kept / size, want / size, most / size, want_most / size)
+
+
+def test_parts_of_a_layer_that_is_one_node_look_at_their_own():
+    """A weight changed in place since the forward pass is refused by gradients that take it, and by no others; a graph is used up once."""
+    layer = _layer("bfloat16", False)
+    x = torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(DEV).requires_grad_()
+    y = layer(_io(x)).activations
+    assert y.grad_fn.name().endswith("::Layer>")
+    wanted = [layer.mlp.dense_out.weight, layer.mlp.dense_in.weight]
+    before = torch.autograd.grad(y.sum(), wanted, retain_graph=True)
+    with torch.no_grad():
+        layer.self_attention.query.weight.mul_(2.0)
+    assert all(torch.equal(p, q) for p, q in zip(before, torch.autograd.grad(y.sum(), wanted, retain_graph=True)))
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y.sum(), x, retain_graph=True)
+    assert all(torch.equal(p, q) for p, q in zip(before, torch.autograd.grad(y.sum(), wanted)))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(y.sum(), wanted)
