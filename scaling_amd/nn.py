@@ -92,11 +92,20 @@ def _direct(*modules: torch.nn.Module) -> bool:
     return _unhooked(*modules)
 
 
+def _attributes(m: torch.nn.Module, own: dict, *names: str) -> list:
+    """Attributes of a module, from its dictionary `own` of modules or parameters where they are there and nothing is looked at first: an entry of the
+    instance, or something of a class that was derived from the package's."""
+    d = m.__dict__
+    if type(m).__bases__ != (torch.nn.Module,):
+        return [getattr(m, n) for n in names]
+    return [own[n] if n in own and n not in d else getattr(m, n) for n in names]
+
+
 def _weights(modules) -> Tuple[list, list]:
     """Weights and biases (RMSNorm: none) of this package's projections and norms."""
-    kept = [(m._parameters, m) for m in modules]
-    return [p["weight"] if "weight" in p else m.weight for p, m in kept], \
-        [None if type(m) is RMSNorm else p["bias"] if "bias" in p else m.bias for p, m in kept]
+    kept = [(m._parameters, m.__dict__, m) for m in modules]
+    return [p["weight"] if "weight" in p and "weight" not in d else m.weight for p, d, m in kept], \
+        [None if type(m) is RMSNorm else p["bias"] if "bias" in p and "bias" not in d else m.bias for p, d, m in kept]
 
 
 def idle_dropout(m: torch.nn.Module) -> bool:
@@ -741,22 +750,20 @@ def layer_in_one_call(layer, x: torch.Tensor, cumulative_seq_lengths: torch.Tens
     issue; with a cache: of a prefill.  None, with nothing done, where a module below is not the package's own as it is or the operands are not what
     the kernels take: the modules then compute or refuse it."""
     # Modules and parameters come from their dictionaries: as some 40 attributes they took half of the time spent here
-    parts = layer._modules
-    att, mlp, norm1, norm2 = parts["self_attention"], parts["mlp"], parts["input_layernorm"], parts["post_attention_layernorm"]
+    att, mlp, norm1, norm2, *dropouts = _attributes(layer, layer._modules, "self_attention", "mlp", "input_layernorm", "post_attention_layernorm",
+                                                    "dropout_attention", "dropout_mlp")
     if not (type(att) is ParallelSelfAttention and type(mlp) in (ParallelSwiGLUMLP, ParallelMLP)):
         return None
-    own = att._modules
-    sdpa, rot, dtype, training = own["scaled_dot_product_attention"], att.rotary_embedding, att.dtype, layer.training
+    sdpa, rot, dtype, training = *_attributes(att, att._modules, "scaled_dot_product_attention"), att.rotary_embedding, att.dtype, layer.training
     if not (x.is_cuda and x.dim() == 3 and x.dtype == dtype and x.numel() > 0 and not torch.is_autocast_enabled() and _unhooked(att, mlp) and
-            idle_dropout(parts["dropout_attention"]) and idle_dropout(parts["dropout_mlp"]) and not att.key_query_norm and
+            idle_dropout(dropouts[0]) and idle_dropout(dropouts[1]) and not att.key_query_norm and
             type(sdpa) is ScaledDotProductAttention and not (training and sdpa.dropout_p > 0.0) and
             (rot is None or type(rot) in (RotaryEmbedding, RotaryEmbeddingComplex)) and
             _nothing_overridden(att, sdpa, norm1, norm2, *(() if rot is None else (rot,)))):
         return None
     swiglu = type(mlp) is ParallelSwiGLUMLP
-    inner = mlp._modules
-    rest = [own["dense"], inner["dense_in"], inner["siglu_weight"], inner["dense_out"]] if swiglu else [own["dense"], inner["dense_in"], inner["dense_out"]]
-    into = [own["query_key_value"]] if att.qkv_in_one else [own["query"], own["key"], own["value"]]
+    *into, dense = _attributes(att, att._modules, *(("query_key_value",) if att.qkv_in_one else ("query", "key", "value")), "dense")
+    rest = [dense, *_attributes(mlp, mlp._modules, "dense_in", *(("siglu_weight",) if swiglu else ()), "dense_out")]
     if not _direct(*into, *rest) or [True for m in (att, sdpa, mlp, *into, *rest) if m.training != training]:
         return None
     b, s, hidden = x.shape

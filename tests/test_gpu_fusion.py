@@ -771,3 +771,24 @@ def test_parts_of_a_layer_that_is_one_node_look_at_their_own():
     assert all(torch.equal(p, q) for p, q in zip(before, torch.autograd.grad(y.sum(), wanted)))
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(y.sum(), wanted)
+
+
+@pytest.mark.parametrize("case", ["no module", "instance's module", "instance's weight", "class's module"])
+def test_layer_whose_parts_are_not_where_modules_keep_them(case):
+    """A layer reads its parts as attributes do: an identity that is no module, entries of the instance and properties of a derived class count."""
+    layer, other = _layer("float32", True), _layer("float32", True)
+    with torch.no_grad():
+        other.mlp.dense_in.weight.mul_(2.0)
+    io = _io(torch.randn(2, 33, 256, generator=torch.Generator().manual_seed(8)).to(DEV))
+    plain = layer(io).activations
+    if case == "no module":
+        del layer.dropout_attention, layer.dropout_mlp
+        layer.dropout_attention = layer.dropout_mlp = lambda x: x
+    elif case == "instance's module":
+        layer.__dict__["mlp"] = other.mlp
+    elif case == "instance's weight":
+        layer.mlp.dense_in.__dict__["weight"] = other.mlp.dense_in.weight
+    else:
+        layer.__class__ = type("Derived", (TransformerLayer,), dict(mlp=property(lambda self: other.mlp)))
+    got, want = layer(io).activations, _watched(layer, io)
+    assert torch.equal(got, want) and torch.equal(got, plain) == (case == "no module")
