@@ -482,8 +482,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void attn_f32_dkdv_kernel(const 
     constexpr int DT = D / 32, QS = kF32Waves / KGRP, BQ = 32 * QS, BK = 32 * KGRP;
     constexpr int NS = n_stages<D, BQ>(), TILE = BQ * 4 * D;
     // A wavefront has its SIMD to itself and a product takes the matrix pipe 64 cycles, so loads, softmax and moves between two stages of a step cost what they
-    // take: the pipe was busy 0.68 of the time, 0.74 with all of them between products (the rest: a clock of 2.07 GHz instead of 2.17, the barrier of a step, the last
-    // blocks of the launch).  us, before / after: 32 / 8 heads of 128, 4096 tokens 2600 / 2380, 32 / 32, 1101 245 / 230, 8 / 8, 700 (KGRP 1) 70.2 / 66.9; of 96, 32 / 32, 1101
+    // take: 0.68 of the pipe's rate at 2.4 GHz, 0.74 with all of them between products (busy 0.80 of a compute unit's cycles; the rest: a clock of 2.07 GHz instead of 2.17,
+    // the barrier of a step, the last blocks of the launch).  us, before / after: 32 / 8 heads of 128, 4096 tokens 2600 / 2380, 32 / 32, 1101 245 / 230, 8 / 8, 700 (KGRP 1) 70.2 / 66.9; of 96, 32 / 32, 1101
     // 201 / 186.  Where stages are short or one tile deep it does not pay: of 96, KGRP 1 564 / 583, of 64, KGRP 1 100.0 / 101.1 and 11.1 / 11.7, of 32 358 / 359.
     constexpr bool kBetween = D == 128 || (D == 96 && KGRP == 2);
     static_assert(!kBetween || DT >= 2, "dS is formed one row of products behind dP");

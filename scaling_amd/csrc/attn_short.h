@@ -2,9 +2,9 @@
 //
 // The tiled kernels give a workgroup 128 - 256 rows and walk its keys (queries) in one chain of barriers; with short documents that
 // chain is most of the launch, its workgroups leave compute units idle, and 256 rows span several documents.  Here a workgroup of
-// four (two: mi_attn_short_pairs) wavefronts owns 32 rows, and the wavefronts split the other axis: wavefront w takes tiles w, w + 4, ... of 32 tokens,
-// each through its own LDS stages with direct global -> LDS loads and no barrier, and the partial results meet in
-// LDS at the end, in a fixed order.  A document of 512 tokens is a chain of at most four tiles.  The mask interval of a row comes from one
+// four (two: mi_attn_short_pairs) wavefronts owns 32 rows, and the wavefronts split the other axis: wavefront w takes tiles w, w + 4 (w + 2), ... of 32
+// tokens, each through its own LDS stages with direct global -> LDS loads and no barrier, and the partial results meet in
+// LDS at the end, in a fixed order.  A document of 512 tokens is a chain of at most four (eight) tiles.  The mask interval of a row comes from one
 // load of the cumulative lengths and a search in registers.
 // The price is operand traffic: a tile serves 32 rows instead of 128 or 256, so long contexts stay with the tiled kernels
 // (see mi_attn_fwd_is_short and mi_attn_bwd_short).
@@ -140,20 +140,7 @@ template <int D> __device__ __forceinline__ void short_write(elem_t* row, const 
         *reinterpret_cast<uint2*>(row + 32 * dt) = make_uint2(pack_elem2(x[dt][0] * scale, x[dt][1] * scale), pack_elem2(x[dt][2] * scale, x[dt][3] * scale));
 }
 
-// Host side: whether a forward pass goes to these kernels, by its workgroups of 32 rows (rows / 32 x query heads).  A compute unit holds eight of
-// them up to 64 features, two above.  The tiled kernels wait for the longest chain of a workgroup, which is what these kernels shorten; they
-// gain where that chain runs alone: few workgroups, and causal documents, whose last rows have twice the average work.  They lose where the
-// tiled kernels have work for every compute unit all along.  Short / tiled, at 512 | 1024 | 1536 | 2048 workgroups:
-//   64 features:   one causal document .33 - .49 | .37 - .51 | .53 - .64 | .60 - .70     ragged, mean 100 - 800 | | .59 - .80 | .61 - .86
-//                  not causal .41 - .58 | .62 - .73 | .90 - .96 | 1.06 - 1.18            documents of 512 .47 | .70 - .78 | | .91 - 1.06
-//   128 features:  causal .38 - .53 | .51 - .84 | .72 - 1.06 | .91 - 1.2      not causal .50 - .78 | .87 - 1.10 | 1.3 | 1.5
-// (4 / 4, 12 / 12, 16 / 4 and 32 / 8 heads, the rows that make up the count; 1 and 2 heads with documents of up to 65536 tokens alike: the
-// length of a context alone does not decide.)  us at some of these, tiled / short: 32 / 8 heads of 128, 1024 tokens 34.7 / 23.9; 16 heads of
-// 128, 8 documents of 512: 29.3 / 41.3; 12 heads of 64, 3001 tokens in documents of 17 - 400: 20.9 / 12.3; 1 head of 64, 65536 tokens: 1280 / 762.
-// Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
-// backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
-
-// Two wavefronts to a block instead of four.  What comes before and after a chain of tiles costs every wavefront of a block alike, and of four the short
+// Host side: two wavefronts to a block instead of four.  What comes before and after a chain of tiles costs every wavefront of a block alike, and of four the short
 // chains of packed documents leave some without a tile; so two do a block in half as many turns of the chip again, as long as there are blocks
 // enough for it to wait for all of them and not for the longest chain.  That is twice as long now, and its length is not known here, only
 // the mean: hence enough heads, so that one document of half the tokens among 16 small ones is level too (8 heads of 64: 1.25 forward, 1.28
@@ -176,6 +163,18 @@ static inline int64_t mi_attn_short_blocks(const mi_attn_args* a, int64_t heads)
     return (rows + kShortRows - 1) / kShortRows * heads;
 }
 
+// Whether a forward pass goes to these kernels, by its workgroups of 32 rows (rows / 32 x query heads).  A compute unit holds eight of
+// them up to 64 features, two above.  The tiled kernels wait for the longest chain of a workgroup, which is what these kernels shorten; they
+// gain where that chain runs alone: few workgroups, and causal documents, whose last rows have twice the average work.  They lose where the
+// tiled kernels have work for every compute unit all along.  Short / tiled, at 512 | 1024 | 1536 | 2048 workgroups:
+//   64 features:   one causal document .33 - .49 | .37 - .51 | .53 - .64 | .60 - .70     ragged, mean 100 - 800 | | .59 - .80 | .61 - .86
+//                  not causal .41 - .58 | .62 - .73 | .90 - .96 | 1.06 - 1.18            documents of 512 .47 | .70 - .78 | | .91 - 1.06
+//   128 features:  causal .38 - .53 | .51 - .84 | .72 - 1.06 | .91 - 1.2      not causal .50 - .78 | .87 - 1.10 | 1.3 | 1.5
+// (4 / 4, 12 / 12, 16 / 4 and 32 / 8 heads, the rows that make up the count; 1 and 2 heads with documents of up to 65536 tokens alike: the
+// length of a context alone does not decide.)  us at some of these, tiled / short: 32 / 8 heads of 128, 1024 tokens 34.7 / 23.9; 16 heads of
+// 128, 8 documents of 512: 29.3 / 41.3; 12 heads of 64, 3001 tokens in documents of 17 - 400: 20.9 / 12.3; 1 head of 64, 65536 tokens: 1280 / 762.
+// Up to 128 rows are a single workgroup per head and a chain of two key tiles in the tiled kernels: 8.0 / 5.0 us forward and 20 / 14
+// backward (100 rows, 2 heads of 64), both less than the host takes to issue them; such calls stay where they were.
 static inline bool mi_attn_fwd_is_short(const mi_attn_args* a) {
     if (a->flags & (MI_ATTN_QG1 | MI_ATTN_QG2 | MI_ATTN_TILED)) return false;
     if (a->flags & MI_ATTN_SHORT) return true;

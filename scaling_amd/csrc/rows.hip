@@ -252,7 +252,7 @@ template <typename T> int launch(const mi_rows_args& a, hipStream_t st) {
     // Two blocks per workgroup once that leaves four workgroups per compute unit: the rows are read half as often.  Eight wavefronts
     // while there is less than one workgroup of four per SIMD, to have more of the weights in flight.
     const bool wide = !a.glu && blocks16 >= 2048, many = blocks16 >= 1024;
-    // Folded where a compute unit is left with less: 256 workgroups of a quarter or of half a block instead of as many whole ones or fewer, or three halves on
+    // Folded where a compute unit (of 256: the lines count blocks) is left with less: 256 workgroups of a quarter or of half a block instead of as many whole ones or fewer, or three halves on
     // a compute unit instead of two blocks.  us, one / two / four slices, weights from memory: 3 rows, k 1024 -> 1024 4.53 / 3.60 / 3.16, 2816 -> 1024 7.09 / 5.59 /
     // 4.44, 4096 -> 1024 with norm and glu 14.9 / 11.2 / 9.1; 1024 -> 1536 4.77 / 3.90 / 4.20; 4096 -> 6144 15.3 / 13.6 / 14.6 (8 rows 17.2 / 16.3); elsewhere
     // the rows are only read more often: 1024 -> 2816 4.87 / 5.23 / 4.96, 4096 -> 4096 9.00 / 10.0 / 10.7, 8 rows, 4096 -> 10240 25.5 / 27.2.

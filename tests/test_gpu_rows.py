@@ -77,7 +77,6 @@ def test_few_rows_with_norm(rows, k, n, glu, dtype):
     assert _lib.load().mi_rows_product(ctypes.byref(a)) == -3
 
 
-# each side of the lines between the norm inside the product and a launch of its own: (features, k)
 # both sides of the lines between whole, half and quarter blocks (64, 128, 256 and 384 of 16 features); slices that are shorter than others or empty
 @pytest.mark.parametrize("rows,k,n,glu", [(1, 32, 5, False), (4, 2816, 1024, True), (4, 544, 1025, False), (5, 544, 1024, False), (8, 1056, 2048, True),
                                           (8, 96, 2049, False), (3, 64, 4097, False), (8, 2080, 6144, True), (2, 352, 6145, False)])
@@ -106,6 +105,7 @@ def test_folded_rows_equal_whole_blocks(rows, k, n, glu, norm, dtype):
     assert int((~want.isfinite()).sum()) <= rows
 
 
+# each side of the lines between the norm inside the product and a launch of its own: (features, k)
 @pytest.mark.parametrize("n,k,inside", [(4096, 2048, True), (4097, 2048, False), (8192, 1024, True), (8200, 1024, False), (16, 2080, False),
                                         (1536, 4096, False), (1000, 288, True)])
 def test_norm_in_front_of_a_product(n, k, inside):
