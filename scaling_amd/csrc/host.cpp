@@ -1381,7 +1381,8 @@ Tensor op_layer(const Tensor& x, const Tensor& cu, const OptTensor& pos, std::ve
     // One node instead of 9 to 14, views included: the engine takes 4 us for a node beside its launches, and a small step waits for the host.  Forward and backward
     // of 256 x 256, float32: 354 us with nodes of their own, 286 so; 512 x 1024, bf16: 430 and 380 (on a slower host); 1000 x 1024, where the device is what a step
     // waits for: 370 and 370.  What the parts keep is given back one by one either way.
-    if (x.numel() > kOneNode || (c->qkv_w.size() == 1 && !in_one)) return layer_forward(*c, Apart{*c});
+    // An inference tensor can be no input of it: the node keeps x, which nodes of their own need not.
+    if (x.numel() > kOneNode || x.is_inference() || (c->qkv_w.size() == 1 && !in_one)) return layer_forward(*c, Apart{*c});
     return Layer::apply(at::TensorList(inputs), c);
 }
 

@@ -792,3 +792,14 @@ def test_layer_whose_parts_are_not_where_modules_keep_them(case):
         layer.__class__ = type("Derived", (TransformerLayer,), dict(mlp=property(lambda self: other.mlp)))
     got, want = layer(io).activations, _watched(layer, io)
     assert torch.equal(got, want) and torch.equal(got, plain) == (case == "no module")
+
+
+def test_training_of_a_small_layer_on_an_inference_tensor():
+    """x from inference mode, a frozen norm in front of what is trained: nothing that may not be kept has to be."""
+    layer = _layer("bfloat16", True)
+    layer.input_layernorm.requires_grad_(False)
+    with torch.inference_mode():
+        x = torch.randn(2, 33, 256, device=DEV).to(torch.bfloat16)
+    io, inputs = _io(x), [p for p in layer.parameters() if p.requires_grad]
+    got, want = (torch.autograd.grad(y.float().sum(), inputs) for y in (layer(io).activations, _watched(layer, io)))
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
