@@ -9,9 +9,7 @@ import pytest
 from scaling_amd.csrc.build import LIB_PATH
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
-PASSES = 16                                                # of v_mfma_f32_32x32x2_f32: the next product starts no earlier
-RESULT = 18                                                # wait states between this product and another instruction's use of its result
-OPERAND = 2                                                # between a vector instruction's result and a product that takes it
+OPERAND = 2                                                # wait states between a vector instruction's result and a product that takes it
 
 
 def _code_objects(path):
@@ -60,15 +58,16 @@ def _function(lines):
     return code, after
 
 
-def _early(code, after, n, limit, meets):
-    """Instructions that `meets` names and that some way through the code reaches less than `limit` wait states behind instruction n"""
+def _early(code, after, n, limit, passes, meets):
+    """Instructions that `meets` names and that some way through the code reaches less than `limit` wait states behind instruction n; a product starts `passes`
+    behind another at the soonest"""
     found, best = [], {}
-    todo = [(m, 0, 0 if code[n].matrix else -PASSES) for m in after[n]]     # where, states since n, when the last product started
+    todo = [(m, 0, 0 if code[n].matrix else -passes) for m in after[n]]     # where, states since n, when the last product started
     while todo:
         m, states, product = todo.pop()
         i = code[m]
         if i.matrix:
-            states = max(states, product + PASSES)
+            states = max(states, product + passes)
         if states >= limit or best.get(m, (limit, 0)) <= (states, -product):
             continue
         best[m] = (states, -product)
@@ -89,21 +88,25 @@ def _kernels(pattern):
 
 
 @pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(LIB_PATH)), reason="no library, or nothing to list its code with")
-def test_products_and_their_neighbours_in_float32_backward():
-    """dK / dV of float32: nothing reads or overwrites a product's result, and no product takes a vector instruction's, too early"""
-    kernels = dict(_kernels("attn_f32_dkdv_kernel"))
-    assert len(kernels) >= 11
+# kernels, their products, the passes that one takes at least, wait states between it and another instruction's use of its result
+@pytest.mark.parametrize("pattern,count,product,passes,states", [
+    ("attn_f32_dkdv_kernel", 11, r"v_mfma_f32_32x32x2_f32", 16, 18), ("11wide_kernelI", 4, r"v_mfma_f32_16x16x32_b?f16", 4, 12),
+])
+def test_products_and_their_neighbours(pattern, count, product, passes, states):
+    """Nothing reads or overwrites a product's result, and no product takes a vector instruction's, too early."""
+    kernels = dict(_kernels(pattern))
+    assert len(kernels) >= count
     for name, (code, after) in kernels.items():
         assert any(i.matrix for i in code), name
         for n, i in enumerate(code):
             result = i.operands[0]
             if i.matrix:
-                assert i.name == "v_mfma_f32_32x32x2_f32", i.text
+                assert re.fullmatch(product, i.name), i.text
                 # a product that adds to the whole of it may follow at once
-                early = _early(code, after, n, RESULT, lambda j: (result & j.uses) and not (
+                early = _early(code, after, n, states, passes, lambda j: (result & j.uses) and not (
                     j.matrix and j.operands[0] == result and j.operands[3] in (result, frozenset()) and not result & (j.operands[1] | j.operands[2])))
             elif i.vector and result:
-                early = _early(code, after, n, OPERAND, lambda j: j.matrix and result & (j.operands[1] | j.operands[2] | j.operands[3]))
+                early = _early(code, after, n, OPERAND, passes, lambda j: j.matrix and result & (j.operands[1] | j.operands[2] | j.operands[3]))
             else:
                 continue
             assert not early, f"{name}: {i.text}: {early}"
